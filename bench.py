@@ -155,8 +155,8 @@ def config3_extra(T, torch, build_index, run, args):
     for nq, steps in ((1024, max(3, args.steps // 2)), (1, max(args.steps, 15))):
         dt, scan_ms, launches, q_full = run(nq, steps, 1, ix=ix, k=k, dim=dim)
         launch_s = scan_ms * 1e-3 / max(launches, 1)
-        # byte tables serve single queries; sixteen queries per pass stream their tables through LDS
-        kern = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
+        # byte tables serve single queries; a batch is one launch of the sparse matrix-unit scan
+        kern = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut_mx" if q_full > 16 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
         res[f"batch{nq}"] = {"queries_per_s": nq * steps / dt, "ms_per_step": dt / steps * 1e3,
                              "queries_per_launch": q_full, "scan_launch_ms": launch_s * 1e3,
                              "roofline": {"bound": "hbm", "achieved": alg / launch_s / 1e9, "peak": 8000.0,
@@ -394,7 +394,7 @@ def main():
     if mode_p:
         kernel = "k_scan_p4_wide" if q_full >= 256 else "k_scan_p4_multi" if q_full > 32 else "k_scan_p4"
     else:
-        kernel = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
+        kernel = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut_mx" if q_full > 16 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
     traffic = MEASURED_TRAFFIC.get((kernel, n, dim, bits))
     int8_ops = 2.0 * q_per_launch * n * dim        # multiply-adds x2 of one launch, permute-dot mode
 

@@ -8,7 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libturbovec_hip.so")
 
-SOURCES = ["tv_kernels.hip", "tv_kernels2.hip", "tv_kernels3.hip", "tv_kernels4.hip", "tv_encode.hip", "tv_api.hip", "host_tables.cpp", "tv_snapshot.cpp"]
+SOURCES = ["tv_kernels.hip", "tv_kernels2.hip", "tv_kernels3.hip", "tv_kernels4.hip", "tv_kernels5.hip", "tv_encode.hip", "tv_api.hip", "host_tables.cpp", "tv_snapshot.cpp"]
 
 # -ffp-contract=off: the parity contract is bit-exact float arithmetic, fused
 # only where the code says fmaf.  The packed-FP32 feature is switched off for
@@ -28,9 +28,12 @@ FLAGS = [
 # The scan kernels request LDS and global loads through inline assembly the compiler's wait-count
 # bookkeeping does not see, and wait for them by hand: a register spilled or reloaded between such
 # a request and its wait would be read stale, silently.  So none of them may touch scratch memory.
-# (k_scan_p4, k_scan_p4_multi, k_scan_p4_wide, k_scan_lut16 and the matrix-unit probe;
+# (k_scan_p4, k_scan_p4_multi, k_scan_p4_wide, k_scan_lut16, k_scan_lut_mx and the matrix-unit probe;
 # k_scan_p4_batched and the other LUT scans leave every wait to the compiler.)
-NO_SCRATCH = re.compile(r"k_scan_p4I|k_scan_p4_multiI|k_scan_p4_wideI|k_scan_lut16I|k_probe_mfma")
+NO_SCRATCH = re.compile(r"k_scan_p4I|k_scan_p4_multiI|k_scan_p4_wideI|k_scan_lut16I|k_scan_lut_mxI|k_probe_mfma")
+# A scalar register kept in a lane of a vector register (no memory, and never a register a request
+# is on its way to) is harmless; this kernel's operand constants overflow the scalar file.
+SGPR_LANES = re.compile(r"k_scan_lut_mxI")
 # These address their byte -> levels table by the byte's value alone: the table must sit at LDS
 # address 0, i.e. the kernel may have no static LDS allocation in front of its dynamic one
 # (k_scan_p4, k_scan_p4_multi, and the instances of k_scan_p4_wide whose last template argument,
@@ -54,7 +57,7 @@ def check_resources(src, remarks):
         if what.startswith("LDS"):
             if value and NO_STATIC_LDS.search(name):
                 problems.append(f"{name}: {value} bytes of static LDS in front of the byte table")
-        elif value and NO_SCRATCH.search(name):
+        elif value and NO_SCRATCH.search(name) and not (what == "SGPRs Spill" and SGPR_LANES.search(name)):
             problems.append(f"{name}: {what} = {value}")
     if problems:
         raise RuntimeError(f"{src}: kernels with hand-placed waits must not spill or use scratch:\n  " + "\n  ".join(problems))

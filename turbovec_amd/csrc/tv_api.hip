@@ -174,17 +174,30 @@ int upload_tables(tv_index *ix) {
 int effective_mode(const tv_index *ix);
 // Queries one LUT-scan launch serves: the scalar definition's float chain runs one query at a time.
 int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCORE_L_SCALAR ? 1 : tv::lut_tile_queries(ix->geo.nch, k); }
-// Queries one append-mode LUT launch serves: sixteen with the u32 and the classic epilogues (tables
-// streamed through LDS), one for the scalar definition's chain.
+// Batches of u8-LUT queries beyond what the whole-table scan serves in one pass (eight queries, fewer
+// where the rows are long) go sixteen queries per pass through k_scan_lut16 or, with the u32
+// epilogue, all in one launch of the sparse matrix-unit scan; the scalar definition's chain of adds
+// takes one query at a time.  One pass for up to sixteen queries beats the matrix-unit scan's
+// half-empty tile (1M x 1536 2-bit, 16 queries: 0.26 ms a search against 0.30); from 17 on it
+// would be two (33 queries: 0.56 against 0.40 ms; 400: 4.6 against 2.2).  Below about 4096 (block,
+// query tile) pairs most of the matrix-unit scan's waves have no block, and the sixteen-query passes
+// are the faster ones (20K x 1536 2-bit, 33 queries, 1250 pairs: 153 us against 155; 65K rows, 4096
+// pairs: 165 against 131).
+constexpr size_t kMxMinPairs = 4096;
+bool lut_mx_serves(const tv_index *ix, size_t cq) {
+    const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
+    return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && cq > size_t(tv::kLut16Queries) &&
+           n_blocks * tiles >= kMxMinPairs;
+}
 bool lut16_serves(const tv_index *ix) {
     return (effective_mode(ix) == TV_SCORE_L_U32 || effective_mode(ix) == TV_SCORE_L_CLASSIC) && !ix->no_lut16;
 }
-int lut_append_q(const tv_index *ix) {
-    if (effective_mode(ix) == TV_SCORE_L_SCALAR) return 1;
-    return lut16_serves(ix) ? tv::kLut16Queries : tv::lut_append_queries(ix->geo.nch);
-}
 // Tiles of fewer queries than this keep the whole-table scan (its pass is as long for 8 queries as for 1).
-constexpr int kLut16MinQueries = 9;
+int lut16_min_queries(const tv_index *ix) { return tv::lut_append_queries(ix->geo.nch) + 1; }
+int lut_append_q(const tv_index *ix, size_t cq) {
+    if (effective_mode(ix) == TV_SCORE_L_SCALAR) return 1;
+    return lut_mx_serves(ix, cq) ? tv::kQTile : lut16_serves(ix) ? tv::kLut16Queries : tv::lut_append_queries(ix->geo.nch);
+}
 
 int effective_mode(const tv_index *ix) {
     int m = ix->score_mode;
@@ -196,6 +209,7 @@ struct Prepared {
     float *d_qrot = nullptr;   // rotated (and calibrated) rows
     uint8_t *d_tables = nullptr;
     uint8_t *d_tables16 = nullptr;   // mode L: the same tables entry-major for the sixteen-query scan (or null)
+    uint8_t *d_tables_mx = nullptr;  // mode L: the same tables as matrix operands for the sparse scan (or null)
     float *d_qscale = nullptr, *d_qbias = nullptr;
     size_t table_bytes_per_tile = 0;
 };
@@ -205,7 +219,7 @@ struct Prepared {
 // `split`: permute-dot weights in the order k_scan_p4 reads them (the batched scans take plane order)
 // `keep_rotated`: the rotated rows are wanted in device memory too (the debug read-back); a search
 // in permute-dot mode does not need them and prepares its queries in a single launch.
-// `for_append`: u8-LUT tables are wanted entry-major too, for the sixteen-query append scan.
+// `for_append`: u8-LUT tables are wanted in the order of the batch's append scan too.
 int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepared &out, bool split = true,
                     bool keep_rotated = false, bool for_append = false) {
     const tv::Geometry &g = ix->geo;
@@ -248,7 +262,10 @@ int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepar
         out.d_tables = ar.take<uint8_t>(nq_pad * size_t(g.nch) * 1024);
         TV_HIP(tv::launch_build_lut(d_cal, d_bias_corr, ix->d_centroids, out.d_tables, out.d_qscale, out.d_qbias,
                                     g.dim, g.bits, g.G, g.nch, nq, nq_pad, ix->stream));
-        if (for_append && lut16_serves(ix) && nq >= size_t(kLut16MinQueries)) {
+        if (for_append && lut_mx_serves(ix, nq)) {
+            out.d_tables_mx = ar.take<uint8_t>(tv::mx_table_bytes(g.nch, g.bits, nq));
+            TV_HIP(tv::launch_lut_fragments(out.d_tables, out.d_tables_mx, g.nch, g.bits, nq, ix->stream));
+        } else if (for_append && lut16_serves(ix) && nq >= size_t(lut16_min_queries(ix))) {
             out.d_tables16 = ar.take<uint8_t>(tv::lut16_table_bytes(g.nch, nq));
             TV_HIP(tv::launch_lut_interleave16(out.d_tables, out.d_tables16, g.nch, nq, ix->stream));
         }
@@ -261,7 +278,8 @@ size_t prepare_bytes(const tv_index *ix, size_t nq) {
     const size_t nq_pad = round_up(nq, tv::kQTile);
     size_t b = 2 * round_up(nq * g.dim * 4, 256) + 3 * round_up(nq_pad * 4, 256);
     b += round_up(nq_pad * size_t(g.nch) * 1024, 256) + 4096;
-    if (lut16_serves(ix)) b += round_up(tv::lut16_table_bytes(g.nch, nq), 256);
+    if (lut_mx_serves(ix, nq)) b += round_up(tv::mx_table_bytes(g.nch, g.bits, nq), 256);
+    else if (lut16_serves(ix)) b += round_up(tv::lut16_table_bytes(g.nch, nq), 256);
     return b;
 }
 
@@ -318,6 +336,7 @@ size_t robust_need(const tv_index *ix, size_t cq, size_t k_eff) {
 struct SampledPlan {
     size_t tile_q, n_tiles, cq_pad, seg_stride, need;
     bool wide;
+    bool lut_mx;        // u8-LUT queries of this chunk take the sparse matrix-unit scan, all in one launch
     bool lut16;         // u8-LUT tiles of this chunk take the sixteen-query scan
     bool lut_single;    // one u8-LUT query, served by the byte-table scan
     int nt_batched;     // query tiles one launch of the tile-group kernels serves (0: one tile per launch)
@@ -327,19 +346,20 @@ SampledPlan sampled_plan(const tv_index *ix, size_t cq) {
     const tv::Geometry &g = ix->geo;
     const bool mode_p = effective_mode(ix) == TV_SCORE_P;
     SampledPlan p;
-    p.tile_q = mode_p ? size_t(tv::kQTile) : size_t(lut_append_q(ix));
+    p.tile_q = mode_p ? size_t(tv::kQTile) : size_t(lut_append_q(ix, cq));
     p.n_tiles = (cq + p.tile_q - 1) / p.tile_q;
     p.cq_pad = p.n_tiles * p.tile_q;
     // large chunks of high-dimensional queries take the wide kernel: all of them in one pass per level
     const int wide_min = tv::wide_min_queries(g.nch);
     p.wide = mode_p && !ix->no_batched && !ix->no_wide && wide_min > 0 && cq >= size_t(wide_min);
-    p.lut16 = !mode_p && lut16_serves(ix) && cq >= size_t(kLut16MinQueries);
+    p.lut_mx = !mode_p && lut_mx_serves(ix, cq);
+    p.lut16 = !mode_p && !p.lut_mx && lut16_serves(ix) && cq >= size_t(lut16_min_queries(ix));
     p.nt_batched = (mode_p && cq > size_t(tv::kQTile) && !ix->no_batched) ? tv::batched_tiles(g.nch) : 0;
     p.grid = p.wide ? tv::wide_grid_blocks(ix->device)
            : mode_p ? tv::scan_grid_blocks(ix->device, mode_p, g.nch, 0, int(p.tile_q))
                     : tv::lut_append_grid(ix->device, g.nch);
     p.lut_single = !mode_p && cq == 1 && effective_mode(ix) != TV_SCORE_L_SCALAR && tv::lut_single_uses_byte_tables(g.nch, p.grid);
-    p.seg_stride = size_t(p.grid);
+    p.seg_stride = p.lut_mx ? size_t(tv::mx_segments()) : size_t(p.grid);
     // (a query keeps one candidate segment per workgroup of the launches that serve it: every launch
     // of a chunk the tile-group kernels serve is one of theirs, and their grid is not the single-tile scan's)
     if (p.nt_batched > 0 && !p.wide) p.seg_stride = size_t(tv::batched_grid_blocks(ix->device, g.nch));
@@ -570,6 +590,7 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
     }
     // (the sixteen-query LUT scan works in rounds too: every wave of the grid carries two blocks through the row)
     return plan.wide    ? sampling_steps(n_blocks, k_floor, size_t(plan.grid) * tv::wide_blocks_per_workgroup(ix->geo.nch))
+           : plan.lut_mx ? sampling_steps(n_blocks, k_floor, size_t(tv::mx_round_blocks(ix->device, plan.cq_pad)))
            : plan.lut16 ? sampling_steps(n_blocks, k_floor, size_t(plan.grid) * tv::lut16_blocks_per_workgroup(effective_mode(ix) == TV_SCORE_L_CLASSIC))
                         : sampling_steps(n_blocks, k_floor);
 }
@@ -676,7 +697,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
 
             const int bgrid = tv::batched_grid_blocks(ix->device, g.nch);
             const bool batched = nt_batched > 0 && !wide;
-            const size_t tiles_per_launch = wide ? n_tiles : batched ? size_t(nt_batched) : 1;
+            const size_t tiles_per_launch = wide || plan.lut_mx ? n_tiles : batched ? size_t(nt_batched) : 1;
             if (!repeat && q0 == 0) ix->last_queries_per_launch = int(std::min(pq_n, tile_q * tiles_per_launch));   // the call's first chunk
             for (size_t lv = 0; lv < steps.size(); ++lv) {
                 const bool last = lv + 1 == steps.size();
@@ -700,7 +721,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                     // sampling levels of the sixteen-query LUT scan: all the chunk's tiles it serves in one
                     // launch, side by side (one tile leaves most of the chip idle for a round's time)
                     const size_t side_by_side = (plan.lut16 && !last && pq.d_tables16 != nullptr)
-                                                    ? pq_n / tile_q + (pq_n % tile_q >= size_t(kLut16MinQueries) ? 1 : 0) : 0;
+                                                    ? pq_n / tile_q + (pq_n % tile_q >= size_t(lut16_min_queries(ix)) ? 1 : 0) : 0;
                     for (size_t t = 0; t < n_tiles; t += (t < side_by_side ? side_by_side : tiles_per_launch), ++launch_no) {
                         tv::ScanArgs a;
                         fill_scan_args(ix, a);
@@ -734,11 +755,16 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                             TV_HIP(tv::launch_scan_p4_batched(a, n_seg, ix->stream));
                         } else if (mode_p) {
                             TV_HIP(tv::launch_scan_p4(a, lgrid, (best_first && lv == 0) ? tv::kModeBest : tv::kModeAppend, ix->stream));
+                        } else if (plan.lut_mx) {
+                            const tv::MxShape shape = tv::mx_shape(ix->device, pq_n, level_blocks, lv == 0 && !repeat);
+                            n_seg = int(shape.wgs * shape.sub);
+                            a.tables = pq.d_tables_mx;
+                            TV_HIP(tv::launch_scan_lut_mx(a, shape, g.bits, ix->stream));
                         } else if (t < side_by_side) {
                             a.tables = pq.d_tables16;
                             a.nq_tile = int(std::min<size_t>(pq_n, side_by_side * tile_q));
                             TV_HIP(tv::launch_scan_lut16(a, lgrid, int(side_by_side), ix->stream));
-                        } else if (pq.d_tables16 != nullptr && a.nq_tile >= kLut16MinQueries) {
+                        } else if (pq.d_tables16 != nullptr && a.nq_tile >= lut16_min_queries(ix)) {
                             a.tables = pq.d_tables16 + t * tv::lut16_table_bytes(g.nch, tile_q);
                             TV_HIP(tv::launch_scan_lut16(a, lgrid, 1, ix->stream));
                         } else {

@@ -121,6 +121,17 @@ size_t lut16_table_bytes(int nch, size_t nq);
 hipError_t launch_lut_interleave16(const uint8_t *d_src, uint8_t *d_dst, int nch, size_t nq, hipStream_t s);
 hipError_t launch_scan_lut16(const ScanArgs &a, int grid, int tiles, hipStream_t s);
 int lut16_blocks_per_workgroup(bool classic);   // blocks one workgroup carries through a round of the row's chunks
+// Batches in score mode L with the u32 epilogue, on the sparse matrix instructions (tv_kernels5.hip).
+struct MxShape {
+    unsigned groups, wgs, sub;   // query groups, workgroups per group, segments per workgroup and query
+    int nt, blk;                 // query tiles per group, blocks per wave and round
+};
+size_t mx_table_bytes(int nch, int bits, size_t nq);
+hipError_t launch_lut_fragments(const uint8_t *d_src, uint8_t *d_dst, int nch, int bits, size_t nq, hipStream_t s);
+MxShape mx_shape(int device, size_t nq, size_t level_blocks, bool open_floors);
+int mx_segments();
+int mx_round_blocks(int device, size_t nq);   // blocks a launch over nq queries works through per round
+hipError_t launch_scan_lut_mx(const ScanArgs &a, const MxShape &m, int bits, hipStream_t s);
 hipError_t launch_scan_p4(const ScanArgs &a, int grid, int mode, hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).
