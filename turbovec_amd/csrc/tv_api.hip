@@ -164,6 +164,9 @@ int upload_tables(tv_index *ix) {
                           ix->stream));
     TV_HIP(hipMemcpyAsync(ix->d_perms, ix->rot.perms.data(), 2 * dim * sizeof(uint32_t), hipMemcpyHostToDevice,
                           ix->stream));
+    std::vector<uint32_t> packed(dim);
+    ix->packed_ok = tv::encode_pack_tables(ix->rot.signs.data(), ix->rot.perms.data(), int(dim), packed.data());
+    if (ix->packed_ok) TV_HIP(hipMemcpyAsync(ix->d_packed, packed.data(), dim * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
     float cen[16] = {0};
     for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
     TV_HIP(hipMemcpyAsync(ix->d_centroids, cen, sizeof cen, hipMemcpyHostToDevice, ix->stream));
@@ -1125,6 +1128,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         if (hipStreamCreateWithFlags(&ix->stream, hipStreamNonBlocking) != hipSuccess) { rc = TV_ERR_HIP; break; }
         if (hipMalloc(reinterpret_cast<void **>(&ix->d_signs), 2 * size_t(dim) * sizeof(float)) != hipSuccess ||
             hipMalloc(reinterpret_cast<void **>(&ix->d_perms), 2 * size_t(dim) * sizeof(uint32_t)) != hipSuccess ||
+            hipMalloc(reinterpret_cast<void **>(&ix->d_packed), size_t(dim) * sizeof(uint32_t)) != hipSuccess ||
             hipMalloc(reinterpret_cast<void **>(&ix->d_centroids), 16 * sizeof(float)) != hipSuccess ||
             hipMalloc(reinterpret_cast<void **>(&ix->d_tq_shift), size_t(dim) * sizeof(float)) != hipSuccess ||
             hipMalloc(reinterpret_cast<void **>(&ix->d_tq_scale), size_t(dim) * sizeof(float)) != hipSuccess ||
@@ -1163,7 +1167,7 @@ int tv_index_destroy(tv_index *ix) {
     if (!ix) return TV_OK;
     (void)hipSetDevice(ix->device);
     if (ix->stream) (void)hipStreamSynchronize(ix->stream);
-    void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
+    void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
                     ix->d_codes, ix->d_scales, ix->ws, ix->io, ix->d_tau_open};
     for (void *p : ptrs) if (p) (void)hipFree(p);
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
@@ -1319,7 +1323,7 @@ static int add_device_rows(tv_index *ix, const float *d_vectors, size_t n_new) {
     for (size_t r0 = 0; r0 < n_new; r0 += slice) {
         const size_t nr = std::min(slice, n_new - r0);
         TV_HIP(tv::launch_encode(d_vectors + r0 * size_t(g.dim), nr, ix->n + r0, ix->d_signs, ix->d_perms,
-                                 cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr,
+                                 ix->packed_ok ? ix->d_packed : nullptr, cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr,
                                  ix->cb.centroids.data(), ix->cb.boundaries.data(), g, ix->rot.block,
                                  ix->rot.inv_sqrt_block, ix->d_codes, ix->d_scales, nullptr, ix->stream));
     }
@@ -1394,7 +1398,7 @@ int tv_index_calibrate(tv_index *ix, const float *sample, size_t n) {
         for (size_t r0 = 0; r0 < n; r0 += slice) {
             const size_t nr = std::min(slice, n - r0);
             TV_HIP(hipMemcpyAsync(d_in, sample + r0 * dim, nr * dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
-            TV_HIP(tv::launch_encode(d_in, nr, 0, ix->d_signs, ix->d_perms, nullptr, nullptr, ix->cb.centroids.data(),
+            TV_HIP(tv::launch_encode(d_in, nr, 0, ix->d_signs, ix->d_perms, nullptr, nullptr, nullptr, ix->cb.centroids.data(),
                                      ix->cb.boundaries.data(), ix->geo, ix->rot.block, ix->rot.inv_sqrt_block,
                                      nullptr, nullptr, d_out, ix->stream));
             TV_HIP(hipMemcpyAsync(rotated.data() + r0 * dim, d_out, nr * dim * sizeof(float), hipMemcpyDeviceToHost, ix->stream));

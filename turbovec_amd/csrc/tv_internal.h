@@ -81,11 +81,14 @@ hipError_t launch_native_to_seq(const uint8_t *d_native, uint8_t *d_seq, const G
 hipError_t launch_append_rows(const uint8_t *d_rows, uint8_t *d_native, const Geometry &g, size_t old_n,
                               size_t n_new, hipStream_t s);
 hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const float *d_signs,
-                         const uint32_t *d_perms, const float *d_shift, const float *d_scale,
+                         const uint32_t *d_perms, const uint32_t *d_packed, const float *d_shift, const float *d_scale,
                          const float *centroids, const float *boundaries, const Geometry &g, int block,
                          float inv_sqrt_block, uint8_t *d_native, float *d_scales, float *d_rot_out,
                          hipStream_t s);
 size_t encode_lds_bytes(int dim);
+// The rotation tables of both rounds in one word per position for the several-rows-per-workgroup
+// encoder; false where it does not apply (long rows, signs other than +-1).
+bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint32_t *packed);
 hipError_t launch_move_lane(uint8_t *d_native, float *d_scales, const Geometry &g, size_t src, size_t dst,
                             hipStream_t s);
 
@@ -198,6 +201,8 @@ struct tv_index {
     bool events_ready = false;
     float *d_signs = nullptr;
     uint32_t *d_perms = nullptr;
+    uint32_t *d_packed = nullptr;  // both rounds' gathers and signs in one word per position (encode_pack_tables) ...
+    bool packed_ok = false;        // ... when the tables in use have that form
     float *d_centroids = nullptr;
     float *d_tq_shift = nullptr, *d_tq_scale = nullptr;
     int *d_tau_open = nullptr;     // order key of -inf per query: the floors before any level has run
