@@ -1219,68 +1219,29 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 
 // ===========================================================================
 // Final selection over the candidates an append-mode scan collected: one
-// workgroup per query sorts its (few) candidate keys in LDS and emits the first
-// k_eff.  A query whose candidates did not fit is flagged for the caller to
-// redo through the list path.
+// workgroup per query finds the `need` largest keys and emits them in order, or
+// takes the last of them as a floor.  A query whose candidates did not fit is
+// flagged for the caller to redo.
+//
+// The work is a few thousand keys in a few hundred short segments, and all of
+// it is latency; a thousand queries share the chip.  So: a thread per segment,
+// its head requested together with its count; one pass of counting into 1024
+// bins between the smallest and the largest key gives a threshold few keys
+// reach (a bin that still holds too many is divided again); those are collected
+// in LDS and ranked by comparing each with all -- no sort, a handful of
+// barriers, 28 KiB of LDS, and workgroups no larger than the segments need.
+// Per launch under the profiler, before (waves sorting chunks in 64 KiB of LDS,
+// 1024 threads per query) and now: one query, k = 10, 12 -> 6 to 10 us; k = 100,
+// 60 and 33 -> 22 and 17 us; 1000 queries, k = 10, 61 to 75 -> 12 to 18 us.
 // ===========================================================================
+constexpr uint32_t kFinalBins = 1024;
+constexpr uint32_t kFinalKept = 1024;      // keys ranked at the end: more than are ever wanted (kMaxSampledK)
+constexpr uint32_t kFinalStage = 2048;     // candidates copied to LDS when some segment is long
+constexpr uint32_t kFinalLong = 128;       // ... of which this many segments can be
+static_assert(kFinalKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
 
-__device__ __forceinline__ uint64_t wave_umax64(uint64_t v) {
-    const uint32_t hi = uint32_t(v >> 32), lo = uint32_t(v);
-    const uint32_t mhi = wave_umax(hi);
-    const uint32_t mlo = wave_umax(hi == mhi ? lo : 0u);
-    return (uint64_t(mhi) << 32) | mlo;
-}
-// Eight keys in descending order (Batcher's odd-even merge network, 19 exchanges).
-__device__ __forceinline__ void sort8_desc(uint64_t (&r)[8]) {
-    auto ce = [&](int i, int j) { if (r[i] < r[j]) { const uint64_t x = r[i]; r[i] = r[j]; r[j] = x; } };
-    ce(0, 1); ce(2, 3); ce(4, 5); ce(6, 7);
-    ce(0, 2); ce(1, 3); ce(4, 6); ce(5, 7);
-    ce(1, 2); ce(5, 6);
-    ce(0, 4); ce(1, 5); ce(2, 6); ce(3, 7);
-    ce(2, 4); ce(3, 5);
-    ce(1, 2); ce(3, 4); ce(5, 6);
-}
-// Sixteen keys in descending order: two sorted eights, then a bitonic merge (70 exchanges).
-__device__ __forceinline__ void sort16_desc(uint64_t (&r)[16]) {
-    auto ce = [&](int i, int j) { if (r[i] < r[j]) { const uint64_t x = r[i]; r[i] = r[j]; r[j] = x; } };
-    uint64_t a[8], b[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { a[e] = r[e]; b[e] = r[8 + e]; }
-    sort8_desc(a);
-    sort8_desc(b);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { r[e] = a[e]; r[8 + e] = b[e]; }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ce(i, 15 - i);              // the eight larger in front, both halves bitonic
-#pragma unroll
-    for (int stride = 4; stride >= 1; stride >>= 1) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if ((i & stride) == 0) ce(i, i + stride);
-    }
-}
-// The `need` (<= 32) largest of the wave's keys -- N per lane, sorted descending, 0 = none,
-// non-zero keys distinct -- in order: lane i returns the i-th largest (0 beyond what there is).
-// One largest key is found and retired per turn; nothing touches LDS.
-template <int N>
-__device__ __forceinline__ uint64_t wave_top(uint64_t (&r)[N], uint32_t need, uint32_t lane) {
-    uint64_t mine = 0ull;
-    for (uint32_t it = 0; it < need; ++it) {
-        const uint64_t m = wave_umax64(r[0]);
-        if (lane == it) mine = m;
-        if (r[0] == m && m != 0ull) {
-#pragma unroll
-            for (int e = 0; e < N - 1; ++e) r[e] = r[e + 1];
-            r[N - 1] = 0ull;
-        }
-    }
-    return mine;
-}
-
-constexpr int kFinalThreads = 1024;
-constexpr int kFinalLong = kFinalCap / 8;   // segments of more than 8 keys that fit the sort buffer
-
-__global__ __launch_bounds__(kFinalThreads) void k_final(const uint64_t *__restrict__ cand,
+template <uint32_t T>
+__global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                const uint32_t *__restrict__ cand_cnt, uint32_t n_seg,
                                                uint32_t seg_stride, int k_eff, int k_floor,
                                                float *__restrict__ out_scores, int64_t *__restrict__ out_idx,
@@ -1288,26 +1249,30 @@ __global__ __launch_bounds__(kFinalThreads) void k_final(const uint64_t *__restr
                                                int tau_stride_q, int keep_floor, int *__restrict__ raise_out,
                                                const uint32_t *__restrict__ row_map, uint32_t *level_over,
                                                uint32_t *clear_flag, const uint32_t *run_if) {
-    __shared__ uint64_t keys[kFinalCap];
-    __shared__ uint32_t wave_sum[kFinalThreads / 64];
-    __shared__ uint32_t any_full, long_n, any_long, any_over8;
+    constexpr uint32_t W = T / 64, kPerBin = kFinalBins / T;
+    __shared__ __align__(16) uint64_t kept[kFinalKept + 2];
+    __shared__ uint64_t stage[kFinalStage];
+    __shared__ uint32_t bins[kFinalBins];
+    __shared__ uint32_t w_sum[W], w_max[W], w_min[W];
+    __shared__ uint32_t any_full, any_long, long_n, n_kept, s_bin, s_at, s_above;
     __shared__ uint32_t long_seg[kFinalLong], long_pos[kFinalLong], long_cnt[kFinalLong];
+    if (launch_switched_off(run_if)) return;
     const int qn = blockIdx.x;
-    const int t = threadIdx.x;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
     const bool sampling = tau_out != nullptr;
     int *tau_slot = sampling ? tau_out + (qn / tau_stride_q) * kQTile + qn % tau_stride_q : nullptr;
-    if (launch_switched_off(run_if)) return;
     if (clear_flag != nullptr && qn == 0 && t == 0) *clear_flag = 0u;
-    if (t == 0) { any_full = 0u; long_n = 0u; any_long = 0u; any_over8 = 0u; }
+    if (t == 0) { any_full = 0u; any_long = 0u; long_n = 0u; n_kept = 0u; }
+    for (uint32_t i = t; i < kFinalBins; i += T) bins[i] = 0u;
     __syncthreads();
     // every thread owns a contiguous run of this query's segments
-    const uint32_t per = (n_seg + kFinalThreads - 1) / kFinalThreads;
-    const uint32_t s0 = min(uint32_t(t) * per, n_seg), s1 = min(s0 + per, n_seg);
+    const uint32_t per = (n_seg + T - 1) / T;
+    const uint32_t s0 = min(t * per, n_seg), s1 = min(s0 + per, n_seg);
     const uint32_t *cnt = cand_cnt + size_t(qn) * seg_stride;
+    const uint64_t *segs = cand + size_t(qn) * seg_stride * kSegCap;
     constexpr uint32_t kShort = 16;
     // One segment per thread (the usual case): its head is requested together with its count, not
-    // after it -- the segment's memory is there whatever the count says -- which takes one trip to
-    // memory out of a kernel that is nothing but latency.
+    // after it -- the segment's memory is there whatever the count says.
     const bool one_each = per == 1;
     uint64_t head[kShort];
 #pragma unroll
@@ -1315,14 +1280,13 @@ __global__ __launch_bounds__(kFinalThreads) void k_final(const uint64_t *__restr
     uint32_t mine = 0;
     if (one_each) {
         if (s0 < s1) {
-            const uint64_t *src = cand + (size_t(qn) * seg_stride + s0) * kSegCap;
+            const uint64_t *src = segs + size_t(s0) * kSegCap;
             const uint32_t c = cnt[s0];
 #pragma unroll
             for (uint32_t e = 0; e < kShort; ++e) head[e] = src[e];
             if (c > kSegCap) any_full = 1u;
             mine = min(c, uint32_t(kSegCap));
             if (mine > kShort) any_long = 1u;
-            if (mine > 8u) any_over8 = 1u;
         }
     } else {
         for (uint32_t sg = s0; sg < s1; ++sg) {
@@ -1331,16 +1295,27 @@ __global__ __launch_bounds__(kFinalThreads) void k_final(const uint64_t *__restr
             mine += min(c, uint32_t(kSegCap));
         }
     }
-    // exclusive prefix over the 256 threads
+    // exclusive prefix over the threads, and the total
     uint32_t incl = mine;
     for (int off = 1; off < 64; off <<= 1) {
         const uint32_t v = __shfl_up(incl, off);
-        if ((t & 63) >= off) incl += v;
+        if (lane >= uint32_t(off)) incl += v;
     }
-    if ((t & 63) == 63) wave_sum[t >> 6] = incl;
+    // (largest and smallest score word of what the thread holds, for the usual case)
+    uint32_t hi_max = 0u, hi_min_inv = 0u;
+#pragma unroll
+    for (uint32_t e = 0; e < kShort; ++e) {
+        if (e < mine) {
+            hi_max = max(hi_max, uint32_t(head[e] >> 32));
+            hi_min_inv = max(hi_min_inv, ~uint32_t(head[e] >> 32));
+        }
+    }
+    hi_max = wave_umax(hi_max);
+    hi_min_inv = wave_umax(hi_min_inv);
+    if (lane == 63u) { w_sum[wv] = incl; w_max[wv] = hi_max; w_min[wv] = hi_min_inv; }
     __syncthreads();
     uint32_t base = incl - mine, total = 0;
-    for (int w = 0; w < kFinalThreads / 64; ++w) { if (w < (t >> 6)) base += wave_sum[w]; total += wave_sum[w]; }
+    for (uint32_t w = 0; w < W; ++w) { if (w < wv) base += w_sum[w]; total += w_sum[w]; }
     const bool too_many = total > uint32_t(kFinalCap);
     // A sampling level whose candidates did not all fit yields its floor from the subset that was
     // kept: a valid floor, but possibly far below the k_floor-th best of the level.  The flag lets
@@ -1365,180 +1340,138 @@ __global__ __launch_bounds__(kFinalThreads) void k_final(const uint64_t *__restr
         if (t == 0 && !keep_floor) *tau_slot = kTauInit;
         return;
     }
-    const uint32_t c_all = min(total, uint32_t(kFinalCap));
-    const uint32_t need = (sampling || raising) ? min(uint32_t(k_floor), c_all) : uint32_t(k_eff);   // leading keys wanted, in order
-    // Few keys wanted and every thread already holds its whole segment in registers (the usual
-    // single-query case: some thousand candidates, a few per workgroup of the scan): no gather, no
-    // sort.  Every wave picks its `need` largest by rounds of wave-wide maxima, the 16 x 32 picks
-    // meet in LDS, and the first wave picks the `need` largest of those the same way.
-    const bool in_registers = one_each && any_long == 0u && need <= 32u;
-    if (in_registers) {
-        const uint32_t lane = uint32_t(t) & 63u, wv = uint32_t(t) >> 6;
+    const uint32_t need = (sampling || raising) ? min(uint32_t(k_floor), total) : uint32_t(k_eff);   // leading keys wanted
+    const bool held = one_each && any_long == 0u;              // every key sits in a register
+    const bool staged = !held && total <= kFinalStage;
+    if (staged) {
+        // A thread copies a short segment itself; long ones (the first sampling level fills a few
+        // segments to the brim) go on a list the waves then share, a key per lane.
+        uint32_t pos = base;
+        for (uint32_t sg = s0; sg < s1; ++sg) {
+            const uint32_t c = one_each ? mine : min(cnt[sg], uint32_t(kSegCap));
+            if (c <= kShort) {
+                const uint64_t *src = segs + size_t(sg) * kSegCap;
+                uint64_t v[kShort];
 #pragma unroll
-        for (uint32_t e = 0; e < kShort; ++e) if (e >= mine) head[e] = 0ull;
-        uint64_t pick;
-        if (any_over8 == 0u) {          // the usual case: eight keys per thread at most
-            uint64_t r8[8];
+                for (uint32_t e = 0; e < kShort; ++e) v[e] = one_each ? head[e] : (e < c ? src[e] : 0ull);
 #pragma unroll
-            for (uint32_t e = 0; e < 8; ++e) r8[e] = head[e];
-            sort8_desc(r8);
-            pick = wave_top(r8, need, lane);
-        } else {
-            sort16_desc(head);
-            pick = wave_top(head, need, lane);
-        }
-        if (lane < 32u) keys[wv * 32u + lane] = pick;
-        __syncthreads();
-        if (wv == 0) {
-            uint64_t r[8];
-#pragma unroll
-            for (uint32_t e = 0; e < 8; ++e) r[e] = keys[lane * 8u + e];
-            sort8_desc(r);
-            const uint64_t best = wave_top(r, need, lane);
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (lane < 32u) keys[lane] = best;
+                for (uint32_t e = 0; e < kShort; ++e)
+                    if (e < c) stage[pos + e] = v[e];
+            } else {
+                const uint32_t i = atomicAdd(&long_n, 1u);
+                long_seg[i] = sg;
+                long_pos[i] = pos;
+                long_cnt[i] = c;
+            }
+            pos += c;
         }
         __syncthreads();
-    } else {
-    // gather (a sampling level may keep any subset: dropping what does not fit only loosens the floor).
-    // A thread copies a short segment itself, its loads in flight together; long ones (the first
-    // sampling level fills a few segments to the brim) go on a list the waves then share, four
-    // segments per wave and turn, a key per lane.
-    uint32_t pos = base;
-    for (uint32_t sg = s0; sg < s1; ++sg) {
-        const uint32_t c = one_each ? mine : min(cnt[sg], uint32_t(kSegCap));
-        const uint64_t *src = cand + (size_t(qn) * seg_stride + sg) * kSegCap;
-        if (c <= kShort) {
-            uint64_t v[kShort];
-#pragma unroll
-            for (uint32_t e = 0; e < kShort; ++e) v[e] = one_each ? head[e] : (e < c ? src[e] : 0ull);
+        for (uint32_t i = wv; i < long_n; i += W)
+            if (lane < long_cnt[i]) stage[long_pos[i] + lane] = segs[size_t(long_seg[i]) * kSegCap + lane];
+        __syncthreads();
+    }
+    // every candidate once, wherever it is
+    auto each = [&](auto &&f) {
+        if (held) {
 #pragma unroll
             for (uint32_t e = 0; e < kShort; ++e)
-                if (e < c && pos + e < uint32_t(kFinalCap)) keys[pos + e] = v[e];
+                if (e < mine) f(head[e]);
+        } else if (staged) {
+            for (uint32_t i = t; i < total; i += T) f(stage[i]);
         } else {
-            const uint32_t slot = atomicAdd(&long_n, 1u);
-            if (slot < uint32_t(kFinalLong)) {
-                long_seg[slot] = sg;
-                long_pos[slot] = pos;
-                long_cnt[slot] = c;
-            } else {                      // more long segments than the list holds: copy in place
-                for (uint32_t e = 0; e < c; ++e)
-                    if (pos + e < uint32_t(kFinalCap)) keys[pos + e] = src[e];
+            for (uint32_t sg = s0; sg < s1; ++sg) {
+                const uint32_t c = min(cnt[sg], uint32_t(kSegCap));
+                const uint64_t *src = segs + size_t(sg) * kSegCap;
+                for (uint32_t e = 0; e < c; ++e) f(src[e]);
             }
         }
-        pos += c;
-    }
-    __syncthreads();
-    const uint32_t n_long = min(long_n, uint32_t(kFinalLong));
-    constexpr uint32_t kWavesF = kFinalThreads / 64;
-    for (uint32_t i0 = uint32_t(t >> 6); i0 < n_long; i0 += kWavesF * 4) {   // four segments' loads in flight per wave
-        uint64_t v[4];
-        uint32_t at[4];
-        bool ok[4];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const uint32_t i = i0 + u * kWavesF;
-            ok[u] = false;
-            at[u] = 0;
-            v[u] = 0ull;
-            if (i < n_long) {
-                at[u] = long_pos[i] + uint32_t(t & 63);
-                ok[u] = uint32_t(t & 63) < long_cnt[i] && at[u] < uint32_t(kFinalCap);
-                if (ok[u]) v[u] = cand[(size_t(qn) * seg_stride + long_seg[i]) * kSegCap + (t & 63)];
-            }
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u)
-            if (ok[u]) keys[at[u]] = v[u];
-    }
-    // leading keys kept in order by the per-wave sorts and merges below (a power of two >= need), or 0: full sort
-    const uint32_t keep = need <= 64u ? 64u : need <= 128u ? 128u : need <= 256u ? 256u : 0u;
-    uint32_t sort_n = keep ? keep : 2u;
-    while (sort_n < c_all) sort_n <<= 1;
-    __syncthreads();
-    for (uint32_t i = c_all + t; i < sort_n; i += kFinalThreads) keys[i] = 0ull;
-    __syncthreads();
-    if (keep != 0u) {
-        // Few keys wanted: every wave sorts a chunk of its own, no barrier inside (LDS serves a
-        // wave's requests in order), and a tree of merges -- the `keep` larger of two sorted runs
-        // of `keep` form a bitonic run, log2(keep) strides sort it -- leaves the `keep` best of all
-        // in front.
-        const uint32_t lane = uint32_t(t) & 63u, wv = uint32_t(t) >> 6;
-        const uint32_t len = max(keep, sort_n / (kFinalThreads / 64));
-        const uint32_t n_chunks = sort_n / len;
-        auto wave_sync = []() {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        };
-        auto swap_down = [&](uint32_t lo, uint32_t hi) {   // larger key to the lower index
-            const uint64_t x = keys[lo], y = keys[hi];
-            if (x < y) { keys[lo] = y; keys[hi] = x; }
-        };
-        if (wv < n_chunks) {
-            const uint32_t at = wv * len;
-            for (uint32_t size = 2; size <= len; size <<= 1) {
-                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                    for (uint32_t i = lane; i < len / 2; i += 64) {
-                        const uint32_t lo = 2 * i - (i & (stride - 1));
-                        const uint32_t hi = lo + stride;
-                        if ((lo & size) == 0) swap_down(at + lo, at + hi);
-                        else swap_down(at + hi, at + lo);
-                    }
-                    wave_sync();
-                }
-            }
-        }
-        for (uint32_t step = 1; step < n_chunks; step <<= 1) {
+    };
+    uint64_t threshold = 0ull;
+    if (total > 256u) {
+        if (!held) {
+            hi_max = 0u;
+            hi_min_inv = 0u;
+            each([&](uint64_t k) {
+                hi_max = max(hi_max, uint32_t(k >> 32));
+                hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+            });
+            hi_max = wave_umax(hi_max);
+            hi_min_inv = wave_umax(hi_min_inv);
+            if (lane == 63u) { w_max[wv] = hi_max; w_min[wv] = hi_min_inv; }
             __syncthreads();
-            if (wv % (2 * step) == 0 && wv + step < n_chunks) {
-                const uint32_t at = wv * len, other = (wv + step) * len;
-                for (uint32_t i = lane; i < keep; i += 64) {
-                    const uint64_t x = keys[at + i], y = keys[other + keep - 1u - i];
-                    if (x < y) keys[at + i] = y;
-                }
-                wave_sync();
-                for (uint32_t stride = keep / 2; stride > 0; stride >>= 1) {
-                    for (uint32_t i = lane; i < keep / 2; i += 64) {
-                        const uint32_t lo = 2 * i - (i & (stride - 1));
-                        swap_down(at + lo, at + lo + stride);
-                    }
-                    wave_sync();
-                }
+        }
+        uint32_t mx = 0u, mn_inv = 0u;
+        for (uint32_t w = 0; w < W; ++w) { mx = max(mx, w_max[w]); mn_inv = max(mn_inv, w_min[w]); }
+        // keys lie in [low, low + 2^width): 1024 bins of 2^shift; `above` of them were counted beyond that range
+        // before, and `rest` are still wanted from it
+        uint64_t low = uint64_t(~mn_inv) << 32;
+        uint32_t width = 32u + (mx == ~mn_inv ? 0u : 32u - uint32_t(__clz(int(mx - ~mn_inv))));
+        uint32_t above = 0u, rest = need;
+        for (;;) {
+            const uint32_t shift = width > 10u ? width - 10u : 0u;
+            each([&](uint64_t k) {
+                const uint64_t d = k - low;
+                if (k >= low && (width >= 64u || (d >> width) == 0ull)) atomicAdd(&bins[uint32_t(d >> shift)], 1u);
+            });
+            __syncthreads();
+            // from the top: the bin in which the count passes `rest`
+            uint32_t own[kPerBin], sum = 0u;
+#pragma unroll
+            for (uint32_t i = 0; i < kPerBin; ++i) { own[i] = bins[kFinalBins - 1u - (t * kPerBin + i)]; sum += own[i]; }
+            uint32_t run = sum;
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t v = __shfl_up(run, off);
+                if (lane >= uint32_t(off)) run += v;
             }
-        }
-        __syncthreads();
-    } else {
-        for (uint32_t size = 2; size <= sort_n; size <<= 1) {
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                for (uint32_t i = t; i < sort_n / 2; i += kFinalThreads) {
-                    const uint32_t lo = 2 * i - (i & (stride - 1));
-                    const uint32_t hi = lo + stride;
-                    const bool desc = (lo & size) == 0;
-                    const uint64_t x = keys[lo], y = keys[hi];
-                    if ((x < y) == desc) { keys[lo] = y; keys[hi] = x; }
+            if (lane == 63u) w_sum[wv] = run;
+            __syncthreads();
+            uint32_t before = run - sum;
+            for (uint32_t w = 0; w < W; ++w) if (w < wv) before += w_sum[w];
+#pragma unroll
+            for (uint32_t i = 0; i < kPerBin; ++i) {
+                if (before < rest && before + own[i] >= rest) {
+                    s_bin = kFinalBins - 1u - (t * kPerBin + i);
+                    s_above = before;
+                    s_at = before + own[i];
                 }
-                __syncthreads();
+                before += own[i];
+                bins[kFinalBins - 1u - (t * kPerBin + i)] = 0u;
             }
+            __syncthreads();
+            low += uint64_t(s_bin) << shift;
+            if (above + s_at <= kFinalKept) break;             // (a bin of width one holds one key: this ends)
+            above += s_above;
+            rest -= s_above;
+            width = shift;
+            __syncthreads();                                   // s_* are read by all before they are written again
         }
+        threshold = low;
     }
-    }   // gather and sort through LDS
-    if (sampling || raising) {
-        if (t == 0) {
-            // the floor: the k_floor-th best sampled score (k_floor >= k_eff steadies the estimate)
-            const uint32_t pick = min(uint32_t(k_floor), c_all) - 1;
-            float s; uint32_t idx;
-            sort_unkey(keys[pick], s, idx);
-            *(sampling ? tau_slot : raise_out + qn) = order_key(s == 0.0f ? -0.0f : s);
-        }
-        return;
-    }
+    each([&](uint64_t k) {
+        if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
+    });
+    __syncthreads();
+    const uint32_t n = n_kept;
+    if (t < 2u) kept[n + t] = 0ull;                             // (ranked in pairs)
+    __syncthreads();
     const size_t row = row_map ? size_t(row_map[qn]) : size_t(qn);   // a repeated pass writes to the rows of the queries it repeats
-    for (int jj = t; jj < k_eff; jj += kFinalThreads) {
+    for (uint32_t i = t; i < n; i += T) {
+        const uint64_t k = kept[i];
+        uint32_t rank = 0u;
+        for (uint32_t j = 0; j < n; j += 2u) {
+            const ulonglong2 o = *reinterpret_cast<const ulonglong2 *>(&kept[j]);
+            rank += (o.x > k ? 1u : 0u) + (o.y > k ? 1u : 0u);
+        }
+        if (rank >= need) continue;
         float s; uint32_t idx;
-        sort_unkey(keys[jj], s, idx);
-        out_scores[row * k_eff + jj] = s;
-        out_idx[row * k_eff + jj] = int64_t(idx);
+        sort_unkey(k, s, idx);
+        if (sampling || raising) {
+            // the floor: the k_floor-th best sampled score (k_floor >= k_eff steadies the estimate)
+            if (rank == need - 1u) *(sampling ? tau_slot : raise_out + qn) = order_key(s == 0.0f ? -0.0f : s);
+        } else {
+            out_scores[row * k_eff + rank] = s;
+            out_idx[row * k_eff + rank] = int64_t(idx);
+        }
     }
 }
 
@@ -1899,9 +1832,13 @@ hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
                         uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, hipStream_t s) {
     if (nq == 0 || k_eff == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_final, dim3(nq), dim3(kFinalThreads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor,
-                       out_scores, out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over,
-                       clear_flag, run_if);
+    auto launch = [&](auto kernel, unsigned threads) {
+        hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
+                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if);
+    };
+    if (n_seg <= 256) launch(k_final<256>, 256);
+    else if (n_seg <= 512) launch(k_final<512>, 512);
+    else launch(k_final<1024>, 1024);
     return hipGetLastError();
 }
 
