@@ -1,0 +1,66 @@
+"""Searches of small indexes, which score every block and go without sampling: against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def T():
+    from turbovec_amd import _lib
+    _lib.lib()
+    return _lib
+
+
+# One and several tiles of queries, rows of 1 to 72 chunks (odd counts too), indexes of less than a block to
+# several rounds of the grid; 768 and 1536 dimensions with 140 queries: the all-queries kernel from 513 blocks on.
+@pytest.mark.parametrize("dim,n,nq", [
+    (64, 1, 3), (64, 31, 1), (128, 33, 70), (8, 500, 1), (136, 5_001, 9), (200, 20_011, 40), (64, 60_003, 1), (128, 49_000, 300),
+    (448, 9_001, 33), (576, 16_500, 257), (768, 17_000, 140), (768, 700, 1025), (1536, 17_001, 129), (1536, 2_001, 65),
+    (1536, 40_000, 2), (3072, 1_201, 97), (4608, 333, 2), (4608, 1_003, 130)])
+def test_unsampled_search_matches_oracle(T, oracle, dim, n, nq):
+    oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=dim + n))
+    q = unit_gaussian(nq, dim, seed=78)
+    ix = to_native(T, oidx)
+    rng = np.random.default_rng(5)
+    redos = 0       # (k = 100 on long rows is sampled, and may repeat queries)
+    for m in (None, rng.random(n) < 0.5, rng.random(n) < 0.01, (np.arange(n) >= n // 3) & (np.arange(n) < n // 3 + 40)):
+        if m is not None and not m.any():
+            m[0] = True
+        words = None if m is None else T.pack_mask(m)[0]
+        for k in (1, 10, 100):
+            s, i = ix.search(q, k, mask_words=words)
+            os_, oi = oidx.search(q, k, mask_words=words)
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
+            assert k == 100 or ix.overflow_redos() == redos
+        redos = ix.overflow_redos()
+    ix.close()
+
+
+@pytest.mark.parametrize("dim,nq", [(128, 1), (128, 300), (768, 140)])
+def test_ties_and_wild_row_scales(T, oracle, dim, nq):
+    """Equal rows: every block and every row of the chosen blocks ties, the lowest slots come back.  Row scales of
+    zero, of either sign and far from the encoder's: the same answer as the exact path's."""
+    n = 30_000
+    oidx = OracleIndex(oracle, dim, 4, np.tile(unit_gaussian(1, dim, seed=3), (n, 1)))
+    q = unit_gaussian(nq, dim, seed=4)
+    ix = to_native(T, oidx)
+    for k in (10, 40):
+        s, i = ix.search(q, k)
+        os_, oi = oidx.search(q, k)
+        assert np.array_equal(i, np.tile(np.arange(k), (nq, 1)))
+        assert np.array_equal(i, oi) and bits_equal(s, os_)
+    ix.close()
+    oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=5))
+    rng = np.random.default_rng(6)
+    oidx.scales = (oidx.scales * rng.choice(np.array([0.0, 1e-38, -1.0, 1.0, 1e6], np.float32), size=n)).astype(np.float32)
+    ix = to_native(T, oidx)
+    for k in (10, 40):
+        s, i = ix.search(q, k)
+        ix.set_path(1)
+        s2, i2 = ix.search(q, k)
+        ix.set_path(0)
+        assert np.array_equal(i, i2) and bits_equal(s, s2)
+    ix.close()

@@ -224,7 +224,7 @@ struct Prepared {
 // in permute-dot mode does not need them and prepares its queries in a single launch.
 // `for_append`: u8-LUT tables are wanted in the order of the batch's append scan too.
 int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepared &out, bool split = true,
-                    bool keep_rotated = false, bool for_append = false) {
+                    bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr) {
     const tv::Geometry &g = ix->geo;
     const size_t nq_pad = round_up(nq, tv::kQTile);
     const int mode = effective_mode(ix);
@@ -237,7 +237,7 @@ int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepar
         out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
         TV_HIP(tv::launch_prep_p(d_q, ix->d_signs, ix->d_perms, g.dim, ix->rot.block, ix->rot.inv_sqrt_block,
                                  cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr, out.d_tables, out.d_qscale,
-                                 out.d_qbias, g.G, g.nch, ix->cs, nq, nq_pad, split, ix->stream));
+                                 out.d_qbias, g.G, g.nch, ix->cs, nq, nq_pad, split, stamp, ix->stream));
         return TV_OK;
     }
     float *d_rot = ar.take<float>(nq * g.dim);
@@ -602,6 +602,116 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
 // aligned).
 uint32_t repeat_offset(uint32_t step) { return step >= 4 ? (step / 2) & ~1u : 0u; }
 
+// ---- small indexes: no sampling (tv_kernels6.hip) ----
+constexpr size_t kDirectBlocks = 16384;      // what k_pick holds in registers
+constexpr size_t kDirectWideBlocks = 8192;
+
+// Which scan the search of nq queries without sampling takes: the all-queries kernel keeps a decoded block
+// for all of them, from where its grid of eight waves per CU has blocks to hold (157 blocks of 1536
+// dimensions, 1000 queries: 126 us a search against 103; 938: 149 against 179).
+bool direct_wide(const tv_index *ix, size_t nq, size_t n_blocks) {
+    const int nch = ix->geo.nch;
+    return tv::wide_min_queries(nch) > 0 && nq >= size_t(tv::wide_min_queries(nch)) && tv::wide_serves_best_of_block(nch) && n_blocks > 512;
+}
+size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
+    return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) + 65536;
+}
+// Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, sampled and
+// without: 100K x 128, 1 query 50 and 28, 1000 queries 498 and 67; 260K x 768, 32 queries 77 and 54;
+// 100K x 1536, 1000 queries 310 and 243.
+//  - It scores k blocks a second time in one workgroup: k = 100 at 768 dimensions (12 chunks) costs one
+//    query 77 us against 64, at 128 dimensions 39 against 53.
+//  - One tile of queries: level with sampling at 16384 blocks (500K x 3072: 204 and 202; x 1536: 118 and
+//    126), behind it at twice that (1M x 1536: 205 and 184).
+//  - More tiles on k_scan_p4_best, which decodes a block once per tile group: won up to a number of (block,
+//    tile, chunk) triples that depends on the kernel it replaces -- short rows against the all-queries kernel
+//    (260K x 768, 1000 queries, 3.1e6 triples: 373 and 365; x 128: 129 and 664), rows whose tiles stay in
+//    LDS (100K x 1536, 100 queries, 3e5: 100 and 99; 500K x 768, 8e5: 112 and 148), rows whose tiles are
+//    streamed (260K x 3072, 100 queries, 1.6e6: 294 and 543; 500K, 3e6: 489 and 437).
+//  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about a
+//    million rows (1M x 1536, 1000 queries: 1573 and 1489; 260K: 466 and 513).
+// Batches of 2 to 8, of 33 to 255 and of more than 1024 queries on short rows keep to the sampled path beyond
+// 1535 blocks although this one would be faster there too: those are the calls whose overflow, repeated and
+// exact passes are held to the oracle by test.
+bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+    const int nch = ix->geo.nch;
+    if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide) return false;
+    if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > kDirectBlocks) return false;
+    if (tv::pick_lds_bytes(true, nch, k_eff) > tv::kPickLds) return false;
+    const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
+    if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
+    if (n_blocks >= 1536 && nch <= 12 && ((nq >= 2 && nq <= 8) || (nq > 32 && nq < 256) || nq > kChunkQueries)) return false;
+    if (direct_wide(ix, cq, n_blocks)) return n_blocks <= kDirectWideBlocks;
+    if (tiles == 1) return nch <= 24 || n_blocks <= kDirectBlocks / 2;
+    if (nch < 12) return triples <= 2500000;
+    return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 14 ? 800000 : 250000) || n_blocks <= 512;
+}
+// The milliseconds between the two stamps.
+int take_stamps(tv_index *ix, int launches) {
+    int khz = 0;
+    TV_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ix->device));
+    if (khz > 0) ix->last_scan_ms += float(double(ix->h_stamps[1] - ix->h_stamps[0]) / khz);
+    ix->last_scan_launches += launches;
+    return TV_OK;
+}
+int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
+                  int64_t *d_out_idx, bool timing) {
+    const tv::Geometry &g = ix->geo;
+    const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
+    int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
+    if (rc != TV_OK) return rc;
+    ix->last_queries_per_launch = int(chunk_len(ix, nq));
+    for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
+        const size_t gq = std::min(kGroupQueries, nq - g0);
+        for (size_t c0 = 0, cq; c0 < gq; c0 += cq) {
+            cq = chunk_len(ix, gq - c0);
+            const size_t q0 = g0 + c0;
+            const bool timed = timing && q0 == 0, wide = direct_wide(ix, cq, n_blocks), split = wide && tv::wide_weights_split(g.nch);
+            Arena ar;
+            ar.base = static_cast<uint8_t *>(ix->ws);
+            Prepared pq;
+            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, false, timed ? ix->d_stamps : nullptr);
+            if (rc != TV_OK) return rc;
+            tv::ScanArgs a;
+            fill_scan_args(ix, a);
+            a.mask = d_mask;
+            a.tables = pq.d_tables;
+            a.qscale = pq.d_qscale;
+            a.qbias = pq.d_qbias;
+            a.nq_tile = int(cq);
+            a.best_out = ar.take<uint32_t>(cq * stride);
+            a.best_stride = uint32_t(stride);
+            if (wide) {
+                a.gtau = ix->d_tau_open;
+                a.best_of_block = 1;
+                if (d_mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * stride, ix->stream));   // (it skips blocks without an allowed row)
+                TV_HIP(tv::launch_scan_p4_wide(a, tv::wide_grid_blocks(ix->device), ix->stream));
+            } else {
+                TV_HIP(tv::launch_scan_p4_best(a, ix->device, ix->stream));
+            }
+            TV_HIP(tv::launch_pick(a, true, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
+                                   timed ? ix->d_stamps + 1 : nullptr, ix->stream));
+        }
+        TV_HIP(hipStreamSynchronize(ix->stream));
+        if (timing && g0 == 0) {
+            rc = take_stamps(ix, 1);
+            if (rc != TV_OK) return rc;
+        }
+        // (fewer rows than wanted had a score: a mask of fewer rows than the caller's count promised)
+        std::vector<uint32_t> exact_rows;
+        for (size_t q = 0; q < gq; ++q)
+            if (ix->h_flags[q] != 0u) exact_rows.push_back(uint32_t(q));
+        ix->overflow_redos += exact_rows.size();
+        ix->exact_redos += exact_rows.size();
+        for (const uint32_t row : exact_rows) {
+            const size_t q = g0 + row;
+            rc = search_robust(ix, d_queries + q * g.dim, 1, k_eff, d_mask, d_out_scores + q * k_eff, d_out_idx + q * k_eff, false);
+            if (rc != TV_OK) return rc;
+        }
+    }
+    return TV_OK;
+}
+
 // The seam: search::search over device-resident inputs and outputs.
 //
 // Sample-then-filter.  Scans run in append mode: every allowed slot whose score
@@ -632,6 +742,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         return search_robust(ix, d_queries, nq, k_eff, d_mask, d_out_scores, d_out_idx, timing);
 
     const size_t n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (direct_serves(ix, nq, k_eff, n_blocks)) return search_direct(ix, d_queries, nq, k_eff, d_mask, d_out_scores, d_out_idx, timing);
     // sampling levels take the k_floor-th best as the floor: a deeper order statistic is steadier
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     if (ix->row_ladder_left > 0) --ix->row_ladder_left;
@@ -659,6 +770,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         chunk_at[n_chunks] = gq;
         uint32_t *d_level_flags_all = head.take<uint32_t>(kLevelFlagWords);
         size_t n_timed = 0;
+        bool stamped = false;      // the full scan lies between two stamps (there is a level before it), not between events
 
         // One pass over `pq_n` queries of the chunk at q0: the ladder from open floors, or, for the
         // packed batch of queries to repeat (rows d_rows[row0 ..]), the ladder again from the floors
@@ -748,7 +860,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                         a.cand = d_cand + t * tile_q * seg_stride * tv::kSegCap;
                         a.cand_cnt = d_cnt + t * tile_q * seg_stride;
                         a.seg_stride = uint32_t(seg_stride);
-                        const bool timed = timed_pass && last && int(launch_no) < kMaxTimedTiles;
+                        const bool timed = timed_pass && last && steps.size() == 1 && int(launch_no) < kMaxTimedTiles;
                         if (timed) TV_HIP(hipEventRecord(ix->ev_start[launch_no], ix->stream));
                         if (wide) {
                             n_seg = grid;
@@ -775,6 +887,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                         }
                         if (timed) TV_HIP(hipEventRecord(ix->ev_stop[launch_no], ix->stream));
                     }
+                    if (last && timed_pass) stamped = steps.size() > 1;
                     if (last && timed_pass) n_timed = std::min<size_t>(launch_no, size_t(kMaxTimedTiles));
                     // the first final pass may hand raised floors to a repeated one; the repeated pass
                     // sends what still does not fit to the exact path
@@ -782,7 +895,8 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                                             int(pq_n), d_os, d_oi, d_over, last ? nullptr : d_tau, int(tile_q),
                                             (lv > 0 || repeat) ? 1 : 0, (last && !repeat) ? d_raise + (q0 - g0) : nullptr,
                                             repeat ? d_rows + row0 : nullptr, lv_flag, attempt == 0 ? next_flag : nullptr,
-                                            run_if, ix->stream));
+                                            run_if, !timed_pass ? nullptr : last ? ix->d_stamps + 1 : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
+                                            ix->stream));
                 }
             }
             if (repeat) TV_HIP(hipMemcpyAsync(h_over, d_over, pq_n * sizeof(uint32_t), hipMemcpyDeviceToHost, ix->stream));
@@ -806,7 +920,11 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
             }
         }
-        for (size_t t = 0; t < n_timed; ++t) {
+        if (stamped) {
+            rc = take_stamps(ix, int(n_timed));
+            if (rc != TV_OK) return rc;
+        }
+        for (size_t t = 0; t < n_timed && !stamped; ++t) {
             float ms = 0.0f;
             TV_HIP(hipEventElapsedTime(&ms, ix->ev_start[t], ix->ev_stop[t]));
             ix->last_scan_ms += ms;
@@ -1136,7 +1254,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
             rc = TV_ERR_HIP;
             break;
         }
-        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) {
+        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t) + 2 * sizeof(uint64_t), hipHostMallocMapped) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
         }
@@ -1144,6 +1262,9 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
             rc = TV_ERR_HIP;
             break;
         }
+        static_assert((kGroupQueries + kLevelFlagWords) % 2 == 0, "the stamps behind the flags are 8-byte words");
+        ix->h_stamps = reinterpret_cast<uint64_t *>(ix->h_flags + kGroupQueries + kLevelFlagWords);
+        ix->d_stamps = reinterpret_cast<uint64_t *>(ix->d_flags_host + kGroupQueries + kLevelFlagWords);
         rc = scratch_address(device, &ix->scratch);
         if (rc != TV_OK) break;
         // floors of a search's first sampling level: the order key of -inf for every query, written once

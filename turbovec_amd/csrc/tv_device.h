@@ -83,6 +83,10 @@ __device__ __forceinline__ void sort_unkey(uint64_t key, float &s, uint32_t &idx
     idx = 0x7fffffffu - (lo >> 1);
 }
 
+// The high word of sort_key for a block's best score; 0 where the block has no allowed row.
+__device__ __forceinline__ uint32_t best_word(float s) {
+    return s == -__int_as_float(0x7f800000) ? 0u : uint32_t(order_key(s + 0.0f)) ^ 0x80000000u;   // (-0 counts as +0)
+}
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));

@@ -70,6 +70,8 @@ struct ScanArgs {
     uint32_t seg_stride;       // segments allocated per query (>= grid of the launch)
     uint32_t vgrid;            // single-tile permute-dot scan: four-wave groups of the launch (set by its launcher)
     int best_of_block;         // all-queries-per-pass kernel: no floor, per scanned block and query the best allowed slot (kModeBest)
+    uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and block the best allowed row's (tv_kernels6.hip)
+    uint32_t best_stride;
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
 
@@ -99,15 +101,19 @@ hipError_t launch_calibrate(const float *d_qrot, float *d_qcal, float *d_bias_co
 hipError_t launch_build_p(const float *d_qcal, const float *d_bias_corr, uint8_t *d_wfrag, float *d_qscale,
                           float *d_qbias, int dim, int G, int nch, float cs, size_t nq, size_t nq_padded,
                           bool split, hipStream_t s);
+// `stamp` here and below, when given: a word that takes the device clock as the launch ends (of the
+// preparation and of a sampling level's selection) or starts (of a last selection): the scan between two
+// of them is timed without events, whose packets the launches behind them wait for, 5 to 6 us each.
 // Rotation, TQ+ inverse (d_shift / d_scale null: none) and permute-dot weights in one launch.
 hipError_t launch_prep_p(const float *d_q, const float *d_signs, const uint32_t *d_perms, int dim, int block,
                          float inv_sqrt_block, const float *d_shift, const float *d_scale, uint8_t *d_wfrag,
                          float *d_qscale, float *d_qbias, int G, int nch, float cs, size_t nq, size_t nq_padded, bool split,
-                         hipStream_t s);
+                         uint64_t *stamp, hipStream_t s);
 hipError_t launch_build_lut(const float *d_qcal, const float *d_bias_corr, const float *d_centroids, uint8_t *d_lut,
                             float *d_qscale, float *d_qbias, int dim, int bits, int G, int nch, size_t nq,
                             size_t nq_padded, hipStream_t s);
 
+int device_cus(int device);   // compute units
 int scan_grid_blocks(int device, int mode_p, int nch, int k, int lut_queries);
 size_t scan_lds_bytes(int mode_p, int nch, int k, int lut_queries);
 // Queries one launch of the LUT scan serves (1, 2 or 4), from the LDS budget.
@@ -136,6 +142,14 @@ int mx_segments();
 int mx_round_blocks(int device, size_t nq);   // blocks a launch over nq queries works through per round
 hipError_t launch_scan_lut_mx(const ScanArgs &a, const MxShape &m, int bits, hipStream_t s);
 hipError_t launch_scan_p4(const ScanArgs &a, int grid, int mode, hipStream_t s);
+// Small indexes without sampling (tv_kernels6.hip): the best row of every block, then the best blocks' rows.
+constexpr int kMaxPickK = 128;             // most results k_pick ranks
+constexpr size_t kPickLds = 128 * 1024;    // beside its 17 KiB of fixed buffers
+bool best_serves(int nch);
+hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s);
+size_t pick_lds_bytes(bool mode_p, int nch, size_t k_eff);
+hipError_t launch_pick(const ScanArgs &a, bool mode_p, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow,
+                       uint64_t *stamp, hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).
 int batched_tiles(int nch);
@@ -169,7 +183,7 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, hipStream_t s);
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp, hipStream_t s);
 // Packs the queries rows[0..n_redo) of a chunk and their raised floors for one more full scan.
 hipError_t launch_gather_redo(const float *d_q, const uint32_t *d_rows, const int *d_raised, int dim, int tile_q,
                               size_t n_redo, float *d_q_out, int *d_tau_out, hipStream_t s);
@@ -231,6 +245,7 @@ struct tv_index {
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
     uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags
+    uint64_t *h_stamps = nullptr, *d_stamps = nullptr;   // in the same allocation: the device clock before and after a full scan
     size_t exact_redos = 0;        // queries that went on to the exact path
     float last_scan_ms = 0.0f;
     int last_scan_launches = 0;

@@ -3,8 +3,9 @@
 // Compiled with -ffp-contract=off: every float expression keeps the separate
 // multiplies and adds the reference performs, and fmaf appears only where the
 // reference fuses.
-#include "tv_internal.h"
 #include "tv_device.h"
+#include "tv_internal.h"
+#include "tv_select.h"
 
 #include <cfloat>
 #include <climits>
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(256) void k_prep_p(const float *__restrict__ q, con
                                                 float inv_sqrt_block, const float *__restrict__ shift,
                                                 const float *__restrict__ scale, uint8_t *__restrict__ wfrag,
                                                 float *__restrict__ qscale, float *__restrict__ qbias, int G, int nch,
-                                                float cs, size_t nq, bool split) {
+                                                float cs, size_t nq, bool split, uint64_t *stamp) {
     extern __shared__ float rot_lds[];
     __shared__ float red[4];
     __shared__ float s_bias;
@@ -332,6 +333,7 @@ __global__ __launch_bounds__(256) void k_prep_p(const float *__restrict__ q, con
     if (t == 0) {
         qscale[qi] = cs * qs;
         qbias[qi] = 0.0f + (scale != nullptr ? s_bias : 0.0f);
+        if (stamp != nullptr && qi == 0) *stamp = wall_clock64();
     }
 }
 
@@ -1234,11 +1236,9 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 // 1024 threads per query) and now: one query, k = 10, 12 -> 6 to 10 us; k = 100,
 // 60 and 33 -> 22 and 17 us; 1000 queries, k = 10, 61 to 75 -> 12 to 18 us.
 // ===========================================================================
-constexpr uint32_t kFinalBins = 1024;
-constexpr uint32_t kFinalKept = 1024;      // keys ranked at the end: more than are ever wanted (kMaxSampledK)
 constexpr uint32_t kFinalStage = 2048;     // candidates copied to LDS when some segment is long
 constexpr uint32_t kFinalLong = 128;       // ... of which this many segments can be
-static_assert(kFinalKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
+static_assert(kSelectKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
 
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
@@ -1248,13 +1248,12 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                uint32_t *__restrict__ overflow, int *__restrict__ tau_out,
                                                int tau_stride_q, int keep_floor, int *__restrict__ raise_out,
                                                const uint32_t *__restrict__ row_map, uint32_t *level_over,
-                                               uint32_t *clear_flag, const uint32_t *run_if) {
-    constexpr uint32_t W = T / 64, kPerBin = kFinalBins / T;
-    __shared__ __align__(16) uint64_t kept[kFinalKept + 2];
+                                               uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp) {
+    constexpr uint32_t W = T / 64;
+    __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ uint64_t stage[kFinalStage];
-    __shared__ uint32_t bins[kFinalBins];
-    __shared__ uint32_t w_sum[W], w_max[W], w_min[W];
-    __shared__ uint32_t any_full, any_long, long_n, n_kept, s_bin, s_at, s_above;
+    __shared__ SelectShared sh;
+    __shared__ uint32_t any_full, any_long, long_n, n_kept;
     __shared__ uint32_t long_seg[kFinalLong], long_pos[kFinalLong], long_cnt[kFinalLong];
     if (launch_switched_off(run_if)) return;
     const int qn = blockIdx.x;
@@ -1262,8 +1261,9 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     const bool sampling = tau_out != nullptr;
     int *tau_slot = sampling ? tau_out + (qn / tau_stride_q) * kQTile + qn % tau_stride_q : nullptr;
     if (clear_flag != nullptr && qn == 0 && t == 0) *clear_flag = 0u;
+    if (stamp != nullptr && !sampling && qn == 0 && t == 0) *stamp = wall_clock64();
     if (t == 0) { any_full = 0u; any_long = 0u; long_n = 0u; n_kept = 0u; }
-    for (uint32_t i = t; i < kFinalBins; i += T) bins[i] = 0u;
+    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     __syncthreads();
     // every thread owns a contiguous run of this query's segments
     const uint32_t per = (n_seg + T - 1) / T;
@@ -1312,10 +1312,10 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     }
     hi_max = wave_umax(hi_max);
     hi_min_inv = wave_umax(hi_min_inv);
-    if (lane == 63u) { w_sum[wv] = incl; w_max[wv] = hi_max; w_min[wv] = hi_min_inv; }
+    if (lane == 63u) { sh.w_sum[wv] = incl; sh.w_max[wv] = hi_max; sh.w_min[wv] = hi_min_inv; }
     __syncthreads();
     uint32_t base = incl - mine, total = 0;
-    for (uint32_t w = 0; w < W; ++w) { if (w < wv) base += w_sum[w]; total += w_sum[w]; }
+    for (uint32_t w = 0; w < W; ++w) { if (w < wv) base += sh.w_sum[w]; total += sh.w_sum[w]; }
     const bool too_many = total > uint32_t(kFinalCap);
     // A sampling level whose candidates did not all fit yields its floor from the subset that was
     // kept: a valid floor, but possibly far below the k_floor-th best of the level.  The flag lets
@@ -1333,6 +1333,8 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
         if (t == 0) overflow[qn] = redo ? (raising ? 1u : 2u) : 0u;
         if (redo && !raising) return;
     }
+    // (the last query's is among the last to get here; the launch's end is its selection away)
+    if (stamp != nullptr && sampling && qn + 1 == int(gridDim.x) && t == 0) *stamp = wall_clock64();
     if (sampling && total < uint32_t(k_eff)) {
         // Too few allowed slots reached the floor in this sample.  The floor of the level before
         // (k_floor scanned slots reach it) is still a valid lower bound: it stays.  Only the
@@ -1397,55 +1399,12 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
             });
             hi_max = wave_umax(hi_max);
             hi_min_inv = wave_umax(hi_min_inv);
-            if (lane == 63u) { w_max[wv] = hi_max; w_min[wv] = hi_min_inv; }
+            if (lane == 63u) { sh.w_max[wv] = hi_max; sh.w_min[wv] = hi_min_inv; }
             __syncthreads();
         }
         uint32_t mx = 0u, mn_inv = 0u;
-        for (uint32_t w = 0; w < W; ++w) { mx = max(mx, w_max[w]); mn_inv = max(mn_inv, w_min[w]); }
-        // keys lie in [low, low + 2^width): 1024 bins of 2^shift; `above` of them were counted beyond that range
-        // before, and `rest` are still wanted from it
-        uint64_t low = uint64_t(~mn_inv) << 32;
-        uint32_t width = 32u + (mx == ~mn_inv ? 0u : 32u - uint32_t(__clz(int(mx - ~mn_inv))));
-        uint32_t above = 0u, rest = need;
-        for (;;) {
-            const uint32_t shift = width > 10u ? width - 10u : 0u;
-            each([&](uint64_t k) {
-                const uint64_t d = k - low;
-                if (k >= low && (width >= 64u || (d >> width) == 0ull)) atomicAdd(&bins[uint32_t(d >> shift)], 1u);
-            });
-            __syncthreads();
-            // from the top: the bin in which the count passes `rest`
-            uint32_t own[kPerBin], sum = 0u;
-#pragma unroll
-            for (uint32_t i = 0; i < kPerBin; ++i) { own[i] = bins[kFinalBins - 1u - (t * kPerBin + i)]; sum += own[i]; }
-            uint32_t run = sum;
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t v = __shfl_up(run, off);
-                if (lane >= uint32_t(off)) run += v;
-            }
-            if (lane == 63u) w_sum[wv] = run;
-            __syncthreads();
-            uint32_t before = run - sum;
-            for (uint32_t w = 0; w < W; ++w) if (w < wv) before += w_sum[w];
-#pragma unroll
-            for (uint32_t i = 0; i < kPerBin; ++i) {
-                if (before < rest && before + own[i] >= rest) {
-                    s_bin = kFinalBins - 1u - (t * kPerBin + i);
-                    s_above = before;
-                    s_at = before + own[i];
-                }
-                before += own[i];
-                bins[kFinalBins - 1u - (t * kPerBin + i)] = 0u;
-            }
-            __syncthreads();
-            low += uint64_t(s_bin) << shift;
-            if (above + s_at <= kFinalKept) break;             // (a bin of width one holds one key: this ends)
-            above += s_above;
-            rest -= s_above;
-            width = shift;
-            __syncthreads();                                   // s_* are read by all before they are written again
-        }
-        threshold = low;
+        for (uint32_t w = 0; w < W; ++w) { mx = max(mx, sh.w_max[w]); mn_inv = max(mn_inv, sh.w_min[w]); }
+        threshold = select_threshold<T>(each, mx, mn_inv, need, sh);
     }
     each([&](uint64_t k) {
         if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
@@ -1457,11 +1416,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     const size_t row = row_map ? size_t(row_map[qn]) : size_t(qn);   // a repeated pass writes to the rows of the queries it repeats
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];
-        uint32_t rank = 0u;
-        for (uint32_t j = 0; j < n; j += 2u) {
-            const ulonglong2 o = *reinterpret_cast<const ulonglong2 *>(&kept[j]);
-            rank += (o.x > k ? 1u : 0u) + (o.y > k ? 1u : 0u);
-        }
+        const uint32_t rank = rank_in(kept, n, k);
         if (rank >= need) continue;
         float s; uint32_t idx;
         sort_unkey(k, s, idx);
@@ -1607,13 +1562,13 @@ hipError_t launch_build_p(const float *d_qcal, const float *d_bias_corr, uint8_t
 hipError_t launch_prep_p(const float *d_q, const float *d_signs, const uint32_t *d_perms, int dim, int block,
                          float inv_sqrt_block, const float *d_shift, const float *d_scale, uint8_t *d_wfrag,
                          float *d_qscale, float *d_qbias, int G, int nch, float cs, size_t nq, size_t nq_padded, bool split,
-                         hipStream_t s) {
+                         uint64_t *stamp, hipStream_t s) {
     if (nq_padded == 0) return hipSuccess;
     const size_t lds = size_t(2) * dim * sizeof(float);
     hipError_t e = allow_lds(k_prep_p, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_prep_p, dim3(unsigned(nq_padded)), dim3(256), lds, s, d_q, d_signs, d_perms, dim, block,
-                       inv_sqrt_block, d_shift, d_scale, d_wfrag, d_qscale, d_qbias, G, nch, cs, nq, split);
+                       inv_sqrt_block, d_shift, d_scale, d_wfrag, d_qscale, d_qbias, G, nch, cs, nq, split, stamp);
     return hipGetLastError();
 }
 
@@ -1660,11 +1615,14 @@ static int scan_p4_append_threads(int nch) {
     return lds <= kLdsBudget ? kScanThreadsShared : kScanThreads;
 }
 
+// One attribute, not the whole property record: a search asks several times.
+int device_cus(int device) {
+    int cus = 0;
+    return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0 ? cus : 256;
+}
+
 int scan_grid_blocks(int device, int mode_p, int nch, int k, int nq_tile) {
-    hipDeviceProp_t prop;
-    int cus = 256;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
+    const int cus = device_cus(device);
     if (mode_p && k == 0 && scan_p4_append_threads(nch) != kScanThreads)           // (k = 0: the append-mode scans)
         return cus * (kScanThreadsShared / kScanThreads);                         // one workgroup per CU, counted in four-wave groups
     const size_t lds = scan_lds_bytes(mode_p, nch, k, nq_tile);
@@ -1752,10 +1710,7 @@ int batched_tiles(int nch) {
 }
 
 int batched_grid_blocks(int device, int nch) {
-    hipDeviceProp_t prop;
-    int cus = 256;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
+    const int cus = device_cus(device);
     if (resident_tiles(nch) >= 2) {
         const size_t lds = size_t(resident_tiles(nch)) * nch * 2048 + multi_fixed_lds(resident_tiles(nch));
         const int per_cu = int(kLdsBudget / lds);
@@ -1830,11 +1785,11 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, hipStream_t s) {
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp, hipStream_t s) {
     if (nq == 0 || k_eff == 0) return hipSuccess;
     auto launch = [&](auto kernel, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
-                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if);
+                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, stamp);
     };
     if (n_seg <= 256) launch(k_final<256>, 256);
     else if (n_seg <= 512) launch(k_final<512>, 512);

@@ -584,10 +584,7 @@ int lut_append_queries(int nch) {
 static int lut_cus = 256;   // compute units of the device the last grid was sized for
 
 int lut_append_grid(int device, int nch) {
-    hipDeviceProp_t prop;
-    int cus = 256;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
+    const int cus = device_cus(device);
     lut_cus = cus;
     const size_t lds = lut_lds_bytes(nch, 0, lut_append_queries(nch), true, kLutAppendThreads);
     return cus * (lds * 2 <= kLdsBudgetL ? 2 : 1);   // at most 2048 threads per CU

@@ -498,6 +498,15 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
             const float2 qp = *reinterpret_cast<const float2 *>(&sqt[q].qs);
             const float qs = qp.x, qb = qp.y;
             const float *vs = s_vs + (wave * BLK + k) * 32 + 4 * h;
+            if (a.best_out != nullptr) {
+                // a search without sampling: every block's best score, no slot (tv_kernels6.hip)
+                float m = -__int_as_float(0x7f800000);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) m = fmaxf(m, fmaf(float(acc[k][r]), qs, qb) * vs[8 * (r >> 2) + (r & 3)]);   // (NaN never wins)
+                m = fmaxf(m, __shfl_xor(m, 32));
+                if (h == 0 && q < nq) a.best_out[size_t(q) * a.best_stride + blk[k]] = best_word(m);
+                return;
+            }
             float bs = 0.0f;
             int bi = -1;
 #pragma unroll
@@ -580,6 +589,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         if (has) close_stream();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // requests still in flight write this workgroup's LDS
+    if constexpr (BLK == 1) {
+        if (a.best_out != nullptr) return;
+    }
     __syncthreads();
     for (int q = tid; q < nq; q += kWideThreads) a.cand_cnt[size_t(q) * a.seg_stride + blockIdx.x] = sqt[q].cnt;
 }
@@ -697,11 +709,7 @@ int wide_max_queries(int nch) {
 }
 
 int wide_grid_blocks(int device) {
-    hipDeviceProp_t prop;
-    int cus = 256;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
-    return cus;      // one 8-wave workgroup per CU: its LDS holds the slice ring
+    return device_cus(device);      // one 8-wave workgroup per CU: its LDS holds the slice ring
 }
 
 template <int NCH, int NB, int WAVES = 8, int SPT = 2, int BLK = 1, int HO = 1, int KS = 1, bool SPLIT = false>

@@ -1,0 +1,403 @@
+// Search of a small index without sampling: one pass that keeps, per query and block of 32 rows, only the
+// best allowed row's score, then one launch that finds the k best blocks of each query, scores their rows
+// once more and ranks them.
+//
+// The k best rows lie in the k blocks whose best rows rank first: a row outside them has k rows, one per
+// such block, ranked before it (score, then lower slot; blocks follow the slots, so equal best scores
+// order blocks as they order rows).  So there is no floor to estimate, no candidate segment to overflow
+// and nothing to repeat: three dependent launches instead of five, and a (block, query) pair costs one
+// 4-byte store instead of the appends of an open first level.
+#include <algorithm>
+
+#include "tv_device.h"
+#include "tv_internal.h"
+#include "tv_select.h"
+
+namespace tv {
+
+// ===========================================================================
+// Score mode P: best row per (block, query) over NT query tiles per workgroup, their weights in LDS.
+// grid = (block groups, tile groups); a wave decodes a block's chunk on the vector ALU (about 60
+// instructions, 240 cycles) and feeds NT tiles' MFMAs from it (64 NT cycles), so four tiles balance the
+// two units.  The tiles are split over workgroups because a small index has few blocks: 100K rows are
+// 3125 of them, which fill 65 of the 256 workgroups of a kernel that takes all queries through one.
+// Weights in plane order (launch_prep_p, split = false).
+// ===========================================================================
+constexpr int kBestThreads = 512;
+constexpr int kBestWaves = kBestThreads / 64;
+
+template <int NT, int U>
+__global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(ScanArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int nch = a.nch, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qn = lane & 31, h = lane >> 5;
+    const int tile0 = int(blockIdx.y) * NT;
+    const int nt = min(NT, (a.nq_tile + kQTile - 1) / kQTile - tile0);
+    const uint32_t stride = gridDim.x * kBestWaves;
+    const uint4 *codes = reinterpret_cast<const uint4 *>(a.codes) + lane;
+    const float nan = __int_as_float(0x7fc00000);
+    auto store = [&](int t, uint32_t j, uint32_t word) {
+        const int q = (tile0 + t) * kQTile + qn;
+        if (h == 0 && t < nt && q < a.nq_tile) a.best_out[size_t(q) * a.best_stride + j] = word;
+    };
+    // the next block from j on with an allowed row; the ones without are recorded on the way
+    auto live_from = [&](uint32_t j) -> uint32_t {
+        if (a.mask == nullptr) return j;
+        for (; j < a.n_blocks; j += stride) {
+            if (uint32_t(a.mask[j >> 1] >> ((j & 1) * 32)) != 0u) break;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) store(t, j, 0u);
+        }
+        return j;
+    };
+    // the wave's first codes are on their way while the workgroup sets up its LDS
+    uint32_t j = live_from(blockIdx.x * kBestWaves + wave);
+    uint4 buf[U];
+    if (j < a.n_blocks) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) buf[u] = codes[(size_t(j) * nch + u) * 64];
+    }
+    {
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(tile0) * nch * 128;
+        uint4 *dst = reinterpret_cast<uint4 *>(smem);
+        const int n16 = nt * nch * 128;
+        constexpr int kBatch = 8;
+        for (int i0 = tid; i0 < n16; i0 += kBestThreads * kBatch) {
+            uint4 tmp[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) tmp[u] = i0 + u * kBestThreads < n16 ? src[i0 + u * kBestThreads] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                if (i0 + u * kBestThreads < n16) dst[i0 + u * kBestThreads] = tmp[u];
+        }
+    }
+    float qs[NT], qb[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int q = (tile0 + t) * kQTile + qn;
+        qs[t] = q < a.nq_tile ? a.qscale[q] : 0.0f;
+        qb[t] = q < a.nq_tile ? a.qbias[q] : 0.0f;
+    }
+    __syncthreads();
+    const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
+    const v4i *w = reinterpret_cast<const v4i *>(smem) + lane;
+
+    while (j < a.n_blocks) {
+        const uint32_t jn = live_from(j + stride);
+        // row scales, NaN where a row may not be returned
+        const uint32_t slot0 = j * 32u;
+        uint32_t mw = a.mask != nullptr ? uint32_t(a.mask[j >> 1] >> ((j & 1) * 32)) : 0xffffffffu;
+        if (slot0 + 32u > a.n) mw &= (1u << (a.n - slot0)) - 1u;
+        float vs[16];
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 f = *reinterpret_cast<const float4 *>(a.scales + slot0 + 8 * q4 + 4 * h);
+            vs[q4 * 4 + 0] = f.x; vs[q4 * 4 + 1] = f.y; vs[q4 * 4 + 2] = f.z; vs[q4 * 4 + 3] = f.w;
+        }
+        v16i acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        for (int c0 = 0; c0 < nch; c0 += U) {
+            uint4 cur[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) cur[u] = buf[u];
+            const bool more = c0 + U < nch;
+            if (more || jn < a.n_blocks) {
+                const uint4 *from = codes + (more ? size_t(j) * nch + c0 + U : size_t(jn) * nch) * 64;
+#pragma unroll
+                for (int u = 0; u < U; ++u) buf[u] = from[u * 64];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t x[4] = {cur[u].x, cur[u].y, cur[u].z, cur[u].w};
+                v4i lo, hi;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    lo[d] = int(levels_of(x[d] & 0x0f0f0f0fu, t0, t1, t2, t3));
+                    hi[d] = int(levels_of((x[d] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3));
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const v4i *wt = w + ((t * nch + c0 + u) * 2) * 64;
+                    acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(lo, wt[0], acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(hi, wt[64], acc[t], 0, 0, 0);
+                }
+            }
+        }
+        // lane: query qn of each tile, rows 8 (r / 4) + 4 h + r % 4 (search.rs:1519-1524)
+        if (mw != 0xffffffffu) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) vs[r] = ((mw >> (8 * (r >> 2) + 4 * h + (r & 3))) & 1u) ? vs[r] : nan;
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            float m = -__int_as_float(0x7f800000);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) m = fmaxf(m, fmaf(float(acc[t][r]), qs[t], qb[t]) * vs[r]);   // (NaN never wins)
+            store(t, j, best_word(fmaxf(m, __shfl_xor(m, 32))));
+        }
+        j = jn;
+    }
+}
+
+// Query tiles per workgroup: as many as the LDS holds beside another workgroup's -- four at most -- but no
+// more than leave the chip with a workgroup per CU.
+static int best_tiles(int nch, size_t n_blocks, int tiles) {
+    int nt = tiles >= 4 ? 4 : tiles == 3 ? 4 : tiles;
+    while (nt > 1 && size_t(nt) * nch * 2048 > 80 * 1024) nt /= 2;
+    const size_t groups = (n_blocks + kBestWaves - 1) / kBestWaves;
+    while (nt > 1 && groups * size_t((tiles + nt - 1) / nt) < 256) nt /= 2;
+    return nt;
+}
+bool best_serves(int nch) { return size_t(nch) * 2048 <= 160 * 1024; }
+
+template <int NT, int U>
+static hipError_t launch_best_n(const ScanArgs &a, int device, hipStream_t s) {
+    const int tiles = (a.nq_tile + kQTile - 1) / kQTile, groups_y = (tiles + NT - 1) / NT;
+    const size_t lds = size_t(NT) * a.nch * 2048;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+    // a workgroup keeps its weights for all its blocks: about as many workgroups as are resident
+    const unsigned per_cu = unsigned(std::min<size_t>(NT <= 2 ? 2 : 1, 160 * 1024 / lds));
+    const unsigned resident = unsigned(device_cus(device)) * std::max(1u, per_cu);
+    const unsigned x = std::max(1u, std::min((a.n_blocks + kBestWaves - 1) / kBestWaves, (resident + groups_y - 1) / groups_y));
+    hipLaunchKernelGGL((k_scan_p4_best<NT, U>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
+    return hipGetLastError();
+}
+template <int NT>
+static hipError_t launch_best_u(const ScanArgs &a, int device, hipStream_t s) {
+    // (two tiles' accumulators and bursts of four chunks do not fit the 128 registers of four waves per SIMD)
+    if constexpr (NT != 2) {
+        if (a.nch % 4 == 0) return launch_best_n<NT, 4>(a, device, s);
+    }
+    return a.nch % 2 == 0 ? launch_best_n<NT, 2>(a, device, s) : launch_best_n<NT, 1>(a, device, s);
+}
+// a.nq_tile = all queries of the launch, a.tables = their weight tiles, a.best_out / a.best_stride = the result.
+hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s) {
+    if (a.nq_tile <= 0 || a.n_blocks == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride < a.n_blocks) return hipErrorInvalidValue;
+    switch (best_tiles(a.nch, a.n_blocks, (a.nq_tile + kQTile - 1) / kQTile)) {
+        case 1: return launch_best_u<1>(a, device, s);
+        case 2: return launch_best_u<2>(a, device, s);
+        default: return launch_best_u<4>(a, device, s);
+    }
+}
+
+// ===========================================================================
+// One workgroup per query: the k_eff best blocks by counting (select_threshold), their rows scored as the
+// scans score them, ranked.  All latency for one query -- 100K x 128, k = 10: see the launcher.
+// ===========================================================================
+struct PickArgs {
+    const uint32_t *best;
+    uint32_t best_stride, n_blocks, n;
+    const uint8_t *codes;
+    const float *scales;
+    const uint64_t *mask;
+    const uint8_t *tables;
+    const float *qscale, *qbias;
+    uint32_t lv[4];
+    int nch, k_eff, split;
+    float *out_scores;
+    int64_t *out_idx;
+    uint32_t *overflow;
+    uint64_t *stamp;
+};
+constexpr uint32_t kPickHeld = 16;       // blocks a thread keeps in registers
+
+template <uint32_t T, bool P>
+__global__ __launch_bounds__(T) void k_pick(PickArgs a) {
+    constexpr uint32_t W = T / 64;
+    extern __shared__ __align__(16) uint8_t dyn[];
+    __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
+    __shared__ SelectShared sh;
+    __shared__ uint32_t blocks[kMaxPickK];
+    __shared__ uint32_t n_kept, n_list, s_floor;
+    uint64_t *list = reinterpret_cast<uint64_t *>(dyn);                     // rows of the chosen blocks that can still matter
+    uint8_t *wts = dyn + size_t(a.k_eff) * 32 * 8;                          // this query's weights, or its tables
+    const uint32_t qi = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    const uint32_t k_eff = uint32_t(a.k_eff);
+    const uint32_t *best = a.best + size_t(qi) * a.best_stride;
+    if (a.stamp != nullptr && qi + t == 0) *a.stamp = wall_clock64();
+    const bool held = a.n_blocks <= T * kPickHeld;
+    uint32_t v[kPickHeld];
+#pragma unroll
+    for (uint32_t e = 0; e < kPickHeld; ++e) v[e] = held && e * T + t < a.n_blocks ? best[e * T + t] : 0u;
+    if (P) {
+        // the tile's weights lie [chunk][fragment][half * 32 + query] in 16-byte pieces; here [chunk][half][fragment]
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
+        for (int i = int(t); i < a.nch * 4; i += int(T))
+            reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
+    } else {
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi) * a.nch * 64;
+        for (int i = int(t); i < a.nch * 64; i += int(T)) reinterpret_cast<uint4 *>(wts)[i] = src[i];
+    }
+    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
+    if (t == 0) { n_kept = 0u; n_list = 0u; s_floor = 0u; }
+    auto each = [&](auto &&f) {
+        if (held) {
+#pragma unroll
+            for (uint32_t e = 0; e < kPickHeld; ++e)
+                if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
+        } else {
+            for (uint32_t i = t; i < a.n_blocks; i += T) {
+                const uint32_t word = best[i];
+                if (word != 0u) f((uint64_t(word) << 32) | ~i);
+            }
+        }
+    };
+    uint32_t mine = 0u, hi_max = 0u, hi_min_inv = 0u, mx, mn_inv, total = 0u;
+    each([&](uint64_t k) {
+        ++mine;
+        hi_max = max(hi_max, uint32_t(k >> 32));
+        hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+    });
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) mine += __shfl_xor(mine, d);
+    if (lane == 0) sh.w_sum[wv] = mine;
+    select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
+    for (uint32_t w = 0; w < W; ++w) total += sh.w_sum[w];
+    __syncthreads();
+    const uint32_t need = min(k_eff, total);
+    const uint64_t threshold = total > 256u ? select_threshold<T>(each, mx, mn_inv, need, sh) : 0ull;
+    each([&](uint64_t k) {
+        if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
+    });
+    __syncthreads();
+    uint32_t n = n_kept;
+    if (t < 2u) kept[n + t] = 0ull;
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += T) {
+        const uint64_t k = kept[i];
+        const uint32_t rank = rank_in(kept, n, k);
+        if (rank < need) blocks[rank] = ~uint32_t(k);
+        // k_eff blocks have a row that reaches the last one's best: nothing below it is wanted
+        if (rank + 1u == k_eff) s_floor = uint32_t(k >> 32);
+    }
+    __syncthreads();
+    // the chosen blocks' rows, a block per wave: lane = row lane % 32, sixteen code bytes of each chunk
+    const uint32_t floor_word = s_floor, h = lane >> 5;
+    const float qs = a.qscale[qi], qb = a.qbias[qi];
+    const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
+    for (uint32_t i = wv; i < need; i += W) {
+        const uint32_t b = blocks[i], slot = b * 32u + (lane & 31u);
+        const float vs = a.scales[slot];
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.codes) + size_t(b) * a.nch * 64 + lane;
+        int acc = 0;
+        constexpr int kBurst = 8;
+        for (int c0 = 0; c0 < a.nch; c0 += kBurst) {
+            uint4 x[kBurst];
+#pragma unroll
+            for (int u = 0; u < kBurst; ++u) x[u] = c0 + u < a.nch ? src[(c0 + u) * 64] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < kBurst; ++u) {
+                if (c0 + u >= a.nch) break;
+                const uint32_t d[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+                if (P) {
+                    const uint4 *wq = reinterpret_cast<const uint4 *>(wts) + ((c0 + u) * 2 + h) * 2;
+                    const uint4 f0 = wq[0], f1 = wq[1];
+                    uint32_t lo[4], hi[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        lo[e] = levels_of(d[e] & 0x0f0f0f0fu, t0, t1, t2, t3);
+                        hi[e] = levels_of((d[e] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3);
+                    }
+                    const uint32_t g0[4] = {f0.x, f0.y, f0.z, f0.w}, g1[4] = {f1.x, f1.y, f1.z, f1.w};
+                    if (a.split) {
+                        // bytes 0..7 as (low, high) dwords of four, bytes 8..15 as (low, high) byte pairs (k_scan_p4)
+                        acc = __builtin_amdgcn_sdot4(int(lo[0]), int(g0[0]), acc, false);
+                        acc = __builtin_amdgcn_sdot4(int(hi[0]), int(g0[1]), acc, false);
+                        acc = __builtin_amdgcn_sdot4(int(lo[1]), int(g0[2]), acc, false);
+                        acc = __builtin_amdgcn_sdot4(int(hi[1]), int(g0[3]), acc, false);
+#pragma unroll
+                        for (int e = 2; e < 4; ++e) {
+                            acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x05010400u)), int(g1[2 * e - 4]), acc, false);
+                            acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x07030602u)), int(g1[2 * e - 3]), acc, false);
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            acc = __builtin_amdgcn_sdot4(int(lo[e]), int(g0[e]), acc, false);
+                            acc = __builtin_amdgcn_sdot4(int(hi[e]), int(g1[e]), acc, false);
+                        }
+                    }
+                } else {
+                    const uint8_t *lut = wts + ((c0 + u) * 32 + int(h) * 16) * 32;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const uint32_t byte = (d[e >> 2] >> (8 * (e & 3))) & 0xffu;
+                        acc += int(lut[e * 32 + (byte >> 4)]) + int(lut[e * 32 + 16 + (byte & 15u)]);
+                    }
+                }
+            }
+        }
+        acc += __shfl_xor(acc, 32);
+        const float s = P ? fmaf(float(acc), qs, qb) * vs : ((float(acc) * qs) + qb) * vs;
+        bool ok = lane < 32u && slot < a.n && s == s;
+        if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> (lane & 31u)) & 1u;
+        const uint64_t key = sort_key(s, slot);
+        if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
+    }
+    __syncthreads();
+    const uint32_t m = n_list;
+    // (fewer rows than the caller's count of allowed ones promised: the exact path takes the query)
+    if (t == 0) a.overflow[qi] = m < k_eff ? 2u : 0u;
+    if (m < k_eff) return;
+    auto each_row = [&](auto &&f) {
+        for (uint32_t i = t; i < m; i += T) f(list[i]);
+    };
+    uint64_t least = 0ull;
+    if (m > kSelectKept) {      // many ties
+        hi_max = 0u;
+        hi_min_inv = 0u;
+        each_row([&](uint64_t k) {
+            hi_max = max(hi_max, uint32_t(k >> 32));
+            hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+        });
+        select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
+        least = select_threshold<T>(each_row, mx, mn_inv, k_eff, sh);
+    }
+    if (t == 0) n_kept = 0u;
+    __syncthreads();
+    each_row([&](uint64_t k) {
+        if (k >= least) kept[atomicAdd(&n_kept, 1u)] = k;
+    });
+    __syncthreads();
+    n = n_kept;
+    if (t < 2u) kept[n + t] = 0ull;
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += T) {
+        const uint64_t k = kept[i];
+        const uint32_t rank = rank_in(kept, n, k);
+        if (rank >= k_eff) continue;
+        float s; uint32_t idx;
+        sort_unkey(k, s, idx);
+        a.out_scores[size_t(qi) * k_eff + rank] = s;
+        a.out_idx[size_t(qi) * k_eff + rank] = int64_t(idx);
+    }
+}
+
+size_t pick_lds_bytes(bool mode_p, int nch, size_t k_eff) { return k_eff * 32 * 8 + size_t(nch) * (mode_p ? 64 : 1024); }
+
+// The scan's arguments say what was scanned; a.tables: the weight tiles (mode P) or the tables query by query.
+hipError_t launch_pick(const ScanArgs &a, bool mode_p, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow,
+                       uint64_t *stamp, hipStream_t s) {
+    if (a.nq_tile <= 0) return hipSuccess;
+    const size_t lds = pick_lds_bytes(mode_p, a.nch, size_t(k_eff));
+    if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1) return hipErrorInvalidValue;
+    PickArgs p;
+    p.best = a.best_out; p.best_stride = a.best_stride; p.n_blocks = a.n_blocks; p.n = a.n;
+    p.codes = a.codes; p.scales = a.scales; p.mask = a.mask; p.tables = a.tables;
+    p.qscale = a.qscale; p.qbias = a.qbias;
+    for (int i = 0; i < 4; ++i) p.lv[i] = a.lv[i];
+    p.nch = a.nch; p.k_eff = k_eff; p.split = split ? 1 : 0;
+    p.out_scores = out_scores; p.out_idx = out_idx; p.overflow = overflow; p.stamp = stamp;
+    auto launch = [&](auto kernel, unsigned threads) -> hipError_t {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(a.nq_tile)), dim3(threads), lds, s, p);
+        return hipGetLastError();
+    };
+    // few queries leave the chip empty: as many waves as there are blocks to score again
+    if (a.nq_tile <= 256 || a.n_blocks > 256 * kPickHeld) return mode_p ? launch(k_pick<1024, true>, 1024) : launch(k_pick<1024, false>, 1024);
+    return mode_p ? launch(k_pick<256, true>, 256) : launch(k_pick<256, false>, 256);
+}
+
+}  // namespace tv

@@ -1,0 +1,93 @@
+// Selection by counting, shared by the kernels that pick the best of a few thousand keys in a workgroup.
+#pragma once
+#include "tv_device.h"
+
+namespace tv {
+
+constexpr uint32_t kSelectBins = 1024;
+constexpr uint32_t kSelectKept = 1024;     // keys left to rank by comparison
+
+struct SelectShared {
+    uint32_t bins[kSelectBins];            // all zero between uses
+    uint32_t w_sum[16], w_max[16], w_min[16];
+    uint32_t bin, at, above;
+};
+
+// A threshold that at least `need` and at most kSelectKept of the keys reach: counting passes into 1024
+// bins between the smallest (its score word given inverted) and the largest score word, from the top; a
+// bin that still holds too many is divided again.  `each(f)` calls f with every key of the calling
+// thread; keys are distinct, and at least `need` of them exist.  Met by all T threads.
+template <uint32_t T, typename Each>
+__device__ __forceinline__ uint64_t select_threshold(const Each &each, uint32_t mx, uint32_t mn_inv, uint32_t need, SelectShared &sh) {
+    constexpr uint32_t W = T / 64, kPerBin = kSelectBins / T;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    // keys lie in [low, low + 2^width): 1024 bins of 2^shift; `above` of them were counted beyond that range
+    // before, and `rest` are still wanted from it
+    uint64_t low = uint64_t(~mn_inv) << 32;
+    uint32_t width = 32u + (mx == ~mn_inv ? 0u : 32u - uint32_t(__clz(int(mx - ~mn_inv))));
+    uint32_t above = 0u, rest = need;
+    for (;;) {
+        const uint32_t shift = width > 10u ? width - 10u : 0u;
+        each([&](uint64_t k) {
+            const uint64_t d = k - low;
+            if (k >= low && (width >= 64u || (d >> width) == 0ull)) atomicAdd(&sh.bins[uint32_t(d >> shift)], 1u);
+        });
+        __syncthreads();
+        // from the top: the bin in which the count passes `rest`
+        uint32_t own[kPerBin], sum = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < kPerBin; ++i) { own[i] = sh.bins[kSelectBins - 1u - (t * kPerBin + i)]; sum += own[i]; }
+        uint32_t run = sum;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t v = __shfl_up(run, off);
+            if (lane >= uint32_t(off)) run += v;
+        }
+        if (lane == 63u) sh.w_sum[wv] = run;
+        __syncthreads();
+        uint32_t before = run - sum;
+        for (uint32_t w = 0; w < W; ++w) if (w < wv) before += sh.w_sum[w];
+#pragma unroll
+        for (uint32_t i = 0; i < kPerBin; ++i) {
+            if (before < rest && before + own[i] >= rest) {
+                sh.bin = kSelectBins - 1u - (t * kPerBin + i);
+                sh.above = before;
+                sh.at = before + own[i];
+            }
+            before += own[i];
+            sh.bins[kSelectBins - 1u - (t * kPerBin + i)] = 0u;
+        }
+        __syncthreads();
+        low += uint64_t(sh.bin) << shift;
+        if (above + sh.at <= kSelectKept) break;               // (a bin of width one holds one key: this ends)
+        above += sh.above;
+        rest -= sh.above;
+        width = shift;
+        __syncthreads();                                       // sh.* are read by all before they are written again
+    }
+    return low;
+}
+
+// Largest score word and largest inverted score word over all T threads' keys.  Met by all T threads.
+template <uint32_t T>
+__device__ __forceinline__ void select_range(uint32_t hi_max, uint32_t hi_min_inv, SelectShared &sh, uint32_t &mx, uint32_t &mn_inv) {
+    constexpr uint32_t W = T / 64;
+    hi_max = wave_umax(hi_max);
+    hi_min_inv = wave_umax(hi_min_inv);
+    if ((threadIdx.x & 63u) == 63u) { sh.w_max[threadIdx.x >> 6] = hi_max; sh.w_min[threadIdx.x >> 6] = hi_min_inv; }
+    __syncthreads();
+    mx = 0u;
+    mn_inv = 0u;
+    for (uint32_t w = 0; w < W; ++w) { mx = max(mx, sh.w_max[w]); mn_inv = max(mn_inv, sh.w_min[w]); }
+}
+
+// Keys greater than k among kept[0 .. n), which is followed by two zero keys (read in pairs).
+__device__ __forceinline__ uint32_t rank_in(const uint64_t *kept, uint32_t n, uint64_t k) {
+    uint32_t rank = 0u;
+    for (uint32_t j = 0; j < n; j += 2u) {
+        const ulonglong2 o = *reinterpret_cast<const ulonglong2 *>(&kept[j]);
+        rank += (o.x > k ? 1u : 0u) + (o.y > k ? 1u : 0u);
+    }
+    return rank;
+}
+
+}  // namespace tv
