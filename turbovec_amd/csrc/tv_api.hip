@@ -220,51 +220,34 @@ struct Prepared {
 // Query preparation for one chunk: rotation, TQ+ inverse, table build
 // (turbovec/src/search.rs:3237-3269).  d_q holds nq*dim floats on the device.
 // `split`: permute-dot weights in the order k_scan_p4 reads them (the batched scans take plane order)
-// `keep_rotated`: the rotated rows are wanted in device memory too (the debug read-back); a search
-// in permute-dot mode does not need them and prepares its queries in a single launch.
+// `keep_rotated`: the rotated rows are wanted in device memory too (the debug read-back).
 // `for_append`: u8-LUT tables are wanted in the order of the batch's append scan too.
 int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepared &out, bool split = true,
                     bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr) {
     const tv::Geometry &g = ix->geo;
     const size_t nq_pad = round_up(nq, tv::kQTile);
     const int mode = effective_mode(ix);
-    if (mode == TV_SCORE_P && !keep_rotated) {
-        const bool cal = !ix->tq_shift.empty();
-        out.d_qrot = nullptr;
-        out.d_qscale = ar.take<float>(nq_pad);
-        out.d_qbias = ar.take<float>(nq_pad);
-        out.table_bytes_per_tile = size_t(g.nch) * 2048;
-        out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
-        TV_HIP(tv::launch_prep_p(d_q, ix->d_signs, ix->d_perms, g.dim, ix->rot.block, ix->rot.inv_sqrt_block,
-                                 cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr, out.d_tables, out.d_qscale,
-                                 out.d_qbias, g.G, g.nch, ix->cs, nq, nq_pad, split, stamp, ix->stream));
-        return TV_OK;
-    }
-    float *d_rot = ar.take<float>(nq * g.dim);
-    float *d_bias_corr = ar.take<float>(nq_pad);
-    TV_HIP(tv::launch_rotate(d_q, d_rot, ix->d_signs, ix->d_perms, g.dim, ix->rot.block, ix->rot.inv_sqrt_block, nq,
-                             ix->stream));
-    float *d_cal = d_rot;
-    if (!ix->tq_shift.empty()) {
-        d_cal = ar.take<float>(nq * g.dim);
-        TV_HIP(tv::launch_calibrate(d_rot, d_cal, d_bias_corr, ix->d_tq_shift, ix->d_tq_scale, g.dim, nq,
-                                    ix->stream));
-    } else {
-        d_bias_corr = nullptr;   // uncalibrated: the table builders add +0.0f themselves (search.rs:3176-3185)
-    }
-    out.d_qrot = d_cal;
-    out.d_qscale = ar.take<float>(nq_pad);
-    out.d_qbias = ar.take<float>(nq_pad);
-    if (mode == TV_SCORE_P) {
-        out.table_bytes_per_tile = size_t(g.nch) * 2048;
-        out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
-        TV_HIP(tv::launch_build_p(d_cal, d_bias_corr, out.d_tables, out.d_qscale, out.d_qbias, g.dim, g.G, g.nch,
-                                  ix->cs, nq, nq_pad, split, ix->stream));
-    } else {
-        out.table_bytes_per_tile = size_t(g.nch) * 1024 * tv::kQTile;
-        out.d_tables = ar.take<uint8_t>(nq_pad * size_t(g.nch) * 1024);
-        TV_HIP(tv::launch_build_lut(d_cal, d_bias_corr, ix->d_centroids, out.d_tables, out.d_qscale, out.d_qbias,
-                                    g.dim, g.bits, g.G, g.nch, nq, nq_pad, ix->stream));
+    const bool cal = !ix->tq_shift.empty(), mode_p = mode == TV_SCORE_P;
+    tv::PrepRequest r{};
+    r.q = d_q;
+    r.signs = ix->d_signs;
+    r.perms = ix->d_perms;
+    r.block = ix->rot.block;
+    r.inv_sqrt_block = ix->rot.inv_sqrt_block;
+    r.shift = cal ? ix->d_tq_shift : nullptr;
+    r.scale = cal ? ix->d_tq_scale : nullptr;
+    r.permute_dot = mode_p;
+    r.split = split;
+    r.cs = ix->cs;
+    r.centroids = ix->d_centroids;
+    r.rot_out = out.d_qrot = keep_rotated ? ar.take<float>(nq * g.dim) : nullptr;
+    r.qscale = out.d_qscale = ar.take<float>(nq_pad);
+    r.qbias = out.d_qbias = ar.take<float>(nq_pad);
+    out.table_bytes_per_tile = mode_p ? size_t(g.nch) * 2048 : size_t(g.nch) * 1024 * tv::kQTile;
+    r.tables = out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
+    r.stamp = stamp;
+    TV_HIP(tv::launch_prep(r, g, nq, nq_pad, ix->stream));
+    if (!mode_p) {
         if (for_append && lut_mx_serves(ix, nq)) {
             out.d_tables_mx = ar.take<uint8_t>(tv::mx_table_bytes(g.nch, g.bits, nq));
             TV_HIP(tv::launch_lut_fragments(out.d_tables, out.d_tables_mx, g.nch, g.bits, nq, ix->stream));

@@ -176,6 +176,20 @@ __device__ __forceinline__ bool launch_switched_off(const uint32_t *run_if) {
     return run_if != nullptr && *reinterpret_cast<const volatile uint32_t *>(run_if) == 0u;
 }
 
+// R butterfly stages on 2^R values, the first of stride 2^S in the row: a, b -> a + b, a - b.
+template <int R>
+__device__ __forceinline__ void butterflies(float *v) {
+#pragma unroll
+    for (int st = 0; st < R; ++st) {
+#pragma unroll
+        for (int i = 0; i < (1 << R); ++i) {
+            if ((i >> st) & 1) continue;
+            const float x = v[i], y = v[i | (1 << st)];
+            v[i] = x + y;
+            v[i | (1 << st)] = x - y;
+        }
+    }
+}
 // Compile-time loop: f(IntC<0>{}), ..., f(IntC<N-1>{}), for bodies that index register arrays.
 template <int V> struct IntC { static constexpr int value = V; };
 template <int N, int I = 0, typename F>

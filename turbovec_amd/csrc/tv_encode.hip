@@ -200,20 +200,6 @@ struct EncodeRowsArgs {
     size_t old_n, n_new;
 };
 
-// R butterfly stages on 2^R values, the first of stride 2^S in the row: a, b -> a + b, a - b.
-template <int R>
-__device__ __forceinline__ void enc_stages(float *v) {
-#pragma unroll
-    for (int st = 0; st < R; ++st) {
-#pragma unroll
-        for (int i = 0; i < (1 << R); ++i) {
-            if ((i >> st) & 1) continue;
-            const float x = v[i], y = v[i | (1 << st)];
-            v[i] = x + y;
-            v[i | (1 << st)] = x - y;
-        }
-    }
-}
 // Orders a wave's LDS accesses with each other (the LDS serves a wave's requests in order; this keeps
 // the compiler from reordering them).
 __device__ __forceinline__ void enc_wave_sync() {
@@ -276,7 +262,7 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
             float v[N];
 #pragma unroll
             for (int e = 0; e < N; ++e) v[e] = at[e * apart];
-            enc_stages<decltype(rr_)::value>(v);
+            butterflies<decltype(rr_)::value>(v);
             if (last) {
 #pragma unroll
                 for (int e = 0; e < N; ++e) v[e] = v[e] * a.inv_sqrt_block;
@@ -365,7 +351,7 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
 #pragma unroll
             for (int i = 0; i < NG; ++i) {
                 const int g = l + i * L;
-                enc_stages<3>(v[i]);
+                butterflies<3>(v[i]);
                 if (round == 1 && a.log_block == 3) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * a.inv_sqrt_block;

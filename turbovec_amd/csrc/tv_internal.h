@@ -94,24 +94,26 @@ bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint
 hipError_t launch_move_lane(uint8_t *d_native, float *d_scales, const Geometry &g, size_t src, size_t dst,
                             hipStream_t s);
 
-hipError_t launch_rotate(const float *d_q, float *d_out, const float *d_signs, const uint32_t *d_perms, int dim,
-                         int block, float inv_sqrt_block, size_t nq, hipStream_t s);
-hipError_t launch_calibrate(const float *d_qrot, float *d_qcal, float *d_bias_corr, const float *d_shift,
-                            const float *d_scale, int dim, size_t nq, hipStream_t s);
-hipError_t launch_build_p(const float *d_qcal, const float *d_bias_corr, uint8_t *d_wfrag, float *d_qscale,
-                          float *d_qbias, int dim, int G, int nch, float cs, size_t nq, size_t nq_padded,
-                          bool split, hipStream_t s);
-// `stamp` here and below, when given: a word that takes the device clock as the launch ends (of the
-// preparation and of a sampling level's selection) or starts (of a last selection): the scan between two
-// of them is timed without events, whose packets the launches behind them wait for, 5 to 6 us each.
-// Rotation, TQ+ inverse (d_shift / d_scale null: none) and permute-dot weights in one launch.
-hipError_t launch_prep_p(const float *d_q, const float *d_signs, const uint32_t *d_perms, int dim, int block,
-                         float inv_sqrt_block, const float *d_shift, const float *d_scale, uint8_t *d_wfrag,
-                         float *d_qscale, float *d_qbias, int G, int nch, float cs, size_t nq, size_t nq_padded, bool split,
-                         uint64_t *stamp, hipStream_t s);
-hipError_t launch_build_lut(const float *d_qcal, const float *d_bias_corr, const float *d_centroids, uint8_t *d_lut,
-                            float *d_qscale, float *d_qbias, int dim, int bits, int G, int nch, size_t nq,
-                            size_t nq_padded, hipStream_t s);
+// Query preparation in one launch (tv_prep.hip).  `stamp` here and below, when given: a word that takes the
+// device clock as the launch ends (of the preparation and of a sampling level's selection) or starts (of a
+// last selection): the scan between two of them is timed without events, whose packets the launches behind
+// them wait for, 5 to 6 us each.
+struct PrepRequest {
+    const float *q, *signs;
+    const uint32_t *perms;
+    int block;
+    float inv_sqrt_block;
+    const float *shift, *scale;     // the TQ+ pair, or null
+    bool permute_dot;               // int8 weights (cs, split: k_scan_p4's order) or u8 tables (centroids)
+    bool split;
+    float cs;
+    const float *centroids;
+    uint8_t *tables;
+    float *qscale, *qbias;
+    float *rot_out;                 // or null
+    uint64_t *stamp;                // or null (permute-dot only)
+};
+hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s);
 
 int device_cus(int device);   // compute units
 int scan_grid_blocks(int device, int mode_p, int nch, int k, int lut_queries);

@@ -115,308 +115,6 @@ __global__ void k_fill_i32(int *p, int v, size_t n) {
 }
 
 // ===========================================================================
-// Query preparation
-// ===========================================================================
-
-// turbovec/src/rotation.rs:265-320 (apply_with_scratch) + :964-982 (wht_block_scalar).
-// One workgroup per query row; both rounds run in LDS.  Every output element is
-// produced by the same IEEE adds, subtracts and multiplies, in the same
-// operand pairing, as the scalar butterfly, so the result is bit-identical.
-__global__ __launch_bounds__(256) void k_rotate(const float *__restrict__ q, float *__restrict__ out,
-                                                const float *__restrict__ signs,
-                                                const uint32_t *__restrict__ perms, int dim, int block,
-                                                float inv_sqrt_block) {
-    extern __shared__ float rot_lds[];
-    float *A = rot_lds;
-    float *B = rot_lds + dim;
-    const float *src = q + size_t(blockIdx.x) * dim;
-    const int t = threadIdx.x;
-    for (int i = t; i < dim; i += 256) A[i] = src[perms[i]] * signs[i];
-    __syncthreads();
-    for (int len = 1; len < block; len <<= 1) {
-        for (int p = t; p < dim / 2; p += 256) {
-            const int j = 2 * p - (p & (len - 1));
-            const float a = A[j], b = A[j + len];
-            A[j] = a + b;
-            A[j + len] = a - b;
-        }
-        __syncthreads();
-    }
-    // the 1/sqrt(B) scale of round 0 rides the round-1 gather: (x * inv) * sign
-    for (int i = t; i < dim; i += 256) B[i] = (A[perms[dim + i]] * inv_sqrt_block) * signs[dim + i];
-    __syncthreads();
-    for (int len = 1; len < block; len <<= 1) {
-        for (int p = t; p < dim / 2; p += 256) {
-            const int j = 2 * p - (p & (len - 1));
-            const float a = B[j], b = B[j + len];
-            B[j] = a + b;
-            B[j + len] = a - b;
-        }
-        __syncthreads();
-    }
-    float *dst = out + size_t(blockIdx.x) * dim;
-    for (int i = t; i < dim; i += 256) dst[i] = B[i] * inv_sqrt_block;
-}
-
-// turbovec/src/search.rs:3154-3186 calibrate_queries.  The f64 bias sum is
-// sequential over d, so one thread carries it.
-__global__ __launch_bounds__(256) void k_calibrate(const float *__restrict__ qrot, float *__restrict__ qcal,
-                                                   float *__restrict__ bias_corr,
-                                                   const float *__restrict__ shift,
-                                                   const float *__restrict__ scale, int dim) {
-    const float *src = qrot + size_t(blockIdx.x) * dim;
-    float *dst = qcal + size_t(blockIdx.x) * dim;
-    for (int i = threadIdx.x; i < dim; i += 256) dst[i] = src[i] / scale[i];
-    if (threadIdx.x == 0) {
-        double bc = 0.0;
-        for (int d = 0; d < dim; ++d) bc -= double(src[d]) * double(shift[d]);
-        bias_corr[blockIdx.x] = float(bc);
-    }
-}
-
-__device__ __forceinline__ float block_max_256(float v, float *red) {
-    // exact: max is order-free
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
-    return v;
-}
-
-__device__ __forceinline__ float clamp_round_i8(float v) {
-    // Rust f32::round is half-away-from-zero, like roundf; then clamp(-127, 127)
-    v = roundf(v);
-    return v < -127.0f ? -127.0f : (v > 127.0f ? 127.0f : v);
-}
-
-// turbovec/src/search.rs:2806-2846 build_permute_dot, emitting the weights in
-// the MFMA B-fragment order of the scan.  Plane order (the batched scans, whose
-// decode yields one A operand of low nibbles and one of high nibbles per chunk):
-// for query tile t, chunk c and nibble plane p (0 = low nibble = odd dimension,
-// 1 = high nibble = even dimension) a 1 KiB fragment whose lane (h*32 + n) holds
-// the 16 weights of query n for groups 32c + 16h .. +15.  Split order (k_scan_p4,
-// which decodes the first 8 code bytes of a lane on the vector ALU, four at a
-// time, and looks the other 8 up whole, both levels of a byte side by side):
-// fragment 0 of chunk c holds, in lane (h*32 + n), for e = 0..7, the plane-p
-// weight of group 32c + 16h + e at byte 8*(e/4) + 4p + e%4; fragment 1 the
-// plane-p weight of group 32c + 16h + 8 + e at byte 2e + p.
-__device__ __forceinline__ size_t wfrag_offset(int g, int n, int plane, bool split) {
-    const size_t lane16 = size_t(((g & 31) >> 4) * 32 + n) * 16;
-    if (split) {
-        const int e = g & 7;
-        const int at = (g & 8) ? 2 * e + plane : 8 * (e >> 2) + 4 * plane + (e & 3);
-        return size_t(g >> 5) * 2048 + size_t((g & 15) >> 3) * 1024 + lane16 + size_t(at);
-    }
-    return size_t(g >> 5) * 2048 + size_t(plane) * 1024 + lane16 + size_t(g & 15);
-}
-
-__global__ __launch_bounds__(256) void k_build_p(const float *__restrict__ qcal,
-                                                 const float *__restrict__ bias_corr,
-                                                 uint8_t *__restrict__ wfrag, float *__restrict__ qscale,
-                                                 float *__restrict__ qbias, int dim, int G, int nch, float cs,
-                                                 size_t nq, bool split) {
-    __shared__ float red[4];
-    const size_t qi = blockIdx.x;
-    const size_t tile = qi / kQTile;
-    const int n = int(qi % kQTile);
-    uint8_t *base = wfrag + tile * size_t(nch) * 2048;
-    const int t = threadIdx.x;
-    if (qi >= nq) {  // padding query of the last tile: zero weights
-        for (int g = t; g < nch * 32; g += 256) {
-            base[wfrag_offset(g, n, 0, split)] = 0;
-            base[wfrag_offset(g, n, 1, split)] = 0;
-        }
-        if (t == 0) { qscale[qi] = 0.0f; qbias[qi] = 0.0f; }
-        return;
-    }
-    const float *q = qcal + qi * size_t(dim);
-    float m = 0.0f;
-    for (int d = t; d < dim; d += 256) m = fmaxf(m, fabsf(q[d]));
-    const float qmax = block_max_256(m, red);
-    float qs = qmax / 127.0f, inv_qs;
-    if (qs >= FLT_MIN) inv_qs = 1.0f / qs; else { qs = 1.0f; inv_qs = 1.0f; }
-    for (int g = t; g < nch * 32; g += 256) {
-        int8_t lo = 0, hi = 0;
-        if (g < G) {
-            lo = int8_t(clamp_round_i8(q[2 * g + 1] * inv_qs));
-            hi = int8_t(clamp_round_i8(q[2 * g] * inv_qs));
-        }
-        base[wfrag_offset(g, n, 0, split)] = uint8_t(lo);
-        base[wfrag_offset(g, n, 1, split)] = uint8_t(hi);
-    }
-    if (t == 0) {
-        qscale[qi] = cs * qs;
-        qbias[qi] = 0.0f + (bias_corr ? bias_corr[qi] : 0.0f);
-    }
-}
-
-// Query preparation of the permute-dot mode in one launch, one workgroup per query: k_rotate,
-// k_calibrate and k_build_p back to back with the row kept in LDS between them -- the same
-// operations on the same values in the same order, so the same bits (search.rs:3237-3269).  A
-// single query's preparation is three dependent launches' worth of latency otherwise.
-__global__ __launch_bounds__(256) void k_prep_p(const float *__restrict__ q, const float *__restrict__ signs,
-                                                const uint32_t *__restrict__ perms, int dim, int block,
-                                                float inv_sqrt_block, const float *__restrict__ shift,
-                                                const float *__restrict__ scale, uint8_t *__restrict__ wfrag,
-                                                float *__restrict__ qscale, float *__restrict__ qbias, int G, int nch,
-                                                float cs, size_t nq, bool split, uint64_t *stamp) {
-    extern __shared__ float rot_lds[];
-    __shared__ float red[4];
-    __shared__ float s_bias;
-    float *A = rot_lds;
-    float *B = rot_lds + dim;
-    const size_t qi = blockIdx.x;
-    const size_t tile = qi / kQTile;
-    const int n = int(qi % kQTile);
-    uint8_t *base = wfrag + tile * size_t(nch) * 2048;
-    const int t = threadIdx.x;
-    if (qi >= nq) {  // padding query of the last tile: zero weights
-        for (int g = t; g < nch * 32; g += 256) {
-            base[wfrag_offset(g, n, 0, split)] = 0;
-            base[wfrag_offset(g, n, 1, split)] = 0;
-        }
-        if (t == 0) { qscale[qi] = 0.0f; qbias[qi] = 0.0f; }
-        return;
-    }
-    const float *src = q + qi * size_t(dim);
-    for (int i = t; i < dim; i += 256) A[i] = src[perms[i]] * signs[i];
-    __syncthreads();
-    for (int len = 1; len < block; len <<= 1) {
-        for (int p = t; p < dim / 2; p += 256) {
-            const int j = 2 * p - (p & (len - 1));
-            const float a = A[j], b = A[j + len];
-            A[j] = a + b;
-            A[j + len] = a - b;
-        }
-        __syncthreads();
-    }
-    for (int i = t; i < dim; i += 256) B[i] = (A[perms[dim + i]] * inv_sqrt_block) * signs[dim + i];
-    __syncthreads();
-    for (int len = 1; len < block; len <<= 1) {
-        for (int p = t; p < dim / 2; p += 256) {
-            const int j = 2 * p - (p & (len - 1));
-            const float a = B[j], b = B[j + len];
-            B[j] = a + b;
-            B[j + len] = a - b;
-        }
-        __syncthreads();
-    }
-    // the rotated row (k_rotate's output) into A; with a TQ+ pair, k_calibrate's output over it
-    for (int i = t; i < dim; i += 256) A[i] = B[i] * inv_sqrt_block;
-    __syncthreads();
-    if (scale != nullptr) {
-        if (t == 0) {
-            double bc = 0.0;
-            for (int d = 0; d < dim; ++d) bc -= double(A[d]) * double(shift[d]);
-            s_bias = float(bc);
-        }
-        __syncthreads();
-        for (int i = t; i < dim; i += 256) A[i] = A[i] / scale[i];
-        __syncthreads();
-    }
-    const float *qc = A;
-    float m = 0.0f;
-    for (int d = t; d < dim; d += 256) m = fmaxf(m, fabsf(qc[d]));
-    const float qmax = block_max_256(m, red);
-    float qs = qmax / 127.0f, inv_qs;
-    if (qs >= FLT_MIN) inv_qs = 1.0f / qs; else { qs = 1.0f; inv_qs = 1.0f; }
-    for (int g = t; g < nch * 32; g += 256) {
-        int8_t lo = 0, hi = 0;
-        if (g < G) {
-            lo = int8_t(clamp_round_i8(qc[2 * g + 1] * inv_qs));
-            hi = int8_t(clamp_round_i8(qc[2 * g] * inv_qs));
-        }
-        base[wfrag_offset(g, n, 0, split)] = uint8_t(lo);
-        base[wfrag_offset(g, n, 1, split)] = uint8_t(hi);
-    }
-    if (t == 0) {
-        qscale[qi] = cs * qs;
-        qbias[qi] = 0.0f + (scale != nullptr ? s_bias : 0.0f);
-        if (stamp != nullptr && qi == 0) *stamp = wall_clock64();
-    }
-}
-
-// turbovec/src/search.rs:2856-2994 build_query_neon_lut_from_slice.  Output per
-// query: nch*32 rows of 32 bytes, row g = [16 entries indexed by the byte's HIGH
-// nibble (the group's first dimensions) | 16 entries indexed by the LOW nibble];
-// rows of padding groups are zero.
-template <int BITS>
-__device__ __forceinline__ float lut_entry(const float *q, const float *cen, int dim_start, int sub, int nv) {
-    constexpr int cpb = 8 / BITS, cpn = cpb / 2;
-    constexpr unsigned code_mask = (1u << BITS) - 1;
-    float s = 0.0f;
-#pragma unroll
-    for (int c = 0; c < cpn; ++c) {
-        const int sh = (cpn - 1 - c) * BITS;
-        const unsigned code = (unsigned(nv) >> sh) & code_mask;
-        s += q[dim_start + sub * cpn + c] * cen[code];
-    }
-    return s;
-}
-
-template <int BITS>
-__global__ __launch_bounds__(256) void k_build_lut(const float *__restrict__ qcal,
-                                                   const float *__restrict__ bias_corr,
-                                                   const float *__restrict__ centroids,
-                                                   uint8_t *__restrict__ lut, float *__restrict__ qscale,
-                                                   float *__restrict__ qbias, int dim, int G, int nch, size_t nq) {
-    extern __shared__ float lut_lds[];  // mins: 2*G floats
-    __shared__ float red[4];
-    __shared__ float cen[16];
-    constexpr int cpb = 8 / BITS;
-    const size_t qi = blockIdx.x;
-    uint8_t *dst = lut + qi * size_t(nch) * 1024;
-    const int t = threadIdx.x;
-    if (qi >= nq) {
-        for (int i = t; i < nch * 256; i += 256) reinterpret_cast<uint32_t *>(dst)[i] = 0;
-        if (t == 0) { qscale[qi] = 0.0f; qbias[qi] = 0.0f; }
-        return;
-    }
-    if (t < (1 << BITS)) cen[t] = centroids[t];
-    __syncthreads();
-    const float *q = qcal + qi * size_t(dim);
-    float span = 0.0f;
-    for (int g = t; g < G; g += 256) {
-        for (int sub = 0; sub < 2; ++sub) {
-            float mn = FLT_MAX, mx = -FLT_MAX;
-            for (int nv = 0; nv < 16; ++nv) {
-                const float s = lut_entry<BITS>(q, cen, g * cpb, sub, nv);
-                if (s < mn) mn = s;
-                if (s > mx) mx = s;
-            }
-            lut_lds[2 * g + sub] = mn;
-            span = fmaxf(span, mx - mn);
-        }
-    }
-    const float max_span = block_max_256(span, red);  // also orders the lut_lds writes
-    float scale = max_span > 0.0f ? max_span / 127.0f : 1.0f, inv_scale;
-    if (scale >= FLT_MIN) inv_scale = 1.0f / scale; else { scale = 1.0f; inv_scale = 1.0f; }
-    if (t == 0) {
-        float bias = 0.0f;  // sequential f32 sum over groups, inner add first (search.rs:2910)
-        for (int g = 0; g < G; ++g) bias += lut_lds[2 * g] + lut_lds[2 * g + 1];
-        qscale[qi] = scale;
-        qbias[qi] = bias + (bias_corr ? bias_corr[qi] : 0.0f);
-    }
-    for (int g = t; g < nch * 32; g += 256) {
-        uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (g < G) {
-            for (int sub = 0; sub < 2; ++sub) {
-                const float mn = lut_lds[2 * g + sub];
-                for (int nv = 0; nv < 16; ++nv) {
-                    float v = roundf((lut_entry<BITS>(q, cen, g * cpb, sub, nv) - mn) * inv_scale);
-                    v = v < 0.0f ? 0.0f : (v > 127.0f ? 127.0f : v);
-                    w[sub * 4 + nv / 4] |= uint32_t(uint8_t(v)) << (8 * (nv & 3));
-                }
-            }
-        }
-        uint4 *o = reinterpret_cast<uint4 *>(dst + size_t(g) * 32);
-        o[0] = make_uint4(w[0], w[1], w[2], w[3]);
-        o[1] = make_uint4(w[4], w[5], w[6], w[7]);
-    }
-}
-
-// ===========================================================================
 // Scan, score mode P: 4-bit codes -> int8 codebook levels -> i8 MFMA against
 // int8 query weights (turbovec/src/search.rs:1392-1567 computes the same
 // integers with vpdpbusd).  acc = sum_d w[d] * level[code[d]], exact in i32;
@@ -1529,65 +1227,6 @@ static hipError_t allow_lds(K kernel, size_t bytes) {
     if (bytes <= 48 * 1024) return hipSuccess;
     return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(bytes));
-}
-
-hipError_t launch_rotate(const float *d_q, float *d_out, const float *d_signs, const uint32_t *d_perms, int dim,
-                         int block, float inv_sqrt_block, size_t nq, hipStream_t s) {
-    if (nq == 0) return hipSuccess;
-    const size_t lds = size_t(2) * dim * sizeof(float);
-    hipError_t e = allow_lds(k_rotate, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_rotate, dim3(unsigned(nq)), dim3(256), lds, s, d_q, d_out, d_signs, d_perms, dim, block,
-                       inv_sqrt_block);
-    return hipGetLastError();
-}
-
-hipError_t launch_calibrate(const float *d_qrot, float *d_qcal, float *d_bias_corr, const float *d_shift,
-                            const float *d_scale, int dim, size_t nq, hipStream_t s) {
-    if (nq == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_calibrate, dim3(unsigned(nq)), dim3(256), 0, s, d_qrot, d_qcal, d_bias_corr, d_shift,
-                       d_scale, dim);
-    return hipGetLastError();
-}
-
-hipError_t launch_build_p(const float *d_qcal, const float *d_bias_corr, uint8_t *d_wfrag, float *d_qscale,
-                          float *d_qbias, int dim, int G, int nch, float cs, size_t nq, size_t nq_padded,
-                          bool split, hipStream_t s) {
-    if (nq_padded == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_build_p, dim3(unsigned(nq_padded)), dim3(256), 0, s, d_qcal, d_bias_corr, d_wfrag, d_qscale,
-                       d_qbias, dim, G, nch, cs, nq, split);
-    return hipGetLastError();
-}
-
-hipError_t launch_prep_p(const float *d_q, const float *d_signs, const uint32_t *d_perms, int dim, int block,
-                         float inv_sqrt_block, const float *d_shift, const float *d_scale, uint8_t *d_wfrag,
-                         float *d_qscale, float *d_qbias, int G, int nch, float cs, size_t nq, size_t nq_padded, bool split,
-                         uint64_t *stamp, hipStream_t s) {
-    if (nq_padded == 0) return hipSuccess;
-    const size_t lds = size_t(2) * dim * sizeof(float);
-    hipError_t e = allow_lds(k_prep_p, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_prep_p, dim3(unsigned(nq_padded)), dim3(256), lds, s, d_q, d_signs, d_perms, dim, block,
-                       inv_sqrt_block, d_shift, d_scale, d_wfrag, d_qscale, d_qbias, G, nch, cs, nq, split, stamp);
-    return hipGetLastError();
-}
-
-hipError_t launch_build_lut(const float *d_qcal, const float *d_bias_corr, const float *d_centroids, uint8_t *d_lut,
-                            float *d_qscale, float *d_qbias, int dim, int bits, int G, int nch, size_t nq,
-                            size_t nq_padded, hipStream_t s) {
-    if (nq_padded == 0) return hipSuccess;
-    const size_t lds = size_t(2) * G * sizeof(float);
-    hipError_t e = hipSuccess;
-#define TV_LAUNCH_LUT(B)                                                                                         \
-    e = allow_lds(k_build_lut<B>, lds);                                                                          \
-    if (e != hipSuccess) return e;                                                                               \
-    hipLaunchKernelGGL(k_build_lut<B>, dim3(unsigned(nq_padded)), dim3(256), lds, s, d_qcal, d_bias_corr,        \
-                       d_centroids, d_lut, d_qscale, d_qbias, dim, G, nch, nq)
-    if (bits == 2) { TV_LAUNCH_LUT(2); }
-    else if (bits == 3) { TV_LAUNCH_LUT(3); }
-    else { TV_LAUNCH_LUT(4); }
-#undef TV_LAUNCH_LUT
-    return hipGetLastError();
 }
 
 static constexpr size_t kLdsBudget = 160 * 1024;

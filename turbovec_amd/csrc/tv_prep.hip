@@ -1,0 +1,307 @@
+// HIP kernels that prepare queries: rotation, TQ+ inverse, int8 weights (permute-dot) or byte tables (u8 LUT),
+// one workgroup per query and one launch for all of it.
+//
+// Compiled with -ffp-contract=off like every file here: the operations, their operands and their order
+// are the reference's (turbovec/src/search.rs:3237-3269), so the bits are.
+#include "tv_device.h"
+#include "tv_internal.h"
+
+#include <cfloat>
+
+namespace tv {
+
+constexpr int kPrepThreads = 256;
+constexpr int kPrepPiece = 1024;     // products of the bias chain in LDS at a time
+
+struct PrepArgs {
+    const float *q, *signs;
+    const uint32_t *perms;
+    const float *shift, *scale;     // null without a TQ+ pair
+    float inv_sqrt_block;
+    int dim, log_block, G, nch;
+    uint8_t *tables;
+    float *qscale, *qbias;
+    float *rot_out;                 // when given: the rotated (and calibrated) rows
+    size_t nq;
+    uint64_t *stamp;
+};
+
+// A row lies in LDS with eight floats of padding after every 64: lanes whose elements are 64 apart in
+// groups of eight then spread over the banks.
+__host__ __device__ constexpr int prep_at(int j) { return j + (j >> 6) * 8; }
+__host__ __device__ constexpr int prep_floats(int dim) { return prep_at(dim - 1) + 1 + 7 - (prep_at(dim - 1) & 7); }
+
+// R butterfly stages from stride 2^S on over the whole row.
+template <int R>
+__device__ __forceinline__ void prep_pass(float *buf, int dim, int S) {
+    constexpr int N = 1 << R;
+    for (int g = threadIdx.x; g < dim / N; g += kPrepThreads) {
+        const int base = ((g >> S) << (S + R)) + (g & ((1 << S) - 1));
+        float v[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = buf[prep_at(base + (e << S))];
+        butterflies<R>(v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) buf[prep_at(base + (e << S))] = v[e];
+    }
+    __syncthreads();
+}
+
+// turbovec/src/rotation.rs:265-320 (apply_with_scratch) + :964-982 (wht_block_scalar): the rotated row, still
+// to be multiplied by inv_sqrt_block, at B's padded places.  Three stages at a time through registers: a
+// barrier per pass instead of one per stage (1536 dimensions: 8 instead of 20, which was most of the time
+// one query's preparation took).
+__device__ __forceinline__ void rotate_row(const float *src, const float *signs, const uint32_t *perms, int dim, int log_block,
+                                           float inv_sqrt_block, float *A, float *B) {
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+        float *buf = round == 0 ? A : B;
+        for (int g = threadIdx.x; g < dim / 8; g += kPrepThreads) {
+            const uint4 *p4 = reinterpret_cast<const uint4 *>(perms + size_t(round) * dim + 8 * g);
+            const float4 *s4 = reinterpret_cast<const float4 *>(signs + size_t(round) * dim + 8 * g);
+            const uint4 pa = p4[0], pb = p4[1];
+            const float4 sa = s4[0], sb = s4[1];
+            const uint32_t p[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+            const float s[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)      // the 1/sqrt(B) scale of round 0 rides the round-1 gather: (x * inv) * sign
+                v[e] = round == 0 ? src[p[e]] * s[e] : (A[prep_at(int(p[e]))] * inv_sqrt_block) * s[e];
+            butterflies<3>(v);
+            float4 *dst = reinterpret_cast<float4 *>(buf + prep_at(8 * g));
+            dst[0] = float4{v[0], v[1], v[2], v[3]};
+            dst[1] = float4{v[4], v[5], v[6], v[7]};
+        }
+        __syncthreads();
+        for (int S = 3; S < log_block; S += 3) {
+            if (log_block - S >= 3) prep_pass<3>(buf, dim, S);
+            else if (log_block - S == 2) prep_pass<2>(buf, dim, S);
+            else prep_pass<1>(buf, dim, S);
+        }
+    }
+}
+
+// The rotated row at A[0 .. dim), its TQ+ inverse where there is a pair (search.rs:3154-3186
+// calibrate_queries), and the pair's bias term (for thread 0).  The f64 sum is sequential over d: one
+// thread adds, all threads form its products (one thread doing both, from global memory, took 57 us for
+// 1000 dimensions).
+__device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs &a, float *A, float *B, double *prod) {
+    const int t = threadIdx.x, dim = a.dim;
+    rotate_row(src, a.signs, a.perms, dim, a.log_block, a.inv_sqrt_block, A, B);
+    float bias = 0.0f;
+    if (a.scale != nullptr) {
+        double bc = 0.0;
+        for (int d0 = 0; d0 < dim; d0 += kPrepPiece) {
+            const int m = min(kPrepPiece, dim - d0);      // (a multiple of eight, as dim is)
+            for (int i = t; i < m; i += kPrepThreads) prod[i] = double(B[prep_at(d0 + i)] * a.inv_sqrt_block) * double(a.shift[d0 + i]);
+            __syncthreads();
+            if (t == 0) {
+                for (int i = 0; i < m; i += 8) {
+                    double p[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) p[e] = prod[i + e];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) bc -= p[e];
+                }
+            }
+            __syncthreads();
+        }
+        bias = float(bc);
+    }
+    for (int i = t; i < dim; i += kPrepThreads) {
+        float x = B[prep_at(i)] * a.inv_sqrt_block;
+        if (a.scale != nullptr) x = x / a.scale[i];
+        A[i] = x;
+        if (a.rot_out != nullptr) a.rot_out[size_t(blockIdx.x) * dim + i] = x;
+    }
+    __syncthreads();
+    return bias;
+}
+
+__device__ __forceinline__ float block_max_256(float v, float *red) {
+    // exact: max is order-free
+    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    __syncthreads();
+    return v;
+}
+
+__device__ __forceinline__ float clamp_round_i8(float v) {
+    // Rust f32::round is half-away-from-zero, like roundf; then clamp(-127, 127)
+    v = roundf(v);
+    return v < -127.0f ? -127.0f : (v > 127.0f ? 127.0f : v);
+}
+
+// turbovec/src/search.rs:2806-2846 build_permute_dot, emitting the weights in
+// the MFMA B-fragment order of the scan.  Plane order (the batched scans, whose
+// decode yields one A operand of low nibbles and one of high nibbles per chunk):
+// for query tile t, chunk c and nibble plane p (0 = low nibble = odd dimension,
+// 1 = high nibble = even dimension) a 1 KiB fragment whose lane (h*32 + n) holds
+// the 16 weights of query n for groups 32c + 16h .. +15.  Split order (k_scan_p4,
+// which decodes the first 8 code bytes of a lane on the vector ALU, four at a
+// time, and looks the other 8 up whole, both levels of a byte side by side):
+// fragment 0 of chunk c holds, in lane (h*32 + n), for e = 0..7, the plane-p
+// weight of group 32c + 16h + e at byte 8*(e/4) + 4p + e%4; fragment 1 the
+// plane-p weight of group 32c + 16h + 8 + e at byte 2e + p.
+__device__ __forceinline__ size_t wfrag_offset(int g, int n, int plane, bool split) {
+    const size_t lane16 = size_t(((g & 31) >> 4) * 32 + n) * 16;
+    if (split) {
+        const int e = g & 7;
+        const int at = (g & 8) ? 2 * e + plane : 8 * (e >> 2) + 4 * plane + (e & 3);
+        return size_t(g >> 5) * 2048 + size_t((g & 15) >> 3) * 1024 + lane16 + size_t(at);
+    }
+    return size_t(g >> 5) * 2048 + size_t(plane) * 1024 + lane16 + size_t(g & 15);
+}
+
+__global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split) {
+    extern __shared__ __align__(16) float prep_lds[];
+    __shared__ float red[4];
+    __shared__ __align__(16) double prod[kPrepPiece];
+    float *A = prep_lds, *B = prep_lds + prep_floats(a.dim);
+    const size_t qi = blockIdx.x;
+    const int n = int(qi % kQTile), t = threadIdx.x;
+    uint8_t *base = a.tables + qi / kQTile * size_t(a.nch) * 2048;
+    if (qi >= a.nq) {  // padding query of the last tile: zero weights
+        for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+            base[wfrag_offset(g, n, 0, split)] = 0;
+            base[wfrag_offset(g, n, 1, split)] = 0;
+        }
+        if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
+        return;
+    }
+    const float bias = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod);
+    float m = 0.0f;
+    for (int d = t; d < a.dim; d += kPrepThreads) m = fmaxf(m, fabsf(A[d]));
+    const float qmax = block_max_256(m, red);
+    float qs = qmax / 127.0f, inv_qs;
+    if (qs >= FLT_MIN) inv_qs = 1.0f / qs; else { qs = 1.0f; inv_qs = 1.0f; }
+    for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+        int8_t lo = 0, hi = 0;
+        if (g < a.G) {
+            lo = int8_t(clamp_round_i8(A[2 * g + 1] * inv_qs));
+            hi = int8_t(clamp_round_i8(A[2 * g] * inv_qs));
+        }
+        base[wfrag_offset(g, n, 0, split)] = uint8_t(lo);
+        base[wfrag_offset(g, n, 1, split)] = uint8_t(hi);
+    }
+    if (t == 0) {
+        a.qscale[qi] = cs * qs;
+        a.qbias[qi] = 0.0f + bias;
+        if (a.stamp != nullptr && qi == 0) *a.stamp = wall_clock64();
+    }
+}
+
+// turbovec/src/search.rs:2856-2994 build_query_neon_lut_from_slice.  Output per
+// query: nch*32 rows of 32 bytes, row g = [16 entries indexed by the byte's HIGH
+// nibble (the group's first dimensions) | 16 entries indexed by the LOW nibble];
+// rows of padding groups are zero.
+template <int BITS>
+__device__ __forceinline__ float lut_entry(const float *q, const float *cen, int dim_start, int sub, int nv) {
+    constexpr int cpb = 8 / BITS, cpn = cpb / 2;
+    constexpr unsigned code_mask = (1u << BITS) - 1;
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < cpn; ++c) {
+        const int sh = (cpn - 1 - c) * BITS;
+        const unsigned code = (unsigned(nv) >> sh) & code_mask;
+        s += q[dim_start + sub * cpn + c] * cen[code];
+    }
+    return s;
+}
+
+template <int BITS>
+__global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
+    extern __shared__ __align__(16) float prep_lds[];
+    __shared__ float red[4];
+    __shared__ __align__(16) double prod[kPrepPiece];
+    __shared__ float cen[16];
+    constexpr int cpb = 8 / BITS;
+    float *A = prep_lds, *B = prep_lds + prep_floats(a.dim);
+    const size_t qi = blockIdx.x;
+    uint8_t *dst = a.tables + qi * size_t(a.nch) * 1024;
+    const int t = threadIdx.x, G = a.G;
+    if (qi >= a.nq) {
+        for (int i = t; i < a.nch * 64; i += kPrepThreads) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
+        if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
+        return;
+    }
+    if (t < (1 << BITS)) cen[t] = centroids[t];
+    const float bias_corr = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod);
+    float *mins = B;                                   // two per group: at most a row's length
+    float span = 0.0f;
+    for (int g = t; g < G; g += kPrepThreads) {
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            float mn = FLT_MAX, mx = -FLT_MAX;
+#pragma unroll
+            for (int nv = 0; nv < 16; ++nv) {
+                const float s = lut_entry<BITS>(A, cen, g * cpb, sub, nv);
+                if (s < mn) mn = s;
+                if (s > mx) mx = s;
+            }
+            mins[2 * g + sub] = mn;
+            span = fmaxf(span, mx - mn);
+        }
+    }
+    const float max_span = block_max_256(span, red);   // also orders the writes of mins
+    float scale = max_span > 0.0f ? max_span / 127.0f : 1.0f, inv_scale;
+    if (scale >= FLT_MIN) inv_scale = 1.0f / scale; else { scale = 1.0f; inv_scale = 1.0f; }
+    if (t == 0) {
+        float bias = 0.0f;  // sequential f32 sum over groups, inner add first (search.rs:2910)
+        int g = 0;
+        for (; g + 8 <= G; g += 8) {
+            float4 m[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = reinterpret_cast<const float4 *>(mins + 2 * g)[e];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { bias += m[e].x + m[e].y; bias += m[e].z + m[e].w; }
+        }
+        for (; g < G; ++g) bias += mins[2 * g] + mins[2 * g + 1];
+        a.qscale[qi] = scale;
+        a.qbias[qi] = bias + bias_corr;      // (+0 without a pair, search.rs:3176-3185)
+    }
+    for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+        uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (g < G) {
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub) {
+                const float mn = mins[2 * g + sub];
+#pragma unroll
+                for (int nv = 0; nv < 16; ++nv) {
+                    float v = roundf((lut_entry<BITS>(A, cen, g * cpb, sub, nv) - mn) * inv_scale);
+                    v = v < 0.0f ? 0.0f : (v > 127.0f ? 127.0f : v);
+                    w[sub * 4 + nv / 4] |= uint32_t(uint8_t(v)) << (8 * (nv & 3));
+                }
+            }
+        }
+        uint4 *o = reinterpret_cast<uint4 *>(dst + size_t(g) * 32);
+        o[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        o[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+}
+
+static_assert(size_t(2) * prep_floats(16384) * sizeof(float) + kPrepPiece * sizeof(double) + 128 <= 160 * 1024,
+              "the longest row the index accepts must fit a workgroup's LDS");
+
+hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s) {
+    if (nq_padded == 0) return hipSuccess;
+    PrepArgs a;
+    a.q = r.q; a.signs = r.signs; a.perms = r.perms; a.shift = r.shift; a.scale = r.scale;
+    a.inv_sqrt_block = r.inv_sqrt_block;
+    a.dim = g.dim; a.log_block = __builtin_ctz(unsigned(r.block)); a.G = g.G; a.nch = g.nch;
+    a.tables = r.tables; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
+    a.nq = nq; a.stamp = r.stamp;
+    const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
+    auto launch = [&](auto kernel, auto... rest) -> hipError_t {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nq_padded)), dim3(kPrepThreads), lds, s, a, rest...);
+        return hipGetLastError();
+    };
+    if (r.permute_dot) return launch(k_prep_p, r.cs, r.split);
+    return g.bits == 2 ? launch(k_prep_lut<2>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3>, r.centroids) : launch(k_prep_lut<4>, r.centroids);
+}
+
+}  // namespace tv
