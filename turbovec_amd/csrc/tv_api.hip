@@ -2,6 +2,7 @@
 #include "../../include/turbovec_hip.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -9,6 +10,8 @@
 #include <cstdlib>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "tv_internal.h"
@@ -75,6 +78,97 @@ int scratch_address(int device, void **out) {
     return TV_OK;
 }
 
+// f(lo, hi) over [0, n) in parts of at least min_part on up to eight threads, the calling one among them.
+// (What cannot start a thread runs on this one.)
+constexpr size_t kMaxParts = 8;
+template <typename F>
+void in_parts(size_t n, size_t min_part, const F &f) {
+    const size_t parts = std::min<size_t>({kMaxParts, std::max<size_t>(1, std::thread::hardware_concurrency()), std::max<size_t>(1, n / min_part)});
+    const size_t per = (n + parts - 1) / parts;
+    std::thread started[kMaxParts];
+    for (size_t i = 1; i < parts; ++i) {
+        const size_t lo = std::min(i * per, n), hi = std::min(lo + per, n);
+        try {
+            started[i] = std::thread([&f, lo, hi] { f(lo, hi); });
+        } catch (const std::system_error &) {
+            f(lo, hi);
+        }
+    }
+    f(0, std::min(per, n));
+    for (std::thread &t : started) if (t.joinable()) t.join();
+}
+// Faults in fresh host memory about to be overwritten, several threads at once: a copy into 77 MB that
+// nothing has touched yet takes 18 ms, into touched memory 4.4.
+void touch_pages(uint8_t *p, size_t n) {
+    in_parts(n, size_t(4) << 20, [p](size_t lo, size_t hi) {
+        for (size_t i = lo; i < hi; i += 4096) *static_cast<volatile uint8_t *>(p + i) = 0;
+    });
+}
+constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
+
+// ---- device memory of indexes ----------------------------------------------------------------
+// Large blocks that an index gives up (it grew, or went) are kept for the next one, per device: up to
+// kPoolBytes, handed on only to requests they exceed by a quarter at most, and given back when the last
+// index of the device goes or an allocation fails.  An index built by adds allocates 2.6 times its size on
+// the way; fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
+// 1536 rows in four adds: 4 ms a build while cleared memory lasts, 22.8 ms after).
+constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
+struct DevicePool {
+    std::mutex mu;
+    std::vector<std::pair<size_t, void *>> blocks;
+    size_t held = 0, indexes = 0;
+    void drop() {          // mu held
+        for (auto &b : blocks) (void)hipFree(b.second);
+        blocks.clear();
+        held = 0;
+    }
+};
+DevicePool g_pool[kMaxDevices];
+
+// `device` is current.  *got: what the block holds.
+hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
+    DevicePool &pool = g_pool[device];
+    std::lock_guard<std::mutex> lock(pool.mu);
+    size_t best = pool.blocks.size();
+    for (size_t i = 0; i < pool.blocks.size(); ++i) {
+        const size_t have = pool.blocks[i].first;
+        if (have >= bytes && have <= bytes + bytes / 4 && (best == pool.blocks.size() || have < pool.blocks[best].first)) best = i;
+    }
+    if (best < pool.blocks.size()) {
+        *out = pool.blocks[best].second;
+        *got = pool.blocks[best].first;
+        pool.held -= *got;
+        pool.blocks[best] = pool.blocks.back();
+        pool.blocks.pop_back();
+        return hipSuccess;
+    }
+    *got = bytes;
+    hipError_t e = hipMalloc(out, bytes);
+    if (e != hipSuccess && !pool.blocks.empty()) {
+        (void)hipGetLastError();
+        pool.drop();
+        e = hipMalloc(out, bytes);
+    }
+    return e;
+}
+// Waits for the whole device first, as hipFree does: an index's memory is visible outside it
+// (tv_index_device_ptrs), and work of other streams may still be reading.
+hipError_t device_free(int device, void *p, size_t bytes) {
+    if (p == nullptr) return hipSuccess;
+    DevicePool &pool = g_pool[device];
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (bytes >= kPoolMinBytes && pool.held + bytes <= kPoolBytes && pool.indexes != 0) {
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipSuccess) return e;
+            pool.blocks.emplace_back(bytes, p);
+            pool.held += bytes;
+            return hipSuccess;
+        }
+    }
+    return hipFree(p);
+}
+
 int ensure_workspace(tv_index *ix, size_t bytes) {
     if (bytes <= ix->ws_bytes) return TV_OK;
     if (ix->ws_fixed) {   // the caller lent a buffer of fixed size: never replaced
@@ -82,19 +176,17 @@ int ensure_workspace(tv_index *ix, size_t bytes) {
                        std::to_string(ix->ws_bytes);
         return TV_ERR_BAD_ARGUMENT;
     }
-    if (ix->ws) { TV_HIP(hipFree(ix->ws)); ix->ws = nullptr; ix->ws_bytes = 0; }
+    if (ix->ws) { TV_HIP(device_free(ix->device, ix->ws, ix->ws_bytes)); ix->ws = nullptr; ix->ws_bytes = 0; }
     bytes = round_up(bytes + bytes / 4, size_t(1) << 20);
-    TV_HIP(hipMalloc(&ix->ws, bytes));
-    ix->ws_bytes = bytes;
+    TV_HIP(device_alloc(ix->device, bytes, &ix->ws, &ix->ws_bytes));
     return TV_OK;
 }
 
 int ensure_io(tv_index *ix, size_t bytes) {
     if (bytes <= ix->io_bytes) return TV_OK;
-    if (ix->io) { TV_HIP(hipFree(ix->io)); ix->io = nullptr; ix->io_bytes = 0; }
+    if (ix->io) { TV_HIP(device_free(ix->device, ix->io, ix->io_bytes)); ix->io = nullptr; ix->io_bytes = 0; }
     bytes = round_up(bytes + bytes / 4, size_t(1) << 16);
-    TV_HIP(hipMalloc(&ix->io, bytes));
-    ix->io_bytes = bytes;
+    TV_HIP(device_alloc(ix->device, bytes, &ix->io, &ix->io_bytes));
     return TV_OK;
 }
 
@@ -106,12 +198,13 @@ int ensure_capacity(tv_index *ix, size_t n_vectors) {
     uint8_t *codes = nullptr;
     float *scales = nullptr;
     const size_t bb = ix->geo.block_bytes();
-    TV_HIP(hipMalloc(reinterpret_cast<void **>(&codes), cap * bb));
+    size_t codes_bytes = 0, scales_bytes = 0;
+    TV_HIP(device_alloc(ix->device, cap * bb, reinterpret_cast<void **>(&codes), &codes_bytes));
     {
-        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&scales), cap * tv::kVecBlock * sizeof(float));
+        const hipError_t e = device_alloc(ix->device, cap * tv::kVecBlock * sizeof(float), reinterpret_cast<void **>(&scales), &scales_bytes);
         if (e != hipSuccess) {
-            (void)hipFree(codes);
-            return fail_hip(e, "hipMalloc(scales)");
+            (void)device_free(ix->device, codes, codes_bytes);
+            return fail_hip(e, "device_alloc(scales)");
         }
     }
     const size_t old_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
@@ -125,10 +218,12 @@ int ensure_capacity(tv_index *ix, size_t n_vectors) {
                               hipMemcpyDeviceToDevice, ix->stream));
     }
     TV_HIP(hipStreamSynchronize(ix->stream));
-    if (ix->d_codes) TV_HIP(hipFree(ix->d_codes));
-    if (ix->d_scales) TV_HIP(hipFree(ix->d_scales));
+    TV_HIP(device_free(ix->device, ix->d_codes, ix->codes_bytes));
+    TV_HIP(device_free(ix->device, ix->d_scales, ix->scales_bytes));
     ix->d_codes = codes;
     ix->d_scales = scales;
+    ix->codes_bytes = codes_bytes;
+    ix->scales_bytes = scales_bytes;
     ix->cap_blocks = cap;
     return TV_OK;
 }
@@ -1110,12 +1205,14 @@ bool compatible(const tv_request &a, const tv_request &b) {
 // with their next call (they were all released at the same moment and are a few microseconds of
 // host code away from asking again).  Only after a batch that did merge calls.
 constexpr auto kGatherWait = std::chrono::microseconds(300);
+constexpr auto kContendedWait = std::chrono::microseconds(20);
 
 int search_merged(tv_index *ix, tv_request &r) {
     std::vector<tv_request *> batch;
     {
         std::unique_lock<std::mutex> reg(ix->waiting_mu);
         ix->waiting.push_back(&r);
+        bool had_to_wait = false;
         ix->waiting_cv.notify_all();       // a serving caller gathering its batch may be waiting for this one
         for (;;) {
             if (r.done) {                  // served by another caller's launch
@@ -1123,6 +1220,7 @@ int search_merged(tv_index *ix, tv_request &r) {
                 return r.rc;
             }
             if (!ix->serving) break;
+            had_to_wait = true;
             ix->waiting_cv.wait(reg);
         }
         ix->serving = true;
@@ -1133,6 +1231,15 @@ int search_merged(tv_index *ix, tv_request &r) {
             const auto deadline = std::chrono::steady_clock::now() + kGatherWait;
             while (ix->waiting.size() < ix->last_batch_calls)
                 if (ix->waiting_cv.wait_until(reg, deadline) == std::cv_status::timeout) break;
+        }
+        // A caller that had to wait is not the only one in a hurry: a search of a small index takes less time
+        // than the callers' own work between two calls, and without a moment's pause they would line up one
+        // behind the other.
+        const auto pause = std::chrono::steady_clock::now() + kContendedWait;
+        while (had_to_wait && ix->waiting.size() < 2 && std::chrono::steady_clock::now() < pause) {
+            reg.unlock();
+            std::this_thread::yield();
+            reg.lock();
         }
         // this call first, then the compatible ones in order of arrival, up to the batch limit
         batch.push_back(&r);
@@ -1202,10 +1309,15 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         g_last_error = "no HIP device with that ordinal";
         return TV_ERR_NO_DEVICE;
     }
+    if (device >= kMaxDevices) { g_last_error = "device ordinal beyond the scratch table"; return TV_ERR_NO_DEVICE; }
     TV_HIP(hipSetDevice(device));
     tv_index *ix = new (std::nothrow) tv_index();
     if (!ix) return TV_ERR_BAD_ARGUMENT;
     ix->device = device;
+    {
+        std::lock_guard<std::mutex> lock(g_pool[device].mu);
+        ++g_pool[device].indexes;
+    }
     ix->geo.dim = dim;
     ix->geo.bits = bits;
     ix->geo.G = dim / (8 / bits);
@@ -1272,8 +1384,17 @@ int tv_index_destroy(tv_index *ix) {
     (void)hipSetDevice(ix->device);
     if (ix->stream) (void)hipStreamSynchronize(ix->stream);
     void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
-                    ix->d_codes, ix->d_scales, ix->ws, ix->io, ix->d_tau_open};
+                    ix->d_tau_open};
+    (void)device_free(ix->device, ix->d_codes, ix->codes_bytes);
+    (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
+    (void)device_free(ix->device, ix->ws, ix->ws_bytes);
+    (void)device_free(ix->device, ix->io, ix->io_bytes);
     for (void *p : ptrs) if (p) (void)hipFree(p);
+    {
+        DevicePool &pool = g_pool[ix->device];
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (--pool.indexes == 0) pool.drop();
+    }
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
     if (ix->events_ready)
         for (int i = 0; i < tv::kTimedLaunches; ++i) {
@@ -1545,7 +1666,7 @@ static int download_seq_locked(tv_index *ix, uint8_t *seq_out, float *scales_out
         if (rc != TV_OK) return rc;
         for (size_t b0 = 0; b0 < n_blocks; b0 += slice_blocks) {
             const size_t nb = std::min(slice_blocks, n_blocks - b0);
-            TV_HIP(tv::launch_native_to_seq(ix->d_codes, static_cast<uint8_t *>(ix->ws), g, b0, nb, ix->stream));
+            TV_HIP(tv::launch_native_to_seq(ix->d_codes, static_cast<uint8_t *>(ix->ws), g, b0, nb, seq_block, nullptr, ix->stream));
             TV_HIP(hipMemcpyAsync(seq_out + b0 * seq_block, ix->ws, nb * seq_block, hipMemcpyDeviceToHost, ix->stream));
             TV_HIP(hipStreamSynchronize(ix->stream));
         }
@@ -1570,13 +1691,30 @@ int tv_index_bits(const tv_index *ix) { return ix ? ix->geo.bits : 0; }
 
 int tv_validate_queries(const float *queries, size_t len, int dim, size_t *bad_index) {
     if (dim <= 0 || len % size_t(dim) != 0) return TV_ERR_QUERY_BUFFER_NOT_MULTIPLE_OF_DIM;
-    for (size_t i = 0; i < len; ++i) {
-        if (!(std::fabs(queries[i]) < 1e16f)) {
-            if (bad_index) *bad_index = i;
-            return TV_ERR_INVALID_QUERY_VALUE;
+    // A run of values at a time, without a branch per value: |x| < 1e16 and not NaN is an unsigned compare
+    // of the bits without the sign.
+    constexpr size_t kRun = 4096;
+    std::atomic<size_t> first_bad{len};
+    in_parts(len, size_t(1) << 20, [&](size_t lo, size_t hi) {
+        for (size_t r = lo; r < hi && r < first_bad.load(std::memory_order_relaxed); r += kRun) {
+            const size_t e = std::min(r + kRun, hi);
+            uint32_t any = 0;
+            for (size_t i = r; i < e; ++i) {
+                uint32_t u;
+                std::memcpy(&u, queries + i, 4);
+                any |= uint32_t(int32_t((u & 0x7fffffffu) >= kTooLargeBits));
+            }
+            if (!any) continue;
+            size_t i = r;
+            while (std::fabs(queries[i]) < 1e16f) ++i;
+            size_t seen = first_bad.load();
+            while (i < seen && !first_bad.compare_exchange_weak(seen, i)) {}
+            return;
         }
-    }
-    return TV_OK;
+    });
+    if (first_bad.load() == len) return TV_OK;
+    if (bad_index) *bad_index = first_bad.load();
+    return TV_ERR_INVALID_QUERY_VALUE;
 }
 
 int tv_pack_mask(const uint8_t *mask_bytes, size_t n, uint64_t *words_out, size_t *n_allowed) {
@@ -1806,6 +1944,37 @@ int tv_index_to_bytes(const tv_index *cix, const uint64_t *ids, int format, uint
     if (!out) return TV_OK;
     if (cap < *len) return TV_ERR_BAD_ARGUMENT;
     const size_t nb = (n + 31) / 32;
+    if (format == 7) {
+        // The device writes the units as the image holds them and they are copied straight to their place;
+        // only the rows behind the last whole block pass through the host's composer.
+        TV_HIP(hipSetDevice(ix->device));
+        const tv::Geometry &g = ix->geo;
+        const size_t whole = n / 32, unit = tv::snapshot_unit_len(g.dim, g.bits, kind), seq_block = size_t(g.G) * 32;
+        std::vector<uint8_t> tail_seq(whole < nb ? seq_block : 0);
+        float tail_scales[32] = {0};
+        const size_t slice = std::max<size_t>(1, (size_t(256) << 20) / unit);
+        int rc = ensure_workspace(ix, std::max(std::min(whole, slice) * unit, seq_block) + 256);
+        if (rc != TV_OK) return rc;
+        if (whole < nb) {
+            TV_HIP(tv::launch_native_to_seq(ix->d_codes, static_cast<uint8_t *>(ix->ws), g, whole, 1, seq_block, nullptr, ix->stream));
+            TV_HIP(hipMemcpyAsync(tail_seq.data(), ix->ws, seq_block, hipMemcpyDeviceToHost, ix->stream));
+            TV_HIP(hipMemcpyAsync(tail_scales, ix->d_scales + whole * 32, (n - whole * 32) * sizeof(float), hipMemcpyDeviceToHost, ix->stream));
+            TV_HIP(hipStreamSynchronize(ix->stream));
+        }
+        const tv::SnapshotParts s{kind, g.dim, g.bits, ix->cb.boundaries.data(), ix->cb.centroids.data(), n_calib,
+                                  ix->tq_shift.data(), ix->tq_scale.data(), tail_seq.data(), n, tail_scales, ids ? ids + whole * 32 : nullptr};
+        uint8_t *units = out + tv::snapshot_head(s, out);
+        touch_pages(units, whole * unit);
+        for (size_t b0 = 0; b0 < whole; b0 += slice) {
+            const size_t m = std::min(slice, whole - b0);
+            TV_HIP(tv::launch_native_to_seq(ix->d_codes, static_cast<uint8_t *>(ix->ws), g, b0, m, unit, ix->d_scales, ix->stream));
+            TV_HIP(hipMemcpyAsync(units + b0 * unit, ix->ws, m * unit, hipMemcpyDeviceToHost, ix->stream));
+            TV_HIP(hipStreamSynchronize(ix->stream));
+        }
+        if (ids)
+            for (size_t b = 0; b < whole; ++b) std::memcpy(units + (b + 1) * unit - 32 * sizeof(uint64_t), ids + b * 32, 32 * sizeof(uint64_t));
+        return TV_OK;
+    }
     std::vector<uint8_t> seq(nb * size_t(ix->geo.G) * 32);
     std::vector<float> scales(n);
     int rc = download_seq_locked(ix, seq.data(), scales.data());

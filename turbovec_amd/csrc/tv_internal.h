@@ -78,8 +78,9 @@ struct ScanArgs {
 // ---- launchers (tv_kernels.hip) ----
 hipError_t launch_seq_to_native(const uint8_t *d_seq, uint8_t *d_native, const Geometry &g, size_t first_block,
                                 size_t n_blocks, hipStream_t s);
+// d_seq takes a block's codes every block_bytes, and behind them its row scales when d_scales is given.
 hipError_t launch_native_to_seq(const uint8_t *d_native, uint8_t *d_seq, const Geometry &g, size_t first_block,
-                                size_t n_blocks, hipStream_t s);
+                                size_t n_blocks, size_t block_bytes, const float *d_scales, hipStream_t s);
 hipError_t launch_append_rows(const uint8_t *d_rows, uint8_t *d_native, const Geometry &g, size_t old_n,
                               size_t n_new, hipStream_t s);
 hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const float *d_signs,
@@ -225,6 +226,7 @@ struct tv_index {
 
     uint8_t *d_codes = nullptr;
     float *d_scales = nullptr;
+    size_t codes_bytes = 0, scales_bytes = 0;   // allocated
     size_t cap_blocks = 0;
     size_t n = 0;
 

@@ -46,7 +46,8 @@ __global__ __launch_bounds__(256) void k_seq_to_native(const uint8_t *__restrict
 }
 
 __global__ __launch_bounds__(256) void k_native_to_seq(const uint8_t *__restrict__ nat, uint8_t *__restrict__ seq,
-                                                       int G, int nch, size_t first_block) {
+                                                       int G, int nch, size_t first_block, size_t block_bytes,
+                                                       const float *__restrict__ scales) {
     __shared__ uint8_t tile[32 * 36];
     const size_t b = first_block + blockIdx.x / nch;
     const int c = blockIdx.x % nch;
@@ -62,9 +63,12 @@ __global__ __launch_bounds__(256) void k_native_to_seq(const uint8_t *__restrict
         const int gl = t >> 3, l4 = (t & 7) * 4;
         const int g = c * 32 + gl;
         if (g < G)
-            *reinterpret_cast<uint32_t *>(seq + ((b - first_block) * size_t(G) + g) * 32 + l4) =
+            *reinterpret_cast<uint32_t *>(seq + (b - first_block) * block_bytes + size_t(g) * 32 + l4) =
                 *reinterpret_cast<const uint32_t *>(tile + gl * 36 + l4);
     }
+    // (a snapshot's unit: the block's row scales behind its codes)
+    if (scales != nullptr && c == 0 && t < 32)
+        *reinterpret_cast<float *>(seq + (b - first_block) * block_bytes + size_t(G) * 32 + t * 4) = scales[b * 32 + t];
 }
 
 __device__ __forceinline__ size_t native_byte_index(size_t v, int g, int nch) {
@@ -1185,10 +1189,10 @@ hipError_t launch_seq_to_native(const uint8_t *d_seq, uint8_t *d_native, const G
 }
 
 hipError_t launch_native_to_seq(const uint8_t *d_native, uint8_t *d_seq, const Geometry &g, size_t first_block,
-                                size_t n_blocks, hipStream_t s) {
+                                size_t n_blocks, size_t block_bytes, const float *d_scales, hipStream_t s) {
     if (n_blocks == 0) return hipSuccess;
     hipLaunchKernelGGL(k_native_to_seq, dim3(unsigned(n_blocks * g.nch)), dim3(256), 0, s, d_native, d_seq, g.G,
-                       g.nch, first_block);
+                       g.nch, first_block, block_bytes, d_scales);
     return hipGetLastError();
 }
 

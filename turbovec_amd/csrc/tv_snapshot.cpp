@@ -152,8 +152,9 @@ static void compose_flat6(const SnapshotParts &s, uint8_t *out) {
     std::memcpy(p, v.data(), v.size());
 }
 
-void snapshot_compose(int format, const SnapshotParts &s, uint8_t *out) {
-    if (format == 6) { compose_flat6(s, out); return; }
+size_t snapshot_unit_len(int dim, int bits, int kind) { return Geo{kind, dim, bits, 0}.unit_len(); }
+
+size_t snapshot_head(const SnapshotParts &s, uint8_t *out) {
     const Geo g{s.kind, s.dim, s.bits, s.n_calib};
     const size_t G = g.row_bytes();
     std::vector<uint8_t> sb;
@@ -174,12 +175,11 @@ void snapshot_compose(int format, const SnapshotParts &s, uint8_t *out) {
     std::vector<uint8_t> h;
     put_u64(h, 0);                     // generation
     put_u64(h, uint64_t(s.n));
-    const size_t n_tail = s.n % kBlock, first_tail = s.n - n_tail;
+    const size_t n_tail = s.n % kBlock;
     for (size_t k = 0; k < n_tail; ++k) {
-        const size_t r = first_tail + k, b = r / kBlock, lane = r % kBlock;
-        for (size_t gi = 0; gi < G; ++gi) h.push_back(s.seq[(b * G + gi) * kBlock + lane]);   // lib.rs:1648-1675
-        put_f32(h, s.scales[r]);
-        if (s.kind == 1) put_u64(h, s.ids[r]);
+        for (size_t gi = 0; gi < G; ++gi) h.push_back(s.seq[gi * kBlock + k]);   // lib.rs:1648-1675
+        put_f32(h, s.scales[k]);
+        if (s.kind == 1) put_u64(h, s.ids[k]);
     }
     put_u32(h, 0);                     // no pending op groups
     put_u32(h, 0);                     // delta: nothing materialised,
@@ -197,7 +197,19 @@ void snapshot_compose(int format, const SnapshotParts &s, uint8_t *out) {
     std::memcpy(p, sb.data(), sb.size()); p += sb.size();
     std::memset(p, 0, 2 * g.hdr_len());
     std::memcpy(p, h.data(), h.size()); p += 2 * g.hdr_len();
-    const size_t n_blocks = s.n / kBlock;
+    return size_t(p - out);
+}
+
+void snapshot_compose(int format, const SnapshotParts &s, uint8_t *out) {
+    if (format == 6) { compose_flat6(s, out); return; }
+    const size_t G = Geo{s.kind, s.dim, s.bits, s.n_calib}.row_bytes(), n_blocks = s.n / kBlock;
+    SnapshotParts tail = s;
+    if (s.n % kBlock != 0) {
+        tail.seq = s.seq + n_blocks * G * kBlock;
+        tail.scales = s.scales + n_blocks * kBlock;
+        if (s.kind == 1) tail.ids = s.ids + n_blocks * kBlock;
+    }
+    uint8_t *p = out + snapshot_head(tail, out);
     for (size_t b = 0; b < n_blocks; ++b) {
         std::memcpy(p, s.seq + b * G * kBlock, G * kBlock); p += G * kBlock;
         for (size_t l = 0; l < kBlock; ++l) { uint32_t x; std::memcpy(&x, &s.scales[b * kBlock + l], 4); for (int i = 0; i < 4; ++i) *p++ = uint8_t(x >> (8 * i)); }

@@ -28,6 +28,10 @@ struct SnapshotInfo {
 
 uint32_t snapshot_crc32(const uint8_t *p, size_t n);
 size_t snapshot_len(int format, int dim, int bits, int kind, size_t n_calib, size_t n);
+// Everything of a TV7 image before its units (one per whole block); s.seq, s.scales and s.ids hold the rows
+// behind the last whole block only.  Returns its length.
+size_t snapshot_head(const SnapshotParts &s, uint8_t *out);
+size_t snapshot_unit_len(int dim, int bits, int kind);    // codes, scales, ids of one block
 void snapshot_compose(int format, const SnapshotParts &s, uint8_t *out);
 std::string snapshot_parse(const uint8_t *bytes, size_t len, SnapshotInfo &info);
 void snapshot_extract(const uint8_t *bytes, const SnapshotInfo &info, uint8_t *seq, float *scales, uint64_t *ids);
