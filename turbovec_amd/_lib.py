@@ -124,6 +124,12 @@ def ptr(a):
     return None if a is None else a.ctypes.data
 
 
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.argtypes, _new_bytes.restype = [C.c_char_p, C.c_ssize_t], C.py_object
+_bytes_at = C.pythonapi.PyBytes_AsString
+_bytes_at.argtypes, _bytes_at.restype = [C.py_object], C.c_void_p
+
+
 class NativeIndex:
     """Thin owner of a tv_index handle (device-resident codes, scales and tables)."""
 
@@ -220,9 +226,11 @@ class NativeIndex:
             idp = ptr(ids)
         n = C.c_size_t(0)
         check(lib().tv_index_to_bytes(self.h, idp, format, None, 0, C.byref(n)))
-        out = np.zeros(n.value, np.uint8)
-        check(lib().tv_index_to_bytes(self.h, idp, format, ptr(out), n.value, C.byref(n)))
-        return out.tobytes()
+        # the image is written into the bytes object itself, before anyone else has seen it
+        out = _new_bytes(None, n.value)
+        check(lib().tv_index_to_bytes(self.h, idp, format, _bytes_at(out), n.value, C.byref(n)))
+        assert n.value == len(out), "the index changed while its image was taken"
+        return out
 
     @classmethod
     def from_bytes(cls, data, device=0):

@@ -28,7 +28,6 @@ import numpy as np
 from . import _lib as T
 
 _MAX_DIM = 16384            # turbovec/src/lib.rs:101
-_MAX_INPUT_MAGNITUDE = 1e16  # turbovec/src/lib.rs:109
 
 
 def _desc(obj):
@@ -60,9 +59,11 @@ def _size(name, obj):
 
 def _check_values(name, arr, what):
     """turbovec/src/lib.rs:1363-1380, encode.rs:76-83: every value finite and |x| < 1e16."""
-    ok = np.abs(arr) < _MAX_INPUT_MAGNITUDE          # NaN compares false
-    if not ok.all():
-        r, c = np.argwhere(~ok)[0]
+    if arr.size == 0:
+        return
+    rc, bad = T.validate_queries(arr, arr.shape[1])
+    if rc == T.ERR_INVALID_QUERY_VALUE:
+        r, c = divmod(bad, arr.shape[1])
         raise ValueError(f"{what} {r} has a non-finite or out-of-range value at coordinate {c} "
                          f"(must be finite with magnitude < 1e16)")
 
@@ -157,9 +158,13 @@ class TurboQuantIndex:
             raise ValueError(f"vector dim {v.shape[1]} does not match index dim {self.dim}")
         if len(v) == 0:
             return
-        _check_values("vectors", v, "vector")
         with self._lock:
-            self._ix.add(v)
+            try:
+                self._ix.add(v)                         # checks every value before it changes anything
+            except T.TurbovecHipError as e:
+                if e.status == T.ERR_INVALID_QUERY_VALUE:
+                    _check_values("vectors", v, "vector")
+                raise
 
     def swap_remove(self, idx):
         """Move the last vector into slot idx; returns the slot it came from (lib.rs:2864-3028)."""
@@ -239,6 +244,7 @@ class IdMapIndex:
     def __init__(self, dim, bit_width=4, device=0):
         self._inner = TurboQuantIndex(dim, bit_width, device)
         self._slot_to_id = []            # id_map.rs:181: slot -> external id
+        self._ids = None                 # the same as an array; None after a change
         self._id_to_slot = {}
 
     @property
@@ -252,12 +258,18 @@ class IdMapIndex:
     def __len__(self):
         return len(self._slot_to_id)
 
+    def _id_array(self):
+        """Slot -> id as an array; the inner lock is held."""
+        if self._ids is None:
+            self._ids = np.asarray(self._slot_to_id, np.uint64)
+        return self._ids
+
     def prepare(self):
         return None
 
     def to_bytes(self):
         with self._inner._lock:
-            return self._inner._ix.to_bytes(ids=np.asarray(self._slot_to_id, np.uint64))
+            return self._inner._ix.to_bytes(ids=self._id_array())
 
     @classmethod
     def from_bytes(cls, data, device=0):
@@ -265,6 +277,7 @@ class IdMapIndex:
         self = cls.__new__(cls)
         self._inner = TurboQuantIndex._adopt(native, None)
         self._slot_to_id = ids.tolist()
+        self._ids = ids
         self._id_to_slot = {x: i for i, x in enumerate(self._slot_to_id)}
         if len(self._id_to_slot) != len(self._slot_to_id):
             raise OSError("image holds duplicate ids")
@@ -312,6 +325,7 @@ class IdMapIndex:
         with self._inner._lock:
             self._inner.add(v)
             base = len(self._slot_to_id)
+            self._ids = None
             for off, x in enumerate(ids.tolist()):
                 self._id_to_slot[x] = base + off
                 self._slot_to_id.append(x)
@@ -329,6 +343,7 @@ class IdMapIndex:
             last = len(self._slot_to_id) - 1
             self._inner.swap_remove(slot)
             del self._id_to_slot[v]
+            self._ids = None
             if slot != last:
                 moved = self._slot_to_id[last]
                 self._slot_to_id[slot] = moved
@@ -365,6 +380,5 @@ class IdMapIndex:
                 mask_bytes = np.zeros(len(self._slot_to_id), np.uint8)      # duplicates collapse here
                 mask_bytes[[self._id_to_slot[x] for x in allow]] = 1
             scores, slots = self._inner._search_locked(q, k, mask_bytes)
-            table = np.asarray(self._slot_to_id, np.uint64)
-            ids = table[slots] if slots.size else np.zeros(slots.shape, np.uint64)
+            ids = self._id_array()[slots] if slots.size else np.zeros(slots.shape, np.uint64)
             return scores, ids
