@@ -8,9 +8,9 @@
 #include <cstdio>
 #include <cstring>
 #include <cstdlib>
+#include <exception>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -90,7 +90,7 @@ void in_parts(size_t n, size_t min_part, const F &f) {
         const size_t lo = std::min(i * per, n), hi = std::min(lo + per, n);
         try {
             started[i] = std::thread([&f, lo, hi] { f(lo, hi); });
-        } catch (const std::system_error &) {
+        } catch (const std::exception &) {     // no thread, or no memory for one
             f(lo, hi);
         }
     }
@@ -125,7 +125,7 @@ struct DevicePool {
 };
 DevicePool g_pool[kMaxDevices];
 
-// `device` is current.  *got: what the block holds.
+// `device` is current.  *got: what the block holds, 0 on failure.
 hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
     DevicePool &pool = g_pool[device];
     std::lock_guard<std::mutex> lock(pool.mu);
@@ -142,13 +142,14 @@ hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
         pool.blocks.pop_back();
         return hipSuccess;
     }
-    *got = bytes;
     hipError_t e = hipMalloc(out, bytes);
     if (e != hipSuccess && !pool.blocks.empty()) {
         (void)hipGetLastError();
         pool.drop();
         e = hipMalloc(out, bytes);
     }
+    *got = e == hipSuccess ? bytes : 0;     // (callers keep it: a size without a block would pass for one)
+    if (e != hipSuccess) (void)hipGetLastError();     // reported by this call, not by a later launch
     return e;
 }
 // Waits for the whole device first, as hipFree does: an index's memory is visible outside it
