@@ -127,3 +127,31 @@ def test_noalloc_takes_no_device_memory(T):
     ix.search_dev(q.data_ptr(), 96, 10, s.data_ptr(), i.data_ptr())      # the regular entry point does grow it
     assert ix.workspace_bytes()[0] > ws0[0]
     ix.close()
+
+
+@pytest.mark.parametrize("dim,bits", [(512, 2), (1536, 2), (1000, 3)])
+def test_noalloc_limit_of_table_batches_follows_the_sixteen_query_passes(T, dim, bits):
+    """What the array must hold for a batch of u8-LUT queries grows by steps of 16 queries (their candidate
+    segments alone are 16 x 256 x 64 keys), and the largest batch that fits gives tv_search_dev's results."""
+    ix, gen = build(T, 66_000, dim, bits, seed=dim)      # 2063 blocks: the matrix-unit scan serves these batches
+    q = torch.randn(1024, dim, device="cuda:0", generator=gen)
+    s = torch.zeros(1024, 10, device="cuda:0")
+    i = torch.zeros(1024, 10, dtype=torch.int64, device="cuda:0")
+    torch.cuda.synchronize()
+
+    def wants(nq):
+        """0 when the call is taken, else the bytes it may need."""
+        try:
+            ix.search_dev_noalloc(q.data_ptr(), nq, 10, s.data_ptr(), i.data_ptr())
+        except T.TurbovecHipError as e:
+            assert e.status == T.ERR_BAD_ARGUMENT
+            return int(str(e).split("may need ")[1].split()[0])
+        return 0
+
+    assert wants(1024) - wants(1008) >= 16 * 256 * 64 * 8
+    lo, hi = 17, 1008                                   # taken, refused
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if wants(mid) else (mid, hi)
+    assert_same(both(ix, q[:lo].contiguous(), 10))
+    ix.close()

@@ -285,7 +285,7 @@ int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCOR
 constexpr size_t kMxMinPairs = 4096;
 bool lut_mx_serves(const tv_index *ix, size_t cq) {
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
-    return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && cq > size_t(tv::kLut16Queries) &&
+    return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && !ix->no_lut_mx && cq > size_t(tv::kLut16Queries) &&
            n_blocks * tiles >= kMxMinPairs;
 }
 bool lut16_serves(const tv_index *ix) {
@@ -1756,13 +1756,21 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     const size_t k_eff = std::min(std::min(k, ix->n), n_allowed);
     // What the search may carve, worst case: the sampled path's chunk, and the exact path a query
     // falls back to when its candidates overflow.  Refused up front when that exceeds the array.
-    size_t need = 0;
-    if (k_eff != 0 && nq != 0) {
+    // (The matrix-unit scan of u8-LUT batches pads a call to 32 queries, the sixteen-query passes to 16:
+    // a call that only the smaller working set fits takes those.)
+    auto carve = [&] {
+        if (k_eff == 0 || nq == 0) return size_t(0);
         const size_t cq = std::min(nq, kChunkQueries);    // the exact path works in chunks of this size throughout
-        need = robust_need(ix, cq, k_eff);
-        if (k_eff <= size_t(tv::kMaxSampledK) && !ix->force_robust) need = std::max(need, sampled_need_worst(ix, nq));
+        const size_t exact = robust_need(ix, cq, k_eff);
+        return k_eff <= size_t(tv::kMaxSampledK) && !ix->force_robust ? std::max(exact, sampled_need_worst(ix, nq)) : exact;
+    };
+    size_t need = carve();
+    if (need > kScratchBytes) {
+        ix->no_lut_mx = true;
+        need = carve();
     }
     if (need > kScratchBytes) {
+        ix->no_lut_mx = false;
         g_last_error = "tv_search_dev_noalloc: " + std::to_string(nq) + " queries, k=" + std::to_string(k) + " over " +
                        std::to_string(ix->n) + " rows may need " + std::to_string(need) +
                        " bytes of scratch; the fixed buffer holds " + std::to_string(kScratchBytes) +
@@ -1779,6 +1787,7 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     ix->ws = own_ws;
     ix->ws_bytes = own_bytes;
     ix->ws_fixed = false;
+    ix->no_lut_mx = false;
     return rc;
 }
 

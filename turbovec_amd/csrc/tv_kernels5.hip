@@ -47,7 +47,7 @@ size_t mx_table_bytes(int nch, int bits, size_t nq) {
     return (nq + kQTile - 1) / kQTile * size_t(nch) * size_t(mx_steps(bits == 3 ? 8 : 16)) * 2048;
 }
 
-// The row-major tables of k_build_lut -> B operands.  Piece ((tile, chunk, step j, part p), lane
+// The row-major tables of k_prep_lut -> B operands.  Piece ((tile, chunk, step j, part p), lane
 // (u, n)) is 16 bytes of query 32 tile + n: the 16 lanes-halves p of the A operand meet part p, and
 // of that lane's stored bytes 0..7 half u = 0, 8..15 half u = 1.
 //   16-entry tables: byte-group 16 p + j of the chunk, its high (u = 0) or low (u = 1) nibble's table
