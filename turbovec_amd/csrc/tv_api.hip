@@ -716,7 +716,7 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks)
     const int nch = ix->geo.nch;
     if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide) return false;
     if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > kDirectBlocks) return false;
-    if (tv::pick_lds_bytes(true, nch, k_eff) > tv::kPickLds) return false;
+    if (tv::pick_lds_bytes(nch, k_eff) > tv::kPickLds) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
     if (n_blocks >= 1536 && nch <= 12 && ((nq >= 2 && nq <= 8) || (nq > 32 && nq < 256) || nq > kChunkQueries)) return false;
@@ -768,7 +768,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             } else {
                 TV_HIP(tv::launch_scan_p4_best(a, ix->device, ix->stream));
             }
-            TV_HIP(tv::launch_pick(a, true, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
+            TV_HIP(tv::launch_pick(a, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
                                    timed ? ix->d_stamps + 1 : nullptr, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));

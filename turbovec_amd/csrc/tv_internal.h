@@ -150,9 +150,9 @@ constexpr int kMaxPickK = 128;             // most results k_pick ranks
 constexpr size_t kPickLds = 128 * 1024;    // beside its 17 KiB of fixed buffers
 bool best_serves(int nch);
 hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s);
-size_t pick_lds_bytes(bool mode_p, int nch, size_t k_eff);
-hipError_t launch_pick(const ScanArgs &a, bool mode_p, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow,
-                       uint64_t *stamp, hipStream_t s);
+size_t pick_lds_bytes(int nch, size_t k_eff);
+hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
+                       hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).
 int batched_tiles(int nch);

@@ -202,7 +202,7 @@ struct PickArgs {
 };
 constexpr uint32_t kPickHeld = 16;       // blocks a thread keeps in registers
 
-template <uint32_t T, bool P>
+template <uint32_t T>
 __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     constexpr uint32_t W = T / 64;
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     __shared__ uint32_t blocks[kMaxPickK];
     __shared__ uint32_t n_kept, n_list, s_floor;
     uint64_t *list = reinterpret_cast<uint64_t *>(dyn);                     // rows of the chosen blocks that can still matter
-    uint8_t *wts = dyn + size_t(a.k_eff) * 32 * 8;                          // this query's weights, or its tables
+    uint8_t *wts = dyn + size_t(a.k_eff) * 32 * 8;                          // this query's weights
     const uint32_t qi = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
     const uint32_t k_eff = uint32_t(a.k_eff);
     const uint32_t *best = a.best + size_t(qi) * a.best_stride;
@@ -220,15 +220,10 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     uint32_t v[kPickHeld];
 #pragma unroll
     for (uint32_t e = 0; e < kPickHeld; ++e) v[e] = held && e * T + t < a.n_blocks ? best[e * T + t] : 0u;
-    if (P) {
-        // the tile's weights lie [chunk][fragment][half * 32 + query] in 16-byte pieces; here [chunk][half][fragment]
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
-        for (int i = int(t); i < a.nch * 4; i += int(T))
-            reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
-    } else {
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi) * a.nch * 64;
-        for (int i = int(t); i < a.nch * 64; i += int(T)) reinterpret_cast<uint4 *>(wts)[i] = src[i];
-    }
+    // the tile's weights lie [chunk][fragment][half * 32 + query] in 16-byte pieces; here [chunk][half][fragment]
+    const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
+    for (int i = int(t); i < a.nch * 4; i += int(T))
+        reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
     for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     if (t == 0) { n_kept = 0u; n_list = 0u; s_floor = 0u; }
     auto each = [&](auto &&f) {
@@ -290,46 +285,37 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
             for (int u = 0; u < kBurst; ++u) {
                 if (c0 + u >= a.nch) break;
                 const uint32_t d[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-                if (P) {
-                    const uint4 *wq = reinterpret_cast<const uint4 *>(wts) + ((c0 + u) * 2 + h) * 2;
-                    const uint4 f0 = wq[0], f1 = wq[1];
-                    uint32_t lo[4], hi[4];
+                const uint4 *wq = reinterpret_cast<const uint4 *>(wts) + ((c0 + u) * 2 + h) * 2;
+                const uint4 f0 = wq[0], f1 = wq[1];
+                uint32_t lo[4], hi[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        lo[e] = levels_of(d[e] & 0x0f0f0f0fu, t0, t1, t2, t3);
-                        hi[e] = levels_of((d[e] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3);
-                    }
-                    const uint32_t g0[4] = {f0.x, f0.y, f0.z, f0.w}, g1[4] = {f1.x, f1.y, f1.z, f1.w};
-                    if (a.split) {
-                        // bytes 0..7 as (low, high) dwords of four, bytes 8..15 as (low, high) byte pairs (k_scan_p4)
-                        acc = __builtin_amdgcn_sdot4(int(lo[0]), int(g0[0]), acc, false);
-                        acc = __builtin_amdgcn_sdot4(int(hi[0]), int(g0[1]), acc, false);
-                        acc = __builtin_amdgcn_sdot4(int(lo[1]), int(g0[2]), acc, false);
-                        acc = __builtin_amdgcn_sdot4(int(hi[1]), int(g0[3]), acc, false);
+                for (int e = 0; e < 4; ++e) {
+                    lo[e] = levels_of(d[e] & 0x0f0f0f0fu, t0, t1, t2, t3);
+                    hi[e] = levels_of((d[e] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3);
+                }
+                const uint32_t g0[4] = {f0.x, f0.y, f0.z, f0.w}, g1[4] = {f1.x, f1.y, f1.z, f1.w};
+                if (a.split) {
+                    // bytes 0..7 as (low, high) dwords of four, bytes 8..15 as (low, high) byte pairs (k_scan_p4)
+                    acc = __builtin_amdgcn_sdot4(int(lo[0]), int(g0[0]), acc, false);
+                    acc = __builtin_amdgcn_sdot4(int(hi[0]), int(g0[1]), acc, false);
+                    acc = __builtin_amdgcn_sdot4(int(lo[1]), int(g0[2]), acc, false);
+                    acc = __builtin_amdgcn_sdot4(int(hi[1]), int(g0[3]), acc, false);
 #pragma unroll
-                        for (int e = 2; e < 4; ++e) {
-                            acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x05010400u)), int(g1[2 * e - 4]), acc, false);
-                            acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x07030602u)), int(g1[2 * e - 3]), acc, false);
-                        }
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            acc = __builtin_amdgcn_sdot4(int(lo[e]), int(g0[e]), acc, false);
-                            acc = __builtin_amdgcn_sdot4(int(hi[e]), int(g1[e]), acc, false);
-                        }
+                    for (int e = 2; e < 4; ++e) {
+                        acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x05010400u)), int(g1[2 * e - 4]), acc, false);
+                        acc = __builtin_amdgcn_sdot4(int(__builtin_amdgcn_perm(hi[e], lo[e], 0x07030602u)), int(g1[2 * e - 3]), acc, false);
                     }
                 } else {
-                    const uint8_t *lut = wts + ((c0 + u) * 32 + int(h) * 16) * 32;
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const uint32_t byte = (d[e >> 2] >> (8 * (e & 3))) & 0xffu;
-                        acc += int(lut[e * 32 + (byte >> 4)]) + int(lut[e * 32 + 16 + (byte & 15u)]);
+                    for (int e = 0; e < 4; ++e) {
+                        acc = __builtin_amdgcn_sdot4(int(lo[e]), int(g0[e]), acc, false);
+                        acc = __builtin_amdgcn_sdot4(int(hi[e]), int(g1[e]), acc, false);
                     }
                 }
             }
         }
         acc += __shfl_xor(acc, 32);
-        const float s = P ? fmaf(float(acc), qs, qb) * vs : ((float(acc) * qs) + qb) * vs;
+        const float s = fmaf(float(acc), qs, qb) * vs;
         bool ok = lane < 32u && slot < a.n && s == s;
         if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> (lane & 31u)) & 1u;
         const uint64_t key = sort_key(s, slot);
@@ -374,13 +360,13 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     }
 }
 
-size_t pick_lds_bytes(bool mode_p, int nch, size_t k_eff) { return k_eff * 32 * 8 + size_t(nch) * (mode_p ? 64 : 1024); }
+size_t pick_lds_bytes(int nch, size_t k_eff) { return k_eff * 32 * 8 + size_t(nch) * 64; }
 
-// The scan's arguments say what was scanned; a.tables: the weight tiles (mode P) or the tables query by query.
-hipError_t launch_pick(const ScanArgs &a, bool mode_p, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow,
-                       uint64_t *stamp, hipStream_t s) {
+// The scan's arguments say what was scanned; a.tables: its weight tiles.
+hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
+                       hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
-    const size_t lds = pick_lds_bytes(mode_p, a.nch, size_t(k_eff));
+    const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff));
     if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1) return hipErrorInvalidValue;
     PickArgs p;
     p.best = a.best_out; p.best_stride = a.best_stride; p.n_blocks = a.n_blocks; p.n = a.n;
@@ -396,8 +382,8 @@ hipError_t launch_pick(const ScanArgs &a, bool mode_p, bool split, int k_eff, fl
         return hipGetLastError();
     };
     // few queries leave the chip empty: as many waves as there are blocks to score again
-    if (a.nq_tile <= 256 || a.n_blocks > 256 * kPickHeld) return mode_p ? launch(k_pick<1024, true>, 1024) : launch(k_pick<1024, false>, 1024);
-    return mode_p ? launch(k_pick<256, true>, 256) : launch(k_pick<256, false>, 256);
+    if (a.nq_tile <= 256 || a.n_blocks > 256 * kPickHeld) return launch(k_pick<1024>, 1024);
+    return launch(k_pick<256>, 256);
 }
 
 }  // namespace tv
