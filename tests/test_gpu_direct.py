@@ -64,3 +64,23 @@ def test_ties_and_wild_row_scales(T, oracle, dim, nq):
         ix.set_path(0)
         assert np.array_equal(i, i2) and bits_equal(s, s2)
     ix.close()
+
+
+@pytest.mark.parametrize("k", [3, 10, 60])
+def test_rows_that_score_minus_infinity(T, oracle, k):
+    """Row scales that take most rows' scores beyond the float range: the blocks of the few finite rows hold -infinity
+    too, and rows of other blocks with lower slots tie with it."""
+    dim, n = 64, 96
+    oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=1))
+    q = unit_gaussian(1, dim, seed=2) * np.float32(1e6)
+    ix = to_native(T, oidx)
+    raw = ix.debug_scan(q)[1][0]
+    ix.close()
+    oidx.scales = (np.float32(3e38) * -np.sign(raw)).astype(np.float32)
+    oidx.scales[[40, 41, 50, 60]] = 1.0
+    ix = to_native(T, oidx)
+    s, i = ix.search(q, k)
+    os_, oi = oidx.search(q, k)
+    assert np.isneginf(os_[0, 4:]).all() and np.isfinite(os_[0, :4]).all()
+    assert np.array_equal(i, oi) and bits_equal(s, os_)
+    ix.close()

@@ -83,7 +83,7 @@ __device__ __forceinline__ void sort_unkey(uint64_t key, float &s, uint32_t &idx
     idx = 0x7fffffffu - (lo >> 1);
 }
 
-// The high word of sort_key for a block's best score; 0 where the block has no allowed row.
+// The high word of sort_key for a block's best score; 0 where the block has no allowed row, or none above -infinity.
 __device__ __forceinline__ uint32_t best_word(float s) {
     return s == -__int_as_float(0x7f800000) ? 0u : uint32_t(order_key(s + 0.0f)) ^ 0x80000000u;   // (-0 counts as +0)
 }

@@ -316,14 +316,17 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         }
         acc += __shfl_xor(acc, 32);
         const float s = fmaf(float(acc), qs, qb) * vs;
-        bool ok = lane < 32u && slot < a.n && s == s;
+        // (A score of -infinity does not count here either, as it does not in a block's best word: rows that tie there
+        // with rows of blocks that were not chosen are for the exact path to order.)
+        bool ok = lane < 32u && slot < a.n && s > -__int_as_float(0x7f800000);
         if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> (lane & 31u)) & 1u;
         const uint64_t key = sort_key(s, slot);
         if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
     }
     __syncthreads();
     const uint32_t m = n_list;
-    // (fewer rows than the caller's count of allowed ones promised: the exact path takes the query)
+    // (fewer rows with a score than wanted -- an overstated count of allowed rows, scores of NaN or -infinity: the exact
+    // path takes the query)
     if (t == 0) a.overflow[qi] = m < k_eff ? 2u : 0u;
     if (m < k_eff) return;
     auto each_row = [&](auto &&f) {
