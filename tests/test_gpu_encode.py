@@ -202,3 +202,23 @@ def test_write_and_load(T, tmp_path):
         TurboQuantIndex.load(bad)
     with pytest.raises(OSError):
         TurboQuantIndex.load(pm)                     # an id-map image is not a slot-addressed index
+
+
+@pytest.mark.parametrize("at,value", [(0, np.nan), (4, np.nan), (15, np.nan), (7, np.inf), (6, 0.9)])
+def test_boundaries_in_no_order(T, at, value):
+    """Handed-over centroids that leave boundaries out of order or NaN: a code still is the number of boundaries
+    below the value (encode.rs:600-640)."""
+    dim, n = 64, 200
+    v = unit_gaussian(n, dim, seed=3)
+    ix = T.NativeIndex(dim, 4)
+    centroids = ix.tables()[2]
+    centroids[at] = value
+    ix.set_tables(centroids=centroids)
+    boundaries = ix.tables()[3]
+    ix.add(v)
+    rotated = ix.debug_prepare(v)[0]
+    want = (rotated[:, :, None] > boundaries).sum(axis=-1)
+    seq, _ = ix.download_seq()
+    rows = seq.reshape(-1, dim // 2, 32).transpose(0, 2, 1).reshape(-1, dim // 2)[:n]
+    assert np.array_equal(np.stack([rows >> 4, rows & 15], axis=-1).reshape(n, dim), want)
+    ix.close()

@@ -510,7 +510,8 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
         a.lanes = 8;
         while (a.lanes < 64 && a.lanes * 8 < g.dim) a.lanes *= 2;
         a.row_stride = enc_row_stride(g.dim, a.lanes);
-        a.by_quarters = g.bits == 4 && std::is_sorted(a.bnd, a.bnd + 15);
+        // (each no larger than the next: handed-over centroids may be out of order, or NaN, which is in no order)
+        a.by_quarters = g.bits == 4 && std::adjacent_find(a.bnd, a.bnd + 15, [](float x, float y) { return !(x <= y); }) == a.bnd + 15;
         a.inv_sqrt_block = inv_sqrt_block;
         a.nat = d_native; a.scales = d_scales; a.old_n = old_n; a.n_new = n_new;
         switch ((g.dim / 8 + a.lanes - 1) / a.lanes) {
