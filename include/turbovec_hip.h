@@ -118,7 +118,7 @@ int tv_index_add(tv_index *ix, const float *vectors, size_t n_new);
 int tv_index_calibrate(tv_index *ix, const float *sample, size_t n);
 /* The committed pair: *n_calib is 0 (uncalibrated) or dim; shift/scale may be NULL. */
 int tv_index_get_calibration(const tv_index *ix, float *shift, float *scale, size_t *n_calib);
-/* Same, rows already in device memory (not validated: the caller checked them). */
+/* Same, rows already in device memory, at any address a float may have (not validated: the caller checked them). */
 int tv_index_add_dev(tv_index *ix, const float *d_vectors, size_t n_new);
 /* lib.rs:2864-3028: move the last vector into slot idx, zero the vacated lane. */
 int tv_index_swap_remove(tv_index *ix, size_t idx);

@@ -222,3 +222,24 @@ def test_boundaries_in_no_order(T, at, value):
     rows = seq.reshape(-1, dim // 2, 32).transpose(0, 2, 1).reshape(-1, dim // 2)[:n]
     assert np.array_equal(np.stack([rows >> 4, rows & 15], axis=-1).reshape(n, dim), want)
     ix.close()
+
+
+@pytest.mark.parametrize("dim,bits", [(8, 4), (64, 2), (520, 3), (1536, 4), (4096, 4), (4104, 4)])
+def test_rows_at_any_float_address(T, dim, bits):
+    """Device rows that start 4, 8 and 12 bytes behind a 16-byte boundary."""
+    torch = pytest.importorskip("torch")
+    n = 71
+    v = unit_gaussian(n, dim, seed=dim)
+    want = T.NativeIndex(dim, bits)
+    want.add(v)
+    seq, scales = want.download_seq()
+    want.close()
+    for off in range(4):
+        buf = torch.zeros(n * dim + 4, device="cuda:0")
+        buf[off:off + n * dim] = torch.from_numpy(v).to("cuda:0").ravel()
+        torch.cuda.synchronize()
+        ix = T.NativeIndex(dim, bits)
+        ix.add_dev(buf.data_ptr() + 4 * off, n)
+        seq2, scales2 = ix.download_seq()
+        assert np.array_equal(seq2, seq) and bits_equal(scales2, scales), off
+        ix.close()

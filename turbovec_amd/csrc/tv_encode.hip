@@ -183,6 +183,10 @@ bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint
     return true;
 }
 
+// Sixteen bytes of the caller's rows: a row starts where the caller's pointer says, so four-byte alignment is all
+// that is known (the load is the same 16-byte one).
+typedef float RowPiece __attribute__((ext_vector_type(4), aligned(4)));
+
 struct EncodeRowsArgs {
     const float *vecs;
     const uint32_t *packed;   // dim entries (encode_pack_tables)
@@ -232,15 +236,15 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
     if (t < 4) s_quarter[t] = float4{a.bnd[4 * t], a.bnd[4 * t + 1], a.bnd[4 * t + 2], 0.0f};
 
     const size_t n_groups = (a.n_new + R - 1) / R;
-    float4 pre[NG][2];
+    RowPiece pre[NG][2];
     auto fetch = [&](size_t grp) {
         const size_t rr = grp * R + r;
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
             const int g = l + i * L;
-            pre[i][0] = pre[i][1] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+            pre[i][0] = pre[i][1] = RowPiece{0.0f, 0.0f, 0.0f, 0.0f};
             if (rr < a.n_new && g < ng) {
-                const float4 *src = reinterpret_cast<const float4 *>(a.vecs + rr * size_t(dim)) + 2 * g;
+                const RowPiece *src = reinterpret_cast<const RowPiece *>(a.vecs + rr * size_t(dim)) + 2 * g;
                 pre[i][0] = src[0];
                 pre[i][1] = src[1];
             }
@@ -304,8 +308,8 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
             const int g = l + i * L;
             if (g < ng) {
                 float4 *dst = reinterpret_cast<float4 *>(row + enc_at(8 * g));
-                dst[0] = pre[i][0];
-                dst[1] = pre[i][1];
+                dst[0] = float4{pre[i][0].x, pre[i][0].y, pre[i][0].z, pre[i][0].w};
+                dst[1] = float4{pre[i][1].x, pre[i][1].y, pre[i][1].z, pre[i][1].w};
             }
         }
         __syncthreads();
