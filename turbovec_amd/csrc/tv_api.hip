@@ -1699,15 +1699,17 @@ int tv_validate_queries(const float *queries, size_t len, int dim, size_t *bad_i
     in_parts(len, size_t(1) << 20, [&](size_t lo, size_t hi) {
         for (size_t r = lo; r < hi && r < first_bad.load(std::memory_order_relaxed); r += kRun) {
             const size_t e = std::min(r + kRun, hi);
-            uint32_t any = 0;
-            for (size_t i = r; i < e; ++i) {
+            auto bad = [&](size_t i) {
                 uint32_t u;
                 std::memcpy(&u, queries + i, 4);
-                any |= uint32_t(int32_t((u & 0x7fffffffu) >= kTooLargeBits));
-            }
+                return (u & 0x7fffffffu) >= kTooLargeBits;
+            };
+            uint32_t any = 0;
+            for (size_t i = r; i < e; ++i) any |= uint32_t(bad(i));
             if (!any) continue;
             size_t i = r;
-            while (std::fabs(queries[i]) < 1e16f) ++i;
+            while (i < e && !bad(i)) ++i;
+            if (i == e) continue;      // (the caller's array: another thread has overwritten the value since)
             size_t seen = first_bad.load();
             while (i < seen && !first_bad.compare_exchange_weak(seen, i)) {}
             return;
