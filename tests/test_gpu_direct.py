@@ -84,3 +84,14 @@ def test_rows_that_score_minus_infinity(T, oracle, k):
     assert np.isneginf(os_[0, 4:]).all() and np.isfinite(os_[0, :4]).all()
     assert np.array_equal(i, oi) and bits_equal(s, os_)
     ix.close()
+
+
+@pytest.mark.parametrize("mode,nq,launches", [("L_CLASSIC", 1024, 64), ("L_CLASSIC", 80, 5), ("L_SCALAR", 40, 40), ("L_U32", 1024, 1)])
+def test_every_launch_of_the_timed_scan_counts(T, mode, nq, launches):
+    ix = T.NativeIndex(64, 2)
+    ix.set_score_mode(getattr(T, "SCORE_" + mode))
+    ix.add(unit_gaussian(70_000, 64, seed=5))
+    ix.search(unit_gaussian(nq, 64, seed=6), 10)
+    assert len(ix.sampling_plan(nq, 10)[0]) == 2      # a level before the full scan: timed between stamps
+    assert ix.last_scan_ms()[1] == launches
+    ix.close()

@@ -966,8 +966,10 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                         }
                         if (timed) TV_HIP(hipEventRecord(ix->ev_stop[launch_no], ix->stream));
                     }
-                    if (last && timed_pass) stamped = steps.size() > 1;
-                    if (last && timed_pass) n_timed = std::min<size_t>(launch_no, size_t(kMaxTimedTiles));
+                    if (last && timed_pass) {      // (two stamps enclose every launch, events the first ones only)
+                        stamped = steps.size() > 1;
+                        n_timed = stamped ? launch_no : std::min<size_t>(launch_no, size_t(kMaxTimedTiles));
+                    }
                     // the first final pass may hand raised floors to a repeated one; the repeated pass
                     // sends what still does not fit to the exact path
                     TV_HIP(tv::launch_final(d_cand, d_cnt, uint32_t(n_seg), uint32_t(seg_stride), int(k_eff), int(k_floor),
