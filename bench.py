@@ -10,8 +10,8 @@ i.i.d. Gaussian rows (seed 0) generated on the device and encoded there by the
 library's own ingest kernel, in 100k-row chunks.
 
 Prints ONE JSON line.  `roofline` prices the dominant kernel (the code scan) by
-its mean launch duration, measured with HIP events on the library's own stream
-inside the timed region.  A 1024-query chunk of this workload is one launch of
+its mean launch duration, measured with device clock stamps (HIP events where no
+launch comes before the scan) on the library's own stream inside the timed region.  A 1024-query chunk of this workload is one launch of
 the wide permute-dot kernel, which reads the codes once for all 1024 queries and
 is bound by the matrix unit: algorithmic operations per launch = 2 * queries *
 vectors * dim int8 multiply-adds (reported in the TFLOP/s field; they are

@@ -224,9 +224,13 @@ int tv_debug_scan(tv_index *ix, const float *queries, size_t nq, int32_t *acc_ou
  * query scale and bias of the active score mode (any may be NULL). */
 int tv_debug_prepare(tv_index *ix, const float *queries, size_t nq,
                      float *q_rot_out, float *scale_out, float *bias_out);
-/* Duration in milliseconds of the scan kernel launches of the most recent
- * tv_search* call on this index, measured with HIP events on its stream, and
- * how many launches that was. */
+/* Duration in milliseconds of the full scans of the most recent tv_search* call
+ * on this index (of its first chunk of queries, or the first one of each 8192)
+ * and how many launches they were.  Where another launch of the call comes
+ * before the full scan, the duration is the span between two readings of the
+ * device clock -- as that launch ends, and as the selection behind the scan
+ * starts -- and the gaps between the launches count; a scan from open floors
+ * and the exact path are measured with HIP events around the first 32 launches. */
 int tv_last_scan_ms(const tv_index *ix, float *ms, int *launches);
 /* Queries one full-scan launch of the last search served (a full launch of a large batch). */
 int tv_debug_queries_per_launch(const tv_index *ix, int *queries);

@@ -96,9 +96,9 @@ hipError_t launch_move_lane(uint8_t *d_native, float *d_scales, const Geometry &
                             hipStream_t s);
 
 // Query preparation in one launch (tv_prep.hip).  `stamp` here and below, when given: a word that takes the
-// device clock as the launch ends (of the preparation and of a sampling level's selection) or starts (of a
-// last selection): the scan between two of them is timed without events, whose packets the launches behind
-// them wait for, 5 to 6 us each.
+// device clock as the last query's workgroup ends (of the preparation and of a sampling level's selection) or the
+// first one's starts (of a last selection): the full scan between two of them, gaps between launches included, is
+// timed without events, whose packets the launches behind them wait for, 5 to 6 us each.
 struct PrepRequest {
     const float *q, *signs;
     const uint32_t *perms;

@@ -1035,13 +1035,16 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
         if (t == 0) overflow[qn] = redo ? (raising ? 1u : 2u) : 0u;
         if (redo && !raising) return;
     }
-    // (the last query's is among the last to get here; the launch's end is its selection away)
-    if (stamp != nullptr && sampling && qn + 1 == int(gridDim.x) && t == 0) *stamp = wall_clock64();
+    // (the last query's workgroup is among the last to end)
+    auto stamp_end = [&]() {
+        if (stamp != nullptr && sampling && qn + 1 == int(gridDim.x) && t == 0) *stamp = wall_clock64();
+    };
     if (sampling && total < uint32_t(k_eff)) {
         // Too few allowed slots reached the floor in this sample.  The floor of the level before
         // (k_floor scanned slots reach it) is still a valid lower bound: it stays.  Only the
         // first level, which reads the standing array of open floors, has none to keep.
         if (t == 0 && !keep_floor) *tau_slot = kTauInit;
+        stamp_end();
         return;
     }
     const uint32_t need = (sampling || raising) ? min(uint32_t(k_floor), total) : uint32_t(k_eff);   // leading keys wanted
@@ -1130,6 +1133,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
             out_idx[row * k_eff + rank] = int64_t(idx);
         }
     }
+    stamp_end();
 }
 
 // ===========================================================================

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split
     if (t == 0) {
         a.qscale[qi] = cs * qs;
         a.qbias[qi] = 0.0f + bias;
-        if (a.stamp != nullptr && qi == 0) *a.stamp = wall_clock64();
+        if (a.stamp != nullptr && qi + 1 == a.nq) *a.stamp = wall_clock64();      // (among the last to end)
     }
 }
 
