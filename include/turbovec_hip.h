@@ -75,7 +75,13 @@ const char *tv_last_error(void);
 /* Replaces the lazily built caches of TurboQuantIndex (lib.rs:1404-1415): the
  * rotation tables (rotation.rs:141-187) and Lloyd-Max centroids
  * (codebook.rs:50) are derived inside and uploaded.  dim: positive multiple of
- * 8, <= 16384; bits in {2,3,4} (lib.rs:629-668).  device: HIP ordinal. */
+ * 8, <= 16384; bits in {2,3,4} (lib.rs:629-668).  device: HIP ordinal.
+ * Device blocks of 1 MiB and more that an index gives up -- it grew, or was
+ * destroyed -- are kept for the indexes of that device, up to 2 GiB, while any
+ * index lives there: handed on to a request they exceed by a quarter at most,
+ * given back to the device when an allocation of this library fails and when
+ * the device's last index is destroyed.  Other allocators of the process do
+ * not see them. */
 int tv_index_create(int dim, int bits, int device, tv_index **out);
 int tv_index_destroy(tv_index *ix);
 

@@ -1,0 +1,82 @@
+/* A HIP runtime without a device, for tests of the library's host side: device memory is host memory with a limit,
+ * launches do nothing, and the test decides how long a wait takes.  Loaded with RTLD_GLOBAL before the library, whose
+ * references then resolve here. */
+#define _GNU_SOURCE
+#include <pthread.h>
+#include <stdatomic.h>
+#include <stddef.h>
+#include <stdint.h>
+#include <stdlib.h>
+#include <string.h>
+#include <time.h>
+#include <unistd.h>
+
+enum { ok = 0, out_of_memory = 2 };
+typedef struct { uint32_t x, y, z; } dim3_t;
+
+/* ---- what a test sets and reads ---- */
+atomic_size_t fake_limit = (size_t)1 << 34, fake_used;
+atomic_int fake_stream_wait_us;       /* how long a stream's wait takes */
+atomic_int fake_device_busy;          /* the device's wait does not end while this is set ... */
+atomic_int fake_device_waits;         /* ... and this many threads are in one */
+atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
+
+int hipGetDeviceCount(int *n) { *n = 1; return ok; }
+int hipSetDevice(int d) { (void)d; return ok; }
+int hipDeviceGetAttribute(int *v, int attr, int d) { (void)attr; (void)d; *v = 256; return ok; }
+const char *hipGetErrorString(int e) { return e == ok ? "ok" : "out of memory"; }
+static _Thread_local int last;
+int hipGetLastError(void) { const int e = last; last = ok; return e; }
+
+static int take(void **p, size_t n) {
+    size_t used = fake_used;
+    do {
+        if (used + n > fake_limit) return last = out_of_memory;
+    } while (!atomic_compare_exchange_weak(&fake_used, &used, used + n));
+    size_t *at = calloc(1, n + 256);
+    at[0] = n;
+    *p = (char *)at + 256;
+    return ok;
+}
+static int give(void *p) {
+    if (p) { size_t *at = (size_t *)((char *)p - 256); fake_used -= at[0]; free(at); }
+    return ok;
+}
+int hipDeviceSynchronize(void) {
+    ++fake_device_waits;
+    while (fake_device_busy) usleep(100);
+    --fake_device_waits;
+    return ok;
+}
+int hipMalloc(void **p, size_t n) { return take(p, n); }
+int hipFree(void *p) { if (p) hipDeviceSynchronize(); return give(p); }
+int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(1, n); return ok; }
+int hipHostFree(void *p) { free(p); return ok; }
+int hipHostGetDevicePointer(void **d, void *h, unsigned flags) { (void)flags; *d = h; return ok; }
+int hipGetSymbolAddress(void **p, const void *symbol) { (void)symbol; static char *at; if (!at) at = calloc(1, 64 << 20); *p = at; return ok; }
+int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) { (void)kind; (void)s; memmove(to, from, n); return ok; }
+int hipMemsetAsync(void *p, int v, size_t n, void *s) { (void)s; memset(p, v, n); return ok; }
+int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &last; return ok; }
+int hipStreamDestroy(void *s) { (void)s; return ok; }
+int hipStreamSynchronize(void *s) { (void)s; if (fake_stream_wait_us) usleep(fake_stream_wait_us); return ok; }
+int hipEventCreate(void **e) { *e = &last; return ok; }
+int hipEventDestroy(void *e) { (void)e; return ok; }
+int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }
+int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0.0f; return ok; }
+int hipFuncSetAttribute(const void *f, int attr, int v) { (void)f; (void)attr; (void)v; return ok; }
+int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) { (void)f; (void)g; (void)b; (void)args; (void)lds; (void)s; return ok; }
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *s) { (void)g; (void)b; (void)lds; (void)s; return ok; }
+int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *lds, void **s) {
+    *g = *b = (dim3_t){1, 1, 1};
+    *lds = 0;
+    *s = NULL;
+    return ok;
+}
+
+/* std::chrono::steady_clock::now() */
+int64_t _ZNSt6chrono3_V212steady_clock3nowEv(void) {
+    struct timespec t;
+    ++fake_clock_reads;
+    clock_gettime(CLOCK_MONOTONIC, &t);
+    return (int64_t)t.tv_sec * 1000000000 + t.tv_nsec;
+}

@@ -1,0 +1,51 @@
+"""The library's host side on a HIP runtime without a device (fake_hip.c): device memory that runs out, waits that take
+as long as the test says.  Each test runs in a process of its own, which loads that runtime in front of the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+HEAD = '''
+import ctypes as C, sys, threading, time
+import numpy as np
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+from turbovec_amd import _lib as T
+def var(name, kind=C.c_int):
+    return kind.in_dll(fake, "fake_" + name)
+limit, used = var("limit", C.c_size_t), var("used", C.c_size_t)
+def index(rows, dim=64):
+    ix = T.NativeIndex(dim, 4)
+    if rows:
+        ix.append_rows(np.zeros((rows, dim // 2), np.uint8), np.zeros(rows, np.float32))
+    return ix
+'''
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-pthread", "-o", out, os.path.join(HERE, "fake_hip.c")], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", HEAD + body, out, ROOT], capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_an_index_is_made_from_memory_the_library_holds(fake):
+    """Blocks a grown index gave up are kept for later ones; memory that a new index needs is not refused for them."""
+    fake('''
+a = index(100_000)
+a.append_rows(np.zeros((200_000, 32), np.uint8), np.zeros(200_000, np.float32))
+before = used.value
+limit.value = before                     # nothing is left but what the library keeps
+b = index(0)
+assert used.value < before
+b.close(); a.close()
+assert used.value == 0
+''')

@@ -109,7 +109,8 @@ constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
 // ---- device memory of indexes ----------------------------------------------------------------
 // Large blocks that an index gives up (it grew, or went) are kept for the next one, per device: up to
 // kPoolBytes, handed on only to requests they exceed by a quarter at most, and given back when the last
-// index of the device goes or an allocation fails.  An index built by adds allocates 2.6 times its size on
+// index of the device goes or an allocation fails -- any of an index's, so all of them come through
+// device_alloc.  An index built by adds allocates 2.6 times its size on
 // the way; fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
 // 1536 rows in four adds: 4 ms a build while cleared memory lasts, 22.8 ms after).
 constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
@@ -1342,13 +1343,14 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
     int rc = TV_OK;
     do {
         if (hipStreamCreateWithFlags(&ix->stream, hipStreamNonBlocking) != hipSuccess) { rc = TV_ERR_HIP; break; }
-        if (hipMalloc(reinterpret_cast<void **>(&ix->d_signs), 2 * size_t(dim) * sizeof(float)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_perms), 2 * size_t(dim) * sizeof(uint32_t)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_packed), size_t(dim) * sizeof(uint32_t)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_centroids), 16 * sizeof(float)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_tq_shift), size_t(dim) * sizeof(float)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_tq_scale), size_t(dim) * sizeof(float)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void **>(&ix->d_tau_open), kTauOpenInts * sizeof(int)) != hipSuccess) {
+        // (through device_alloc, which empties the pool before it refuses; too small for the pool themselves)
+        auto table = [&](auto *&p, size_t count) {
+            size_t got = 0;
+            return device_alloc(device, count * sizeof *p, reinterpret_cast<void **>(&p), &got) == hipSuccess;
+        };
+        if (!table(ix->d_signs, 2 * size_t(dim)) || !table(ix->d_perms, 2 * size_t(dim)) || !table(ix->d_packed, size_t(dim)) ||
+            !table(ix->d_centroids, 16) || !table(ix->d_tq_shift, size_t(dim)) || !table(ix->d_tq_scale, size_t(dim)) ||
+            !table(ix->d_tau_open, kTauOpenInts)) {
             rc = TV_ERR_HIP;
             break;
         }
