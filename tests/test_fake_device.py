@@ -49,3 +49,27 @@ assert used.value < before
 b.close(); a.close()
 assert used.value == 0
 ''')
+
+
+def test_a_wait_for_the_device_holds_up_no_other_index(fake):
+    """An index that gives its blocks up waits for the device's work first; another one is made meanwhile."""
+    fake('''
+a = index(100_000)
+b = index(0)
+busy, waits = var("device_busy"), var("device_waits")
+busy.value = 1
+closing = threading.Thread(target=a.close)
+closing.start()
+while waits.value == 0:
+    time.sleep(0.001)
+made = []
+making = threading.Thread(target=lambda: made.append(index(0)))
+making.start()
+making.join(10)
+held_up = making.is_alive()
+busy.value = 0
+making.join(); closing.join()
+assert not held_up
+made[0].close(); b.close()
+assert used.value == 0
+''')

@@ -12,6 +12,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "tv_internal.h"
@@ -115,38 +116,49 @@ constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
 // 1536 rows in four adds: 4 ms a build while cleared memory lasts, 22.8 ms after).
 constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
 struct DevicePool {
-    std::mutex mu;
+    std::mutex mu;         // held for the bookkeeping only: allocations, frees and waits are long
+    std::mutex giving;     // held while an allocation that failed empties the pool and tries again
     std::vector<std::pair<size_t, void *>> blocks;
     size_t held = 0, indexes = 0;
-    void drop() {          // mu held
-        for (auto &b : blocks) (void)hipFree(b.second);
-        blocks.clear();
+    bool takes(size_t bytes) const { return bytes >= kPoolMinBytes && held + bytes <= kPoolBytes && indexes != 0; }   // mu held
+    std::vector<std::pair<size_t, void *>> empty() {      // mu held
         held = 0;
+        return std::exchange(blocks, {});
     }
 };
 DevicePool g_pool[kMaxDevices];
 
+void free_blocks(const std::vector<std::pair<size_t, void *>> &blocks) {
+    for (auto &b : blocks) (void)hipFree(b.second);
+}
+
 // `device` is current.  *got: what the block holds, 0 on failure.
 hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
     DevicePool &pool = g_pool[device];
-    std::lock_guard<std::mutex> lock(pool.mu);
-    size_t best = pool.blocks.size();
-    for (size_t i = 0; i < pool.blocks.size(); ++i) {
-        const size_t have = pool.blocks[i].first;
-        if (have >= bytes && have <= bytes + bytes / 4 && (best == pool.blocks.size() || have < pool.blocks[best].first)) best = i;
-    }
-    if (best < pool.blocks.size()) {
-        *out = pool.blocks[best].second;
-        *got = pool.blocks[best].first;
-        pool.held -= *got;
-        pool.blocks[best] = pool.blocks.back();
-        pool.blocks.pop_back();
-        return hipSuccess;
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        size_t best = pool.blocks.size();
+        for (size_t i = 0; i < pool.blocks.size(); ++i) {
+            const size_t have = pool.blocks[i].first;
+            if (have >= bytes && have <= bytes + bytes / 4 && (best == pool.blocks.size() || have < pool.blocks[best].first)) best = i;
+        }
+        if (best < pool.blocks.size()) {
+            *out = pool.blocks[best].second;
+            *got = pool.blocks[best].first;
+            pool.held -= *got;
+            pool.blocks[best] = pool.blocks.back();
+            pool.blocks.pop_back();
+            return hipSuccess;
+        }
     }
     hipError_t e = hipMalloc(out, bytes);
-    if (e != hipSuccess && !pool.blocks.empty()) {
+    if (e != hipSuccess) {
         (void)hipGetLastError();
-        pool.drop();
+        std::lock_guard<std::mutex> giving(pool.giving);      // (another thread's blocks may be on their way back)
+        std::unique_lock<std::mutex> lock(pool.mu);
+        const auto blocks = pool.empty();
+        lock.unlock();
+        free_blocks(blocks);
         e = hipMalloc(out, bytes);
     }
     *got = e == hipSuccess ? bytes : 0;     // (callers keep it: a size without a block would pass for one)
@@ -158,15 +170,17 @@ hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
 hipError_t device_free(int device, void *p, size_t bytes) {
     if (p == nullptr) return hipSuccess;
     DevicePool &pool = g_pool[device];
-    {
-        std::lock_guard<std::mutex> lock(pool.mu);
-        if (bytes >= kPoolMinBytes && pool.held + bytes <= kPoolBytes && pool.indexes != 0) {
-            const hipError_t e = hipDeviceSynchronize();
-            if (e != hipSuccess) return e;
+    std::unique_lock<std::mutex> lock(pool.mu);
+    const bool room = pool.takes(bytes);
+    lock.unlock();
+    if (room && hipDeviceSynchronize() == hipSuccess) {
+        lock.lock();
+        if (pool.takes(bytes)) {
             pool.blocks.emplace_back(bytes, p);
             pool.held += bytes;
             return hipSuccess;
         }
+        lock.unlock();
     }
     return hipFree(p);
 }
@@ -1397,8 +1411,10 @@ int tv_index_destroy(tv_index *ix) {
     for (void *p : ptrs) if (p) (void)hipFree(p);
     {
         DevicePool &pool = g_pool[ix->device];
-        std::lock_guard<std::mutex> lock(pool.mu);
-        if (--pool.indexes == 0) pool.drop();
+        std::unique_lock<std::mutex> lock(pool.mu);
+        const auto blocks = --pool.indexes == 0 ? pool.empty() : decltype(pool.blocks){};
+        lock.unlock();
+        free_blocks(blocks);
     }
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
     if (ix->events_ready)
