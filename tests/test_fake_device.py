@@ -73,3 +73,24 @@ assert not held_up
 made[0].close(); b.close()
 assert used.value == 0
 ''')
+
+
+def test_no_pause_for_callers_that_cannot_be_merged(fake):
+    """A caller that waited for another's search gives callers a moment to register, but not where the two could not
+    have shared a launch (another k).  (The moment would be seen by the clock: it is read in a loop.)"""
+    fake('''
+ix = index(64)
+clock, wait = var("clock_reads", C.c_long), var("stream_wait_us")
+wait.value = 2000                        # the other caller is always there before a search ends
+turns = 20
+q = np.ones((1, 64), np.float32)
+def caller(k):
+    for _ in range(turns):
+        ix.search(q, k)
+before = clock.value
+callers = [threading.Thread(target=caller, args=(k,)) for k in (1, 2)]
+for t in callers: t.start()
+for t in callers: t.join()
+per_search = (clock.value - before) / (2 * turns)
+assert per_search <= 2, per_search
+''')

@@ -1238,10 +1238,11 @@ int search_merged(tv_index *ix, tv_request &r) {
                 return r.rc;
             }
             if (!ix->serving) break;
-            had_to_wait = true;
+            had_to_wait |= compatible(*ix->served, r);
             ix->waiting_cv.wait(reg);
         }
         ix->serving = true;
+        ix->served = &r;
         // Callers in a loop come back together: when the batch before held several calls, give the
         // same number a moment to register again instead of serving this one alone and all of them
         // in the launch after.
@@ -1252,7 +1253,7 @@ int search_merged(tv_index *ix, tv_request &r) {
         }
         // A caller that had to wait is not the only one in a hurry: a search of a small index takes less time
         // than the callers' own work between two calls, and without a moment's pause they would line up one
-        // behind the other.
+        // behind the other.  (Only behind a search it could have shared: callers of other k or masks never can.)
         const auto pause = std::chrono::steady_clock::now() + kContendedWait;
         while (had_to_wait && ix->waiting.size() < 2 && std::chrono::steady_clock::now() < pause) {
             reg.unlock();
@@ -1288,6 +1289,7 @@ int search_merged(tv_index *ix, tv_request &r) {
         ix->merged_calls += batch.size() - 1;
         ix->last_batch_calls = batch.size();
         ix->serving = false;
+        ix->served = nullptr;
     }
     ix->waiting_cv.notify_all();
     return rc;

@@ -235,7 +235,8 @@ struct tv_index {
     std::mutex waiting_mu;
     std::condition_variable waiting_cv;   // a call registered, or a batch was served
     std::vector<tv_request *> waiting;
-    bool serving = false;          // some caller is serving a batch right now
+    bool serving = false;          // some caller is serving a batch right now ...
+    const tv_request *served = nullptr;   // ... this call's and what could join it
     size_t last_batch_calls = 0;   // calls in the batch served last: how many callers to expect again shortly
     size_t merged_calls = 0;       // calls that were served by another caller's launch
 
