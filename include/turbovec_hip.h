@@ -245,14 +245,16 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * sample-then-filter; bit 1 keeps large batches on the one-tile-per-launch scan
  * instead of the batched ones; bit 2 keeps them off the all-queries-per-pass
  * kernel only; bit 3 keeps u8-LUT batches on the scan that holds whole tables in
- * LDS (at most 8 queries per pass) instead of the sixteen-query one. */
+ * LDS (at most 8 queries per pass) instead of the larger ones; bit 4 samples
+ * small indexes like large ones (bits 1 and 2 do too). */
 int tv_debug_set_path(tv_index *ix, int force_full_lists);
 /* The sampling ladder a search for the k best of nq queries (its first chunk of up to 1024) runs
  * on this index as it stands, unfiltered: block strides of the successive scans, strides[0 ..
  * *count), the last one 1 (the full scan); level i reads blocks 0, strides[i], 2*strides[i], ...,
  * and in the repeated pass of queries whose candidates overflowed it starts at block
  * repeat_offsets[i].  At most cap entries are written (either array may be NULL); *count = 0 means
- * the search does not sample (large k, or the exact path is forced).  For tests and the bench,
+ * the search does not sample (large k, an index so small that every block is scored and its best
+ * row kept, or the exact path is forced).  For tests and the bench,
  * which lay rows out against the ladder. */
 int tv_debug_sampling_plan(const tv_index *ix, size_t nq, size_t k, uint32_t *strides, uint32_t *repeat_offsets,
                            size_t cap, size_t *count);

@@ -45,6 +45,9 @@ def to_native(T, oidx, mode=None):
     return ix
 
 
+SAMPLED = 16     # set_path: small indexes are sampled like large ones
+
+
 def bits_equal(a, b):
     a = np.ascontiguousarray(a, np.float32)
     b = np.ascontiguousarray(b, np.float32)
@@ -53,8 +56,10 @@ def bits_equal(a, b):
 
 def ladder_for(T, dim, bits, n, nq, k):
     """(strides, repeat_offsets) of the sampling ladder the library runs for nq queries, k best, on an index of
-    n rows of this shape (the ladder depends on nothing else): asked of a throw-away index of zero rows."""
+    n rows of this shape (the ladder depends on nothing else): asked of a throw-away index of zero rows.  The tests
+    that lay rows out against it search with SAMPLED set."""
     probe = T.NativeIndex(dim, bits)
+    probe.set_path(SAMPLED)
     probe.append_rows(np.zeros((n, probe.n_byte_groups), np.uint8), np.zeros(n, np.float32))
     plan = probe.sampling_plan(nq, k)
     probe.close()

@@ -14,6 +14,11 @@ def T():
     return _lib
 
 
+def unsampled(ix, nq, k, mask=None):
+    """Whether the library searches without sampling here: it has no ladder then."""
+    return len(ix.sampling_plan(nq, k if mask is None else min(k, int(mask.sum())))[0]) == 0
+
+
 # One and several tiles of queries, rows of 1 to 72 chunks (odd counts too), indexes of less than a block to
 # several rounds of the grid; 768 and 1536 dimensions with 140 queries: the all-queries kernel from 513 blocks on.
 @pytest.mark.parametrize("dim,n,nq", [
@@ -30,11 +35,12 @@ def test_unsampled_search_matches_oracle(T, oracle, dim, n, nq):
         if m is not None and not m.any():
             m[0] = True
         words = None if m is None else T.pack_mask(m)[0]
-        for k in (1, 10, 100):
+        for k in (1, 10 if dim <= 3840 else 8, 100):      # (k times the chunks of a row is bounded)
+            assert k == 100 or unsampled(ix, nq, k, m)
             s, i = ix.search(q, k, mask_words=words)
             os_, oi = oidx.search(q, k, mask_words=words)
             assert np.array_equal(i, oi) and bits_equal(s, os_), k
-            assert k == 100 or ix.overflow_redos() == redos
+            assert not unsampled(ix, nq, k, m) or ix.overflow_redos() == redos
         redos = ix.overflow_redos()
     ix.close()
 
@@ -48,8 +54,10 @@ def test_ties_and_wild_row_scales(T, oracle, dim, nq):
     q = unit_gaussian(nq, dim, seed=4)
     ix = to_native(T, oidx)
     for k in (10, 40):
+        assert unsampled(ix, nq, k)
         s, i = ix.search(q, k)
         os_, oi = oidx.search(q, k)
+        assert ix.overflow_redos() == 0
         assert np.array_equal(i, np.tile(np.arange(k), (nq, 1)))
         assert np.array_equal(i, oi) and bits_equal(s, os_)
     ix.close()
@@ -58,6 +66,7 @@ def test_ties_and_wild_row_scales(T, oracle, dim, nq):
     oidx.scales = (oidx.scales * rng.choice(np.array([0.0, 1e-38, -1.0, 1.0, 1e6], np.float32), size=n)).astype(np.float32)
     ix = to_native(T, oidx)
     for k in (10, 40):
+        assert unsampled(ix, nq, k)
         s, i = ix.search(q, k)
         ix.set_path(1)
         s2, i2 = ix.search(q, k)
@@ -79,6 +88,7 @@ def test_rows_that_score_minus_infinity(T, oracle, k):
     oidx.scales = (np.float32(3e38) * -np.sign(raw)).astype(np.float32)
     oidx.scales[[40, 41, 50, 60]] = 1.0
     ix = to_native(T, oidx)
+    assert unsampled(ix, 1, k)
     s, i = ix.search(q, k)
     os_, oi = oidx.search(q, k)
     assert np.isneginf(os_[0, 4:]).all() and np.isfinite(os_[0, :4]).all()
@@ -105,6 +115,7 @@ def test_scan_time_leaves_out_the_preparation(T):
         for _ in range(10):
             ix.search_dev(q.data_ptr(), nq, k, s.data_ptr(), i.data_ptr())
             ms.append(ix.last_scan_ms())
+        assert unsampled(ix, nq, k)
         assert all(launches == 1 for _, launches in ms)
         least.append(min(ms)[0])
         ix.close()

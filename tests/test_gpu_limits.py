@@ -3,7 +3,7 @@ over a larger index, row scales far outside the encoder's range."""
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -99,8 +99,10 @@ def test_wide_scan_with_subnormal_and_huge_row_scales(T, oracle):
     for m in (None, kind != 2, kind == 0, (kind == 0) | (kind == 3)):       # with the huge blocks allowed, and not
         words = None if m is None else T.pack_mask(m)[0]
         for k in (1, 10, 100):
-            s, i = ix.search(q, k, mask_words=words)
-            assert ix.queries_per_launch() == nq
             os_, oi = oidx.search(q, k, mask_words=words)
-            assert np.array_equal(i, oi) and bits_equal(s, os_), k
+            for path in (0, SAMPLED):
+                ix.set_path(path)
+                s, i = ix.search(q, k, mask_words=words)
+                assert ix.queries_per_launch() == nq
+                assert np.array_equal(i, oi) and bits_equal(s, os_), k
     ix.close()

@@ -6,7 +6,7 @@ import threading
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, ladder_for, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, ladder_for, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +55,7 @@ def test_first_level_poisoned_repeats_the_second_level_only(T, oracle, bits, nq)
     oidx = OracleIndex(oracle, dim, bits, rows_against(strides[:1], n, dim, u, seed=2))
     q = queries_near(u, nq, dim, seed=3)
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     ix.level_repeats(track=1)
     s, i = ix.search(q, k)
     assert ix.level_repeats() >= 1, "the layout did not overflow the second level: the test tests nothing"
@@ -80,6 +81,7 @@ def test_every_level_poisoned_goes_through_the_repeated_pass(T, oracle, bits, nq
     oidx = OracleIndex(oracle, dim, bits, rows_against(strides[:-1], n, dim, u, seed=5))
     q = queries_near(u, nq, dim, seed=6)
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     s, i = ix.search(q, k)
     assert ix.overflow_redos() == nq and ix.exact_redos() == 0
     os_, oi = oracle.search_fast(oidx.rot, oidx.seq, oidx.scales, q, k, bits, dim, n)
@@ -152,11 +154,13 @@ def test_calls_of_several_chunks(T, oracle):
     oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=21))
     ix = to_native(T, oidx)
     q = unit_gaussian(4096 + 77, dim, seed=22)
-    s, i = ix.search(q, k)
     os_, oi = oracle.search_fast(oidx.rot, oidx.seq, oidx.scales, q, k, 4, dim, n)
-    assert np.array_equal(i, oi) and bits_equal(s, os_)
-    s2, i2 = ix.search(q[4090:4100], k)
-    assert np.array_equal(i2, i[4090:4100]) and bits_equal(s2, s[4090:4100])
+    for path in (0, SAMPLED):
+        ix.set_path(path)
+        s, i = ix.search(q, k)
+        assert np.array_equal(i, oi) and bits_equal(s, os_)
+        s2, i2 = ix.search(q[4090:4100], k)
+        assert np.array_equal(i2, i[4090:4100]) and bits_equal(s2, s[4090:4100])
     ix.close()
 
 
@@ -172,6 +176,7 @@ def test_several_chunks_with_overflow_in_some(T, oracle):
     q = unit_gaussian(2048 + 300, dim, seed=33)
     q[1024 + 100: 1024 + 400] = queries_near(u, 300, dim, seed=34)
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     s, i = ix.search(q, k)
     assert ix.overflow_redos() >= 300 and ix.exact_redos() == 0
     os_, oi = oracle.search_fast(oidx.rot, oidx.seq, oidx.scales, q, k, 4, dim, n)
@@ -182,12 +187,14 @@ def test_several_chunks_with_overflow_in_some(T, oracle):
 # The reference refuses non-finite and huge query values before the seam (lib.rs:1374-1380).  A
 # caller that skipped tv_validate_queries must still get the call back: any status, any rows for
 # the bad queries, the good rows of the batch untouched, no hang.
+@pytest.mark.parametrize("path", [0, SAMPLED])
 @pytest.mark.parametrize("dim,nq", [(256, 5), (256, 64), (1536, 140), (128, 200)])
 @pytest.mark.timeout(60)
-def test_unvalidated_queries_return(T, oracle, dim, nq):
+def test_unvalidated_queries_return(T, oracle, dim, nq, path):
     n, k = 6_007, 10
     oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=41))
     ix = to_native(T, oidx)
+    ix.set_path(path)
     q = unit_gaussian(nq, dim, seed=42)
     want_s, want_i = ix.search(q, k)
     poison = {0: np.nan, 1: np.inf, 2: -np.inf, 3: 1e30, 4: -3e38}
@@ -242,6 +249,7 @@ def test_clustered_insertion_order_switches_to_the_row_level_ladder(T, nq):
     torch.cuda.synchronize()
     ix.add_dev(v.data_ptr(), n)
     q = (v[:: n // nq][:nq] + 0.05 * torch.randn(nq, dim, device=dev, generator=gen)).cpu().numpy()
+    ix.set_path(SAMPLED)
     before = ix.sampling_plan(nq, k)[0].tolist()           # the floorless level and the full scan
     assert len(before) == 2
     s, i = ix.search(q, k)

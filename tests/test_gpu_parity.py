@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from golden_data import parity_fixture_inputs
-from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -466,7 +466,7 @@ def test_sampled_path_matches_oracle_and_full_path(T, oracle, bits, mode):
             os_, oi = oidx.search(q, k, mask_words=words, mode=omode(O, mode))
             assert np.array_equal(i, oi), (mode, k)
             assert bits_equal(s, os_), (mode, k)
-            for path in (1, 2):                   # full-range lists; one tile per launch
+            for path in (1, 2, SAMPLED):          # full-range lists; one tile per launch; not without sampling
                 ix.set_path(path)
                 s2, i2 = ix.search(q, k, mask_words=words)
                 ix.set_path(0)
@@ -490,6 +490,7 @@ def test_candidate_overflow_is_redone_exactly(T, oracle):
     v[good] = np.tile(q[0], (int(good.sum()), 1)) + 0.3 * rng.standard_normal((int(good.sum()), dim)).astype(np.float32)
     oidx = OracleIndex(O, dim, bits, v.astype(np.float32))
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     s, i = ix.search(q, 10)
     os_, oi = oidx.search(q, 10)
     assert np.array_equal(i, oi) and bits_equal(s, os_)
@@ -510,10 +511,12 @@ def test_all_equal_scores(T, oracle):
     ix = to_native(T, oidx)
     q = unit_gaussian(2, dim, seed=4)
     for k in (10, 100):
-        s, i = ix.search(q, k)
-        assert np.array_equal(i, np.tile(np.arange(k), (2, 1)))
         os_, oi = oidx.search(q, k)
-        assert np.array_equal(i, oi) and bits_equal(s, os_)
+        for path in (0, SAMPLED):
+            ix.set_path(path)
+            s, i = ix.search(q, k)
+            assert np.array_equal(i, np.tile(np.arange(k), (2, 1)))
+            assert np.array_equal(i, oi) and bits_equal(s, os_)
     ix.close()
 
 
@@ -596,8 +599,9 @@ def test_batched_scan_matches_oracle(T, oracle, dim, n, nq):
             os_, oi = oidx.search(q, k, mask_words=words)
             assert np.array_equal(i, oi), k
             assert bits_equal(s, os_), k
-            ix.set_path(2)
-            s2, i2 = ix.search(q, k, mask_words=words)
-            ix.set_path(0)
-            assert np.array_equal(i2, i) and bits_equal(s2, s)
+            for path in (2, SAMPLED):
+                ix.set_path(path)
+                s2, i2 = ix.search(q, k, mask_words=words)
+                ix.set_path(0)
+                assert np.array_equal(i2, i) and bits_equal(s2, s)
     ix.close()

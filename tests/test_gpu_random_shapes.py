@@ -6,7 +6,7 @@ limits, batches around the tile sizes.  Each case is compared with the oracle bi
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -73,8 +73,9 @@ def test_random_shape(T, oracle, case):
     acc, raw = ix.debug_scan(q[:2])
     _s, _i, oacc, oraw = oidx.search(q[:2], k, mode=omode, dump=True)
     assert np.array_equal(acc, oacc) and bits_equal(raw, oraw)
-    ix.set_path(1)                                    # exact list / select path
-    s2, i2 = ix.search(q, k, mask_words=words)
-    ix.set_path(0)
-    assert np.array_equal(i2, idx) and bits_equal(s2, s)
+    for path in (1, SAMPLED):                         # exact list / select path; not without sampling
+        ix.set_path(path)
+        s2, i2 = ix.search(q, k, mask_words=words)
+        ix.set_path(0)
+        assert np.array_equal(i2, idx) and bits_equal(s2, s)
     ix.close()

@@ -4,7 +4,7 @@ batches.  Bar: slots and float scores bit-exact."""
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, ladder_for, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, ladder_for, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -50,11 +50,13 @@ def test_wide_scan_matches_oracle(T, oracle, dim, n, nq):
     ix = to_native(T, oidx)
     for words in masks_for(T, n, 8):
         for k in (1, 10, 100):
-            s, i = ix.search(q, k, mask_words=words)
-            assert ix.queries_per_launch() == min(nq, 2048 if dim == 1536 else 1024)
             os_, oi = oidx.search(q, k, mask_words=words)
-            assert np.array_equal(i, oi), k
-            assert bits_equal(s, os_), k
+            for path in (0, SAMPLED):      # (without sampling where the library does so, and in append mode)
+                ix.set_path(path)
+                s, i = ix.search(q, k, mask_words=words)
+                assert ix.queries_per_launch() == min(nq, 2048 if dim == 1536 else 1024)
+                assert np.array_equal(i, oi), k
+                assert bits_equal(s, os_), k
     ix.close()
 
 
@@ -80,6 +82,7 @@ def test_wide_launch_covers_the_chunk(T, oracle):
     oidx = OracleIndex(oracle, 1536, 4, unit_gaussian(2_000, 1536, seed=5))
     ix = to_native(T, oidx)
     q = unit_gaussian(512, 1536, seed=6)
+    ix.set_path(SAMPLED)
     ix.search(q, 10)
     assert ix.queries_per_launch() == 512
     ix.set_path(4)
@@ -105,10 +108,11 @@ def test_wide_scan_matches_other_paths(T, dim, n, nq):
     for words in masks_for(T, n, 9):
         for k in (10, 1000):
             s, i = ix.search(q, k, mask_words=words)
-            ix.set_path(4)
-            s2, i2 = ix.search(q, k, mask_words=words)
-            ix.set_path(0)
-            assert np.array_equal(i, i2) and bits_equal(s, s2), k
+            for path in (SAMPLED, 4):
+                ix.set_path(path)
+                s2, i2 = ix.search(q, k, mask_words=words)
+                ix.set_path(0)
+                assert np.array_equal(i, i2) and bits_equal(s, s2), k
         ix.set_path(1)
         s3, i3 = ix.search(q[:40], 10, mask_words=words)
         ix.set_path(0)
@@ -142,6 +146,7 @@ def test_wide_scan_stops_early_when_every_query_overflows(T):
         torch.cuda.synchronize()
         ix.add_dev(v.data_ptr(), m)
     q = (c + 0.3 * torch.randn(nq, dim, device=dev, generator=gen) / dim ** 0.5).cpu().numpy()
+    ix.set_path(SAMPLED)
     s, i = ix.search(q, 10)
     assert ix.queries_per_launch() == nq
     assert ix.overflow_redos() >= nq and ix.exact_redos() == 0
@@ -167,20 +172,25 @@ def test_wide_scan_with_wild_row_scales(T, oracle):
     q = unit_gaussian(nq, dim, seed=33)
     ix = to_native(T, oidx)
     for k in (1, 10, 100):
-        s, i = ix.search(q, k)
-        assert ix.queries_per_launch() == nq
         os_, oi = oidx.search(q, k)
-        assert np.array_equal(i, oi) and bits_equal(s, os_), k
+        for path in (0, SAMPLED):
+            ix.set_path(path)
+            s, i = ix.search(q, k)
+            assert ix.queries_per_launch() == nq
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
     ix.close()
     oidx.scales[rng.random(n) < 0.02] *= np.float32(-1.0)
     ix = to_native(T, oidx)
     for k in (10, 100):
+        ix.set_path(SAMPLED)
         s, i = ix.search(q, k)
         ix.set_path(4)
         s2, i2 = ix.search(q, k)
         ix.set_path(1)
         s3, i3 = ix.search(q, k)
         ix.set_path(0)
+        s4, i4 = ix.search(q, k)
+        assert np.array_equal(i, i4) and bits_equal(s, s4), k
         assert np.array_equal(i, i2) and bits_equal(s, s2), k
         assert np.array_equal(i, i3) and bits_equal(s, s3), k
     ix.close()
@@ -193,6 +203,7 @@ def test_wide_batch_equals_single_and_scale_invariance(T, oracle):
     dim, n = 1536, 4_003
     oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=51))
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     q = unit_gaussian(130, dim, seed=52)
     s, i = ix.search(q, 10)
     assert ix.queries_per_launch() == 130
@@ -206,11 +217,13 @@ def test_wide_batch_equals_single_and_scale_invariance(T, oracle):
 
 
 # concurrent_search.rs: threads searching one index at once see identical results
-def test_wide_concurrent_searches(T, oracle):
+@pytest.mark.parametrize("path", [0, SAMPLED])
+def test_wide_concurrent_searches(T, oracle, path):
     import threading
     dim, n = 1280, 3_001
     oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=53))
     ix = to_native(T, oidx)
+    ix.set_path(path)
     q = unit_gaussian(150, dim, seed=54)
     want_s, want_i = ix.search(q, 10)
     bad = []
@@ -267,7 +280,7 @@ def test_paths_agree_on_random_shapes(T):
             m[rng.integers(0, n, size=min(n, 7))] = True
         words = None if m is None else T.pack_mask(m)[0]
         res = []
-        for path in (0, 4, 1):
+        for path in (0, SAMPLED, 4, 1):
             ix.set_path(path)
             res.append(ix.search(q, k, mask_words=words))
         for s, i in res[1:]:
@@ -312,10 +325,11 @@ def test_small_batches_agree_with_the_exact_path_on_random_shapes(T):
             m[rng.integers(0, n, size=min(n, 7))] = True
         words = None if m is None else T.pack_mask(m)[0]
         res = []
-        for path in (0, 1):
+        for path in (0, SAMPLED, 1):
             ix.set_path(path)
             res.append(ix.search(q, k, mask_words=words))
-        assert np.array_equal(res[0][1], res[1][1]) and bits_equal(res[0][0], res[1][0]), (case, dim, n, nq, k, kind)
+        for s, i in res[1:]:
+            assert np.array_equal(res[0][1], i) and bits_equal(res[0][0], s), (case, dim, n, nq, k, kind)
         ix.close()
         del v
 
@@ -335,22 +349,27 @@ def test_tile_group_scan_with_wild_row_scales_and_query_scales(T, oracle, dim, n
     q = unit_gaussian(nq, dim, seed=63)
     ix = to_native(T, oidx)
     for k in (1, 10, 100):
-        s, i = ix.search(q, k)
-        assert 32 < ix.queries_per_launch() <= 128
         os_, oi = oidx.search(q, k)
-        assert np.array_equal(i, oi) and bits_equal(s, os_), k
+        for path in (0, SAMPLED):      # (the tile-group kernels where the index is sampled)
+            ix.set_path(path)
+            s, i = ix.search(q, k)
+            assert 32 < ix.queries_per_launch() <= 128
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
     for e in (-120, -60, 40, 100):
         qe = q * np.float32(2.0 ** e)
-        s, i = ix.search(qe, 10)
         os_, oi = oidx.search(qe, 10)
-        assert np.array_equal(i, oi) and bits_equal(s, os_), e
+        for path in (0, SAMPLED):
+            ix.set_path(path)
+            s, i = ix.search(qe, 10)
+            assert np.array_equal(i, oi) and bits_equal(s, os_), e
     ix.close()
     oidx.scales[rng.random(n) < 0.02] *= np.float32(-1.0)
     ix = to_native(T, oidx)
     for k in (10, 100):
-        s, i = ix.search(q, k)
         ix.set_path(1)
         s3, i3 = ix.search(q, k)
-        ix.set_path(0)
-        assert np.array_equal(i, i3) and bits_equal(s, s3), k
+        for path in (0, SAMPLED):
+            ix.set_path(path)
+            s, i = ix.search(q, k)
+            assert np.array_equal(i, i3) and bits_equal(s, s3), k
     ix.close()

@@ -729,7 +729,7 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
 // exact passes are held to the oracle by test.
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
-    if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide) return false;
+    if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
     if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > kDirectBlocks) return false;
     if (tv::pick_lds_bytes(nch, k_eff) > tv::kPickLds) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
@@ -2096,6 +2096,7 @@ int tv_debug_set_path(tv_index *ix, int force_full_lists) {
     ix->no_batched = (force_full_lists & 2) != 0;
     ix->no_wide = (force_full_lists & 4) != 0;
     ix->no_lut16 = (force_full_lists & 8) != 0;
+    ix->no_direct = (force_full_lists & 16) != 0;
     return TV_OK;
 }
 
@@ -2108,6 +2109,7 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t k_eff = std::min(k, ix->n);
     if (k_eff == 0 || nq == 0 || k_eff > size_t(tv::kMaxSampledK) || ix->force_robust) return TV_OK;   // no ladder
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (direct_serves(ix, nq, k_eff, n_blocks)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
     const SamplingSteps steps = level_strides(ix, plan, n_blocks, std::max<size_t>(k_eff, 16), false);
     *count = steps.size();

@@ -260,6 +260,7 @@ struct tv_index {
     int no_lut16 = 0;              // test hook: mode L batches stay on the scan with whole tables in LDS (8 queries per pass at most)
     bool no_lut_mx = false;        // for the length of a call: the scratch array holds only the sixteen-query passes' working set
     int no_wide = 0;               // test hook: large batches go through the tile-group kernels, not the wide one
+    int no_direct = 0;             // test hook: small indexes are sampled like large ones
     size_t overflow_redos = 0;     // queries redone because their candidate buffer overflowed
     // The floorless first level (best row per block) misjudges the floor when a query's neighbours
     // sit together in a few blocks (a clustered corpus in insertion order): after a search in which
