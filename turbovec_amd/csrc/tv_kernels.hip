@@ -933,7 +933,7 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 // bins between the smallest and the largest key gives a threshold few keys
 // reach (a bin that still holds too many is divided again); those are collected
 // in LDS and ranked by comparing each with all -- no sort, a handful of
-// barriers, 28 KiB of LDS, and workgroups no larger than the segments need.
+// barriers, 30 KiB of LDS, and workgroups no larger than the segments need.
 // Per launch under the profiler, before (waves sorting chunks in 64 KiB of LDS,
 // 1024 threads per query) and now: one query, k = 10, 12 -> 6 to 10 us; k = 100,
 // 60 and 33 -> 22 and 17 us; 1000 queries, k = 10, 61 to 75 -> 12 to 18 us.
