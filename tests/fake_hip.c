@@ -20,10 +20,12 @@ atomic_int fake_stream_wait_us;       /* how long a stream's wait takes */
 atomic_int fake_device_busy;          /* the device's wait does not end while this is set ... */
 atomic_int fake_device_waits;         /* ... and this many threads are in one */
 atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
+atomic_int fake_cus = 256;            /* compute units the device says it has */
+atomic_int fake_largest_grid;         /* workgroups of the largest launch */
 
 int hipGetDeviceCount(int *n) { *n = 1; return ok; }
 int hipSetDevice(int d) { (void)d; return ok; }
-int hipDeviceGetAttribute(int *v, int attr, int d) { (void)attr; (void)d; *v = 256; return ok; }
+int hipDeviceGetAttribute(int *v, int attr, int d) { (void)attr; (void)d; *v = fake_cus; return ok; }
 const char *hipGetErrorString(int e) { return e == ok ? "ok" : "out of memory"; }
 static _Thread_local int last;
 int hipGetLastError(void) { const int e = last; last = ok; return e; }
@@ -65,7 +67,12 @@ int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0.0f; return ok; }
 int hipFuncSetAttribute(const void *f, int attr, int v) { (void)f; (void)attr; (void)v; return ok; }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) { (void)f; (void)g; (void)b; (void)args; (void)lds; (void)s; return ok; }
-int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *s) { (void)g; (void)b; (void)lds; (void)s; return ok; }
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *s) {
+    (void)b; (void)lds; (void)s;
+    const int n = (int)(g.x * g.y * g.z);
+    if (n > fake_largest_grid) fake_largest_grid = n;
+    return ok;
+}
 int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *lds, void **s) {
     *g = *b = (dim3_t){1, 1, 1};
     *lds = 0;

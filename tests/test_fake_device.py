@@ -94,3 +94,14 @@ for t in callers: t.join()
 per_search = (clock.value - before) / (2 * turns)
 assert per_search <= 2, per_search
 ''')
+
+
+@pytest.mark.parametrize("cus", [256, 64])
+def test_the_encoder_fills_the_device_it_runs_on(fake, cus):
+    """Rows beyond what is resident at once are turns of the same workgroups: three of these to a CU (128 dimensions, LDS)."""
+    fake(f'''
+var("cus").value = {cus}
+ix = index(0, 128)
+ix.add(np.ones((100_000, 128), np.float32))
+assert var("largest_grid").value == 3 * {cus}, var("largest_grid").value
+''')

@@ -1573,7 +1573,7 @@ static int add_device_rows(tv_index *ix, const float *d_vectors, size_t n_new) {
         TV_HIP(tv::launch_encode(d_vectors + r0 * size_t(g.dim), nr, ix->n + r0, ix->d_signs, ix->d_perms,
                                  ix->packed_ok ? ix->d_packed : nullptr, cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr,
                                  ix->cb.centroids.data(), ix->cb.boundaries.data(), g, ix->rot.block,
-                                 ix->rot.inv_sqrt_block, ix->d_codes, ix->d_scales, nullptr, ix->stream));
+                                 ix->rot.inv_sqrt_block, ix->d_codes, ix->d_scales, nullptr, ix->device, ix->stream));
     }
     TV_HIP(hipStreamSynchronize(ix->stream));
     ix->n += n_new;
@@ -1648,7 +1648,7 @@ int tv_index_calibrate(tv_index *ix, const float *sample, size_t n) {
             TV_HIP(hipMemcpyAsync(d_in, sample + r0 * dim, nr * dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
             TV_HIP(tv::launch_encode(d_in, nr, 0, ix->d_signs, ix->d_perms, nullptr, nullptr, nullptr, ix->cb.centroids.data(),
                                      ix->cb.boundaries.data(), ix->geo, ix->rot.block, ix->rot.inv_sqrt_block,
-                                     nullptr, nullptr, d_out, ix->stream));
+                                     nullptr, nullptr, d_out, ix->device, ix->stream));
             TV_HIP(hipMemcpyAsync(rotated.data() + r0 * dim, d_out, nr * dim * sizeof(float), hipMemcpyDeviceToHost, ix->stream));
             TV_HIP(hipStreamSynchronize(ix->stream));
         }

@@ -480,14 +480,14 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
 }
 
 template <int NG, int W>
-static hipError_t launch_encode_rows_n(EncodeRowsArgs &a, hipStream_t s) {
+static hipError_t launch_encode_rows_n(EncodeRowsArgs &a, int device, hipStream_t s) {
     const int R = W * 64 / a.lanes, ng = a.dim / 8;
     const size_t lds = size_t(R * a.row_stride + R * ng + 9 * R + 4) * 4 + (16 + 4 * size_t(R)) * 8 + 64;
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_encode_rows<NG, W>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     const size_t groups = (a.n_new + R - 1) / R;
-    const size_t resident = size_t(256) * std::max<size_t>(1, std::min<size_t>(size_t(2048) / (W * 64), 160 * 1024 / lds));   // (a workgroup keeps its tables for all its turns)
+    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(2048) / (W * 64), 160 * 1024 / lds));   // (a workgroup keeps its tables for all its turns)
     hipLaunchKernelGGL((k_encode_rows<NG, W>), dim3(unsigned(std::min(groups, resident))), dim3(W * 64), lds, s, a);
     return hipGetLastError();
 }
@@ -502,7 +502,7 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
                          const uint32_t *d_perms, const uint32_t *d_packed, const float *d_shift, const float *d_scale,
                          const float *centroids, const float *boundaries, const Geometry &g, int block,
                          float inv_sqrt_block, uint8_t *d_native, float *d_scales, float *d_rot_out,
-                         hipStream_t s) {
+                         int device, hipStream_t s) {
     if (n_new == 0) return hipSuccess;
     if (d_packed != nullptr && d_rot_out == nullptr) {
         EncodeRowsArgs a;
@@ -519,12 +519,12 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
         a.inv_sqrt_block = inv_sqrt_block;
         a.nat = d_native; a.scales = d_scales; a.old_n = old_n; a.n_new = n_new;
         switch ((g.dim / 8 + a.lanes - 1) / a.lanes) {
-            case 1: return launch_encode_rows_n<1, 8>(a, s);
-            case 2: return launch_encode_rows_n<2, 8>(a, s);
-            case 3: return launch_encode_rows_n<3, 8>(a, s);
-            case 4: return launch_encode_rows_n<4, 8>(a, s);
-            case 5: case 6: return launch_encode_rows_n<6, 4>(a, s);
-            default: return launch_encode_rows_n<8, 4>(a, s);
+            case 1: return launch_encode_rows_n<1, 8>(a, device, s);
+            case 2: return launch_encode_rows_n<2, 8>(a, device, s);
+            case 3: return launch_encode_rows_n<3, 8>(a, device, s);
+            case 4: return launch_encode_rows_n<4, 8>(a, device, s);
+            case 5: case 6: return launch_encode_rows_n<6, 4>(a, device, s);
+            default: return launch_encode_rows_n<8, 4>(a, device, s);
         }
     }
     EncodeArgs a;

@@ -87,7 +87,7 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
                          const uint32_t *d_perms, const uint32_t *d_packed, const float *d_shift, const float *d_scale,
                          const float *centroids, const float *boundaries, const Geometry &g, int block,
                          float inv_sqrt_block, uint8_t *d_native, float *d_scales, float *d_rot_out,
-                         hipStream_t s);
+                         int device, hipStream_t s);
 size_t encode_lds_bytes(int dim);
 // The rotation tables of both rounds in one word per position for the several-rows-per-workgroup
 // encoder; false where it does not apply (long rows, signs other than +-1).
