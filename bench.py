@@ -144,9 +144,21 @@ def cpu_baseline(args):
     return out
 
 
+def sparse_roofline(launch_s, queries, n, dim, bits):
+    """Roofline of the table scan on the sparse int8 matrix instruction (k_scan_lut_mx): a nibble's table is a
+    one-hot contraction of 16 entries (8 for 3-bit codes), half of them stored, two nibbles to a code byte.  The
+    stored operations are priced against the dense int8 peak: the instruction contracts twice a dense one's
+    entries in its time, and stores half of them."""
+    ops = 2.0 * queries * n * (dim * 2 // 8 if bits == 2 else dim // 2) * (8 if bits == 3 else 16)
+    return {"bound": "mfma", "achieved": ops / launch_s / 1e12, "peak": 5000.0, "unit": "TFLOP/s",
+            "frac": ops / launch_s / 1e12 / 5000.0, "traffic": None, "kernel": "k_scan_lut_mx",
+            "stored_ops_per_launch": ops}
+
+
 def config3_extra(T, torch, build_index, run, args):
     """Configuration 3 beside the headline: 10M x 1536 2-bit, k=100 (u8 LUT, u32 epilogue), batches 1
-    and 1024, each with the HBM roofline of its scan launch (algorithmic bytes = codes + row scales)."""
+    and 1024, each with the roofline of its scan launch: HBM for the single query (algorithmic bytes = codes +
+    row scales), the sparse matrix instruction for the batch."""
     n, dim, bits, k = 10_000_000, 1536, 2, 100
     ix = build_index(dim, bits, n)
     alg = ((n + 31) // 32) * (dim // 4) * 32 + 4 * n
@@ -157,11 +169,13 @@ def config3_extra(T, torch, build_index, run, args):
         launch_s = scan_ms * 1e-3 / max(launches, 1)
         # byte tables serve single queries; a batch is one launch of the sparse matrix-unit scan
         kern = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut_mx" if q_full > 16 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
+        roofline = {"bound": "hbm", "achieved": alg / launch_s / 1e9, "peak": 8000.0,
+                    "unit": "GB/s", "frac": alg / launch_s / 1e9 / 8000.0,
+                    "traffic": MEASURED_TRAFFIC.get((kern, n, dim, bits)), "kernel": kern}
+        if kern == "k_scan_lut_mx":
+            roofline = sparse_roofline(launch_s, min(nq, q_full), n, dim, bits)
         res[f"batch{nq}"] = {"queries_per_s": nq * steps / dt, "ms_per_step": dt / steps * 1e3,
-                             "queries_per_launch": q_full, "scan_launch_ms": launch_s * 1e3,
-                             "roofline": {"bound": "hbm", "achieved": alg / launch_s / 1e9, "peak": 8000.0,
-                                          "unit": "GB/s", "frac": alg / launch_s / 1e9 / 8000.0,
-                                          "traffic": MEASURED_TRAFFIC.get((kern, n, dim, bits)), "kernel": kern}}
+                             "queries_per_launch": q_full, "scan_launch_ms": launch_s * 1e3, "roofline": roofline}
     res["overflow_redos"] = ix.overflow_redos()
     ix.close()
     return res
@@ -465,6 +479,13 @@ def main():
                                               "algorithmic_bytes_per_launch", "achievable_read_GBps")}
         else:
             out["mfma"] = mfma
+    elif kernel == "k_scan_lut_mx":
+        hbm = out["roofline"]
+        out["roofline"] = {**sparse_roofline(launch_s, q_per_launch, n, dim, bits), "launches_timed": launches,
+                           "mean_launch_ms": launch_s * 1e3, "queries_per_launch": q_per_launch,
+                           "queries_per_full_launch": q_full}
+        out["hbm"] = {k: hbm[k] for k in ("achieved", "peak", "unit", "frac", "traffic",
+                                          "algorithmic_bytes_per_launch", "achievable_read_GBps")}
     # queries of the timed steps that left the sampled path for the exact one (candidate overflow);
     # Gaussian rows never do, and a non-zero count would mean the timed steps include that path's cost
     out["overflow_redos"] = ix.overflow_redos()
