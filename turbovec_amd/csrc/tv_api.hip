@@ -710,23 +710,25 @@ bool direct_wide(const tv_index *ix, size_t nq, size_t n_blocks) {
 size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
     return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) + 65536;
 }
-// Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, sampled and
-// without: 100K x 128, 1 query 50 and 28, 1000 queries 498 and 67; 260K x 768, 32 queries 77 and 54;
-// 100K x 1536, 1000 queries 310 and 243.
+// Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, each pair
+// without sampling and with it: 100K x 128, 1 query 30 and 45, 1000 queries 67 and 493; 260K x 768, 32 queries
+// 54 and 71; 100K x 1536, 1000 queries 246 and 304.
 //  - It scores k blocks a second time in one workgroup: k = 100 at 768 dimensions (12 chunks) costs one
-//    query 77 us against 64, at 128 dimensions 39 against 53.
-//  - One tile of queries: level with sampling at 16384 blocks (500K x 3072: 204 and 202; x 1536: 118 and
-//    126), behind it at twice that (1M x 1536: 205 and 184).
+//    query 77 us against 64, at 128 dimensions 40 against 72.
+//  - One tile of queries: level with sampling at 16384 blocks (500K x 3072: 204 and 202; x 1536: 110 and
+//    116), behind it at twice that (1M x 1536: 205 and 184).
 //  - More tiles on k_scan_p4_best, which decodes a block once per tile group: won up to a number of (block,
 //    tile, chunk) triples that depends on the kernel it replaces -- short rows against the all-queries kernel
-//    (260K x 768, 1000 queries, 3.1e6 triples: 373 and 365; x 128: 129 and 664), rows whose tiles stay in
-//    LDS (100K x 1536, 100 queries, 3e5: 100 and 99; 500K x 768, 8e5: 112 and 148), rows whose tiles are
-//    streamed (260K x 3072, 100 queries, 1.6e6: 294 and 543; 500K, 3e6: 489 and 437).
+//    (260K x 768, 1000 queries, 3.1e6 triples: 373 and 365; x 128: 134 and 661), rows whose tiles stay in
+//    LDS (100K x 1536, 100 queries, 3e5: 100 and 99; 500K x 768, 8e5: 117 and 145), rows whose tiles are
+//    streamed (260K x 3072, 100 queries, 1.6e6: 308 and 528; 500K, 3e6: 489 and 437).
 //  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about a
-//    million rows (1M x 1536, 1000 queries: 1573 and 1489; 260K: 466 and 513).
+//    million rows (1M x 1536, 1000 queries: 1573 and 1489; 260K: 476 and 519; 260K x 768: 289 and 354).
 // Batches of 2 to 8, of 33 to 255 and of more than 1024 queries on short rows keep to the sampled path beyond
-// 1535 blocks although this one would be faster there too: those are the calls whose overflow, repeated and
-// exact passes are held to the oracle by test.
+// 1535 blocks, and not for its speed: without sampling (a build without that line, same bits) and with it, 100K x
+// 128, 64 queries 31 and 60, 2048 queries 123 and 977; 100K x 768, 4 queries 43 and 57; 260K x 768, 128 queries 78
+// and 122; 500K x 128, 200 queries 69 and 206.  The line dates from when these calls were the tests' way to the
+// sampled path on a small index, which tv_debug_set_path's bit 4 is now.
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
     if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;

@@ -21,10 +21,9 @@
 // one or two of them and their tables stay in its L2), and each reads all of the codes.
 //
 // What bounds it: 192 sparse instructions per (block, tile) at 1536 dimensions and 2 bits, 1.26e14
-// stored operations for 10M rows and 1024 queries.  The instruction alone, operands in registers,
-// sustains 3.9e15 a second at the clock the chip holds under it (32 ms), with its operands' eight vector
-// instructions beside every two about 10 % less; the scan takes 42 to 44 ms, the matrix unit 71 %
-// busy at 1.9 GHz, against 64 passes of 1.5 ms of the table lookups, which are bound by LDS reads.  Two
+// stored operations for 10M rows and 1024 queries.  At 32 clocks each they take 32 ms on a matrix unit that does
+// nothing else, at the 1.87 GHz the chip holds under them; the scan takes 44 ms, the matrix unit 72 % busy and the
+// vector ALU 48 % (by counters), against 64 passes of 1.5 ms of the table lookups, which are bound by LDS reads.  Two
 // tiles and four blocks per wave: the operands of a block are built once for two instructions, every
 // LDS read feeds four, and the sums (128 registers) still leave room for two waves per SIMD.
 //
