@@ -38,6 +38,7 @@ MEASURED_TRAFFIC = {
     ("k_scan_p4_multi", 10_000_000, 1536, 4): 7.7359e9,   # 3,775,570 x 2 KiB fetched + 3,451 KiB written
     ("k_scan_p4", 10_000_000, 1536, 4): 7.7208e9,         # 3,769,800 x 2 KiB fetched + 265 KiB written
     ("k_scan_lut_bt", 10_000_000, 1536, 2): 3.8802e9,     # 1,894,650 x 2 KiB fetched
+    ("k_scan_lut_mx", 10_000_000, 1536, 2): 5.455e10,     # 26,600,000 x 2 KiB fetched + 70,660 KiB written, 1024 queries
     ("k_scan_lut16", 10_000_000, 1536, 2): 3.8830e9,      # 1,895,400 x 2 KiB fetched + 1,189 KiB written
     ("k_scan_lut", 10_000_000, 1536, 2): 3.8809e9,        # 1,894,970 x 2 KiB fetched
 }
@@ -151,7 +152,8 @@ def sparse_roofline(launch_s, queries, n, dim, bits):
     entries in its time, and stores half of them."""
     ops = 2.0 * queries * n * (dim * 2 // 8 if bits == 2 else dim // 2) * (8 if bits == 3 else 16)
     return {"bound": "mfma", "achieved": ops / launch_s / 1e12, "peak": 5000.0, "unit": "TFLOP/s",
-            "frac": ops / launch_s / 1e12 / 5000.0, "traffic": None, "kernel": "k_scan_lut_mx",
+            "frac": ops / launch_s / 1e12 / 5000.0, "kernel": "k_scan_lut_mx",
+            "traffic": MEASURED_TRAFFIC.get(("k_scan_lut_mx", n, dim, bits)) if queries == 1024 else None,
             "stored_ops_per_launch": ops}
 
 
@@ -409,6 +411,7 @@ def main():
         kernel = "k_scan_p4_wide" if q_full >= 256 else "k_scan_p4_multi" if q_full > 32 else "k_scan_p4"
     else:
         kernel = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut_mx" if q_full > 16 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
+    kernel64 = "k_scan_p4_multi" if mode_p else "k_scan_lut16" if q64_full > 8 else "k_scan_lut"
     traffic = MEASURED_TRAFFIC.get((kernel, n, dim, bits))
     int8_ops = 2.0 * q_per_launch * n * dim        # multiply-adds x2 of one launch, permute-dot mode
 
@@ -437,10 +440,10 @@ def main():
                    "end_to_end_frac_of_hbm_peak": alg_bytes / (dt1 / b1_steps) / 1e9 / 8000.0},
         "batch64": {"queries_per_s": 64 * b64_steps / dt64, "ms_per_step": dt64 / b64_steps * 1e3,
                     "queries_per_launch": q64_full, "scan_launch_ms": b64_launch_s * 1e3,
-                    "roofline": {"bound": "hbm", "achieved": alg_bytes / b64_launch_s / 1e9, "peak": 8000.0, "unit": "GB/s",
+                    "roofline": sparse_roofline(b64_launch_s, 64, n, dim, bits) if not mode_p and q64_full > 16 else
+                                {"bound": "hbm", "achieved": alg_bytes / b64_launch_s / 1e9, "peak": 8000.0, "unit": "GB/s",
                                  "frac": alg_bytes / b64_launch_s / 1e9 / 8000.0,
-                                 "traffic": MEASURED_TRAFFIC.get(("k_scan_p4_multi", n, dim, bits)),
-                                 "kernel": "k_scan_p4_multi" if mode_p else "k_scan_lut",
+                                 "traffic": MEASURED_TRAFFIC.get((kernel64, n, dim, bits)), "kernel": kernel64,
                                  "int8_TOPs": 2.0 * min(64, q64_full) * n * dim / b64_launch_s / 1e12 if mode_p else None}},
         "threads8_batch1": {"queries_per_s": t8_qps, "one_thread_queries_per_s": 1.0 / host_single_s,
                             "vs_one_thread": t8_qps * host_single_s, "calls_served_by_another_callers_launch": t8_merged,
