@@ -14,7 +14,7 @@
 //
 // Three shapes of one template: rows of 16 to 24 chunks, one block per wave, 8
 // waves per workgroup at 256 registers; rows of 32 to 48 chunks, 4 waves at 512
-// registers (A operands partly in AGPRs); rows of 4 to 12 chunks, 2 to 4 blocks
+// registers (A operands partly in AGPRs); rows of 2 to 10 chunks, 2 to 6 blocks
 // per wave, every B operand feeding as many MFMAs.
 //
 // Integers and float epilogue are those of k_scan_p4 (turbovec/src/search.rs:
@@ -656,10 +656,11 @@ hipError_t launch_probe_mfma(int device, int iters, uint32_t *sink, double *ops,
 // level at 97 to 128 queries (two tile-group passes); from 2560 dimensions the tile-group kernel
 // streams four tiles' weights and serves 128 queries in one pass, 1 to 7 % faster than the wide
 // kernel there, which takes over from 129 (1.2 to 1.4 times faster at 160 to 384 queries, 1.6 to
-// 1.7 times at 1024).
+// 1.7 times at 1024).  3, 5 and 7 chunks (no padding below 9): 665K x 176, 815 queries 642 -> 519 us a search, 2M x 320,
+// 1000 queries 1435 -> 1089, 1.5M x 432, 500 queries 736 -> 584, 130 to 150 queries 7 to 18 % less.
 int wide_min_queries(int nch) {
     switch (nch) {
-        case 2: case 4: case 6: case 8: case 10: case 12: case 14: case 16: case 18: return 129;
+        case 2: case 3: case 4: case 5: case 6: case 7: case 8: case 10: case 12: case 14: case 16: case 18: return 129;
         case 20: case 22: case 24: return 97;
         case 28: case 32: case 36: return 97;
         case 40: case 44: case 48: return 129;
@@ -676,9 +677,9 @@ bool wide_serves_best_of_block(int nch) { return nch >= 12 && wide_blocks_per_wo
 int wide_blocks_per_workgroup(int nch) {
     switch (nch) {
         case 2: return 48;
-        case 4: return 32;
-        case 6: return 24;
-        case 8: case 10: return 16;
+        case 3: case 4: return 32;
+        case 5: case 6: return 24;
+        case 7: case 8: case 10: return 16;
         case 12: case 14: case 16: case 18: case 20: case 22: case 24: return 8;
         case 28: case 32: case 36: case 40: case 44: case 48: return 4;
         case 56: case 64: case 72: case 80: case 88: case 96: return 2;
@@ -737,8 +738,11 @@ hipError_t launch_scan_p4_wide(const ScanArgs &a, int grid, hipStream_t s) {
         // One hand-over per tile (two slices) measured 2.5 to 5 % faster than one per slice in the
         // eight-wave forms with two slices per tile, and 2 % slower in the four-wave forms.
         case 2: return launch_wide_n<2, 2, 8, 1, 6>(a, grid, s);
+        case 3: return launch_wide_n<3, 2, 8, 1, 4>(a, grid, s);
         case 4: return launch_wide_n<4, 2, 8, 1, 4>(a, grid, s);
+        case 5: return launch_wide_n<5, 2, 8, 1, 3>(a, grid, s);
         case 6: return launch_wide_n<6, 2, 8, 1, 3>(a, grid, s);
+        case 7: return launch_wide_n<7, 2, 8, 1, 2>(a, grid, s);
         case 8: return launch_wide_n<8, 4, 8, 1, 2>(a, grid, s);
         case 10: return launch_wide_n<10, 2, 8, 2, 2, 2>(a, grid, s);
         case 12: return launch_wide_n<12, 2, 8, 2, 1, 2, 1, true>(a, grid, s);   // two blocks per wave would spill 21 registers
