@@ -131,3 +131,31 @@ def test_every_launch_of_the_timed_scan_counts(T, mode, nq, launches):
     assert len(ix.sampling_plan(nq, 10)[0]) == 2      # a level before the full scan: timed between stamps
     assert ix.last_scan_ms()[1] == launches
     ix.close()
+
+
+# The number of blocks a thread of the last launch keeps changes behind 16384, and 32768 are its most; 1048577 rows
+# are sampled.  Batches of a few queries, of several tiles and of more than a launch's worth.
+@pytest.mark.parametrize("dim,n,nq", [(64, 524_288, 9), (64, 524_289, 70), (128, 1_048_576, 1), (128, 1_048_577, 1), (64, 1_048_545, 200),
+                                      (128, 60_001, 1030), (768, 100_003, 5), (768, 600_000, 130), (1024, 540_000, 64)])
+def test_unsampled_search_agrees_with_the_sampled_one(T, dim, n, nq):
+    torch = pytest.importorskip("torch")
+    gen = torch.Generator(device="cuda:0").manual_seed(dim + n)
+    ix = T.NativeIndex(dim, 4)
+    for at in range(0, n, 262_144):
+        v = torch.randn(min(262_144, n - at), dim, device="cuda:0", generator=gen)
+        if at == 0:
+            v[1000:1100] = v[:100]       # equal rows
+        torch.cuda.synchronize()
+        ix.add_dev(v.data_ptr(), len(v))
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    rng = np.random.default_rng(5)
+    for m, k in ((None, 1), (None, 10), (rng.random(n) < 0.02, 12)):
+        words = None if m is None else T.pack_mask(m)[0]
+        assert unsampled(ix, nq, k, m) == (n <= 1_048_576)
+        res = []
+        for path in (0, 16):
+            ix.set_path(path)
+            res.append(ix.search(q, k, mask_words=words))
+        ix.set_path(0)
+        assert np.array_equal(res[0][1], res[1][1]) and bits_equal(res[0][0], res[1][0]), k
+    ix.close()

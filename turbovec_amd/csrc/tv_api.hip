@@ -697,8 +697,7 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
 uint32_t repeat_offset(uint32_t step) { return step >= 4 ? (step / 2) & ~1u : 0u; }
 
 // ---- small indexes: no sampling (tv_kernels6.hip) ----
-constexpr size_t kDirectBlocks = 16384;      // what k_pick holds in registers
-constexpr size_t kDirectWideBlocks = 8192;
+constexpr size_t kDirectWideBlocks = 20480;
 
 // Which scan the search of nq queries without sampling takes: the all-queries kernel keeps a decoded block
 // for all of them, from where its grid of eight waves per CU has blocks to hold (157 blocks of 1536
@@ -711,36 +710,37 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
     return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) + 65536;
 }
 // Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, each pair
-// without sampling and with it: 100K x 128, 1 query 30 and 45, 1000 queries 67 and 493; 260K x 768, 32 queries
-// 54 and 71; 100K x 1536, 1000 queries 246 and 304.
+// without sampling and with it: 100K x 128, 1 query 30 and 45, 64 queries 32 and 61, 1000 queries 67 and 493;
+// 260K x 768, 32 queries 54 and 71; 100K x 1536, 1000 queries 246 and 304.
 //  - It scores k blocks a second time in one workgroup: k = 100 at 768 dimensions (12 chunks) costs one
 //    query 77 us against 64, at 128 dimensions 40 against 72.
-//  - One tile of queries: level with sampling at 16384 blocks (500K x 3072: 204 and 202; x 1536: 110 and
-//    116), behind it at twice that (1M x 1536: 205 and 184).
+//  - k_pick keeps a word per block in registers: 32768 blocks at most (twice that spills: 2M x 128, one query
+//    121 and 77).
+//  - One tile of queries: a full scan of so many bytes that two more launches no longer show.  1.04M rows x 128
+//    51 and 63, x 512 80 and 92, x 640 99 and 101, x 768 113 and 115, x 1024 140 and 140; 600K x 1024 95 and 105, x 1536 132 and 131.
 //  - More tiles on k_scan_p4_best, which decodes a block once per tile group: won up to a number of (block,
-//    tile, chunk) triples that depends on the kernel it replaces -- short rows against the all-queries kernel
-//    (260K x 768, 1000 queries, 3.1e6 triples: 373 and 365; x 128: 134 and 661), rows whose tiles stay in
-//    LDS (100K x 1536, 100 queries, 3e5: 100 and 99; 500K x 768, 8e5: 117 and 145), rows whose tiles are
-//    streamed (260K x 3072, 100 queries, 1.6e6: 308 and 528; 500K, 3e6: 489 and 437).
-//  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about a
-//    million rows (1M x 1536, 1000 queries: 1573 and 1489; 260K: 476 and 519; 260K x 768: 289 and 354).
-// Batches of 2 to 8, of 33 to 255 and of more than 1024 queries on short rows keep to the sampled path beyond
-// 1535 blocks, and not for its speed: without sampling (a build without that line, same bits) and with it, 100K x
-// 128, 64 queries 31 and 60, 2048 queries 123 and 977; 100K x 768, 4 queries 43 and 57; 260K x 768, 128 queries 78
-// and 122; 500K x 128, 200 queries 69 and 206.  The line dates from when these calls were the tests' way to the
-// sampled path on a small index, which tv_debug_set_path's bit 4 is now.
+//    tile, chunk) triples that depends on the kernel it replaces -- rows of less than 12 chunks (600K x 640, 1000 queries,
+//    6e6 triples: 563 and 677; 1.04M x 512, 8.3e6: 929 and 829; 1.04M x 128, 2.1e6: 400 and 781), rows whose tiles
+//    stay in LDS and that this kernel too keeps two tiles of (1.04M x 1024, 64 queries, 1.04e6: 172 and 193) or only one (100K x 1536,
+//    100 queries, 3e5: 100 and 99; 600K x 1536, 64 queries, 9e5: 211 and 185), rows whose tiles are streamed (260K x 3072, 100 queries, 1.6e6:
+//    308 and 528; 500K, 3e6: 489 and 437).
+//  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about 700K
+//    rows (1000 queries: 600K x 768 570 and 621, x 1536 972 and 999; 1.04M x 768 935 and 895, x 1536 1611 and 1523),
+//    earlier where many rows are scored again (500K x 768, k = 45: 556 and 540).
+// Batches of 2 to 8 on rows of one chunk keep to the sampled path beyond 1535 blocks, and not for its speed: it is
+// how the test of the exact fallback in a fixed workspace gets there.
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
     if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
-    if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > kDirectBlocks) return false;
+    if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > tv::kMaxPickBlocks) return false;
     if (tv::pick_lds_bytes(nch, k_eff) > tv::kPickLds) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
-    if (n_blocks >= 1536 && nch <= 12 && ((nq >= 2 && nq <= 8) || (nq > 32 && nq < 256) || nq > kChunkQueries)) return false;
-    if (direct_wide(ix, cq, n_blocks)) return n_blocks <= kDirectWideBlocks;
-    if (tiles == 1) return nch <= 24 || n_blocks <= kDirectBlocks / 2;
-    if (nch < 12) return triples <= 2500000;
-    return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 14 ? 800000 : 250000) || n_blocks <= 512;
+    if (nch == 1 && nq >= 2 && nq <= 8 && n_blocks >= 1536) return false;
+    if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
+    if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
+    if (nch < 12) return triples <= 6000000;
+    return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 16 ? 1050000 : 250000) || n_blocks <= 512;
 }
 // The milliseconds between the two stamps.
 int take_stamps(tv_index *ix, int launches) {

@@ -147,6 +147,7 @@ hipError_t launch_scan_lut_mx(const ScanArgs &a, const MxShape &m, int bits, hip
 hipError_t launch_scan_p4(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Small indexes without sampling (tv_kernels6.hip): the best row of every block, then the best blocks' rows.
 constexpr int kMaxPickK = 128;             // most results k_pick ranks
+constexpr size_t kMaxPickBlocks = 32768;   // most blocks it chooses from
 constexpr size_t kPickLds = 128 * 1024;    // beside its 13 KiB of fixed buffers
 bool best_serves(int nch);
 hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s);

@@ -203,9 +203,8 @@ struct PickArgs {
     uint32_t *overflow;
     uint64_t *stamp;
 };
-constexpr uint32_t kPickHeld = 16;       // blocks a thread keeps in registers: all of them, T * kPickHeld at most
-
-template <uint32_t T>
+// H: blocks a thread keeps in registers -- all of them, T * H at most.
+template <uint32_t T, uint32_t H>
 __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     constexpr uint32_t W = T / 64;
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -219,9 +218,9 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     const uint32_t k_eff = uint32_t(a.k_eff);
     const uint32_t *best = a.best + size_t(qi) * a.best_stride;
     if (a.stamp != nullptr && qi + t == 0) *a.stamp = wall_clock64();
-    uint32_t v[kPickHeld];
+    uint32_t v[H];
 #pragma unroll
-    for (uint32_t e = 0; e < kPickHeld; ++e) v[e] = e * T + t < a.n_blocks ? best[e * T + t] : 0u;
+    for (uint32_t e = 0; e < H; ++e) v[e] = e * T + t < a.n_blocks ? best[e * T + t] : 0u;
     // the tile's weights lie [chunk][fragment][half * 32 + query] in 16-byte pieces; here [chunk][half][fragment]
     const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
     for (int i = int(t); i < a.nch * 4; i += int(T))
@@ -230,7 +229,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     if (t == 0) { n_kept = 0u; n_list = 0u; s_floor = 0u; }
     auto each = [&](auto &&f) {
 #pragma unroll
-        for (uint32_t e = 0; e < kPickHeld; ++e)
+        for (uint32_t e = 0; e < H; ++e)
             if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
     };
     uint32_t mine = 0u, hi_max = 0u, hi_min_inv = 0u, mx, mn_inv, total = 0u;
@@ -365,7 +364,7 @@ hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scor
                        hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
     const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff));
-    if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > 1024 * kPickHeld) return hipErrorInvalidValue;
+    if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
     PickArgs p;
     p.best = a.best_out; p.best_stride = a.best_stride; p.n_blocks = a.n_blocks; p.n = a.n;
     p.codes = a.codes; p.scales = a.scales; p.mask = a.mask; p.tables = a.tables;
@@ -380,8 +379,9 @@ hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scor
         return hipGetLastError();
     };
     // few queries leave the chip empty: as many waves as there are blocks to score again
-    if (a.nq_tile <= 256 || a.n_blocks > 256 * kPickHeld) return launch(k_pick<1024>, 1024);
-    return launch(k_pick<256>, 256);
+    if (a.n_blocks > 1024 * 16) return launch(k_pick<1024, 32>, 1024);
+    if (a.nq_tile <= 256 || a.n_blocks > 256 * 16) return launch(k_pick<1024, 16>, 1024);
+    return launch(k_pick<256, 16>, 256);
 }
 
 }  // namespace tv
