@@ -9,7 +9,9 @@
 //   * the rotation is the query rotation with the 1/norm folded into the first
 //     gather: (x[perm0[i]] * inv) * sign0[i];
 //   * the reconstruction inner product runs in 4 interleaved f64 chains
-//     (element j feeds chain j % 4), folded pairwise; 4 lanes carry them.
+//     (element j feeds chain j % 4), folded pairwise; only its f32 rounding is used, so
+//     k_encode_rows adds in an order of its own and falls back to the chains where the
+//     rounding could depend on it.
 //
 // k_encode_rows takes rows of up to 4096 dimensions, a wave (or part of one) per
 // row and a group of eight waves' rows through each step together, so that the
@@ -19,6 +21,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
+#include <vector>
 
 #include "tv_device.h"
 #include "tv_internal.h"
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(256) void k_encode(EncodeArgs a) {
 // stride of 8 modulo 64 floats: the passes below, whose lanes are 64 floats apart in groups of eight,
 // and the chains, whose lanes are a row apart, then spread over all banks.
 __host__ __device__ constexpr int enc_at(int j) { return j + (j >> 6) * 8; }
-// (and a row's place holds the f64 products of one run of its groups, 16 lanes + 16 floats, later on)
+// (and a row's place holds the f64 products of one run of its groups, 16 lanes floats, where enc_in_order needs it)
 static int enc_row_stride(int dim, int lanes) {
     int s = std::max(enc_at(dim - 1) + 1, 16 * lanes + 16);
     while (s % 64 != 8) ++s;
@@ -171,6 +175,14 @@ constexpr int kEncMaxDim = 4096;
 static_assert(enc_at(kEncMaxDim - 1) < (1 << 15), "a padded place takes fifteen bits");
 bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint32_t *packed) {
     if (dim > kEncMaxDim) return false;
+    // (a rotation keeps a row's length, which enc_slack counts on: both gathers must be permutations)
+    for (int r = 0; r < 2; ++r) {
+        std::vector<bool> seen(size_t(dim), false);
+        for (int j = 0; j < dim; ++j) {
+            if (seen[perms[size_t(r) * dim + j]]) return false;
+            seen[perms[size_t(r) * dim + j]] = true;
+        }
+    }
     for (int j = 0; j < dim; ++j) {
         uint32_t w = 0;
         for (int r = 0; r < 2; ++r) {
@@ -197,7 +209,9 @@ struct EncodeRowsArgs {
     int dim, bits, G, nch, log_block;
     int lanes;                // lanes per row: a power of two, 8 to 64
     int row_stride;           // floats
-    int by_quarters;          // fifteen boundaries, in rising order
+    int cells;                // boundaries found by cell (enc_cells) instead of one by one
+    float cell_mul, cell_add;
+    double slack;             // no TQ+ pair: how far the two orders of inner's additions can lie apart
     float inv_sqrt_block;
     uint8_t *nat;
     float *scales;
@@ -211,31 +225,82 @@ __device__ __forceinline__ void enc_wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// The number of boundaries below a value, from the cell it falls into: a rising map of values to kEncCells cells
+// leaves the boundaries of earlier cells below it and those of later cells not, so where no cell holds two
+// boundaries one comparison is left (15 boundaries: four levels of three comparisons before).
+constexpr int kEncCells = 64;
+struct EncCell { float bound; uint32_t below; };
+__host__ __device__ __forceinline__ int enc_cell(float x, float mul, float add) {
+#ifdef __HIP_DEVICE_COMPILE__
+    uint32_t c;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(c) : "v"(fmaf(x, mul, add)));               // saturates; NaN: cell 0, where it exceeds nothing
+    return int(min(c, uint32_t(kEncCells - 1)));
+#else
+    return int(std::fmin(std::fmax(std::fmaf(x, mul, add), 0.0f), float(kEncCells - 1)));
+#endif
+}
+// How far two orders of adding dim terms of the given total magnitude in f64 lie apart at most: dim / 4 + 3
+// roundings on the way of any term in the four chains (its product's among them), 8 NG + 6 in k_encode_rows, and the
+// few of the magnitude itself and of stepping this far to either side.
+__host__ __device__ __forceinline__ double enc_slack(int dim, double mass) { return double(dim + 256) * 0x1p-53 * mass; }
+
+// The row scale with the additions of inner in the reference's order: element j feeds chain j % 4, each chain
+// sequential, folded pairwise.  Met by the whole wave; L lanes per row, lane l of them holding groups l, l + L, ...
+template <int NG, typename Recon>
+__device__ __forceinline__ float enc_in_order(const float (&v)[NG][8], const Recon &recon_of, float *row, int dim, int l, int L, float nrm) {
+    const int ng = dim / 8;
+    double *terms = reinterpret_cast<double *>(row);               // a run's products: [group of the run][8]
+    double chain[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        enc_wave_sync();                                           // the run before has been read
+        if (l + i * L < ng) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) terms[l * 8 + e] = double(v[i][e]) * recon_of(i, e);
+        }
+        enc_wave_sync();
+        const int n_here = 8 * min(L, ng - i * L);
+        for (int j = 0; j < n_here; j += 4) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) chain[c] = chain[c] + terms[j + c];
+        }
+    }
+    const double inner = (chain[0] + chain[1]) + (chain[2] + chain[3]);
+    return inner > 0.1 ? nrm / float(inner) : 0.0f;
+}
+
 // NG = groups of eight elements per lane; W = waves per workgroup.  The float work of a row is a few
-// thousand instructions of its wave, but the two chains are 192 dependent f32 and 384 f64 additions
-// (1536 dimensions): a workgroup per row spent 40 us on a row, nearly all of it waiting for them.
-// Here the chains of a workgroup's rows run in one or two waves, while the other workgroup of the CU is
-// in its parallel part.  A row's rotation goes through LDS three stages at a time in registers
-// (the same additions in the same pairs), and its codes leave as 16-byte stores that consecutive
-// rows complete to whole lines.  100K rows of 1536 dimensions: 2.02 ms with a workgroup per row, 0.50 now (1.4 TB/s,
-// every byte once).  By counters the vector ALU issues in 60 % of the clocks (1750 instructions a row) and a wave
-// waits 56 % of its time, for the steps of its row that follow one another: barriers, chains, LDS.
-template <int NG, int W>
-__global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeRowsArgs a) {
+// thousand instructions of its wave, but its norm is a chain of 192 dependent f32 additions (1536 dimensions): a workgroup
+// per row spent most of its time waiting for chains.  Here the norm chains of a workgroup's rows run in one wave, while
+// other workgroups of the CU are in their parallel part; the f64 sum needs no chain (enc_slack).  A row's rotation
+// goes through LDS three stages at a time in registers (the same additions in the same pairs), and its codes leave as
+// 16-byte stores that consecutive rows complete to whole lines.  100K rows of 1536 dimensions: 2.02 ms with a workgroup per
+// row, 0.50 with the f64 chains too in one wave and four levels of three comparisons per value, 0.39 now (1.8 TB/s, every
+// byte once); of 2048: 1.15 -> 0.62.
+// CAL: there is a TQ+ pair.
+template <int NG, int W, bool CAL>
+__global__ __launch_bounds__(W * 64, NG <= 4 ? 4 : 2) void k_encode_rows(EncodeRowsArgs a) {
     extern __shared__ __align__(16) float enc_lds[];
     const int dim = a.dim, t = threadIdx.x, ng = dim / 8, rs = a.row_stride, L = a.lanes;
     const int R = W * 64 / L;                                      // rows of a workgroup
     uint32_t *s_codes = reinterpret_cast<uint32_t *>(enc_lds + R * rs);   // [R][ng] eight codes each, packed as in the index
-    float *s_nrm = reinterpret_cast<float *>(s_codes + R * ng);
-    float *s_part = s_nrm + R;                                     // [R][8] chains of the squared norm
-    double *s_cen = reinterpret_cast<double *>(enc_lds + (R * rs + R * ng + 9 * R + 3) / 4 * 4);   // centroids in f64
-    double *s_chain = s_cen + 16;                                  // [R][4]
+    float *s_part = reinterpret_cast<float *>(s_codes + R * ng);   // [R][8] chains of the squared norm
+    double *s_cen = reinterpret_cast<double *>(enc_lds + (R * rs + R * ng + 8 * R + 3) / 4 * 4);   // centroids in f64
     const int r = t / L;                                           // this thread's row of the group ...
     int l = t % L;                                                 // ... and its lane in the row
     float *row = enc_lds + r * rs;
-    float4 *s_quarter = reinterpret_cast<float4 *>(s_chain + 4 * R);       // [4] the boundaries inside each quarter
+    EncCell *s_cell = reinterpret_cast<EncCell *>(s_cen + 16);
     if (t < 16) s_cen[t] = double(a.cen[t]);
-    if (t < 4) s_quarter[t] = float4{a.bnd[4 * t], a.bnd[4 * t + 1], a.bnd[4 * t + 2], 0.0f};
+    if (t < kEncCells) {
+        // (the boundary of this cell, if it has one, and how many lie in the cells before it)
+        EncCell cell{__int_as_float(0x7f800000), 0u};
+        for (int b = 0; b < (1 << a.bits) - 1; ++b) {
+            const int k = enc_cell(a.bnd[b], a.cell_mul, a.cell_add);
+            if (k < t) ++cell.below;
+            if (k == t) cell.bound = a.bnd[b];
+        }
+        s_cell[t] = cell;
+    }
 
     const size_t n_groups = (a.n_new + R - 1) / R;
     RowPiece pre[NG][2];
@@ -320,12 +385,27 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
             const float *x = enc_lds + (idx >> 3) * rs + (idx & 7);
             float c = 0.0f;
             int i = 0;
-            for (; i + 8 <= ng; i += 8) {                          // eight groups of eight: 64 floats and their padding
-                float v[8];
+            if (ng >= 8) {
+                // eight groups of eight -- 64 floats and their padding -- at a time, the next ones on their way
+                float v[2][8];
+                auto load = [&](float (&to)[8], int at) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = x[9 * i + 8 * e];
+                    for (int e = 0; e < 8; ++e) to[e] = x[9 * at + 8 * e];
+                };
+                auto add = [&](const float (&from)[8]) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) c = c + v[e] * v[e];
+                    for (int e = 0; e < 8; ++e) c = c + from[e] * from[e];
+                };
+                load(v[0], 0);
+                for (; i + 24 <= ng; i += 16) {
+                    load(v[1], i + 8);
+                    add(v[0]);
+                    load(v[0], i + 16);
+                    add(v[1]);
+                }
+                add(v[0]);
+                i += 8;
+                if (i + 8 <= ng) { load(v[1], i); add(v[1]); i += 8; }
             }
             for (; i < ng; ++i) { const float v = x[8 * i + (i >> 3) * 8]; c = c + v * v; }
             s_part[idx] = c;
@@ -334,7 +414,6 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
         const float *p8 = s_part + r * 8;
         const float nrm = sqrtf(((p8[0] + p8[1]) + (p8[2] + p8[3])) + ((p8[4] + p8[5]) + (p8[6] + p8[7])));
         const float inv = nrm > 1e-10f ? 1.0f / nrm : 0.0f;   // lib.rs:163 MIN_INPUT_NORM
-        if (l == 0) s_nrm[r] = nrm;
 
         // rotation (rotation.rs:218-255): gather, sign, stages; the factor rides the gather
 #pragma unroll
@@ -387,12 +466,10 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float x = v[i][e];
-                if (a.scale != nullptr) x = (x + a.shift[8 * g + e]) * a.scale[8 * g + e];
-                if (a.by_quarters) {
-                    // fifteen boundaries in rising order: the quarter first, then its three
-                    const uint32_t q = (x > a.bnd[3] ? 1u : 0u) + (x > a.bnd[7] ? 1u : 0u) + (x > a.bnd[11] ? 1u : 0u);
-                    const float4 b = s_quarter[q];
-                    c[e] = 4u * q + (x > b.x ? 1u : 0u) + (x > b.y ? 1u : 0u) + (x > b.z ? 1u : 0u);
+                if constexpr (CAL) x = (x + a.shift[8 * g + e]) * a.scale[8 * g + e];
+                if (a.cells) {
+                    const EncCell cell = s_cell[enc_cell(x, a.cell_mul, a.cell_add)];
+                    c[e] = cell.below + (x > cell.bound ? 1u : 0u);
                 } else {
                     c[e] = 0u;
                     for (int b = 0; b < (1 << a.bits) - 1; ++b) c[e] += x > a.bnd[b] ? 1u : 0u;
@@ -404,94 +481,82 @@ __global__ __launch_bounds__(W * 64, NG <= 3 ? 4 : 2) void k_encode_rows(EncodeR
                                               : ((code4[i] >> 4) & 0x0f0f0f0fu) | ((code4[i] & 0x0f0f0f0fu) << 4);
             __builtin_amdgcn_sched_barrier(0);      // (one group after the other: several at once would spill)
         }
-        enc_wave_sync();                                           // every lane has its elements: their places are free
-        // encode.rs:1442-1475: inner = <rotated, reconstruction> in f64, four chains by j % 4, NG runs of L
-        // groups one after the other: the products by all lanes, in pairs at (element pair, lane) ...
-        const int pair = 16 * L + 16;                              // bytes from one element pair's line to the next
+        // encode.rs:1442-1475: inner = <rotated, reconstruction> in f64, four chains by j % 4.  The row scale takes
+        // float(inner), so the order of the additions shows only where it moves inner across a rounding boundary: the
+        // lanes add their own elements, then each other's sums, and where every value within the two orders' distance
+        // gives the same row scale, that is it.
+        auto recon_of = [&](int i, int e) -> double {
+            double recon = s_cen[(code4[i] >> (4 * e)) & 15u];                                 // (no TQ+ pair: * 1 - 0)
+            if constexpr (CAL) {
+                const int j = 8 * (l + i * L) + e;
+                recon = recon * double(1.0f / a.scale[j]) - double(a.shift[j]);                // encode.rs:594
+            }
+            return recon;
+        };
+        double inner = 0.0, mass = 0.0;                            // the sum, and (for a pair) the sum of the terms' magnitudes
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
-            const int g = l + i * L;
-            if (g < ng) {
+            if (l + i * L >= ng) continue;
 #pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    double p[2];
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        double recon = s_cen[(code4[i] >> (4 * (e + u))) & 15u];          // (no TQ+ pair: * 1 - 0)
-                        if (a.scale != nullptr)
-                            recon = recon * double(1.0f / a.scale[8 * g + e + u]) - double(a.shift[8 * g + e + u]);   // encode.rs:594
-                        p[u] = double(v[i][e + u]) * recon;
-                    }
-                    *reinterpret_cast<double2 *>(reinterpret_cast<uint8_t *>(row) + (e / 2) * pair + l * 16) = double2{p[0], p[1]};
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+            for (int e = 0; e < 8; ++e) {
+                const double recon = recon_of(i, e), x = double(v[i][e]);
+                inner = fma(x, recon, inner);
+                if constexpr (CAL) mass = fma(fabs(x), fabs(recon), mass);
+                if (e == 3) __builtin_amdgcn_sched_barrier(0);
             }
-            __syncthreads();
-            // ... and the additions by the chains: elements 8 g + c and 8 g + 4 + c of every group in turn
-            const int n_here = min(L, ng - i * L);
-            for (int idx = t; idx < 4 * R; idx += W * 64) {
-                const int c = idx & 3;
-                const uint8_t *x = reinterpret_cast<const uint8_t *>(enc_lds + (idx >> 2) * rs) + (c >> 1) * pair + (c & 1) * 8;
-                double sum = i == 0 ? 0.0 : s_chain[idx];
-                int k = 0;
-                for (; k + 8 <= n_here; k += 8) {
-                    double y[16];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        y[2 * u] = *reinterpret_cast<const double *>(x + (k + u) * 16);
-                        y[2 * u + 1] = *reinterpret_cast<const double *>(x + (k + u) * 16 + 2 * pair);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) sum = sum + y[u];
-                }
-                for (; k < n_here; ++k) {
-                    sum = sum + *reinterpret_cast<const double *>(x + k * 16);
-                    sum = sum + *reinterpret_cast<const double *>(x + k * 16 + 2 * pair);
-                }
-                s_chain[idx] = sum;
-            }
-            if (i == 0) {
-                // the rows' code bytes, 16 at a time, into their lanes of the device layout (pack.rs:211-233
-                // append_lanes); the bytes past a row's last group are zero there and stay so
-                const int per = a.bits == 2 ? 8 : 4, pieces = (a.G + 15) / 16;
-                for (int idx = W * 64 - 1 - t; idx < R * pieces; idx += W * 64) {     // (the last waves first: the first one carries the chains)
-                    const int rr = idx % R, p = idx / R;
-                    const size_t vec = grp * R + rr;
-                    if (vec >= a.n_new) continue;
-                    uint32_t o[4] = {0u, 0u, 0u, 0u};
-                    const uint32_t *src = s_codes + rr * ng + p * per;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (e >= per || p * per + e >= ng) continue;
-                        if (a.bits == 2) o[e >> 1] |= src[e] << (16 * (e & 1));
-                        else o[e & 3] = src[e];
-                    }
-                    *reinterpret_cast<uint4 *>(a.nat + enc_byte_index(a.old_n + vec, 16 * p, a.nch)) = uint4{o[0], o[1], o[2], o[3]};
-                }
-            }
-            if (i + 1 < NG) __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        if (t < R && grp * R + t < a.n_new) {
-            const double *d = s_chain + 4 * t;
-            const double inner = (d[0] + d[1]) + (d[2] + d[3]);
-            a.scales[a.old_n + grp * R + t] = inner > 0.1 ? s_nrm[t] / float(inner) : 0.0f;   // encode.rs:1194-1200
+        for (int d = 1; d < L; d <<= 1) {
+            inner += __shfl_xor(inner, d);
+            if constexpr (CAL) mass += __shfl_xor(mass, d);
+        }
+        const double slack = CAL ? enc_slack(dim, mass) : a.slack;
+        const double lo = inner - slack, hi = inner + slack;
+        float scale = lo > 0.1 ? nrm / float(lo) : 0.0f;                                       // encode.rs:1194-1200
+        const bool settled = lo > 0.1 ? float(lo) == float(hi) : hi <= 0.1;                    // (NaN: not settled)
+        if (__any(!settled)) scale = enc_in_order<NG>(v, recon_of, row, dim, l, L, nrm);       // one row in 10^5
+        if (l == 0 && grp * R + r < a.n_new) a.scales[a.old_n + grp * R + r] = scale;
+        __syncthreads();                                           // every row's codes are there
+        // the rows' code bytes, 16 at a time, into their lanes of the device layout (pack.rs:211-233
+        // append_lanes); the bytes past a row's last group are zero there and stay so
+        const int per = a.bits == 2 ? 8 : 4, pieces = (a.G + 15) / 16;
+        for (int idx = t; idx < R * pieces; idx += W * 64) {
+            const int rr = idx % R, p = idx / R;
+            const size_t vec = grp * R + rr;
+            if (vec >= a.n_new) continue;
+            uint32_t o[4] = {0u, 0u, 0u, 0u};
+            const uint32_t *src = s_codes + rr * ng + p * per;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (e >= per || p * per + e >= ng) continue;
+                if (a.bits == 2) o[e >> 1] |= src[e] << (16 * (e & 1));
+                else o[e & 3] = src[e];
+            }
+            *reinterpret_cast<uint4 *>(a.nat + enc_byte_index(a.old_n + vec, 16 * p, a.nch)) = uint4{o[0], o[1], o[2], o[3]};
         }
         if (NG > 3 && grp + gridDim.x < n_groups) fetch(grp + gridDim.x);
     }
 }
 
-template <int NG, int W>
-static hipError_t launch_encode_rows_n(EncodeRowsArgs &a, int device, hipStream_t s) {
+template <int NG, int W, bool CAL>
+static hipError_t launch_encode_rows_cal(const EncodeRowsArgs &a, int device, hipStream_t s) {
     const int R = W * 64 / a.lanes, ng = a.dim / 8;
-    const size_t lds = size_t(R * a.row_stride + R * ng + 9 * R + 4) * 4 + (16 + 4 * size_t(R)) * 8 + 64;
+    const size_t lds = size_t(R * a.row_stride + R * ng + 8 * R + 4) * 4 + 16 * 8 + kEncCells * sizeof(EncCell);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_encode_rows<NG, W>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    const void *kernel = reinterpret_cast<const void *>(k_encode_rows<NG, W, CAL>);
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
-    const size_t groups = (a.n_new + R - 1) / R;
-    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(2048) / (W * 64), 160 * 1024 / lds));   // (a workgroup keeps its tables for all its turns)
-    hipLaunchKernelGGL((k_encode_rows<NG, W>), dim3(unsigned(std::min(groups, resident))), dim3(W * 64), lds, s, a);
+    // a workgroup keeps its tables for all its turns: as many as are resident at once, by registers and LDS
+    int per_cu = 0;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, W * 64, lds);
+    if (e != hipSuccess) return e;
+    const size_t groups = (a.n_new + R - 1) / R, resident = size_t(device_cus(device)) * size_t(std::max(1, per_cu));
+    hipLaunchKernelGGL((k_encode_rows<NG, W, CAL>), dim3(unsigned(std::min(groups, resident))), dim3(W * 64), lds, s, a);
     return hipGetLastError();
+}
+template <int NG, int W>
+static hipError_t launch_encode_rows_n(const EncodeRowsArgs &a, int device, hipStream_t s) {
+    return a.scale != nullptr ? launch_encode_rows_cal<NG, W, true>(a, device, s) : launch_encode_rows_cal<NG, W, false>(a, device, s);
 }
 
 // A and B, one float row each; codes and the f64 products overlay A.  128 KiB at the largest
@@ -516,15 +581,28 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
         a.lanes = 8;
         while (a.lanes < 64 && a.lanes * 8 < g.dim) a.lanes *= 2;
         a.row_stride = enc_row_stride(g.dim, a.lanes);
-        // (each no larger than the next: handed-over centroids may be out of order, or NaN, which is in no order)
-        a.by_quarters = g.bits == 4 && std::adjacent_find(a.bnd, a.bnd + 15, [](float x, float y) { return !(x <= y); }) == a.bnd + 15;
+        // cells of equal width from the first boundary to the last; no two boundaries may share one, and handed-over
+        // centroids may be in any order, equal, infinite or NaN
+        const int nb = nl - 1;
+        a.cell_mul = float(kEncCells - 2) / (a.bnd[nb - 1] - a.bnd[0]);
+        a.cell_add = 1.0f - a.bnd[0] * a.cell_mul;
+        a.cells = a.cell_mul > 0.0f && a.cell_mul < 1e30f && std::fabs(a.cell_add) < 1e30f;
+        for (int i = 0; a.cells && i + 1 < nb; ++i)
+            a.cells = a.bnd[i] < a.bnd[i + 1] && enc_cell(a.bnd[i], a.cell_mul, a.cell_add) < enc_cell(a.bnd[i + 1], a.cell_mul, a.cell_add);
+        // without a pair the terms are x * centroid over a row of length 1: |x c| <= (x^2 + c^2) / 2
+        double c_max = 0.0;
+        for (int i = 0; i < nl; ++i) c_max = std::fabs(double(centroids[i])) >= c_max ? std::fabs(double(centroids[i])) : c_max;
+        a.slack = enc_slack(g.dim, (1.01 + double(g.dim) * c_max * c_max) / 2.0);
         a.inv_sqrt_block = inv_sqrt_block;
         a.nat = d_native; a.scales = d_scales; a.old_n = old_n; a.n_new = n_new;
+        // Waves per workgroup: a wave's worth of norm chains (eight rows) where two such workgroups fit a CU's LDS and
+        // registers, fewer where one would (ms for 300K x 2048 rows in three adds: 3.1 with eight, 2.23 with four, 2.13
+        // with two; 400K x 1024: 1.98 with six, 1.45 with four, 1.48 with two; 200K x 3072: 2.78 with four, 4.2 with two).
         switch ((g.dim / 8 + a.lanes - 1) / a.lanes) {
             case 1: return launch_encode_rows_n<1, 8>(a, device, s);
-            case 2: return launch_encode_rows_n<2, 8>(a, device, s);
+            case 2: return launch_encode_rows_n<2, 4>(a, device, s);
             case 3: return launch_encode_rows_n<3, 8>(a, device, s);
-            case 4: return launch_encode_rows_n<4, 8>(a, device, s);
+            case 4: return launch_encode_rows_n<4, 2>(a, device, s);
             case 5: case 6: return launch_encode_rows_n<6, 4>(a, device, s);
             default: return launch_encode_rows_n<8, 4>(a, device, s);
         }
