@@ -729,13 +729,32 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
 //    earlier where many rows are scored again (500K x 768, k = 45: 556 and 540).
 // Batches of 2 to 8 on rows of one chunk keep to the sampled path beyond 1535 blocks, and not for its speed: it is
 // how the test of the exact fallback in a fixed workspace gets there.
+// The same for u8-LUT queries with the u32 epilogue.  k = 10, us a search without sampling and with it, 2 bits: 100K x 128, 1 query
+// 34 and 43, 12 queries 42 and 62, 100 queries 61 and 96; 400K x 512, 4 queries 52 and 86; 20K x 1536, 100 queries
+// 89 and 164; 1M x 1536, 12 queries 198 and 236.
+//  - Rows are scored a second time at two table reads a byte: 100 blocks of 12 chunks take 50 us (400K x 768 3-bit, one
+//    query, k = 60: 95 and 85; 60K x 1536, 8 queries, k = 100: 99 and 97; 400K: 133 and 138; 64 queries: 147 and
+//    177; 60K, 400 queries: 309 and 285).
+//  - The matrix-unit scan pays its epilogue on every (block, tile) pair: 400K x 1536, 500 queries (200K pairs) 983 and 1038, 1M x
+//    512 (500K pairs) 1060 and 955.
+// One query of up to 8192 chunks in all, and the matrix-unit scan on rows of up to 16 byte-groups, keep to the sampled
+// path, and not for its speed: they are how the tests of the kernels' append form get there.
+bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+    const size_t nch = size_t(ix->geo.nch), rescored = k_eff * nch, tiles = (std::min(nq, kChunkQueries) + tv::kQTile - 1) / tv::kQTile;
+    if (effective_mode(ix) != TV_SCORE_L_U32 || ix->no_lut16 || tv::pick_lds_bytes(int(nch), k_eff, true) > tv::kPickLds) return false;
+    if (nq == 1) return n_blocks * nch > 8192 && rescored <= 400;
+    if (nq <= size_t(tv::kLut16Queries)) return rescored <= (n_blocks >= 4096 ? 1200u : 720u);
+    if (ix->geo.G <= 16 && lut_mx_serves(ix, nq)) return false;
+    return n_blocks * tiles <= 200000 && rescored <= (tiles <= 4 ? 1200u : 600u);
+}
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
-    if (effective_mode(ix) != TV_SCORE_P || ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
-    if (!tv::best_serves(nch) || k_eff > size_t(tv::kMaxPickK) || k_eff * nch > 600 || n_blocks > tv::kMaxPickBlocks) return false;
-    if (tv::pick_lds_bytes(nch, k_eff) > tv::kPickLds) return false;
+    if (ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
+    if (k_eff > size_t(tv::kMaxPickK) || n_blocks > tv::kMaxPickBlocks) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
+    if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks);
+    if (!tv::best_serves(nch) || k_eff * nch > 600 || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds) return false;
     if (nch == 1 && nq >= 2 && nq <= 8 && n_blocks >= 1536) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
@@ -750,6 +769,28 @@ int take_stamps(tv_index *ix, int launches) {
     ix->last_scan_launches += launches;
     return TV_OK;
 }
+// The unsampled scan of u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
+// whole tables in LDS for a few, tables streamed for up to sixteen (tiles side by side beyond) or the
+// sparse matrix instruction.
+int direct_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
+    const int nch = a.nch;
+    a.k = 1;
+    a.gtau = ix->d_tau_open;
+    if (pq.d_tables_mx != nullptr) {
+        a.tables = pq.d_tables_mx;
+        if (a.mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * a.best_stride, ix->stream));   // (it skips blocks without an allowed row)
+        TV_HIP(tv::launch_scan_lut_mx(a, tv::mx_shape(ix->device, cq, a.n_blocks, false), ix->geo.bits, ix->stream));
+    } else if (pq.d_tables16 != nullptr) {
+        a.tables = pq.d_tables16;
+        const int tiles = int((cq + tv::kLut16Queries - 1) / tv::kLut16Queries);
+        const int grid = int(std::min<size_t>(size_t(tv::device_cus(ix->device)), (size_t(a.n_blocks) + 7) / 8));
+        TV_HIP(tv::launch_scan_lut16(a, grid, tiles, ix->stream));
+    } else {
+        const int grid = int(std::min<size_t>(size_t(tv::lut_append_grid(ix->device, nch)), (size_t(a.n_blocks) + 1) / 2));
+        TV_HIP(tv::launch_scan_lut(a, grid, tv::kModeAppend, ix->stream));
+    }
+    return TV_OK;
+}
 int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
                   int64_t *d_out_idx, bool timing) {
     const tv::Geometry &g = ix->geo;
@@ -757,16 +798,19 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
     int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
     if (rc != TV_OK) return rc;
     ix->last_queries_per_launch = int(chunk_len(ix, nq));
+    if (effective_mode(ix) != TV_SCORE_P && !lut_mx_serves(ix, chunk_len(ix, nq)))
+        ix->last_queries_per_launch = std::min(ix->last_queries_per_launch, tv::kLut16Queries);     // (a pass serves so many; passes share a launch)
     for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
         const size_t gq = std::min(kGroupQueries, nq - g0);
         for (size_t c0 = 0, cq; c0 < gq; c0 += cq) {
             cq = chunk_len(ix, gq - c0);
             const size_t q0 = g0 + c0;
-            const bool timed = timing && q0 == 0, wide = direct_wide(ix, cq, n_blocks), split = wide && tv::wide_weights_split(g.nch);
+            const bool mode_p = effective_mode(ix) == TV_SCORE_P, timed = timing && q0 == 0;
+            const bool wide = mode_p && direct_wide(ix, cq, n_blocks), split = wide && tv::wide_weights_split(g.nch);
             Arena ar;
             ar.base = static_cast<uint8_t *>(ix->ws);
             Prepared pq;
-            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, false, timed ? ix->d_stamps : nullptr);
+            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, true, timed ? ix->d_stamps : nullptr);
             if (rc != TV_OK) return rc;
             tv::ScanArgs a;
             fill_scan_args(ix, a);
@@ -782,10 +826,13 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                 a.best_of_block = 1;
                 if (d_mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * stride, ix->stream));   // (it skips blocks without an allowed row)
                 TV_HIP(tv::launch_scan_p4_wide(a, tv::wide_grid_blocks(ix->device), ix->stream));
-            } else {
+            } else if (mode_p) {
                 TV_HIP(tv::launch_scan_p4_best(a, ix->device, ix->stream));
+            } else {
+                rc = direct_scan_lut(ix, a, pq, cq);
+                if (rc != TV_OK) return rc;
             }
-            TV_HIP(tv::launch_pick(a, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
+            TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
                                    timed ? ix->d_stamps + 1 : nullptr, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));

@@ -112,7 +112,7 @@ struct PrepRequest {
     uint8_t *tables;
     float *qscale, *qbias;
     float *rot_out;                 // or null
-    uint64_t *stamp;                // or null (permute-dot only)
+    uint64_t *stamp;                // or null
 };
 hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s);
 
@@ -148,11 +148,11 @@ hipError_t launch_scan_p4(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Small indexes without sampling (tv_kernels6.hip): the best row of every block, then the best blocks' rows.
 constexpr int kMaxPickK = 128;             // most results k_pick ranks
 constexpr size_t kMaxPickBlocks = 32768;   // most blocks it chooses from
-constexpr size_t kPickLds = 128 * 1024;    // beside its 13 KiB of fixed buffers
+constexpr size_t kPickLds = 128 * 1024;    // rows' keys and the query's tables, beside its 13 KiB of fixed buffers
 bool best_serves(int nch);
 hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s);
-size_t pick_lds_bytes(int nch, size_t k_eff);
-hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
+size_t pick_lds_bytes(int nch, size_t k_eff, bool lut);
+hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
                        hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).

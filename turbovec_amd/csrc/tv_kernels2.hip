@@ -183,6 +183,7 @@ __global__ __launch_bounds__(THREADS) void k_scan_lut(ScanArgs a) {
             const uint32_t b = j * step;
             const uint64_t w = a.mask[b >> 1];
             if (uint32_t(w >> ((b & 1) * 32)) != 0u) break;
+            if (APPEND && a.best_out != nullptr && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = 0u;
             j += total_waves;
         }
         return j;
@@ -342,7 +343,18 @@ __global__ __launch_bounds__(THREADS) void k_scan_lut(ScanArgs a) {
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
             __builtin_amdgcn_wave_barrier();
-            if (APPEND) {
+            if (APPEND && a.best_out != nullptr) {
+                // a search without sampling (tv_kernels6.hip): the block's best score per query, no slot
+                float m = -__int_as_float(0x7f800000);
+#pragma unroll
+                for (int e = 0; e < per; ++e) {
+                    const int i = (vg * per + e) & 31;
+                    if (slot0 + i < a.n && ((mw >> i) & 1u)) m = fmaxf(m, my_sct[oq * 32 + i]);   // (NaN never wins)
+                }
+#pragma unroll
+                for (int d = QL; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+                if (lane < QL && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = best_word(m);
+            } else if (APPEND) {
 #pragma unroll
                 for (int e = 0; e < per; ++e) {
                     const int i = (vg * per + e) & 31;
@@ -382,7 +394,7 @@ __global__ __launch_bounds__(THREADS) void k_scan_lut(ScanArgs a) {
 
     if (APPEND) {
         __syncthreads();
-        if (tid < a.nq_tile) a.cand_cnt[size_t(tid) * a.seg_stride + blockIdx.x] = scnt[tid];
+        if (tid < a.nq_tile && a.best_out == nullptr) a.cand_cnt[size_t(tid) * a.seg_stride + blockIdx.x] = scnt[tid];
     }
     if (LISTS) {
         const size_t total_threads = size_t(gridDim.x) * THREADS;
@@ -451,6 +463,7 @@ __global__ __launch_bounds__(kLutBtThreads) void k_scan_lut_bt(ScanArgs a, int n
         while (j < nj) {
             const uint32_t b = j * step;
             if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
+            if (a.best_out != nullptr && lane == 0) a.best_out[b] = 0u;
             j += total_waves;
         }
         return j;
@@ -522,7 +535,11 @@ __global__ __launch_bounds__(kLutBtThreads) void k_scan_lut_bt(ScanArgs a, int n
             // classic: fa * vec_scale; u32: ((f32(acc) * scale) + bias) * vec_scale (search.rs:1174-1177)
             sc = a.classic == 1 ? fa * vs : ((float(int(total)) * qs) + qb) * vs;
         }
-        if (a.best_of_block) {
+        if (a.best_out != nullptr) {
+            // a search without sampling (tv_kernels6.hip): the block's best score, no slot
+            const uint32_t m = wave_umax(allowed && sc == sc ? best_word(sc) : 0u);
+            if (lane == 0) a.best_out[b] = m;
+        } else if (a.best_of_block) {
             // A first sampling level without a floor: the block's best allowed row (score order, then
             // the lower slot: the larger sort key), one candidate per block -- a real score of a real
             // row, so the k-th best of these is a floor k scanned rows reach.
@@ -545,7 +562,7 @@ __global__ __launch_bounds__(kLutBtThreads) void k_scan_lut_bt(ScanArgs a, int n
         j = nj_live;
     }
     __syncthreads();
-    if (tid == 0) a.cand_cnt[blockIdx.x] = *scnt;
+    if (tid == 0 && a.best_out == nullptr) a.cand_cnt[blockIdx.x] = *scnt;
 }
 
 // Chunks of a row that get byte tables when `budget` bytes of LDS are available, and the bytes used.

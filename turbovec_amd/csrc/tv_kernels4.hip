@@ -87,7 +87,9 @@ __device__ __forceinline__ void lut_wait(v4i &r) {
 // float every 256 byte-groups -- four pairs of chunks -- with fma(scale, f32(sum), fa), fa starting
 // at the bias; the score is fa * vec_scale.  (Its sixteen running floats per block take the
 // registers of the second block and of two reads in flight.)
-template <int RB, bool CLASSIC, int kLutAhead>
+// BEST: a search without sampling (tv_kernels6.hip), every block's best score per query; one block per wave, as two and
+// the maximum would spill two registers.
+template <int RB, bool CLASSIC, int kLutAhead, bool BEST>
 __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     if (launch_switched_off(a.run_if)) return;
@@ -104,6 +106,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
         a.gtau += ty * kQTile;
         a.cand += ty * kLut16Queries * a.seg_stride * kSegCap;
         a.cand_cnt += ty * kLut16Queries * a.seg_stride;
+        if (BEST) a.best_out += ty * kLut16Queries * a.best_stride;
         a.nq_tile -= int(ty) * kLut16Queries;
     }
     if (a.nq_tile > kLut16Queries) a.nq_tile = kLut16Queries;
@@ -148,6 +151,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
         while (j < nj) {
             const uint32_t b = j * step;
             if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
+            if (BEST && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = 0u;
             j += total_waves;
         }
         return j;
@@ -259,6 +263,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
             const uint32_t b = blk[i];
             uint32_t mw = 0xffffffffu;
             if (a.mask != nullptr) mw = uint32_t(a.mask[b >> 1] >> ((b & 1) * 32));
+            float best = -__int_as_float(0x7f800000);      // (a search without sampling: the block's best score per query)
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
                 const int v0 = 16 * half + 4 * kb;
@@ -268,17 +273,25 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
                 for (int rr = 0; rr < 4; ++rr) {
                     const uint32_t slot = b * 32u + uint32_t(v0 + rr);
                     const float s = CLASSIC ? fa[i][half][rr] * vsr[rr] : ((float(acc[i][half][rr]) * qs) + qb) * vsr[rr];
-                    if (s >= tau && slot < a.n && ((mw >> (v0 + rr)) & 1u)) {
+                    const bool allowed = slot < a.n && ((mw >> (v0 + rr)) & 1u);
+                    if (BEST) {
+                        if (allowed) best = fmaxf(best, s);                  // (NaN never wins)
+                    } else if (s >= tau && allowed) {
                         const uint32_t pos = atomicAdd(&scnt[r], 1u);
                         if (pos < kSegCap) a.cand[(size_t(r) * a.seg_stride + blockIdx.x) * kSegCap + pos] = sort_key(s, slot);
                         else if (pos == kSegCap) atomicAdd(s_over, 1u);      // the one append that finds the segment just full
                     }
                 }
             }
+            if (BEST) {
+                best = fmaxf(best, __shfl_xor(best, 16));
+                best = fmaxf(best, __shfl_xor(best, 32));
+                if (kb == 0 && qact) a.best_out[size_t(r) * a.best_stride + b] = best_word(best);
+            }
         }
     }
     __syncthreads();
-    if (tid < a.nq_tile) a.cand_cnt[size_t(tid) * a.seg_stride + blockIdx.x] = scnt[tid];
+    if (!BEST && tid < a.nq_tile) a.cand_cnt[size_t(tid) * a.seg_stride + blockIdx.x] = scnt[tid];
 }
 
 constexpr int kLut16RoundBlocks = 2, kLut16RoundBlocksClassic = 1;   // per wave
@@ -289,7 +302,7 @@ int lut16_blocks_per_workgroup(bool classic) { return kLut16Threads / 64 * (clas
 // scales and candidate segments those of the first tile, the others' following at the strides of
 // the chunk's layout; a.classic 0 (u32 epilogue) or 1 (classic).
 hipError_t launch_scan_lut16(const ScanArgs &a, int grid, int tiles, hipStream_t s) {
-    if ((a.classic != 0 && a.classic != 1) || tiles < 1 || a.nq_tile <= (tiles - 1) * kLut16Queries || a.nq_tile > tiles * kLut16Queries)
+    if ((a.classic != 0 && (a.classic != 1 || a.best_out != nullptr)) || tiles < 1 || a.nq_tile <= (tiles - 1) * kLut16Queries || a.nq_tile > tiles * kLut16Queries)
         return hipErrorInvalidValue;
     const size_t lds = 2 * size_t(kLut16PairBytes) + 128;
     auto launch = [&](auto kernel) -> hipError_t {
@@ -298,7 +311,8 @@ hipError_t launch_scan_lut16(const ScanArgs &a, int grid, int tiles, hipStream_t
         hipLaunchKernelGGL(kernel, dim3(grid, tiles), dim3(kLut16Threads), lds, s, a);
         return hipSuccess;
     };
-    hipError_t e = a.classic == 1 ? launch(k_scan_lut16<kLut16RoundBlocksClassic, true, 6>) : launch(k_scan_lut16<kLut16RoundBlocks, false, 6>);
+    hipError_t e = a.best_out != nullptr ? launch(k_scan_lut16<1, false, 6, true>)
+                 : a.classic == 1 ? launch(k_scan_lut16<kLut16RoundBlocksClassic, true, 6, false>) : launch(k_scan_lut16<kLut16RoundBlocks, false, 6, false>);
     if (e != hipSuccess) return e;
     return hipGetLastError();
 }

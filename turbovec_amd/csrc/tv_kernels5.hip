@@ -434,6 +434,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
             m1 = max(max(m1, v[14]), v[15]);
             if (__any(max(max(m0, m1), max(m2, m3)) >= bound)) hits |= 1u << decltype(ii)::value;
         });
+        if (a.best_out != nullptr) hits = (1u << (BLK * NT)) - 1u;         // (a search without sampling: every pair's best score)
         // (One body for all pairs, on a copy of the sums: unrolled, it would outgrow the instruction cache.)
 #pragma unroll 1
         while (hits != 0u) {
@@ -450,6 +451,14 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
             const int bound = bound_of(i, inv, k);
             const float qs = sq[i].qs, qb = sq[i].qb, tau = sq[i].tau;
             const float *vs = s_vs + (wave * BLK + k) * 32 + 4 * h;
+            if (a.best_out != nullptr) {
+                float m = -__int_as_float(0x7f800000);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) m = fmaxf(m, ((float(v[r]) * qs) + qb) * vs[8 * (r >> 2) + (r & 3)]);     // (NaN never wins)
+                m = fmaxf(m, __shfl_xor(m, 32));
+                if (h == 0 && q0 + i < a.nq_tile && jb < nj) a.best_out[size_t(q0 + i) * a.best_stride + block_of(jb)] = best_word(m);
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 if (v[r] >= bound) {
@@ -473,6 +482,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
         for (int k = 0; k < BLK; ++k) blk[k] = nblk[k];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // requests still in flight write this workgroup's LDS
+    if (a.best_out != nullptr) return;
     __syncthreads();
     for (int i = tid; i < kQ * int(sub); i += kMxThreads) {
         const int q = q0 + i % kQ, sb = i / kQ;
@@ -521,7 +531,7 @@ static hipError_t launch_mx_blk(const ScanArgs &a, const MxShape &m, hipStream_t
 // One append-mode launch: a.nq_tile = all queries of the chunk, a.tables = their B operands
 // (k_lut_fragments), scales, floors and segments by query.
 hipError_t launch_scan_lut_mx(const ScanArgs &a, const MxShape &m, int bits, hipStream_t s) {
-    if (a.classic != 0 || a.nq_tile <= 0 || size_t(m.wgs) * m.sub > a.seg_stride) return hipErrorInvalidValue;
+    if (a.classic != 0 || a.nq_tile <= 0 || (a.best_out == nullptr && size_t(m.wgs) * m.sub > a.seg_stride)) return hipErrorInvalidValue;
     if (bits == 3) return m.nt == 1 ? launch_mx_blk<8, 1>(a, m, s) : launch_mx_blk<8, 2>(a, m, s);
     return m.nt == 1 ? launch_mx_blk<16, 1>(a, m, s) : launch_mx_blk<16, 2>(a, m, s);
 }

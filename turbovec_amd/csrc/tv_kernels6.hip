@@ -204,7 +204,8 @@ struct PickArgs {
     uint64_t *stamp;
 };
 // H: blocks a thread keeps in registers -- all of them, T * H at most.
-template <uint32_t T, uint32_t H>
+// LUT: score mode L with the u32 epilogue.
+template <uint32_t T, uint32_t H, bool LUT>
 __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     constexpr uint32_t W = T / 64;
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -222,9 +223,15 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
 #pragma unroll
     for (uint32_t e = 0; e < H; ++e) v[e] = e * T + t < a.n_blocks ? best[e * T + t] : 0u;
     // the tile's weights lie [chunk][fragment][half * 32 + query] in 16-byte pieces; here [chunk][half][fragment]
-    const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
-    for (int i = int(t); i < a.nch * 4; i += int(T))
-        reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
+    if constexpr (LUT) {
+        // (two tables of 16 entries per byte-group, as they are)
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi) * a.nch * 64;
+        for (int i = int(t); i < a.nch * 64; i += int(T)) reinterpret_cast<uint4 *>(wts)[i] = src[i];
+    } else {
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(qi / kQTile) * a.nch * 128 + qi % kQTile;
+        for (int i = int(t); i < a.nch * 4; i += int(T))
+            reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
+    }
     for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     if (t == 0) { n_kept = 0u; n_list = 0u; s_floor = 0u; }
     auto each = [&](auto &&f) {
@@ -279,6 +286,15 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
             for (int u = 0; u < kBurst; ++u) {
                 if (c0 + u >= a.nch) break;
                 const uint32_t d[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+                if constexpr (LUT) {
+                    const uint8_t *row = wts + ((c0 + u) * 32 + int(h) * 16) * 32;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const uint32_t byte = (d[e >> 2] >> (8 * (e & 3))) & 0xffu;
+                        acc += int(row[e * 32 + int(byte >> 4)]) + int(row[e * 32 + 16 + int(byte & 15u)]);
+                    }
+                    continue;
+                }
                 const uint4 *wq = reinterpret_cast<const uint4 *>(wts) + ((c0 + u) * 2 + h) * 2;
                 const uint4 f0 = wq[0], f1 = wq[1];
                 uint32_t lo[4], hi[4];
@@ -309,7 +325,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
             }
         }
         acc += __shfl_xor(acc, 32);
-        const float s = fmaf(float(acc), qs, qb) * vs;
+        const float s = LUT ? ((float(acc) * qs) + qb) * vs : fmaf(float(acc), qs, qb) * vs;      // search.rs:1174-1177, 1519-1524
         // (A score of -infinity does not count here either, as it does not in a block's best word: rows that tie there
         // with rows of blocks that were not chosen are for the exact path to order.)
         bool ok = lane < 32u && slot < a.n && s > -__int_as_float(0x7f800000);
@@ -357,13 +373,13 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     }
 }
 
-size_t pick_lds_bytes(int nch, size_t k_eff) { return k_eff * 32 * 8 + size_t(nch) * 64; }
+size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64); }
 
-// The scan's arguments say what was scanned; a.tables: its weight tiles.
-hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
+// The scan's arguments say what was scanned; a.tables: its weight tiles, or (lut) the queries' tables as k_prep_lut leaves them.
+hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
                        hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
-    const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff));
+    const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff), lut);
     if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
     PickArgs p;
     p.best = a.best_out; p.best_stride = a.best_stride; p.n_blocks = a.n_blocks; p.n = a.n;
@@ -379,9 +395,9 @@ hipError_t launch_pick(const ScanArgs &a, bool split, int k_eff, float *out_scor
         return hipGetLastError();
     };
     // few queries leave the chip empty: as many waves as there are blocks to score again
-    if (a.n_blocks > 1024 * 16) return launch(k_pick<1024, 32>, 1024);
-    if (a.nq_tile <= 256 || a.n_blocks > 256 * 16) return launch(k_pick<1024, 16>, 1024);
-    return launch(k_pick<256, 16>, 256);
+    const bool small = a.nq_tile > 256 && a.n_blocks <= 256 * 16;
+    if (lut) return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, true>, 1024) : small ? launch(k_pick<256, 16, true>, 256) : launch(k_pick<1024, 16, true>, 1024);
+    return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, false>, 1024) : small ? launch(k_pick<256, 16, false>, 256) : launch(k_pick<1024, 16, false>, 1024);
 }
 
 }  // namespace tv
