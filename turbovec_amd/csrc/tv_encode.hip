@@ -278,8 +278,9 @@ __device__ __forceinline__ float enc_in_order(const float (&v)[NG][8], const Rec
 // row, 0.50 with the f64 chains too in one wave and four levels of three comparisons per value, 0.39 now (1.8 TB/s, every
 // byte once); of 2048: 1.15 -> 0.62.
 // CAL: there is a TQ+ pair.
+constexpr int enc_waves_per_simd(int ng) { return ng == 1 ? 6 : ng == 2 ? 5 : ng <= 4 ? 4 : 2; }    // what their registers leave room for
 template <int NG, int W, bool CAL>
-__global__ __launch_bounds__(W * 64, NG <= 4 ? 4 : 2) void k_encode_rows(EncodeRowsArgs a) {
+__global__ __launch_bounds__(W * 64, enc_waves_per_simd(NG)) void k_encode_rows(EncodeRowsArgs a) {
     extern __shared__ __align__(16) float enc_lds[];
     const int dim = a.dim, t = threadIdx.x, ng = dim / 8, rs = a.row_stride, L = a.lanes;
     const int R = W * 64 / L;                                      // rows of a workgroup
@@ -547,10 +548,8 @@ static hipError_t launch_encode_rows_cal(const EncodeRowsArgs &a, int device, hi
     hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     // a workgroup keeps its tables for all its turns: as many as are resident at once, by registers and LDS
-    int per_cu = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, W * 64, lds);
-    if (e != hipSuccess) return e;
-    const size_t groups = (a.n_new + R - 1) / R, resident = size_t(device_cus(device)) * size_t(std::max(1, per_cu));
+    const size_t groups = (a.n_new + R - 1) / R;
+    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(4 * enc_waves_per_simd(NG)) / W, 160 * 1024 / lds));
     hipLaunchKernelGGL((k_encode_rows<NG, W, CAL>), dim3(unsigned(std::min(groups, resident))), dim3(W * 64), lds, s, a);
     return hipGetLastError();
 }
