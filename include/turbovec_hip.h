@@ -154,6 +154,13 @@ int tv_search(tv_index *ix, const float *queries, size_t nq, size_t k,
               const uint64_t *mask_words, size_t n_mask_words,
               float *out_scores, int64_t *out_indices, size_t *out_k_eff);
 
+/* tv_validate_queries and tv_search in one: the values checked are the snapshot of them that is searched
+ * (turbovec-python/src/lib.rs:617-629 copies the array first for that).  On TV_ERR_INVALID_QUERY_VALUE
+ * *bad_index is the flat offset and nothing is searched. */
+int tv_search_checked(tv_index *ix, const float *queries, size_t nq, size_t k,
+                      const uint64_t *mask_words, size_t n_mask_words,
+                      float *out_scores, int64_t *out_indices, size_t *out_k_eff, size_t *bad_index);
+
 /* Same, with queries, mask words and outputs already in device memory and the
  * mask's popcount supplied by the caller (the reference's caller counts it
  * while packing, lib.rs:1446).  Returns after the work is enqueued and

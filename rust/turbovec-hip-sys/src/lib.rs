@@ -66,6 +66,7 @@ extern "C" {
     pub fn tv_validate_queries(queries: *const c_float, len: usize, dim: c_int, bad_index: *mut usize) -> c_int;
     pub fn tv_pack_mask(mask_bytes: *const u8, n: usize, words_out: *mut u64, n_allowed: *mut usize) -> c_int;
     pub fn tv_search(ix: *mut tv_index, queries: *const c_float, nq: usize, k: usize, mask_words: *const u64, n_mask_words: usize, out_scores: *mut c_float, out_indices: *mut i64, out_k_eff: *mut usize) -> c_int;
+    pub fn tv_search_checked(ix: *mut tv_index, queries: *const c_float, nq: usize, k: usize, mask_words: *const u64, n_mask_words: usize, out_scores: *mut c_float, out_indices: *mut i64, out_k_eff: *mut usize, bad_index: *mut usize) -> c_int;
     pub fn tv_search_dev(ix: *mut tv_index, d_queries: *const c_float, nq: usize, k: usize, d_mask_words: *const u64, n_allowed: usize, d_out_scores: *mut c_float, d_out_indices: *mut i64, out_k_eff: *mut usize) -> c_int;
     pub fn tv_search_dev_noalloc(ix: *mut tv_index, d_queries: *const c_float, nq: usize, k: usize, d_mask_words: *const u64, n_allowed: usize, d_out_scores: *mut c_float, d_out_indices: *mut i64, out_k_eff: *mut usize) -> c_int;
     pub fn tv_noalloc_scratch_bytes() -> usize;

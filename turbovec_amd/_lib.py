@@ -28,7 +28,7 @@ EXPORTS = [
     "tv_status_string", "tv_last_error", "tv_index_create", "tv_index_destroy", "tv_index_set_tables",
     "tv_index_set_calibration", "tv_index_set_score_mode", "tv_index_get_tables", "tv_index_upload_seq",
     "tv_index_upload_seq_dev", "tv_index_append_rows", "tv_index_add", "tv_index_add_dev", "tv_index_calibrate", "tv_index_get_calibration", "tv_index_swap_remove", "tv_index_download_seq", "tv_index_len", "tv_index_dim",
-    "tv_index_bits", "tv_validate_queries", "tv_pack_mask", "tv_search", "tv_search_dev", "tv_debug_scan",
+    "tv_index_bits", "tv_validate_queries", "tv_pack_mask", "tv_search", "tv_search_checked", "tv_search_dev", "tv_debug_scan",
     "tv_debug_prepare", "tv_last_scan_ms", "tv_debug_queries_per_launch", "tv_index_device_ptrs", "tv_host_rotation_tables", "tv_host_codebook",
     "tv_debug_stream_probe", "tv_debug_mfma_probe", "tv_debug_set_path", "tv_debug_overflow_redos",
     "tv_host_snapshot_len", "tv_host_snapshot_compose", "tv_host_snapshot_info", "tv_host_snapshot_extract",
@@ -40,8 +40,9 @@ _lib = None
 
 
 class TurbovecHipError(RuntimeError):
-    def __init__(self, status, detail=""):
+    def __init__(self, status, detail="", bad_index=None):
         self.status = status
+        self.bad_index = bad_index           # of a refused value, where the call reports it
         super().__init__(f"turbovec_hip status {status}: {detail}")
 
 
@@ -88,6 +89,7 @@ def lib():
     L.tv_validate_queries.argtypes = [vp, sz, i32, C.POINTER(sz)]
     L.tv_pack_mask.argtypes = [vp, sz, vp, C.POINTER(sz)]
     L.tv_search.argtypes = [vp, vp, sz, sz, vp, sz, vp, vp, C.POINTER(sz)]
+    L.tv_search_checked.argtypes = [vp, vp, sz, sz, vp, sz, vp, vp, C.POINTER(sz), C.POINTER(sz)]
     L.tv_search_dev.argtypes = [vp, vp, sz, sz, vp, sz, vp, vp, C.POINTER(sz)]
     L.tv_search_dev_noalloc.argtypes = [vp, vp, sz, sz, vp, sz, vp, vp, C.POINTER(sz)]
     L.tv_noalloc_scratch_bytes.restype = sz
@@ -253,17 +255,24 @@ class NativeIndex:
         check(lib().tv_index_download_seq(self.h, ptr(seq), ptr(sc)))
         return seq, sc
 
-    def search(self, queries, k, mask_words=None):
+    def search(self, queries, k, mask_words=None, checked=False):
+        """tv_search, or with `checked` tv_search_checked (an error of status ERR_INVALID_QUERY_VALUE has the place)."""
         q = np.ascontiguousarray(queries, np.float32).reshape(-1, self.dim)
         nq = q.shape[0]
         n = len(self)
         cap = min(k, n)
-        out_s = np.zeros((nq, cap), np.float32)
-        out_i = np.zeros((nq, cap), np.int64)
-        k_eff = C.c_size_t(0)
+        out_s = np.empty((nq, cap), np.float32)
+        out_i = np.empty((nq, cap), np.int64)
+        k_eff, bad = C.c_size_t(0), C.c_size_t(0)
         mw = None if mask_words is None else np.ascontiguousarray(mask_words, np.uint64)
-        check(lib().tv_search(self.h, ptr(q), nq, k, ptr(mw), 0 if mw is None else mw.size, ptr(out_s), ptr(out_i),
-                              C.byref(k_eff)))
+        args = (self.h, ptr(q), nq, k, ptr(mw), 0 if mw is None else mw.size, ptr(out_s), ptr(out_i), C.byref(k_eff))
+        if checked:
+            rc = lib().tv_search_checked(*args, C.byref(bad))
+            if rc == ERR_INVALID_QUERY_VALUE:
+                raise TurbovecHipError(rc, "invalid query value", bad.value)
+            check(rc)
+        else:
+            check(lib().tv_search(*args))
         ke = k_eff.value
         if ke == cap:
             return out_s, out_i

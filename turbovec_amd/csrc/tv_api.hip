@@ -206,6 +206,67 @@ int ensure_io(tv_index *ix, size_t bytes) {
     return TV_OK;
 }
 
+// ---- host arrays ---------------------------------------------------------------------------------
+// A copy from or to pageable memory is staged by the runtime, on one thread and with a wait of its own: 500 KB 30 us, 614 MB
+// 20 to 39 ms.  Here calls on host arrays pass through pinned blocks that belong to the index: queries are copied in
+// on the calling thread -- the snapshot of them that the search then reads -- and read by the device where they lie,
+// results are written there by the last kernel; rows to add go through in pieces, several threads filling.  Through the Python
+// surface, before and now: one query over 100K x 128 73 us and 37, 1000 queries 138 and 101, 1024 of 3072 dimensions 2.41 ms and 1.22; 100K
+// x 1536 rows to an image 37.9 ms and 21.5.
+constexpr size_t kPinnedBytes = size_t(128) << 20, kPinnedLargest = size_t(32) << 20;
+constexpr size_t kReadInPlace = size_t(1) << 20;      // larger sets of queries are copied to the device first, by the copy engine
+
+// A block of at least `bytes`, or null: none to spare, or none to be had (the caller then does without).  The index's device is current.
+tv_pinned *pinned_take(tv_index *ix, size_t bytes) {
+    if (bytes > kPinnedLargest) return nullptr;
+    size_t want = size_t(64) << 10;
+    while (want < bytes) want *= 2;
+    std::lock_guard<std::mutex> lock(ix->pinned_mu);
+    size_t total = 0;
+    tv_pinned *fits = nullptr, *spare = nullptr;
+    for (tv_pinned &b : ix->pinned) {
+        total += b.bytes;
+        if (b.lent) continue;
+        if (b.bytes >= want && (!fits || b.bytes < fits->bytes)) fits = &b;
+        if (b.bytes < want && (!spare || b.bytes < spare->bytes)) spare = &b;
+    }
+    if (fits) { fits->lent = true; return fits; }
+    if (!spare || total - spare->bytes + want > kPinnedBytes) return nullptr;
+    if (spare->host) (void)hipHostFree(spare->host);
+    *spare = tv_pinned{};
+    void *host = nullptr, *dev = nullptr;
+    if (hipHostMalloc(&host, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (hipHostGetDevicePointer(&dev, host, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(host); return nullptr; }
+    spare->host = static_cast<uint8_t *>(host);
+    spare->dev = static_cast<uint8_t *>(dev);
+    spare->bytes = want;
+    spare->lent = true;
+    return spare;
+}
+struct PinnedLoan {      // given back when it goes out of scope; whoever reads or writes the block has finished by then
+    tv_index *ix;
+    tv_pinned *b;
+    PinnedLoan(tv_index *ix_, size_t bytes) : ix(ix_), b(pinned_take(ix_, bytes)) {}
+    PinnedLoan(const PinnedLoan &) = delete;
+    ~PinnedLoan() {
+        if (!b) return;
+        std::lock_guard<std::mutex> lock(ix->pinned_mu);
+        b->lent = false;
+    }
+};
+// Copies values and says whether any of the copied ones is not finite or 1e16 or larger (tv_validate_queries).
+bool copy_checked(float *to, const float *from, size_t n) {
+    constexpr size_t kRun = 4096;      // copied, then looked at while in the first-level cache
+    uint32_t any = 0;
+    for (size_t r = 0; r < n; r += kRun) {
+        const size_t m = std::min(kRun, n - r);
+        std::memcpy(to + r, from + r, m * sizeof(float));
+        const uint32_t *v = reinterpret_cast<const uint32_t *>(to + r);
+        for (size_t i = 0; i < m; ++i) any |= uint32_t(int32_t(v[i] & 0x7fffffffu) >= int32_t(kTooLargeBits));
+    }
+    return any != 0;
+}
+
 int ensure_capacity(tv_index *ix, size_t n_vectors) {
     const size_t blocks = (n_vectors + tv::kVecBlock - 1) / tv::kVecBlock;
     if (blocks <= ix->cap_blocks) return TV_OK;
@@ -1155,6 +1216,11 @@ struct tv_request {
     size_t mask_arg = 0;           // host: number of mask words; device: the mask's popcount
     float *out_s = nullptr;
     int64_t *out_i = nullptr;
+    // host arrays that have been staged in pinned memory (q, out_s, out_i and staged_mask point into it): the device's addresses
+    const uint64_t *staged_mask = nullptr;     // (mask stays the caller's: calls with one mask are told by its address)
+    const float *dev_q = nullptr;  // or null: not staged
+    float *dev_s = nullptr;
+    int64_t *dev_i = nullptr;
     size_t k_eff = 0;
     int rc = TV_OK;
     std::string err;
@@ -1205,7 +1271,7 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
         TV_HIP(hipStreamSynchronize(ix->stream));
         return TV_OK;
     }
-    const uint64_t *mask_words = r0.mask;
+    const uint64_t *mask_words = r0.staged_mask ? r0.staged_mask : r0.mask;
     const size_t n_mask_words = r0.mask_arg;
     size_t n_allowed = n;
     if (mask_words) {
@@ -1222,21 +1288,24 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
     ix->last_scan_ms = 0.0f;
     ix->last_scan_launches = 0;
     if (k_eff == 0 || nq == 0) return TV_OK;
-    // host staging: queries, mask and results live in the index's own staging allocation (kept
-    // between calls, so a search allocates nothing once it has seen its largest batch), apart
-    // from the per-chunk workspace, which is re-carved freely
-    const size_t q_bytes = round_up(nq * dim * sizeof(float), 256), s_bytes = round_up(nq * k_eff * sizeof(float), 256);
-    const size_t i_bytes = round_up(nq * k_eff * sizeof(int64_t), 256), m_bytes = mask_words ? round_up(n_mask_words * 8, 256) : 0;
+    // The device reads a staged caller's queries and writes its results where they lie (a large set of queries is
+    // copied over first); several callers' are gathered on the device, as are arrays that are not staged, in an
+    // allocation the index keeps between calls, apart from the per-chunk workspace, which is re-carved freely.
+    const bool in_place = batch.size() == 1 && r0.dev_q != nullptr;
+    const bool read_in_place = in_place && nq * dim * sizeof(float) <= kReadInPlace;
+    const size_t q_bytes = read_in_place ? 0 : round_up(nq * dim * sizeof(float), 256), m_bytes = mask_words ? round_up(n_mask_words * 8, 256) : 0;
+    const size_t s_bytes = in_place ? 0 : round_up(nq * k_eff * sizeof(float), 256), i_bytes = in_place ? 0 : round_up(nq * k_eff * sizeof(int64_t), 256);
     int rc = ensure_io(ix, q_bytes + s_bytes + i_bytes + m_bytes);
     if (rc != TV_OK) return rc;
     uint8_t *base = static_cast<uint8_t *>(ix->io);
-    float *d_q = reinterpret_cast<float *>(base);
-    float *d_s = reinterpret_cast<float *>(base + q_bytes);
-    int64_t *d_i = reinterpret_cast<int64_t *>(base + q_bytes + s_bytes);
+    const float *d_q = read_in_place ? r0.dev_q : reinterpret_cast<float *>(base);
+    float *d_s = in_place ? r0.dev_s : reinterpret_cast<float *>(base + q_bytes);
+    int64_t *d_i = in_place ? r0.dev_i : reinterpret_cast<int64_t *>(base + q_bytes + s_bytes);
     uint64_t *d_m = mask_words ? reinterpret_cast<uint64_t *>(base + q_bytes + s_bytes + i_bytes) : nullptr;
     size_t at = 0;
     for (const tv_request *r : batch) {
-        if (r->nq && hipMemcpyAsync(d_q + at * dim, r->q, r->nq * dim * sizeof(float), hipMemcpyHostToDevice, ix->stream) != hipSuccess) {
+        if (read_in_place) break;
+        if (r->nq && hipMemcpyAsync(reinterpret_cast<float *>(base) + at * dim, r->q, r->nq * dim * sizeof(float), hipMemcpyHostToDevice, ix->stream) != hipSuccess) {
             g_last_error = "host to device copy failed";
             return TV_ERR_HIP;
         }
@@ -1247,7 +1316,7 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
         return TV_ERR_HIP;
     }
     rc = search_device(ix, d_q, nq, r0.k, d_m, n_allowed, d_s, d_i, nullptr);
-    if (rc != TV_OK) return rc;
+    if (rc != TV_OK || in_place) return rc;
     at = 0;
     for (const tv_request *r : batch) {
         if (r->nq && (hipMemcpyAsync(r->out_s, d_s + at * k_eff, r->nq * k_eff * sizeof(float), hipMemcpyDeviceToHost, ix->stream) != hipSuccess ||
@@ -1326,6 +1395,8 @@ int search_merged(tv_index *ix, tv_request &r) {
         std::lock_guard<std::mutex> lock(ix->mu);   // against the entry points that change the index
         g_last_error.clear();
         rc = serve_batch(ix, batch, &k_eff);
+        // (staged arrays go back to their pool: nothing may still be on its way from or to them)
+        if (rc != TV_OK) (void)hipStreamSynchronize(ix->stream);
     }
     {
         std::lock_guard<std::mutex> reg(ix->waiting_mu);
@@ -1468,6 +1539,7 @@ int tv_index_destroy(tv_index *ix) {
         free_blocks(blocks);
     }
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
+    for (tv_pinned &b : ix->pinned) if (b.host) (void)hipHostFree(b.host);
     if (ix->events_ready)
         for (int i = 0; i < tv::kTimedLaunches; ++i) {
             (void)hipEventDestroy(ix->ev_start[i]);
@@ -1640,29 +1712,113 @@ int tv_index_add_dev(tv_index *ix, const float *d_vectors, size_t n_new) {
     return add_device_rows(ix, d_vectors, n_new);
 }
 
+// Rows on their way to the device, checked as they pass through pinned memory, a few megabytes at a time: each of up
+// to four threads fills its piece while the others' are copied (614 MB: 13 ms, at the rate of the bus; fresh pageable memory 20 to 39, and
+// a pass over it for the check).  *bad: a value was refused; the rest need not have arrived.  Met with the index's lock held.
+static int stage_rows(tv_index *ix, const float *rows, size_t values, float *d_rows, bool *bad) {
+    constexpr size_t kPiece = (size_t(4) << 20) / sizeof(float), kThreads = 4;
+    *bad = false;
+    const size_t pieces = (values + kPiece - 1) / kPiece, threads = std::min<size_t>(kThreads, pieces);
+    PinnedLoan loan(ix, threads * std::min(kPiece, values) * sizeof(float));
+    if (!loan.b) {
+        *bad = tv_validate_queries(rows, values, 1, nullptr) != TV_OK;
+        if (!*bad) TV_HIP(hipMemcpyAsync(d_rows, rows, values * sizeof(float), hipMemcpyHostToDevice, ix->stream));
+        return TV_OK;
+    }
+    std::atomic<size_t> next{0};
+    std::atomic<bool> refused{false}, failed{false};
+    in_parts(threads, 1, [&](size_t lo, size_t hi) {
+        if (lo == hi) return;
+        if (hipSetDevice(ix->device) != hipSuccess) { failed = true; return; }
+        float *mine = reinterpret_cast<float *>(loan.b->host) + lo * kPiece;
+        for (size_t p; !refused && !failed && (p = next.fetch_add(1)) < pieces;) {
+            const size_t at = p * kPiece, m = std::min(kPiece, values - at);
+            if (copy_checked(mine, rows + at, m)) { refused = true; break; }
+            // (the wait is for whatever the threads have enqueued so far, this piece among it)
+            if (hipMemcpyAsync(d_rows + at, mine, m * sizeof(float), hipMemcpyHostToDevice, ix->stream) != hipSuccess ||
+                hipStreamSynchronize(ix->stream) != hipSuccess) failed = true;
+        }
+    });
+    *bad = refused;
+    if (failed) { g_last_error = "host to device copy failed"; return TV_ERR_HIP; }
+    return TV_OK;
+}
+
+// Device bytes into fresh host memory, the other way round: threads share the copies out of pinned memory, whose
+// page faults are most of the time (77 MB: one thread 18 ms, untouched; 4.4 with the pages touched by eight before).
+static int fetch_bytes(tv_index *ix, const uint8_t *d_from, uint8_t *to, size_t bytes) {
+    constexpr size_t kPiece = size_t(2) << 20;
+    const size_t pieces = (bytes + kPiece - 1) / kPiece, threads = std::min(kMaxParts, pieces);
+    PinnedLoan loan(ix, threads * std::min(kPiece, bytes));
+    if (bytes == 0) return TV_OK;
+    if (!loan.b) {
+        touch_pages(to, bytes);
+        TV_HIP(hipMemcpyAsync(to, d_from, bytes, hipMemcpyDeviceToHost, ix->stream));
+        TV_HIP(hipStreamSynchronize(ix->stream));
+        return TV_OK;
+    }
+    std::atomic<size_t> next{0};
+    std::atomic<bool> failed{false};
+    in_parts(threads, 1, [&](size_t lo, size_t hi) {
+        if (lo == hi) return;
+        if (hipSetDevice(ix->device) != hipSuccess) { failed = true; return; }
+        uint8_t *mine = loan.b->host + lo * kPiece;
+        for (size_t p; !failed && (p = next.fetch_add(1)) < pieces;) {
+            const size_t at = p * kPiece, m = std::min(kPiece, bytes - at);
+            if (hipMemcpyAsync(mine, d_from + at, m, hipMemcpyDeviceToHost, ix->stream) != hipSuccess ||
+                hipStreamSynchronize(ix->stream) != hipSuccess) { failed = true; break; }
+            std::memcpy(to + at, mine, m);
+        }
+    });
+    if (failed) { g_last_error = "device to host copy failed"; return TV_ERR_HIP; }
+    return TV_OK;
+}
+
+// Rows [first, ix->n) are taken back: their bytes and scales are zero again, as if they had never been added.
+static int drop_rows(tv_index *ix, size_t first) {
+    const tv::Geometry &g = ix->geo;
+    const size_t end = ix->n, block = (first + tv::kVecBlock - 1) / tv::kVecBlock, end_block = (end + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (end == first) return TV_OK;
+    const size_t lanes = std::min(end, block * tv::kVecBlock) - first;      // in a block that holds earlier rows
+    ix->n = first;
+    if (lanes) {
+        int rc = ensure_workspace(ix, lanes * size_t(g.G) + 256);
+        if (rc != TV_OK) return rc;
+        TV_HIP(hipMemsetAsync(ix->ws, 0, lanes * size_t(g.G), ix->stream));
+        TV_HIP(tv::launch_append_rows(static_cast<const uint8_t *>(ix->ws), ix->d_codes, g, first, lanes, ix->stream));
+    }
+    TV_HIP(hipMemsetAsync(ix->d_scales + first, 0, (end - first) * sizeof(float), ix->stream));
+    if (end_block > block) TV_HIP(hipMemsetAsync(ix->d_codes + block * g.block_bytes(), 0, (end_block - block) * g.block_bytes(), ix->stream));
+    TV_HIP(hipStreamSynchronize(ix->stream));
+    return TV_OK;
+}
+
 int tv_index_add(tv_index *ix, const float *vectors, size_t n_new) {
     if (!ix || (n_new && !vectors)) return TV_ERR_BAD_ARGUMENT;
     if (n_new == 0) return TV_OK;
     const size_t dim = size_t(ix->geo.dim);
-    size_t bad = 0;
-    int rc = tv_validate_queries(vectors, n_new * dim, ix->geo.dim, &bad);   // same predicate, encode.rs:76-83
-    if (rc != TV_OK) {
-        g_last_error = "vector " + std::to_string(bad / dim) + " holds a non-finite or too large value";
-        return rc;
-    }
     std::lock_guard<std::mutex> lock(ix->mu);
     TV_HIP(hipSetDevice(ix->device));
     if (ix->n + n_new >= (size_t(1) << 31)) return TV_ERR_BAD_ARGUMENT;
-    rc = ensure_capacity(ix, ix->n + n_new);
+    int rc = ensure_capacity(ix, ix->n + n_new);
     if (rc != TV_OK) return rc;
-    const size_t slice = std::max<size_t>(1, (size_t(256) << 20) / (dim * sizeof(float)));
+    const size_t before = ix->n, slice = std::max<size_t>(1, (size_t(256) << 20) / (dim * sizeof(float)));
     rc = ensure_workspace(ix, std::min(n_new, slice) * dim * sizeof(float) + 256);
     if (rc != TV_OK) return rc;
     for (size_t r0 = 0; r0 < n_new; r0 += slice) {
         const size_t nr = std::min(slice, n_new - r0);
-        TV_HIP(hipMemcpyAsync(ix->ws, vectors + r0 * dim, nr * dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
-        rc = add_device_rows(ix, static_cast<const float *>(ix->ws), nr);
+        bool bad = false;
+        rc = stage_rows(ix, vectors + r0 * dim, nr * dim, static_cast<float *>(ix->ws), &bad);
+        if (rc == TV_OK && !bad) rc = add_device_rows(ix, static_cast<const float *>(ix->ws), nr);
         if (rc != TV_OK) return rc;
+        if (bad) {      // the same predicate as for queries (encode.rs:76-83), and nothing is added
+            rc = drop_rows(ix, before);
+            if (rc != TV_OK) return rc;
+            size_t at = r0 * dim;
+            (void)tv_validate_queries(vectors, n_new * dim, int(dim), &at);
+            g_last_error = "vector " + std::to_string(at / dim) + " holds a non-finite or too large value";
+            return TV_ERR_INVALID_QUERY_VALUE;
+        }
     }
     return TV_OK;
 }
@@ -1797,7 +1953,14 @@ int tv_pack_mask(const uint8_t *mask_bytes, size_t n, uint64_t *words_out, size_
     for (size_t w = 0; w * 64 < n; ++w) {
         uint64_t word = 0;
         const size_t lim = std::min<size_t>(64, n - w * 64);
-        for (size_t bit = 0; bit < lim; ++bit) word |= uint64_t(mask_bytes[w * 64 + bit] != 0) << bit;
+        size_t bit = 0;
+        for (; bit + 8 <= lim; bit += 8) {      // eight bytes at a time: 1 where a byte is not zero, the ones gathered by a multiplication
+            uint64_t x;
+            std::memcpy(&x, mask_bytes + w * 64 + bit, 8);
+            x = ((((x & 0x7f7f7f7f7f7f7f7full) + 0x7f7f7f7f7f7f7f7full) | x) >> 7) & 0x0101010101010101ull;
+            word |= (x * 0x0102040810204080ull >> 56) << bit;
+        }
+        for (; bit < lim; ++bit) word |= uint64_t(mask_bytes[w * 64 + bit] != 0) << bit;
         allowed += size_t(__builtin_popcountll(word));
         words_out[w] = word;
     }
@@ -1864,17 +2027,66 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     return rc;
 }
 
-int tv_search(tv_index *ix, const float *queries, size_t nq, size_t k, const uint64_t *mask_words,
-              size_t n_mask_words, float *out_scores, int64_t *out_indices, size_t *out_k_eff) {
+// bad_index: values are checked, on the snapshot of them that is searched (null: they are not).
+static int search_host(tv_index *ix, const float *queries, size_t nq, size_t k, const uint64_t *mask_words,
+                       size_t n_mask_words, float *out_scores, int64_t *out_indices, size_t *out_k_eff, size_t *bad_index) {
     if (!ix || (nq && !queries)) return TV_ERR_BAD_ARGUMENT;
+    const size_t dim = size_t(ix->geo.dim), values = nq * dim;
     tv_request r;
     r.host = true;
     r.q = queries; r.nq = nq; r.k = k;
     r.mask = mask_words; r.mask_arg = mask_words ? n_mask_words : 0;
     r.out_s = out_scores; r.out_i = out_indices;
-    const int rc = search_merged(ix, r);
+    size_t need = 0, s_at = 0, i_at = 0, m_at = 0;
+    if (nq != 0 && k != 0 && nq <= (kPinnedLargest >> 2) && k <= (kPinnedLargest >> 2)) {      // (no product below overflows)
+        s_at = round_up(values * sizeof(float), 256);
+        i_at = s_at + round_up(nq * k * sizeof(float), 256);
+        m_at = i_at + round_up(nq * k * sizeof(int64_t), 256);
+        need = m_at + r.mask_arg * sizeof(uint64_t);
+    }
+    if (need != 0) TV_HIP(hipSetDevice(ix->device));
+    PinnedLoan loan(ix, need != 0 ? need : kPinnedLargest + 1);
+    int rc = TV_OK;
+    if (loan.b) {
+        float *q = reinterpret_cast<float *>(loan.b->host);
+        std::atomic<bool> bad{false};
+        in_parts(values, size_t(1) << 18, [&](size_t lo, size_t hi) {
+            if (copy_checked(q + lo, queries + lo, hi - lo)) bad.store(true, std::memory_order_relaxed);
+        });
+        if (bad_index && bad.load()) rc = tv_validate_queries(q, values, int(dim), bad_index);
+        if (rc != TV_OK) return rc;
+        if (mask_words) {
+            std::memcpy(loan.b->host + m_at, mask_words, r.mask_arg * sizeof(uint64_t));
+            r.staged_mask = reinterpret_cast<uint64_t *>(loan.b->host + m_at);
+        }
+        r.q = q;
+        r.out_s = reinterpret_cast<float *>(loan.b->host + s_at);
+        r.out_i = reinterpret_cast<int64_t *>(loan.b->host + i_at);
+        r.dev_q = reinterpret_cast<const float *>(loan.b->dev);
+        r.dev_s = reinterpret_cast<float *>(loan.b->dev + s_at);
+        r.dev_i = reinterpret_cast<int64_t *>(loan.b->dev + i_at);
+    } else if (bad_index) {
+        rc = tv_validate_queries(queries, values, int(dim), bad_index);
+        if (rc != TV_OK) return rc;
+    }
+    rc = search_merged(ix, r);
     if (out_k_eff) *out_k_eff = r.k_eff;
+    if (rc == TV_OK && loan.b && r.k_eff != 0) {
+        std::memcpy(out_scores, r.out_s, nq * r.k_eff * sizeof(float));
+        std::memcpy(out_indices, r.out_i, nq * r.k_eff * sizeof(int64_t));
+    }
     return rc;
+}
+
+int tv_search(tv_index *ix, const float *queries, size_t nq, size_t k, const uint64_t *mask_words,
+              size_t n_mask_words, float *out_scores, int64_t *out_indices, size_t *out_k_eff) {
+    return search_host(ix, queries, nq, k, mask_words, n_mask_words, out_scores, out_indices, out_k_eff, nullptr);
+}
+
+int tv_search_checked(tv_index *ix, const float *queries, size_t nq, size_t k, const uint64_t *mask_words,
+                      size_t n_mask_words, float *out_scores, int64_t *out_indices, size_t *out_k_eff, size_t *bad_index) {
+    size_t unused = 0;
+    return search_host(ix, queries, nq, k, mask_words, n_mask_words, out_scores, out_indices, out_k_eff, bad_index ? bad_index : &unused);
 }
 
 int tv_debug_scan(tv_index *ix, const float *queries, size_t nq, int32_t *acc_out, float *scores_out) {
@@ -2047,12 +2259,11 @@ int tv_index_to_bytes(const tv_index *cix, const uint64_t *ids, int format, uint
         const tv::SnapshotParts s{kind, g.dim, g.bits, ix->cb.boundaries.data(), ix->cb.centroids.data(), n_calib,
                                   ix->tq_shift.data(), ix->tq_scale.data(), tail_seq.data(), n, tail_scales, ids ? ids + whole * 32 : nullptr};
         uint8_t *units = out + tv::snapshot_head(s, out);
-        touch_pages(units, whole * unit);
         for (size_t b0 = 0; b0 < whole; b0 += slice) {
             const size_t m = std::min(slice, whole - b0);
             TV_HIP(tv::launch_native_to_seq(ix->d_codes, static_cast<uint8_t *>(ix->ws), g, b0, m, unit, ix->d_scales, ix->stream));
-            TV_HIP(hipMemcpyAsync(units + b0 * unit, ix->ws, m * unit, hipMemcpyDeviceToHost, ix->stream));
-            TV_HIP(hipStreamSynchronize(ix->stream));
+            rc = fetch_bytes(ix, static_cast<const uint8_t *>(ix->ws), units + b0 * unit, m * unit);
+            if (rc != TV_OK) return rc;
         }
         if (ids)
             for (size_t b = 0; b < whole; ++b) std::memcpy(units + (b + 1) * unit - 32 * sizeof(uint64_t), ids + b * 32, 32 * sizeof(uint64_t));

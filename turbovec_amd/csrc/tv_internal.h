@@ -203,6 +203,13 @@ size_t select_tmp_keys(size_t k_eff);
 
 struct tv_request;   // a search call waiting for the index (tv_api.hip)
 
+// Pinned host memory an index lends its host-array calls, one block at a time to a call.
+struct tv_pinned {
+    uint8_t *host = nullptr, *dev = nullptr;   // the same bytes, as the host and as the device address them
+    size_t bytes = 0;
+    bool lent = false;
+};
+
 // The opaque handle of the C ABI.
 struct tv_index {
     tv::Geometry geo;
@@ -248,6 +255,9 @@ struct tv_index {
     size_t io_bytes = 0;
     size_t ws_bytes = 0;
     bool ws_fixed = false;         // ws is a lent buffer of fixed size (tv_search_dev_noalloc): never reallocated
+    static constexpr int kPinned = 8;
+    std::mutex pinned_mu;
+    tv_pinned pinned[kPinned];     // allocated on first use, at most kPinnedBytes in all (tv_api.hip), freed with the index
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
     uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags

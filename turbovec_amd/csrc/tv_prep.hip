@@ -31,6 +31,9 @@ struct PrepArgs {
 __host__ __device__ constexpr int prep_at(int j) { return j + (j >> 6) * 8; }
 __host__ __device__ constexpr int prep_floats(int dim) { return prep_at(dim - 1) + 1 + 7 - (prep_at(dim - 1) & 7); }
 
+// Sixteen bytes of the caller's rows, whose alignment is a float's (the load is the same 16-byte one).
+typedef float RowPiece __attribute__((ext_vector_type(4), aligned(4)));
+
 // R butterfly stages from stride 2^S on over the whole row.
 template <int R>
 __device__ __forceinline__ void prep_pass(float *buf, int dim, int S) {
@@ -53,6 +56,12 @@ __device__ __forceinline__ void prep_pass(float *buf, int dim, int S) {
 // one query's preparation took).
 __device__ __forceinline__ void rotate_row(const float *src, const float *signs, const uint32_t *perms, int dim, int log_block,
                                            float inv_sqrt_block, float *A, float *B) {
+    // the row itself first, 16 bytes at a time: it may lie in host memory, where a gather would fetch it piece by piece
+    for (int i = threadIdx.x; i < dim / 4; i += kPrepThreads) {
+        const RowPiece p = reinterpret_cast<const RowPiece *>(src)[i];
+        *reinterpret_cast<float4 *>(B + 4 * i) = float4{p.x, p.y, p.z, p.w};
+    }
+    __syncthreads();
 #pragma unroll
     for (int round = 0; round < 2; ++round) {
         float *buf = round == 0 ? A : B;
@@ -66,7 +75,7 @@ __device__ __forceinline__ void rotate_row(const float *src, const float *signs,
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e)      // the 1/sqrt(B) scale of round 0 rides the round-1 gather: (x * inv) * sign
-                v[e] = round == 0 ? src[p[e]] * s[e] : (A[prep_at(int(p[e]))] * inv_sqrt_block) * s[e];
+                v[e] = round == 0 ? B[p[e]] * s[e] : (A[prep_at(int(p[e]))] * inv_sqrt_block) * s[e];
             butterflies<3>(v);
             float4 *dst = reinterpret_cast<float4 *>(buf + prep_at(8 * g));
             dst[0] = float4{v[0], v[1], v[2], v[3]};

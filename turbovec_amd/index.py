@@ -57,15 +57,19 @@ def _size(name, obj):
     raise TypeError(f"{name} must be an integer, got {type(obj).__name__}")
 
 
+def _bad_value(bad, dim, what):
+    r, c = divmod(bad, dim)
+    return ValueError(f"{what} {r} has a non-finite or out-of-range value at coordinate {c} "
+                      f"(must be finite with magnitude < 1e16)")
+
+
 def _check_values(name, arr, what):
     """turbovec/src/lib.rs:1363-1380, encode.rs:76-83: every value finite and |x| < 1e16."""
     if arr.size == 0:
         return
     rc, bad = T.validate_queries(arr, arr.shape[1])
     if rc == T.ERR_INVALID_QUERY_VALUE:
-        r, c = divmod(bad, arr.shape[1])
-        raise ValueError(f"{what} {r} has a non-finite or out-of-range value at coordinate {c} "
-                         f"(must be finite with magnitude < 1e16)")
+        raise _bad_value(bad, arr.shape[1], what)
 
 
 class TurboQuantIndex:
@@ -193,24 +197,27 @@ class TurboQuantIndex:
             m = np.frombuffer(np.ndarray.tobytes(mask), np.uint8)
         if q.shape[1] != self.dim:
             raise ValueError(f"query dim {q.shape[1]} does not match index dim {self.dim}")
-        q = q.copy()                                    # snapshot, as the binding does (:617-629)
-        _check_values("queries", q, "query")
         with self._lock:
             n = len(self._ix)
             if m is not None and len(m) != n:
+                _check_values("queries", q, "query")
                 raise ValueError(f"mask length {len(m)} does not match index size {n}")
-            return self._search_locked(q, k, m)
+            words, n_allowed = (None, n) if m is None else T.pack_mask(m)
+            return self._search_locked(q, k, words, n_allowed)
 
-    def _search_locked(self, q, k, mask_bytes):
+    def _search_locked(self, q, k, words, n_allowed):
+        """The values of `q` are checked on the library's own copy of them, the snapshot it searches (:617-629)."""
         n = len(self._ix)
-        words, n_allowed = (None, n)
-        if mask_bytes is not None:
-            words, n_allowed = T.pack_mask(mask_bytes)
         k_eff = min(k, n, n_allowed)
         if len(q) == 0 or k_eff == 0:
+            _check_values("queries", q, "query")
             return np.zeros((len(q), k_eff), np.float32), np.zeros((len(q), k_eff), np.int64)
-        k_lib = min(k, n)                               # the library clamps again; keep the argument small
-        return self._ix.search(q, k_lib, mask_words=words)
+        try:
+            return self._ix.search(q, min(k, n), mask_words=words, checked=True)       # (it clamps again; the argument stays small)
+        except T.TurbovecHipError as e:
+            if e.status == T.ERR_INVALID_QUERY_VALUE:
+                raise _bad_value(e.bad_index, self.dim, "query") from None
+            raise
 
 
 def _load_image(data, device, want_kind):
@@ -363,22 +370,24 @@ class IdMapIndex:
                 raise ValueError("allowlist is empty")          # SearchError::AllowlistEmpty
         if q.shape[1] != self.dim:
             raise ValueError(f"query dim {q.shape[1]} does not match index dim {self.dim}")
-        q = q.copy()
-        _check_values("queries", q, "query")
         with self._inner._lock:
-            mask_bytes = None
+            words, n_allowed = None, len(self._slot_to_id)
             if allow is not None:
-                unknown = []
-                for x in allow:
-                    if x not in self._id_to_slot:
-                        unknown.append(x)
-                        if len(unknown) > 5:
-                            break
-                if unknown:
+                try:
+                    slots = np.fromiter(map(self._id_to_slot.__getitem__, allow), np.int64, len(allow))
+                except KeyError:
+                    _check_values("queries", q, "query")
+                    unknown = []
+                    for x in allow:
+                        if x not in self._id_to_slot:
+                            unknown.append(x)
+                            if len(unknown) > 5:
+                                break
                     raise KeyError(f"allowlist contains id(s) not present in index: {unknown[:5]}"
-                                   f"{', ...' if len(unknown) > 5 else ''}")
+                                   f"{', ...' if len(unknown) > 5 else ''}") from None
                 mask_bytes = np.zeros(len(self._slot_to_id), np.uint8)      # duplicates collapse here
-                mask_bytes[[self._id_to_slot[x] for x in allow]] = 1
-            scores, slots = self._inner._search_locked(q, k, mask_bytes)
+                mask_bytes[slots] = 1
+                words, n_allowed = T.pack_mask(mask_bytes)
+            scores, slots = self._inner._search_locked(q, k, words, n_allowed)
             ids = self._id_array()[slots] if slots.size else np.zeros(slots.shape, np.uint64)
             return scores, ids
