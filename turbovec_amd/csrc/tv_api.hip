@@ -539,7 +539,8 @@ struct SamplingSteps {
     static constexpr int kMax = 32;   // levels grow at least fourfold: 2^31 slots need 16 at most
     uint32_t step[kMax];
     size_t count = 0;
-    bool best_first = false;   // the first level runs without floors and hands over the best row of every block it reads
+    bool best_first = false;   // the first level runs without floors and hands over the best row of every block it reads ...
+    bool best_words = false;   // ... as a score word, from a launch of the unsampled search's scan (launch_floor takes the floors)
     size_t size() const { return count; }
     uint32_t operator[](size_t i) const { return step[i]; }
 };
@@ -719,7 +720,24 @@ bool first_level_is_best_of_block(const tv_index *ix, const SampledPlan &plan, s
     if (k_floor > kBestLevelMaxK) return false;
     return plan.wide ? tv::wide_serves_best_of_block(ix->geo.nch) : plan.nt_batched == 0;
 }
-SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool repeat) {
+// The other kernels have no floorless mode -- a second epilogue does not fit their registers -- but the scans of the unsampled
+// search keep every block's best score, and on a sample of the blocks those give a floor as good: one launch of
+// them and k_floor_of_best instead of two row-level samples, their selections and the second one's conditional
+// repeat.  From 16384 blocks (smaller indexes are searched without sampling).  Large or filtered batches of the matrix-unit
+// scan keep the row-level ladder: its floors cost them less than a sample of whole (block, tile) epilogues (889K x 920 2-bit, 640
+// queries: 1842 us with the ladder, 1884 without; 3M x 512 3-bit, 50 queries, 1 % allowed: 249 and 279).
+bool first_level_is_best_words(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool masked) {
+    if (ix->row_ladder_left != 0 || k_floor > size_t(tv::kMaxPickK) || n_blocks <= 16384) return false;
+    if (effective_mode(ix) == TV_SCORE_P) return tv::best_serves(ix->geo.nch) && (plan.wide || plan.nt_batched > 0);
+    return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && (!plan.lut_mx || (plan.cq_pad <= 160 && k_floor <= 64 && !masked));
+}
+// Rows per query the full scan then appends, about: a smaller sample against more appends, which weigh most on short rows
+// and on the matrix-unit scan (3M x 128, 1000 queries: 256 rows 657 us a search, 512 741, 1024 888, without this level 1223;
+// 1M x 1536, 64 queries: 212, 223, 204, 237; 3M x 384 2-bit, 141 queries: 878, 878, 958, 946).
+size_t floor_rows(const tv_index *ix, const SampledPlan &plan) {
+    return plan.lut_mx ? 512 : effective_mode(ix) == TV_SCORE_P && ix->geo.nch < 12 ? 256 : 1024;
+}
+SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool repeat, bool masked) {
     if (!repeat && first_level_is_best_of_block(ix, plan, k_floor)) {
         SamplingSteps steps;
         // (the all-queries kernel pays for every candidate of the full scan -- a tile with one in it
@@ -745,6 +763,14 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
         }
         // (an index too small for that level -- it would read a quarter of it or more -- takes the
         // row-level ladder below: a full scan from open floors alone would append every row)
+    }
+    if (!repeat && first_level_is_best_words(ix, plan, n_blocks, k_floor, masked)) {
+        SamplingSteps steps;
+        const size_t sample = std::min<size_t>({std::max<size_t>(n_blocks * k_floor / floor_rows(ix, plan), 8 * k_floor), size_t(tv::kMaxFloorBlocks), n_blocks / 4});
+        steps.step[steps.count++] = uint32_t((n_blocks + sample - 1) / sample);
+        steps.step[steps.count++] = 1;
+        steps.best_first = steps.best_words = true;
+        return steps;
     }
     // (the sixteen-query LUT scan works in rounds too: every wave of the grid carries two blocks through the row)
     return plan.wide    ? sampling_steps(n_blocks, k_floor, size_t(plan.grid) * tv::wide_blocks_per_workgroup(ix->geo.nch))
@@ -822,34 +848,35 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks)
     if (nch < 12) return triples <= 6000000;
     return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 16 ? 1050000 : 250000) || n_blocks <= 512;
 }
+// The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
+// whole tables in LDS for a few, tables streamed for up to sixteen (tiles side by side beyond) or the
+// sparse matrix instruction.
+int best_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
+    const int nch = a.nch;
+    const size_t blocks = (a.n_blocks + a.b_step - 1) / a.b_step;
+    a.k = 1;
+    a.gtau = ix->d_tau_open;
+    if (pq.d_tables_mx != nullptr) {
+        a.tables = pq.d_tables_mx;
+        if (a.mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * a.best_stride, ix->stream));   // (it skips blocks without an allowed row)
+        TV_HIP(tv::launch_scan_lut_mx(a, tv::mx_shape(ix->device, cq, blocks, false), ix->geo.bits, ix->stream));
+    } else if (pq.d_tables16 != nullptr) {
+        a.tables = pq.d_tables16;
+        const int tiles = int((cq + tv::kLut16Queries - 1) / tv::kLut16Queries);
+        const int grid = int(std::min<size_t>(size_t(tv::device_cus(ix->device)), (blocks + 7) / 8));
+        TV_HIP(tv::launch_scan_lut16(a, grid, tiles, ix->stream));
+    } else {
+        const int grid = int(std::min<size_t>(size_t(tv::lut_append_grid(ix->device, nch)), (blocks + 1) / 2));
+        TV_HIP(tv::launch_scan_lut(a, grid, tv::kModeAppend, ix->stream));
+    }
+    return TV_OK;
+}
 // The milliseconds between the two stamps.
 int take_stamps(tv_index *ix, int launches) {
     int khz = 0;
     TV_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ix->device));
     if (khz > 0) ix->last_scan_ms += float(double(ix->h_stamps[1] - ix->h_stamps[0]) / khz);
     ix->last_scan_launches += launches;
-    return TV_OK;
-}
-// The unsampled scan of u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
-// whole tables in LDS for a few, tables streamed for up to sixteen (tiles side by side beyond) or the
-// sparse matrix instruction.
-int direct_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
-    const int nch = a.nch;
-    a.k = 1;
-    a.gtau = ix->d_tau_open;
-    if (pq.d_tables_mx != nullptr) {
-        a.tables = pq.d_tables_mx;
-        if (a.mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * a.best_stride, ix->stream));   // (it skips blocks without an allowed row)
-        TV_HIP(tv::launch_scan_lut_mx(a, tv::mx_shape(ix->device, cq, a.n_blocks, false), ix->geo.bits, ix->stream));
-    } else if (pq.d_tables16 != nullptr) {
-        a.tables = pq.d_tables16;
-        const int tiles = int((cq + tv::kLut16Queries - 1) / tv::kLut16Queries);
-        const int grid = int(std::min<size_t>(size_t(tv::device_cus(ix->device)), (size_t(a.n_blocks) + 7) / 8));
-        TV_HIP(tv::launch_scan_lut16(a, grid, tiles, ix->stream));
-    } else {
-        const int grid = int(std::min<size_t>(size_t(tv::lut_append_grid(ix->device, nch)), (size_t(a.n_blocks) + 1) / 2));
-        TV_HIP(tv::launch_scan_lut(a, grid, tv::kModeAppend, ix->stream));
-    }
     return TV_OK;
 }
 int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
@@ -888,9 +915,9 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                 if (d_mask) TV_HIP(tv::launch_fill_i32(reinterpret_cast<int *>(a.best_out), 0, cq * stride, ix->stream));   // (it skips blocks without an allowed row)
                 TV_HIP(tv::launch_scan_p4_wide(a, tv::wide_grid_blocks(ix->device), ix->stream));
             } else if (mode_p) {
-                TV_HIP(tv::launch_scan_p4_best(a, ix->device, ix->stream));
+                TV_HIP(tv::launch_scan_p4_best(a, split, ix->device, ix->stream));
             } else {
-                rc = direct_scan_lut(ix, a, pq, cq);
+                rc = best_scan_lut(ix, a, pq, cq);
                 if (rc != TV_OK) return rc;
             }
             TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
@@ -987,7 +1014,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
             const size_t tile_q = plan.tile_q, n_tiles = plan.n_tiles, cq_pad = plan.cq_pad, seg_stride = plan.seg_stride;
             const bool wide = plan.wide;
             const int grid = plan.grid;
-            const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat);
+            const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat, d_mask != nullptr);
             const bool best_first = steps.best_first;
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
@@ -1005,8 +1032,8 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
             }
             Prepared pq;
             const int nt_batched = plan.nt_batched;
-            int prc = prepare_queries(ix, ar, repeat ? d_redo_q : d_q, pq_n, pq,
-                                      wide ? tv::wide_weights_split(g.nch) : (nt_batched == 0 || tv::batched_weights_split(g.nch)), false, true);
+            const bool split = wide ? tv::wide_weights_split(g.nch) : (nt_batched == 0 || tv::batched_weights_split(g.nch));
+            int prc = prepare_queries(ix, ar, repeat ? d_redo_q : d_q, pq_n, pq, split, false, true);
             if (prc != TV_OK) return prc;
             uint64_t *d_cand = ar.take<uint64_t>(cq_pad * seg_stride * tv::kSegCap);
             uint32_t *d_cnt = ar.take<uint32_t>(cq_pad * seg_stride);
@@ -1033,6 +1060,25 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                 // is set.  The full scan then starts from the floor the level was meant to give.
                 uint32_t *lv_flag = (!last && (lv > 0 || repeat)) ? d_level_flags + lv : nullptr;
                 uint32_t *next_flag = (lv + 2 < steps.size()) ? d_level_flags + lv + 1 : nullptr;
+                if (lv == 0 && steps.best_words) {
+                    tv::ScanArgs a;
+                    fill_scan_args(ix, a);
+                    a.mask = d_mask;
+                    a.tables = pq.d_tables;
+                    a.qscale = pq.d_qscale;
+                    a.qbias = pq.d_qbias;
+                    a.nq_tile = int(pq_n);
+                    a.b_step = steps[0];
+                    // (in the candidates' place, which nothing has been written to yet: 512 bytes a segment against four a block)
+                    a.best_out = reinterpret_cast<uint32_t *>(d_cand);
+                    a.best_stride = uint32_t(round_up(level_blocks, 64));
+                    if (a.best_stride > seg_stride * tv::kSegCap * 2) { g_last_error = "internal: a sample larger than the candidates' place"; return TV_ERR_BAD_ARGUMENT; }
+                    if (mode_p) TV_HIP(tv::launch_scan_p4_best(a, split, ix->device, ix->stream));
+                    else if (const int lrc = best_scan_lut(ix, a, pq, pq_n)) return lrc;
+                    TV_HIP(tv::launch_floor(a.best_out, a.best_stride, uint32_t(level_blocks), int(k_floor), int(pq_n), d_tau, int(tile_q),
+                                            timed_pass ? ix->d_stamps : nullptr, ix->stream));
+                    continue;
+                }
                 for (int attempt = 0; attempt < (lv_flag ? 2 : 1); ++attempt) {
                     const uint32_t *run_if = attempt == 0 ? nullptr : lv_flag;
                     int n_seg = lgrid;
@@ -1121,7 +1167,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
                 const SampledPlan plan = sampled_plan(ix, chunk_at[c + 1] - chunk_at[c]);
-                const size_t n_levels = level_strides(ix, plan, n_blocks, k_floor, false).size();
+                const size_t n_levels = level_strides(ix, plan, n_blocks, k_floor, false, d_mask != nullptr).size();
                 for (size_t lv = 1; lv + 1 < n_levels; ++lv)
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
             }
@@ -1147,7 +1193,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         }
         ix->overflow_redos += redo_rows.size() + exact_rows.size();
         if ((redo_rows.size() + exact_rows.size()) * 8 >= gq) {
-            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, k_floor, false).best_first) {
+            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, k_floor, false, d_mask != nullptr).best_first) {
                 // from here on, the repeated passes below included -- unless the row-level ladder has just failed too
                 if (ix->floorless_kept_left == 0) ix->row_ladder_left = kRowLadderSearches;
             } else if (ix->row_ladder_left > 0) {
@@ -2371,7 +2417,7 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (direct_serves(ix, nq, k_eff, n_blocks)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
-    const SamplingSteps steps = level_strides(ix, plan, n_blocks, std::max<size_t>(k_eff, 16), false);
+    const SamplingSteps steps = level_strides(ix, plan, n_blocks, std::max<size_t>(k_eff, 16), false, false);
     *count = steps.size();
     for (size_t i = 0; i < steps.size() && i < cap; ++i) {
         if (strides) strides[i] = steps[i];

@@ -70,7 +70,7 @@ struct ScanArgs {
     uint32_t seg_stride;       // segments allocated per query (>= grid of the launch)
     uint32_t vgrid;            // single-tile permute-dot scan: four-wave groups of the launch (set by its launcher)
     int best_of_block;         // all-queries-per-pass kernel: no floor, per scanned block and query the best allowed slot (kModeBest)
-    uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and block the best allowed row's (tv_kernels6.hip)
+    uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and scanned block the best allowed row's (tv_kernels6.hip)
     uint32_t best_stride;
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
@@ -150,7 +150,11 @@ constexpr int kMaxPickK = 128;             // most results k_pick ranks
 constexpr size_t kMaxPickBlocks = 32768;   // most blocks it chooses from
 constexpr size_t kPickLds = 128 * 1024;    // rows' keys and the query's tables, beside its 13 KiB of fixed buffers
 bool best_serves(int nch);
-hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s);
+hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStream_t s);
+// The k_floor-th best of n score words per query as its floor, to tau_out like launch_final.
+constexpr uint32_t kMaxFloorBlocks = 8192;
+hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,
+                        hipStream_t s);
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut);
 hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
                        hipStream_t s);

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(THREADS) void k_scan_lut(ScanArgs a) {
             const uint32_t b = j * step;
             const uint64_t w = a.mask[b >> 1];
             if (uint32_t(w >> ((b & 1) * 32)) != 0u) break;
-            if (APPEND && a.best_out != nullptr && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = 0u;
+            if (APPEND && a.best_out != nullptr && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + j] = 0u;
             j += total_waves;
         }
         return j;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(THREADS) void k_scan_lut(ScanArgs a) {
                 }
 #pragma unroll
                 for (int d = QL; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-                if (lane < QL && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = best_word(m);
+                if (lane < QL && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + j] = best_word(m);
             } else if (APPEND) {
 #pragma unroll
                 for (int e = 0; e < per; ++e) {
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(kLutBtThreads) void k_scan_lut_bt(ScanArgs a, int n
         while (j < nj) {
             const uint32_t b = j * step;
             if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
-            if (a.best_out != nullptr && lane == 0) a.best_out[b] = 0u;
+            if (a.best_out != nullptr && lane == 0) a.best_out[j] = 0u;
             j += total_waves;
         }
         return j;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kLutBtThreads) void k_scan_lut_bt(ScanArgs a, int n
         if (a.best_out != nullptr) {
             // a search without sampling (tv_kernels6.hip): the block's best score, no slot
             const uint32_t m = wave_umax(allowed && sc == sc ? best_word(sc) : 0u);
-            if (lane == 0) a.best_out[b] = m;
+            if (lane == 0) a.best_out[j] = m;
         } else if (a.best_of_block) {
             // A first sampling level without a floor: the block's best allowed row (score order, then
             // the lower slot: the larger sort key), one candidate per block -- a real score of a real

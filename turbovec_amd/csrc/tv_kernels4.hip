@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
         while (j < nj) {
             const uint32_t b = j * step;
             if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
-            if (BEST && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + b] = 0u;
+            if (BEST && lane < a.nq_tile) a.best_out[size_t(lane) * a.best_stride + j] = 0u;
             j += total_waves;
         }
         return j;
@@ -170,6 +170,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
     int buf = 0;
     for (;;) {
         uint32_t blk[RB];
+        const uint32_t j0 = j;             // (BEST, one block: which of the scanned ones it is)
         bool has[RB];
         // Once every query's segment of this workgroup is full, every query of the launch is certain
         // to be flagged as overflowed and scanned again from a raised floor: nothing this workgroup
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(kLut16Threads) void k_scan_lut16(ScanArgs a) {
             if (BEST) {
                 best = fmaxf(best, __shfl_xor(best, 16));
                 best = fmaxf(best, __shfl_xor(best, 32));
-                if (kb == 0 && qact) a.best_out[size_t(r) * a.best_stride + b] = best_word(best);
+                if (kb == 0 && qact) a.best_out[size_t(r) * a.best_stride + j0] = best_word(best);
             }
         }
     }

@@ -159,8 +159,9 @@ struct MxQuery {
 };
 
 // sub (a power of two up to 8): candidate segments a workgroup keeps per query, its waves sharing
-// them out.
-template <int ENT, int NT, int BLK>
+// them out.  BEST: no candidates, every (block, query)'s best score (tv_kernels6.hip); an instance of its own, as the
+// branch costs the append form 1.4 %.
+template <int ENT, int NT, int BLK, bool BEST>
 __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint32_t groups, uint32_t sub) {
     extern __shared__ __align__(16) uint8_t smem[];
     if (launch_switched_off(a.run_if)) return;
@@ -434,7 +435,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
             m1 = max(max(m1, v[14]), v[15]);
             if (__any(max(max(m0, m1), max(m2, m3)) >= bound)) hits |= 1u << decltype(ii)::value;
         });
-        if (a.best_out != nullptr) hits = (1u << (BLK * NT)) - 1u;         // (a search without sampling: every pair's best score)
+        if constexpr (BEST) hits = (1u << (BLK * NT)) - 1u;
         // (One body for all pairs, on a copy of the sums: unrolled, it would outgrow the instruction cache.)
 #pragma unroll 1
         while (hits != 0u) {
@@ -451,12 +452,12 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
             const int bound = bound_of(i, inv, k);
             const float qs = sq[i].qs, qb = sq[i].qb, tau = sq[i].tau;
             const float *vs = s_vs + (wave * BLK + k) * 32 + 4 * h;
-            if (a.best_out != nullptr) {
+            if constexpr (BEST) {
                 float m = -__int_as_float(0x7f800000);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) m = fmaxf(m, ((float(v[r]) * qs) + qb) * vs[8 * (r >> 2) + (r & 3)]);     // (NaN never wins)
                 m = fmaxf(m, __shfl_xor(m, 32));
-                if (h == 0 && q0 + i < a.nq_tile && jb < nj) a.best_out[size_t(q0 + i) * a.best_stride + block_of(jb)] = best_word(m);
+                if (h == 0 && q0 + i < a.nq_tile && jb < nj) a.best_out[size_t(q0 + i) * a.best_stride + jb] = best_word(m);
                 continue;
             }
 #pragma unroll
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_scan_lut_mx(ScanArgs a, uint3
         for (int k = 0; k < BLK; ++k) blk[k] = nblk[k];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // requests still in flight write this workgroup's LDS
-    if (a.best_out != nullptr) return;
+    if constexpr (BEST) return;
     __syncthreads();
     for (int i = tid; i < kQ * int(sub); i += kMxThreads) {
         const int q = q0 + i % kQ, sb = i / kQ;
@@ -514,14 +515,18 @@ int mx_round_blocks(int device, size_t nq) {
     return int(m.wgs) * kMxWaves * m.blk;
 }
 
-template <int ENT, int NT, int BLK>
-static hipError_t launch_mx(const ScanArgs &a, const MxShape &m, hipStream_t s) {
+template <int ENT, int NT, int BLK, bool BEST>
+static hipError_t launch_mx_best(const ScanArgs &a, const MxShape &m, hipStream_t s) {
     constexpr int kS = mx_steps(ENT) < 16 / NT ? mx_steps(ENT) : 16 / NT;
     const size_t lds = size_t(kMxRing) * NT * kS * 2048 + NT * kQTile * (sizeof(MxQuery) + 8 * 4) + kMxWaves * BLK * 32 * 4 + 64;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_lut_mx<ENT, NT, BLK>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_lut_mx<ENT, NT, BLK, BEST>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_scan_lut_mx<ENT, NT, BLK>), dim3(m.wgs * m.groups), dim3(kMxThreads), lds, s, a, m.groups, m.sub);
+    hipLaunchKernelGGL((k_scan_lut_mx<ENT, NT, BLK, BEST>), dim3(m.wgs * m.groups), dim3(kMxThreads), lds, s, a, m.groups, m.sub);
     return hipGetLastError();
+}
+template <int ENT, int NT, int BLK>
+static hipError_t launch_mx(const ScanArgs &a, const MxShape &m, hipStream_t s) {
+    return a.best_out != nullptr ? launch_mx_best<ENT, NT, BLK, true>(a, m, s) : launch_mx_best<ENT, NT, BLK, false>(a, m, s);
 }
 template <int ENT, int NT>
 static hipError_t launch_mx_blk(const ScanArgs &a, const MxShape &m, hipStream_t s) {

@@ -23,18 +23,19 @@ namespace tv {
 // 3125 of them, which fill 65 of the 256 workgroups of a kernel that takes all queries through one.
 // 100K x 128, 1000 queries: 35 us, the vector ALU busy in 60 % of the clocks and the matrix unit in 15 %.  Rows that
 // short have two chunks, so of the 530 vector instructions per block and four tiles the decode is 120, the rest epilogue.
-// Weights in plane order (launch_prep_p, split = false).
+// Weights in plane order, or (SPLIT) in the order of k_scan_p4, whose operands then take four byte permutes a chunk.
+// a.b_step: every so many blocks only (the sample a floor is taken from), recorded by their place in the sample.
 // ===========================================================================
 constexpr int kBestThreads = 512;
 constexpr int kBestWaves = kBestThreads / 64;
 
-template <int NT, int U>
+template <int NT, int U, bool SPLIT>
 __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(ScanArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int nch = a.nch, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qn = lane & 31, h = lane >> 5;
     const int tile0 = int(blockIdx.y) * NT;
     const int nt = min(NT, (a.nq_tile + kQTile - 1) / kQTile - tile0);
-    const uint32_t stride = gridDim.x * kBestWaves;
+    const uint32_t stride = gridDim.x * kBestWaves, step = a.b_step, nj = (a.n_blocks + step - 1) / step;
     const uint4 *codes = reinterpret_cast<const uint4 *>(a.codes) + lane;
     const float nan = __int_as_float(0x7fc00000);
     auto store = [&](int t, uint32_t j, uint32_t word) {
@@ -44,8 +45,9 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
     // the next block from j on with an allowed row; the ones without are recorded on the way
     auto live_from = [&](uint32_t j) -> uint32_t {
         if (a.mask == nullptr) return j;
-        for (; j < a.n_blocks; j += stride) {
-            if (uint32_t(a.mask[j >> 1] >> ((j & 1) * 32)) != 0u) break;
+        for (; j < nj; j += stride) {
+            const uint32_t b = j * step;
+            if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
 #pragma unroll
             for (int t = 0; t < NT; ++t) store(t, j, 0u);
         }
@@ -54,9 +56,9 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
     // the wave's first codes are on their way while the workgroup sets up its LDS
     uint32_t j = live_from(blockIdx.x * kBestWaves + wave);
     uint4 buf[U];
-    if (j < a.n_blocks) {
+    if (j < nj) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) buf[u] = codes[(size_t(j) * nch + u) * 64];
+        for (int u = 0; u < U; ++u) buf[u] = codes[(size_t(j) * step * nch + u) * 64];
     }
     {
         const uint4 *src = reinterpret_cast<const uint4 *>(a.tables) + size_t(tile0) * nch * 128;
@@ -83,11 +85,11 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
     const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
     const v4i *w = reinterpret_cast<const v4i *>(smem) + lane;
 
-    while (j < a.n_blocks) {
-        const uint32_t jn = live_from(j + stride);
+    while (j < nj) {
+        const uint32_t jn = live_from(j + stride), b = j * step;
         // row scales, NaN where a row may not be returned
-        const uint32_t slot0 = j * 32u;
-        uint32_t mw = a.mask != nullptr ? uint32_t(a.mask[j >> 1] >> ((j & 1) * 32)) : 0xffffffffu;
+        const uint32_t slot0 = b * 32u;
+        uint32_t mw = a.mask != nullptr ? uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) : 0xffffffffu;
         if (slot0 + 32u > a.n) mw &= (1u << (a.n - slot0)) - 1u;
         float vs[16];
 #pragma unroll
@@ -103,8 +105,8 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
 #pragma unroll
             for (int u = 0; u < U; ++u) cur[u] = buf[u];
             const bool more = c0 + U < nch;
-            if (more || jn < a.n_blocks) {
-                const uint4 *from = codes + (more ? size_t(j) * nch + c0 + U : size_t(jn) * nch) * 64;
+            if (more || jn < nj) {
+                const uint4 *from = codes + (more ? size_t(b) * nch + c0 + U : size_t(jn) * step * nch) * 64;
 #pragma unroll
                 for (int u = 0; u < U; ++u) buf[u] = from[u * 64];
             }
@@ -116,6 +118,12 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
                 for (int d = 0; d < 4; ++d) {
                     lo[d] = int(levels_of(x[d] & 0x0f0f0f0fu, t0, t1, t2, t3));
                     hi[d] = int(levels_of((x[d] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3));
+                }
+                if constexpr (SPLIT) {
+                    const v4i l = lo, g = hi;
+                    lo = v4i{l[0], g[0], l[1], g[1]};
+                    hi = v4i{int(__builtin_amdgcn_perm(uint32_t(g[2]), uint32_t(l[2]), 0x05010400u)), int(__builtin_amdgcn_perm(uint32_t(g[2]), uint32_t(l[2]), 0x07030602u)),
+                             int(__builtin_amdgcn_perm(uint32_t(g[3]), uint32_t(l[3]), 0x05010400u)), int(__builtin_amdgcn_perm(uint32_t(g[3]), uint32_t(l[3]), 0x07030602u))};
                 }
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
@@ -152,35 +160,94 @@ static int best_tiles(int nch, size_t n_blocks, int tiles, int cus) {
 }
 bool best_serves(int nch) { return size_t(nch) * 2048 <= 160 * 1024; }
 
-template <int NT, int U>
-static hipError_t launch_best_n(const ScanArgs &a, int device, hipStream_t s) {
+template <int NT, int U, bool SPLIT>
+static hipError_t launch_best_n(const ScanArgs &a, uint32_t nj, int device, hipStream_t s) {
     const int tiles = (a.nq_tile + kQTile - 1) / kQTile, groups_y = (tiles + NT - 1) / NT;
     const size_t lds = size_t(NT) * a.nch * 2048;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     // a workgroup keeps its weights for all its blocks: about as many workgroups as are resident
     const unsigned per_cu = unsigned(std::min<size_t>(NT <= 2 ? 2 : 1, 160 * 1024 / lds));
     const unsigned resident = unsigned(device_cus(device)) * std::max(1u, per_cu);
-    const unsigned x = std::max(1u, std::min((a.n_blocks + kBestWaves - 1) / kBestWaves, (resident + groups_y - 1) / groups_y));
-    hipLaunchKernelGGL((k_scan_p4_best<NT, U>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
+    const unsigned x = std::max(1u, std::min((nj + kBestWaves - 1) / kBestWaves, (resident + groups_y - 1) / groups_y));
+    hipLaunchKernelGGL((k_scan_p4_best<NT, U, SPLIT>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
     return hipGetLastError();
 }
-template <int NT>
-static hipError_t launch_best_u(const ScanArgs &a, int device, hipStream_t s) {
+template <int NT, bool SPLIT>
+static hipError_t launch_best_u(const ScanArgs &a, uint32_t nj, int device, hipStream_t s) {
     // (two tiles' accumulators and bursts of four chunks do not fit the 128 registers of four waves per SIMD)
     if constexpr (NT != 2) {
-        if (a.nch % 4 == 0) return launch_best_n<NT, 4>(a, device, s);
+        if (a.nch % 4 == 0) return launch_best_n<NT, 4, SPLIT>(a, nj, device, s);
     }
-    return a.nch % 2 == 0 ? launch_best_n<NT, 2>(a, device, s) : launch_best_n<NT, 1>(a, device, s);
+    return a.nch % 2 == 0 ? launch_best_n<NT, 2, SPLIT>(a, nj, device, s) : launch_best_n<NT, 1, SPLIT>(a, nj, device, s);
 }
 // a.nq_tile = all queries of the launch, a.tables = their weight tiles, a.best_out / a.best_stride = the result.
-hipError_t launch_scan_p4_best(const ScanArgs &a, int device, hipStream_t s) {
-    if (a.nq_tile <= 0 || a.n_blocks == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride < a.n_blocks) return hipErrorInvalidValue;
-    switch (best_tiles(a.nch, a.n_blocks, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device))) {
-        case 1: return launch_best_u<1>(a, device, s);
-        case 2: return launch_best_u<2>(a, device, s);
-        default: return launch_best_u<4>(a, device, s);
+hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStream_t s) {
+    const uint32_t nj = a.b_step ? (a.n_blocks + a.b_step - 1) / a.b_step : 0u;
+    if (a.nq_tile <= 0 || nj == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride < nj) return hipErrorInvalidValue;
+    const int nt = best_tiles(a.nch, nj, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device));
+    if (split) return nt == 1 ? launch_best_u<1, true>(a, nj, device, s) : nt == 2 ? launch_best_u<2, true>(a, nj, device, s) : launch_best_u<4, true>(a, nj, device, s);
+    return nt == 1 ? launch_best_u<1, false>(a, nj, device, s) : nt == 2 ? launch_best_u<2, false>(a, nj, device, s) : launch_best_u<4, false>(a, nj, device, s);
+}
+
+// ===========================================================================
+// The floor a sample's best rows give: a workgroup per query takes the k_floor-th best of the sampled blocks' best
+// scores, which k_floor scanned rows reach.
+// ===========================================================================
+constexpr uint32_t kFloorThreads = 512, kFloorHeld = kMaxFloorBlocks / kFloorThreads;
+__global__ __launch_bounds__(kFloorThreads) void k_floor_of_best(const uint32_t *__restrict__ words, uint32_t stride, uint32_t n, uint32_t k_floor,
+                                                        int *tau_out, int tau_stride_q, uint64_t *stamp) {
+    constexpr uint32_t T = kFloorThreads, W = T / 64;
+    __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
+    __shared__ SelectShared sh;
+    __shared__ uint32_t n_kept;
+    const uint32_t qi = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    const uint32_t *best = words + size_t(qi) * stride;
+    uint32_t v[kFloorHeld];
+#pragma unroll
+    for (uint32_t e = 0; e < kFloorHeld; ++e) v[e] = e * T + t < n ? best[e * T + t] : 0u;
+    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
+    if (t == 0) n_kept = 0u;
+    auto each = [&](auto &&f) {
+#pragma unroll
+        for (uint32_t e = 0; e < kFloorHeld; ++e)
+            if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
+    };
+    uint32_t mine = 0u, hi_max = 0u, hi_min_inv = 0u, mx, mn_inv, total = 0u;
+    each([&](uint64_t k) {
+        ++mine;
+        hi_max = max(hi_max, uint32_t(k >> 32));
+        hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+    });
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) mine += __shfl_xor(mine, d);
+    if (lane == 0) sh.w_sum[wv] = mine;
+    select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
+    for (uint32_t w = 0; w < W; ++w) total += sh.w_sum[w];
+    __syncthreads();
+    int *out = tau_out + (qi / uint32_t(tau_stride_q)) * kQTile + qi % uint32_t(tau_stride_q);
+    if (total < k_floor) {      // (a mask that leaves the sample too few rows)
+        if (t == 0) *out = kTauInit;
+    } else {
+        const uint64_t threshold = total > kSelectKept ? select_threshold<T>(each, mx, mn_inv, k_floor, sh) : 0ull;
+        each([&](uint64_t k) {
+            if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
+        });
+        __syncthreads();
+        const uint32_t m = n_kept;
+        if (t < 2u) kept[m + t] = 0ull;
+        __syncthreads();
+        for (uint32_t i = t; i < m; i += T)
+            if (rank_in(kept, m, kept[i]) + 1u == k_floor) *out = int(uint32_t(kept[i] >> 32) ^ 0x80000000u);
     }
+    if (t == 0 && stamp != nullptr && qi + 1u == gridDim.x) *stamp = wall_clock64();      // (among the last to end)
+}
+hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,
+                        hipStream_t s) {
+    if (nq <= 0) return hipSuccess;
+    if (n > kMaxFloorBlocks || n > stride || k_floor <= 0 || k_floor > int(kSelectKept)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_floor_of_best, dim3(unsigned(nq)), dim3(kFloorThreads), 0, s, words, stride, n, uint32_t(k_floor), tau_out, tau_stride_q, stamp);
+    return hipGetLastError();
 }
 
 // ===========================================================================
