@@ -253,7 +253,9 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * instead of the batched ones; bit 2 keeps them off the all-queries-per-pass
  * kernel only; bit 3 keeps u8-LUT batches on the scan that holds whole tables in
  * LDS (at most 8 queries per pass) instead of the larger ones; bit 4 samples
- * small indexes like large ones (bits 1 and 2 do too). */
+ * small indexes like large ones (bits 1 and 2 do too); bit 6 has filtered searches
+ * gather the allowed rows first whatever their number; without it any other bit, bit 5
+ * of no other meaning too, has them read the mask as they scan. */
 int tv_debug_set_path(tv_index *ix, int force_full_lists);
 /* The sampling ladder a search for the k best of nq queries (its first chunk of up to 1024) runs
  * on this index as it stands, unfiltered: block strides of the successive scans, strides[0 ..
@@ -273,6 +275,8 @@ int tv_debug_level_repeats(tv_index *ix, int track, size_t *count);
 /* Bytes of the index's cached search workspace and of its host-call staging allocation (either
  * pointer may be NULL): both only ever grow, and tv_search_dev_noalloc touches neither. */
 int tv_debug_workspace_bytes(const tv_index *ix, size_t *workspace, size_t *staging);
+/* How many filtered searches so far ran on a copy of their allowed rows. */
+int tv_debug_gathered_searches(const tv_index *ix, size_t *count);
 /* How many queries so far did not finish in the single sampled pass because their
  * candidate buffer overflowed (they are scanned once more, all together, from a raised
  * floor), and how many of those went on to the exact list / select path. */

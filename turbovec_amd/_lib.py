@@ -34,6 +34,7 @@ EXPORTS = [
     "tv_host_snapshot_len", "tv_host_snapshot_compose", "tv_host_snapshot_info", "tv_host_snapshot_extract",
     "tv_index_to_bytes", "tv_index_from_bytes", "tv_search_dev_noalloc", "tv_noalloc_scratch_bytes",
     "tv_debug_exact_redos", "tv_debug_sampling_plan", "tv_debug_merged_calls", "tv_debug_level_repeats", "tv_debug_workspace_bytes",
+    "tv_debug_gathered_searches",
 ]
 
 _lib = None
@@ -102,6 +103,7 @@ def lib():
     L.tv_debug_set_path.argtypes = [vp, i32]
     L.tv_debug_overflow_redos.argtypes = [vp, C.POINTER(sz)]
     L.tv_debug_exact_redos.argtypes = [vp, C.POINTER(sz)]
+    L.tv_debug_gathered_searches.argtypes = [vp, C.POINTER(sz)]
     L.tv_debug_workspace_bytes.argtypes = [vp, C.POINTER(sz), C.POINTER(sz)]
     L.tv_debug_level_repeats.argtypes = [vp, i32, C.POINTER(sz)]
     L.tv_debug_merged_calls.argtypes = [vp, C.POINTER(sz)]
@@ -321,6 +323,11 @@ class NativeIndex:
 
     def set_path(self, force_full_lists):
         check(lib().tv_debug_set_path(self.h, int(force_full_lists)))
+
+    def gathered_searches(self):
+        c = C.c_size_t(0)
+        check(lib().tv_debug_gathered_searches(self.h, C.byref(c)))
+        return c.value
 
     def overflow_redos(self):
         c = C.c_size_t(0)

@@ -198,13 +198,15 @@ int ensure_workspace(tv_index *ix, size_t bytes) {
     return TV_OK;
 }
 
-int ensure_io(tv_index *ix, size_t bytes) {
-    if (bytes <= ix->io_bytes) return TV_OK;
-    if (ix->io) { TV_HIP(device_free(ix->device, ix->io, ix->io_bytes)); ix->io = nullptr; ix->io_bytes = 0; }
+// An allocation of the index that grows on demand: what it held is gone then.
+int ensure_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
+    if (bytes <= have) return TV_OK;
+    if (p) { TV_HIP(device_free(ix->device, p, have)); p = nullptr; have = 0; }
     bytes = round_up(bytes + bytes / 4, size_t(1) << 16);
-    TV_HIP(device_alloc(ix->device, bytes, &ix->io, &ix->io_bytes));
+    TV_HIP(device_alloc(ix->device, bytes, &p, &have));
     return TV_OK;
 }
+int ensure_io(tv_index *ix, size_t bytes) { return ensure_block(ix, ix->io, ix->io_bytes, bytes); }
 
 // ---- host arrays ---------------------------------------------------------------------------------
 // A copy from or to pageable memory is staged by the runtime, on one thread and with a wait of its own: 500 KB 30 us, 614 MB
@@ -360,7 +362,7 @@ int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCOR
 // pairs: 165 against 131).
 constexpr size_t kMxMinPairs = 4096;
 bool lut_mx_serves(const tv_index *ix, size_t cq) {
-    const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
+    const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
     return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && !ix->no_lut_mx && cq > size_t(tv::kLut16Queries) &&
            n_blocks * tiles >= kMxMinPairs;
 }
@@ -443,10 +445,11 @@ size_t prepare_bytes(const tv_index *ix, size_t nq) {
 
 void fill_scan_args(const tv_index *ix, tv::ScanArgs &a) {
     std::memset(&a, 0, sizeof a);
-    a.codes = ix->d_codes;
-    a.scales = ix->d_scales;
-    a.n = uint32_t(ix->n);
-    a.n_blocks = uint32_t((ix->n + tv::kVecBlock - 1) / tv::kVecBlock);
+    const tv_rows rows = ix->rows();
+    a.codes = rows.codes;
+    a.scales = rows.scales;
+    a.n = uint32_t(rows.n);
+    a.n_blocks = uint32_t((rows.n + tv::kVecBlock - 1) / tv::kVecBlock);
     a.nch = ix->geo.nch;
     std::memcpy(a.lv, ix->levels, 16);
     a.classic = effective_mode(ix) == TV_SCORE_L_CLASSIC ? 1 : effective_mode(ix) == TV_SCORE_L_SCALAR ? 2 : 0;
@@ -485,7 +488,7 @@ size_t robust_need(const tv_index *ix, size_t cq, size_t k_eff) {
     const size_t total_threads = size_t(grid) * tv::kScanThreads;
     size_t need = prepare_bytes(ix, cq) + round_up(n_tiles * tv::kQTile * 4, 256);
     if (lists) need += 2 * round_up(k_eff * total_threads * 4, 256) + round_up(total_threads * 4, 256);
-    else need += round_up(size_t(tv::kQTile) * ix->n * 4, 256) + round_up(tv::select_tmp_keys(k_eff) * 8 * tv::kQTile, 256) +
+    else need += round_up(size_t(tv::kQTile) * ix->rows().n * 4, 256) + round_up(tv::select_tmp_keys(k_eff) * 8 * tv::kQTile, 256) +
                  round_up(size_t(tv::kQTile) * 4096 * 4, 256);
     return need + 65536;
 }
@@ -624,7 +627,7 @@ size_t sampled_need_worst(const tv_index *ix, size_t nq) {
 // queries whose candidate buffer overflowed and for very large k.
 int search_robust(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask,
                   float *d_out_scores, int64_t *d_out_idx, bool timed_run) {
-    const size_t n = ix->n;
+    const size_t n = ix->rows().n;
     const tv::Geometry &g = ix->geo;
     const int mode = effective_mode(ix);
     const bool mode_p = mode == TV_SCORE_P;
@@ -689,6 +692,7 @@ int search_robust(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             } else {
                 TV_HIP(tv::launch_select_topk(d_dense, n, a.nq_tile, k_eff, d_keys, d_hist, os, oi, ix->stream));
             }
+            if (ix->rows().slots) TV_HIP(tv::launch_map_slots(oi, size_t(a.nq_tile) * k_eff, ix->rows().slots, n, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));
         for (size_t t = 0; timed_run && t < n_tiles && int(t) < kMaxTimedTiles; ++t) {
@@ -882,7 +886,7 @@ int take_stamps(tv_index *ix, int launches) {
 int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
                   int64_t *d_out_idx, bool timing) {
     const tv::Geometry &g = ix->geo;
-    const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
+    const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
     int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
     if (rc != TV_OK) return rc;
     ix->last_queries_per_launch = int(chunk_len(ix, nq));
@@ -920,7 +924,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                 rc = best_scan_lut(ix, a, pq, cq);
                 if (rc != TV_OK) return rc;
             }
-            TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->d_flags_host + c0,
+            TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->rows().slots, ix->d_flags_host + c0,
                                    timed ? ix->d_stamps + 1 : nullptr, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));
@@ -952,9 +956,9 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
 // scanned, hence a lower bound of the true k-th best, so the full scan appends
 // every member of the true top-k; ties at the floor are kept (>=) and resolved
 // by the same total order as everywhere else.
-int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
-                  size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
-    const size_t n = ix->n;
+int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
+                size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
+    const size_t n = ix->rows().n;
     size_t k_eff = std::min(std::min(k, n), n_allowed);  // lib.rs:1460, search.rs:3222-3225
     if (out_k_eff) *out_k_eff = k_eff;
     ix->last_scan_ms = 0.0f;
@@ -1147,7 +1151,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
                                             int(pq_n), d_os, d_oi, d_over, last ? nullptr : d_tau, int(tile_q),
                                             (lv > 0 || repeat) ? 1 : 0, (last && !repeat) ? d_raise + (q0 - g0) : nullptr,
                                             repeat ? d_rows + row0 : nullptr, lv_flag, attempt == 0 ? next_flag : nullptr,
-                                            run_if, !timed_pass ? nullptr : last ? ix->d_stamps + 1 : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
+                                            run_if, ix->rows().slots, !timed_pass ? nullptr : last ? ix->d_stamps + 1 : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
                                             ix->stream));
                 }
             }
@@ -1240,6 +1244,89 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         }
     }
     return TV_OK;
+}
+
+// ---- filtered searches on the allowed rows alone (tv_filter.hip) ----
+// What a scan costs per block, in ns, about: its codes at 6.4 TB/s, or the products and the epilogue of each tile of 32 queries, or
+// passes over u8 tables.  (P: 4M x 768, 300 queries 1.3 ms, 1024 3.3, 2M x 1536 1.2 and 3.1; tables: 1M x 1536 2-bit, 300 queries 1.7 ms,
+// 1024 4.6, 4M x 256 1.8 and 5.2, 778K x 1000 3-bit 1.2 and 2.9, all with 10 % of the rows allowed.)
+double scan_block_ns(const tv_index *ix, size_t nq) {
+    const double tiles = double((nq + tv::kQTile - 1) / tv::kQTile), nch = double(ix->geo.nch);
+    if (effective_mode(ix) == TV_SCORE_P) return std::max(0.165 * nch, tiles * (0.055 * nch + 0.25) + 0.1 * nch);
+    if (effective_mode(ix) != TV_SCORE_L_U32) return std::max(0.165, 0.025 * double(nq)) * nch;
+    if (nq <= size_t(tv::kLut16Queries)) return (0.165 + 0.02 * double(nq)) * nch + 0.3;
+    return tiles * ((ix->geo.bits == 2 ? 0.37 : 0.22) * nch + 0.6);
+}
+// What any block costs a tile of a large batch, one without an allowed row too: passing it, its place among the best words (a
+// range of 1 % of the rows, 1024 queries: 4M x 256 2-bit 522 us with the mask and 144 gathered, 1M x 128 215 and 86).
+constexpr double kPassedBlockNs = 0.08;
+// Gathering, per gathered block and chunk: the lines its rows lie in, up to eight times their bytes, and the write; and its
+// launches and the wait for the count, 15 us of it spent once it is known.  The launches that a search without sampling saves.
+constexpr double kGatherNs = 0.2, kGatherFixedNs = 20000.0, kCountedNs = 5000.0, kUnsampledNs = 25000.0;
+constexpr size_t kGatheredBytes = size_t(1) << 30;      // the largest such copy an index keeps room for
+bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed) {
+    const double blocks = n_allowed / tv::kVecBlock + 1.0, each = scan_block_ns(ix, nq);
+    const double passed = nq > size_t(tv::kQTile) ? kPassedBlockNs * double((nq + tv::kQTile - 1) / tv::kQTile) : 0.0;
+    const double gather = kGatherNs * double(ix->geo.nch) * (1.0 + std::min(8.0, live_blocks / blocks));
+    const bool shorter = direct_serves(ix, nq, k, size_t(blocks)) && !direct_serves(ix, nq, k, size_t(n_blocks));
+    return live_blocks * each + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > blocks * (each + passed + gather) + fixed;
+}
+size_t gathered_need(const tv_index *ix, size_t n_allowed) {
+    const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
+    return round_up(blocks * ix->geo.block_bytes(), 256) + blocks * tv::kVecBlock * sizeof(float);
+}
+// With the mask read during the scan, and gathered, us a search (k = 10): 10 % of the rows allowed at random, 4M x 256 2-bit, 1024 queries 5210 and
+// 680; 4M x 768, 300 queries 1359 and 403; 1M x 768, 40 queries 131 and 105, 1 query 112 and 104; 1 %: 2M x 1536, 1024 queries 1295 and
+// 165, 1 query 152 and 74; 50 %: 4M x 768, 1024 queries 3337 and 2030, 300 queries 1310 and 1050, 64 queries 425 and 660.  A range of
+// rows, 20 %: 4M x 768, 300 queries 376 and 470; such a search pays up to 13 us for the count that tells (100K x 128, 1024 queries: 54
+// and 67).
+// Gathers the rows `d_mask` allows where a search of nq queries is faster on them; ix->allowed then has them.  Whether rows
+// lie scattered, which it depends on, is counted on the device and waited for; from the number of allowed rows
+// alone, taken to be scattered, most calls that it cannot pay for are told without.
+int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t nq, size_t k_eff) {
+    const size_t n = ix->n, n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (ix->ws_fixed || ix->no_gather || n_allowed == 0 || n_allowed >= n || n >= (size_t(1) << 31)) return TV_OK;
+    if (gathered_need(ix, n_allowed) > kGatheredBytes) return TV_OK;
+    const double scattered = double(n_blocks) * (1.0 - std::pow(1.0 - double(n_allowed) / double(n), double(tv::kVecBlock)));
+    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs)) return TV_OK;
+    // (no memory for it: the search reads the mask as it scans, as it would have)
+    auto room = [&](void *&p, size_t &have, size_t bytes) {
+        if (ensure_block(ix, p, have, bytes) == TV_OK) return true;
+        g_last_error.clear();
+        return false;
+    };
+    const size_t count_bytes = round_up(tv::mask_counts(n) * 2 * sizeof(uint32_t), 256);
+    if (!room(ix->slots, ix->slots_bytes, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
+    uint32_t *counts = static_cast<uint32_t *>(ix->slots), *slots = counts + count_bytes / sizeof(uint32_t);
+    volatile uint32_t *totals = ix->h_flags;
+    totals[2] = 0;
+    TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->d_flags_host, ix->stream));
+    // (a wait of a few microseconds, which through the runtime takes ten more; beyond that it is the runtime's)
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (totals[2] == 0 && std::chrono::steady_clock::now() < until) {}
+    if (totals[2] == 0) TV_HIP(hipStreamSynchronize(ix->stream));
+    std::atomic_thread_fence(std::memory_order_acquire);
+    const size_t total = totals[0], live = totals[1];
+    if (total != n_allowed) return TV_OK;      // (the caller's count is not the mask's)
+    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs)) return TV_OK;
+    if (!room(ix->gathered, ix->gathered_bytes, gathered_need(ix, total))) return TV_OK;
+    uint8_t *codes = static_cast<uint8_t *>(ix->gathered);
+    float *scales = reinterpret_cast<float *>(codes + round_up((total + tv::kVecBlock - 1) / tv::kVecBlock * ix->geo.block_bytes(), 256));
+    TV_HIP(tv::launch_gather_rows(ix->d_codes, ix->d_scales, ix->geo.nch, slots, total, codes, scales, ix->stream));
+    ix->allowed = tv_rows{codes, scales, total, slots};
+    ++ix->gathered_searches;
+    return TV_OK;
+}
+int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
+                  size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
+    if (d_mask && k != 0 && nq != 0) {
+        const int rc = gather_allowed(ix, d_mask, n_allowed, nq, std::min(std::min(k, ix->n), n_allowed));
+        if (rc != TV_OK) return rc;
+    }
+    if (ix->allowed.codes) d_mask = nullptr;
+    const int rc = search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    ix->allowed = tv_rows{};
+    return rc;
 }
 
 // ---- search calls, merged ----------------------------------------------------------------------
@@ -1576,6 +1663,8 @@ int tv_index_destroy(tv_index *ix) {
     (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
     (void)device_free(ix->device, ix->ws, ix->ws_bytes);
     (void)device_free(ix->device, ix->io, ix->io_bytes);
+    (void)device_free(ix->device, ix->slots, ix->slots_bytes);
+    (void)device_free(ix->device, ix->gathered, ix->gathered_bytes);
     for (void *p : ptrs) if (p) (void)hipFree(p);
     {
         DevicePool &pool = g_pool[ix->device];
@@ -2403,6 +2492,8 @@ int tv_debug_set_path(tv_index *ix, int force_full_lists) {
     ix->no_wide = (force_full_lists & 4) != 0;
     ix->no_lut16 = (force_full_lists & 8) != 0;
     ix->no_direct = (force_full_lists & 16) != 0;
+    ix->force_gather = (force_full_lists & 64) != 0;
+    ix->no_gather = !ix->force_gather && force_full_lists != 0;     // (a call that names its kernels means them with the mask)
     return TV_OK;
 }
 
@@ -2452,6 +2543,12 @@ int tv_debug_overflow_redos(const tv_index *ix, size_t *count) {
 int tv_debug_exact_redos(const tv_index *ix, size_t *count) {
     if (!ix || !count) return TV_ERR_BAD_ARGUMENT;
     *count = ix->exact_redos;
+    return TV_OK;
+}
+
+int tv_debug_gathered_searches(const tv_index *ix, size_t *count) {
+    if (!ix || !count) return TV_ERR_BAD_ARGUMENT;
+    *count = ix->gathered_searches;
     return TV_OK;
 }
 

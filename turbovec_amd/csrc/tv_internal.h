@@ -156,8 +156,8 @@ constexpr uint32_t kMaxFloorBlocks = 8192;
 hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,
                         hipStream_t s);
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut);
-hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
-                       hipStream_t s);
+hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, const uint32_t *slots, uint32_t *overflow,
+                       uint64_t *stamp, hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).
 int batched_tiles(int nch);
@@ -187,11 +187,12 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 // nothing otherwise); row_map, when given, names the output row of each query.
 // level_over (sampling levels): set to 1 when some query's candidates of this level did not all fit
 // (its floor then comes from a subset and may be far too low); clear_flag: a word this launch resets
-// to 0 (the flag of the level after); run_if: when given and *run_if == 0 the launch does nothing.
+// to 0 (the flag of the level after); run_if: when given and *run_if == 0 the launch does nothing; slots: when
+// given, the slot of each row, for out_idx.
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp, hipStream_t s);
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, hipStream_t s);
 // Packs the queries rows[0..n_redo) of a chunk and their raised floors for one more full scan.
 hipError_t launch_gather_redo(const float *d_q, const uint32_t *d_rows, const int *d_raised, int dim, int tile_q,
                               size_t n_redo, float *d_q_out, int *d_tau_out, hipStream_t s);
@@ -202,6 +203,14 @@ hipError_t launch_probe_mfma(int device, int iters, uint32_t *sink, double *ops,
 hipError_t launch_select_topk(const float *d_scores, size_t n, int nq_tile, size_t k_eff, uint64_t *d_keys_tmp,
                               uint32_t *d_hist, float *out_scores, int64_t *out_idx, hipStream_t s);
 size_t select_tmp_keys(size_t k_eff);
+// Filtered searches on the allowed rows alone (tv_filter.hip).  The rows of the mask's set bits below n, in order, to slots[0 .. room), and
+// how many there are and in how many blocks to totals[0], totals[1] (host memory; totals[2] is 1 after them); counts: two words for each of mask_counts(n) workgroups.
+size_t mask_counts(size_t n);
+hipError_t launch_mask_slots(const uint64_t *mask, size_t n, uint32_t *counts, uint32_t *slots, size_t room, uint32_t *totals, hipStream_t s);
+// The rows slots[0 .. n) into blocks of their own, the last one's missing rows zero.
+hipError_t launch_gather_rows(const uint8_t *codes, const float *scales, int nch, const uint32_t *slots, size_t n, uint8_t *out, float *out_scales, hipStream_t s);
+// idx[i] = slots[idx[i]] where idx[i] is below n.
+hipError_t launch_map_slots(int64_t *idx, size_t count, const uint32_t *slots, size_t n, hipStream_t s);
 
 }  // namespace tv
 
@@ -212,6 +221,14 @@ struct tv_pinned {
     uint8_t *host = nullptr, *dev = nullptr;   // the same bytes, as the host and as the device address them
     size_t bytes = 0;
     bool lent = false;
+};
+
+// What a search reads: n rows in blocks of 32, scales padded to whole blocks.
+struct tv_rows {
+    const uint8_t *codes = nullptr;
+    const float *scales = nullptr;
+    size_t n = 0;
+    const uint32_t *slots = nullptr;   // the index's slot of each row, when that is not its place
 };
 
 // The opaque handle of the C ABI.
@@ -262,8 +279,12 @@ struct tv_index {
     static constexpr int kPinned = 8;
     std::mutex pinned_mu;
     tv_pinned pinned[kPinned];     // allocated on first use, at most kPinnedBytes in all (tv_api.hip), freed with the index
+    void *slots = nullptr, *gathered = nullptr;   // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
+    size_t slots_bytes = 0, gathered_bytes = 0;
+    tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
+    tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr}; }
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
-    uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat
+    uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat (before a search: a mask's totals)
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags
     uint64_t *h_stamps = nullptr, *d_stamps = nullptr;   // in the same allocation: the device clock before and after a full scan
     size_t exact_redos = 0;        // queries that went on to the exact path
@@ -276,6 +297,9 @@ struct tv_index {
     bool no_lut_mx = false;        // for the length of a call: the scratch array holds only the sixteen-query passes' working set
     int no_wide = 0;               // test hook: large batches go through the tile-group kernels, not the wide one
     int no_direct = 0;             // test hook: small indexes are sampled like large ones
+    int no_gather = 0;             // test hook: filtered searches read the mask as they scan ...
+    int force_gather = 0;          // ... or gather their allowed rows whatever their number
+    size_t gathered_searches = 0;  // searches that did
     size_t overflow_redos = 0;     // queries redone because their candidate buffer overflowed
     // The floorless first level (best row per block) misjudges the floor when a query's neighbours
     // sit together in a few blocks (a clustered corpus in insertion order): after a search in which

@@ -950,7 +950,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                uint32_t *__restrict__ overflow, int *__restrict__ tau_out,
                                                int tau_stride_q, int keep_floor, int *__restrict__ raise_out,
                                                const uint32_t *__restrict__ row_map, uint32_t *level_over,
-                                               uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp) {
+                                               uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp) {
     constexpr uint32_t W = T / 64;
     __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ uint64_t stage[kFinalStage];
@@ -1130,7 +1130,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
             if (rank == need - 1u) *(sampling ? tau_slot : raise_out + qn) = order_key(s == 0.0f ? -0.0f : s);
         } else {
             out_scores[row * k_eff + rank] = s;
-            out_idx[row * k_eff + rank] = int64_t(idx);
+            out_idx[row * k_eff + rank] = int64_t(slots != nullptr ? slots[idx] : idx);
         }
     }
     stamp_end();
@@ -1432,11 +1432,11 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, uint64_t *stamp, hipStream_t s) {
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, hipStream_t s) {
     if (nq == 0 || k_eff == 0) return hipSuccess;
     auto launch = [&](auto kernel, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
-                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, stamp);
+                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp);
     };
     if (n_seg <= 256) launch(k_final<256>, 256);
     else if (n_seg <= 512) launch(k_final<512>, 512);

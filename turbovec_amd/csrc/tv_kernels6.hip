@@ -267,6 +267,7 @@ struct PickArgs {
     int nch, k_eff, split;
     float *out_scores;
     int64_t *out_idx;
+    const uint32_t *slots;      // when given: the slot of each row, for out_idx
     uint32_t *overflow;
     uint64_t *stamp;
 };
@@ -436,15 +437,15 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         float s; uint32_t idx;
         sort_unkey(k, s, idx);
         a.out_scores[size_t(qi) * k_eff + rank] = s;
-        a.out_idx[size_t(qi) * k_eff + rank] = int64_t(idx);
+        a.out_idx[size_t(qi) * k_eff + rank] = int64_t(a.slots != nullptr ? a.slots[idx] : idx);
     }
 }
 
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64); }
 
 // The scan's arguments say what was scanned; a.tables: its weight tiles, or (lut) the queries' tables as k_prep_lut leaves them.
-hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, uint32_t *overflow, uint64_t *stamp,
-                       hipStream_t s) {
+hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, const uint32_t *slots, uint32_t *overflow,
+                       uint64_t *stamp, hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
     const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff), lut);
     if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
@@ -454,7 +455,7 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     p.qscale = a.qscale; p.qbias = a.qbias;
     for (int i = 0; i < 4; ++i) p.lv[i] = a.lv[i];
     p.nch = a.nch; p.k_eff = k_eff; p.split = split ? 1 : 0;
-    p.out_scores = out_scores; p.out_idx = out_idx; p.overflow = overflow; p.stamp = stamp;
+    p.out_scores = out_scores; p.out_idx = out_idx; p.slots = slots; p.overflow = overflow; p.stamp = stamp;
     auto launch = [&](auto kernel, unsigned threads) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
