@@ -275,8 +275,9 @@ int tv_debug_level_repeats(tv_index *ix, int track, size_t *count);
 /* Bytes of the index's cached search workspace and of its host-call staging allocation (either
  * pointer may be NULL): both only ever grow, and tv_search_dev_noalloc touches neither. */
 int tv_debug_workspace_bytes(const tv_index *ix, size_t *workspace, size_t *staging);
-/* How many filtered searches so far ran on a copy of their allowed rows. */
-int tv_debug_gathered_searches(const tv_index *ix, size_t *count);
+/* How many filtered searches so far ran on their allowed rows alone, and how many of
+ * those read them in place, without a copy. */
+int tv_debug_gathered_searches(const tv_index *ix, size_t *count, size_t *in_place);
 /* How many queries so far did not finish in the single sampled pass because their
  * candidate buffer overflowed (they are scanned once more, all together, from a raised
  * floor), and how many of those went on to the exact list / select path. */

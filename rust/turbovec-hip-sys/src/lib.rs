@@ -95,7 +95,7 @@ extern "C" {
     pub fn tv_debug_overflow_redos(ix: *const tv_index, count: *mut usize) -> c_int;
     pub fn tv_debug_exact_redos(ix: *const tv_index, count: *mut usize) -> c_int;
     pub fn tv_debug_merged_calls(ix: *const tv_index, count: *mut usize) -> c_int;
-    pub fn tv_debug_gathered_searches(ix: *const tv_index, count: *mut usize) -> c_int;
+    pub fn tv_debug_gathered_searches(ix: *const tv_index, count: *mut usize, in_place: *mut usize) -> c_int;
     pub fn tv_debug_stream_probe(ix: *mut tv_index, d_src: *const c_void, d_dst: *mut c_void, bytes: usize, reps: c_int, ms_per_rep: *mut c_float) -> c_int;
     pub fn tv_debug_mfma_probe(ix: *mut tv_index, iters: c_int, reps: c_int, ms_per_rep: *mut c_float, ops_per_rep: *mut c_double) -> c_int;
     pub fn tv_index_device_ptrs(ix: *const tv_index, d_codes: *mut *mut c_void, d_scales: *mut *mut c_void, code_bytes: *mut usize) -> c_int;

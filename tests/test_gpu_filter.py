@@ -60,10 +60,10 @@ def test_gathered_rows_give_the_masked_scan_s_bits(T, dim, bits, n, nq):
         for k in (1, 10, 600) if allowed < 5000 else (10,):
             ix.set_path(MASKED)
             s, i = ix.search(q, k, mask_words=words)
-            before = ix.gathered_searches()
+            before = ix.gathered_searches()[0]
             ix.set_path(GATHERED)
             s2, i2 = ix.search(q, k, mask_words=words)
-            assert ix.gathered_searches() == before + 1
+            assert ix.gathered_searches()[0] == before + 1
             assert np.array_equal(i, i2) and bits_equal(s, s2), (allowed, k)
     ix.close()
 
@@ -107,7 +107,7 @@ def test_a_count_that_is_not_the_mask_s(T, stated):
         ix.set_path(path)
         ix.search_dev(q.data_ptr(), nq, k, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed + stated)
         out.append((s.cpu().numpy(), i.cpu().numpy()))
-    assert ix.gathered_searches() == 0
+    assert ix.gathered_searches()[0] == 0
     assert np.array_equal(out[0][1], out[1][1]) and bits_equal(out[0][0], out[1][0])
     ix.close()
 
@@ -120,11 +120,56 @@ def test_where_the_rows_are_gathered(T):
     few = np.random.default_rng(5).random(n) < 0.01
     for m, nq, yes in ((few, 1024, True), (np.arange(n) < 40_000, 1024, False), (few, 1, False), (np.ones(n, bool), 1024, False)):
         words, _ = T.pack_mask(m)
-        before = ix.gathered_searches()
+        before = ix.gathered_searches()[0]
         ix.set_path(0)
         s, i = ix.search(q[:nq], 10, mask_words=words)
-        assert ix.gathered_searches() == before + yes
+        assert ix.gathered_searches()[0] == before + yes
         ix.set_path(MASKED)
         s2, i2 = ix.search(q[:nq], 10, mask_words=words)
         assert np.array_equal(i, i2) and bits_equal(s, s2)
+    ix.close()
+
+
+def wide_masks(n, rng):
+    m = rng.random(n) < 0.5
+    yield m
+    m = rng.random(n) < 0.9
+    m[[0, n - 1]] = True
+    yield m
+    yield (np.arange(n) % 64 < 32) | (np.arange(n) > n - 100)
+
+
+# every instance that reads rows from a list; k large enough for the sampled search, a last block of a few rows
+@pytest.mark.parametrize("dim,nq,k", [(768, 300, 60), (768, 1024, 64), (1024, 150, 45), (1536, 130, 30), (1536, 1500, 26), (2048, 140, 20), (3072, 257, 13)])
+def test_rows_read_in_place(T, dim, nq, k):
+    n = 60_001
+    ix, gen = filled(T, dim, 4, n)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    for m in wide_masks(n, np.random.default_rng(dim)):
+        words, _ = T.pack_mask(m)
+        ix.set_path(MASKED)
+        s, i = ix.search(q, k, mask_words=words)
+        before = ix.gathered_searches()
+        ix.set_path(GATHERED)
+        s2, i2 = ix.search(q, k, mask_words=words)
+        after = ix.gathered_searches()
+        assert (after[0] - before[0], after[1] - before[1]) == (1, 1)
+        assert np.array_equal(i, i2) and bits_equal(s, s2)
+    ix.close()
+
+
+def test_rows_in_place_whose_candidates_do_not_fit(T):
+    """Every row ties, so every candidate passes: the search is done again on a copy, and on the exact path."""
+    dim, n, nq, k = 768, 60_001, 140, 60
+    one = torch.randn(1, dim, device="cuda:0", generator=torch.Generator(device="cuda:0").manual_seed(1))
+    v = one.repeat(n, 1).contiguous()
+    torch.cuda.synchronize()
+    ix = T.NativeIndex(dim, 4)
+    ix.add_dev(v.data_ptr(), n)
+    m = np.random.default_rng(3).random(n) < 0.5
+    words, _ = T.pack_mask(m)
+    ix.set_path(GATHERED)
+    s, i = ix.search(v[:nq].cpu().numpy(), k, mask_words=words)
+    assert ix.gathered_searches() == (1, 0) and ix.exact_redos() > 0
+    assert np.array_equal(i, np.tile(np.flatnonzero(m)[:k], (nq, 1)))
     ix.close()

@@ -103,7 +103,7 @@ def lib():
     L.tv_debug_set_path.argtypes = [vp, i32]
     L.tv_debug_overflow_redos.argtypes = [vp, C.POINTER(sz)]
     L.tv_debug_exact_redos.argtypes = [vp, C.POINTER(sz)]
-    L.tv_debug_gathered_searches.argtypes = [vp, C.POINTER(sz)]
+    L.tv_debug_gathered_searches.argtypes = [vp, C.POINTER(sz), C.POINTER(sz)]
     L.tv_debug_workspace_bytes.argtypes = [vp, C.POINTER(sz), C.POINTER(sz)]
     L.tv_debug_level_repeats.argtypes = [vp, i32, C.POINTER(sz)]
     L.tv_debug_merged_calls.argtypes = [vp, C.POINTER(sz)]
@@ -325,9 +325,10 @@ class NativeIndex:
         check(lib().tv_debug_set_path(self.h, int(force_full_lists)))
 
     def gathered_searches(self):
-        c = C.c_size_t(0)
-        check(lib().tv_debug_gathered_searches(self.h, C.byref(c)))
-        return c.value
+        """Filtered searches that ran on their allowed rows alone, and those of them that read the rows in place."""
+        c, p = C.c_size_t(0), C.c_size_t(0)
+        check(lib().tv_debug_gathered_searches(self.h, C.byref(c), C.byref(p)))
+        return c.value, p.value
 
     def overflow_redos(self):
         c = C.c_size_t(0)

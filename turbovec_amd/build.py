@@ -36,9 +36,9 @@ NO_SCRATCH = re.compile(r"k_scan_p4I|k_scan_p4_multiI|k_scan_p4_wideI|k_scan_lut
 SGPR_LANES = re.compile(r"k_scan_lut_mxI")
 # These address their byte -> levels table by the byte's value alone: the table must sit at LDS
 # address 0, i.e. the kernel may have no static LDS allocation in front of its dynamic one
-# (k_scan_p4, k_scan_p4_multi, and the instances of k_scan_p4_wide whose last template argument,
-# the split decode, is true).
-NO_STATIC_LDS = re.compile(r"k_scan_p4(_multi)?I|k_scan_p4_wideI.*Lb1EEEv")
+# (k_scan_p4, k_scan_p4_multi, and the instances of k_scan_p4_wide whose last template argument but
+# one, the split decode, is true).
+NO_STATIC_LDS = re.compile(r"k_scan_p4(_multi)?I|k_scan_p4_wideI.*Lb1ELb[01]EEEv")
 
 
 def check_resources(src, remarks):

@@ -449,6 +449,7 @@ void fill_scan_args(const tv_index *ix, tv::ScanArgs &a) {
     a.codes = rows.codes;
     a.scales = rows.scales;
     a.n = uint32_t(rows.n);
+    a.rows = rows.in_place ? rows.slots : nullptr;
     a.n_blocks = uint32_t((rows.n + tv::kVecBlock - 1) / tv::kVecBlock);
     a.nch = ix->geo.nch;
     std::memcpy(a.lv, ix->levels, 16);
@@ -622,11 +623,13 @@ size_t sampled_need_worst(const tv_index *ix, size_t nq) {
     return need + group_header_bytes(ix, gq);
 }
 
+constexpr int kNeedsCopy = -1000;     // not a status of the library: a search of rows in place that has to run on a copy of them
 // Full-range search without sampling: per-lane lists with shared thresholds for
 // k <= 32, dense scores + radix select beyond.  Always exact; used for the
 // queries whose candidate buffer overflowed and for very large k.
 int search_robust(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask,
                   float *d_out_scores, int64_t *d_out_idx, bool timed_run) {
+    if (ix->allowed.in_place) return kNeedsCopy;
     const size_t n = ix->rows().n;
     const tv::Geometry &g = ix->geo;
     const int mode = effective_mode(ix);
@@ -885,6 +888,7 @@ int take_stamps(tv_index *ix, int launches) {
 }
 int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
                   int64_t *d_out_idx, bool timing) {
+    if (ix->allowed.in_place) return kNeedsCopy;
     const tv::Geometry &g = ix->geo;
     const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
     int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
@@ -1020,6 +1024,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const int grid = plan.grid;
             const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat, d_mask != nullptr);
             const bool best_first = steps.best_first;
+            if (ix->allowed.in_place && (!wide || steps.best_words)) return kNeedsCopy;
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
                 g_last_error = "internal: workspace smaller than the pass it was sized for";
@@ -1208,6 +1213,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 ix->floorless_kept_left = kRowLadderSearches;
             }
         }
+        if (ix->allowed.in_place && !(redo_rows.empty() && exact_rows.empty())) return kNeedsCopy;     // (the passes below run on every kernel)
         const size_t room = ix->ws_bytes - head.used;
         for (size_t i = 0; i < redo_rows.size();) {
             // rows of one chunk go together: all of them in one pass when the workspace holds that
@@ -1264,10 +1270,10 @@ constexpr double kPassedBlockNs = 0.08;
 // launches and the wait for the count, 15 us of it spent once it is known.  The launches that a search without sampling saves.
 constexpr double kGatherNs = 0.2, kGatherFixedNs = 20000.0, kCountedNs = 5000.0, kUnsampledNs = 25000.0;
 constexpr size_t kGatheredBytes = size_t(1) << 30;      // the largest such copy an index keeps room for
-bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed) {
+bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed, bool in_place) {
     const double blocks = n_allowed / tv::kVecBlock + 1.0, each = scan_block_ns(ix, nq);
     const double passed = nq > size_t(tv::kQTile) ? kPassedBlockNs * double((nq + tv::kQTile - 1) / tv::kQTile) : 0.0;
-    const double gather = kGatherNs * double(ix->geo.nch) * (1.0 + std::min(8.0, live_blocks / blocks));
+    const double gather = kGatherNs * double(ix->geo.nch) * ((in_place ? -1.0 : 1.0) + std::min(8.0, live_blocks / blocks));
     const bool shorter = direct_serves(ix, nq, k, size_t(blocks)) && !direct_serves(ix, nq, k, size_t(n_blocks));
     return live_blocks * each + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > blocks * (each + passed + gather) + fixed;
 }
@@ -1275,28 +1281,54 @@ size_t gathered_need(const tv_index *ix, size_t n_allowed) {
     const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
     return round_up(blocks * ix->geo.block_bytes(), 256) + blocks * tv::kVecBlock * sizeof(float);
 }
+// Whether a search over n_allowed rows runs on the all-queries kernel throughout, which can read them where they lie
+// (its addresses within a row's index are 32 bits).
+bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowed) {
+    const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock, codes_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (!wide_serves(ix) || !tv::wide_serves_best_of_block(ix->geo.nch) || codes_blocks * ix->geo.block_bytes() > 0xffffffffull) return false;
+    if (k_eff > size_t(tv::kMaxSampledK) || ix->force_robust || direct_serves(ix, nq, k_eff, blocks)) return false;
+    for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
+        const size_t gq = std::min(kGroupQueries, nq - g0);
+        for (size_t c0 = 0, cq; c0 < gq; c0 += cq) {
+            cq = chunk_len(ix, gq - c0);
+            const SampledPlan plan = sampled_plan(ix, cq);
+            if (!plan.wide || !tv::wide_reads_rows(ix->geo.nch, int(cq)) || level_strides(ix, plan, blocks, std::max<size_t>(k_eff, 16), false, false).best_words) return false;
+        }
+    }
+    return true;
+}
+// A block where there is memory for it.  (The search reads the mask as it scans otherwise, as it would have.)
+bool have_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
+    if (ensure_block(ix, p, have, bytes) == TV_OK) return true;
+    g_last_error.clear();
+    return false;
+}
+int copy_allowed(tv_index *ix, const uint32_t *slots, size_t total) {
+    if (!have_block(ix, ix->gathered, ix->gathered_bytes, gathered_need(ix, total))) return TV_OK;
+    uint8_t *codes = static_cast<uint8_t *>(ix->gathered);
+    float *scales = reinterpret_cast<float *>(codes + round_up((total + tv::kVecBlock - 1) / tv::kVecBlock * ix->geo.block_bytes(), 256));
+    TV_HIP(tv::launch_gather_rows(ix->d_codes, ix->d_scales, ix->geo.nch, slots, total, codes, scales, ix->stream));
+    ix->allowed = tv_rows{codes, scales, total, slots, false};
+    return TV_OK;
+}
 // With the mask read during the scan, and gathered, us a search (k = 10): 10 % of the rows allowed at random, 4M x 256 2-bit, 1024 queries 5210 and
 // 680; 4M x 768, 300 queries 1359 and 403; 1M x 768, 40 queries 131 and 105, 1 query 112 and 104; 1 %: 2M x 1536, 1024 queries 1295 and
-// 165, 1 query 152 and 74; 50 %: 4M x 768, 1024 queries 3337 and 2030, 300 queries 1310 and 1050, 64 queries 425 and 660.  A range of
-// rows, 20 %: 4M x 768, 300 queries 376 and 470; such a search pays up to 13 us for the count that tells (100K x 128, 1024 queries: 54
-// and 67).
+// 165, 1 query 152 and 74; 50 %: 4M x 768, 64 queries 425 and 660.  A range of 20 % of the
+// rows: 4M x 768, 300 queries 376 and 470; such a search pays up to 13 us for the count that tells (100K x 128, 1024 queries: 54
+// and 67).  Read in place (with the mask, copied, in place): 50 %, 4M x 768, 1024 queries 3337, 2030 and 1650, 300 queries 1310, 1050 and
+// 700; 80 % 1330 and 970 in place; 30 %, 2M x 1536, 300 queries 1181 and 754; a range of half the rows, 1024 queries 1601 and 1576.
 // Gathers the rows `d_mask` allows where a search of nq queries is faster on them; ix->allowed then has them.  Whether rows
 // lie scattered, which it depends on, is counted on the device and waited for; from the number of allowed rows
 // alone, taken to be scattered, most calls that it cannot pay for are told without.
 int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t nq, size_t k_eff) {
     const size_t n = ix->n, n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (ix->ws_fixed || ix->no_gather || n_allowed == 0 || n_allowed >= n || n >= (size_t(1) << 31)) return TV_OK;
-    if (gathered_need(ix, n_allowed) > kGatheredBytes) return TV_OK;
+    const bool in_place = scans_in_place(ix, nq, k_eff, n_allowed);
+    if (!in_place && gathered_need(ix, n_allowed) > kGatheredBytes) return TV_OK;
     const double scattered = double(n_blocks) * (1.0 - std::pow(1.0 - double(n_allowed) / double(n), double(tv::kVecBlock)));
-    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs)) return TV_OK;
-    // (no memory for it: the search reads the mask as it scans, as it would have)
-    auto room = [&](void *&p, size_t &have, size_t bytes) {
-        if (ensure_block(ix, p, have, bytes) == TV_OK) return true;
-        g_last_error.clear();
-        return false;
-    };
+    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs, in_place)) return TV_OK;
     const size_t count_bytes = round_up(tv::mask_counts(n) * 2 * sizeof(uint32_t), 256);
-    if (!room(ix->slots, ix->slots_bytes, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
+    if (!have_block(ix, ix->slots, ix->slots_bytes, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
     uint32_t *counts = static_cast<uint32_t *>(ix->slots), *slots = counts + count_bytes / sizeof(uint32_t);
     volatile uint32_t *totals = ix->h_flags;
     totals[2] = 0;
@@ -1308,25 +1340,27 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
     std::atomic_thread_fence(std::memory_order_acquire);
     const size_t total = totals[0], live = totals[1];
     if (total != n_allowed) return TV_OK;      // (the caller's count is not the mask's)
-    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs)) return TV_OK;
-    if (!room(ix->gathered, ix->gathered_bytes, gathered_need(ix, total))) return TV_OK;
-    uint8_t *codes = static_cast<uint8_t *>(ix->gathered);
-    float *scales = reinterpret_cast<float *>(codes + round_up((total + tv::kVecBlock - 1) / tv::kVecBlock * ix->geo.block_bytes(), 256));
-    TV_HIP(tv::launch_gather_rows(ix->d_codes, ix->d_scales, ix->geo.nch, slots, total, codes, scales, ix->stream));
-    ix->allowed = tv_rows{codes, scales, total, slots};
-    ++ix->gathered_searches;
+    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs, in_place)) return TV_OK;
+    if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, total, slots, true};
+    else if (const int rc = copy_allowed(ix, slots, total)) return rc;
+    if (ix->allowed.codes) ++ix->gathered_searches;
     return TV_OK;
 }
 int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
                   size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
+    struct Back { tv_index *ix; ~Back() { ix->allowed = tv_rows{}; } } back{ix};
     if (d_mask && k != 0 && nq != 0) {
         const int rc = gather_allowed(ix, d_mask, n_allowed, nq, std::min(std::min(k, ix->n), n_allowed));
         if (rc != TV_OK) return rc;
     }
-    if (ix->allowed.codes) d_mask = nullptr;
-    const int rc = search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    int rc = search_rows(ix, d_queries, nq, k, ix->allowed.codes ? nullptr : d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    if (ix->allowed.in_place && rc == TV_OK) ++ix->in_place_searches;
+    if (rc != kNeedsCopy) return rc;
+    const tv_rows was = ix->allowed;
     ix->allowed = tv_rows{};
-    return rc;
+    rc = gathered_need(ix, was.n) <= kGatheredBytes ? copy_allowed(ix, was.slots, was.n) : TV_OK;
+    if (rc != TV_OK) return rc;
+    return search_rows(ix, d_queries, nq, k, ix->allowed.codes ? nullptr : d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
 }
 
 // ---- search calls, merged ----------------------------------------------------------------------
@@ -2546,9 +2580,10 @@ int tv_debug_exact_redos(const tv_index *ix, size_t *count) {
     return TV_OK;
 }
 
-int tv_debug_gathered_searches(const tv_index *ix, size_t *count) {
+int tv_debug_gathered_searches(const tv_index *ix, size_t *count, size_t *in_place) {
     if (!ix || !count) return TV_ERR_BAD_ARGUMENT;
     *count = ix->gathered_searches;
+    if (in_place) *in_place = ix->in_place_searches;
     return TV_OK;
 }
 

@@ -72,6 +72,7 @@ struct ScanArgs {
     int best_of_block;         // all-queries-per-pass kernel: no floor, per scanned block and query the best allowed slot (kModeBest)
     uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and scanned block the best allowed row's (tv_kernels6.hip)
     uint32_t best_stride;
+    const uint32_t *rows;      // all-queries-per-pass kernel: when given, the slot of each of the n rows to scan, in order; all codes within 4 GiB
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
 
@@ -174,6 +175,7 @@ int wide_blocks_per_workgroup(int nch);
 bool wide_serves_best_of_block(int nch);
 int wide_max_queries(int nch);
 bool wide_weights_split(int nch);
+bool wide_reads_rows(int nch, int nq);
 
 hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, const int *part_cnt, int total_threads,
                         int qmod, int k, int k_eff, int nq_tile, float *out_scores, int64_t *out_idx,
@@ -229,6 +231,7 @@ struct tv_rows {
     const float *scales = nullptr;
     size_t n = 0;
     const uint32_t *slots = nullptr;   // the index's slot of each row, when that is not its place
+    bool in_place = false;             // ... and codes and scales are the index's own: the rows lie at their slots
 };
 
 // The opaque handle of the C ABI.
@@ -282,7 +285,7 @@ struct tv_index {
     void *slots = nullptr, *gathered = nullptr;   // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
     size_t slots_bytes = 0, gathered_bytes = 0;
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
-    tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr}; }
+    tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr, false}; }
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
     uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat (before a search: a mask's totals)
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags
@@ -299,7 +302,7 @@ struct tv_index {
     int no_direct = 0;             // test hook: small indexes are sampled like large ones
     int no_gather = 0;             // test hook: filtered searches read the mask as they scan ...
     int force_gather = 0;          // ... or gather their allowed rows whatever their number
-    size_t gathered_searches = 0;  // searches that did
+    size_t gathered_searches = 0, in_place_searches = 0;   // searches that ran on the allowed rows alone, and those of them to the end without a copy
     size_t overflow_redos = 0;     // queries redone because their candidate buffer overflowed
     // The floorless first level (best row per block) misjudges the floor when a query's neighbours
     // sit together in a few blocks (a clustered corpus in insertion order): after a search in which

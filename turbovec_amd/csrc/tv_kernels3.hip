@@ -118,16 +118,22 @@ constexpr int kWideTableBytes = 1024;    // the byte table of the split decode (
 // and does the tile's bound test and scoring.  Two blocks per workgroup instead of four, one more
 // barrier per tile: the form for rows beyond what one wave holds.
 //
+// ROWS: the rows to scan lie anywhere, in order (a filter's allowed rows): row i of block b is slot a.rows[32 b + i], and a lane
+// loads its 16 bytes of a chunk from there; blocks, floors and candidates count in places of that list.  Blocks are
+// then full of allowed rows without a copy of them.  (An instance of its own: the registers for the addresses are not there in
+// every form, and the others keep their code.)
+//
 // SPLIT: the block phase decodes half of every chunk through the byte table in LDS, like
 // k_scan_p4 (code bytes 0-7 of a lane on the vector ALU, bytes 8-15 looked up whole); the weights
 // then come in that kernel's split order.  The decode is the block phase -- both waves of a SIMD
 // at it together, the matrix unit idle -- and the LDS has nothing else to do then.
-template <int NCH, int NB, int WAVES, int SPT, int BLK, int HO, int KS, bool SPLIT = false>
+template <int NCH, int NB, int WAVES, int SPT, int BLK, int HO, int KS, bool SPLIT = false, bool ROWS = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide(ScanArgs a) {
     static_assert(NCH % SPT == 0, "a slice is a whole number of chunks");
     static_assert(!SPLIT || (WAVES == 8 && BLK == 1 && KS == 1), "the split decode is built for the one-block eight-wave forms");
     static_assert(KS == 1 || (KS == 2 && WAVES == 4 && BLK == 1 && HO == 1), "row halves go to the wave pairs of the four-wave form");
     constexpr int kWideRing = wide_ring(HO);
+    static_assert(!ROWS || KS == 1, "a row whole");
     static_assert(HO == 1 || (SPT % HO == 0 && kWideRing >= 2 * HO + 1), "slices handed over together must fit the ring twice");
     extern __shared__ __align__(16) uint8_t smem_all[];
     if (launch_switched_off(a.run_if)) return;
@@ -358,14 +364,21 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                 // the whole block in one burst: the previous block's operands are dead by now, so
                 // the raw codes (4 VGPRs per chunk) and the operands decoded from them so far (8 per
                 // chunk) fit the registers the operands alone need at the end
-                const uint8_t *p = a.codes + (size_t(b) * KS + size_t(part)) * (NCH * 1024);
+                const uint8_t *p = ROWS ? a.codes : a.codes + (size_t(b) * KS + size_t(part)) * (NCH * 1024);
+                uint32_t slot = b * 32u + uint32_t(lane & 31), at = lane16;
+                const bool real = slot < a.n;
+                if constexpr (ROWS) {
+                    asm("" : "+s"(p));      // (the chunks' addresses made here: made once, outside the loop, they take a scalar register pair each)
+                    slot = real ? a.rows[slot] : 0u;
+                    at = (slot >> 5) * uint32_t(NCH * 1024) + (uint32_t(h) * 32u + (slot & 31u)) * 16u;
+                }
                 u32x4 raw[NCH];
                 // with hand-written MFMAs the chunks bound for the accumulation registers come
                 // first: their raw codes leave the vector registers before the others' operands grow
                 constexpr int kFirst = kHandMfma && NCH > kVecChunks ? kVecChunks : 0;
                 static_for<NCH>([&](auto ii) {
                     constexpr int c = (decltype(ii)::value + kFirst) % NCH;
-                    load16_async_s(raw[c], p + size_t(c) * 1024, lane16);
+                    load16_async_s(raw[c], p + size_t(c) * 1024, at);
                 });
                 uint32_t te[2][4], to[2][4];    // (split decode) table entries on their way, this chunk's and the next's
                 static_for<NCH>([&](auto ii) {
@@ -425,8 +438,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                         asm volatile("" : "+a"(ahi[k][c]));
                     }
                 });
-                const uint32_t slot = b * 32u + uint32_t(lane & 31);
-                ok = slot < a.n;
+                ok = real;
                 if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> (lane & 31)) & 1u;
                 if (ok) sc = a.scales[slot];
             }
@@ -713,16 +725,16 @@ int wide_grid_blocks(int device) {
     return device_cus(device);      // one 8-wave workgroup per CU: its LDS holds the slice ring
 }
 
-template <int NCH, int NB, int WAVES = 8, int SPT = 2, int BLK = 1, int HO = 1, int KS = 1, bool SPLIT = false>
+template <int NCH, int NB, int WAVES = 8, int SPT = 2, int BLK = 1, int HO = 1, int KS = 1, bool SPLIT = false, bool ROWS = false>
 static hipError_t launch_wide_n(const ScanArgs &a, int grid, hipStream_t s) {
     const size_t lds = wide_lds_bytes(wide_ring(HO), KS * 2 * (NCH / SPT) * 1024, a.nq_tile, BLK, KS, SPLIT);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT>), dim3(grid), dim3(WAVES * 64), lds, s, a);
+    hipLaunchKernelGGL((k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS>), dim3(grid), dim3(WAVES * 64), lds, s, a);
     return hipGetLastError();
 }
 
@@ -730,9 +742,25 @@ static hipError_t launch_wide_n(const ScanArgs &a, int grid, hipStream_t s) {
 // come in the split order of k_scan_p4 (launch_build_p / launch_prep_p, `split`).
 bool wide_weights_split(int nch) { return nch >= 12 && nch <= 24; }
 
+// Whether a launch of nq queries can take the rows to scan from a list (a.rows): 768, 1024, 1536, 2048 and 3072 dimensions.
+bool wide_reads_rows(int nch, int nq) {
+    if (nch == 24) return nq <= wide_max_queries_of(wide_ring(2), 24 * 1024, 1, 1, true);
+    return nch == 12 || nch == 16 || nch == 32 || nch == 48;
+}
+
 // a.nq_tile = all queries of the launch (any number up to the chunk size), a.tables = their
 // ceil(nq/32) weight tiles back to back, a.qscale / a.qbias / a.gtau indexed by query.
 hipError_t launch_scan_p4_wide(const ScanArgs &a, int grid, hipStream_t s) {
+    if (a.rows != nullptr) {
+        switch (a.mask == nullptr ? a.nch : 0) {
+            case 12: return launch_wide_n<12, 2, 8, 2, 1, 2, 1, true, true>(a, grid, s);
+            case 16: return launch_wide_n<16, 4, 8, 2, 1, 2, 1, true, true>(a, grid, s);
+            case 24: return launch_wide_n<24, 2, 8, 2, 1, 2, 1, true, true>(a, grid, s);
+            case 32: return launch_wide_n<32, 4, 4, 4, 1, 1, 1, false, true>(a, grid, s);
+            case 48: return launch_wide_n<48, 4, 4, 4, 1, 1, 1, false, true>(a, grid, s);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (a.nch) {
         // <chunks, B-operand registers, waves, slices per tile, blocks per wave, slices per hand-over>
         // One hand-over per tile (two slices) measured 2.5 to 5 % faster than one per slice in the
