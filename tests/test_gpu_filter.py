@@ -173,3 +173,24 @@ def test_rows_in_place_whose_candidates_do_not_fit(T):
     assert ix.gathered_searches() == (1, 0) and ix.exact_redos() > 0
     assert np.array_equal(i, np.tile(np.flatnonzero(m)[:k], (nq, 1)))
     ix.close()
+
+
+def test_rows_in_place_of_more_than_4_gib(T):
+    """Rows of one block 4 GiB of codes apart are copied instead; scattered over such an index they are read in place."""
+    dim, n, nq, k = 3072, 2_900_000, 140, 13
+    ix, gen = filled(T, dim, 4, n)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    ends = np.zeros(n, bool)
+    ends[:20_016] = True
+    ends[-16:] = True                   # the last block: sixteen rows of either end
+    for m, in_place in ((np.random.default_rng(1).random(n) < 0.5, 1), (ends, 0)):
+        words, _ = T.pack_mask(m)
+        ix.set_path(MASKED)
+        s, i = ix.search(q, k, mask_words=words)
+        before = ix.gathered_searches()
+        ix.set_path(GATHERED)
+        s2, i2 = ix.search(q, k, mask_words=words)
+        after = ix.gathered_searches()
+        assert (after[0] - before[0], after[1] - before[1]) == (1, in_place)
+        assert np.array_equal(i, i2) and bits_equal(s, s2)
+    ix.close()

@@ -1281,11 +1281,10 @@ size_t gathered_need(const tv_index *ix, size_t n_allowed) {
     const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
     return round_up(blocks * ix->geo.block_bytes(), 256) + blocks * tv::kVecBlock * sizeof(float);
 }
-// Whether a search over n_allowed rows runs on the all-queries kernel throughout, which can read them where they lie
-// (its addresses within a row's index are 32 bits).
+// Whether a search over n_allowed rows runs on the all-queries kernel throughout, which can read them where they lie.
 bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowed) {
-    const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock, codes_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
-    if (!wide_serves(ix) || !tv::wide_serves_best_of_block(ix->geo.nch) || codes_blocks * ix->geo.block_bytes() > 0xffffffffull) return false;
+    const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (!wide_serves(ix) || !tv::wide_serves_best_of_block(ix->geo.nch)) return false;
     if (k_eff > size_t(tv::kMaxSampledK) || ix->force_robust || direct_serves(ix, nq, k_eff, blocks)) return false;
     for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
         const size_t gq = std::min(kGroupQueries, nq - g0);
@@ -1316,14 +1315,15 @@ int copy_allowed(tv_index *ix, const uint32_t *slots, size_t total) {
 // 165, 1 query 152 and 74; 50 %: 4M x 768, 64 queries 425 and 660.  A range of 20 % of the
 // rows: 4M x 768, 300 queries 376 and 470; such a search pays up to 13 us for the count that tells (100K x 128, 1024 queries: 54
 // and 67).  Read in place (with the mask, copied, in place): 50 %, 4M x 768, 1024 queries 3337, 2030 and 1650, 300 queries 1310, 1050 and
-// 700; 80 % 1330 and 970 in place; 30 %, 2M x 1536, 300 queries 1181 and 754; a range of half the rows, 1024 queries 1601 and 1576.
+// 700; 10M x 1536, 1024 queries 13270 and, in place, 7130; 80 % 1330 and 970 in place; 30 %, 2M x 1536, 300 queries 1181 and 754; a range of half the rows, 1024 queries 1601 and 1576.
 // Gathers the rows `d_mask` allows where a search of nq queries is faster on them; ix->allowed then has them.  Whether rows
 // lie scattered, which it depends on, is counted on the device and waited for; from the number of allowed rows
 // alone, taken to be scattered, most calls that it cannot pay for are told without.
 int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t nq, size_t k_eff) {
     const size_t n = ix->n, n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (ix->ws_fixed || ix->no_gather || n_allowed == 0 || n_allowed >= n || n >= (size_t(1) << 31)) return TV_OK;
-    const bool in_place = scans_in_place(ix, nq, k_eff, n_allowed);
+    bool in_place = scans_in_place(ix, nq, k_eff, n_allowed);
+    const bool large = in_place && n_blocks * ix->geo.block_bytes() > 0xffffffffull;      // rows of a block may lie too far apart
     if (!in_place && gathered_need(ix, n_allowed) > kGatheredBytes) return TV_OK;
     const double scattered = double(n_blocks) * (1.0 - std::pow(1.0 - double(n_allowed) / double(n), double(tv::kVecBlock)));
     if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs, in_place)) return TV_OK;
@@ -1331,8 +1331,12 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
     if (!have_block(ix, ix->slots, ix->slots_bytes, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
     uint32_t *counts = static_cast<uint32_t *>(ix->slots), *slots = counts + count_bytes / sizeof(uint32_t);
     volatile uint32_t *totals = ix->h_flags;
-    totals[2] = 0;
+    totals[2] = totals[3] = 0;
     TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->d_flags_host, ix->stream));
+    if (large) {
+        TV_HIP(tv::launch_rows_apart(slots, n_allowed, ix->geo.block_bytes(), ix->d_flags_host + 3, ix->stream));
+        TV_HIP(hipStreamSynchronize(ix->stream));
+    }
     // (a wait of a few microseconds, which through the runtime takes ten more; beyond that it is the runtime's)
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (totals[2] == 0 && std::chrono::steady_clock::now() < until) {}
@@ -1340,6 +1344,10 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
     std::atomic_thread_fence(std::memory_order_acquire);
     const size_t total = totals[0], live = totals[1];
     if (total != n_allowed) return TV_OK;      // (the caller's count is not the mask's)
+    if (totals[3] != 0) {
+        in_place = false;
+        if (gathered_need(ix, total) > kGatheredBytes) return TV_OK;
+    }
     if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs, in_place)) return TV_OK;
     if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, total, slots, true};
     else if (const int rc = copy_allowed(ix, slots, total)) return rc;

@@ -121,6 +121,14 @@ __global__ __launch_bounds__(256) void k_gather_rows(const uint4 *codes, const f
     if (c0 == 0u && lane < 32u) out_scales[row] = real ? scales[slot] : 0.0f;
 }
 
+// A scan of rows in place addresses a block's rows with 32 bits from the first one's block.
+__global__ __launch_bounds__(256) void k_rows_apart(const uint32_t *slots, uint32_t n, uint32_t block_bytes, uint32_t *far) {
+    const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 32u;
+    if (i >= n) return;
+    const uint32_t a = slots[i] >> 5, b = slots[min(i + 31u, n - 1u)] >> 5;
+    if (uint64_t(b - a + 1u) * block_bytes > 0xffffffffull) *far = 1u;
+}
+
 // Results of the exact path name gathered rows: back to the index's own.  (What is no row, a place beyond the last one with a score, stays.)
 __global__ __launch_bounds__(256) void k_map_slots(int64_t *idx, size_t count, const uint32_t *slots, uint32_t n) {
     const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
@@ -148,6 +156,12 @@ hipError_t launch_gather_rows(const uint8_t *codes, const float *scales, int nch
     if (n == 0 || nch <= 0 || (n_blocks * runs + 3) / 4 > 0x7fffffffull) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gather_rows, dim3(unsigned((n_blocks * runs + 3) / 4)), dim3(256), 0, s, reinterpret_cast<const uint4 *>(codes), scales, uint32_t(nch),
                        uint32_t(runs), uint32_t(run), slots, uint32_t(n), uint32_t(n_blocks), reinterpret_cast<uint4 *>(out), out_scales);
+    return hipGetLastError();
+}
+
+hipError_t launch_rows_apart(const uint32_t *slots, size_t n, size_t block_bytes, uint32_t *far, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_rows_apart, dim3(unsigned((n + 8191) / 8192)), dim3(256), 0, s, slots, uint32_t(n), uint32_t(block_bytes), far);
     return hipGetLastError();
 }
 

@@ -72,7 +72,7 @@ struct ScanArgs {
     int best_of_block;         // all-queries-per-pass kernel: no floor, per scanned block and query the best allowed slot (kModeBest)
     uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and scanned block the best allowed row's (tv_kernels6.hip)
     uint32_t best_stride;
-    const uint32_t *rows;      // all-queries-per-pass kernel: when given, the slot of each of the n rows to scan, in order; all codes within 4 GiB
+    const uint32_t *rows;      // all-queries-per-pass kernel: when given, the slot of each of the n rows to scan, in order, 32 neighbours of them within 4 GiB
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
 
@@ -209,6 +209,8 @@ size_t select_tmp_keys(size_t k_eff);
 // how many there are and in how many blocks to totals[0], totals[1] (host memory; totals[2] is 1 after them); counts: two words for each of mask_counts(n) workgroups.
 size_t mask_counts(size_t n);
 hipError_t launch_mask_slots(const uint64_t *mask, size_t n, uint32_t *counts, uint32_t *slots, size_t room, uint32_t *totals, hipStream_t s);
+// *far becomes 1 (host memory; cleared by the caller) where the rows of a block of 32 among slots[0 .. n) lie 4 GiB of codes or more apart.
+hipError_t launch_rows_apart(const uint32_t *slots, size_t n, size_t block_bytes, uint32_t *far, hipStream_t s);
 // The rows slots[0 .. n) into blocks of their own, the last one's missing rows zero.
 hipError_t launch_gather_rows(const uint8_t *codes, const float *scales, int nch, const uint32_t *slots, size_t n, uint8_t *out, float *out_scales, hipStream_t s);
 // idx[i] = slots[idx[i]] where idx[i] is below n.

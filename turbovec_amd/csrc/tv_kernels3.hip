@@ -368,9 +368,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                 uint32_t slot = b * 32u + uint32_t(lane & 31), at = lane16;
                 const bool real = slot < a.n;
                 if constexpr (ROWS) {
-                    asm("" : "+s"(p));      // (the chunks' addresses made here: made once, outside the loop, they take a scalar register pair each)
-                    slot = real ? a.rows[slot] : 0u;
-                    at = (slot >> 5) * uint32_t(NCH * 1024) + (uint32_t(h) * 32u + (slot & 31u)) * 16u;
+                    slot = a.rows[real ? slot : b * 32u];
+                    const uint32_t first = uint32_t(__builtin_amdgcn_readfirstlane(int(slot >> 5)));
+                    p += size_t(first) * (NCH * 1024);
+                    at = ((slot >> 5) - first) * uint32_t(NCH * 1024) + (uint32_t(h) * 32u + (slot & 31u)) * 16u;
                 }
                 u32x4 raw[NCH];
                 // with hand-written MFMAs the chunks bound for the accumulation registers come
