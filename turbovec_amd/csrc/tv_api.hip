@@ -773,7 +773,8 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
     }
     if (!repeat && first_level_is_best_words(ix, plan, n_blocks, k_floor, masked)) {
         SamplingSteps steps;
-        const size_t sample = std::min<size_t>({std::max<size_t>(n_blocks * k_floor / floor_rows(ix, plan), 8 * k_floor), size_t(tv::kMaxFloorBlocks), n_blocks / 4});
+        const size_t sample = std::min<size_t>({std::max<size_t>(n_blocks * k_floor / floor_rows(ix, plan), 8 * k_floor), size_t(tv::kMaxFloorBlocks), n_blocks / 4,
+                                                 plan.seg_stride * tv::kSegCap * 2});      // (the words lie in the candidates' place)
         steps.step[steps.count++] = uint32_t((n_blocks + sample - 1) / sample);
         steps.step[steps.count++] = 1;
         steps.best_first = steps.best_words = true;
