@@ -22,6 +22,8 @@ atomic_int fake_device_waits;         /* ... and this many threads are in one */
 atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
 atomic_int fake_cus = 256;            /* compute units the device says it has */
 atomic_int fake_largest_grid;         /* workgroups of the largest launch */
+uint32_t fake_marker;                 /* when not 0: copies to the device are searched for this word ... */
+atomic_int fake_marker_copies;        /* ... and those that hold it counted */
 
 int hipGetDeviceCount(int *n) { *n = 1; return ok; }
 int hipSetDevice(int d) { (void)d; return ok; }
@@ -56,7 +58,17 @@ int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc
 int hipHostFree(void *p) { free(p); return ok; }
 int hipHostGetDevicePointer(void **d, void *h, unsigned flags) { (void)flags; *d = h; return ok; }
 int hipGetSymbolAddress(void **p, const void *symbol) { (void)symbol; static char *at; if (!at) at = calloc(1, 64 << 20); *p = at; return ok; }
-int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) { (void)kind; (void)s; memmove(to, from, n); return ok; }
+int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) {
+    (void)s;
+    if (fake_marker != 0 && kind == 1 /* host to device */) {
+        const uint32_t *w = from;
+        size_t i = 0;
+        while (i < n / 4 && w[i] != fake_marker) ++i;
+        fake_marker_copies += i < n / 4;
+    }
+    memmove(to, from, n);
+    return ok;
+}
 int hipMemsetAsync(void *p, int v, size_t n, void *s) { (void)s; memset(p, v, n); return ok; }
 int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &last; return ok; }
 int hipStreamDestroy(void *s) { (void)s; return ok; }

@@ -105,3 +105,36 @@ ix = index(0, 128)
 ix.add(np.ones((100_000, 128), np.float32))
 assert var("largest_grid").value == 3 * {cus}, var("largest_grid").value
 ''')
+
+
+# 32 MiB in all is the most that is staged in pinned memory: beyond it the snapshot is the call's own
+@pytest.mark.parametrize("rows", [1000, 140_000])
+def test_the_values_that_were_checked_are_the_ones_searched(fake, rows):
+    """A caller's array changes while its call waits for another search to end: what then goes to the device is what was checked."""
+    fake(f'''
+ix = index(64)
+fake_marker = var("marker", C.c_uint32)
+fake_marker.value = 0x7fc0dead           # a NaN
+other = threading.Thread(target=lambda: ix.search(np.ones((1, 64), np.float32), 2))
+var("stream_wait_us").value = 1_000_000
+other.start()
+time.sleep(0.2)                          # it holds the index
+q = np.ones(({rows}, 64), np.float32)
+said = []
+def caller():
+    try:
+        ix.search(q, 1, checked=True)
+        said.append("searched")
+    except T.TurbovecHipError as e:
+        said.append(e.status)
+waiting = threading.Thread(target=caller)
+waiting.start()
+time.sleep(0.4)                          # checked, and waiting for the index
+assert other.is_alive() and waiting.is_alive()
+q.view(np.uint32)[{rows} // 2, 5] = 0x7fc0dead
+other.join()
+var("stream_wait_us").value = 0
+waiting.join()
+assert said == ["searched"], said
+assert var("marker_copies").value == 0
+''')

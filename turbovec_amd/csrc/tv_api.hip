@@ -9,6 +9,7 @@
 #include <cstring>
 #include <cstdlib>
 #include <exception>
+#include <memory>
 #include <new>
 #include <string>
 #include <thread>
@@ -2224,27 +2225,32 @@ static int search_host(tv_index *ix, const float *queries, size_t nq, size_t k, 
     }
     if (need != 0) TV_HIP(hipSetDevice(ix->device));
     PinnedLoan loan(ix, need != 0 ? need : kPinnedLargest + 1);
-    int rc = TV_OK;
-    if (loan.b) {
-        float *q = reinterpret_cast<float *>(loan.b->host);
+    std::unique_ptr<float[]> own;      // where no block was lent, the snapshot of the values to be checked
+    auto snapshot = [&](float *to) -> int {
         std::atomic<bool> bad{false};
         in_parts(values, size_t(1) << 18, [&](size_t lo, size_t hi) {
-            if (copy_checked(q + lo, queries + lo, hi - lo)) bad.store(true, std::memory_order_relaxed);
+            if (copy_checked(to + lo, queries + lo, hi - lo)) bad.store(true, std::memory_order_relaxed);
         });
-        if (bad_index && bad.load()) rc = tv_validate_queries(q, values, int(dim), bad_index);
+        r.q = to;
+        return bad_index && bad.load() ? tv_validate_queries(to, values, int(dim), bad_index) : TV_OK;
+    };
+    int rc = TV_OK;
+    if (loan.b) {
+        rc = snapshot(reinterpret_cast<float *>(loan.b->host));
         if (rc != TV_OK) return rc;
         if (mask_words) {
             std::memcpy(loan.b->host + m_at, mask_words, r.mask_arg * sizeof(uint64_t));
             r.staged_mask = reinterpret_cast<uint64_t *>(loan.b->host + m_at);
         }
-        r.q = q;
         r.out_s = reinterpret_cast<float *>(loan.b->host + s_at);
         r.out_i = reinterpret_cast<int64_t *>(loan.b->host + i_at);
         r.dev_q = reinterpret_cast<const float *>(loan.b->dev);
         r.dev_s = reinterpret_cast<float *>(loan.b->dev + s_at);
         r.dev_i = reinterpret_cast<int64_t *>(loan.b->dev + i_at);
-    } else if (bad_index) {
-        rc = tv_validate_queries(queries, values, int(dim), bad_index);
+    } else if (bad_index && values != 0) {
+        own.reset(new (std::nothrow) float[values]);
+        if (!own) { g_last_error = "no memory for a copy of the queries"; return TV_ERR_BAD_ARGUMENT; }
+        rc = snapshot(own.get());
         if (rc != TV_OK) return rc;
     }
     rc = search_merged(ix, r);
