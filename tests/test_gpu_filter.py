@@ -194,3 +194,37 @@ def test_rows_in_place_of_more_than_4_gib(T):
         assert (after[0] - before[0], after[1] - before[1]) == (1, in_place)
         assert np.array_equal(i, i2) and bits_equal(s, s2)
     ix.close()
+
+
+# the wide kernel's forms of two waves per SIMD and of one; two groups of queries, one in each (and a third without) to repeat
+@pytest.mark.parametrize("dim,nq,k,rows", [(768, 300, 60, [7, 150]), (3072, 140, 13, [139]), (768, 3 * 8192, 60, [5, 8192 + 9])])
+def test_only_the_queries_that_do_not_fit_are_repeated(T, dim, nq, k, rows):
+    """A few queries find their row stored many times over, in blocks that one workgroup of 256 reads: those queries are
+    repeated, once, and the others' results stand."""
+    n = 60_001
+    gen = torch.Generator(device="cuda:0").manual_seed(7)
+    v = torch.randn(n, dim, device="cuda:0", generator=gen)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen)
+    others = torch.ones(nq, dtype=torch.bool, device="cuda:0")
+    others[rows] = False
+    basis = torch.linalg.qr(q[rows].T.cpu())[0].cuda()
+    q[others] -= q[others] @ basis @ basis.T                # at right angles to those rows
+    for j, row in enumerate(rows):
+        for at in range(1000 + 5000 * j, n - 800, 2 * 256 * 32):      # (every second row is allowed)
+            v[at:at + 800] = q[row]
+    torch.cuda.synchronize()
+    ix = T.NativeIndex(dim, 4)
+    ix.add_dev(v.data_ptr(), n)
+    words, allowed = T.pack_mask(np.random.default_rng(5).random(n) < 0.5)
+    mask = torch.from_numpy(words.view(np.int64)).cuda()
+    out = []
+    for path in (GATHERED, MASKED):
+        s, i = torch.zeros(nq, k, device="cuda:0"), torch.zeros(nq, k, dtype=torch.int64, device="cuda:0")
+        torch.cuda.synchronize()
+        ix.set_path(path)
+        ix.search_dev(q.data_ptr(), nq, k, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed)
+        out.append((s.cpu().numpy(), i.cpu().numpy()))
+        if path == GATHERED:
+            assert ix.gathered_searches() == (1, 0) and ix.overflow_redos() == len(rows)
+    assert np.array_equal(out[0][1], out[1][1]) and bits_equal(out[0][0], out[1][0])
+    ix.close()

@@ -624,13 +624,11 @@ size_t sampled_need_worst(const tv_index *ix, size_t nq) {
     return need + group_header_bytes(ix, gq);
 }
 
-constexpr int kNeedsCopy = -1000;     // not a status of the library: a search of rows in place that has to run on a copy of them
 // Full-range search without sampling: per-lane lists with shared thresholds for
 // k <= 32, dense scores + radix select beyond.  Always exact; used for the
 // queries whose candidate buffer overflowed and for very large k.
 int search_robust(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask,
                   float *d_out_scores, int64_t *d_out_idx, bool timed_run) {
-    if (ix->allowed.in_place) return kNeedsCopy;
     const size_t n = ix->rows().n;
     const tv::Geometry &g = ix->geo;
     const int mode = effective_mode(ix);
@@ -736,6 +734,7 @@ bool first_level_is_best_of_block(const tv_index *ix, const SampledPlan &plan, s
 // queries: 1842 us with the ladder, 1884 without; 3M x 512 3-bit, 50 queries, 1 % allowed: 249 and 279).
 bool first_level_is_best_words(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool masked) {
     if (ix->row_ladder_left != 0 || k_floor > size_t(tv::kMaxPickK) || n_blocks <= 16384) return false;
+    if (ix->allowed.in_place) return false;      // (the best-of-block scans read whole blocks)
     if (effective_mode(ix) == TV_SCORE_P) return tv::best_serves(ix->geo.nch) && (plan.wide || plan.nt_batched > 0);
     return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && (!plan.lut_mx || (plan.cq_pad <= 160 && k_floor <= 64 && !masked));
 }
@@ -890,7 +889,6 @@ int take_stamps(tv_index *ix, int launches) {
 }
 int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff, const uint64_t *d_mask, float *d_out_scores,
                   int64_t *d_out_idx, bool timing) {
-    if (ix->allowed.in_place) return kNeedsCopy;
     const tv::Geometry &g = ix->geo;
     const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
     int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
@@ -953,6 +951,8 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
     return TV_OK;
 }
 
+int leave_in_place(tv_index *ix, size_t nq, size_t k_eff);
+
 // The seam: search::search over device-resident inputs and outputs.
 //
 // Sample-then-filter.  Scans run in append mode: every allowed slot whose score
@@ -962,9 +962,13 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
 // scanned, hence a lower bound of the true k-th best, so the full scan appends
 // every member of the true top-k; ties at the floor are kept (>=) and resolved
 // by the same total order as everywhere else.
+//
+// Where ix->allowed has the rows `d_mask` allows, those are searched and the mask is not read -- but for queries
+// whose candidates did not fit in a scan of rows in place, which alone are repeated with it (or on a copy).
 int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
                 size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
     const size_t n = ix->rows().n;
+    const uint64_t *mask = ix->allowed.codes ? nullptr : d_mask;
     size_t k_eff = std::min(std::min(k, n), n_allowed);  // lib.rs:1460, search.rs:3222-3225
     if (out_k_eff) *out_k_eff = k_eff;
     ix->last_scan_ms = 0.0f;
@@ -980,10 +984,10 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     int rc = timing ? ensure_events(ix) : TV_OK;
     if (rc != TV_OK) return rc;
     if (k_eff > size_t(tv::kMaxSampledK) || ix->force_robust)
-        return search_robust(ix, d_queries, nq, k_eff, d_mask, d_out_scores, d_out_idx, timing);
+        return search_robust(ix, d_queries, nq, k_eff, mask, d_out_scores, d_out_idx, timing);
 
-    const size_t n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
-    if (direct_serves(ix, nq, k_eff, n_blocks)) return search_direct(ix, d_queries, nq, k_eff, d_mask, d_out_scores, d_out_idx, timing);
+    size_t n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (direct_serves(ix, nq, k_eff, n_blocks)) return search_direct(ix, d_queries, nq, k_eff, mask, d_out_scores, d_out_idx, timing);
     // sampling levels take the k_floor-th best as the floor: a deeper order statistic is steadier
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     if (ix->row_ladder_left > 0) --ix->row_ladder_left;
@@ -994,8 +998,17 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     rc = ensure_workspace(ix, sampled_need_worst(ix, nq));
     if (rc != TV_OK) return rc;
 
+    // (which rows a scan reads, and through which mask, changes between a group's first passes and its repeated ones)
+    const tv_rows asked = ix->allowed;
+    auto read = [&](const tv_rows &rows) {
+        ix->allowed = rows;
+        mask = rows.codes ? nullptr : d_mask;
+        n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock;
+    };
+    bool left_in_place = false;
     for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
         const size_t gq = std::min(kGroupQueries, nq - g0);
+        if (left_in_place && !ix->allowed.codes) read(asked);      // (a copy, once made, serves the rest of the call)
         Arena head;
         head.base = static_cast<uint8_t *>(ix->ws);
         int *d_raise = head.take<int>(gq);
@@ -1024,9 +1037,8 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const size_t tile_q = plan.tile_q, n_tiles = plan.n_tiles, cq_pad = plan.cq_pad, seg_stride = plan.seg_stride;
             const bool wide = plan.wide;
             const int grid = plan.grid;
-            const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat, d_mask != nullptr);
+            const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat, mask != nullptr);
             const bool best_first = steps.best_first;
-            if (ix->allowed.in_place && (!wide || steps.best_words)) return kNeedsCopy;
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
                 g_last_error = "internal: workspace smaller than the pass it was sized for";
@@ -1074,7 +1086,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 if (lv == 0 && steps.best_words) {
                     tv::ScanArgs a;
                     fill_scan_args(ix, a);
-                    a.mask = d_mask;
+                    a.mask = mask;
                     a.tables = pq.d_tables;
                     a.qscale = pq.d_qscale;
                     a.qbias = pq.d_qbias;
@@ -1101,7 +1113,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                     for (size_t t = 0; t < n_tiles; t += (t < side_by_side ? side_by_side : tiles_per_launch), ++launch_no) {
                         tv::ScanArgs a;
                         fill_scan_args(ix, a);
-                        a.mask = d_mask;
+                        a.mask = mask;
                         a.tables = pq.d_tables + t * (mode_p ? pq.table_bytes_per_tile : tile_q * size_t(g.nch) * 1024);
                         a.qscale = pq.d_qscale + t * tile_q;
                         a.qbias = pq.d_qbias + t * tile_q;
@@ -1178,7 +1190,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
                 const SampledPlan plan = sampled_plan(ix, chunk_at[c + 1] - chunk_at[c]);
-                const size_t n_levels = level_strides(ix, plan, n_blocks, k_floor, false, d_mask != nullptr).size();
+                const size_t n_levels = level_strides(ix, plan, n_blocks, k_floor, false, mask != nullptr).size();
                 for (size_t lv = 1; lv + 1 < n_levels; ++lv)
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
             }
@@ -1204,7 +1216,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         }
         ix->overflow_redos += redo_rows.size() + exact_rows.size();
         if ((redo_rows.size() + exact_rows.size()) * 8 >= gq) {
-            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, k_floor, false, d_mask != nullptr).best_first) {
+            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, k_floor, false, mask != nullptr).best_first) {
                 // from here on, the repeated passes below included -- unless the row-level ladder has just failed too
                 if (ix->floorless_kept_left == 0) ix->row_ladder_left = kRowLadderSearches;
             } else if (ix->row_ladder_left > 0) {
@@ -1215,7 +1227,12 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 ix->floorless_kept_left = kRowLadderSearches;
             }
         }
-        if (ix->allowed.in_place && !(redo_rows.empty() && exact_rows.empty())) return kNeedsCopy;     // (the passes below run on every kernel)
+        if (ix->allowed.in_place && !(redo_rows.empty() && exact_rows.empty())) {     // (the passes below run on every kernel)
+            left_in_place = true;
+            rc = leave_in_place(ix, redo_rows.size() + exact_rows.size(), k_eff);
+            if (rc != TV_OK) return rc;
+            read(ix->allowed);
+        }
         const size_t room = ix->ws_bytes - head.used;
         for (size_t i = 0; i < redo_rows.size();) {
             // rows of one chunk go together: all of them in one pass when the workspace holds that
@@ -1245,12 +1262,13 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             size_t e = i + 1;
             while (e < exact_rows.size() && exact_rows[e] == exact_rows[e - 1] + 1) ++e;     // runs of neighbours go together
             const size_t qa = g0 + exact_rows[i], cnt = e - i;
-            rc = search_robust(ix, d_queries + qa * g.dim, cnt, k_eff, d_mask, d_out_scores + qa * k_eff, d_out_idx + qa * k_eff,
+            rc = search_robust(ix, d_queries + qa * g.dim, cnt, k_eff, mask, d_out_scores + qa * k_eff, d_out_idx + qa * k_eff,
                                false);
             if (rc != TV_OK) return rc;
             i = e;
         }
     }
+    if (asked.in_place && !left_in_place) ++ix->in_place_searches;
     return TV_OK;
 }
 
@@ -1304,13 +1322,21 @@ bool have_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
     g_last_error.clear();
     return false;
 }
-int copy_allowed(tv_index *ix, const uint32_t *slots, size_t total) {
+int copy_allowed(tv_index *ix, const uint32_t *slots, size_t total, size_t live) {
     if (!have_block(ix, ix->gathered, ix->gathered_bytes, gathered_need(ix, total))) return TV_OK;
     uint8_t *codes = static_cast<uint8_t *>(ix->gathered);
     float *scales = reinterpret_cast<float *>(codes + round_up((total + tv::kVecBlock - 1) / tv::kVecBlock * ix->geo.block_bytes(), 256));
     TV_HIP(tv::launch_gather_rows(ix->d_codes, ix->d_scales, ix->geo.nch, slots, total, codes, scales, ix->stream));
-    ix->allowed = tv_rows{codes, scales, total, slots, false};
+    ix->allowed = tv_rows{codes, scales, total, slots, live, false};
     return TV_OK;
+}
+// What queries whose candidates did not fit in a scan of rows in place are repeated on: a copy of the rows where so
+// many queries pay for it, the mask otherwise.
+int leave_in_place(tv_index *ix, size_t nq, size_t k_eff) {
+    const tv_rows was = std::exchange(ix->allowed, tv_rows{});
+    const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (gathered_need(ix, was.n) > kGatheredBytes || !gather_pays(ix, nq, k_eff, double(n_blocks), double(was.live), double(was.n), kCountedNs, false)) return TV_OK;
+    return copy_allowed(ix, was.slots, was.n, was.live);
 }
 // With the mask read during the scan, and gathered, us a search (k = 10): 10 % of the rows allowed at random, 4M x 256 2-bit, 1024 queries 5210 and
 // 680; 4M x 768, 300 queries 1359 and 403; 1M x 768, 40 queries 131 and 105, 1 query 112 and 104; 1 %: 2M x 1536, 1024 queries 1295 and
@@ -1351,8 +1377,8 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
         if (gathered_need(ix, total) > kGatheredBytes) return TV_OK;
     }
     if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs, in_place)) return TV_OK;
-    if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, total, slots, true};
-    else if (const int rc = copy_allowed(ix, slots, total)) return rc;
+    if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, total, slots, live, true};
+    else if (const int rc = copy_allowed(ix, slots, total, live)) return rc;
     if (ix->allowed.codes) ++ix->gathered_searches;
     return TV_OK;
 }
@@ -1363,14 +1389,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         const int rc = gather_allowed(ix, d_mask, n_allowed, nq, std::min(std::min(k, ix->n), n_allowed));
         if (rc != TV_OK) return rc;
     }
-    int rc = search_rows(ix, d_queries, nq, k, ix->allowed.codes ? nullptr : d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
-    if (ix->allowed.in_place && rc == TV_OK) ++ix->in_place_searches;
-    if (rc != kNeedsCopy) return rc;
-    const tv_rows was = ix->allowed;
-    ix->allowed = tv_rows{};
-    rc = gathered_need(ix, was.n) <= kGatheredBytes ? copy_allowed(ix, was.slots, was.n) : TV_OK;
-    if (rc != TV_OK) return rc;
-    return search_rows(ix, d_queries, nq, k, ix->allowed.codes ? nullptr : d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    return search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
 }
 
 // ---- search calls, merged ----------------------------------------------------------------------

@@ -233,6 +233,7 @@ struct tv_rows {
     const float *scales = nullptr;
     size_t n = 0;
     const uint32_t *slots = nullptr;   // the index's slot of each row, when that is not its place
+    size_t live = 0;                   // ... and the index's blocks with such a row
     bool in_place = false;             // ... and codes and scales are the index's own: the rows lie at their slots
 };
 
@@ -287,7 +288,7 @@ struct tv_index {
     void *slots = nullptr, *gathered = nullptr;   // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
     size_t slots_bytes = 0, gathered_bytes = 0;
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
-    tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr, false}; }
+    tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr, 0, false}; }
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
     uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat (before a search: a mask's totals)
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags
@@ -304,7 +305,7 @@ struct tv_index {
     int no_direct = 0;             // test hook: small indexes are sampled like large ones
     int no_gather = 0;             // test hook: filtered searches read the mask as they scan ...
     int force_gather = 0;          // ... or gather their allowed rows whatever their number
-    size_t gathered_searches = 0, in_place_searches = 0;   // searches that ran on the allowed rows alone, and those of them to the end without a copy
+    size_t gathered_searches = 0, in_place_searches = 0;   // searches that ran on the allowed rows alone, and those of them that read all of their queries' rows in place
     size_t overflow_redos = 0;     // queries redone because their candidate buffer overflowed
     // The floorless first level (best row per block) misjudges the floor when a query's neighbours
     // sit together in a few blocks (a clustered corpus in insertion order): after a search in which
