@@ -80,7 +80,9 @@ const char *tv_last_error(void);
  * destroyed -- are kept for the indexes of that device, up to 2 GiB, while any
  * index lives there: handed on to a request they exceed by a quarter at most,
  * given back to the device when an allocation of this library fails and when
- * the device's last index is destroyed.  Other allocators of the process do
+ * the device's last index is destroyed.  When that is not enough, a failing
+ * allocation also takes what the device's indexes keep of filtered searches'
+ * allowed rows (tv_debug_workspace_bytes).  Other allocators of the process do
  * not see them. */
 int tv_index_create(int dim, int bits, int device, tv_index **out);
 int tv_index_destroy(tv_index *ix);
@@ -272,8 +274,10 @@ int tv_debug_sampling_plan(const tv_index *ix, size_t nq, size_t k, uint32_t *st
  * makes searches report such levels (a few hundred bytes more in the flag copy), 0 stops that,
  * negative leaves it as it is; *count (may be NULL) = levels repeated so far while tracking. */
 int tv_debug_level_repeats(tv_index *ix, int track, size_t *count);
-/* Bytes of the index's cached search workspace and of its host-call staging allocation (either
- * pointer may be NULL): both only ever grow, and tv_search_dev_noalloc touches neither. */
+/* Bytes of the index's cached search workspace -- with what its filtered searches keep of their
+ * allowed rows, up to 1.25 GiB and four bytes a row, which is given back when an allocation of this
+ * library fails on that device -- and of its host-call staging allocation (either pointer may be
+ * NULL).  They grow otherwise, and tv_search_dev_noalloc touches neither. */
 int tv_debug_workspace_bytes(const tv_index *ix, size_t *workspace, size_t *staging);
 /* How many filtered searches so far ran on their allowed rows alone, and how many of
  * those read them in place, without a copy. */

@@ -1,5 +1,5 @@
 /* A HIP runtime without a device, for tests of the library's host side: device memory is host memory with a limit,
- * launches do nothing, and the test decides how long a wait takes.  Loaded with RTLD_GLOBAL before the library, whose
+ * launches do nothing (but the one whose counts the host waits for), and the test decides how long a wait takes.  Loaded with RTLD_GLOBAL before the library, whose
  * references then resolve here. */
 #define _GNU_SOURCE
 #include <pthread.h>
@@ -22,6 +22,7 @@ atomic_int fake_device_waits;         /* ... and this many threads are in one */
 atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
 atomic_int fake_cus = 256;            /* compute units the device says it has */
 atomic_int fake_largest_grid;         /* workgroups of the largest launch */
+atomic_int fake_launches;             /* kernels launched */
 uint32_t fake_marker;                 /* when not 0: copies to the device are searched for this word ... */
 atomic_int fake_marker_copies;        /* ... and those that hold it counted */
 
@@ -78,7 +79,30 @@ int hipEventDestroy(void *e) { (void)e; return ok; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0.0f; return ok; }
 int hipFuncSetAttribute(const void *f, int attr, int v) { (void)f; (void)attr; (void)v; return ok; }
-int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) { (void)f; (void)g; (void)b; (void)args; (void)lds; (void)s; return ok; }
+/* tv_filter.hip's list of a mask's rows: its launch counts them and the blocks they lie in */
+static const void *mask_slots;
+void __hipRegisterFunction(void **modules, const void *host, char *device, const char *name, unsigned limit, void *a, void *b, void *c, void *d, int *e) {
+    (void)modules; (void)device; (void)limit; (void)a; (void)b; (void)c; (void)d; (void)e;
+    if (strstr(name, "k_mask_slots")) mask_slots = host;
+}
+int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) {
+    (void)g; (void)b; (void)lds; (void)s;
+    ++fake_launches;
+    if (f == mask_slots) {
+        const uint32_t *mask = *(const uint32_t **)args[0];
+        const uint32_t n = *(uint32_t *)args[1];
+        uint32_t *totals = *(uint32_t **)args[6], rows = 0, live = 0;
+        for (uint32_t w = 0; w * 32 < n; ++w) {
+            const uint32_t x = n - w * 32 < 32 ? mask[w] & ((1u << (n - w * 32)) - 1u) : mask[w];
+            rows += (uint32_t)__builtin_popcount(x);
+            live += x != 0;
+        }
+        totals[0] = rows;
+        totals[1] = live;
+        totals[2] = 1;
+    }
+    return ok;
+}
 int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *s) {
     (void)b; (void)lds; (void)s;
     const int n = (int)(g.x * g.y * g.z);

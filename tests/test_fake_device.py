@@ -138,3 +138,55 @@ waiting.join()
 assert said == ["searched"], said
 assert var("marker_copies").value == 0
 ''')
+
+
+FILTERED = '''
+def filtered(ix, path, nq=4):
+    """A search of half the rows; path 64 gathers them, 32 reads the mask."""
+    words = T.pack_mask(np.arange(len(ix)) % 2 == 1)[0]
+    ix.set_path(path)
+    before = ix.gathered_searches()[0]
+    ix.search(np.ones((nq, 64), np.float32), 3, mask_words=words)
+    return ix.gathered_searches()[0] - before
+'''
+
+
+def test_rows_kept_of_a_filtered_search_give_way(fake):
+    """Rows that fitted beside an index are not refused for the copy its filtered search left behind."""
+    fake(FILTERED + '''
+a, b = index(400_000), index(0)
+assert filtered(a, 32) == 0
+plain, before = a.workspace_bytes()[0], used.value
+assert filtered(a, 64) == 1
+kept = used.value - before
+assert kept >= 6_400_000                 # 200000 rows of 32 bytes
+# b wants 31 MB: 8 are free, the pool holds the 17 of a's first workspace, and the copy its 10
+limit.value = used.value + 8_000_000
+b.append_rows(np.zeros((400_000, 32), np.uint8), np.zeros(400_000, np.float32))
+limit.value = used.value
+assert filtered(a, 64) == 0 and filtered(a, 32) == 0           # the mask is read, as there is no memory for a copy
+assert a.workspace_bytes()[0] < plain + kept
+limit.value = 1 << 34
+assert filtered(a, 64) == 1 and a.workspace_bytes()[0] == plain + kept
+a.close(); b.close()
+assert used.value == 0
+''')
+
+
+def test_a_copy_of_rows_gives_way_to_the_search_it_is_made_for(fake):
+    """Memory for the copy or for the workspace, not for both: the mask is read, as where there is none for the copy."""
+    fake(FILTERED + '''
+a = index(400_000)
+filtered(a, 32)
+grown, before = a.workspace_bytes()[0] - 16_777_216, used.value
+filtered(a, 64)
+kept = used.value - before
+a.close()
+b = index(400_000)
+assert b.workspace_bytes()[0] == 16_777_216 and 2_000_000 < grown < kept
+limit.value = used.value + kept + 1_000_000
+filtered(b, 64)
+assert used.value <= limit.value
+b.close()
+assert used.value == 0
+''')

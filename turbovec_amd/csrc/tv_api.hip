@@ -112,7 +112,8 @@ constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
 // Large blocks that an index gives up (it grew, or went) are kept for the next one, per device: up to
 // kPoolBytes, handed on only to requests they exceed by a quarter at most, and given back when the last
 // index of the device goes or an allocation fails -- any of an index's, so all of them come through
-// device_alloc.  An index built by adds allocates 2.6 times its size on
+// device_alloc.  What filtered searches keep of their allowed rows (tv_spare) goes the same way when the pool was not
+// enough.  An index built by adds allocates 2.6 times its size on
 // the way; fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
 // 1536 rows in four adds: 4 ms a build while cleared memory lasts, 22.8 ms after).
 constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
@@ -121,6 +122,7 @@ struct DevicePool {
     std::mutex giving;     // held while an allocation that failed empties the pool and tries again
     std::vector<std::pair<size_t, void *>> blocks;
     size_t held = 0, indexes = 0;
+    tv_index *newest = nullptr;      // of the device's indexes
     bool takes(size_t bytes) const { return bytes >= kPoolMinBytes && held + bytes <= kPoolBytes && indexes != 0; }   // mu held
     std::vector<std::pair<size_t, void *>> empty() {      // mu held
         held = 0;
@@ -133,6 +135,15 @@ void free_blocks(const std::vector<std::pair<size_t, void *>> &blocks) {
     for (auto &b : blocks) (void)hipFree(b.second);
 }
 
+// A block some index of the device keeps for its filtered searches and is not using, or null.  pool.mu held.
+void *take_spare(DevicePool &pool) {
+    for (tv_index *ix = pool.newest; ix != nullptr; ix = ix->older)
+        for (tv_spare *s : {&ix->gathered, &ix->slots})
+            if (s->p != nullptr && !s->in_use) { s->bytes = 0; return std::exchange(s->p, nullptr); }
+    return nullptr;
+}
+
+thread_local bool g_refused;      // an allocation of this thread's call was refused for good
 // `device` is current.  *got: what the block holds, 0 on failure.
 hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
     DevicePool &pool = g_pool[device];
@@ -161,6 +172,16 @@ hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
         lock.unlock();
         free_blocks(blocks);
         e = hipMalloc(out, bytes);
+        while (e != hipSuccess) {
+            (void)hipGetLastError();
+            lock.lock();
+            void *spare = take_spare(pool);
+            lock.unlock();
+            if (spare == nullptr) break;
+            (void)hipFree(spare);
+            e = hipMalloc(out, bytes);
+        }
+        g_refused |= e != hipSuccess;
     }
     *got = e == hipSuccess ? bytes : 0;     // (callers keep it: a size without a block would pass for one)
     if (e != hipSuccess) (void)hipGetLastError();     // reported by this call, not by a later launch
@@ -1316,15 +1337,20 @@ bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowe
     }
     return true;
 }
-// A block where there is memory for it.  (The search reads the mask as it scans otherwise, as it would have.)
-bool have_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
-    if (ensure_block(ix, p, have, bytes) == TV_OK) return true;
+// Spares in use, or free to be taken again.
+void use_spares(tv_index *ix, bool in_use) {
+    std::lock_guard<std::mutex> lock(g_pool[ix->device].mu);
+    ix->slots.in_use = ix->gathered.in_use = in_use;
+}
+// A block, in use already, where there is memory for it.  (The search reads the mask as it scans otherwise, as it would have.)
+bool have_block(tv_index *ix, tv_spare &s, size_t bytes) {
+    if (ensure_block(ix, s.p, s.bytes, bytes) == TV_OK) return true;
     g_last_error.clear();
     return false;
 }
 int copy_allowed(tv_index *ix, const uint32_t *slots, size_t total, size_t live) {
-    if (!have_block(ix, ix->gathered, ix->gathered_bytes, gathered_need(ix, total))) return TV_OK;
-    uint8_t *codes = static_cast<uint8_t *>(ix->gathered);
+    if (!have_block(ix, ix->gathered, gathered_need(ix, total))) return TV_OK;
+    uint8_t *codes = static_cast<uint8_t *>(ix->gathered.p);
     float *scales = reinterpret_cast<float *>(codes + round_up((total + tv::kVecBlock - 1) / tv::kVecBlock * ix->geo.block_bytes(), 256));
     TV_HIP(tv::launch_gather_rows(ix->d_codes, ix->d_scales, ix->geo.nch, slots, total, codes, scales, ix->stream));
     ix->allowed = tv_rows{codes, scales, total, slots, live, false};
@@ -1356,8 +1382,9 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
     const double scattered = double(n_blocks) * (1.0 - std::pow(1.0 - double(n_allowed) / double(n), double(tv::kVecBlock)));
     if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs, in_place)) return TV_OK;
     const size_t count_bytes = round_up(tv::mask_counts(n) * 2 * sizeof(uint32_t), 256);
-    if (!have_block(ix, ix->slots, ix->slots_bytes, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
-    uint32_t *counts = static_cast<uint32_t *>(ix->slots), *slots = counts + count_bytes / sizeof(uint32_t);
+    use_spares(ix, true);
+    if (!have_block(ix, ix->slots, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
+    uint32_t *counts = static_cast<uint32_t *>(ix->slots.p), *slots = counts + count_bytes / sizeof(uint32_t);
     volatile uint32_t *totals = ix->h_flags;
     totals[2] = totals[3] = 0;
     TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->d_flags_host, ix->stream));
@@ -1384,11 +1411,24 @@ int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_
 }
 int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
                   size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
-    struct Back { tv_index *ix; ~Back() { ix->allowed = tv_rows{}; } } back{ix};
+    struct Back {
+        tv_index *ix;
+        void give() {
+            ix->allowed = tv_rows{};
+            if (ix->slots.in_use) use_spares(ix, false);
+        }
+        ~Back() { give(); }
+    } back{ix};
     if (d_mask && k != 0 && nq != 0) {
         const int rc = gather_allowed(ix, d_mask, n_allowed, nq, std::min(std::min(k, ix->n), n_allowed));
         if (rc != TV_OK) return rc;
     }
+    g_refused = false;
+    const int rc = search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    if (rc == TV_OK || !g_refused || !ix->slots.in_use) return rc;
+    // no memory for the search beside its list and copy of rows, which are given up for it
+    TV_HIP(hipStreamSynchronize(ix->stream));
+    back.give();
     return search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
 }
 
@@ -1651,8 +1691,12 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
     if (!ix) return TV_ERR_BAD_ARGUMENT;
     ix->device = device;
     {
-        std::lock_guard<std::mutex> lock(g_pool[device].mu);
-        ++g_pool[device].indexes;
+        DevicePool &pool = g_pool[device];
+        std::lock_guard<std::mutex> lock(pool.mu);
+        ++pool.indexes;
+        ix->older = pool.newest;
+        if (ix->older) ix->older->newer = ix;
+        pool.newest = ix;
     }
     ix->geo.dim = dim;
     ix->geo.bits = bits;
@@ -1722,16 +1766,19 @@ int tv_index_destroy(tv_index *ix) {
     if (ix->stream) (void)hipStreamSynchronize(ix->stream);
     void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
                     ix->d_tau_open};
+    use_spares(ix, true);      // (from here on they are freed below)
     (void)device_free(ix->device, ix->d_codes, ix->codes_bytes);
     (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
     (void)device_free(ix->device, ix->ws, ix->ws_bytes);
     (void)device_free(ix->device, ix->io, ix->io_bytes);
-    (void)device_free(ix->device, ix->slots, ix->slots_bytes);
-    (void)device_free(ix->device, ix->gathered, ix->gathered_bytes);
+    (void)device_free(ix->device, ix->slots.p, ix->slots.bytes);
+    (void)device_free(ix->device, ix->gathered.p, ix->gathered.bytes);
     for (void *p : ptrs) if (p) (void)hipFree(p);
     {
         DevicePool &pool = g_pool[ix->device];
         std::unique_lock<std::mutex> lock(pool.mu);
+        (ix->newer ? ix->newer->older : pool.newest) = ix->older;
+        if (ix->older) ix->older->newer = ix->newer;
         const auto blocks = --pool.indexes == 0 ? pool.empty() : decltype(pool.blocks){};
         lock.unlock();
         free_blocks(blocks);
@@ -2597,7 +2644,8 @@ int tv_debug_workspace_bytes(const tv_index *cix, size_t *workspace, size_t *sta
     tv_index *ix = const_cast<tv_index *>(cix);
     if (!ix) return TV_ERR_BAD_ARGUMENT;
     std::lock_guard<std::mutex> lock(ix->mu);
-    if (workspace) *workspace = ix->ws_bytes;
+    std::lock_guard<std::mutex> kept(g_pool[ix->device].mu);
+    if (workspace) *workspace = ix->ws_bytes + ix->slots.bytes + ix->gathered.bytes;
     if (staging) *staging = ix->io_bytes;
     return TV_OK;
 }

@@ -237,6 +237,14 @@ struct tv_rows {
     bool in_place = false;             // ... and codes and scales are the index's own: the rows lie at their slots
 };
 
+// Device memory that an index keeps between searches and does without where an allocation of the device needs it (tv_api.hip:
+// device_alloc takes it then, unless a search is using it).
+struct tv_spare {
+    void *p = nullptr;
+    size_t bytes = 0;
+    bool in_use = false;
+};
+
 // The opaque handle of the C ABI.
 struct tv_index {
     tv::Geometry geo;
@@ -285,8 +293,8 @@ struct tv_index {
     static constexpr int kPinned = 8;
     std::mutex pinned_mu;
     tv_pinned pinned[kPinned];     // allocated on first use, at most kPinnedBytes in all (tv_api.hip), freed with the index
-    void *slots = nullptr, *gathered = nullptr;   // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
-    size_t slots_bytes = 0, gathered_bytes = 0;
+    tv_spare slots, gathered;      // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
+    tv_index *older = nullptr, *newer = nullptr;   // the device's indexes, linked (guarded as their pool of blocks is)
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
     tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr, 0, false}; }
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
