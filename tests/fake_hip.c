@@ -23,6 +23,8 @@ atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
 atomic_int fake_cus = 256;            /* compute units the device says it has */
 atomic_int fake_largest_grid;         /* workgroups of the largest launch */
 atomic_int fake_launches;             /* kernels launched */
+atomic_int fake_pinned_blocks;        /* blocks of pinned memory of 64 KiB and more allocated so far ... */
+atomic_size_t fake_pinned, fake_pinned_peak;      /* ... and their bytes now, and at most */
 uint32_t fake_marker;                 /* when not 0: copies to the device are searched for this word ... */
 atomic_int fake_marker_copies;        /* ... and those that hold it counted */
 
@@ -55,8 +57,21 @@ int hipDeviceSynchronize(void) {
 }
 int hipMalloc(void **p, size_t n) { return take(p, n); }
 int hipFree(void *p) { if (p) hipDeviceSynchronize(); return give(p); }
-int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(1, n); return ok; }
-int hipHostFree(void *p) { free(p); return ok; }
+int hipHostMalloc(void **p, size_t n, unsigned flags) {
+    (void)flags;
+    const size_t counted = n >= 65536 ? n : 0;
+    size_t *at = calloc(1, n + 256);
+    at[0] = counted;
+    *p = (char *)at + 256;
+    fake_pinned_blocks += counted != 0;
+    const size_t now = atomic_fetch_add(&fake_pinned, counted) + counted;
+    for (size_t peak = fake_pinned_peak; now > peak && !atomic_compare_exchange_weak(&fake_pinned_peak, &peak, now);) {}
+    return ok;
+}
+int hipHostFree(void *p) {
+    if (p) { size_t *at = (size_t *)((char *)p - 256); fake_pinned -= at[0]; free(at); }
+    return ok;
+}
 int hipHostGetDevicePointer(void **d, void *h, unsigned flags) { (void)flags; *d = h; return ok; }
 int hipGetSymbolAddress(void **p, const void *symbol) { (void)symbol; static char *at; if (!at) at = calloc(1, 64 << 20); *p = at; return ok; }
 int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) {

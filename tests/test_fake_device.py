@@ -190,3 +190,49 @@ assert used.value <= limit.value
 b.close()
 assert used.value == 0
 ''')
+
+
+def test_pinned_memory_is_shared_by_the_devices_indexes(fake):
+    """A new index's first calls on host arrays find what another one's calls had allocated; it all goes with the last index."""
+    fake('''
+blocks, pinned = var("pinned_blocks"), var("pinned", C.c_size_t)
+a = index(64)
+for nq in (1, 1000):
+    a.search(np.ones((nq, 64), np.float32), 3)
+before = blocks.value
+assert before == 2
+b = index(64)
+a.close()
+for nq in (1000, 1):
+    b.search(np.ones((nq, 64), np.float32), 3)
+assert blocks.value == before
+b.close()
+assert pinned.value == 0
+''')
+
+
+def test_pinned_memory_has_a_limit(fake):
+    """256 MiB on a device, whatever its indexes' calls want at once; what is idle makes room, and a call that gets none does without."""
+    fake('''
+pinned, peak = var("pinned", C.c_size_t), var("pinned_peak", C.c_size_t)
+made = [index(64) for _ in range(9)]
+rows = 1
+while rows <= 32768:                     # blocks of 64 KiB to 16 MiB, idle
+    made[0].search(np.ones((rows, 64), np.float32), 1)
+    rows *= 2
+idle = pinned.value
+assert idle >= 16 << 20
+q = np.ones((100_000, 64), np.float32)   # 32 MiB each
+var("stream_wait_us").value = 100_000
+started = threading.Barrier(len(made))
+def call(ix):
+    started.wait()
+    ix.search(q, 1, checked=True)
+calls = [threading.Thread(target=call, args=(ix,)) for ix in made]
+for t in calls: t.start()
+for t in calls: t.join()
+var("stream_wait_us").value = 0
+assert 128 << 20 < peak.value <= 256 << 20, peak.value
+for ix in made: ix.close()
+assert pinned.value == 0 and used.value == 0
+''')

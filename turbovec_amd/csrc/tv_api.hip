@@ -123,6 +123,8 @@ struct DevicePool {
     std::vector<std::pair<size_t, void *>> blocks;
     size_t held = 0, indexes = 0;
     tv_index *newest = nullptr;      // of the device's indexes
+    static constexpr int kPinned = 64;
+    tv_pinned pinned[kPinned];       // host memory: pinned_take
     bool takes(size_t bytes) const { return bytes >= kPoolMinBytes && held + bytes <= kPoolBytes && indexes != 0; }   // mu held
     std::vector<std::pair<size_t, void *>> empty() {      // mu held
         held = 0;
@@ -232,49 +234,66 @@ int ensure_io(tv_index *ix, size_t bytes) { return ensure_block(ix, ix->io, ix->
 
 // ---- host arrays ---------------------------------------------------------------------------------
 // A copy from or to pageable memory is staged by the runtime, on one thread and with a wait of its own: 500 KB 30 us, 614 MB
-// 20 to 39 ms.  Here calls on host arrays pass through pinned blocks that belong to the index: queries are copied in
+// 20 to 39 ms.  Here calls on host arrays pass through pinned blocks that the device's indexes share: queries are copied in
 // on the calling thread -- the snapshot of them that the search then reads -- and read by the device where they lie,
 // results are written there by the last kernel; rows to add go through in pieces, several threads filling.  Through the Python
 // surface, before and now: one query over 100K x 128 73 us and 37, 1000 queries 138 and 101, 1024 of 3072 dimensions 2.41 ms and 1.22; 100K
 // x 1536 rows to an image 37.9 ms and 21.5.
-constexpr size_t kPinnedBytes = size_t(128) << 20, kPinnedLargest = size_t(32) << 20;
+constexpr size_t kPinnedBytes = size_t(256) << 20, kPinnedLargest = size_t(32) << 20;
 constexpr size_t kReadInPlace = size_t(1) << 20;      // larger sets of queries are copied to the device first, by the copy engine
 
-// A block of at least `bytes`, or null: none to spare, or none to be had (the caller then does without).  The index's device is current.
-tv_pinned *pinned_take(tv_index *ix, size_t bytes) {
+// A block of at least `bytes`, or null: none to spare, or none to be had (the caller then does without).  They are allocated on
+// first use, at most kPinnedBytes of them, and freed with the device's last index; `device` is current.  (Pinning is slow: a
+// new index's first search of 1000 queries of 128 dimensions 141 us with blocks of its own and 115 with another index's, of one query 70 and 44;
+// with no other index it is 170, and 142 without pinned blocks.)
+tv_pinned *pinned_take(int device, size_t bytes) {
     if (bytes > kPinnedLargest) return nullptr;
     size_t want = size_t(64) << 10;
     while (want < bytes) want *= 2;
-    std::lock_guard<std::mutex> lock(ix->pinned_mu);
-    size_t total = 0;
-    tv_pinned *fits = nullptr, *spare = nullptr;
-    for (tv_pinned &b : ix->pinned) {
-        total += b.bytes;
+    DevicePool &pool = g_pool[device];
+    std::unique_lock<std::mutex> lock(pool.mu);
+    size_t lent = 0, idle = 0;
+    tv_pinned *fits = nullptr, *place = nullptr;
+    for (tv_pinned &b : pool.pinned) {
+        (b.lent ? lent : idle) += b.bytes;
         if (b.lent) continue;
         if (b.bytes >= want && (!fits || b.bytes < fits->bytes)) fits = &b;
-        if (b.bytes < want && (!spare || b.bytes < spare->bytes)) spare = &b;
+        if (b.bytes == 0 && !place) place = &b;
     }
     if (fits) { fits->lent = true; return fits; }
-    if (!spare || total - spare->bytes + want > kPinnedBytes) return nullptr;
-    if (spare->host) (void)hipHostFree(spare->host);
-    *spare = tv_pinned{};
+    if (lent + want > kPinnedBytes) return nullptr;
+    uint8_t *given_up[DevicePool::kPinned];      // of the idle blocks, all smaller, the largest first
+    int n_given_up = 0;
+    while (!place || lent + idle + want > kPinnedBytes) {
+        tv_pinned *largest = nullptr;
+        for (tv_pinned &b : pool.pinned)
+            if (!b.lent && b.bytes != 0 && (!largest || b.bytes > largest->bytes)) largest = &b;
+        if (!largest) return nullptr;     // (every block is lent)
+        idle -= largest->bytes;
+        given_up[n_given_up++] = largest->host;
+        *largest = tv_pinned{};
+        place = largest;
+    }
+    place->bytes = want;      // (counted, and nobody else's, while it is allocated)
+    place->lent = true;
+    lock.unlock();
+    for (int i = 0; i < n_given_up; ++i) (void)hipHostFree(given_up[i]);
     void *host = nullptr, *dev = nullptr;
-    if (hipHostMalloc(&host, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    if (hipHostGetDevicePointer(&dev, host, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(host); return nullptr; }
-    spare->host = static_cast<uint8_t *>(host);
-    spare->dev = static_cast<uint8_t *>(dev);
-    spare->bytes = want;
-    spare->lent = true;
-    return spare;
+    bool got = hipHostMalloc(&host, want, hipHostMallocMapped) == hipSuccess;
+    if (got && hipHostGetDevicePointer(&dev, host, 0) != hipSuccess) { (void)hipHostFree(host); got = false; }
+    if (!got) (void)hipGetLastError();
+    lock.lock();
+    *place = got ? tv_pinned{static_cast<uint8_t *>(host), static_cast<uint8_t *>(dev), want, true} : tv_pinned{};
+    return got ? place : nullptr;
 }
 struct PinnedLoan {      // given back when it goes out of scope; whoever reads or writes the block has finished by then
-    tv_index *ix;
+    int device;
     tv_pinned *b;
-    PinnedLoan(tv_index *ix_, size_t bytes) : ix(ix_), b(pinned_take(ix_, bytes)) {}
+    PinnedLoan(int device_, size_t bytes) : device(device_), b(pinned_take(device_, bytes)) {}
     PinnedLoan(const PinnedLoan &) = delete;
     ~PinnedLoan() {
         if (!b) return;
-        std::lock_guard<std::mutex> lock(ix->pinned_mu);
+        std::lock_guard<std::mutex> lock(g_pool[device].mu);
         b->lent = false;
     }
 };
@@ -1779,12 +1798,17 @@ int tv_index_destroy(tv_index *ix) {
         std::unique_lock<std::mutex> lock(pool.mu);
         (ix->newer ? ix->newer->older : pool.newest) = ix->older;
         if (ix->older) ix->older->newer = ix->newer;
-        const auto blocks = --pool.indexes == 0 ? pool.empty() : decltype(pool.blocks){};
+        const bool last = --pool.indexes == 0;
+        const auto blocks = last ? pool.empty() : decltype(pool.blocks){};
+        uint8_t *pinned[DevicePool::kPinned];
+        int n_pinned = 0;
+        for (tv_pinned &b : pool.pinned)
+            if (last && !b.lent && b.host) { pinned[n_pinned++] = b.host; b = tv_pinned{}; }
         lock.unlock();
         free_blocks(blocks);
+        for (int i = 0; i < n_pinned; ++i) (void)hipHostFree(pinned[i]);
     }
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
-    for (tv_pinned &b : ix->pinned) if (b.host) (void)hipHostFree(b.host);
     if (ix->events_ready)
         for (int i = 0; i < tv::kTimedLaunches; ++i) {
             (void)hipEventDestroy(ix->ev_start[i]);
@@ -1964,7 +1988,7 @@ static int stage_rows(tv_index *ix, const float *rows, size_t values, float *d_r
     constexpr size_t kPiece = (size_t(4) << 20) / sizeof(float), kThreads = 4;
     *bad = false;
     const size_t pieces = (values + kPiece - 1) / kPiece, threads = std::min<size_t>(kThreads, pieces);
-    PinnedLoan loan(ix, threads * std::min(kPiece, values) * sizeof(float));
+    PinnedLoan loan(ix->device, threads * std::min(kPiece, values) * sizeof(float));
     if (!loan.b) {
         *bad = tv_validate_queries(rows, values, 1, nullptr) != TV_OK;
         if (!*bad) TV_HIP(hipMemcpyAsync(d_rows, rows, values * sizeof(float), hipMemcpyHostToDevice, ix->stream));
@@ -1994,7 +2018,7 @@ static int stage_rows(tv_index *ix, const float *rows, size_t values, float *d_r
 static int fetch_bytes(tv_index *ix, const uint8_t *d_from, uint8_t *to, size_t bytes) {
     constexpr size_t kPiece = size_t(2) << 20;
     const size_t pieces = (bytes + kPiece - 1) / kPiece, threads = std::min(kMaxParts, pieces);
-    PinnedLoan loan(ix, threads * std::min(kPiece, bytes));
+    PinnedLoan loan(ix->device, threads * std::min(kPiece, bytes));
     if (bytes == 0) return TV_OK;
     if (!loan.b) {
         touch_pages(to, bytes);
@@ -2290,7 +2314,7 @@ static int search_host(tv_index *ix, const float *queries, size_t nq, size_t k, 
         need = m_at + r.mask_arg * sizeof(uint64_t);
     }
     if (need != 0) TV_HIP(hipSetDevice(ix->device));
-    PinnedLoan loan(ix, need != 0 ? need : kPinnedLargest + 1);
+    PinnedLoan loan(ix->device, need != 0 ? need : kPinnedLargest + 1);
     std::unique_ptr<float[]> own;      // where no block was lent, the snapshot of the values to be checked
     auto snapshot = [&](float *to) -> int {
         std::atomic<bool> bad{false};

@@ -220,7 +220,7 @@ hipError_t launch_map_slots(int64_t *idx, size_t count, const uint32_t *slots, s
 
 struct tv_request;   // a search call waiting for the index (tv_api.hip)
 
-// Pinned host memory an index lends its host-array calls, one block at a time to a call.
+// Pinned host memory that the indexes of a device share: one block at a time is lent to a call on host arrays.
 struct tv_pinned {
     uint8_t *host = nullptr, *dev = nullptr;   // the same bytes, as the host and as the device address them
     size_t bytes = 0;
@@ -290,9 +290,6 @@ struct tv_index {
     size_t io_bytes = 0;
     size_t ws_bytes = 0;
     bool ws_fixed = false;         // ws is a lent buffer of fixed size (tv_search_dev_noalloc): never reallocated
-    static constexpr int kPinned = 8;
-    std::mutex pinned_mu;
-    tv_pinned pinned[kPinned];     // allocated on first use, at most kPinnedBytes in all (tv_api.hip), freed with the index
     tv_spare slots, gathered;      // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
     tv_index *older = nullptr, *newer = nullptr;   // the device's indexes, linked (guarded as their pool of blocks is)
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
