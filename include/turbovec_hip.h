@@ -115,7 +115,9 @@ int tv_index_append_rows(tv_index *ix, const uint8_t *rows, const float *scales,
  * bit-identical to the CPU encoder's.  Replaces the encode half of
  * TurboQuantIndex::add (lib.rs:738-966 -> encode.rs:1418-1476, :560-664,
  * :900-932).  Values must be finite with |x| < 1e16 (encode.rs:76-83):
- * TV_ERR_INVALID_QUERY_VALUE otherwise, and nothing is added. */
+ * TV_ERR_INVALID_QUERY_VALUE otherwise, and nothing is added: tv_index_len counts
+ * the rows once all of them have passed.  The index's buffers may have grown all
+ * the same (tv_index_device_ptrs). */
 int tv_index_add(tv_index *ix, const float *vectors, size_t n_new);
 /* Fit the TQ+ per-coordinate pair from n >= 2 sample rows and commit it
  * (TurboQuantIndex::calibrate, lib.rs:2599; fit encode.rs:737-857): the sample is

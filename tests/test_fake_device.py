@@ -236,3 +236,33 @@ assert 128 << 20 < peak.value <= 256 << 20, peak.value
 for ix in made: ix.close()
 assert pinned.value == 0 and used.value == 0
 ''')
+
+
+@pytest.mark.parametrize("bad", [True, False])
+def test_rows_count_once_all_of_them_have_passed(fake, bad):
+    """An add of several slices shows none of its rows before the last one is there, and none at all if it refuses one."""
+    fake(f'''
+ix = index(64)
+v = np.ones((1_050_000, 64), np.float32)           # a slice is 256 MiB: 1048576 rows
+if {bad}: v[-1, 3] = np.nan
+var("stream_wait_us").value = 1000
+said = []
+def add():
+    try:
+        ix.add(v)
+        said.append("added")
+    except T.TurbovecHipError as e:
+        said.append(e.status)
+adding = threading.Thread(target=add)
+adding.start()
+seen = set()
+while adding.is_alive():
+    seen.add(len(ix))
+    time.sleep(1e-4)
+var("stream_wait_us").value = 0
+assert said == ([T.ERR_INVALID_QUERY_VALUE] if {bad} else ["added"]), said
+end = 64 if {bad} else 64 + len(v)
+assert 64 in seen and seen <= {{64, end}}, seen
+assert len(ix) == end
+ix.close()
+''')

@@ -1953,20 +1953,20 @@ int tv_index_append_rows(tv_index *ix, const uint8_t *rows, const float *scales,
     return TV_OK;
 }
 
-// lib.rs add -> encode.rs:1418-1476 on the device, then append_lanes (pack.rs:211-233).
-static int add_device_rows(tv_index *ix, const float *d_vectors, size_t n_new) {
+// lib.rs add -> encode.rs:1418-1476 on the device, then append_lanes (pack.rs:211-233).  The rows go to slots `at` and on, which
+// the caller counts among the index's.
+static int encode_rows(tv_index *ix, const float *d_vectors, size_t n_new, size_t at) {
     const tv::Geometry &g = ix->geo;
     const bool cal = !ix->tq_shift.empty();
     const size_t slice = size_t(1) << 20;
     for (size_t r0 = 0; r0 < n_new; r0 += slice) {
         const size_t nr = std::min(slice, n_new - r0);
-        TV_HIP(tv::launch_encode(d_vectors + r0 * size_t(g.dim), nr, ix->n + r0, ix->d_signs, ix->d_perms,
+        TV_HIP(tv::launch_encode(d_vectors + r0 * size_t(g.dim), nr, at + r0, ix->d_signs, ix->d_perms,
                                  ix->packed_ok ? ix->d_packed : nullptr, cal ? ix->d_tq_shift : nullptr, cal ? ix->d_tq_scale : nullptr,
                                  ix->cb.centroids.data(), ix->cb.boundaries.data(), g, ix->rot.block,
                                  ix->rot.inv_sqrt_block, ix->d_codes, ix->d_scales, nullptr, ix->device, ix->stream));
     }
     TV_HIP(hipStreamSynchronize(ix->stream));
-    ix->n += n_new;
     return TV_OK;
 }
 
@@ -1978,7 +1978,9 @@ int tv_index_add_dev(tv_index *ix, const float *d_vectors, size_t n_new) {
     if (ix->n + n_new >= (size_t(1) << 31)) return TV_ERR_BAD_ARGUMENT;
     int rc = ensure_capacity(ix, ix->n + n_new);
     if (rc != TV_OK) return rc;
-    return add_device_rows(ix, d_vectors, n_new);
+    rc = encode_rows(ix, d_vectors, n_new, ix->n);
+    if (rc == TV_OK) ix->n += n_new;
+    return rc;
 }
 
 // Rows on their way to the device, checked as they pass through pinned memory, a few megabytes at a time: each of up
@@ -2043,13 +2045,12 @@ static int fetch_bytes(tv_index *ix, const uint8_t *d_from, uint8_t *to, size_t 
     return TV_OK;
 }
 
-// Rows [first, ix->n) are taken back: their bytes and scales are zero again, as if they had never been added.
-static int drop_rows(tv_index *ix, size_t first) {
+// Slots from the index's last row up to `end` are cleared, as if no rows had ever gone there.
+static int clear_slots(tv_index *ix, size_t end) {
     const tv::Geometry &g = ix->geo;
-    const size_t end = ix->n, block = (first + tv::kVecBlock - 1) / tv::kVecBlock, end_block = (end + tv::kVecBlock - 1) / tv::kVecBlock;
-    if (end == first) return TV_OK;
+    const size_t first = ix->n, block = (first + tv::kVecBlock - 1) / tv::kVecBlock, end_block = (end + tv::kVecBlock - 1) / tv::kVecBlock;
+    if (end <= first) return TV_OK;
     const size_t lanes = std::min(end, block * tv::kVecBlock) - first;      // in a block that holds earlier rows
-    ix->n = first;
     if (lanes) {
         int rc = ensure_workspace(ix, lanes * size_t(g.G) + 256);
         if (rc != TV_OK) return rc;
@@ -2071,24 +2072,27 @@ int tv_index_add(tv_index *ix, const float *vectors, size_t n_new) {
     if (ix->n + n_new >= (size_t(1) << 31)) return TV_ERR_BAD_ARGUMENT;
     int rc = ensure_capacity(ix, ix->n + n_new);
     if (rc != TV_OK) return rc;
-    const size_t before = ix->n, slice = std::max<size_t>(1, (size_t(256) << 20) / (dim * sizeof(float)));
+    const size_t slice = std::max<size_t>(1, (size_t(256) << 20) / (dim * sizeof(float)));
     rc = ensure_workspace(ix, std::min(n_new, slice) * dim * sizeof(float) + 256);
     if (rc != TV_OK) return rc;
     for (size_t r0 = 0; r0 < n_new; r0 += slice) {
         const size_t nr = std::min(slice, n_new - r0);
         bool bad = false;
         rc = stage_rows(ix, vectors + r0 * dim, nr * dim, static_cast<float *>(ix->ws), &bad);
-        if (rc == TV_OK && !bad) rc = add_device_rows(ix, static_cast<const float *>(ix->ws), nr);
+        if (rc == TV_OK && !bad) rc = encode_rows(ix, static_cast<const float *>(ix->ws), nr, ix->n + r0);
+        if (rc != TV_OK || bad) {      // nothing is added: the index's rows are counted once the last slice is there
+            const int cleared = clear_slots(ix, ix->n + r0 + (bad ? 0 : nr));
+            if (rc == TV_OK) rc = cleared;
+        }
         if (rc != TV_OK) return rc;
-        if (bad) {      // the same predicate as for queries (encode.rs:76-83), and nothing is added
-            rc = drop_rows(ix, before);
-            if (rc != TV_OK) return rc;
+        if (bad) {      // the same predicate as for queries (encode.rs:76-83)
             size_t at = r0 * dim;
             (void)tv_validate_queries(vectors, n_new * dim, int(dim), &at);
             g_last_error = "vector " + std::to_string(at / dim) + " holds a non-finite or too large value";
             return TV_ERR_INVALID_QUERY_VALUE;
         }
     }
+    ix->n += n_new;
     return TV_OK;
 }
 

@@ -164,7 +164,7 @@ class TurboQuantIndex:
             return
         with self._lock:
             try:
-                self._ix.add(v)                         # checks every value before it changes anything
+                self._ix.add(v)                         # adds all rows, or none
             except T.TurbovecHipError as e:
                 if e.status == T.ERR_INVALID_QUERY_VALUE:
                     _check_values("vectors", v, "vector")
