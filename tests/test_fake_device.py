@@ -266,3 +266,20 @@ assert 64 in seen and seen <= {{64, end}}, seen
 assert len(ix) == end
 ix.close()
 ''')
+
+
+def test_a_mask_of_another_length_is_refused_unread(fake):
+    """The words a call says there are beyond the index's rows are not looked at."""
+    fake('''
+import mmap
+ix = index(64)
+page = mmap.mmap(-1, 2 * mmap.PAGESIZE)
+at = C.addressof(C.c_char.from_buffer(page))
+assert C.CDLL(None).mprotect(C.c_void_p(at + mmap.PAGESIZE), C.c_size_t(mmap.PAGESIZE), 0) == 0
+q, s, i = np.ones((2, 64), np.float32), np.zeros(2, np.float32), np.zeros(2, np.int64)
+mask = at + mmap.PAGESIZE - 8            # one word before memory nobody may read
+ke, bad = C.c_size_t(0), C.c_size_t(0)
+for words in (2, 300_000, 1 << 62):
+    assert T.lib().tv_search(ix.h, T.ptr(q), 2, 1, mask, words, T.ptr(s), T.ptr(i), C.byref(ke)) == T.ERR_MASK_LENGTH_MISMATCH
+    assert T.lib().tv_search_checked(ix.h, T.ptr(q), 2, 1, mask, words, T.ptr(s), T.ptr(i), C.byref(ke), C.byref(bad)) == T.ERR_MASK_LENGTH_MISMATCH
+''')

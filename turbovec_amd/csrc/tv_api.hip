@@ -2311,7 +2311,9 @@ static int search_host(tv_index *ix, const float *queries, size_t nq, size_t k, 
     r.mask = mask_words; r.mask_arg = mask_words ? n_mask_words : 0;
     r.out_s = out_scores; r.out_i = out_indices;
     size_t need = 0, s_at = 0, i_at = 0, m_at = 0;
-    if (nq != 0 && k != 0 && nq <= (kPinnedLargest >> 2) && k <= (kPinnedLargest >> 2)) {      // (no product below overflows)
+    // (no product below overflows; a mask of another length is refused when the call is served, and not read)
+    if (nq != 0 && k != 0 && nq <= (kPinnedLargest >> 2) && k <= (kPinnedLargest >> 2) &&
+        (!mask_words || n_mask_words == (tv_index_len(ix) + 63) / 64)) {
         s_at = round_up(values * sizeof(float), 256);
         i_at = s_at + round_up(nq * k * sizeof(float), 256);
         m_at = i_at + round_up(nq * k * sizeof(int64_t), 256);
