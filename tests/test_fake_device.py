@@ -283,3 +283,28 @@ for words in (2, 300_000, 1 << 62):
     assert T.lib().tv_search(ix.h, T.ptr(q), 2, 1, mask, words, T.ptr(s), T.ptr(i), C.byref(ke)) == T.ERR_MASK_LENGTH_MISMATCH
     assert T.lib().tv_search_checked(ix.h, T.ptr(q), 2, 1, mask, words, T.ptr(s), T.ptr(i), C.byref(ke), C.byref(bad)) == T.ERR_MASK_LENGTH_MISMATCH
 ''')
+
+
+def test_a_mask_that_changed_is_another_mask(fake):
+    """A call waits with what its mask array held; one made after the array changed is searched with what it holds then."""
+    fake('''
+ix = index(64 * 64)
+words = np.full(64, 1, np.uint64)
+q, bad = np.ones((2, 64), np.float32), []
+def search(mask):
+    ke, s, i = C.c_size_t(0), np.zeros(2, np.float32), np.zeros(2, np.int64)
+    bad.append(T.lib().tv_search(ix.h, T.ptr(q), 2, 1, mask, 64, T.ptr(s), T.ptr(i), C.byref(ke)))
+calls = [threading.Thread(target=search, args=(m,)) for m in (None, T.ptr(words), T.ptr(words))]
+var("stream_wait_us").value = 300_000
+calls[0].start()
+time.sleep(0.1)                          # it holds the index
+calls[1].start()
+time.sleep(0.1)                          # waits
+marker = var("marker", C.c_uint32)
+marker.value = 0x7fc0dead
+words.view(np.uint32)[7] = marker.value
+calls[2].start()
+for t in calls: t.join()
+assert bad == [T.OK] * 3, bad
+assert ix.merged_calls() == 0 and var("marker_copies").value == 1
+''')

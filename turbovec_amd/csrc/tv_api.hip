@@ -1589,7 +1589,10 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
 }
 
 bool compatible(const tv_request &a, const tv_request &b) {
-    return a.host == b.host && a.k == b.k && a.mask == b.mask && a.mask_arg == b.mask_arg;
+    if (a.host != b.host || a.k != b.k || a.mask != b.mask || a.mask_arg != b.mask_arg) return false;
+    // (one array, but each call searches what was in it when it was made)
+    const uint64_t *x = a.staged_mask ? a.staged_mask : a.mask, *y = b.staged_mask ? b.staged_mask : b.mask;
+    return x == y || std::memcmp(x, y, a.mask_arg * sizeof(uint64_t)) == 0;
 }
 
 // How long a caller that is about to serve waits for the callers of the batch before to come back
