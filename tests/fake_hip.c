@@ -94,27 +94,29 @@ int hipEventDestroy(void *e) { (void)e; return ok; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0.0f; return ok; }
 int hipFuncSetAttribute(const void *f, int attr, int v) { (void)f; (void)attr; (void)v; return ok; }
-/* tv_filter.hip's list of a mask's rows: its launch counts them and the blocks they lie in */
-static const void *mask_slots;
+/* tv_filter.hip's count of a mask's rows and of the blocks they lie in */
+atomic_int fake_counts;               /* launches of it that the host waits for */
+static const void *mask_count;
 void __hipRegisterFunction(void **modules, const void *host, char *device, const char *name, unsigned limit, void *a, void *b, void *c, void *d, int *e) {
     (void)modules; (void)device; (void)limit; (void)a; (void)b; (void)c; (void)d; (void)e;
-    if (strstr(name, "k_mask_slots")) mask_slots = host;
+    if (strstr(name, "k_mask_count")) mask_count = host;
 }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) {
     (void)g; (void)b; (void)lds; (void)s;
     ++fake_launches;
-    if (f == mask_slots) {
+    if (f == mask_count && *(uint64_t **)args[5] != NULL) {
+        ++fake_counts;
         const uint32_t *mask = *(const uint32_t **)args[0];
         const uint32_t n = *(uint32_t *)args[1];
-        uint32_t *totals = *(uint32_t **)args[6], rows = 0, live = 0;
+        const uint32_t pieces = *(uint32_t *)args[3];
+        uint64_t *totals = *(uint64_t **)args[5], rows = 0, live = 0;
         for (uint32_t w = 0; w * 32 < n; ++w) {
             const uint32_t x = n - w * 32 < 32 ? mask[w] & ((1u << (n - w * 32)) - 1u) : mask[w];
             rows += (uint32_t)__builtin_popcount(x);
             live += x != 0;
         }
-        totals[0] = rows;
-        totals[1] = live;
-        totals[2] = 1;
+        for (uint32_t i = 1; i < (pieces + 3) / 4 && i < 256; ++i) totals[i] = (uint64_t)1 << 63;
+        totals[0] = (uint64_t)1 << 63 | live << 31 | rows;
     }
     return ok;
 }

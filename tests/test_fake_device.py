@@ -308,3 +308,19 @@ for t in calls: t.join()
 assert bad == [T.OK] * 3, bad
 assert ix.merged_calls() == 0 and var("marker_copies").value == 1
 ''')
+
+
+def test_masks_of_host_arrays_are_counted_on_the_host(fake):
+    """Whether a mask's rows lie scattered is counted on the device, and waited for, only where the mask lies there."""
+    fake('''
+ix, n, counts = index(100_000, 1536), 100_000, var("counts")
+q, s, i = np.ones((1024, 1536), np.float32), np.zeros((1024, 10), np.float32), np.zeros((1024, 10), np.int64)
+for rows, gathers in ((np.arange(n) // 2 % 10 == 0, True), ((np.arange(n) > 30_000) & (np.arange(n) < 50_000), False)):
+    words, allowed = T.pack_mask(rows)
+    before = ix.gathered_searches()[0]
+    ix.search(q, 10, mask_words=words)
+    assert ix.gathered_searches()[0] == before + gathers and counts.value == 0
+    ix.search_dev(q.ctypes.data, 1024, 10, s.ctypes.data, i.ctypes.data, words.ctypes.data, allowed)
+    assert ix.gathered_searches()[0] == before + 2 * gathers and counts.value == 1
+    counts.value = 0
+''')

@@ -228,3 +228,27 @@ def test_only_the_queries_that_do_not_fit_are_repeated(T, dim, nq, k, rows):
             assert ix.gathered_searches() == (1, 0) and ix.overflow_redos() == len(rows)
     assert np.array_equal(out[0][1], out[1][1]) and bits_equal(out[0][0], out[1][0])
     ix.close()
+
+
+# the counting workgroups take one piece of 8192 rows to a wave up to 8388608 rows, several beyond
+@pytest.mark.parametrize("n", [8_388_608, 8_388_609, 17_000_003])
+def test_rows_counted_in_several_turns(T, n):
+    ix, gen = filled(T, 8, 4, n)
+    q = torch.randn(2, 8, device="cuda:0", generator=gen)
+    for m in (np.arange(n) % 97 == 5, np.arange(n) >= n - 70_000):
+        words, allowed = T.pack_mask(m)
+        mask = torch.from_numpy(words.view(np.int64)).cuda()
+        out = []
+        for path in (MASKED, GATHERED):
+            s, i = torch.zeros(2, 10, device="cuda:0"), torch.zeros(2, 10, dtype=torch.int64, device="cuda:0")
+            torch.cuda.synchronize()
+            ix.set_path(path)
+            before = ix.gathered_searches()[0]
+            ix.search_dev(q.data_ptr(), 2, 10, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed)
+            assert ix.gathered_searches()[0] - before == (path == GATHERED)
+            out.append((s.cpu().numpy(), i.cpu().numpy()))
+        assert np.array_equal(out[0][1], out[1][1]) and bits_equal(out[0][0], out[1][0])
+        ix.set_path(GATHERED)
+        ix.search_dev(q.data_ptr(), 2, 10, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed - 1)      # not the mask's count
+        assert ix.gathered_searches()[0] == before + 1
+    ix.close()

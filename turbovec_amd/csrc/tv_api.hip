@@ -1327,8 +1327,14 @@ double scan_block_ns(const tv_index *ix, size_t nq) {
 // range of 1 % of the rows, 1024 queries: 4M x 256 2-bit 522 us with the mask and 144 gathered, 1M x 128 215 and 86).
 constexpr double kPassedBlockNs = 0.08;
 // Gathering, per gathered block and chunk: the lines its rows lie in, up to eight times their bytes, and the write; and its
-// launches and the wait for the count, 15 us of it spent once it is known.  The launches that a search without sampling saves.
-constexpr double kGatherNs = 0.2, kGatherFixedNs = 20000.0, kCountedNs = 5000.0, kUnsampledNs = 25000.0;
+// launches and the wait for the count, or what is left of them once the blocks are counted, or where the host knew.  (22 us: half the rows of
+// 100K x 128 at random, 1024 queries, are 20 by this count, and gathering them gains 4 of 78; 10 us from the host: a range of 1 % of
+// 100K x 1536, 1024 queries, is 7.7, and 370 us with the mask and 374 gathered.)  The launches that a search without sampling saves.
+constexpr double kGatherNs = 0.2, kGatherFixedNs = 22000.0, kCountedNs = 5000.0, kKnownNs = 10000.0, kUnsampledNs = 25000.0;
+constexpr size_t kLiveUnknown = ~size_t(0);
+// Rows listed while the host waits for the count, and for nothing where it then reads the mask (2M rows of 4M x 256, 40 queries: 181 us
+// with the mask and 201 listed first).
+constexpr size_t kListedAtOnce = size_t(1) << 18;
 constexpr size_t kGatheredBytes = size_t(1) << 30;      // the largest such copy an index keeps room for
 bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed, bool in_place) {
     const double blocks = n_allowed / tv::kVecBlock + 1.0, each = scan_block_ns(ix, nq);
@@ -1386,50 +1392,68 @@ int leave_in_place(tv_index *ix, size_t nq, size_t k_eff) {
 // With the mask read during the scan, and gathered, us a search (k = 10): 10 % of the rows allowed at random, 4M x 256 2-bit, 1024 queries 5210 and
 // 680; 4M x 768, 300 queries 1359 and 403; 1M x 768, 40 queries 131 and 105, 1 query 112 and 104; 1 %: 2M x 1536, 1024 queries 1295 and
 // 165, 1 query 152 and 74; 50 %: 4M x 768, 64 queries 425 and 660.  A range of 20 % of the
-// rows: 4M x 768, 300 queries 376 and 470; such a search pays up to 13 us for the count that tells (100K x 128, 1024 queries: 54
-// and 67).  Read in place (with the mask, copied, in place): 50 %, 4M x 768, 1024 queries 3337, 2030 and 1650, 300 queries 1310, 1050 and
+// rows: 4M x 768, 300 queries 376 and 470.  Read in place (with the mask, copied, in place): 50 %, 4M x 768, 1024 queries 3337, 2030 and 1650, 300 queries 1310, 1050 and
 // 700; 10M x 1536, 1024 queries 13270 and, in place, 7130; 80 % 1330 and 970 in place; 30 %, 2M x 1536, 300 queries 1181 and 754; a range of half the rows, 1024 queries 1601 and 1576.
 // Gathers the rows `d_mask` allows where a search of nq queries is faster on them; ix->allowed then has them.  Whether rows
-// lie scattered, which it depends on, is counted on the device and waited for; from the number of allowed rows
-// alone, taken to be scattered, most calls that it cannot pay for are told without.
-int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t nq, size_t k_eff) {
+// lie scattered, which it depends on, a caller says who has seen the mask (live, the blocks with an allowed row); otherwise it is counted on
+// the device and waited for, and from the number of allowed rows alone, taken to be scattered, most calls that
+// it cannot pay for are told without.  A search that counts and then reads the mask, of a
+// range of the rows, pays 8 us (100K x 1536, 300 queries, 20 %: 88 and 96).
+int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t live, size_t nq, size_t k_eff) {
     const size_t n = ix->n, n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (ix->ws_fixed || ix->no_gather || n_allowed == 0 || n_allowed >= n || n >= (size_t(1) << 31)) return TV_OK;
     bool in_place = scans_in_place(ix, nq, k_eff, n_allowed);
     const bool large = in_place && n_blocks * ix->geo.block_bytes() > 0xffffffffull;      // rows of a block may lie too far apart
     if (!in_place && gathered_need(ix, n_allowed) > kGatheredBytes) return TV_OK;
+    auto pays = [&](double blocks, double fixed) {
+        return ix->force_gather || gather_pays(ix, nq, k_eff, double(n_blocks), blocks, double(n_allowed), fixed, in_place);
+    };
+    const bool known = live != kLiveUnknown;
     const double scattered = double(n_blocks) * (1.0 - std::pow(1.0 - double(n_allowed) / double(n), double(tv::kVecBlock)));
-    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), scattered, double(n_allowed), kGatherFixedNs, in_place)) return TV_OK;
+    if (!(known ? pays(double(live), kKnownNs) : pays(scattered, kGatherFixedNs))) return TV_OK;
     const size_t count_bytes = round_up(tv::mask_counts(n) * 2 * sizeof(uint32_t), 256);
     use_spares(ix, true);
     if (!have_block(ix, ix->slots, count_bytes + n_allowed * sizeof(uint32_t))) return TV_OK;
     uint32_t *counts = static_cast<uint32_t *>(ix->slots.p), *slots = counts + count_bytes / sizeof(uint32_t);
-    volatile uint32_t *totals = ix->h_flags;
-    totals[2] = totals[3] = 0;
-    TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->d_flags_host, ix->stream));
+    static_assert(kGroupQueries >= 2 * tv::kMaxMaskTotals + 1, "the counts lie where the flags will");
+    volatile uint64_t *totals = reinterpret_cast<uint64_t *>(ix->h_flags);
+    const size_t n_totals = tv::mask_totals(n);
+    for (size_t i = 0; i < n_totals; ++i) totals[i] = 0;
+    TV_HIP(tv::launch_mask_count(d_mask, n, counts, known ? nullptr : reinterpret_cast<uint64_t *>(ix->d_flags_host), ix->stream));
+    // (a short list is there by the time the host has the count and has launched what comes next)
+    const bool at_once = known || n_allowed <= kListedAtOnce;
+    if (at_once) TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->stream));
+    if (!known) {
+        // (a wait of a few microseconds, which through the runtime takes ten more; beyond that it is the runtime's)
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        size_t there = 0;
+        while (there < n_totals && (totals[there] != 0 || std::chrono::steady_clock::now() < until)) there += totals[there] != 0;
+        if (there < n_totals) TV_HIP(hipStreamSynchronize(ix->stream));
+        uint64_t sum = 0;
+        for (size_t i = 0; i < n_totals; ++i) sum += totals[i] & ~tv::kMaskCounted;
+        if ((sum & 0x7fffffffu) != n_allowed) return TV_OK;      // (the caller's count is not the mask's)
+        live = size_t(sum >> 31);
+        if (!pays(double(live), kCountedNs)) return TV_OK;
+    }
+    if (!at_once) TV_HIP(tv::launch_mask_slots(d_mask, n, counts, slots, n_allowed, ix->stream));
     if (large) {
-        TV_HIP(tv::launch_rows_apart(slots, n_allowed, ix->geo.block_bytes(), ix->d_flags_host + 3, ix->stream));
+        volatile uint32_t *far = ix->h_flags + 2 * tv::kMaxMaskTotals;
+        *far = 0;
+        TV_HIP(tv::launch_rows_apart(slots, n_allowed, ix->geo.block_bytes(), ix->d_flags_host + 2 * tv::kMaxMaskTotals, ix->stream));
         TV_HIP(hipStreamSynchronize(ix->stream));
+        if (*far != 0) {
+            in_place = false;
+            if (gathered_need(ix, n_allowed) > kGatheredBytes || !pays(double(live), kCountedNs)) return TV_OK;
+        }
     }
-    // (a wait of a few microseconds, which through the runtime takes ten more; beyond that it is the runtime's)
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-    while (totals[2] == 0 && std::chrono::steady_clock::now() < until) {}
-    if (totals[2] == 0) TV_HIP(hipStreamSynchronize(ix->stream));
-    std::atomic_thread_fence(std::memory_order_acquire);
-    const size_t total = totals[0], live = totals[1];
-    if (total != n_allowed) return TV_OK;      // (the caller's count is not the mask's)
-    if (totals[3] != 0) {
-        in_place = false;
-        if (gathered_need(ix, total) > kGatheredBytes) return TV_OK;
-    }
-    if (!ix->force_gather && !gather_pays(ix, nq, k_eff, double(n_blocks), double(live), double(total), kCountedNs, in_place)) return TV_OK;
-    if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, total, slots, live, true};
-    else if (const int rc = copy_allowed(ix, slots, total, live)) return rc;
+    if (in_place) ix->allowed = tv_rows{ix->d_codes, ix->d_scales, n_allowed, slots, live, true};
+    else if (const int rc = copy_allowed(ix, slots, n_allowed, live)) return rc;
     if (ix->allowed.codes) ++ix->gathered_searches;
     return TV_OK;
 }
+// live: the blocks of 32 rows with one that the mask allows, where the caller knows.
 int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
-                  size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
+                  size_t n_allowed, size_t live, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
     struct Back {
         tv_index *ix;
         void give() {
@@ -1439,7 +1463,7 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         ~Back() { give(); }
     } back{ix};
     if (d_mask && k != 0 && nq != 0) {
-        const int rc = gather_allowed(ix, d_mask, n_allowed, nq, std::min(std::min(k, ix->n), n_allowed));
+        const int rc = gather_allowed(ix, d_mask, n_allowed, live, nq, std::min(std::min(k, ix->n), n_allowed));
         if (rc != TV_OK) return rc;
     }
     g_refused = false;
@@ -1484,6 +1508,35 @@ struct tv_request {
 
 namespace {
 
+// The rows a mask allows, and the blocks of 32 with one.  For the 1.25 MB of 10M rows: 54 us with 256-bit vectors, which the
+// build's flags do not ask for, and 150 without (120 for the rows alone).
+typedef uint32_t HalfWord __attribute__((may_alias));
+__attribute__((always_inline)) inline void count_words(const uint64_t *words, size_t n, size_t &rows, size_t &live) {
+    for (size_t w = 0; w < n; w += 1024) {      // (from the first-level cache the second time)
+        const uint64_t *x = words + w;
+        const size_t m = std::min<size_t>(1024, n - w);
+        uint64_t r = 0;
+        uint32_t l = 0;
+        for (size_t i = 0; i < m; ++i) r += uint64_t(__builtin_popcountll(x[i]));
+        const HalfWord *h = reinterpret_cast<const HalfWord *>(x);      // (their order does not matter)
+        for (size_t i = 0; i < 2 * m; ++i) l += uint32_t(h[i] != 0);
+        rows += r;
+        live += l;
+    }
+}
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+__attribute__((target("avx2"))) void count_words_avx2(const uint64_t *words, size_t n, size_t &rows, size_t &live) { count_words(words, n, rows, live); }
+#endif
+void count_mask(const uint64_t *words, size_t n, size_t &rows, size_t &live) {
+    rows = live = 0;
+    const uint64_t last = n % 64 ? words[n / 64] & ((uint64_t(1) << (n % 64)) - 1) : 0;
+    count_words(&last, 1, rows, live);
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_cpu_supports("avx2")) return count_words_avx2(words, n / 64, rows, live);
+#endif
+    count_words(words, n / 64, rows, live);
+}
+
 // Serves the calls of `batch` (compatible with each other, at least one) as one search.  The index
 // lock is held.  Returns the status every one of them gets.
 int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_eff_out) {
@@ -1495,7 +1548,7 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
     if (!r0.host) {
         const size_t n_allowed = r0.mask ? r0.mask_arg : n;
         if (batch.size() == 1)
-            return search_device(ix, r0.q, nq, r0.k, r0.mask, n_allowed, r0.out_s, r0.out_i, k_eff_out);
+            return search_device(ix, r0.q, nq, r0.k, r0.mask, n_allowed, kLiveUnknown, r0.out_s, r0.out_i, k_eff_out);
         // several callers' device buffers: gathered into the staging allocation, results scattered back
         const size_t k_eff = std::min(std::min(r0.k, n), n_allowed);
         *k_eff_out = k_eff;
@@ -1513,7 +1566,7 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
             if (r->nq) TV_HIP(hipMemcpyAsync(d_q + at * dim, r->q, r->nq * dim * sizeof(float), hipMemcpyDeviceToDevice, ix->stream));
             at += r->nq;
         }
-        rc = search_device(ix, d_q, nq, r0.k, r0.mask, n_allowed, d_s, d_i, nullptr);
+        rc = search_device(ix, d_q, nq, r0.k, r0.mask, n_allowed, kLiveUnknown, d_s, d_i, nullptr);
         if (rc != TV_OK) return rc;
         at = 0;
         for (const tv_request *r : batch) {
@@ -1528,15 +1581,10 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
     }
     const uint64_t *mask_words = r0.staged_mask ? r0.staged_mask : r0.mask;
     const size_t n_mask_words = r0.mask_arg;
-    size_t n_allowed = n;
+    size_t n_allowed = n, live = 0;
     if (mask_words) {
         if (n_mask_words != (n + 63) / 64) return TV_ERR_MASK_LENGTH_MISMATCH;
-        n_allowed = 0;  // search.rs:3222-3225; bits at or past n are ignored
-        for (size_t w = 0; w < n_mask_words; ++w) {
-            uint64_t word = mask_words[w];
-            if (w * 64 + 64 > n) word &= (n - w * 64 >= 64) ? ~uint64_t(0) : ((uint64_t(1) << (n - w * 64)) - 1);
-            n_allowed += size_t(__builtin_popcountll(word));
-        }
+        count_mask(mask_words, n, n_allowed, live);  // search.rs:3222-3225; bits at or past n are ignored
     }
     const size_t k_eff = std::min(std::min(r0.k, n), n_allowed);
     *k_eff_out = k_eff;
@@ -1570,7 +1618,8 @@ int serve_batch(tv_index *ix, const std::vector<tv_request *> &batch, size_t *k_
         g_last_error = "host to device copy failed";
         return TV_ERR_HIP;
     }
-    rc = search_device(ix, d_q, nq, r0.k, d_m, n_allowed, d_s, d_i, nullptr);
+    // (an array that is not staged may change until it has been copied: the device counts what it got)
+    rc = search_device(ix, d_q, nq, r0.k, d_m, n_allowed, r0.staged_mask ? live : kLiveUnknown, d_s, d_i, nullptr);
     if (rc != TV_OK || in_place) return rc;
     at = 0;
     for (const tv_request *r : batch) {
@@ -2295,7 +2344,7 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     ix->ws = ix->scratch;
     ix->ws_bytes = kScratchBytes;
     ix->ws_fixed = true;
-    const int rc = search_device(ix, d_queries, nq, k, d_mask_words, n_allowed, d_out_scores, d_out_indices, out_k_eff);
+    const int rc = search_device(ix, d_queries, nq, k, d_mask_words, n_allowed, kLiveUnknown, d_out_scores, d_out_indices, out_k_eff);
     ix->ws = own_ws;
     ix->ws_bytes = own_bytes;
     ix->ws_fixed = false;

@@ -205,10 +205,17 @@ hipError_t launch_probe_mfma(int device, int iters, uint32_t *sink, double *ops,
 hipError_t launch_select_topk(const float *d_scores, size_t n, int nq_tile, size_t k_eff, uint64_t *d_keys_tmp,
                               uint32_t *d_hist, float *out_scores, int64_t *out_idx, hipStream_t s);
 size_t select_tmp_keys(size_t k_eff);
-// Filtered searches on the allowed rows alone (tv_filter.hip).  The rows of the mask's set bits below n, in order, to slots[0 .. room), and
-// how many there are and in how many blocks to totals[0], totals[1] (host memory; totals[2] is 1 after them); counts: two words for each of mask_counts(n) workgroups.
+// Filtered searches on the allowed rows alone (tv_filter.hip).  How many of the mask's bits below n are set and in how many blocks
+// of 32, piece by piece to counts (two words for each of mask_counts(n) pieces) and, unless null, in all to the words totals[0 .. mask_totals(n))
+// (host memory): those with the bit kMaskCounted are there, and their sum counts both.
+constexpr uint64_t kMaskCounted = uint64_t(1) << 63;
+constexpr size_t kMaxMaskTotals = 256;
+__host__ __device__ constexpr uint64_t mask_total(uint32_t rows, uint32_t blocks) { return uint64_t(blocks) << 31 | rows; }     // (rows below 2^31, of all words too)
 size_t mask_counts(size_t n);
-hipError_t launch_mask_slots(const uint64_t *mask, size_t n, uint32_t *counts, uint32_t *slots, size_t room, uint32_t *totals, hipStream_t s);
+size_t mask_totals(size_t n);
+hipError_t launch_mask_count(const uint64_t *mask, size_t n, uint32_t *counts, uint64_t *totals, hipStream_t s);
+// The rows of those bits, in order, to slots[0 .. room).
+hipError_t launch_mask_slots(const uint64_t *mask, size_t n, const uint32_t *counts, uint32_t *slots, size_t room, hipStream_t s);
 // *far becomes 1 (host memory; cleared by the caller) where the rows of a block of 32 among slots[0 .. n) lie 4 GiB of codes or more apart.
 hipError_t launch_rows_apart(const uint32_t *slots, size_t n, size_t block_bytes, uint32_t *far, hipStream_t s);
 // The rows slots[0 .. n) into blocks of their own, the last one's missing rows zero.
