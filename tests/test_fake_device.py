@@ -140,11 +140,24 @@ assert var("marker_copies").value == 0
 ''')
 
 
+def test_small_indexes_are_searched_without_sampling(fake):
+    """Batches of a few queries on the shortest rows, one query and many on short rows of u8 tables; few blocks of long ones are not."""
+    fake('''
+for dim, bits, rows, nq, k, unsampled in ((64, 4, 60_000, 2, 10, True), (8, 4, 1_000_000, 8, 100, True), (128, 2, 100_000, 1, 10, True), (1536, 2, 20_000, 1, 10, True),
+                                          (64, 2, 131_073, 40, 10, True), (32, 3, 131_072, 400, 10, True), (512, 2, 1000, 1, 10, True), (3072, 2, 1000, 1, 10, False),
+                                          (1024, 3, 2048, 1, 10, False), (1024, 3, 2049, 1, 10, True)):
+    ix = T.NativeIndex(dim, bits)
+    ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
+    assert (len(ix.sampling_plan(nq, k)[0]) == 0) == unsampled, (dim, bits, rows, nq, k)
+    ix.close()
+''')
+
+
 FILTERED = '''
 def filtered(ix, path, nq=4):
-    """A search of half the rows; path 64 gathers them, 32 reads the mask."""
+    """A sampled search (16) of half the rows; path 64 gathers them, 32 reads the mask."""
     words = T.pack_mask(np.arange(len(ix)) % 2 == 1)[0]
-    ix.set_path(path)
+    ix.set_path(path | 16)
     before = ix.gathered_searches()[0]
     ix.search(np.ones((nq, 64), np.float32), 3, mask_words=words)
     return ix.gathered_searches()[0] - before

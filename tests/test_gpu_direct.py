@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -126,6 +126,7 @@ def test_scan_time_leaves_out_the_preparation(T):
 def test_every_launch_of_the_timed_scan_counts(T, mode, nq, launches):
     ix = T.NativeIndex(64, 2)
     ix.set_score_mode(getattr(T, "SCORE_" + mode))
+    ix.set_path(SAMPLED)
     ix.add(unit_gaussian(70_000, 64, seed=5))
     ix.search(unit_gaussian(nq, 64, seed=6), 10)
     assert len(ix.sampling_plan(nq, 10)[0]) == 2      # a level before the full scan: timed between stamps

@@ -4,7 +4,7 @@ sixteen queries over 4096 or more (block, query tile) pairs with the u32 epilogu
 import numpy as np
 import pytest
 
-from helpers import OracleIndex, bits_equal, to_native, unit_gaussian
+from helpers import SAMPLED, OracleIndex, bits_equal, to_native, unit_gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -30,11 +30,13 @@ def test_sparse_scan_matches_oracle(T, oracle, dim, bits, n, nq):
     for m in (None, rng.random(n) < 0.5, rng.random(n) < 0.003, (np.arange(n) >= 9_000) & (np.arange(n) < 11_000)):
         words = None if m is None else T.pack_mask(m)[0]
         for k in (1, 10, 100):
-            s, i = ix.search(q, k, mask_words=words)
             os_, oi = oidx.search(q, k, mask_words=words, mode=oracle.MODE_L_U32)
-            assert np.array_equal(i, oi), k
-            assert bits_equal(s, os_), k
-            assert ix.queries_per_launch() == nq
+            for path in (0, SAMPLED):               # every block's best score; candidates
+                ix.set_path(path)
+                s, i = ix.search(q, k, mask_words=words)
+                assert np.array_equal(i, oi), (k, path)
+                assert bits_equal(s, os_), (k, path)
+                assert ix.queries_per_launch() == nq
     ix.close()
 
 
@@ -43,6 +45,7 @@ def test_equal_rows_overflow_to_the_exact_path(T, oracle):
     dim, bits, n, nq = 32, 2, 131_080, 40
     oidx = OracleIndex(oracle, dim, bits, np.tile(unit_gaussian(1, dim, seed=3), (n, 1)))
     ix = to_native(T, oidx)
+    ix.set_path(SAMPLED)
     q = unit_gaussian(nq, dim, seed=4)
     for k in (10, 40):
         s, i = ix.search(q, k)

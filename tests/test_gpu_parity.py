@@ -567,10 +567,12 @@ def test_lut_single_query_matches_oracle(T, oracle, dim, bits, n, mode):
         q = unit_gaussian(1, dim, seed=70 + qi)
         words = None if m is None else T.pack_mask(m)[0]
         for k in (1, 10, 100, 128, 129):
-            s, i = ix.search(q, k, mask_words=words)
             os_, oi = oidx.search(q, k, mask_words=words, mode=omode(O, mode))
-            assert np.array_equal(i, oi), k
-            assert bits_equal(s, os_), k
+            for path in (0, SAMPLED):
+                ix.set_path(path)
+                s, i = ix.search(q, k, mask_words=words)
+                assert np.array_equal(i, oi), (k, path)
+                assert bits_equal(s, os_), (k, path)
     strides, _ = ix.sampling_plan(1, 10)
     assert len(strides) == 2                      # one level without floors, then the full scan
     strides, _ = ix.sampling_plan(1, 129)         # beyond the floorless level's k: the row-level ladder

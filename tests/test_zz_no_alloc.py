@@ -6,6 +6,8 @@ and the refusal of a search that would not fit."""
 import numpy as np
 import pytest
 
+from helpers import SAMPLED
+
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
@@ -78,6 +80,7 @@ def test_noalloc_exact_fallback_runs_inside_the_scratch(T):
     """Identical rows tie everywhere: the candidate segments overflow and the queries are redone
     through the exact lists, which must come out of the same fixed array."""
     ix, gen = build(T, 60_000, 64, 4, seed=9, duplicate_rows=True)
+    ix.set_path(SAMPLED)
     q = torch.randn(6, 64, device="cuda:0", generator=gen)
     before = ix.overflow_redos()
     pair = both(ix, q, 10)

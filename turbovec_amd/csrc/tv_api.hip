@@ -845,8 +845,8 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
     return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) + 65536;
 }
 // Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, each pair
-// without sampling and with it: 100K x 128, 1 query 30 and 45, 64 queries 32 and 61, 1000 queries 67 and 493;
-// 260K x 768, 32 queries 54 and 71; 100K x 1536, 1000 queries 246 and 304.
+// without sampling and with it: 100K x 128, 1 query 30 and 45, 64 queries 32 and 61, 1000 queries 67 and 493; x 64, 5 queries
+// 29 and 45 (1.04M: 45 and 59); 260K x 768, 32 queries 54 and 71; 100K x 1536, 1000 queries 246 and 304.
 //  - It scores k blocks a second time in one workgroup: k = 100 at 768 dimensions (12 chunks) costs one
 //    query 77 us against 64, at 128 dimensions 40 against 72.
 //  - k_pick keeps a word per block in registers: 32768 blocks at most (twice that spills: 2M x 128, one query
@@ -862,24 +862,20 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
 //  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about 700K
 //    rows (1000 queries: 600K x 768 570 and 621, x 1536 972 and 999; 1.04M x 768 935 and 895, x 1536 1611 and 1523),
 //    earlier where many rows are scored again (500K x 768, k = 45: 556 and 540).
-// Batches of 2 to 8 on rows of one chunk keep to the sampled path beyond 1535 blocks, and not for its speed: it is
-// how the test of the exact fallback in a fixed workspace gets there.
 // The same for u8-LUT queries with the u32 epilogue.  k = 10, us a search without sampling and with it, 2 bits: 100K x 128, 1 query
-// 34 and 43, 12 queries 42 and 62, 100 queries 61 and 96; 400K x 512, 4 queries 52 and 86; 20K x 1536, 100 queries
-// 89 and 164; 1M x 1536, 12 queries 198 and 236.
+// 32 and 42, 12 queries 42 and 62, 100 queries 61 and 96; 400K x 64, 100 queries 84 and 146; 400K x 512, 4 queries 52 and 86; 20K x 1536,
+// 100 queries 89 and 164; 1M x 1536, 12 queries 198 and 236.
 //  - Rows are scored a second time at two table reads a byte: 100 blocks of 12 chunks take 50 us (400K x 768 3-bit, one
 //    query, k = 60: 95 and 85; 60K x 1536, 8 queries, k = 100: 99 and 97; 400K: 133 and 138; 64 queries: 147 and
-//    177; 60K, 400 queries: 309 and 285).
+//    177; 60K, 400 queries: 309 and 285).  One query over up to 64 blocks would be scanned once, without a level in front (1000 rows x
+//    512 34 and 40; x 1536 49 and 50; x 1024 3-bit 54.3 and 53.6; x 3072 71 and 66, k = 1 65.7 and 65.3).
 //  - The matrix-unit scan pays its epilogue on every (block, tile) pair: 400K x 1536, 500 queries (200K pairs) 983 and 1038, 1M x
 //    512 (500K pairs) 1060 and 955.
-// One query of up to 8192 chunks in all, and the matrix-unit scan on rows of up to 16 byte-groups, keep to the sampled
-// path, and not for its speed: they are how the tests of the kernels' append form get there.
 bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const size_t nch = size_t(ix->geo.nch), rescored = k_eff * nch, tiles = (std::min(nq, kChunkQueries) + tv::kQTile - 1) / tv::kQTile;
     if (effective_mode(ix) != TV_SCORE_L_U32 || ix->no_lut16 || tv::pick_lds_bytes(int(nch), k_eff, true) > tv::kPickLds) return false;
-    if (nq == 1) return n_blocks * nch > 8192 && rescored <= 400;
+    if (nq == 1) return rescored <= (n_blocks > 64 ? 400u : nch <= 16 ? 120u : 0u);
     if (nq <= size_t(tv::kLut16Queries)) return rescored <= (n_blocks >= 4096 ? 1200u : 720u);
-    if (ix->geo.G <= 16 && lut_mx_serves(ix, nq)) return false;
     return n_blocks * tiles <= 200000 && rescored <= (tiles <= 4 ? 1200u : 600u);
 }
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
@@ -890,7 +886,6 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks)
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
     if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks);
     if (!tv::best_serves(nch) || k_eff * nch > 600 || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds) return false;
-    if (nch == 1 && nq >= 2 && nq <= 8 && n_blocks >= 1536) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
     if (nch < 12) return triples <= 6000000;
