@@ -252,3 +252,22 @@ def test_rows_counted_in_several_turns(T, n):
         ix.search_dev(q.data_ptr(), 2, 10, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed - 1)      # not the mask's count
         assert ix.gathered_searches()[0] == before + 1
     ix.close()
+
+
+# beyond the k of the all-queries scan's floorless level, over more blocks than are searched without sampling
+def test_rows_in_place_for_many_results(T):
+    n, dim, nq, k = 1_100_000, 768, 140, 100
+    ix, gen = filled(T, dim, 4, n)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen)
+    words, allowed = T.pack_mask(np.random.default_rng(8).random(n) < 0.5)
+    mask = torch.from_numpy(words.view(np.int64)).cuda()
+    out = []
+    for path in (0, MASKED):
+        s, i = torch.zeros(nq, k, device="cuda:0"), torch.zeros(nq, k, dtype=torch.int64, device="cuda:0")
+        torch.cuda.synchronize()
+        ix.set_path(path)
+        ix.search_dev(q.data_ptr(), nq, k, s.data_ptr(), i.data_ptr(), mask.data_ptr(), allowed)
+        out.append((s.cpu().numpy(), i.cpu().numpy()))
+        assert ix.gathered_searches() == (1, 1)
+    assert np.array_equal(out[0][1], out[1][1]) and bits_equal(out[0][0], out[1][0])
+    ix.close()

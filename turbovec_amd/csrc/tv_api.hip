@@ -1352,7 +1352,7 @@ bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowe
         for (size_t c0 = 0, cq; c0 < gq; c0 += cq) {
             cq = chunk_len(ix, gq - c0);
             const SampledPlan plan = sampled_plan(ix, cq);
-            if (!plan.wide || !tv::wide_reads_rows(ix->geo.nch, int(cq)) || level_strides(ix, plan, blocks, std::max<size_t>(k_eff, 16), false, false).best_words) return false;
+            if (!plan.wide || !tv::wide_reads_rows(ix->geo.nch, int(cq))) return false;
         }
     }
     return true;
@@ -1389,6 +1389,8 @@ int leave_in_place(tv_index *ix, size_t nq, size_t k_eff) {
 // 165, 1 query 152 and 74; 50 %: 4M x 768, 64 queries 425 and 660.  A range of 20 % of the
 // rows: 4M x 768, 300 queries 376 and 470.  Read in place (with the mask, copied, in place): 50 %, 4M x 768, 1024 queries 3337, 2030 and 1650, 300 queries 1310, 1050 and
 // 700; 10M x 1536, 1024 queries 13270 and, in place, 7130; 80 % 1330 and 970 in place; 30 %, 2M x 1536, 300 queries 1181 and 754; a range of half the rows, 1024 queries 1601 and 1576.
+// k = 100, 50 %, from the row-level ladder (a copy, searched from best words, and in place): 4M x 768, 300 queries 1166 and 878, 1024 queries 2204 and 2116; 80 %,
+// 300 queries 1363 and 1175; with the mask and in place: 2M x 1536, 300 queries 1118 and 815.
 // Gathers the rows `d_mask` allows where a search of nq queries is faster on them; ix->allowed then has them.  Whether rows
 // lie scattered, which it depends on, a caller says who has seen the mask (live, the blocks with an allowed row); otherwise it is counted on
 // the device and waited for, and from the number of allowed rows alone, taken to be scattered, most calls that
