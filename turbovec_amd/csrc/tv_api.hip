@@ -141,7 +141,7 @@ void free_blocks(const std::vector<std::pair<size_t, void *>> &blocks) {
 void *take_spare(DevicePool &pool) {
     for (tv_index *ix = pool.newest; ix != nullptr; ix = ix->older)
         for (tv_spare *s : {&ix->gathered, &ix->slots})
-            if (s->p != nullptr && !s->in_use) { s->bytes = 0; return std::exchange(s->p, nullptr); }
+            if (!s->in_use && s->p != nullptr) { s->bytes = 0; return std::exchange(s->p, nullptr); }
     return nullptr;
 }
 
