@@ -784,7 +784,8 @@ bool first_level_is_best_words(const tv_index *ix, const SampledPlan &plan, size
 size_t floor_rows(const tv_index *ix, const SampledPlan &plan) {
     return plan.lut_mx ? 512 : effective_mode(ix) == TV_SCORE_P && ix->geo.nch < 12 ? 256 : 1024;
 }
-SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool repeat, bool masked) {
+// sure: of every `step` blocks in turn, sure / step hold a row the search may return, whatever its mask looks like.
+SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t sure, size_t k_floor, bool repeat, bool masked) {
     if (!repeat && first_level_is_best_of_block(ix, plan, k_floor)) {
         SamplingSteps steps;
         // (the all-queries kernel pays for every candidate of the full scan -- a tile with one in it
@@ -815,10 +816,13 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
         SamplingSteps steps;
         const size_t sample = std::min<size_t>({std::max<size_t>(n_blocks * k_floor / floor_rows(ix, plan), 8 * k_floor), size_t(tv::kMaxFloorBlocks), n_blocks / 4,
                                                  plan.seg_stride * tv::kSegCap * 2});      // (the words lie in the candidates' place)
-        steps.step[steps.count++] = uint32_t((n_blocks + sample - 1) / sample);
-        steps.step[steps.count++] = 1;
-        steps.best_first = steps.best_words = true;
-        return steps;
+        const size_t step = (n_blocks + sample - 1) / sample;
+        if (sure / step >= k_floor) {      // (fewer would leave the floor open)
+            steps.step[steps.count++] = uint32_t(step);
+            steps.step[steps.count++] = 1;
+            steps.best_first = steps.best_words = true;
+            return steps;
+        }
     }
     // (the sixteen-query LUT scan works in rounds too: every wave of the grid carries two blocks through the row)
     return plan.wide    ? sampling_steps(n_blocks, k_floor, size_t(plan.grid) * tv::wide_blocks_per_workgroup(ix->geo.nch))
@@ -987,6 +991,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
 }
 
 int leave_in_place(tv_index *ix, size_t nq, size_t k_eff);
+constexpr size_t kLiveUnknown = ~size_t(0);
 
 // The seam: search::search over device-resident inputs and outputs.
 //
@@ -999,10 +1004,13 @@ int leave_in_place(tv_index *ix, size_t nq, size_t k_eff);
 // by the same total order as everywhere else.
 //
 // Where ix->allowed has the rows `d_mask` allows, those are searched and the mask is not read -- but for queries
-// whose candidates did not fit in a scan of rows in place, which alone are repeated with it (or on a copy).
+// whose candidates did not fit in a scan of rows in place, which alone are repeated with it (or on a copy).  live: the
+// blocks of the index with a row that the mask allows, or kLiveUnknown.
 int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const uint64_t *d_mask,
-                size_t n_allowed, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
+                size_t n_allowed, size_t live, float *d_out_scores, int64_t *d_out_idx, size_t *out_k_eff) {
     const size_t n = ix->rows().n;
+    // (counted blocks may lie anywhere: half of a sample's share of them; rows of a mask nobody has looked at: the fewest blocks that hold so many)
+    const size_t sure = live != kLiveUnknown ? live / 2 : n_allowed / tv::kVecBlock;
     const uint64_t *mask = ix->allowed.codes ? nullptr : d_mask;
     size_t k_eff = std::min(std::min(k, n), n_allowed);  // lib.rs:1460, search.rs:3222-3225
     if (out_k_eff) *out_k_eff = k_eff;
@@ -1072,7 +1080,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const size_t tile_q = plan.tile_q, n_tiles = plan.n_tiles, cq_pad = plan.cq_pad, seg_stride = plan.seg_stride;
             const bool wide = plan.wide;
             const int grid = plan.grid;
-            const SamplingSteps steps = level_strides(ix, plan, n_blocks, k_floor, repeat, mask != nullptr);
+            const SamplingSteps steps = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, repeat, mask != nullptr);
             const bool best_first = steps.best_first;
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
@@ -1225,7 +1233,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
                 const SampledPlan plan = sampled_plan(ix, chunk_at[c + 1] - chunk_at[c]);
-                const size_t n_levels = level_strides(ix, plan, n_blocks, k_floor, false, mask != nullptr).size();
+                const size_t n_levels = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).size();
                 for (size_t lv = 1; lv + 1 < n_levels; ++lv)
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
             }
@@ -1251,7 +1259,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         }
         ix->overflow_redos += redo_rows.size() + exact_rows.size();
         if ((redo_rows.size() + exact_rows.size()) * 8 >= gq) {
-            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, k_floor, false, mask != nullptr).best_first) {
+            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).best_first) {
                 // from here on, the repeated passes below included -- unless the row-level ladder has just failed too
                 if (ix->floorless_kept_left == 0) ix->row_ladder_left = kRowLadderSearches;
             } else if (ix->row_ladder_left > 0) {
@@ -1326,7 +1334,6 @@ constexpr double kPassedBlockNs = 0.08;
 // 100K x 128 at random, 1024 queries, are 20 by this count, and gathering them gains 4 of 78; 10 us from the host: a range of 1 % of
 // 100K x 1536, 1024 queries, is 7.7, and 370 us with the mask and 374 gathered.)  The launches that a search without sampling saves.
 constexpr double kGatherNs = 0.2, kGatherFixedNs = 22000.0, kCountedNs = 5000.0, kKnownNs = 10000.0, kUnsampledNs = 25000.0;
-constexpr size_t kLiveUnknown = ~size_t(0);
 // Rows listed while the host waits for the count, and for nothing where it then reads the mask (2M rows of 4M x 256, 40 queries: 181 us
 // with the mask and 201 listed first).
 constexpr size_t kListedAtOnce = size_t(1) << 18;
@@ -1396,7 +1403,7 @@ int leave_in_place(tv_index *ix, size_t nq, size_t k_eff) {
 // the device and waited for, and from the number of allowed rows alone, taken to be scattered, most calls that
 // it cannot pay for are told without.  A search that counts and then reads the mask, of a
 // range of the rows, pays 8 us (100K x 1536, 300 queries, 20 %: 88 and 96).
-int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t live, size_t nq, size_t k_eff) {
+int gather_allowed(tv_index *ix, const uint64_t *d_mask, size_t n_allowed, size_t &live, size_t nq, size_t k_eff) {
     const size_t n = ix->n, n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (ix->ws_fixed || ix->no_gather || n_allowed == 0 || n_allowed >= n || n >= (size_t(1) << 31)) return TV_OK;
     bool in_place = scans_in_place(ix, nq, k_eff, n_allowed);
@@ -1464,12 +1471,12 @@ int search_device(tv_index *ix, const float *d_queries, size_t nq, size_t k, con
         if (rc != TV_OK) return rc;
     }
     g_refused = false;
-    const int rc = search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    const int rc = search_rows(ix, d_queries, nq, k, d_mask, n_allowed, live, d_out_scores, d_out_idx, out_k_eff);
     if (rc == TV_OK || !g_refused || !ix->slots.in_use) return rc;
     // no memory for the search beside its list and copy of rows, which are given up for it
     TV_HIP(hipStreamSynchronize(ix->stream));
     back.give();
-    return search_rows(ix, d_queries, nq, k, d_mask, n_allowed, d_out_scores, d_out_idx, out_k_eff);
+    return search_rows(ix, d_queries, nq, k, d_mask, n_allowed, live, d_out_scores, d_out_idx, out_k_eff);
 }
 
 // ---- search calls, merged ----------------------------------------------------------------------
@@ -2702,7 +2709,7 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (direct_serves(ix, nq, k_eff, n_blocks)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
-    const SamplingSteps steps = level_strides(ix, plan, n_blocks, std::max<size_t>(k_eff, 16), false, false);
+    const SamplingSteps steps = level_strides(ix, plan, n_blocks, n_blocks, std::max<size_t>(k_eff, 16), false, false);
     *count = steps.size();
     for (size_t i = 0; i < steps.size() && i < cap; ++i) {
         if (strides) strides[i] = steps[i];
