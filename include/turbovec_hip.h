@@ -257,7 +257,8 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * instead of the batched ones; bit 2 keeps them off the all-queries-per-pass
  * kernel only; bit 3 keeps u8-LUT batches on the scan that holds whole tables in
  * LDS (at most 8 queries per pass) instead of the larger ones; bit 4 samples
- * small indexes like large ones (bits 1 and 2 do too); bit 6 has filtered searches
+ * small indexes (bits 1 and 2 do too), and those of up to 16384 blocks by the
+ * levels of rows that tests lay data out against; bit 6 has filtered searches
  * gather the allowed rows first whatever their number; without it any other bit, bit 5
  * of no other meaning too, has them read the mask as they scan. */
 int tv_debug_set_path(tv_index *ix, int force_full_lists);

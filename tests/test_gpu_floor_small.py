@@ -1,12 +1,12 @@
-"""Floors from a sample's best words: as long as the sample holds k blocks with a row that may be returned the answer comes from
-one sampled pass, below that from the ladder of rows, and it is the exact path's either way."""
+"""Floors from a sample's best words on indexes of any size: as long as the sample holds k blocks with a row that may be
+returned the answer comes from one sampled pass, below that from the ladder of rows, and it is the exact path's either way."""
 import numpy as np
 import pytest
 
 from helpers import bits_equal, unit_gaussian
 
 pytestmark = pytest.mark.gpu
-EXACT = 1
+EXACT, MASKED = 1, 32
 
 
 @pytest.fixture(scope="module")
@@ -14,6 +14,33 @@ def T():
     from turbovec_amd import _lib
     _lib.lib()
     return _lib
+
+
+# The smallest sample is every fourth block: k of them from 4 k blocks on.  The tile-group kernel, the all-queries one, tables in LDS, the
+# sparse table scan, and the largest k of a search without sampling.
+@pytest.mark.parametrize("dim,bits,nq,k", [(1536, 4, 64, 100), (512, 4, 200, 100), (1536, 2, 12, 100), (2048, 2, 150, 61), (640, 4, 64, 128)])
+def test_small_samples(T, dim, bits, nq, k):
+    ix = T.NativeIndex(dim, bits)
+    q = unit_gaussian(nq, dim, seed=2)
+    rng = np.random.default_rng(3)
+    rows = unit_gaussian(32 * (4 * k + 40), dim, seed=1)
+    n = 0
+    for add, one_level in ((32 * (4 * k - 1), False), (1, True), (31, True), (37, None), (32 * 39 - 5, None)):
+        ix.add(rows[n:n + add])
+        n += add
+        strides = ix.sampling_plan(nq, k)[0]
+        if one_level is not None and bits == 4:     # (tables: few (block, tile) pairs take another scan)
+            assert (strides[0] == 4 and len(strides) == 2) == one_level, strides
+        for m in (None, rng.random(n) < 0.5, (np.arange(n) >= 999) & (np.arange(n) < 999 + n // 3), rng.random(n) < 0.02):
+            words = None if m is None else T.pack_mask(m)[0]
+            out = []
+            for path in (0, MASKED, EXACT):
+                ix.set_path(path)
+                out.append(ix.search(q, k, mask_words=words))
+            ix.set_path(0)
+            for s, i in out[:2]:
+                assert np.array_equal(i, out[2][1]) and bits_equal(s, out[2][0])
+    ix.close()
 
 
 def test_a_range_of_rows_leaves_no_floor_open(T):

@@ -769,11 +769,14 @@ bool first_level_is_best_of_block(const tv_index *ix, const SampledPlan &plan, s
 // The other kernels have no floorless mode -- a second epilogue does not fit their registers -- but the scans of the unsampled
 // search keep every block's best score, and on a sample of the blocks those give a floor as good: one launch of
 // them and k_floor_of_best instead of two row-level samples, their selections and the second one's conditional
-// repeat.  From 16384 blocks (smaller indexes are searched without sampling).  Large or filtered batches of the matrix-unit
-// scan keep the row-level ladder: its floors cost them less than a sample of whole (block, tile) epilogues (889K x 920 2-bit, 640
-// queries: 1842 us with the ladder, 1884 without; 3M x 512 3-bit, 50 queries, 1 % allowed: 249 and 279).
+// repeat.  On indexes of any size that the unsampled search does not take, as long as the sample holds k_floor blocks with a row
+// that may be returned (us a search with the ladder, and so: 500K x 1536, 64 queries 175 and 137; 60K x 1536, 64 queries, k = 50 83
+// and 66; 16K x 1536, k = 100 70 and 58; 100K x 1536, 1000 queries, k = 100 541 and 340; 500K x 3072, 100 queries 415 and 294; 20K x
+// 1000 3-bit, 8 queries, k = 100 75 and 64; from fewer blocks floors stay open and queries are repeated: 20K x 640, 500 queries, k = 128).
+// Large or filtered batches of the matrix-unit scan keep the row-level ladder: its floors cost them less than a sample of whole (block, tile)
+// epilogues (889K x 920 2-bit, 640 queries: 1842 us with the ladder, 1884 without; 3M x 512 3-bit, 50 queries, 1 % allowed: 249 and 279).
 bool first_level_is_best_words(const tv_index *ix, const SampledPlan &plan, size_t n_blocks, size_t k_floor, bool masked) {
-    if (ix->row_ladder_left != 0 || k_floor > size_t(tv::kMaxPickK) || n_blocks <= 16384) return false;
+    if (ix->row_ladder_left != 0 || k_floor > size_t(tv::kMaxPickK) || n_blocks < 4 || (ix->no_direct && n_blocks <= 16384)) return false;
     if (ix->allowed.in_place) return false;      // (the best-of-block scans read whole blocks)
     if (effective_mode(ix) == TV_SCORE_P) return tv::best_serves(ix->geo.nch) && (plan.wide || plan.nt_batched > 0);
     return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && (!plan.lut_mx || (plan.cq_pad <= 160 && k_floor <= 64 && !masked));

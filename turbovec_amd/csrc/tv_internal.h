@@ -314,7 +314,7 @@ struct tv_index {
     int no_lut16 = 0;              // test hook: mode L batches stay on the scan with whole tables in LDS (8 queries per pass at most)
     bool no_lut_mx = false;        // for the length of a call: the scratch array holds only the sixteen-query passes' working set
     int no_wide = 0;               // test hook: large batches go through the tile-group kernels, not the wide one
-    int no_direct = 0;             // test hook: small indexes are sampled like large ones
+    int no_direct = 0;             // test hook: small indexes are sampled, those of up to 16384 blocks by levels of rows where there are such
     int no_gather = 0;             // test hook: filtered searches read the mask as they scan ...
     int force_gather = 0;          // ... or gather their allowed rows whatever their number
     size_t gathered_searches = 0, in_place_searches = 0;   // searches that ran on the allowed rows alone, and those of them that read all of their queries' rows in place
