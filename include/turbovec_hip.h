@@ -83,7 +83,9 @@ const char *tv_last_error(void);
  * the device's last index is destroyed.  When that is not enough, a failing
  * allocation also takes what the device's indexes keep of filtered searches'
  * allowed rows (tv_debug_workspace_bytes).  Other allocators of the process do
- * not see them. */
+ * not see them.  Calls on host arrays pass through pinned host memory that the
+ * device's indexes share too: allocated on first use, up to 256 MiB, freed with
+ * the last index. */
 int tv_index_create(int dim, int bits, int device, tv_index **out);
 int tv_index_destroy(tv_index *ix);
 

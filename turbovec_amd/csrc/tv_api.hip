@@ -238,7 +238,7 @@ int ensure_io(tv_index *ix, size_t bytes) { return ensure_block(ix, ix->io, ix->
 // on the calling thread -- the snapshot of them that the search then reads -- and read by the device where they lie,
 // results are written there by the last kernel; rows to add go through in pieces, several threads filling.  Through the Python
 // surface, before and now: one query over 100K x 128 73 us and 37, 1000 queries 138 and 101, 1024 of 3072 dimensions 2.41 ms and 1.22; 100K
-// x 1536 rows to an image 37.9 ms and 21.5.
+// x 1536 rows to an image 37.9 ms and 22.9.
 constexpr size_t kPinnedBytes = size_t(256) << 20, kPinnedLargest = size_t(32) << 20;
 constexpr size_t kReadInPlace = size_t(1) << 20;      // larger sets of queries are copied to the device first, by the copy engine
 
