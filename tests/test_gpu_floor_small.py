@@ -43,6 +43,22 @@ def test_small_samples(T, dim, bits, nq, k):
     ix.close()
 
 
+# 820 blocks and five tiles of queries are the fewest pairs the sparse table scan takes: a sample of 205 blocks
+@pytest.mark.parametrize("dim,bits,nq,k,n", [(1536, 2, 150, 61, 820 * 32), (1536, 2, 150, 64, 820 * 32 - 31), (1536, 3, 129, 62, 1500 * 32 + 1)])
+def test_small_samples_of_the_sparse_scan(T, dim, bits, nq, k, n):
+    ix = T.NativeIndex(dim, bits)
+    ix.add(unit_gaussian(n, dim, seed=5))
+    q = unit_gaussian(nq, dim, seed=6)
+    strides = ix.sampling_plan(nq, k)[0]
+    assert len(strides) == 2, strides
+    s, i = ix.search(q, k)
+    assert ix.queries_per_launch() == nq and ix.overflow_redos() == 0
+    ix.set_path(EXACT)
+    s2, i2 = ix.search(q, k)
+    assert np.array_equal(i, i2) and bits_equal(s, s2)
+    ix.close()
+
+
 def test_a_range_of_rows_leaves_no_floor_open(T):
     """Of 600,000 rows a sample of best words reads one block in eighteen: a range of 5 % has 52 such blocks, fewer than k.
     The search knows, and no query is repeated."""
