@@ -44,6 +44,18 @@ def test_every_row_width(T, oracle, dim, bits):
         assert np.array_equal(seq, want_seq) and bits_equal(scales, want)
 
 
+# every number of butterfly stages: within a lane, between lanes of a row of sixteen, between rows of sixteen, between a lane's
+# groups; rows that leave lanes and groups idle; a single row, and one more or less than workgroups hold
+@pytest.mark.parametrize("dim", [16, 32, 64, 128, 192, 256, 640, 768, 1024, 1040, 1792, 2560, 3464, 3584, 4096])
+def test_every_block_size(T, oracle, dim):
+    for n, bits in ((1, 4), (63, 3), (65, 2)):
+        v = unit_gaussian(n, dim, seed=dim + n) * np.float32(0.7)
+        v[0, 0] = 0.0
+        for cal in (None, (unit_gaussian(1, dim, seed=4)[0] * np.float32(0.1), np.linspace(2.0, 0.5, dim, dtype=np.float32))):
+            seq, scales, want_seq, want = encoded(T, oracle, v, bits, calibration=cal)
+            assert np.array_equal(seq, want_seq) and bits_equal(scales, want)
+
+
 # A pair with a large shift: the terms are some dim^(1/2) times larger than their sum, and about one row in 7000 (2048
 # dimensions) or 2500 (4096) lies closer to a rounding boundary than the two orders of addition can differ.
 @pytest.mark.parametrize("dim,n,shift", [(1536, 30_000, 1e8), (2048, 20_000, 1e8), (4096, 8_000, 1e8), (256, 4_000, 1e14)])

@@ -379,9 +379,9 @@ int upload_tables(tv_index *ix) {
                           ix->stream));
     TV_HIP(hipMemcpyAsync(ix->d_perms, ix->rot.perms.data(), 2 * dim * sizeof(uint32_t), hipMemcpyHostToDevice,
                           ix->stream));
-    std::vector<uint32_t> packed(dim);
-    ix->packed_ok = tv::encode_pack_tables(ix->rot.signs.data(), ix->rot.perms.data(), int(dim), packed.data());
-    if (ix->packed_ok) TV_HIP(hipMemcpyAsync(ix->d_packed, packed.data(), dim * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
+    std::vector<uint32_t> packed(2 * dim);
+    ix->packed_ok = tv::encode_pack_tables(ix->rot.signs.data(), ix->rot.perms.data(), int(dim), ix->rot.block, packed.data());
+    if (ix->packed_ok) TV_HIP(hipMemcpyAsync(ix->d_packed, packed.data(), 2 * dim * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
     float cen[16] = {0};
     for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
     TV_HIP(hipMemcpyAsync(ix->d_centroids, cen, sizeof cen, hipMemcpyHostToDevice, ix->stream));
@@ -1802,8 +1802,8 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
             size_t got = 0;
             return device_alloc(device, count * sizeof *p, reinterpret_cast<void **>(&p), &got) == hipSuccess;
         };
-        if (!table(ix->d_signs, 2 * size_t(dim)) || !table(ix->d_perms, 2 * size_t(dim)) || !table(ix->d_packed, size_t(dim)) ||
-            !table(ix->d_centroids, 16) || !table(ix->d_tq_shift, size_t(dim)) || !table(ix->d_tq_scale, size_t(dim)) ||
+        if (!table(ix->d_signs, 2 * size_t(dim)) || !table(ix->d_perms, 2 * size_t(dim)) || !table(ix->d_packed, 2 * size_t(dim)) ||
+            !table(ix->d_centroids, 16) || !table(ix->d_tq_shift, size_t(dim)) || !table(ix->d_tq_scale, 2 * size_t(dim)) ||
             !table(ix->d_tau_open, kTauOpenInts)) {
             rc = TV_ERR_HIP;
             break;
@@ -1903,10 +1903,14 @@ int tv_index_set_calibration(tv_index *ix, const float *shift, const float *scal
     TV_HIP(hipSetDevice(ix->device));
     const size_t dim = size_t(ix->geo.dim);
     if (!shift) { ix->tq_shift.clear(); ix->tq_scale.clear(); return TV_OK; }
+    std::unique_ptr<float[]> inverse(new (std::nothrow) float[dim]);      // (the encoder's, behind the scales)
+    if (!inverse) { g_last_error = "out of memory"; return TV_ERR_BAD_ARGUMENT; }
+    for (size_t j = 0; j < dim; ++j) inverse[j] = 1.0f / scale[j];
     ix->tq_shift.assign(shift, shift + dim);
     ix->tq_scale.assign(scale, scale + dim);
     TV_HIP(hipMemcpyAsync(ix->d_tq_shift, shift, dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
     TV_HIP(hipMemcpyAsync(ix->d_tq_scale, scale, dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
+    TV_HIP(hipMemcpyAsync(ix->d_tq_scale + dim, inverse.get(), dim * sizeof(float), hipMemcpyHostToDevice, ix->stream));
     TV_HIP(hipStreamSynchronize(ix->stream));
     return TV_OK;
 }

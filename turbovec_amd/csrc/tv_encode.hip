@@ -14,7 +14,7 @@
 //     rounding could depend on it.
 //
 // k_encode_rows takes rows of up to 4096 dimensions, a wave (or part of one) per
-// row and a group of eight waves' rows through each step together, so that the
+// row and a group of four waves' rows through each step together, so that the
 // sequential chains of all of them run side by side in the lanes of one or two
 // waves.  k_encode takes one workgroup per row: longer rows, the rotated rows of
 // a TQ+ fit, and tables whose signs are not +-1.
@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "tv_device.h"
@@ -159,21 +160,47 @@ __global__ __launch_bounds__(256) void k_encode(EncodeArgs a) {
 }
 
 // ---- rows of up to 4096 dimensions ------------------------------------------------------------
-// A row lies in LDS with eight floats of padding after every 64, and rows follow each other at a
-// stride of 8 modulo 64 floats: the passes below, whose lanes are 64 floats apart in groups of eight,
-// and the chains, whose lanes are a row apart, then spread over all banks.
-__host__ __device__ constexpr int enc_at(int j) { return j + (j >> 6) * 8; }
-// (and a row's place holds the f64 products of one run of its groups, 16 lanes floats, where enc_in_order needs it)
-static int enc_row_stride(int dim, int lanes) {
-    int s = std::max(enc_at(dim - 1) + 1, 16 * lanes + 16);
+// A row of L lanes lies in LDS as its lanes hold it, L groups of eight elements at a time: the groups' first four
+// elements side by side, then their last four, four floats of padding behind each.  A lane's two 16-byte pieces then go to
+// neighbouring places of their neighbours', and with rows at a stride of 8 modulo 64 floats the norm's chains, eight
+// of a row side by side and rows apart, spread over all banks.
+__host__ __device__ constexpr int enc_half(int L) { return 4 * L + 4; }
+__host__ __device__ constexpr int enc_at(int j, int L) { return ((j >> 3) / L) * 2 * enc_half(L) + ((j >> 2) & 1) * enc_half(L) + ((j >> 3) % L) * 4 + (j & 3); }
+// Lanes per row: a power of two, 8 to 64.
+static int enc_lanes(int dim) {
+    int lanes = 8;
+    while (lanes < 64 && lanes * 8 < dim) lanes *= 2;
+    return lanes;
+}
+// (a row's place also holds the f64 products of one run of its groups, 16 lanes floats, where enc_in_order needs it)
+__host__ __device__ constexpr int enc_row_stride(int dim, int lanes) {
+    int s = enc_at(dim - 1, lanes) + 1;
+    if (s < 16 * lanes + 16) s = 16 * lanes + 16;
     while (s % 64 != 8) ++s;
     return s;
 }
-// A position's entry of the packed rotation tables: where each round's gather reads (the padded place),
-// and the round's sign above it.
+// The butterfly stages between lanes whose numbers differ in one of the four lowest bits leave their upper element negated
+// (enc_lane_stage): the group g of a row comes out of a round with this sign.
+constexpr int kEncNegating = 4;
+__host__ __device__ inline bool enc_negated(int g, int log_block) {
+    const int stages = log_block - 3 < kEncNegating ? log_block - 3 : kEncNegating;
+#ifdef __HIP_DEVICE_COMPILE__
+    return __popc(unsigned(g) & ((1u << stages) - 1u)) & 1;
+#else
+    return __builtin_popcount(unsigned(g) & ((1u << stages) - 1u)) & 1;
+#endif
+}
+// Where the first round leaves element j: the stages between lanes 16 and 32 apart exchange an element's two lowest
+// bits with those of the lane (enc_swap_stage), and only the last round changes them back.
+__host__ __device__ constexpr int enc_at_swapped(int j, int L, int log_block) {
+    const int l = (j >> 3) % L, from4 = log_block > 7 ? ((l >> 4) ^ j) & 1 : 0, from5 = log_block > 8 ? ((l >> 5) ^ (j >> 1)) & 1 : 0;
+    return enc_at(j ^ (from4 | from5 << 1) ^ (from4 << 4 | from5 << 5) * 8, L);
+}
+// The packed rotation tables, a word per round and position: where the round's gather reads (the place in bytes) in the lower
+// half, the sign in the highest bit -- the second round's with the sign that the first leaves the element it reads with.
 constexpr int kEncMaxDim = 4096;
-static_assert(enc_at(kEncMaxDim - 1) < (1 << 15), "a padded place takes fifteen bits");
-bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint32_t *packed) {
+static_assert(enc_at(kEncMaxDim - 1, 64) * 4 < (1 << 16), "a place takes half a word");
+bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, int block, uint32_t *packed) {
     if (dim > kEncMaxDim) return false;
     // (a rotation keeps a row's length, which enc_slack counts on: both gathers must be permutations)
     for (int r = 0; r < 2; ++r) {
@@ -183,16 +210,85 @@ bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint
             seen[perms[size_t(r) * dim + j]] = true;
         }
     }
-    for (int j = 0; j < dim; ++j) {
-        uint32_t w = 0;
-        for (int r = 0; r < 2; ++r) {
-            const float s = signs[size_t(r) * dim + j];
-            if (s != 1.0f && s != -1.0f) return false;
-            w |= (uint32_t(enc_at(int(perms[size_t(r) * dim + j]))) | (s < 0.0f ? 0x8000u : 0u)) << (16 * r);
-        }
-        packed[j] = w;
+    const int lanes = enc_lanes(dim), log_block = __builtin_ctz(unsigned(block));
+    for (int j = 0; j < 2 * dim; ++j) {
+        const int from = int(perms[j]);
+        const bool second = j >= dim;
+        if (signs[j] != 1.0f && signs[j] != -1.0f) return false;
+        const bool minus = (signs[j] < 0.0f) != (second && enc_negated(from >> 3, log_block));
+        packed[j] = uint32_t(second ? enc_at_swapped(from, lanes, log_block) : enc_at(from, lanes)) * 4 | (minus ? 0x80000000u : 0u);
     }
     return true;
+}
+
+// A butterfly stage between lanes, on eight elements of each: lanes whose numbers differ in bit S hold the two ends.
+// The lower lane gets the sum, the upper one its own element less the lower lane's -- the difference, negated -- in one
+// fused operation by +1 or -1 (`side`, by the lane's bit S), whose product is exact.
+// Bit 2 of a lane's number in the row is the mirror image within eight lanes (enc_lane), which is what one step of the
+// data-parallel path can reach.  The wait states are those between a write and a read through that path.
+__device__ __forceinline__ int enc_lane(int t, int L) { return (t ^ ((t & 4) ? 3 : 0)) & (L - 1); }
+#define TV_LANE_STAGE(CTRL)                                                                                              \
+    asm volatile("s_nop 1\n\t"                                                                                          \
+                 "v_fmac_f32_dpp %0, %0, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %1, %1, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %2, %2, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %3, %3, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %4, %4, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %5, %5, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %6, %6, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                    \
+                 "v_fmac_f32_dpp %7, %7, %8 " CTRL " row_mask:0xf bank_mask:0xf"                                         \
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])         \
+                 : "v"(side))
+template <int S>
+__device__ __forceinline__ void enc_lane_stage(float (&v)[8], float side) {
+    static_assert(S < kEncNegating, "the lanes of a row of sixteen");
+    if constexpr (S == 0) TV_LANE_STAGE("quad_perm:[1,0,3,2]");
+    if constexpr (S == 1) TV_LANE_STAGE("quad_perm:[2,3,0,1]");
+    if constexpr (S == 2) TV_LANE_STAGE("row_half_mirror");
+    if constexpr (S == 3) TV_LANE_STAGE("row_ror:8");
+}
+#undef TV_LANE_STAGE
+// The same between lanes 16 (S = 4) or 32 (S = 5) apart: elements that differ in their number's bit S - 4 exchange halves,
+// so that a lane holds both ends of one of them, and unless the order they then have will do, change back (nothing is
+// negated).  Written out because the compiler copies the operands of every exchange.
+#define TV_SWAP_STAGE(SWAP, A0, A1, A2, A3, B0, B1, B2, B3)                                                              \
+    asm volatile("s_nop 1\n\t"                                                                                          \
+                 SWAP " %4, %8\n\t" SWAP " %5, %9\n\t" SWAP " %6, %10\n\t" SWAP " %7, %11\n\t"                        \
+                 "v_add_f32 %0, %4, %8\n\t" "v_sub_f32 %8, %4, %8\n\t"                                                 \
+                 "v_add_f32 %1, %5, %9\n\t" "v_sub_f32 %9, %5, %9\n\t"                                                 \
+                 "v_add_f32 %2, %6, %10\n\t" "v_sub_f32 %10, %6, %10\n\t"                                              \
+                 "v_add_f32 %3, %7, %11\n\t" "v_sub_f32 %11, %7, %11"                                                   \
+                 : "=&v"(s0), "=&v"(s1), "=&v"(s2), "=&v"(s3), "+v"(v[A0]), "+v"(v[A1]), "+v"(v[A2]), "+v"(v[A3]),       \
+                   "+v"(v[B0]), "+v"(v[B1]), "+v"(v[B2]), "+v"(v[B3]));                                                  \
+    if (back)                                                                                                            \
+        asm volatile("s_nop 1\n\t"                                                                                      \
+                     SWAP " %0, %4\n\t" SWAP " %1, %5\n\t" SWAP " %2, %6\n\t" SWAP " %3, %7"                          \
+                     : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3), "+v"(v[B0]), "+v"(v[B1]), "+v"(v[B2]), "+v"(v[B3]));      \
+    v[A0] = s0; v[A1] = s1; v[A2] = s2; v[A3] = s3
+template <int S>
+__device__ __forceinline__ void enc_swap_stage(float (&v)[8], bool back) {
+    float s0, s1, s2, s3;
+    if constexpr (S == 4) {
+        TV_SWAP_STAGE("v_permlane16_swap_b32", 0, 2, 4, 6, 1, 3, 5, 7);
+    } else {
+        TV_SWAP_STAGE("v_permlane32_swap_b32", 0, 1, 4, 5, 2, 3, 6, 7);
+    }
+}
+#undef TV_SWAP_STAGE
+// The sum of a row's lanes, in every one of them.
+__device__ __forceinline__ double enc_lane_sum(double x, int L) {
+    auto other = [](double y, auto ctrl) {
+        constexpr int c = decltype(ctrl)::value;
+        return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(y), c, 0xf, 0xf, false),
+                                __builtin_amdgcn_update_dpp(0, __double2loint(y), c, 0xf, 0xf, false));
+    };
+    x += other(x, IntC<0xB1>{});                      // quad_perm [1,0,3,2]
+    x += other(x, IntC<0x4E>{});                      // quad_perm [2,3,0,1]
+    x += other(x, IntC<0x141>{});                     // row_half_mirror
+    if (L > 8) x += other(x, IntC<0x128>{});          // row_ror:8
+    if (L > 16) x += __shfl_xor(x, 16);
+    if (L > 32) x += __shfl_xor(x, 32);
+    return x;
 }
 
 // Sixteen bytes of the caller's rows: a row starts where the caller's pointer says, so four-byte alignment is all
@@ -201,9 +297,9 @@ typedef float RowPiece __attribute__((ext_vector_type(4), aligned(4)));
 
 struct EncodeRowsArgs {
     const float *vecs;
-    const uint32_t *packed;   // dim entries (encode_pack_tables)
+    const uint32_t *packed;   // 2 * dim entries (encode_pack_tables)
     const float *shift;       // nullptr for the identity pair
-    const float *scale;
+    const float *scale;       // dim, and their reciprocals behind them
     float cen[16];
     float bnd[16];
     int dim, bits, G, nch, log_block;
@@ -228,17 +324,23 @@ __device__ __forceinline__ void enc_wave_sync() {
 // The number of boundaries below a value, from the cell it falls into: a rising map of values to kEncCells cells
 // leaves the boundaries of earlier cells below it and those of later cells not, so where no cell holds two
 // boundaries one comparison is left (15 boundaries: four levels of three comparisons before).
+// (The cell is the integer part of a float at which consecutive integers are neighbours: one fused operation rounds to it.
+// NaN goes to cell 0, where it exceeds nothing.)
 constexpr int kEncCells = 64;
+constexpr float kEncCellZero = 12582912.0f;
 struct EncCell { float bound; uint32_t below; };
-__host__ __device__ __forceinline__ int enc_cell(float x, float mul, float add) {
+__host__ __device__ __forceinline__ uint32_t enc_cell_bits(float x, float mul, float add) {
+    const float cell = fmaf(x, mul, add), last = kEncCellZero + float(kEncCells - 1);
 #ifdef __HIP_DEVICE_COMPILE__
-    uint32_t c;
-    asm("v_cvt_u32_f32 %0, %1" : "=v"(c) : "v"(fmaf(x, mul, add)));               // saturates; NaN: cell 0, where it exceeds nothing
-    return int(min(c, uint32_t(kEncCells - 1)));
+    return __float_as_uint(__builtin_amdgcn_fmed3f(cell, kEncCellZero, last));
 #else
-    return int(std::fmin(std::fmax(std::fmaf(x, mul, add), 0.0f), float(kEncCells - 1)));
+    const float in = std::fmin(std::fmax(cell, kEncCellZero), last);
+    uint32_t bits;
+    std::memcpy(&bits, &in, sizeof bits);
+    return bits;
 #endif
 }
+constexpr uint32_t kEncCellZeroBits = 0x4b400000u;
 // How far two orders of adding dim terms of the given total magnitude in f64 lie apart at most: dim / 4 + 3
 // roundings on the way of any term in the four chains (its product's among them), 8 NG + 6 in k_encode_rows, and the
 // few of the magnitude itself and of stepping this far to either side.
@@ -269,135 +371,147 @@ __device__ __forceinline__ float enc_in_order(const float (&v)[NG][8], const Rec
     return inner > 0.1 ? nrm / float(inner) : 0.0f;
 }
 
-// NG = groups of eight elements per lane; W = waves per workgroup.  The float work of a row is a few
-// thousand instructions of its wave, but its norm is a chain of 192 dependent f32 additions (1536 dimensions): a workgroup
+// NG = groups of eight elements per lane.  The float work of a row is 1160 vector instructions of its wave at 1536 dimensions,
+// half of them butterflies, and its norm is a chain of 192 dependent f32 additions: a workgroup
 // per row spent most of its time waiting for chains.  Here the norm chains of a workgroup's rows run in one wave, while
-// other workgroups of the CU are in their parallel part; the f64 sum needs no chain (enc_slack).  A row's rotation
-// goes through LDS three stages at a time in registers (the same additions in the same pairs), and its codes leave as
-// 16-byte stores that consecutive rows complete to whole lines.  100K rows of 1536 dimensions: 2.02 ms with a workgroup per
-// row, 0.50 with the f64 chains too in one wave and four levels of three comparisons per value, 0.39 now (1.8 TB/s, every
-// byte once); of 2048: 1.15 -> 0.62.
-// CAL: there is a TQ+ pair.
-constexpr int enc_waves_per_simd(int ng) { return ng == 1 ? 6 : ng == 2 ? 5 : ng <= 4 ? 4 : 2; }    // what their registers leave room for
-template <int NG, int W, bool CAL>
-__global__ __launch_bounds__(W * 64, enc_waves_per_simd(NG)) void k_encode_rows(EncodeRowsArgs a) {
+// other workgroups of the CU are in their parallel part; the f64 sum needs no chain (enc_slack).  A row is held in
+// registers and all stages of a round are done there (the same additions in the same pairs), between lanes through the
+// data-parallel path; it is in LDS for the norm and for the two gathers alone.  Its codes leave as
+// 16-byte stores that consecutive rows complete to whole lines.  The vector ALU bounds it, busy for 81 % of the clocks.  100K
+// rows of 1536 dimensions: 2.02 ms with a workgroup per row, 0.39 with the stages through LDS three at a time, 1.75K instructions a
+// row, 0.28 now (2.5 TB/s, every byte once); an add of 100K x 1024: 320 us before, 217 now, 30K x 4096: 1020 and 370, 77K x 1000 with a pair 420 and 205.
+// CAL: there is a TQ+ pair.  FULL: rows of NG * 512 dimensions, in blocks as large as they can be: every lane has NG groups and
+// all the stages are there, known at compile time.
+// Waves per workgroup: four, so that the workgroups of a CU are in different steps and the registers of a SIMD are dealt out
+// evenly (us an add with four and eight: 100K x 1536 315 and 319, 200K x 768 387 and 432, 100K x 1024 217 and 238; with six: 40K x 3072
+// 351 and 462; with two: 60K x 2048 264 and 270).
+constexpr int kEncWaves = 4;
+constexpr int enc_waves_per_simd(int ng, bool full) { return ng == 1 ? 6 : ng == 2 ? 5 : ng <= 4 ? 4 : ng <= 6 && !full ? 3 : 2; }    // what their registers leave room for
+template <int NG, bool CAL, bool FULL>
+__global__ __launch_bounds__(kEncWaves * 64, enc_waves_per_simd(NG, FULL)) void k_encode_rows(EncodeRowsArgs a) {
     extern __shared__ __align__(16) float enc_lds[];
-    const int dim = a.dim, t = threadIdx.x, ng = dim / 8, rs = a.row_stride, L = a.lanes;
-    const int R = W * 64 / L;                                      // rows of a workgroup
+    int t = threadIdx.x;
+    const int dim = FULL ? NG * 512 : a.dim, ng = dim / 8, L = FULL ? 64 : a.lanes;
+    const int rs = FULL ? enc_row_stride(NG * 512, 64) : a.row_stride, lb = FULL ? 9 + __builtin_ctz(NG) : a.log_block;
+    const int R = kEncWaves * 64 / L;                                      // rows of a workgroup
     uint32_t *s_codes = reinterpret_cast<uint32_t *>(enc_lds + R * rs);   // [R][ng] eight codes each, packed as in the index
-    float *s_part = reinterpret_cast<float *>(s_codes + R * ng);   // [R][8] chains of the squared norm
-    double *s_cen = reinterpret_cast<double *>(enc_lds + (R * rs + R * ng + 8 * R + 3) / 4 * 4);   // centroids in f64
-    const int r = t / L;                                           // this thread's row of the group ...
-    int l = t % L;                                                 // ... and its lane in the row
-    float *row = enc_lds + r * rs;
+    float2 *s_norm = reinterpret_cast<float2 *>(enc_lds + (R * rs + R * ng + 1) / 2 * 2);   // [R] norm and what rows are multiplied by
+    double *s_cen = reinterpret_cast<double *>(s_norm + R);        // centroids in f64
+    int r = t / L;                                                 // this thread's row of the group ...
+    int l = enc_lane(t, L);                                        // ... and its lane in the row
+    const int half = enc_half(L);
     EncCell *s_cell = reinterpret_cast<EncCell *>(s_cen + 16);
     if (t < 16) s_cen[t] = double(a.cen[t]);
     if (t < kEncCells) {
         // (the boundary of this cell, if it has one, and how many lie in the cells before it)
         EncCell cell{__int_as_float(0x7f800000), 0u};
         for (int b = 0; b < (1 << a.bits) - 1; ++b) {
-            const int k = enc_cell(a.bnd[b], a.cell_mul, a.cell_add);
+            const int k = int(enc_cell_bits(a.bnd[b], a.cell_mul, a.cell_add) - kEncCellZeroBits);
             if (k < t) ++cell.below;
             if (k == t) cell.bound = a.bnd[b];
         }
         s_cell[t] = cell;
     }
 
+    constexpr bool kFetchEarly = NG <= 3 && !(CAL && NG == 2);      // (longer rows, and a pair, leave no registers for it)
     const size_t n_groups = (a.n_new + R - 1) / R;
     RowPiece pre[NG][2];
     auto fetch = [&](size_t grp) {
-        const size_t rr = grp * R + r;
+        // (lanes without a row or a group of their own read the last one's)
+        const uint8_t *rows = reinterpret_cast<const uint8_t *>(a.vecs + grp * R * size_t(dim));
+        const int rr = int(min(size_t(r), a.n_new - 1 - grp * R));
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
-            const int g = l + i * L;
-            pre[i][0] = pre[i][1] = RowPiece{0.0f, 0.0f, 0.0f, 0.0f};
-            if (rr < a.n_new && g < ng) {
-                const RowPiece *src = reinterpret_cast<const RowPiece *>(a.vecs + rr * size_t(dim)) + 2 * g;
-                pre[i][0] = src[0];
-                pre[i][1] = src[1];
-            }
+            const RowPiece *src = reinterpret_cast<const RowPiece *>(rows + uint32_t(rr * dim + (FULL ? l + i * L : min(l + i * L, ng - 1)) * 8) * 4u);
+            pre[i][0] = src[0];
+            pre[i][1] = src[1];
         }
     };
-    // R stages from stride 2^S on, over this wave's rows; `last`: the scale is applied on the way out.
-    // Elements 2^S apart are a fixed distance apart in the padded row: 8 within a run of 64, nine
-    // eighths of their distance beyond.
-    auto pass = [&](auto ss, auto rr_, bool last) {
-        constexpr int S = decltype(ss)::value, N = 1 << decltype(rr_)::value, per = 8 / N;
-        constexpr int apart = S == 3 ? 8 : (1 << S) / 8 * 9;
-        asm volatile("" : "+v"(l));
-        enc_wave_sync();
+    // All butterfly stages of a round on the row's groups, in registers.  (Lanes without a group take part.)
+    const float side[4] = {l & 1 ? -1.0f : 1.0f, l & 2 ? -1.0f : 1.0f, l & 4 ? -1.0f : 1.0f, l & 8 ? -1.0f : 1.0f};
+    auto stages = [&](float (&v)[NG][8], bool back) {
+        auto each = [&](auto &&f) {
 #pragma unroll
-        for (int i = 0; i < per * NG; ++i) {
-            const int g = l + i * L;
-            if (g >= per * ng) continue;
-            float *at = row + enc_at(((g >> S) << S) * N + (g & ((1 << S) - 1)));
-            float v[N];
-#pragma unroll
-            for (int e = 0; e < N; ++e) v[e] = at[e * apart];
-            butterflies<decltype(rr_)::value>(v);
-            if (last) {
-#pragma unroll
-                for (int e = 0; e < N; ++e) v[e] = v[e] * a.inv_sqrt_block;
-            }
-#pragma unroll
-            for (int e = 0; e < N; ++e) at[e * apart] = v[e];
-        }
-    };
-    auto passes = [&](bool scaled) {
-        const int lb = a.log_block;
-        auto from = [&](auto ss) {
-            constexpr int S = decltype(ss)::value;
-            if (lb >= S + 3) pass(ss, IntC<3>{}, scaled && lb == S + 3);
-            else if (lb == S + 2) pass(ss, IntC<2>{}, scaled);
-            else if (lb == S + 1) pass(ss, IntC<1>{}, scaled);
+            for (int i = 0; i < NG; ++i) f(v[i]);
+            __builtin_amdgcn_sched_barrier(0);      // (one stage after the other, nothing loaded ahead: it would spill)
         };
-        from(IntC<3>{});
-        if (NG * 64 * 8 > 64) from(IntC<6>{});
-        if (lb > 9) from(IntC<9>{});
-        enc_wave_sync();
+        each([](float (&x)[8]) { butterflies<3>(x); });
+        if (lb > 3) each([&](float (&x)[8]) { enc_lane_stage<0>(x, side[0]); });
+        if (lb > 4) each([&](float (&x)[8]) { enc_lane_stage<1>(x, side[1]); });
+        if (lb > 5) each([&](float (&x)[8]) { enc_lane_stage<2>(x, side[2]); });
+        if (lb > 6) each([&](float (&x)[8]) { enc_lane_stage<3>(x, side[3]); });
+        if (lb > 7) each([&](float (&x)[8]) { enc_swap_stage<4>(x, back); });
+        if (lb > 8) each([&](float (&x)[8]) { enc_swap_stage<5>(x, back); });
+        static_for<3>([&](auto bb) {      // between a lane's groups
+            constexpr int far = 1 << decltype(bb)::value;
+            if constexpr (NG > far) {
+                if (lb > 9 + decltype(bb)::value) {
+#pragma unroll
+                    for (int i = 0; i < NG; ++i) {
+                        if ((i & far) != 0 || i + far >= NG) continue;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const float x = v[i][e], y = v[i + far][e];
+                            v[i][e] = x + y;
+                            v[i + far][e] = x - y;
+                        }
+                    }
+                }
+            }
+        });
     };
 
+    const float last_factor = enc_negated(l, lb) ? -a.inv_sqrt_block : a.inv_sqrt_block;
     size_t grp = blockIdx.x;
     if (grp < n_groups) fetch(grp);
     for (; grp < n_groups; grp += gridDim.x) {
         // (opaque in every turn and step: the addresses derived from it, kept in registers from one to
         // the next, would spill)
-        asm volatile("" : "+v"(l));
+        asm volatile("" : "+v"(l), "+v"(r), "+v"(t));
+        float *row = enc_lds + r * rs;
+        const uint32_t row_at = uint32_t(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) float *)row));
         uint32_t tab[NG][8];
+        auto fetch_table = [&](int round) {
 #pragma unroll
-        for (int i = 0; i < NG; ++i) {
-            const uint4 *src = reinterpret_cast<const uint4 *>(a.packed) + 2 * min(l + i * L, ng - 1);
-            const uint4 x = src[0], y = src[1];
-            tab[i][0] = x.x; tab[i][1] = x.y; tab[i][2] = x.z; tab[i][3] = x.w;
-            tab[i][4] = y.x; tab[i][5] = y.y; tab[i][6] = y.z; tab[i][7] = y.w;
-        }
-#pragma unroll
-        for (int i = 0; i < NG; ++i) {
-            const int g = l + i * L;
-            if (g < ng) {
-                float4 *dst = reinterpret_cast<float4 *>(row + enc_at(8 * g));
-                dst[0] = float4{pre[i][0].x, pre[i][0].y, pre[i][0].z, pre[i][0].w};
-                dst[1] = float4{pre[i][1].x, pre[i][1].y, pre[i][1].z, pre[i][1].w};
+            for (int i = 0; i < NG; ++i) {
+                const uint4 *src = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint8_t *>(a.packed + round * dim) + uint32_t(FULL ? l + i * L : min(l + i * L, ng - 1)) * 32u);
+                const uint4 x = src[0], y = src[1];
+                tab[i][0] = x.x; tab[i][1] = x.y; tab[i][2] = x.z; tab[i][3] = x.w;
+                tab[i][4] = y.x; tab[i][5] = y.y; tab[i][6] = y.z; tab[i][7] = y.w;
             }
-        }
+        };
+        fetch_table(0);
+        auto put = [&](int i, float4 x, float4 y) {
+            float *at = row + 4 * l + 2 * i * half;
+            if (FULL || l + i * L < ng) {
+                *reinterpret_cast<float4 *>(at) = x;
+                *reinterpret_cast<float4 *>(at + half) = y;
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NG; ++i)
+            put(i, float4{pre[i][0].x, pre[i][0].y, pre[i][0].z, pre[i][0].w}, float4{pre[i][1].x, pre[i][1].y, pre[i][1].z, pre[i][1].w});
         __syncthreads();
         // encode.rs:920-932: c[j % 8] += x * x (separate multiply and add), then the pairwise fold
-        for (int idx = t; idx < 8 * R; idx += W * 64) {
-            const float *x = enc_lds + (idx >> 3) * rs + (idx & 7);
+        for (int idx = t; idx < 8 * R; idx += kEncWaves * 64) {
+            const float *x = enc_lds + (idx >> 3) * rs + ((idx >> 2) & 1) * half + (idx & 3);
+            auto group = [&](int g) { return x + g / L * 2 * half + g % L * 4; };      // (eight from a multiple of eight on lie side by side)
             float c = 0.0f;
             int i = 0;
             if (ng >= 8) {
-                // eight groups of eight -- 64 floats and their padding -- at a time, the next ones on their way
+                // eight groups of eight at a time, the next ones on their way
                 float v[2][8];
-                auto load = [&](float (&to)[8], int at) {
+                auto load = [&](float (&to)[8], int g) {
+                    const float *from = group(g);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) to[e] = x[9 * at + 8 * e];
+                    for (int e = 0; e < 8; ++e) to[e] = from[4 * e];
                 };
                 auto add = [&](const float (&from)[8]) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) c = c + from[e] * from[e];
                 };
                 load(v[0], 0);
+#pragma unroll 1
                 for (; i + 24 <= ng; i += 16) {
                     load(v[1], i + 8);
                     add(v[0]);
@@ -408,73 +522,101 @@ __global__ __launch_bounds__(W * 64, enc_waves_per_simd(NG)) void k_encode_rows(
                 i += 8;
                 if (i + 8 <= ng) { load(v[1], i); add(v[1]); i += 8; }
             }
-            for (; i < ng; ++i) { const float v = x[8 * i + (i >> 3) * 8]; c = c + v * v; }
-            s_part[idx] = c;
+            for (; i < ng; ++i) { const float v = *group(i); c = c + v * v; }
+            // (a row's eight chains lie side by side; a + b is b + a)
+            c += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), 0xB1, 0xf, 0xf, false));
+            c += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), 0x4E, 0xf, 0xf, false));
+            c += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), 0x141, 0xf, 0xf, false));
+            const float nrm = sqrtf(c);
+            if ((idx & 7) == 0) s_norm[idx >> 3] = float2{nrm, nrm > 1e-10f ? 1.0f / nrm : 0.0f};   // lib.rs:163 MIN_INPUT_NORM
         }
         __syncthreads();
-        const float *p8 = s_part + r * 8;
-        const float nrm = sqrtf(((p8[0] + p8[1]) + (p8[2] + p8[3])) + ((p8[4] + p8[5]) + (p8[6] + p8[7])));
-        const float inv = nrm > 1e-10f ? 1.0f / nrm : 0.0f;   // lib.rs:163 MIN_INPUT_NORM
+        const float2 norm = s_norm[r];
+        const float nrm = norm.x, inv = norm.y;
 
         // rotation (rotation.rs:218-255): gather, sign, stages; the factor rides the gather
+        float v[NG][8];
 #pragma unroll
         for (int round = 0; round < 2; ++round) {
             asm volatile("" : "+v"(l));
-            const float factor = round == 0 ? inv : a.inv_sqrt_block;
-            float v[NG][8];
+            const uint32_t factor = __float_as_uint(round == 0 ? inv : a.inv_sqrt_block);
 #pragma unroll
             for (int i = 0; i < NG; ++i) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const uint32_t w = tab[i][e];
-                    const uint32_t at = round == 0 ? w & 0x7fffu : (w >> 16) & 0x7fffu;
-                    const uint32_t sign = (round == 0 ? w << 16 : w) & 0x80000000u;
-                    v[i][e] = __uint_as_float(__float_as_uint(row[at] * factor) ^ sign);     // (x * factor) * +-1
+                    uint32_t at;      // (the row's address and the word's lower half)
+                    asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(at) : "v"(row_at), "v"(w));
+                    const float x = *reinterpret_cast<const __attribute__((address_space(3))) float *>(uintptr_t(at));
+                    v[i][e] = x * __uint_as_float((factor & 0x7fffffffu) | (w & 0x80000000u));      // (x * factor) * +-1; no factor is negative
                 }
             }
             enc_wave_sync();                                       // every lane has gathered before any overwrites
-            if (NG <= 3 && round == 1 && grp + gridDim.x < n_groups) fetch(grp + gridDim.x);    // (longer rows leave no registers for it)
+            __builtin_amdgcn_sched_barrier(0);
+            if (round == 0) fetch_table(1);
+            if (kFetchEarly && round == 1 && grp + gridDim.x < n_groups) fetch(grp + gridDim.x);
+            __builtin_amdgcn_sched_barrier(0);
+            stages(v, round == 1);
+            if (round == 0) {
 #pragma unroll
-            for (int i = 0; i < NG; ++i) {
-                const int g = l + i * L;
-                butterflies<3>(v[i]);
-                if (round == 1 && a.log_block == 3) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * a.inv_sqrt_block;
-                }
-                if (g < ng) {
-                    float4 *dst = reinterpret_cast<float4 *>(row + enc_at(8 * g));
-                    dst[0] = float4{v[i][0], v[i][1], v[i][2], v[i][3]};
-                    dst[1] = float4{v[i][4], v[i][5], v[i][6], v[i][7]};
-                }
+                for (int i = 0; i < NG; ++i) put(i, float4{v[i][0], v[i][1], v[i][2], v[i][3]}, float4{v[i][4], v[i][5], v[i][6], v[i][7]});
+                enc_wave_sync();
             }
-            passes(round == 1);
+        }
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * last_factor;
         }
 
         // encode.rs:600-640: code = number of boundaries below the calibrated value
         asm volatile("" : "+v"(l));
-        float v[NG][8];
         uint32_t code4[NG];
+        // encode.rs:1442-1475: inner = <rotated, reconstruction> in f64, four chains by j % 4.  The row scale takes
+        // float(inner), so the order of the additions shows only where it moves inner across a rounding boundary: the
+        // lanes add their own elements, then each other's sums, and where every value within the two orders' distance
+        // gives the same row scale, that is it.
+        auto recon_of = [&](uint32_t code, int j) -> double {
+            double recon = s_cen[code];                                                        // (no TQ+ pair: * 1 - 0)
+            if constexpr (CAL) recon = recon * double(a.scale[dim + j]) - double(a.shift[j]);  // encode.rs:594
+            return recon;
+        };
+        double inner = 0.0, mass = 0.0;                            // the sum, and (for a pair) the sum of the terms' magnitudes
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
             const int g = l + i * L;
-            if (g >= ng) continue;
-            const float4 *src = reinterpret_cast<const float4 *>(row + enc_at(8 * g));
-            const float4 x = src[0], y = src[1];
-            v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
-            v[i][4] = y.x; v[i][5] = y.y; v[i][6] = y.z; v[i][7] = y.w;
+            if (!FULL && g >= ng) continue;
             uint32_t c[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            auto calibrated = [&](int e) {
                 float x = v[i][e];
                 if constexpr (CAL) x = (x + a.shift[8 * g + e]) * a.scale[8 * g + e];
-                if (a.cells) {
-                    const EncCell cell = s_cell[enc_cell(x, a.cell_mul, a.cell_add)];
+                return x;
+            };
+            if (a.cells) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = calibrated(e);
+                    const EncCell cell = s_cell[enc_cell_bits(x, a.cell_mul, a.cell_add) - kEncCellZeroBits];
                     c[e] = cell.below + (x > cell.bound ? 1u : 0u);
-                } else {
-                    c[e] = 0u;
-                    for (int b = 0; b < (1 << a.bits) - 1; ++b) c[e] += x > a.bnd[b] ? 1u : 0u;
+                    if (CAL && e == 3) __builtin_amdgcn_sched_barrier(0);
                 }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = calibrated(e);
+                    c[e] = 0u;
+#pragma unroll 1
+                    for (int b = 0; b < (1 << a.bits) - 1; ++b) c[e] += x > a.bnd[b] ? 1u : 0u;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (CAL) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const double recon = recon_of(c[e], 8 * g + e), x = double(v[i][e]);
+                inner = fma(x, recon, inner);
+                if constexpr (CAL) mass = fma(fabs(x), fabs(recon), mass);
+                if (e == 3) __builtin_amdgcn_sched_barrier(0);
             }
             code4[i] = c[0] | c[1] << 4 | c[2] << 8 | c[3] << 12 | c[4] << 16 | c[5] << 20 | c[6] << 24 | c[7] << 28;
             // pack.rs:264-282: first dimension in the high bits; 3-bit codes sit in 4-bit fields
@@ -482,46 +624,29 @@ __global__ __launch_bounds__(W * 64, enc_waves_per_simd(NG)) void k_encode_rows(
                                               : ((code4[i] >> 4) & 0x0f0f0f0fu) | ((code4[i] & 0x0f0f0f0fu) << 4);
             __builtin_amdgcn_sched_barrier(0);      // (one group after the other: several at once would spill)
         }
-        // encode.rs:1442-1475: inner = <rotated, reconstruction> in f64, four chains by j % 4.  The row scale takes
-        // float(inner), so the order of the additions shows only where it moves inner across a rounding boundary: the
-        // lanes add their own elements, then each other's sums, and where every value within the two orders' distance
-        // gives the same row scale, that is it.
-        auto recon_of = [&](int i, int e) -> double {
-            double recon = s_cen[(code4[i] >> (4 * e)) & 15u];                                 // (no TQ+ pair: * 1 - 0)
-            if constexpr (CAL) {
-                const int j = 8 * (l + i * L) + e;
-                recon = recon * double(1.0f / a.scale[j]) - double(a.shift[j]);                // encode.rs:594
-            }
-            return recon;
-        };
-        double inner = 0.0, mass = 0.0;                            // the sum, and (for a pair) the sum of the terms' magnitudes
-#pragma unroll
-        for (int i = 0; i < NG; ++i) {
-            if (l + i * L >= ng) continue;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const double recon = recon_of(i, e), x = double(v[i][e]);
-                inner = fma(x, recon, inner);
-                if constexpr (CAL) mass = fma(fabs(x), fabs(recon), mass);
-                if (e == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        for (int d = 1; d < L; d <<= 1) {
-            inner += __shfl_xor(inner, d);
-            if constexpr (CAL) mass += __shfl_xor(mass, d);
-        }
+        inner = enc_lane_sum(inner, L);
+        if constexpr (CAL) mass = enc_lane_sum(mass, L);
         const double slack = CAL ? enc_slack(dim, mass) : a.slack;
         const double lo = inner - slack, hi = inner + slack;
         float scale = lo > 0.1 ? nrm / float(lo) : 0.0f;                                       // encode.rs:1194-1200
         const bool settled = lo > 0.1 ? float(lo) == float(hi) : hi <= 0.1;                    // (NaN: not settled)
-        if (__any(!settled)) scale = enc_in_order<NG>(v, recon_of, row, dim, l, L, nrm);       // one row in 10^5
+        if (__any(!settled)) {                                                                 // one row in 10^5
+            // (opaque: what the sum above was made of, kept in registers for this, would spill)
+            asm volatile("" : "+v"(l));
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                asm volatile("" : "+v"(code4[i]));
+#pragma unroll
+                for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(v[i][e]));
+            }
+            scale = enc_in_order<NG>(v, [&](int i, int e) { return recon_of((code4[i] >> (4 * e)) & 15u, 8 * (l + i * L) + e); }, row, dim, l, L, nrm);
+        }
         if (l == 0 && grp * R + r < a.n_new) a.scales[a.old_n + grp * R + r] = scale;
         __syncthreads();                                           // every row's codes are there
         // the rows' code bytes, 16 at a time, into their lanes of the device layout (pack.rs:211-233
         // append_lanes); the bytes past a row's last group are zero there and stay so
         const int per = a.bits == 2 ? 8 : 4, pieces = (a.G + 15) / 16;
-        for (int idx = t; idx < R * pieces; idx += W * 64) {
+        for (int idx = t; idx < R * pieces; idx += kEncWaves * 64) {
             const int rr = idx % R, p = idx / R;
             const size_t vec = grp * R + rr;
             if (vec >= a.n_new) continue;
@@ -535,27 +660,34 @@ __global__ __launch_bounds__(W * 64, enc_waves_per_simd(NG)) void k_encode_rows(
             }
             *reinterpret_cast<uint4 *>(a.nat + enc_byte_index(a.old_n + vec, 16 * p, a.nch)) = uint4{o[0], o[1], o[2], o[3]};
         }
-        if (NG > 3 && grp + gridDim.x < n_groups) fetch(grp + gridDim.x);
+        if (!kFetchEarly && grp + gridDim.x < n_groups) fetch(grp + gridDim.x);
     }
 }
 
-template <int NG, int W, bool CAL>
-static hipError_t launch_encode_rows_cal(const EncodeRowsArgs &a, int device, hipStream_t s) {
-    const int R = W * 64 / a.lanes, ng = a.dim / 8;
-    const size_t lds = size_t(R * a.row_stride + R * ng + 8 * R + 4) * 4 + 16 * 8 + kEncCells * sizeof(EncCell);
+template <int NG, bool CAL, bool FULL>
+static hipError_t launch_encode_rows_full(const EncodeRowsArgs &a, int device, hipStream_t s) {
+    const int R = kEncWaves * 64 / a.lanes, ng = a.dim / 8;
+    const size_t lds = size_t(R * a.row_stride + R * ng + 2 * R + 2) * 4 + 16 * 8 + kEncCells * sizeof(EncCell);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    const void *kernel = reinterpret_cast<const void *>(k_encode_rows<NG, W, CAL>);
+    const void *kernel = reinterpret_cast<const void *>(k_encode_rows<NG, CAL, FULL>);
     hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     // a workgroup keeps its tables for all its turns: as many as are resident at once, by registers and LDS
     const size_t groups = (a.n_new + R - 1) / R;
-    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(4 * enc_waves_per_simd(NG)) / W, 160 * 1024 / lds));
-    hipLaunchKernelGGL((k_encode_rows<NG, W, CAL>), dim3(unsigned(std::min(groups, resident))), dim3(W * 64), lds, s, a);
+    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(4 * enc_waves_per_simd(NG, FULL)) / kEncWaves, 160 * 1024 / lds));
+    hipLaunchKernelGGL((k_encode_rows<NG, CAL, FULL>), dim3(unsigned(std::min(groups, resident))), dim3(kEncWaves * 64), lds, s, a);
     return hipGetLastError();
 }
-template <int NG, int W>
+template <int NG, bool CAL>
+static hipError_t launch_encode_rows_cal(const EncodeRowsArgs &a, int device, hipStream_t s) {
+    // (with a pair the straight-line code would spill)
+    if constexpr (!CAL)
+        if (a.dim == NG * 512 && a.log_block == 9 + __builtin_ctz(NG)) return launch_encode_rows_full<NG, CAL, true>(a, device, s);
+    return launch_encode_rows_full<NG, CAL, false>(a, device, s);
+}
+template <int NG>
 static hipError_t launch_encode_rows_n(const EncodeRowsArgs &a, int device, hipStream_t s) {
-    return a.scale != nullptr ? launch_encode_rows_cal<NG, W, true>(a, device, s) : launch_encode_rows_cal<NG, W, false>(a, device, s);
+    return a.scale != nullptr ? launch_encode_rows_cal<NG, true>(a, device, s) : launch_encode_rows_cal<NG, false>(a, device, s);
 }
 
 // A and B, one float row each; codes and the f64 products overlay A.  128 KiB at the largest
@@ -577,33 +709,29 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
         for (int i = 0; i < 16; ++i) { a.cen[i] = i < nl ? centroids[i] : 0.0f; a.bnd[i] = i < nl - 1 ? boundaries[i] : 0.0f; }
         a.dim = g.dim; a.bits = g.bits; a.G = g.G; a.nch = g.nch;
         a.log_block = __builtin_ctz(unsigned(block));
-        a.lanes = 8;
-        while (a.lanes < 64 && a.lanes * 8 < g.dim) a.lanes *= 2;
+        a.lanes = enc_lanes(g.dim);
         a.row_stride = enc_row_stride(g.dim, a.lanes);
         // cells of equal width from the first boundary to the last; no two boundaries may share one, and handed-over
         // centroids may be in any order, equal, infinite or NaN
         const int nb = nl - 1;
         a.cell_mul = float(kEncCells - 2) / (a.bnd[nb - 1] - a.bnd[0]);
-        a.cell_add = 1.0f - a.bnd[0] * a.cell_mul;
+        a.cell_add = 1.0f - a.bnd[0] * a.cell_mul + kEncCellZero;
         a.cells = a.cell_mul > 0.0f && a.cell_mul < 1e30f && std::fabs(a.cell_add) < 1e30f;
         for (int i = 0; a.cells && i + 1 < nb; ++i)
-            a.cells = a.bnd[i] < a.bnd[i + 1] && enc_cell(a.bnd[i], a.cell_mul, a.cell_add) < enc_cell(a.bnd[i + 1], a.cell_mul, a.cell_add);
+            a.cells = a.bnd[i] < a.bnd[i + 1] && enc_cell_bits(a.bnd[i], a.cell_mul, a.cell_add) < enc_cell_bits(a.bnd[i + 1], a.cell_mul, a.cell_add);
         // without a pair the terms are x * centroid over a row of length 1: |x c| <= (x^2 + c^2) / 2
         double c_max = 0.0;
         for (int i = 0; i < nl; ++i) c_max = std::fabs(double(centroids[i])) >= c_max ? std::fabs(double(centroids[i])) : c_max;
         a.slack = enc_slack(g.dim, (1.01 + double(g.dim) * c_max * c_max) / 2.0);
         a.inv_sqrt_block = inv_sqrt_block;
         a.nat = d_native; a.scales = d_scales; a.old_n = old_n; a.n_new = n_new;
-        // Waves per workgroup: a wave's worth of norm chains (eight rows) where two such workgroups fit a CU's LDS and
-        // registers, fewer where one would (ms for 300K x 2048 rows in three adds: 3.1 with eight, 2.23 with four, 2.13
-        // with two; 400K x 1024: 1.98 with six, 1.45 with four, 1.48 with two; 200K x 3072: 2.78 with four, 4.2 with two).
         switch ((g.dim / 8 + a.lanes - 1) / a.lanes) {
-            case 1: return launch_encode_rows_n<1, 8>(a, device, s);
-            case 2: return launch_encode_rows_n<2, 4>(a, device, s);
-            case 3: return launch_encode_rows_n<3, 8>(a, device, s);
-            case 4: return launch_encode_rows_n<4, 2>(a, device, s);
-            case 5: case 6: return launch_encode_rows_n<6, 4>(a, device, s);
-            default: return launch_encode_rows_n<8, 4>(a, device, s);
+            case 1: return launch_encode_rows_n<1>(a, device, s);
+            case 2: return launch_encode_rows_n<2>(a, device, s);
+            case 3: return launch_encode_rows_n<3>(a, device, s);
+            case 4: return launch_encode_rows_n<4>(a, device, s);
+            case 5: case 6: return launch_encode_rows_n<6>(a, device, s);
+            default: return launch_encode_rows_n<8>(a, device, s);
         }
     }
     EncodeArgs a;

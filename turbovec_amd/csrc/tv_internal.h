@@ -92,7 +92,7 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
 size_t encode_lds_bytes(int dim);
 // The rotation tables of both rounds in one word per position for the several-rows-per-workgroup
 // encoder; false where it does not apply (long rows, signs other than +-1, gathers that are no permutations).
-bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, uint32_t *packed);
+bool encode_pack_tables(const float *signs, const uint32_t *perms, int dim, int block, uint32_t *packed);
 hipError_t launch_move_lane(uint8_t *d_native, float *d_scales, const Geometry &g, size_t src, size_t dst,
                             hipStream_t s);
 
