@@ -384,16 +384,17 @@ __device__ __forceinline__ float enc_in_order(const float (&v)[NG][8], const Rec
 // all the stages are there, known at compile time.
 // Waves per workgroup: four, so that the workgroups of a CU are in different steps and the registers of a SIMD are dealt out
 // evenly (us an add with four and eight: 100K x 1536 315 and 319, 200K x 768 387 and 432, 100K x 1024 217 and 238; with six: 40K x 3072
-// 351 and 462; with two: 60K x 2048 264 and 270).
-constexpr int kEncWaves = 4;
+// 351 and 462; with two: 60K x 2048 264 and 270); eight where a wave has several rows (400K x 128 120 and 121).
+constexpr int enc_waves(int ng) { return ng == 1 ? 8 : 4; }
 constexpr int enc_waves_per_simd(int ng, bool full) { return ng == 1 ? 6 : ng == 2 ? 5 : ng <= 4 ? 4 : ng <= 6 && !full ? 3 : 2; }    // what their registers leave room for
 template <int NG, bool CAL, bool FULL>
-__global__ __launch_bounds__(kEncWaves * 64, enc_waves_per_simd(NG, FULL)) void k_encode_rows(EncodeRowsArgs a) {
+__global__ __launch_bounds__(enc_waves(NG) * 64, enc_waves_per_simd(NG, FULL)) void k_encode_rows(EncodeRowsArgs a) {
     extern __shared__ __align__(16) float enc_lds[];
     int t = threadIdx.x;
     const int dim = FULL ? NG * 512 : a.dim, ng = dim / 8, L = FULL ? 64 : a.lanes;
     const int rs = FULL ? enc_row_stride(NG * 512, 64) : a.row_stride, lb = FULL ? 9 + __builtin_ctz(NG) : a.log_block;
-    const int R = kEncWaves * 64 / L;                                      // rows of a workgroup
+    constexpr int kThreads = enc_waves(NG) * 64;
+    const int R = kThreads / L;                                      // rows of a workgroup
     uint32_t *s_codes = reinterpret_cast<uint32_t *>(enc_lds + R * rs);   // [R][ng] eight codes each, packed as in the index
     float2 *s_norm = reinterpret_cast<float2 *>(enc_lds + (R * rs + R * ng + 1) / 2 * 2);   // [R] norm and what rows are multiplied by
     double *s_cen = reinterpret_cast<double *>(s_norm + R);        // centroids in f64
@@ -493,7 +494,7 @@ __global__ __launch_bounds__(kEncWaves * 64, enc_waves_per_simd(NG, FULL)) void 
             put(i, float4{pre[i][0].x, pre[i][0].y, pre[i][0].z, pre[i][0].w}, float4{pre[i][1].x, pre[i][1].y, pre[i][1].z, pre[i][1].w});
         __syncthreads();
         // encode.rs:920-932: c[j % 8] += x * x (separate multiply and add), then the pairwise fold
-        for (int idx = t; idx < 8 * R; idx += kEncWaves * 64) {
+        for (int idx = t; idx < 8 * R; idx += kThreads) {
             const float *x = enc_lds + (idx >> 3) * rs + ((idx >> 2) & 1) * half + (idx & 3);
             auto group = [&](int g) { return x + g / L * 2 * half + g % L * 4; };      // (eight from a multiple of eight on lie side by side)
             float c = 0.0f;
@@ -646,7 +647,7 @@ __global__ __launch_bounds__(kEncWaves * 64, enc_waves_per_simd(NG, FULL)) void 
         // the rows' code bytes, 16 at a time, into their lanes of the device layout (pack.rs:211-233
         // append_lanes); the bytes past a row's last group are zero there and stay so
         const int per = a.bits == 2 ? 8 : 4, pieces = (a.G + 15) / 16;
-        for (int idx = t; idx < R * pieces; idx += kEncWaves * 64) {
+        for (int idx = t; idx < R * pieces; idx += kThreads) {
             const int rr = idx % R, p = idx / R;
             const size_t vec = grp * R + rr;
             if (vec >= a.n_new) continue;
@@ -666,7 +667,8 @@ __global__ __launch_bounds__(kEncWaves * 64, enc_waves_per_simd(NG, FULL)) void 
 
 template <int NG, bool CAL, bool FULL>
 static hipError_t launch_encode_rows_full(const EncodeRowsArgs &a, int device, hipStream_t s) {
-    const int R = kEncWaves * 64 / a.lanes, ng = a.dim / 8;
+    constexpr int kThreads = enc_waves(NG) * 64;
+    const int R = kThreads / a.lanes, ng = a.dim / 8;
     const size_t lds = size_t(R * a.row_stride + R * ng + 2 * R + 2) * 4 + 16 * 8 + kEncCells * sizeof(EncCell);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     const void *kernel = reinterpret_cast<const void *>(k_encode_rows<NG, CAL, FULL>);
@@ -674,8 +676,8 @@ static hipError_t launch_encode_rows_full(const EncodeRowsArgs &a, int device, h
     if (e != hipSuccess) return e;
     // a workgroup keeps its tables for all its turns: as many as are resident at once, by registers and LDS
     const size_t groups = (a.n_new + R - 1) / R;
-    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(4 * enc_waves_per_simd(NG, FULL)) / kEncWaves, 160 * 1024 / lds));
-    hipLaunchKernelGGL((k_encode_rows<NG, CAL, FULL>), dim3(unsigned(std::min(groups, resident))), dim3(kEncWaves * 64), lds, s, a);
+    const size_t resident = size_t(device_cus(device)) * std::max<size_t>(1, std::min<size_t>(size_t(4 * enc_waves_per_simd(NG, FULL)) / enc_waves(NG), 160 * 1024 / lds));
+    hipLaunchKernelGGL((k_encode_rows<NG, CAL, FULL>), dim3(unsigned(std::min(groups, resident))), dim3(kThreads), lds, s, a);
     return hipGetLastError();
 }
 template <int NG, bool CAL>
