@@ -94,3 +94,41 @@ def test_rows_with_values_that_are_no_numbers(T, oracle):
     packed, want = oracle.encode(oracle.Rotation(dim), v, 4)
     assert np.array_equal(seq, oracle.repack_seq(packed, n, 4, dim))
     assert np.array_equal(np.isnan(scales), np.isnan(want)) and bits_equal(scales[~np.isnan(want)], want[~np.isnan(want)])
+
+
+class _Bytes:
+    """Device memory as torch takes it."""
+
+    def __init__(self, ptr, count):
+        self.__cuda_array_interface__ = dict(shape=(count,), typestr="|u1", data=(ptr, False), version=2)
+
+
+@pytest.mark.parametrize("dim,bits,pieces", [(1000, 4, (20_000, 33, 40_000, 1)), (1536, 2, (40_000, 31, 64, 9_000)), (4104, 4, (3_000, 100, 4_000))])
+def test_grown_indexes_hold_nothing_else(T, dim, bits, pieces):
+    """Rows added in pieces to an index that grows into memory another one gave up: padding, lanes without a row and scales
+    are those of an index uploaded whole, and rows appended later land in cleared blocks."""
+    torch = pytest.importorskip("torch")
+    n = sum(pieces)
+    x = torch.randn(2 * n, dim, device="cuda")
+    torch.cuda.synchronize()
+    dirty = T.NativeIndex(dim, bits)
+    dirty.add_dev(x.data_ptr(), 2 * n)
+    dirty.close()
+    ix, at = T.NativeIndex(dim, bits), 0
+    for rows in pieces:
+        ix.add_dev(x[at:].data_ptr(), rows)
+        at += rows
+    seq, scales = ix.download_seq()
+    whole = T.NativeIndex(dim, bits)
+    whole.upload_seq(seq, n, scales)
+
+    def contents(index):
+        codes, row_scales, code_bytes = index.device_ptrs()
+        return [torch.as_tensor(_Bytes(p, b), device="cuda").cpu().numpy() for p, b in ((codes, code_bytes), (row_scales, (len(index) + 31) // 32 * 128))]
+
+    for index in (ix, whole):
+        index.append_rows(np.full((1, index.n_byte_groups), 0x55, np.uint8), np.ones(1, np.float32))
+    for got, want in zip(contents(ix), contents(whole)):
+        assert np.array_equal(got, want)
+    ix.close()
+    whole.close()

@@ -310,41 +310,79 @@ bool copy_checked(float *to, const float *from, size_t n) {
     return any != 0;
 }
 
-int ensure_capacity(tv_index *ix, size_t n_vectors) {
+// The allocations of an index that has grown, which the copy out of them may still be reading: given up once the
+// index's stream has been waited for.
+struct Outgrown {
+    tv_index *ix;
+    uint8_t *codes = nullptr;
+    float *scales = nullptr;
+    size_t codes_bytes = 0, scales_bytes = 0;
+    explicit Outgrown(tv_index *ix_) : ix(ix_) {}
+    Outgrown(const Outgrown &) = delete;
+    hipError_t release() {
+        const hipError_t c = device_free(ix->device, std::exchange(codes, nullptr), codes_bytes);
+        const hipError_t s = device_free(ix->device, std::exchange(scales, nullptr), scales_bytes);
+        return c != hipSuccess ? c : s;
+    }
+    ~Outgrown() {
+        if (codes == nullptr && scales == nullptr) return;
+        (void)hipStreamSynchronize(ix->stream);
+        (void)release();
+    }
+};
+// Room for n_vectors rows.  An index grows to twice its size while that is less than kGrowth more, and by half beyond, or
+// as far as there is memory: 100K rows of 1536 dimensions added four times move 231 MB on the way (461 MB by half each time).
+// What is beyond the rows is zero -- but for the blocks that rows from the index's last to n_vectors fill, where the
+// caller says that it is about to write all of those on the index's stream (`whole`), and not before it has waited for the
+// stream, which it does before `outgrown` goes.
+constexpr size_t kGrowth = size_t(1) << 30;
+int ensure_capacity(tv_index *ix, size_t n_vectors, Outgrown &outgrown, bool whole) {
     const size_t blocks = (n_vectors + tv::kVecBlock - 1) / tv::kVecBlock;
     if (blocks <= ix->cap_blocks) return TV_OK;
-    size_t cap = std::max(blocks, ix->cap_blocks + ix->cap_blocks / 2);
+    const size_t bb = ix->geo.block_bytes();
+    size_t cap = std::max(blocks, ix->cap_blocks + std::max(ix->cap_blocks / 2, std::min(ix->cap_blocks, kGrowth / bb)));
     cap = std::max<size_t>(cap, 64);
     uint8_t *codes = nullptr;
     float *scales = nullptr;
-    const size_t bb = ix->geo.block_bytes();
     size_t codes_bytes = 0, scales_bytes = 0;
-    TV_HIP(device_alloc(ix->device, cap * bb, reinterpret_cast<void **>(&codes), &codes_bytes));
-    {
-        const hipError_t e = device_alloc(ix->device, cap * tv::kVecBlock * sizeof(float), reinterpret_cast<void **>(&scales), &scales_bytes);
-        if (e != hipSuccess) {
+    hipError_t e = hipSuccess;
+    for (;; cap = std::max<size_t>(blocks, 64)) {
+        e = device_alloc(ix->device, cap * bb, reinterpret_cast<void **>(&codes), &codes_bytes);
+        if (e == hipSuccess) {
+            e = device_alloc(ix->device, cap * tv::kVecBlock * sizeof(float), reinterpret_cast<void **>(&scales), &scales_bytes);
+            if (e == hipSuccess) break;
             (void)device_free(ix->device, codes, codes_bytes);
-            return fail_hip(e, "device_alloc(scales)");
         }
+        if (cap == std::max<size_t>(blocks, 64)) return fail_hip(e, "device_alloc(rows)");
     }
     const size_t old_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
+    const size_t clear = whole ? std::max(old_blocks, n_vectors / tv::kVecBlock) : old_blocks;
     // fresh bytes are zero so padding lanes match a from-scratch upload
-    TV_HIP(hipMemsetAsync(codes + old_blocks * bb, 0, (cap - old_blocks) * bb, ix->stream));
-    TV_HIP(hipMemsetAsync(scales + old_blocks * tv::kVecBlock, 0,
-                          (cap - old_blocks) * tv::kVecBlock * sizeof(float), ix->stream));
-    if (old_blocks) {
-        TV_HIP(hipMemcpyAsync(codes, ix->d_codes, old_blocks * bb, hipMemcpyDeviceToDevice, ix->stream));
-        TV_HIP(hipMemcpyAsync(scales, ix->d_scales, old_blocks * tv::kVecBlock * sizeof(float),
-                              hipMemcpyDeviceToDevice, ix->stream));
+    e = hipMemsetAsync(codes + clear * bb, 0, (cap - clear) * bb, ix->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(scales + clear * tv::kVecBlock, 0, (cap - clear) * tv::kVecBlock * sizeof(float), ix->stream);
+    if (e == hipSuccess && old_blocks) {
+        e = hipMemcpyAsync(codes, ix->d_codes, old_blocks * bb, hipMemcpyDeviceToDevice, ix->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(scales, ix->d_scales, old_blocks * tv::kVecBlock * sizeof(float), hipMemcpyDeviceToDevice, ix->stream);
     }
-    TV_HIP(hipStreamSynchronize(ix->stream));
-    TV_HIP(device_free(ix->device, ix->d_codes, ix->codes_bytes));
-    TV_HIP(device_free(ix->device, ix->d_scales, ix->scales_bytes));
-    ix->d_codes = codes;
-    ix->d_scales = scales;
-    ix->codes_bytes = codes_bytes;
-    ix->scales_bytes = scales_bytes;
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(ix->stream);
+        (void)device_free(ix->device, codes, codes_bytes);
+        (void)device_free(ix->device, scales, scales_bytes);
+        return fail_hip(e, "growing the index");
+    }
+    outgrown.codes = std::exchange(ix->d_codes, codes);
+    outgrown.scales = std::exchange(ix->d_scales, scales);
+    outgrown.codes_bytes = std::exchange(ix->codes_bytes, codes_bytes);
+    outgrown.scales_bytes = std::exchange(ix->scales_bytes, scales_bytes);
     ix->cap_blocks = cap;
+    return TV_OK;
+}
+int ensure_capacity(tv_index *ix, size_t n_vectors) {
+    Outgrown outgrown(ix);
+    const int rc = ensure_capacity(ix, n_vectors, outgrown, false);
+    if (rc != TV_OK || ix->d_codes == nullptr) return rc;
+    TV_HIP(hipStreamSynchronize(ix->stream));
+    TV_HIP(outgrown.release());
     return TV_OK;
 }
 
@@ -2033,16 +2071,24 @@ static int encode_rows(tv_index *ix, const float *d_vectors, size_t n_new, size_
     return TV_OK;
 }
 
+static int clear_slots(tv_index *ix, size_t end);
+
 int tv_index_add_dev(tv_index *ix, const float *d_vectors, size_t n_new) {
     if (!ix || (n_new && !d_vectors)) return TV_ERR_BAD_ARGUMENT;
     if (n_new == 0) return TV_OK;
     std::lock_guard<std::mutex> lock(ix->mu);
     TV_HIP(hipSetDevice(ix->device));
     if (ix->n + n_new >= (size_t(1) << 31)) return TV_ERR_BAD_ARGUMENT;
-    int rc = ensure_capacity(ix, ix->n + n_new);
+    Outgrown outgrown(ix);
+    int rc = ensure_capacity(ix, ix->n + n_new, outgrown, ix->packed_ok);
     if (rc != TV_OK) return rc;
-    rc = encode_rows(ix, d_vectors, n_new, ix->n);
-    if (rc == TV_OK) ix->n += n_new;
+    rc = encode_rows(ix, d_vectors, n_new, ix->n);      // (waits for the stream)
+    if (rc == TV_OK) {
+        ix->n += n_new;
+        TV_HIP(outgrown.release());
+    } else {
+        (void)clear_slots(ix, ix->n + n_new);
+    }
     return rc;
 }
 

@@ -302,7 +302,7 @@ struct EncodeRowsArgs {
     const float *scale;       // dim, and their reciprocals behind them
     float cen[16];
     float bnd[16];
-    int dim, bits, G, nch, log_block;
+    int dim, bits, nch, log_block;
     int lanes;                // lanes per row: a power of two, 8 to 64
     int row_stride;           // floats
     int cells;                // boundaries found by cell (enc_cells) instead of one by one
@@ -645,8 +645,8 @@ __global__ __launch_bounds__(enc_waves(NG) * 64, enc_waves_per_simd(NG, FULL)) v
         if (l == 0 && grp * R + r < a.n_new) a.scales[a.old_n + grp * R + r] = scale;
         __syncthreads();                                           // every row's codes are there
         // the rows' code bytes, 16 at a time, into their lanes of the device layout (pack.rs:211-233
-        // append_lanes); the bytes past a row's last group are zero there and stay so
-        const int per = a.bits == 2 ? 8 : 4, pieces = (a.G + 15) / 16;
+        // append_lanes), the bytes past a row's last group zero: nothing need have been cleared for a row
+        const int per = a.bits == 2 ? 8 : 4, pieces = 2 * a.nch;
         for (int idx = t; idx < R * pieces; idx += kThreads) {
             const int rr = idx % R, p = idx / R;
             const size_t vec = grp * R + rr;
@@ -709,7 +709,7 @@ hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const 
         a.vecs = d_vecs; a.packed = d_packed; a.shift = d_shift; a.scale = d_scale;
         const int nl = 1 << g.bits;
         for (int i = 0; i < 16; ++i) { a.cen[i] = i < nl ? centroids[i] : 0.0f; a.bnd[i] = i < nl - 1 ? boundaries[i] : 0.0f; }
-        a.dim = g.dim; a.bits = g.bits; a.G = g.G; a.nch = g.nch;
+        a.dim = g.dim; a.bits = g.bits; a.nch = g.nch;
         a.log_block = __builtin_ctz(unsigned(block));
         a.lanes = enc_lanes(g.dim);
         a.row_stride = enc_row_stride(g.dim, a.lanes);

@@ -84,6 +84,7 @@ hipError_t launch_native_to_seq(const uint8_t *d_native, uint8_t *d_seq, const G
                                 size_t n_blocks, size_t block_bytes, const float *d_scales, hipStream_t s);
 hipError_t launch_append_rows(const uint8_t *d_rows, uint8_t *d_native, const Geometry &g, size_t old_n,
                               size_t n_new, hipStream_t s);
+// With d_packed every byte of the rows' lanes is written, and their scales; without, the padding behind a row's last group is not.
 hipError_t launch_encode(const float *d_vecs, size_t n_new, size_t old_n, const float *d_signs,
                          const uint32_t *d_perms, const uint32_t *d_packed, const float *d_shift, const float *d_scale,
                          const float *centroids, const float *boundaries, const Geometry &g, int block,
