@@ -75,6 +75,28 @@ def test_ties_and_wild_row_scales(T, oracle, dim, nq):
     ix.close()
 
 
+@pytest.mark.parametrize("nq", [2, 300])
+def test_best_blocks_in_any_place(T, oracle, nq):
+    """More blocks that tie than are ranked as they are, and allowed rows in blocks a thousand apart only, which one thread of the
+    selection holds: no more are taken for the best than are."""
+    n, dim = 70_000, 64
+    v = unit_gaussian(n, dim, seed=21)
+    v[:40_000] = v[0]
+    oidx = OracleIndex(oracle, dim, 4, v)
+    q = np.concatenate([v[:1] + np.float32(0.01) * unit_gaussian(1, dim, seed=22), unit_gaussian(nq - 1, dim, seed=23)])
+    ix = to_native(T, oidx)
+    block = np.arange(n) // 32
+    for m in (None, block % 1024 == 3, (block % 256 == 5) & (np.arange(n) % 32 == 7)):
+        words = None if m is None else T.pack_mask(m)[0]
+        for k in (1, 16, 17, 100):
+            assert unsampled(ix, nq, k, m)
+            s, i = ix.search(q, k, mask_words=words)
+            os_, oi = oidx.search(q, k, mask_words=words)
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
+    assert ix.overflow_redos() == 0
+    ix.close()
+
+
 @pytest.mark.parametrize("k", [3, 10, 60])
 def test_rows_that_score_minus_infinity(T, oracle, k):
     """Row scales that take most rows' scores beyond the float range: the blocks of the few finite rows hold -infinity

@@ -190,6 +190,41 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
     return nt == 1 ? launch_best_u<1, false>(a, nj, device, s) : nt == 2 ? launch_best_u<2, false>(a, nj, device, s) : launch_best_u<4, false>(a, nj, device, s);
 }
 
+// The keys whose score words reach `least`, which at least `need` of all keys do or which is 1, into kept, two zeros behind
+// them: how many.  Where they are too many for it, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
+// behind a barrier that comes between; met by all T threads.
+template <uint32_t T, typename Each>
+__device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, uint32_t need, uint64_t *kept, uint32_t &n_kept, SelectShared &sh) {
+    const uint32_t t = threadIdx.x;
+    each([&](uint64_t k) {
+        if (uint32_t(k >> 32) < least) return;
+        const uint32_t at = atomicAdd(&n_kept, 1u);
+        if (at < kSelectKept) kept[at] = k;
+    });
+    __syncthreads();
+    uint32_t n = n_kept;
+    if (n > kSelectKept) {
+        for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
+        uint32_t hi_max = 0u, hi_min_inv = 0u, mx, mn_inv;
+        each([&](uint64_t k) {
+            hi_max = max(hi_max, uint32_t(k >> 32));
+            hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+        });
+        select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);       // (everyone has read n_kept)
+        const uint64_t threshold = select_threshold<T>(each, mx, mn_inv, need, sh);
+        if (t == 0) n_kept = 0u;
+        __syncthreads();
+        each([&](uint64_t k) {
+            if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
+        });
+        __syncthreads();
+        n = n_kept;
+    }
+    if (t < 2u) kept[n + t] = 0ull;
+    __syncthreads();
+    return n;
+}
+
 // ===========================================================================
 // The floor a sample's best rows give: a workgroup per query takes the k_floor-th best of the sampled blocks' best
 // scores, which k_floor scanned rows reach.
@@ -197,48 +232,32 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
 constexpr uint32_t kFloorThreads = 512, kFloorHeld = kMaxFloorBlocks / kFloorThreads;
 __global__ __launch_bounds__(kFloorThreads) void k_floor_of_best(const uint32_t *__restrict__ words, uint32_t stride, uint32_t n, uint32_t k_floor,
                                                         int *tau_out, int tau_stride_q, uint64_t *stamp) {
-    constexpr uint32_t T = kFloorThreads, W = T / 64;
+    constexpr uint32_t T = kFloorThreads;
     __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ SelectShared sh;
+    __shared__ TopShared top;
     __shared__ uint32_t n_kept;
-    const uint32_t qi = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    const uint32_t qi = blockIdx.x, t = threadIdx.x;
     const uint32_t *best = words + size_t(qi) * stride;
     uint32_t v[kFloorHeld];
 #pragma unroll
     for (uint32_t e = 0; e < kFloorHeld; ++e) v[e] = e * T + t < n ? best[e * T + t] : 0u;
-    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     if (t == 0) n_kept = 0u;
+    uint32_t most = 0u;
+#pragma unroll
+    for (uint32_t e = 0; e < kFloorHeld; ++e) most = max(most, v[e]);
     auto each = [&](auto &&f) {
 #pragma unroll
         for (uint32_t e = 0; e < kFloorHeld; ++e)
             if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
     };
-    uint32_t mine = 0u, hi_max = 0u, hi_min_inv = 0u, mx, mn_inv, total = 0u;
-    each([&](uint64_t k) {
-        ++mine;
-        hi_max = max(hi_max, uint32_t(k >> 32));
-        hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
-    });
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) mine += __shfl_xor(mine, d);
-    if (lane == 0) sh.w_sum[wv] = mine;
-    select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
-    for (uint32_t w = 0; w < W; ++w) total += sh.w_sum[w];
-    __syncthreads();
+    const uint32_t n_of = keep_best<T>(each, select_top<T>(most, k_floor, top), k_floor, kept, n_kept, sh);
     int *out = tau_out + (qi / uint32_t(tau_stride_q)) * kQTile + qi % uint32_t(tau_stride_q);
-    if (total < k_floor) {      // (a mask that leaves the sample too few rows)
+    if (n_of < k_floor) {      // (a mask that leaves the sample too few rows)
         if (t == 0) *out = kTauInit;
     } else {
-        const uint64_t threshold = total > kSelectKept ? select_threshold<T>(each, mx, mn_inv, k_floor, sh) : 0ull;
-        each([&](uint64_t k) {
-            if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
-        });
-        __syncthreads();
-        const uint32_t m = n_kept;
-        if (t < 2u) kept[m + t] = 0ull;
-        __syncthreads();
-        for (uint32_t i = t; i < m; i += T)
-            if (rank_in(kept, m, kept[i]) + 1u == k_floor) *out = int(uint32_t(kept[i] >> 32) ^ 0x80000000u);
+        for (uint32_t i = t; i < n_of; i += T)
+            if (rank_in(kept, n_of, kept[i]) + 1u == k_floor) *out = int(uint32_t(kept[i] >> 32) ^ 0x80000000u);
     }
     if (t == 0 && stamp != nullptr && qi + 1u == gridDim.x) *stamp = wall_clock64();      // (among the last to end)
 }
@@ -251,9 +270,11 @@ hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int 
 }
 
 // ===========================================================================
-// One workgroup per query: the k_eff best blocks by counting (select_threshold), their rows scored as the
-// scans score them, ranked.  All latency (k = 10, a thousand queries: 18 us over 100K x 128; at 3072 dimensions, twenty-four
-// times the row, 80 over 2000 rows and 133 over 200K, where it takes workgroups of 1024).
+// One workgroup per query: the k_eff best blocks (select_top, and counting where many tie), their rows scored as the
+// scans score them, ranked.  All latency (k = 10, a thousand queries: 17 us over 100K x 128; at 3072 dimensions, twenty-four
+// times the row, 80 over 2000 rows and 133 over 200K, where it takes workgroups of 1024).  With the threshold from groups' best words
+// instead of counted out, us a search: 100K x 128, 1 query 30.2 -> 27.9, 64 queries, k = 100 41.8 -> 40.4; and of the floors' kernel 500K x
+// 768, 45 queries, k = 64 109 -> 92, 1M x 1536, 64 queries 198 -> 194.
 // ===========================================================================
 struct PickArgs {
     const uint32_t *best;
@@ -279,6 +300,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     extern __shared__ __align__(16) uint8_t dyn[];
     __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ SelectShared sh;
+    __shared__ TopShared top;
     __shared__ uint32_t blocks[kMaxPickK];
     __shared__ uint32_t n_kept, n_list, s_floor;
     uint64_t *list = reinterpret_cast<uint64_t *>(dyn);                     // rows of the chosen blocks that can still matter
@@ -300,34 +322,19 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         for (int i = int(t); i < a.nch * 4; i += int(T))
             reinterpret_cast<uint4 *>(wts)[i] = src[(i >> 2) * 128 + (i & 1) * 64 + ((i >> 1) & 1) * 32];
     }
-    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     if (t == 0) { n_kept = 0u; n_list = 0u; s_floor = 0u; }
+    uint32_t most = 0u;
+#pragma unroll
+    for (uint32_t e = 0; e < H; ++e) most = max(most, v[e]);
     auto each = [&](auto &&f) {
 #pragma unroll
         for (uint32_t e = 0; e < H; ++e)
             if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
     };
-    uint32_t mine = 0u, hi_max = 0u, hi_min_inv = 0u, mx, mn_inv, total = 0u;
-    each([&](uint64_t k) {
-        ++mine;
-        hi_max = max(hi_max, uint32_t(k >> 32));
-        hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
-    });
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) mine += __shfl_xor(mine, d);
-    if (lane == 0) sh.w_sum[wv] = mine;
-    select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
-    for (uint32_t w = 0; w < W; ++w) total += sh.w_sum[w];
-    __syncthreads();
-    const uint32_t need = min(k_eff, total);
-    const uint64_t threshold = total > 256u ? select_threshold<T>(each, mx, mn_inv, need, sh) : 0ull;
-    each([&](uint64_t k) {
-        if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
-    });
-    __syncthreads();
-    uint32_t n = n_kept;
-    if (t < 2u) kept[n + t] = 0ull;
-    __syncthreads();
+    // (256 blocks are ranked as they are)
+    if (a.n_blocks <= 256u) __syncthreads();
+    uint32_t n = keep_best<T>(each, a.n_blocks <= 256u ? 1u : select_top<T>(most, k_eff, top), k_eff, kept, n_kept, sh);
+    const uint32_t need = min(k_eff, n);
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];
         const uint32_t rank = rank_in(kept, n, k);
@@ -410,26 +417,9 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     auto each_row = [&](auto &&f) {
         for (uint32_t i = t; i < m; i += T) f(list[i]);
     };
-    uint64_t least = 0ull;
-    if (m > kSelectKept) {      // many ties
-        hi_max = 0u;
-        hi_min_inv = 0u;
-        each_row([&](uint64_t k) {
-            hi_max = max(hi_max, uint32_t(k >> 32));
-            hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
-        });
-        select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);
-        least = select_threshold<T>(each_row, mx, mn_inv, k_eff, sh);
-    }
     if (t == 0) n_kept = 0u;
     __syncthreads();
-    each_row([&](uint64_t k) {
-        if (k >= least) kept[atomicAdd(&n_kept, 1u)] = k;
-    });
-    __syncthreads();
-    n = n_kept;
-    if (t < 2u) kept[n + t] = 0ull;
-    __syncthreads();
+    n = keep_best<T>(each_row, 1u, k_eff, kept, n_kept, sh);       // (all of them, but for many ties)
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];
         const uint32_t rank = rank_in(kept, n, k);

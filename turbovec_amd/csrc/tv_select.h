@@ -67,6 +67,53 @@ __device__ __forceinline__ uint64_t select_threshold(const Each &each, uint32_t 
     return low;
 }
 
+// A score word that at least `need` of the threads' words reach, or 1 where the threads hold fewer: the need-th largest of the
+// best words of groups of threads, 64 of them or, from 17 on, 256.  For words dealt out at random few more than `need` reach it
+// (k = 10 of 64 groups: 10.8; 100 of 256: 126): one pass over them and one barrier (two), where counting them into bins takes a range and two
+// passes of four barriers.  `most`: the largest of the calling thread's words, 0 for none.  Met by all T threads.
+struct TopShared {
+    __attribute__((aligned(16))) uint32_t groups[256 + 16];      // (four words of padding after every 64: lanes that read 64 apart spread over the banks)
+    uint32_t w_top[16];
+};
+template <uint32_t T>
+__device__ __forceinline__ uint32_t select_top(uint32_t most, uint32_t need, TopShared &sh) {
+    constexpr uint32_t W = T / 64;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    auto other = [](uint32_t v, auto ctrl) { return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), decltype(ctrl)::value, 0xf, 0xf, false)); };
+    auto reached = [&](uint32_t from, uint32_t count, uint32_t v) -> uint32_t {      // words of groups[from .. from + count) not below v
+        uint32_t n = 0u;
+        for (uint32_t g = from; g < from + count; g += 4u) {
+            const uint4 x = *reinterpret_cast<const uint4 *>(&sh.groups[g + (g >> 6) * 4u]);
+            n += (x.x >= v ? 1u : 0u) + (x.y >= v ? 1u : 0u) + (x.z >= v ? 1u : 0u) + (x.w >= v ? 1u : 0u);
+        }
+        return n;
+    };
+    const bool few = need <= 16u;
+    // (groups of T / 64 lanes, or of T / 256)
+    if (few || T >= 512) most = max(most, other(most, IntC<0xB1>{}));       // quad_perm [1,0,3,2]
+    if (few || T >= 1024) most = max(most, other(most, IntC<0x4E>{}));      // quad_perm [2,3,0,1]
+    if (few && T >= 512) most = max(most, other(most, IntC<0x141>{}));      // row_half_mirror
+    if (few && T >= 1024) most = max(most, other(most, IntC<0x140>{}));     // row_mirror
+    const uint32_t per = few ? T / 64u : T / 256u, g = t / per;
+    if (t % per == 0u) sh.groups[g + (g >> 6) * 4u] = most;
+    __syncthreads();
+    if (few) {      // every wave for itself
+        const uint32_t v = sh.groups[lane], top = wave_umax(v != 0u && reached(0u, 64u, v) >= need ? v : 0u);
+        return max(top, 1u);
+    }
+    constexpr uint32_t kWords = 256u / W, kLanes = 64u / kWords;              // words of a wave, lanes to a word
+    const uint32_t mine = wv * kWords + lane / kLanes, v = sh.groups[mine + (mine >> 6) * 4u];
+    uint32_t n = reached(lane % kLanes * (256u / kLanes), 256u / kLanes, v);
+    if (kLanes >= 2u) n += other(n, IntC<0xB1>{});
+    if (kLanes >= 4u) n += other(n, IntC<0x4E>{});
+    const uint32_t top = wave_umax(v != 0u && n >= need ? v : 0u);
+    if (lane == 0u) sh.w_top[wv] = top;
+    __syncthreads();
+    uint32_t all = 1u;
+    for (uint32_t w = 0; w < W; ++w) all = max(all, sh.w_top[w]);
+    return all;
+}
+
 // Largest score word and largest inverted score word over all T threads' keys.  Met by all T threads.
 template <uint32_t T>
 __device__ __forceinline__ void select_range(uint32_t hi_max, uint32_t hi_min_inv, SelectShared &sh, uint32_t &mx, uint32_t &mn_inv) {
