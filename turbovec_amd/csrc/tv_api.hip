@@ -475,8 +475,9 @@ struct Prepared {
 // `split`: permute-dot weights in the order k_scan_p4 reads them (the batched scans take plane order)
 // `keep_rotated`: the rotated rows are wanted in device memory too (the debug read-back).
 // `for_append`: u8-LUT tables are wanted in the order of the batch's append scan too.
+// `cleared`: a word per query to set to zero.
 int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepared &out, bool split = true,
-                    bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr) {
+                    bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr, uint64_t *cleared = nullptr) {
     const tv::Geometry &g = ix->geo;
     const size_t nq_pad = round_up(nq, tv::kQTile);
     const int mode = effective_mode(ix);
@@ -499,6 +500,7 @@ int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepar
     out.table_bytes_per_tile = mode_p ? size_t(g.nch) * 2048 : size_t(g.nch) * 1024 * tv::kQTile;
     r.tables = out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
     r.stamp = stamp;
+    r.cleared = cleared;
     TV_HIP(tv::launch_prep(r, g, nq, nq_pad, ix->stream));
     if (!mode_p) {
         if (for_append && lut_mx_serves(ix, nq)) {
@@ -886,14 +888,22 @@ bool direct_wide(const tv_index *ix, size_t nq, size_t n_blocks) {
     const int nch = ix->geo.nch;
     return tv::wide_min_queries(nch) > 0 && nq >= size_t(tv::wide_min_queries(nch)) && tv::wide_serves_best_of_block(nch) && n_blocks > 512;
 }
-size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
-    return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) + 65536;
+// (a fixed scratch array has no room set aside for it)
+int direct_shares(const tv_index *ix, size_t cq, size_t k_eff) {
+    return ix->ws_fixed ? 1 : tv::pick_shares(ix->device, ix->geo.nch, k_eff, cq, effective_mode(ix) != TV_SCORE_P);
+}
+// (enough for a call's shorter last chunk too, which may share where the others do not: chunks of up to half the compute units do)
+size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff) {
+    const size_t sharing = std::min(cq, size_t(tv::device_cus(ix->device)) / 2);
+    return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) +
+           (direct_shares(ix, 1, k_eff) > 1 ? round_up(tv::pick_shared_bytes(k_eff, sharing), 256) : 0) + 65536;
 }
 // Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, each pair
 // without sampling and with it: 100K x 128, 1 query 30 and 45, 64 queries 32 and 61, 1000 queries 67 and 493; x 64, 5 queries
 // 29 and 45 (1.04M: 45 and 59); 260K x 768, 32 queries 54 and 71; 100K x 1536, 1000 queries 246 and 304.
-//  - It scores k blocks a second time in one workgroup: k = 100 at 768 dimensions (12 chunks) costs one
-//    query 77 us against 64, at 128 dimensions 40 against 72.
+//  - It scores k blocks a second time: in one workgroup k = 100 at 768 dimensions (12 chunks) costs one
+//    query 77 us against 64, at 128 dimensions 40 against 72; in up to eight of them, where queries are few (pick_shares), 20K rows x 768
+//    41.5 and 57.2, 400K 64 and 105, 100K x 3072 92 and 137, 32 queries over 100K x 1536 74 and 106; but 60 queries over 100K x 1024 73 and 63.
 //  - k_pick keeps a word per block in registers: 32768 blocks at most (twice that spills: 2M x 128, one query
 //    121 and 77).
 //  - One tile of queries: a full scan of so many bytes that two more launches no longer show.  1.04M rows x 128
@@ -912,25 +922,28 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks) {
 // 100 queries 89 and 164; 1M x 1536, 12 queries 198 and 236.
 //  - Rows are scored a second time at two table reads a byte: 100 blocks of 12 chunks take 50 us (400K x 768 3-bit, one
 //    query, k = 60: 95 and 85; 60K x 1536, 8 queries, k = 100: 99 and 97; 400K: 133 and 138; 64 queries: 147 and
-//    177; 60K, 400 queries: 309 and 285).  One query over up to 64 blocks would be scanned once, without a level in front (1000 rows x
+//    177; 60K, 400 queries: 309 and 285) in one workgroup; shared, one query, k = 100: 100K x 768 44 and 53, 400K x 1536 76 and 86; 60 queries
+//    over 100K x 1536 3-bit 117 and 174, 100 over 100K x 768 3-bit, k = 100 112 either way.  One query over up to 64 blocks would be scanned once, without a level in front (1000 rows x
 //    512 34 and 40; x 1536 49 and 50; x 1024 3-bit 54.3 and 53.6; x 3072 71 and 66, k = 1 65.7 and 65.3).
 //  - The matrix-unit scan pays its epilogue on every (block, tile) pair: 400K x 1536, 500 queries (200K pairs) 983 and 1038, 1M x
 //    512 (500K pairs) 1060 and 955.
+constexpr size_t kSharedMost = 6000;      // (k times the chunks of a row, shared by eight: 100K x 3072, k = 100 is 4800)
 bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const size_t nch = size_t(ix->geo.nch), rescored = k_eff * nch, tiles = (std::min(nq, kChunkQueries) + tv::kQTile - 1) / tv::kQTile;
     if (effective_mode(ix) != TV_SCORE_L_U32 || ix->no_lut16 || tv::pick_lds_bytes(int(nch), k_eff, true) > tv::kPickLds) return false;
-    if (nq == 1) return rescored <= (n_blocks > 64 ? 400u : nch <= 16 ? 120u : 0u);
+    const size_t shares = size_t(direct_shares(ix, nq, k_eff));
+    if (nq == 1) return rescored <= (n_blocks > 64 ? (shares > 1 ? kSharedMost : 400u) : nch <= 16 ? 120u : 0u);
     if (nq <= size_t(tv::kLut16Queries)) return rescored <= (n_blocks >= 4096 ? 1200u : 720u);
-    return n_blocks * tiles <= 200000 && rescored <= (tiles <= 4 ? 1200u : 600u);
+    return n_blocks * tiles <= 200000 && rescored <= std::max<size_t>(tiles <= 4 ? 1200u : 600u, 600u * shares);
 }
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
     if (ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
     if (k_eff > size_t(tv::kMaxPickK) || n_blocks > tv::kMaxPickBlocks) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
-    if (ix->ws_fixed && direct_need(ix, cq, n_blocks) > ix->ws_bytes) return false;
+    if (ix->ws_fixed && direct_need(ix, cq, n_blocks, k_eff) > ix->ws_bytes) return false;
     if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks);
-    if (!tv::best_serves(nch) || k_eff * nch > 600 || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds) return false;
+    if (!tv::best_serves(nch) || k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
     if (nch < 12) return triples <= 6000000;
@@ -971,7 +984,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                   int64_t *d_out_idx, bool timing) {
     const tv::Geometry &g = ix->geo;
     const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, stride = round_up(n_blocks, 64);
-    int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks));
+    int rc = ensure_workspace(ix, direct_need(ix, chunk_len(ix, nq), n_blocks, k_eff));
     if (rc != TV_OK) return rc;
     ix->last_queries_per_launch = int(chunk_len(ix, nq));
     if (effective_mode(ix) != TV_SCORE_P && !lut_mx_serves(ix, chunk_len(ix, nq)))
@@ -986,7 +999,9 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             Arena ar;
             ar.base = static_cast<uint8_t *>(ix->ws);
             Prepared pq;
-            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, true, timed ? ix->d_stamps : nullptr);
+            const int shares = direct_shares(ix, cq, k_eff);
+            uint64_t *shared = shares > 1 ? ar.take<uint64_t>(tv::pick_shared_bytes(k_eff, cq) / sizeof(uint64_t)) : nullptr;
+            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, true, timed ? ix->d_stamps : nullptr, shared);
             if (rc != TV_OK) return rc;
             tv::ScanArgs a;
             fill_scan_args(ix, a);
@@ -1009,7 +1024,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                 if (rc != TV_OK) return rc;
             }
             TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->rows().slots, ix->d_flags_host + c0,
-                                   timed ? ix->d_stamps + 1 : nullptr, ix->stream));
+                                   shares, shared, timed ? ix->d_stamps + 1 : nullptr, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));
         if (timing && g0 == 0) {

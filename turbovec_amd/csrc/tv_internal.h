@@ -115,6 +115,7 @@ struct PrepRequest {
     float *qscale, *qbias;
     float *rot_out;                 // or null
     uint64_t *stamp;                // or null
+    uint64_t *cleared;              // or null: a word per query to set to zero
 };
 hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s);
 
@@ -158,8 +159,11 @@ constexpr uint32_t kMaxFloorBlocks = 8192;
 hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,
                         hipStream_t s);
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut);
+// Workgroups that share a query's work in launch_pick; more than one need pick_shared_bytes of it, the first nq words zero.
+int pick_shares(int device, int nch, size_t k_eff, size_t nq, bool lut);
+size_t pick_shared_bytes(size_t k_eff, size_t nq);
 hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, const uint32_t *slots, uint32_t *overflow,
-                       uint64_t *stamp, hipStream_t s);
+                       int shares, uint64_t *shared, uint64_t *stamp, hipStream_t s);
 hipError_t launch_scan_lut(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Query tiles one batched permute-dot launch serves for this geometry (0: not available).
 int batched_tiles(int nch);

@@ -276,6 +276,9 @@ hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int 
 // instead of counted out, us a search: 100K x 128, 1 query 30.2 -> 27.9, 64 queries, k = 100 41.8 -> 40.4; and of the floors' kernel 500K x
 // 768, 45 queries, k = 64 109 -> 92, 1M x 1536, 64 queries 198 -> 194.
 // ===========================================================================
+// A query's part of the memory that its workgroups share: how many rows each found, and each one's rows.
+constexpr uint32_t kMaxShares = 8;
+__host__ __device__ constexpr uint32_t pick_shared_words(uint32_t k_eff) { return kMaxShares + (k_eff + kMaxShares) * 32u; }
 struct PickArgs {
     const uint32_t *best;
     uint32_t best_stride, n_blocks, n;
@@ -290,11 +293,21 @@ struct PickArgs {
     int64_t *out_idx;
     const uint32_t *slots;      // when given: the slot of each row, for out_idx
     uint32_t *overflow;
+    uint32_t nq, shares;
+    uint64_t *counts, *lists;   // shares > 1: per query the number of workgroups that are through with it, and what they found (pick_shared_words)
     uint64_t *stamp;
 };
+// Chunks of a query to score again (of tables: thirds), from where sharing them pays (less: 100K x 768, 64 queries, k = 10 43.3 us and, shared,
+// 44.2; 100K x 512 2-bit, one query 35.1 and 36.4; 20K x 384, one query, k = 20 31.9 and 31.1).
+constexpr size_t kSharedWork = 200;
 // H: blocks a thread keeps in registers -- all of them, T * H at most.
 // LUT: score mode L with the u32 epilogue.
-template <uint32_t T, uint32_t H, bool LUT>
+// Scoring a block again is 70 (LUT: 200) vector instructions a chunk, on one CU for all of a query's blocks.  Where queries are too few for
+// all CUs, several workgroups choose the same blocks, score their share of them and write its rows to memory;
+// the one that finds itself last ranks it.  Nobody waits for another.  us a search with one workgroup each and so: 100K x 768, one query, k = 50
+// 60.6 -> 43.5; 100K x 1536, 8 queries, k = 25 66.5 -> 54.5, one query, k = 10 55.4 -> 52.6; 778K x 1000 3-bit, 37 queries, k = 33 218 -> 216 (this
+// kernel 37 -> 25).
+template <uint32_t T, uint32_t H, bool LUT, bool SHARED>
 __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     constexpr uint32_t W = T / 64;
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -302,13 +315,14 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     __shared__ SelectShared sh;
     __shared__ TopShared top;
     __shared__ uint32_t blocks[kMaxPickK];
-    __shared__ uint32_t n_kept, n_list, s_floor;
+    __shared__ uint32_t n_kept, n_list, s_floor, s_last;
     uint64_t *list = reinterpret_cast<uint64_t *>(dyn);                     // rows of the chosen blocks that can still matter
     uint8_t *wts = dyn + size_t(a.k_eff) * 32 * 8;                          // this query's weights
-    const uint32_t qi = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    const uint32_t qi = SHARED ? blockIdx.x % a.nq : blockIdx.x, share = SHARED ? blockIdx.x / a.nq : 0u, shares = SHARED ? a.shares : 1u;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
     const uint32_t k_eff = uint32_t(a.k_eff);
     const uint32_t *best = a.best + size_t(qi) * a.best_stride;
-    if (a.stamp != nullptr && qi + t == 0) *a.stamp = wall_clock64();
+    if (a.stamp != nullptr && blockIdx.x + t == 0) *a.stamp = wall_clock64();
     uint32_t v[H];
 #pragma unroll
     for (uint32_t e = 0; e < H; ++e) v[e] = e * T + t < a.n_blocks ? best[e * T + t] : 0u;
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     const uint32_t floor_word = s_floor, h = lane >> 5;
     const float qs = a.qscale[qi], qb = a.qbias[qi];
     const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
-    for (uint32_t i = wv; i < need; i += W) {
+    for (uint32_t i = wv * shares + share; i < need; i += W * shares) {
         const uint32_t b = blocks[i], slot = b * 32u + (lane & 31u);
         const float vs = a.scales[slot];
         const uint4 *src = reinterpret_cast<const uint4 *>(a.codes) + size_t(b) * a.nch * 64 + lane;
@@ -408,6 +422,30 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         const uint64_t key = sort_key(s, slot);
         if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
     }
+    if constexpr (SHARED) {
+        __syncthreads();
+        const uint32_t cap = (k_eff + shares - 1u) / shares * 32u, own = n_list;
+        uint64_t *area = a.lists + size_t(qi) * pick_shared_words(k_eff);
+        auto put = [](uint64_t *to, uint64_t v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        auto get = [](uint64_t *from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        for (uint32_t i = t; i < own; i += T) put(&area[kMaxShares + share * cap + i], list[i]);
+        if (t == 0) put(&area[share], own);
+        // This thread's words are there before its workgroup is counted: they go past the caches, like the count and
+        // like the loads below, so the stores' completion is enough (a fence writes the whole cache of the die back, and
+        // with 200 workgroups of 16 waves takes 80 us).
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (t == 0) s_last = atomicAdd(reinterpret_cast<unsigned long long *>(&a.counts[qi]), 1ull) + 1ull == shares ? 1u : 0u;
+        __syncthreads();
+        if (s_last == 0u) return;
+        uint32_t all = 0u;
+        for (uint32_t o = 0; o < shares; ++o) {
+            const uint32_t theirs = uint32_t(get(&area[o]));
+            for (uint32_t i = t; i < theirs; i += T) list[all + i] = get(&area[kMaxShares + o * cap + i]);
+            all += theirs;
+        }
+        if (t == 0) n_list = all;
+    }
     __syncthreads();
     const uint32_t m = n_list;
     // (fewer rows with a score than wanted -- an overstated count of allowed rows, scores of NaN or -infinity: the exact
@@ -432,11 +470,18 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
 }
 
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64); }
+int pick_shares(int device, int nch, size_t k_eff, size_t nq, bool lut) {
+    // (a SIMD's worth of blocks at least for each workgroup)
+    if (nq == 0 || k_eff * size_t(nch) * (lut ? 3 : 1) < kSharedWork) return 1;
+    return int(std::max<size_t>(1, std::min<size_t>({kMaxShares, k_eff / 4, size_t(device_cus(device)) / nq})));
+}
+size_t pick_shared_bytes(size_t k_eff, size_t nq) { return nq * (1 + pick_shared_words(uint32_t(k_eff))) * sizeof(uint64_t); }
 
 // The scan's arguments say what was scanned; a.tables: its weight tiles, or (lut) the queries' tables as k_prep_lut leaves them.
 hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float *out_scores, int64_t *out_idx, const uint32_t *slots, uint32_t *overflow,
-                       uint64_t *stamp, hipStream_t s) {
+                       int shares, uint64_t *shared, uint64_t *stamp, hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
+    if (shares < 1 || (shares > 1 && shared == nullptr)) return hipErrorInvalidValue;
     const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff), lut);
     if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
     PickArgs p;
@@ -446,16 +491,25 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     for (int i = 0; i < 4; ++i) p.lv[i] = a.lv[i];
     p.nch = a.nch; p.k_eff = k_eff; p.split = split ? 1 : 0;
     p.out_scores = out_scores; p.out_idx = out_idx; p.slots = slots; p.overflow = overflow; p.stamp = stamp;
+    p.nq = uint32_t(a.nq_tile); p.shares = uint32_t(shares); p.counts = shared; p.lists = shared + a.nq_tile;
     auto launch = [&](auto kernel, unsigned threads) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kernel, dim3(unsigned(a.nq_tile)), dim3(threads), lds, s, p);
+        hipLaunchKernelGGL(kernel, dim3(unsigned(a.nq_tile) * unsigned(shares)), dim3(threads), lds, s, p);
         return hipGetLastError();
     };
     // few queries leave the chip empty: as many waves as there are blocks to score again
     const bool small = a.nq_tile > 256 && a.n_blocks <= 256 * 16;
-    if (lut) return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, true>, 1024) : small ? launch(k_pick<256, 16, true>, 256) : launch(k_pick<1024, 16, true>, 1024);
-    return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, false>, 1024) : small ? launch(k_pick<256, 16, false>, 256) : launch(k_pick<1024, 16, false>, 1024);
+    auto form = [&](auto lut_, auto shared_) -> hipError_t {
+        constexpr bool L = decltype(lut_)::value != 0, S = decltype(shared_)::value != 0;
+        if (a.n_blocks > 1024 * 16) return launch(k_pick<1024, 32, L, S>, 1024);
+        if constexpr (!S) {
+            if (small) return launch(k_pick<256, 16, L, S>, 256);
+        }
+        return launch(k_pick<1024, 16, L, S>, 1024);
+    };
+    if (shares > 1) return lut ? form(IntC<1>{}, IntC<1>{}) : form(IntC<0>{}, IntC<1>{});
+    return lut ? form(IntC<1>{}, IntC<0>{}) : form(IntC<0>{}, IntC<0>{});
 }
 
 }  // namespace tv

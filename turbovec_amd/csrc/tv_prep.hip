@@ -24,6 +24,7 @@ struct PrepArgs {
     float *rot_out;                 // when given: the rotated (and calibrated) rows
     size_t nq;
     uint64_t *stamp;
+    uint64_t *cleared;              // when given: a word per query, set to zero
 };
 
 // A row lies in LDS with eight floats of padding after every 64: lanes whose elements are 64 apart in
@@ -218,6 +219,7 @@ __global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split
     if (t == 0) {
         a.qscale[qi] = cs * qs;
         a.qbias[qi] = 0.0f + bias;
+        if (a.cleared != nullptr) a.cleared[qi] = 0;
         if (a.stamp != nullptr && qi + 1 == a.nq) *a.stamp = wall_clock64();      // (among the last to end)
     }
 }
@@ -309,6 +311,7 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         o[0] = make_uint4(w[0], w[1], w[2], w[3]);
         o[1] = make_uint4(w[4], w[5], w[6], w[7]);
     }
+    if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
     if (t == 0 && a.stamp != nullptr && qi + 1 == a.nq) *a.stamp = wall_clock64();      // (among the last to end)
 }
 
@@ -322,7 +325,7 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     a.inv_sqrt_block = r.inv_sqrt_block;
     a.dim = g.dim; a.log_block = __builtin_ctz(unsigned(r.block)); a.G = g.G; a.nch = g.nch;
     a.tables = r.tables; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
-    a.nq = nq; a.stamp = r.stamp;
+    a.nq = nq; a.stamp = r.stamp; a.cleared = r.cleared;
     const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
     auto launch = [&](auto kernel, auto... rest) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
