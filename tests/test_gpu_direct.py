@@ -97,6 +97,27 @@ def test_best_blocks_in_any_place(T, oracle, nq):
     ix.close()
 
 
+@pytest.mark.parametrize("dim,nq", [(64, 3), (64, 257), (768, 33), (1536, 300)])
+@pytest.mark.parametrize("n", [1, 33, 1025, 4096, 4097])
+def test_few_rows(T, oracle, n, dim, nq):
+    """Up to 4096 rows every row's score is kept: on either side of that, of a filter's rows too, and with rows that tie."""
+    v = unit_gaussian(n, dim, seed=n + dim)
+    v[n // 2:n // 2 + 1500] = v[0]
+    oidx = OracleIndex(oracle, dim, 4, v)
+    q = unit_gaussian(nq, dim, seed=31)
+    q[0] = v[0]
+    ix = to_native(T, oidx)
+    for m in (None, np.random.default_rng(3).random(n) < 0.3, np.arange(n) % 32 == 31):
+        if m is not None and not m.any():
+            m[0] = True
+        words = None if m is None else T.pack_mask(m)[0]
+        for k in (1, 16, 17, 100):
+            s, i = ix.search(q, k, mask_words=words)
+            os_, oi = oidx.search(q, k, mask_words=words)
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
+    ix.close()
+
+
 @pytest.mark.parametrize("k", [3, 10, 60])
 def test_rows_that_score_minus_infinity(T, oracle, k):
     """Row scales that take most rows' scores beyond the float range: the blocks of the few finite rows hold -infinity

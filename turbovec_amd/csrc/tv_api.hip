@@ -888,14 +888,23 @@ bool direct_wide(const tv_index *ix, size_t nq, size_t n_blocks) {
     const int nch = ix->geo.nch;
     return tv::wide_min_queries(nch) > 0 && nq >= size_t(tv::wide_min_queries(nch)) && tv::wide_serves_best_of_block(nch) && n_blocks > 512;
 }
+// Whether the scan of that search keeps every row's score: few rows, on the kernel that can, and memory of the index's own.  A score per
+// row and query against whole blocks scored again (us a search, blocks and rows): 2000 x 3072, 1024 queries 129 and 63, k = 1 71 and 62; 4096 x
+// 1536, 300 queries 61 and 39, 8 queries, k = 100 69 and 35; 4000 x 384, 1024 queries 42.4 and 41.8, x 256 38.3 and 40.8, x 128
+// 34.5 and 39.8, k = 50 49 and 44; 2000 x 128 32.6 and 33.5, 1000 x 128 32.2 and 31.0; 4000 x 128, one query 27.9 and 24.4, 128 queries 28.9 and 26.6.
+bool direct_rows(const tv_index *ix, size_t nq, size_t n_blocks, size_t k_eff) {
+    const size_t rows = n_blocks * tv::kVecBlock;
+    return !ix->ws_fixed && effective_mode(ix) == TV_SCORE_P && rows <= tv::kMaxPickRows && !direct_wide(ix, nq, n_blocks) &&
+           (nq <= 256 || rows <= 75 * k_eff * size_t(ix->geo.nch));
+}
 // (a fixed scratch array has no room set aside for it)
 int direct_shares(const tv_index *ix, size_t cq, size_t k_eff) {
     return ix->ws_fixed ? 1 : tv::pick_shares(ix->device, ix->geo.nch, k_eff, cq, effective_mode(ix) != TV_SCORE_P);
 }
-// (enough for a call's shorter last chunk too, which may share where the others do not: chunks of up to half the compute units do)
+// (enough for a call's shorter last chunk too, which may keep rows' scores, or share, where the others do not)
 size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff) {
     const size_t sharing = std::min(cq, size_t(tv::device_cus(ix->device)) / 2);
-    return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * sizeof(uint32_t), 256) +
+    return prepare_bytes(ix, cq) + round_up(cq * round_up(n_blocks, 64) * (direct_rows(ix, 1, n_blocks, k_eff) ? tv::kVecBlock : 1) * sizeof(uint32_t), 256) +
            (direct_shares(ix, 1, k_eff) > 1 ? round_up(tv::pick_shared_bytes(k_eff, sharing), 256) : 0) + 65536;
 }
 // Where the search without sampling is the faster one.  Device buffers, k = 10, us a search, each pair
@@ -943,7 +952,10 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks)
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks, k_eff) > ix->ws_bytes) return false;
     if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks);
-    if (!tv::best_serves(nch) || k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds) return false;
+    if (!tv::best_serves(nch)) return false;
+    // (no block is scored again where rows' scores are kept)
+    if (!direct_rows(ix, cq, n_blocks, k_eff) &&
+        (k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds)) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
     if (nch < 12) return triples <= 6000000;
@@ -976,7 +988,8 @@ int best_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
 int take_stamps(tv_index *ix, int launches) {
     int khz = 0;
     TV_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ix->device));
-    if (khz > 0) ix->last_scan_ms += float(double(ix->h_stamps[1] - ix->h_stamps[0]) / khz);
+    const uint64_t before = *std::max_element(ix->h_stamps, ix->h_stamps + tv::kStampsBefore);      // (those of earlier searches are lower)
+    if (khz > 0) ix->last_scan_ms += float(double(ix->h_stamps[tv::kStampsBefore] - before) / khz);
     ix->last_scan_launches += launches;
     return TV_OK;
 }
@@ -999,7 +1012,7 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             Arena ar;
             ar.base = static_cast<uint8_t *>(ix->ws);
             Prepared pq;
-            const int shares = direct_shares(ix, cq, k_eff);
+            const int shares = direct_rows(ix, cq, n_blocks, k_eff) ? 1 : direct_shares(ix, cq, k_eff);
             uint64_t *shared = shares > 1 ? ar.take<uint64_t>(tv::pick_shared_bytes(k_eff, cq) / sizeof(uint64_t)) : nullptr;
             rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, true, timed ? ix->d_stamps : nullptr, shared);
             if (rc != TV_OK) return rc;
@@ -1010,8 +1023,9 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             a.qscale = pq.d_qscale;
             a.qbias = pq.d_qbias;
             a.nq_tile = int(cq);
-            a.best_out = ar.take<uint32_t>(cq * stride);
-            a.best_stride = uint32_t(stride);
+            a.best_rows = direct_rows(ix, cq, n_blocks, k_eff) ? 1 : 0;
+            a.best_stride = uint32_t(stride * (a.best_rows ? tv::kVecBlock : 1));
+            a.best_out = ar.take<uint32_t>(cq * a.best_stride);
             if (wide) {
                 a.gtau = ix->d_tau_open;
                 a.best_of_block = 1;
@@ -1023,8 +1037,11 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
                 rc = best_scan_lut(ix, a, pq, cq);
                 if (rc != TV_OK) return rc;
             }
-            TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->rows().slots, ix->d_flags_host + c0,
-                                   shares, shared, timed ? ix->d_stamps + 1 : nullptr, ix->stream));
+            if (a.best_rows)
+                TV_HIP(tv::launch_pick_rows(reinterpret_cast<const float *>(a.best_out), a.best_stride, a.n, int(k_eff), int(cq), d_out_scores + q0 * k_eff,
+                                            d_out_idx + q0 * k_eff, ix->rows().slots, ix->d_flags_host + c0, timed ? ix->d_stamps + tv::kStampsBefore : nullptr, ix->stream));
+            else TV_HIP(tv::launch_pick(a, !mode_p, split, int(k_eff), d_out_scores + q0 * k_eff, d_out_idx + q0 * k_eff, ix->rows().slots, ix->d_flags_host + c0,
+                                   shares, shared, timed ? ix->d_stamps + tv::kStampsBefore : nullptr, ix->stream));
         }
         TV_HIP(hipStreamSynchronize(ix->stream));
         if (timing && g0 == 0) {
@@ -1269,7 +1286,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                                             int(pq_n), d_os, d_oi, d_over, last ? nullptr : d_tau, int(tile_q),
                                             (lv > 0 || repeat) ? 1 : 0, (last && !repeat) ? d_raise + (q0 - g0) : nullptr,
                                             repeat ? d_rows + row0 : nullptr, lv_flag, attempt == 0 ? next_flag : nullptr,
-                                            run_if, ix->rows().slots, !timed_pass ? nullptr : last ? ix->d_stamps + 1 : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
+                                            run_if, ix->rows().slots, !timed_pass ? nullptr : last ? ix->d_stamps + tv::kStampsBefore : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
                                             ix->stream));
                 }
             }
@@ -1861,7 +1878,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
             rc = TV_ERR_HIP;
             break;
         }
-        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t) + 2 * sizeof(uint64_t), hipHostMallocMapped) != hipSuccess) {
+        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t) + (tv::kStampsBefore + 1) * sizeof(uint64_t), hipHostMallocMapped) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
         }
@@ -1872,6 +1889,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         static_assert((kGroupQueries + kLevelFlagWords) % 2 == 0, "the stamps behind the flags are 8-byte words");
         ix->h_stamps = reinterpret_cast<uint64_t *>(ix->h_flags + kGroupQueries + kLevelFlagWords);
         ix->d_stamps = reinterpret_cast<uint64_t *>(ix->d_flags_host + kGroupQueries + kLevelFlagWords);
+        std::fill_n(ix->h_stamps, tv::kStampsBefore + 1, uint64_t(0));
         rc = scratch_address(device, &ix->scratch);
         if (rc != TV_OK) break;
         // floors of a search's first sampling level: the order key of -inf for every query, written once

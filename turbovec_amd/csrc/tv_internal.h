@@ -72,6 +72,7 @@ struct ScanArgs {
     int best_of_block;         // all-queries-per-pass kernel: no floor, per scanned block and query the best allowed slot (kModeBest)
     uint32_t *best_out;        // when given: [nq_tile][best_stride] score words, per query and scanned block the best allowed row's (tv_kernels6.hip)
     uint32_t best_stride;
+    int best_rows;             // (of launch_scan_p4_best) ... every row's score as a float instead, NaN for rows that may not be returned: [nq_tile][best_stride], by row
     const uint32_t *rows;      // all-queries-per-pass kernel: when given, the slot of each of the n rows to scan, in order, 32 neighbours of them within 4 GiB
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
@@ -101,6 +102,9 @@ hipError_t launch_move_lane(uint8_t *d_native, float *d_scales, const Geometry &
 // device clock as the last query's workgroup ends (of the preparation and of a sampling level's selection) or the
 // first one's starts (of a last selection): the full scan between two of them, gaps between launches included, is
 // timed without events, whose packets the launches behind them wait for, 5 to 6 us each.
+// (Of the preparation, the last kStampsBefore queries' workgroups, one to a die, and those that add a bias in order take one of as
+// many words each, and the latest counts.)
+constexpr int kStampsBefore = 8;
 struct PrepRequest {
     const float *q, *signs;
     const uint32_t *perms;
@@ -114,7 +118,7 @@ struct PrepRequest {
     uint8_t *tables;
     float *qscale, *qbias;
     float *rot_out;                 // or null
-    uint64_t *stamp;                // or null
+    uint64_t *stamp;                // or null: kStampsBefore words
     uint64_t *cleared;              // or null: a word per query to set to zero
 };
 hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s);
@@ -158,6 +162,10 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
 constexpr uint32_t kMaxFloorBlocks = 8192;
 hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,
                         hipStream_t s);
+// The k_eff best of n row scores per query (ScanArgs::best_rows): the last step of a search of so few rows.
+constexpr uint32_t kMaxPickRows = 4096;
+hipError_t launch_pick_rows(const float *scores, uint32_t stride, uint32_t n, int k_eff, int nq, float *out_scores, int64_t *out_idx, const uint32_t *slots,
+                            uint32_t *overflow, uint64_t *stamp, hipStream_t s);
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut);
 // Workgroups that share a query's work in launch_pick; more than one need pick_shared_bytes of it, the first nq words zero.
 int pick_shares(int device, int nch, size_t k_eff, size_t nq, bool lut);

@@ -23,13 +23,15 @@ namespace tv {
 // 3125 of them, which fill 65 of the 256 workgroups of a kernel that takes all queries through one.
 // 100K x 128, 1000 queries: 35 us, the vector ALU busy in 60 % of the clocks and the matrix unit in 15 %.  Rows that
 // short have two chunks, so of the 530 vector instructions per block and four tiles the decode is 120, the rest epilogue.
-// Weights in plane order, or (SPLIT) in the order of k_scan_p4, whose operands then take four byte permutes a chunk.
+// Weights in plane order, or (kBestSplit) in the order of k_scan_p4, whose operands then take four byte permutes a chunk.  kBestRows: plane order,
+// and every row's score instead of the block's best (ScanArgs::best_rows; an instance of its own, as two of the others would spill).
 // a.b_step: every so many blocks only (the sample a floor is taken from), recorded by their place in the sample.
 // ===========================================================================
+enum { kBestPlane, kBestSplit, kBestRows };
 constexpr int kBestThreads = 512;
 constexpr int kBestWaves = kBestThreads / 64;
 
-template <int NT, int U, bool SPLIT>
+template <int NT, int U, int FORM>
 __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(ScanArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int nch = a.nch, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qn = lane & 31, h = lane >> 5;
@@ -42,6 +44,14 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
         const int q = (tile0 + t) * kQTile + qn;
         if (h == 0 && t < nt && q < a.nq_tile) a.best_out[size_t(q) * a.best_stride + j] = word;
     };
+    // (a.best_rows) the scores of the lane's sixteen rows of block j, four side by side
+    auto store_rows = [&](int t, uint32_t j, auto &&score) {
+        const int q = (tile0 + t) * kQTile + qn;
+        if (t >= nt || q >= a.nq_tile) return;
+        float4 *to = reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.best_out) + size_t(q) * a.best_stride + j * 32u + 4u * uint32_t(h));
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) to[r >> 1] = float4{score(r), score(r + 1), score(r + 2), score(r + 3)};
+    };
     // the next block from j on with an allowed row; the ones without are recorded on the way
     auto live_from = [&](uint32_t j) -> uint32_t {
         if (a.mask == nullptr) return j;
@@ -49,7 +59,10 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
             const uint32_t b = j * step;
             if (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) != 0u) break;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) store(t, j, 0u);
+            for (int t = 0; t < NT; ++t) {
+                if constexpr (FORM == kBestRows) store_rows(t, j, [&](int) { return nan; });
+                else store(t, j, 0u);
+            }
         }
         return j;
     };
@@ -119,7 +132,7 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
                     lo[d] = int(levels_of(x[d] & 0x0f0f0f0fu, t0, t1, t2, t3));
                     hi[d] = int(levels_of((x[d] >> 4) & 0x0f0f0f0fu, t0, t1, t2, t3));
                 }
-                if constexpr (SPLIT) {
+                if constexpr (FORM == kBestSplit) {
                     const v4i l = lo, g = hi;
                     lo = v4i{l[0], g[0], l[1], g[1]};
                     hi = v4i{int(__builtin_amdgcn_perm(uint32_t(g[2]), uint32_t(l[2]), 0x05010400u)), int(__builtin_amdgcn_perm(uint32_t(g[2]), uint32_t(l[2]), 0x07030602u)),
@@ -137,6 +150,12 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
         if (mw != 0xffffffffu) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) vs[r] = ((mw >> (8 * (r >> 2) + 4 * h + (r & 3))) & 1u) ? vs[r] : nan;
+        }
+        if constexpr (FORM == kBestRows) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) store_rows(t, j, [&](int r) { return fmaf(float(acc[t][r]), qs[t], qb[t]) * vs[r]; });
+            j = jn;
+            continue;
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -160,34 +179,37 @@ static int best_tiles(int nch, size_t n_blocks, int tiles, int cus) {
 }
 bool best_serves(int nch) { return size_t(nch) * 2048 <= 160 * 1024; }
 
-template <int NT, int U, bool SPLIT>
+template <int NT, int U, int FORM>
 static hipError_t launch_best_n(const ScanArgs &a, uint32_t nj, int device, hipStream_t s) {
     const int tiles = (a.nq_tile + kQTile - 1) / kQTile, groups_y = (tiles + NT - 1) / NT;
     const size_t lds = size_t(NT) * a.nch * 2048;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     // a workgroup keeps its weights for all its blocks: about as many workgroups as are resident
     const unsigned per_cu = unsigned(std::min<size_t>(NT <= 2 ? 2 : 1, 160 * 1024 / lds));
     const unsigned resident = unsigned(device_cus(device)) * std::max(1u, per_cu);
     const unsigned x = std::max(1u, std::min((nj + kBestWaves - 1) / kBestWaves, (resident + groups_y - 1) / groups_y));
-    hipLaunchKernelGGL((k_scan_p4_best<NT, U, SPLIT>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
+    hipLaunchKernelGGL((k_scan_p4_best<NT, U, FORM>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
     return hipGetLastError();
 }
-template <int NT, bool SPLIT>
+template <int NT, int FORM>
 static hipError_t launch_best_u(const ScanArgs &a, uint32_t nj, int device, hipStream_t s) {
     // (two tiles' accumulators and bursts of four chunks do not fit the 128 registers of four waves per SIMD)
     if constexpr (NT != 2) {
-        if (a.nch % 4 == 0) return launch_best_n<NT, 4, SPLIT>(a, nj, device, s);
+        if (a.nch % 4 == 0) return launch_best_n<NT, 4, FORM>(a, nj, device, s);
     }
-    return a.nch % 2 == 0 ? launch_best_n<NT, 2, SPLIT>(a, nj, device, s) : launch_best_n<NT, 1, SPLIT>(a, nj, device, s);
+    return a.nch % 2 == 0 ? launch_best_n<NT, 2, FORM>(a, nj, device, s) : launch_best_n<NT, 1, FORM>(a, nj, device, s);
 }
 // a.nq_tile = all queries of the launch, a.tables = their weight tiles, a.best_out / a.best_stride = the result.
 hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStream_t s) {
     const uint32_t nj = a.b_step ? (a.n_blocks + a.b_step - 1) / a.b_step : 0u;
-    if (a.nq_tile <= 0 || nj == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride < nj) return hipErrorInvalidValue;
+    if (a.nq_tile <= 0 || nj == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride / (a.best_rows ? 32u : 1u) < nj || (a.best_rows && (a.b_step != 1 || split))) return hipErrorInvalidValue;
     const int nt = best_tiles(a.nch, nj, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device));
-    if (split) return nt == 1 ? launch_best_u<1, true>(a, nj, device, s) : nt == 2 ? launch_best_u<2, true>(a, nj, device, s) : launch_best_u<4, true>(a, nj, device, s);
-    return nt == 1 ? launch_best_u<1, false>(a, nj, device, s) : nt == 2 ? launch_best_u<2, false>(a, nj, device, s) : launch_best_u<4, false>(a, nj, device, s);
+    auto form = [&](auto f) -> hipError_t {
+        constexpr int F = decltype(f)::value;
+        return nt == 1 ? launch_best_u<1, F>(a, nj, device, s) : nt == 2 ? launch_best_u<2, F>(a, nj, device, s) : launch_best_u<4, F>(a, nj, device, s);
+    };
+    return a.best_rows ? form(IntC<kBestRows>{}) : split ? form(IntC<kBestSplit>{}) : form(IntC<kBestPlane>{});
 }
 
 // The keys whose score words reach `least`, which at least `need` of all keys do or which is 1, into kept, two zeros behind
@@ -467,6 +489,57 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         a.out_scores[size_t(qi) * k_eff + rank] = s;
         a.out_idx[size_t(qi) * k_eff + rank] = int64_t(a.slots != nullptr ? a.slots[idx] : idx);
     }
+}
+
+// ===========================================================================
+// Few rows (a filter's, as a rule): the scan has kept every row's score, and nothing is scored again.  Writing and reading
+// a score per row and query takes less than k_pick's second scoring of whole blocks (2000 rows x 3072, 1024 queries, k = 10: this kernel 6 us,
+// k_pick 80; all latency at that size).
+// ===========================================================================
+template <uint32_t T, uint32_t H>
+__global__ __launch_bounds__(T) void k_pick_rows(const float *__restrict__ scores, uint32_t stride, uint32_t n, uint32_t k_eff, float *out_scores,
+                                                 int64_t *out_idx, const uint32_t *slots, uint32_t *overflow, uint64_t *stamp) {
+    __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
+    __shared__ SelectShared sh;
+    __shared__ TopShared top;
+    __shared__ uint32_t n_kept;
+    const uint32_t qi = blockIdx.x, t = threadIdx.x;
+    if (stamp != nullptr && qi + t == 0) *stamp = wall_clock64();
+    const float *mine = scores + size_t(qi) * stride;
+    float v[H];
+#pragma unroll
+    for (uint32_t e = 0; e < H; ++e) v[e] = e * T + t < n ? mine[e * T + t] : __int_as_float(0x7fc00000);
+    if (t == 0) n_kept = 0u;
+    // (a score of -infinity does not count, as in k_pick)
+    auto word = [&](uint32_t e) { return v[e] == v[e] ? best_word(v[e]) : 0u; };
+    uint32_t most = 0u;
+#pragma unroll
+    for (uint32_t e = 0; e < H; ++e) most = max(most, word(e));
+    auto each = [&](auto &&f) {
+#pragma unroll
+        for (uint32_t e = 0; e < H; ++e)
+            if (word(e) != 0u) f(sort_key(v[e], e * T + t));
+    };
+    const uint32_t m = keep_best<T>(each, select_top<T>(most, k_eff, top), k_eff, kept, n_kept, sh);
+    if (t == 0) overflow[qi] = m < k_eff ? 2u : 0u;
+    if (m < k_eff) return;
+    for (uint32_t i = t; i < m; i += T) {
+        const uint64_t k = kept[i];
+        const uint32_t rank = rank_in(kept, m, k);
+        if (rank >= k_eff) continue;
+        float s; uint32_t idx;
+        sort_unkey(k, s, idx);
+        out_scores[size_t(qi) * k_eff + rank] = s;
+        out_idx[size_t(qi) * k_eff + rank] = int64_t(slots != nullptr ? slots[idx] : idx);
+    }
+}
+hipError_t launch_pick_rows(const float *scores, uint32_t stride, uint32_t n, int k_eff, int nq, float *out_scores, int64_t *out_idx, const uint32_t *slots,
+                            uint32_t *overflow, uint64_t *stamp, hipStream_t s) {
+    if (nq <= 0) return hipSuccess;
+    if (n > kMaxPickRows || n > stride || k_eff <= 0 || k_eff > kMaxPickK) return hipErrorInvalidValue;
+    if (nq > 256) hipLaunchKernelGGL((k_pick_rows<256, 16>), dim3(unsigned(nq)), dim3(256), 0, s, scores, stride, n, uint32_t(k_eff), out_scores, out_idx, slots, overflow, stamp);
+    else hipLaunchKernelGGL((k_pick_rows<1024, 4>), dim3(unsigned(nq)), dim3(1024), 0, s, scores, stride, n, uint32_t(k_eff), out_scores, out_idx, slots, overflow, stamp);
+    return hipGetLastError();
 }
 
 size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64); }

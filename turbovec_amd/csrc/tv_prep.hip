@@ -96,7 +96,8 @@ __device__ __forceinline__ void rotate_row(const float *src, const float *signs,
 // rounding is used: all threads add, and where every value within the two orders' distance -- dim roundings at most on the
 // way of a term there, dim / 256 + 9 here, and those of the magnitude's sum -- rounds to the same float, that is it.
 // Otherwise (one query in 10^5) one thread adds in order.  With the chain always: 3032 dimensions 47 us for one query, now 25.
-__device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs &a, float *A, float *B, double *prod) {
+// late: becomes true there.
+__device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs &a, float *A, float *B, double *prod, bool &late) {
     const int t = threadIdx.x, dim = a.dim;
     rotate_row(src, a.signs, a.perms, dim, a.log_block, a.inv_sqrt_block, A, B);
     float bias = 0.0f;
@@ -119,6 +120,7 @@ __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs
         const double slack = double(2 * dim + 256) * 0x1p-53 * mass;
         bias = float(sum - slack);
         if (__float_as_uint(bias) != __float_as_uint(float(sum + slack)) || !(slack < 1e30)) {     // (uniform over the workgroup)
+            late = true;
             double bc = 0.0;
             for (int d0 = 0; d0 < dim; d0 += kPrepPiece) {
                 const int m = min(kPrepPiece, dim - d0);      // (a multiple of eight, as dim is)
@@ -201,7 +203,8 @@ __global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split
         if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
         return;
     }
-    const float bias = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod);
+    bool late = false;
+    const float bias = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod, late);
     float m = 0.0f;
     for (int d = t; d < a.dim; d += kPrepThreads) m = fmaxf(m, fabsf(A[d]));
     const float qmax = block_max_256(m, red);
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split
         a.qscale[qi] = cs * qs;
         a.qbias[qi] = 0.0f + bias;
         if (a.cleared != nullptr) a.cleared[qi] = 0;
-        if (a.stamp != nullptr && qi + 1 == a.nq) *a.stamp = wall_clock64();      // (among the last to end)
+        if (a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
     }
 }
 
@@ -259,7 +262,8 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         return;
     }
     if (t < (1 << BITS)) cen[t] = centroids[t];
-    const float bias_corr = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod);
+    bool late = false;
+    const float bias_corr = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod, late);
     float *mins = B;                                   // two per group: at most a row's length
     float span = 0.0f;
     for (int g = t; g < G; g += kPrepThreads) {
@@ -312,7 +316,7 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         o[1] = make_uint4(w[4], w[5], w[6], w[7]);
     }
     if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
-    if (t == 0 && a.stamp != nullptr && qi + 1 == a.nq) *a.stamp = wall_clock64();      // (among the last to end)
+    if (t == 0 && a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
 }
 
 static_assert(size_t(2) * prep_floats(16384) * sizeof(float) + kPrepPiece * sizeof(double) + 128 <= 160 * 1024,
