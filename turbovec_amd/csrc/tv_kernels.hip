@@ -929,20 +929,21 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 //
 // The work is a few thousand keys in a few hundred short segments, and all of
 // it is latency; a thousand queries share the chip.  So: a thread per segment,
-// its head requested together with its count; one pass of counting into 1024
-// bins between the smallest and the largest key gives a threshold few keys
-// reach (a bin that still holds too many is divided again); those are collected
-// in LDS and ranked by comparing each with all -- no sort, a handful of
+// its head requested together with its count -- four threads where queries are few, and
+// then the whole of it; the need-th largest of groups of threads' best keys is a threshold
+// few keys reach (select_top; more than 128 wanted are counted out into 1024
+// bins); those are collected in LDS and ranked by comparing each with all -- no sort, a handful of
 // barriers, 30 KiB of LDS, and workgroups no larger than the segments need.
-// Per launch under the profiler, before (waves sorting chunks in 64 KiB of LDS,
-// 1024 threads per query) and now: one query, k = 10, 12 -> 6 to 10 us; k = 100,
-// 60 and 33 -> 22 and 17 us; 1000 queries, k = 10, 61 to 75 -> 12 to 18 us.
+// Per launch under the profiler, with waves sorting chunks in 64 KiB of LDS (1024 threads per query), with
+// every threshold counted out, and now: one query, k = 10, 12, 11, 10.5 us; k = 100, 60 and 33, 21 and 18, 12; 1000 queries,
+// k = 10, 61 to 75, 13 to 19, 11 to 17.
 // ===========================================================================
 constexpr uint32_t kFinalStage = 2048;     // candidates copied to LDS when some segment is long
 constexpr uint32_t kFinalLong = 128;       // ... of which this many segments can be
+constexpr int kFinalPartsMost = 1, kFinalPartsFrom = 64;       // so many queries, and so deep a floor: segments that four threads each read (3M x 1536 2-bit, one query, k = 100 260 -> 254 us; four, k = 64 224 and 227)
 static_assert(kSelectKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
 
-template <uint32_t T>
+template <uint32_t T, uint32_t PARTS>
 __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                const uint32_t *__restrict__ cand_cnt, uint32_t n_seg,
                                                uint32_t seg_stride, int k_eff, int k_floor,
@@ -955,6 +956,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ uint64_t stage[kFinalStage];
     __shared__ SelectShared sh;
+    __shared__ TopShared top;
     __shared__ uint32_t any_full, any_long, long_n, n_kept;
     __shared__ uint32_t long_seg[kFinalLong], long_pos[kFinalLong], long_cnt[kFinalLong];
     if (launch_switched_off(run_if)) return;
@@ -965,29 +967,31 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     if (clear_flag != nullptr && qn == 0 && t == 0) *clear_flag = 0u;
     if (stamp != nullptr && !sampling && qn == 0 && t == 0) *stamp = wall_clock64();
     if (t == 0) { any_full = 0u; any_long = 0u; long_n = 0u; n_kept = 0u; }
-    for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
     __syncthreads();
-    // every thread owns a contiguous run of this query's segments
-    const uint32_t per = (n_seg + T - 1) / T;
-    const uint32_t s0 = min(t * per, n_seg), s1 = min(s0 + per, n_seg);
+    // every thread owns a contiguous run of this query's segments, or sixteen places of one
+    const uint32_t per = (n_seg * PARTS + T - 1) / T;
+    const uint32_t s0 = PARTS > 1 ? min(t / PARTS, n_seg) : min(t * per, n_seg), s1 = PARTS > 1 ? min(s0 + 1u, n_seg) : min(s0 + per, n_seg);
     const uint32_t *cnt = cand_cnt + size_t(qn) * seg_stride;
     const uint64_t *segs = cand + size_t(qn) * seg_stride * kSegCap;
     constexpr uint32_t kShort = 16;
+    static_assert(PARTS == 1 || PARTS * kShort == kSegCap, "a segment is dealt out whole");
+    const uint32_t at0 = PARTS > 1 ? t % PARTS * kShort : 0u;
     // One segment per thread (the usual case): its head is requested together with its count, not
     // after it -- the segment's memory is there whatever the count says.
-    const bool one_each = per == 1;
+    const bool one_each = PARTS > 1 || per == 1;
     uint64_t head[kShort];
 #pragma unroll
     for (uint32_t e = 0; e < kShort; ++e) head[e] = 0ull;
     uint32_t mine = 0;
     if (one_each) {
         if (s0 < s1) {
-            const uint64_t *src = segs + size_t(s0) * kSegCap;
+            const uint64_t *src = segs + size_t(s0) * kSegCap + at0;
             const uint32_t c = cnt[s0];
 #pragma unroll
             for (uint32_t e = 0; e < kShort; ++e) head[e] = src[e];
             if (c > kSegCap) any_full = 1u;
             mine = min(c, uint32_t(kSegCap));
+            if (PARTS > 1) mine = min(mine - min(mine, at0), kShort);
             if (mine > kShort) any_long = 1u;
         }
     } else {
@@ -1003,18 +1007,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
         const uint32_t v = __shfl_up(incl, off);
         if (lane >= uint32_t(off)) incl += v;
     }
-    // (largest and smallest score word of what the thread holds, for the usual case)
-    uint32_t hi_max = 0u, hi_min_inv = 0u;
-#pragma unroll
-    for (uint32_t e = 0; e < kShort; ++e) {
-        if (e < mine) {
-            hi_max = max(hi_max, uint32_t(head[e] >> 32));
-            hi_min_inv = max(hi_min_inv, ~uint32_t(head[e] >> 32));
-        }
-    }
-    hi_max = wave_umax(hi_max);
-    hi_min_inv = wave_umax(hi_min_inv);
-    if (lane == 63u) { sh.w_sum[wv] = incl; sh.w_max[wv] = hi_max; sh.w_min[wv] = hi_min_inv; }
+    if (lane == 63u) sh.w_sum[wv] = incl;
     __syncthreads();
     uint32_t base = incl - mine, total = 0;
     for (uint32_t w = 0; w < W; ++w) { if (w < wv) base += sh.w_sum[w]; total += sh.w_sum[w]; }
@@ -1093,31 +1086,14 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
             }
         }
     };
-    uint64_t threshold = 0ull;
-    if (total > 256u) {
-        if (!held) {
-            hi_max = 0u;
-            hi_min_inv = 0u;
-            each([&](uint64_t k) {
-                hi_max = max(hi_max, uint32_t(k >> 32));
-                hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
-            });
-            hi_max = wave_umax(hi_max);
-            hi_min_inv = wave_umax(hi_min_inv);
-            if (lane == 63u) { sh.w_max[wv] = hi_max; sh.w_min[wv] = hi_min_inv; }
-            __syncthreads();
-        }
-        uint32_t mx = 0u, mn_inv = 0u;
-        for (uint32_t w = 0; w < W; ++w) { mx = max(mx, sh.w_max[w]); mn_inv = max(mn_inv, sh.w_min[w]); }
-        threshold = select_threshold<T>(each, mx, mn_inv, need, sh);
+    // (256 keys are ranked as they are)
+    uint32_t least = 1u;
+    if (total > 256u && need <= kSelectTopMost) {
+        uint32_t most = 0u;
+        each([&](uint64_t k) { most = max(most, uint32_t(k >> 32)); });
+        least = select_top<T>(most, need, top);
     }
-    each([&](uint64_t k) {
-        if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
-    });
-    __syncthreads();
-    const uint32_t n = n_kept;
-    if (t < 2u) kept[n + t] = 0ull;                             // (ranked in pairs)
-    __syncthreads();
+    const uint32_t n = keep_best<T>(each, least, need, kept, n_kept, sh, need > kSelectTopMost && total > 256u);
     const size_t row = row_map ? size_t(row_map[qn]) : size_t(qn);   // a repeated pass writes to the rows of the queries it repeats
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];
@@ -1438,9 +1414,10 @@ hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
                            out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp);
     };
-    if (n_seg <= 256) launch(k_final<256>, 256);
-    else if (n_seg <= 512) launch(k_final<512>, 512);
-    else launch(k_final<1024>, 1024);
+    if (n_seg <= 256 && nq <= kFinalPartsMost && k_floor >= kFinalPartsFrom) launch(k_final<1024, 4>, 1024);
+    else if (n_seg <= 256) launch(k_final<256, 1>, 256);
+    else if (n_seg <= 512) launch(k_final<512, 1>, 512);
+    else launch(k_final<1024, 1>, 1024);
     return hipGetLastError();
 }
 

@@ -212,41 +212,6 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
     return a.best_rows ? form(IntC<kBestRows>{}) : split ? form(IntC<kBestSplit>{}) : form(IntC<kBestPlane>{});
 }
 
-// The keys whose score words reach `least`, which at least `need` of all keys do or which is 1, into kept, two zeros behind
-// them: how many.  Where they are too many for it, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
-// behind a barrier that comes between; met by all T threads.
-template <uint32_t T, typename Each>
-__device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, uint32_t need, uint64_t *kept, uint32_t &n_kept, SelectShared &sh) {
-    const uint32_t t = threadIdx.x;
-    each([&](uint64_t k) {
-        if (uint32_t(k >> 32) < least) return;
-        const uint32_t at = atomicAdd(&n_kept, 1u);
-        if (at < kSelectKept) kept[at] = k;
-    });
-    __syncthreads();
-    uint32_t n = n_kept;
-    if (n > kSelectKept) {
-        for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
-        uint32_t hi_max = 0u, hi_min_inv = 0u, mx, mn_inv;
-        each([&](uint64_t k) {
-            hi_max = max(hi_max, uint32_t(k >> 32));
-            hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
-        });
-        select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);       // (everyone has read n_kept)
-        const uint64_t threshold = select_threshold<T>(each, mx, mn_inv, need, sh);
-        if (t == 0) n_kept = 0u;
-        __syncthreads();
-        each([&](uint64_t k) {
-            if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
-        });
-        __syncthreads();
-        n = n_kept;
-    }
-    if (t < 2u) kept[n + t] = 0ull;
-    __syncthreads();
-    return n;
-}
-
 // ===========================================================================
 // The floor a sample's best rows give: a workgroup per query takes the k_floor-th best of the sampled blocks' best
 // scores, which k_floor scanned rows reach.

@@ -71,6 +71,7 @@ __device__ __forceinline__ uint64_t select_threshold(const Each &each, uint32_t 
 // best words of groups of threads, 64 of them or, from 17 on, 256.  For words dealt out at random few more than `need` reach it
 // (k = 10 of 64 groups: 10.8; 100 of 256: 126): one pass over them and one barrier (two), where counting them into bins takes a range and two
 // passes of four barriers.  `most`: the largest of the calling thread's words, 0 for none.  Met by all T threads.
+constexpr uint32_t kSelectTopMost = 128;       // (of 256 groups)
 struct TopShared {
     __attribute__((aligned(16))) uint32_t groups[256 + 16];      // (four words of padding after every 64: lanes that read 64 apart spread over the banks)
     uint32_t w_top[16];
@@ -135,6 +136,45 @@ __device__ __forceinline__ uint32_t rank_in(const uint64_t *kept, uint32_t n, ui
         rank += (o.x > k ? 1u : 0u) + (o.y > k ? 1u : 0u);
     }
     return rank;
+}
+
+// The keys whose score words reach `least`, which at least `need` of all keys do or which no key is below, into kept, two zeros behind
+// them: how many.  Where they are too many for it, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
+// behind a barrier that comes between; met by all T threads.  count: there are too many for it.
+template <uint32_t T, typename Each>
+__device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, uint32_t need, uint64_t *kept, uint32_t &n_kept, SelectShared &sh,
+                                              bool count = false) {
+    const uint32_t t = threadIdx.x;
+    uint32_t n = kSelectKept + 1u;
+    if (!count) {
+        each([&](uint64_t k) {
+            if (uint32_t(k >> 32) < least) return;
+            const uint32_t at = atomicAdd(&n_kept, 1u);
+            if (at < kSelectKept) kept[at] = k;
+        });
+        __syncthreads();
+        n = n_kept;
+    }
+    if (n > kSelectKept) {
+        for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
+        uint32_t hi_max = 0u, hi_min_inv = 0u, mx, mn_inv;
+        each([&](uint64_t k) {
+            hi_max = max(hi_max, uint32_t(k >> 32));
+            hi_min_inv = max(hi_min_inv, ~uint32_t(k >> 32));
+        });
+        select_range<T>(hi_max, hi_min_inv, sh, mx, mn_inv);       // (everyone has read n_kept)
+        const uint64_t threshold = select_threshold<T>(each, mx, mn_inv, need, sh);
+        if (t == 0) n_kept = 0u;
+        __syncthreads();
+        each([&](uint64_t k) {
+            if (k >= threshold) kept[atomicAdd(&n_kept, 1u)] = k;
+        });
+        __syncthreads();
+        n = n_kept;
+    }
+    if (t < 2u) kept[n + t] = 0ull;
+    __syncthreads();
+    return n;
 }
 
 }  // namespace tv
