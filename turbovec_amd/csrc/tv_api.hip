@@ -499,17 +499,14 @@ int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepar
     r.qbias = out.d_qbias = ar.take<float>(nq_pad);
     out.table_bytes_per_tile = mode_p ? size_t(g.nch) * 2048 : size_t(g.nch) * 1024 * tv::kQTile;
     r.tables = out.d_tables = ar.take<uint8_t>(nq_pad / tv::kQTile * out.table_bytes_per_tile);
+    const bool mx = !mode_p && for_append && lut_mx_serves(ix, nq);
+    if (mx) r.tables_mx = out.d_tables_mx = ar.take<uint8_t>(tv::mx_table_bytes(g.nch, g.bits, nq));
     r.stamp = stamp;
     r.cleared = cleared;
     TV_HIP(tv::launch_prep(r, g, nq, nq_pad, ix->stream));
-    if (!mode_p) {
-        if (for_append && lut_mx_serves(ix, nq)) {
-            out.d_tables_mx = ar.take<uint8_t>(tv::mx_table_bytes(g.nch, g.bits, nq));
-            TV_HIP(tv::launch_lut_fragments(out.d_tables, out.d_tables_mx, g.nch, g.bits, nq, ix->stream));
-        } else if (for_append && lut16_serves(ix) && nq >= size_t(lut16_min_queries(ix))) {
-            out.d_tables16 = ar.take<uint8_t>(tv::lut16_table_bytes(g.nch, nq));
-            TV_HIP(tv::launch_lut_interleave16(out.d_tables, out.d_tables16, g.nch, nq, ix->stream));
-        }
+    if (!mode_p && !mx && for_append && lut16_serves(ix) && nq >= size_t(lut16_min_queries(ix))) {
+        out.d_tables16 = ar.take<uint8_t>(tv::lut16_table_bytes(g.nch, nq));
+        TV_HIP(tv::launch_lut_interleave16(out.d_tables, out.d_tables16, g.nch, nq, ix->stream));
     }
     return TV_OK;
 }

@@ -116,6 +116,7 @@ struct PrepRequest {
     float cs;
     const float *centroids;
     uint8_t *tables;
+    uint8_t *tables_mx;             // or null: u8 tables also as the operands of k_scan_lut_mx
     float *qscale, *qbias;
     float *rot_out;                 // or null
     uint64_t *stamp;                // or null: kStampsBefore words
@@ -145,8 +146,9 @@ struct MxShape {
     unsigned groups, wgs, sub;   // query groups, workgroups per group, segments per workgroup and query
     int nt, blk;                 // query tiles per group, blocks per wave and round
 };
-size_t mx_table_bytes(int nch, int bits, size_t nq);
-hipError_t launch_lut_fragments(const uint8_t *d_src, uint8_t *d_dst, int nch, int bits, size_t nq, hipStream_t s);
+// Steps (code bytes per lane half, or pairs of them) in a chunk of 32 byte-groups.
+__host__ __device__ constexpr int mx_steps(int entries) { return entries == 16 ? 16 : 8; }
+constexpr size_t mx_table_bytes(int nch, int bits, size_t nq) { return (nq + kQTile - 1) / kQTile * size_t(nch) * size_t(mx_steps(bits == 3 ? 8 : 16)) * 2048; }
 MxShape mx_shape(int device, size_t nq, size_t level_blocks, bool open_floors);
 int mx_segments();
 int mx_round_blocks(int device, size_t nq);   // blocks a launch over nq queries works through per round

@@ -14,7 +14,7 @@
 //
 // A operands are built on the vector ALU from the raw codes: per code byte two shifts of a one
 // and a byte permute, shared by the NT query tiles the wave works on; B operands -- the tables,
-// laid out by k_lut_fragments in the order the instruction wants them -- pass through LDS, each
+// laid out by k_prep_lut in the order the instruction wants them -- pass through LDS, each
 // read feeding the wave's BLK blocks.  A workgroup of eight waves takes 8 * BLK blocks and one
 // group of NT query tiles through the whole row, chunk by chunk; the launch's groups work side by
 // side, each on its share of the workgroups (dealt so that with eight or sixteen groups an XCD sees
@@ -39,53 +39,6 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 
 constexpr int kMxThreads = 512, kMxWaves = kMxThreads / 64;
 constexpr int kMxRing = 4;       // LDS slots, one slice of the tables each
-
-// Steps (code bytes per lane half, or pairs of them) in a chunk of 32 byte-groups.
-constexpr int mx_steps(int entries) { return entries == 16 ? 16 : 8; }
-size_t mx_table_bytes(int nch, int bits, size_t nq) {
-    return (nq + kQTile - 1) / kQTile * size_t(nch) * size_t(mx_steps(bits == 3 ? 8 : 16)) * 2048;
-}
-
-// The row-major tables of k_prep_lut -> B operands.  Piece ((tile, chunk, step j, part p), lane
-// (u, n)) is 16 bytes of query 32 tile + n: the 16 lanes-halves p of the A operand meet part p, and
-// of that lane's stored bytes 0..7 half u = 0, 8..15 half u = 1.
-//   16-entry tables: byte-group 16 p + j of the chunk, its high (u = 0) or low (u = 1) nibble's table
-//    8-entry tables: byte-group 16 p + 2 j + u, the 8 entries of its high nibble, then of its low
-// A table's entries come in the order the operand's bits are cheapest in: the nibble's low bits are
-// the stored slot's number (three of four bits, two of three), its highest the choice of positions, so
-// that entry 8 p + 2 g + s (4 p + 2 g + s) is the group g's fourth 2 p + s.
-__device__ __forceinline__ uint32_t zip_lo(uint32_t a, uint32_t b) { return (a & 0xffffu) | (b << 16); }
-__device__ __forceinline__ uint32_t zip_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
-template <int ENT>
-__global__ __launch_bounds__(256) void k_lut_fragments(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int nch) {
-    __shared__ uint4 rows[kQTile * 64];          // [query][1 KiB]
-    const int c = blockIdx.x, t = threadIdx.x;
-    const size_t tile = blockIdx.y;
-    for (int i = t; i < kQTile * 64; i += 256)
-        rows[i] = reinterpret_cast<const uint4 *>(src + ((tile * kQTile + i / 64) * nch + c) * 1024)[i % 64];
-    __syncthreads();
-    constexpr int kSteps = mx_steps(ENT);
-    uint4 *out = reinterpret_cast<uint4 *>(dst) + (tile * nch + c) * size_t(kSteps) * 128;
-    for (int i = t; i < kSteps * 128; i += 256) {
-        const int n = i & 31, u = (i >> 5) & 1, p = (i >> 6) & 1, j = i >> 7;
-        const uint4 *row = rows + n * 64;
-        if (ENT == 16) {
-            const uint4 v = row[(16 * p + j) * 2 + u];
-            out[i] = uint4{zip_lo(v.x, v.z), zip_hi(v.x, v.z), zip_lo(v.y, v.w), zip_hi(v.y, v.w)};
-        } else {
-            const uint4 hi = row[(16 * p + 2 * j + u) * 2], lo = row[(16 * p + 2 * j + u) * 2 + 1];
-            out[i] = uint4{zip_lo(hi.x, hi.y), zip_hi(hi.x, hi.y), zip_lo(lo.x, lo.y), zip_hi(lo.x, lo.y)};
-        }
-    }
-}
-
-hipError_t launch_lut_fragments(const uint8_t *d_src, uint8_t *d_dst, int nch, int bits, size_t nq, hipStream_t s) {
-    const unsigned tiles = unsigned((nq + kQTile - 1) / kQTile);
-    if (tiles == 0) return hipSuccess;
-    if (bits == 3) hipLaunchKernelGGL(k_lut_fragments<8>, dim3(unsigned(nch), tiles), dim3(256), 0, s, d_src, d_dst, nch);
-    else hipLaunchKernelGGL(k_lut_fragments<16>, dim3(unsigned(nch), tiles), dim3(256), 0, s, d_src, d_dst, nch);
-    return hipGetLastError();
-}
 
 __device__ __forceinline__ void mx_dma16(uint32_t lds_addr, const void *sbase, uint32_t lane16) {
     const uint32_t u = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_addr)));

@@ -19,7 +19,7 @@ struct PrepArgs {
     const float *shift, *scale;     // null without a TQ+ pair
     float inv_sqrt_block;
     int dim, log_block, G, nch;
-    uint8_t *tables;
+    uint8_t *tables, *mx;           // mx: or null
     float *qscale, *qbias;
     float *rot_out;                 // when given: the rotated (and calibrated) rows
     size_t nq;
@@ -245,6 +245,30 @@ __device__ __forceinline__ float lut_entry(const float *q, const float *cen, int
     return s;
 }
 
+// A byte-group's two tables as B operands of k_scan_lut_mx.  Piece ((tile, chunk, step j, part p), lane
+// (u, n)) is 16 bytes of query 32 tile + n: the 16 lanes-halves p of the A operand meet part p, and
+// of that lane's stored bytes 0..7 half u = 0, 8..15 half u = 1.
+//   16-entry tables: byte-group 16 p + j of the chunk, its high (u = 0) or low (u = 1) nibble's table
+//    8-entry tables: byte-group 16 p + 2 j + u, the 8 entries of its high nibble, then of its low
+// A table's entries come in the order the operand's bits are cheapest in: the nibble's low bits are
+// the stored slot's number (three of four bits, two of three), its highest the choice of positions, so
+// that entry 8 p + 2 g + s (4 p + 2 g + s) is the group g's fourth 2 p + s.
+// (In a launch of their own they took 5 us of 37 queries' 219 and the gap in front of it.)
+__device__ __forceinline__ uint32_t zip_lo(uint32_t a, uint32_t b) { return (a & 0xffffu) | (b << 16); }
+__device__ __forceinline__ uint32_t zip_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
+template <int BITS>
+__device__ __forceinline__ void mx_put(uint8_t *mx, int nch, int qi, int g, uint4 hi, uint4 lo) {
+    constexpr int kSteps = mx_steps(BITS == 3 ? 8 : 16);
+    const int p = (g & 31) >> 4, in = g & 15, j = BITS == 3 ? in >> 1 : in;
+    uint4 *out = reinterpret_cast<uint4 *>(mx) + ((size_t(qi / kQTile) * nch + size_t(g >> 5)) * kSteps + j) * 128 + p * 64 + qi % kQTile;
+    if constexpr (BITS == 3) {
+        out[(in & 1) * 32] = make_uint4(zip_lo(hi.x, hi.y), zip_hi(hi.x, hi.y), zip_lo(lo.x, lo.y), zip_hi(lo.x, lo.y));
+    } else {
+        out[0] = make_uint4(zip_lo(hi.x, hi.z), zip_hi(hi.x, hi.z), zip_lo(hi.y, hi.w), zip_hi(hi.y, hi.w));
+        out[32] = make_uint4(zip_lo(lo.x, lo.z), zip_hi(lo.x, lo.z), zip_lo(lo.y, lo.w), zip_hi(lo.y, lo.w));
+    }
+}
+
 template <int BITS>
 __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
     extern __shared__ __align__(16) float prep_lds[];
@@ -258,6 +282,8 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
     const int t = threadIdx.x, G = a.G;
     if (qi >= a.nq) {
         for (int i = t; i < a.nch * 64; i += kPrepThreads) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
+        if (a.mx != nullptr)
+            for (int g = t; g < a.nch * 32; g += kPrepThreads) mx_put<BITS>(a.mx, a.nch, int(qi), g, make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0));
         if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
         return;
     }
@@ -311,9 +337,11 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
                 }
             }
         }
+        const uint4 hi = make_uint4(w[0], w[1], w[2], w[3]), lo = make_uint4(w[4], w[5], w[6], w[7]);
         uint4 *o = reinterpret_cast<uint4 *>(dst + size_t(g) * 32);
-        o[0] = make_uint4(w[0], w[1], w[2], w[3]);
-        o[1] = make_uint4(w[4], w[5], w[6], w[7]);
+        o[0] = hi;
+        o[1] = lo;
+        if (a.mx != nullptr) mx_put<BITS>(a.mx, a.nch, int(qi), g, hi, lo);
     }
     if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
     if (t == 0 && a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
@@ -328,7 +356,7 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     a.q = r.q; a.signs = r.signs; a.perms = r.perms; a.shift = r.shift; a.scale = r.scale;
     a.inv_sqrt_block = r.inv_sqrt_block;
     a.dim = g.dim; a.log_block = __builtin_ctz(unsigned(r.block)); a.G = g.G; a.nch = g.nch;
-    a.tables = r.tables; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
+    a.tables = r.tables; a.mx = r.tables_mx; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
     a.nq = nq; a.stamp = r.stamp; a.cleared = r.cleared;
     const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
     auto launch = [&](auto kernel, auto... rest) -> hipError_t {
