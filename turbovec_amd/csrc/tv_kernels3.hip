@@ -32,7 +32,7 @@ namespace tv {
 constexpr int kWideThreads = 512;    // the widest form (and the matrix-unit probe): 8 waves, 2 per SIMD
 constexpr int kWideWaves = kWideThreads / 64;
 // LDS slots of one slice each: five when slices are handed over one by one (four requested ahead) or
-// two at a time, 2 HO + 1 when more are handed over together.
+// two at a time, 2 HO + 1 when more are handed over together, whole tiles of one slice or one tile's.
 constexpr int wide_ring(int ho) { return ho <= 2 ? 5 : 2 * ho + 1; }
 
 // 16 bytes per lane from global memory (uniform base + 16 * lane) straight into LDS at
@@ -134,7 +134,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     static_assert(KS == 1 || (KS == 2 && WAVES == 4 && BLK == 1 && HO == 1), "row halves go to the wave pairs of the four-wave form");
     constexpr int kWideRing = wide_ring(HO);
     static_assert(!ROWS || KS == 1, "a row whole");
-    static_assert(HO == 1 || (SPT % HO == 0 && kWideRing >= 2 * HO + 1), "slices handed over together must fit the ring twice");
+    static_assert(HO == 1 || ((SPT % HO == 0 || HO % SPT == 0) && kWideRing >= 2 * HO + 1), "slices handed over together must fit the ring twice");
+    constexpr int kTilesPerHandOver = HO > SPT ? HO / SPT : 1;
     extern __shared__ __align__(16) uint8_t smem_all[];
     if (launch_switched_off(a.run_if)) return;
     // (the byte table, when there is one, sits at the start of the kernel's LDS -- no static
@@ -267,6 +268,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     // slices after g, requested at the hand-over before, must have landed (nothing younger is in
     // flight: the wait is for everything); after the barrier those are whole and the HO slices
     // behind g are free: the next HO slices are requested into their slots.
+    // HO > SPT: in the last slice of every HO / SPT-th tile of the stream, wherever a round of tiles ends.
     auto hand_over_group = [&]() {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -278,12 +280,20 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         for (int i = 0; i < kAhead - 1; ++i) request_next();
         hand_over(IntC<kAhead - 2>{});
     } else {
-        // slices 0 .. 2 HO - 1 requested and whole: the state the first group hand-over expects
+        // slices 0 .. 2 HO - 1 requested, the first HO whole: the state the first group hand-over expects
         for (int i = 0; i < 2 * HO; ++i) request_next();
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (kExtra != 0 && wave < kExtra) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HO * (kPieces + 1)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HO * kPieces) : "memory");
         __syncthreads();
     }
     int use_slot = 0;                                       // ring slot of the slice consumed next
+    // (the same in every wave; a round of tiles may end between two hand-overs)
+    int tiles_since = 0;
+    auto group_ends = [&]() -> bool {
+        if constexpr (kTilesPerHandOver == 1) return true;
+        tiles_since = tiles_since + 1 == kTilesPerHandOver ? 0 : tiles_since + 1;
+        return tiles_since == 0;
+    };
 
     v4i alo[BLK][NCH], ahi[BLK][NCH];
     v16i acc[BLK];
@@ -312,6 +322,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
             if constexpr (m == kM / 2) {
                 if constexpr (HO == 1) hand_over(IntC<kAhead - 2>{});
                 else if constexpr (decltype(slice_no)::value % HO == HO - 1) hand_over_group();
+                else if constexpr (HO > SPT && decltype(slice_no)::value == SPT - 1) {
+                    if (group_ends()) hand_over_group();
+                }
             }
             lds_wait<NB - 1>(w[m % NB]);
             static_for<BLK>([&](auto kk) {
@@ -594,7 +607,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                     for (int i = 0; i < SPT; ++i) hand_over(IntC<kAhead - 2>{});
                 } else {
 #pragma unroll
-                    for (int i = 0; i < SPT / HO; ++i) hand_over_group();
+                    for (int i = 0; i < (HO > SPT ? 1 : SPT / HO); ++i)
+                        if (group_ends()) hand_over_group();
                 }
                 if constexpr (KS == 2) __syncthreads();     // the tile's exchange barrier, met by every wave
             }
@@ -766,13 +780,19 @@ hipError_t launch_scan_p4_wide(const ScanArgs &a, int grid, hipStream_t s) {
         // <chunks, B-operand registers, waves, slices per tile, blocks per wave, slices per hand-over>
         // One hand-over per tile (two slices) measured 2.5 to 5 % faster than one per slice in the
         // eight-wave forms with two slices per tile, and 2 % slower in the four-wave forms.
-        case 2: return launch_wide_n<2, 2, 8, 1, 6>(a, grid, s);
-        case 3: return launch_wide_n<3, 2, 8, 1, 4>(a, grid, s);
-        case 4: return launch_wide_n<4, 2, 8, 1, 4>(a, grid, s);
-        case 5: return launch_wide_n<5, 2, 8, 1, 3>(a, grid, s);
-        case 6: return launch_wide_n<6, 2, 8, 1, 3>(a, grid, s);
-        case 7: return launch_wide_n<7, 2, 8, 1, 2>(a, grid, s);
-        case 8: return launch_wide_n<8, 4, 8, 1, 2>(a, grid, s);
+        // Tiles of up to 8 chunks (a slice each) are over before the waves' scoring evens out: every wave waits for the one with a candidate.
+        // A hand-over for several, as many as leave the ring room beside 1024 queries.  us a search with one a tile, with two,
+        // and so: 6M x 128, 500 queries 775, 719, 673; 4M x 192, 1000 1105, 1018, 950; 2M x 256, 1024 708, 667, 637, 4M, 300 544, 530, 505;
+        // 2M x 320, 1000 803, 765, 750; 3M x 384, 1024 1221 and 1170; 1.5M x 432, 500 483, 458, 451; 2M x 512, 1024 1095, 1062, 1050,
+        // 300 485, 476, 460.  Deeper gives no more (5 and 6 chunks with five, 7 with four), nor do two tiles at 10 to 14 chunks (2M x
+        // 768, 300 queries 637 and 640, 2M x 640, 400 612 and 619, 1.5M x 896, 200 435 and 440).
+        case 2: return launch_wide_n<2, 2, 8, 1, 6, 8>(a, grid, s);
+        case 3: return launch_wide_n<3, 2, 8, 1, 4, 6>(a, grid, s);
+        case 4: return launch_wide_n<4, 2, 8, 1, 4, 6>(a, grid, s);
+        case 5: return launch_wide_n<5, 2, 8, 1, 3, 4>(a, grid, s);
+        case 6: return launch_wide_n<6, 2, 8, 1, 3, 4>(a, grid, s);
+        case 7: return launch_wide_n<7, 2, 8, 1, 2, 3>(a, grid, s);
+        case 8: return launch_wide_n<8, 4, 8, 1, 2, 3>(a, grid, s);
         case 10: return launch_wide_n<10, 2, 8, 2, 2, 2>(a, grid, s);
         case 12: return launch_wide_n<12, 2, 8, 2, 1, 2, 1, true>(a, grid, s);   // two blocks per wave would spill 21 registers
         case 14: return launch_wide_n<14, 2, 8, 2, 1, 2, 1, true>(a, grid, s);

@@ -487,7 +487,7 @@ static hipError_t launch_mx_blk(const ScanArgs &a, const MxShape &m, hipStream_t
 }
 
 // One append-mode launch: a.nq_tile = all queries of the chunk, a.tables = their B operands
-// (k_lut_fragments), scales, floors and segments by query.
+// (of k_prep_lut), scales, floors and segments by query.
 hipError_t launch_scan_lut_mx(const ScanArgs &a, const MxShape &m, int bits, hipStream_t s) {
     if (a.classic != 0 || a.nq_tile <= 0 || (a.best_out == nullptr && size_t(m.wgs) * m.sub > a.seg_stride)) return hipErrorInvalidValue;
     if (bits == 3) return m.nt == 1 ? launch_mx_blk<8, 1>(a, m, s) : launch_mx_blk<8, 2>(a, m, s);

@@ -472,7 +472,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
 
 // ===========================================================================
 // Few rows (a filter's, as a rule): the scan has kept every row's score, and nothing is scored again.  Writing and reading
-// a score per row and query takes less than k_pick's second scoring of whole blocks (2000 rows x 3072, 1024 queries, k = 10: this kernel 6 us,
+// a score per row and query takes less than k_pick's second scoring of whole blocks (2000 rows x 3072, 1024 queries, k = 10: this kernel 6 to 11 us,
 // k_pick 80; all latency at that size).
 // ===========================================================================
 template <uint32_t T, uint32_t H>
