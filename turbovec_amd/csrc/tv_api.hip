@@ -436,14 +436,19 @@ int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCOR
 // takes one query at a time.  One pass for up to sixteen queries beats the matrix-unit scan's
 // half-empty tile (1M x 1536 2-bit, 16 queries: 0.26 ms a search against 0.30); from 17 on it
 // would be two (33 queries: 0.56 against 0.40 ms; 400: 4.6 against 2.2).  Below about 4096 (block,
-// query tile) pairs most of the matrix-unit scan's waves have no block, and the sixteen-query passes
+// query tile) pairs most of the matrix-unit scan's waves have no block, and up to three sixteen-query passes
 // are the faster ones (20K x 1536 2-bit, 33 queries, 1250 pairs: 153 us against 155; 65K rows, 4096
-// pairs: 165 against 131).
-constexpr size_t kMxMinPairs = 4096;
+// pairs: 165 against 131).  From four passes on (us a search, the passes and the matrix-unit scan):
+//  - 1400 pairs: 12K x 1536 2-bit, 100 queries 75 and 62, 15K x 3072, 96 queries 106 and 91; 1000 pairs are level or worse (15K x 3072, 49 queries 83 and 90).
+//  - 3-bit codes, half the products per byte: 2000 x 3072, 65 queries 123 and 115, 700 x 1536, 65 queries, k = 100 183 and 79.
+//  - up to six chunks: 1000 x 768 2-bit, 129 queries 44.5 and 43.1, x 128 37.5 and 32.1; twelve 57.5 and 59.2.
+//  - many passes, one after the other where the search is sampled: 6000 x 3072 2-bit, 1000 queries 197 either way, 3000 1430 and 166, without
+//    sampling 222 and 160; 4000, 400 queries 131 and 112, but 129 queries 86 and 92.
+constexpr size_t kMxMinPairs = 4096, kMxMinPairsMany = 1400, kMxMany = 3 * tv::kLut16Queries, kMxAlways = 384;
 bool lut_mx_serves(const tv_index *ix, size_t cq) {
-    const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
-    return effective_mode(ix) == TV_SCORE_L_U32 && !ix->no_lut16 && !ix->no_lut_mx && cq > size_t(tv::kLut16Queries) &&
-           n_blocks * tiles >= kMxMinPairs;
+    const size_t n_blocks = (ix->rows().n + tv::kVecBlock - 1) / tv::kVecBlock, tiles = (cq + tv::kQTile - 1) / tv::kQTile, pairs = n_blocks * tiles;
+    if (effective_mode(ix) != TV_SCORE_L_U32 || ix->no_lut16 || ix->no_lut_mx || cq <= size_t(tv::kLut16Queries)) return false;
+    return pairs >= kMxMinPairs || (cq > kMxMany && (pairs >= kMxMinPairsMany || ix->geo.bits == 3 || ix->geo.nch <= 6 || cq > kMxAlways));
 }
 bool lut16_serves(const tv_index *ix) {
     return (effective_mode(ix) == TV_SCORE_L_U32 || effective_mode(ix) == TV_SCORE_L_CLASSIC) && !ix->no_lut16;
