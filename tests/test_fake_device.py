@@ -186,6 +186,45 @@ assert used.value == 0
 ''')
 
 
+def test_room_to_grow_is_not_taken_from_others(fake):
+    """Rows that fit as they are: the library gives nothing up, neither pooled blocks nor a filtered search's copy, for the room beyond them."""
+    fake(FILTERED + '''
+a, b, c = index(400_000), index(100_000), index(50_000)
+assert filtered(a, 64) == 1
+c.close()                                # 1.6 MB of codes are in the pool
+held, before = a.workspace_bytes()[0], used.value
+# needed: 3.96 MB; by half: 5.4; twice: 7.2
+limit.value = before + 4_200_000
+b.append_rows(np.zeros((10_000, 32), np.uint8), np.zeros(10_000, np.float32))
+assert len(b) == 110_000 and a.workspace_bytes()[0] == held
+assert used.value > before + 3_000_000   # (100000 rows' codes went to the pool, their scales back to the device)
+a.close(); b.close()
+assert used.value == 0
+''')
+
+
+def test_indexes_that_grow_ahead_hold_no_more_than_a_bound(fake):
+    """Many indexes that have grown once: what they hold beyond growing by half is 256 MiB in all, and is there again once they are gone."""
+    fake('''
+n, row = 1_000_000, 36                   # dim 64: 32 bytes and a scale; a multiple of a block's rows
+def grown():
+    ix = index(n)
+    before = used.value
+    ix.append_rows(np.zeros((1, 32), np.uint8), np.zeros(1, np.float32))
+    return ix, (used.value - before) / (n * row)      # (the old blocks are in the pool)
+made = [grown() for _ in range(20)]
+growth = [g for _, g in made]
+assert abs(growth[0] - 2.0) < 0.01 and abs(growth[-1] - 1.5) < 0.01, growth
+ahead = sum(growth) - 1.5 * len(growth)
+assert ahead * n * row <= 256 << 20, growth
+for ix, _ in made: ix.close()
+assert used.value == 0
+ix, g = grown()
+assert abs(g - 2.0) < 0.01
+ix.close()
+''')
+
+
 def test_a_copy_of_rows_gives_way_to_the_search_it_is_made_for(fake):
     """Memory for the copy or for the workspace, not for both: the mask is read, as where there is none for the copy."""
     fake(FILTERED + '''

@@ -113,15 +113,19 @@ constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
 // kPoolBytes, handed on only to requests they exceed by a quarter at most, and given back when the last
 // index of the device goes or an allocation fails -- any of an index's, so all of them come through
 // device_alloc.  What filtered searches keep of their allowed rows (tv_spare) goes the same way when the pool was not
-// enough.  An index built by adds allocates 2.6 times its size on
+// enough.  An index built by adds allocates up to 2.6 times its size on
 // the way; fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
-// 1536 rows in four adds: 4 ms a build while cleared memory lasts, 22.8 ms after).
+// 1536 rows in four adds that grew by half: 4 ms a build while cleared memory lasts, 22.8 ms after).
 constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
+// What the indexes of a device may hold beyond growing by half (ensure_capacity): nothing takes it back but their end, so it is
+// a thousandth of the device's memory and not a share of its indexes.
+constexpr size_t kAheadBytes = size_t(256) << 20;
 struct DevicePool {
     std::mutex mu;         // held for the bookkeeping only: allocations, frees and waits are long
     std::mutex giving;     // held while an allocation that failed empties the pool and tries again
     std::vector<std::pair<size_t, void *>> blocks;
     size_t held = 0, indexes = 0;
+    size_t ahead = 0;                // at most kAheadBytes, the sum of the indexes'
     tv_index *newest = nullptr;      // of the device's indexes
     static constexpr int kPinned = 64;
     tv_pinned pinned[kPinned];       // host memory: pinned_take
@@ -146,8 +150,9 @@ void *take_spare(DevicePool &pool) {
 }
 
 thread_local bool g_refused;      // an allocation of this thread's call was refused for good
-// `device` is current.  *got: what the block holds, 0 on failure.
-hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
+// `device` is current.  *got: what the block holds, 0 on failure.  insist: nothing is refused for what the library only keeps;
+// without, nothing is given up for a block that the caller can do without.
+hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got, bool insist = true) {
     DevicePool &pool = g_pool[device];
     {
         std::lock_guard<std::mutex> lock(pool.mu);
@@ -166,7 +171,7 @@ hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got) {
         }
     }
     hipError_t e = hipMalloc(out, bytes);
-    if (e != hipSuccess) {
+    if (e != hipSuccess && insist) {
         (void)hipGetLastError();
         std::lock_guard<std::mutex> giving(pool.giving);      // (another thread's blocks may be on their way back)
         std::unique_lock<std::mutex> lock(pool.mu);
@@ -330,30 +335,57 @@ struct Outgrown {
         (void)release();
     }
 };
-// Room for n_vectors rows.  An index grows to twice its size while that is less than kGrowth more, and by half beyond, or
-// as far as there is memory: 100K rows of 1536 dimensions added four times move 231 MB on the way (461 MB by half each time).
+// What an allocation in the making holds beyond growing by half: the index's from keep() on, in the place of what its old one held.
+struct AheadHold {
+    tv_index *ix;
+    DevicePool &pool;
+    size_t bytes = 0;
+    explicit AheadHold(tv_index *ix_) : ix(ix_), pool(g_pool[ix_->device]) {}
+    AheadHold(const AheadHold &) = delete;
+    bool take(size_t more) {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (pool.ahead - ix->ahead + more > kAheadBytes) return false;
+        pool.ahead += more;
+        bytes = more;
+        return true;
+    }
+    void keep() {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        pool.ahead -= std::exchange(ix->ahead, std::exchange(bytes, 0));
+    }
+    void drop() {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        pool.ahead -= std::exchange(bytes, 0);
+    }
+    ~AheadHold() { drop(); }
+};
+// Room for n_vectors rows.  An index grows to twice its size while the device's indexes hold no more than kAheadBytes for that, and by half
+// beyond: 100K rows of 1536 dimensions added four times move 231 MB on the way (461 MB by half each time).  Where there is no
+// memory for either it grows by what is needed, and only that is worth giving up what others keep.
 // What is beyond the rows is zero -- but for the blocks that rows from the index's last to n_vectors fill, where the
 // caller says that it is about to write all of those on the index's stream (`whole`), and not before it has waited for the
 // stream, which it does before `outgrown` goes.
-constexpr size_t kGrowth = size_t(1) << 30;
 int ensure_capacity(tv_index *ix, size_t n_vectors, Outgrown &outgrown, bool whole) {
     const size_t blocks = (n_vectors + tv::kVecBlock - 1) / tv::kVecBlock;
     if (blocks <= ix->cap_blocks) return TV_OK;
     const size_t bb = ix->geo.block_bytes();
-    size_t cap = std::max(blocks, ix->cap_blocks + std::max(ix->cap_blocks / 2, std::min(ix->cap_blocks, kGrowth / bb)));
-    cap = std::max<size_t>(cap, 64);
+    const size_t needed = std::max<size_t>(blocks, 64), half = std::max(needed, ix->cap_blocks + ix->cap_blocks / 2);
+    size_t cap = std::max(half, 2 * ix->cap_blocks);
+    AheadHold ahead(ix);
+    if (cap > half && !ahead.take((cap - half) * (bb + tv::kVecBlock * sizeof(float)))) cap = half;
     uint8_t *codes = nullptr;
     float *scales = nullptr;
     size_t codes_bytes = 0, scales_bytes = 0;
     hipError_t e = hipSuccess;
-    for (;; cap = std::max<size_t>(blocks, 64)) {
-        e = device_alloc(ix->device, cap * bb, reinterpret_cast<void **>(&codes), &codes_bytes);
+    for (;; cap = cap > half ? half : needed) {
+        if (cap <= half) ahead.drop();
+        e = device_alloc(ix->device, cap * bb, reinterpret_cast<void **>(&codes), &codes_bytes, cap == needed);
         if (e == hipSuccess) {
-            e = device_alloc(ix->device, cap * tv::kVecBlock * sizeof(float), reinterpret_cast<void **>(&scales), &scales_bytes);
+            e = device_alloc(ix->device, cap * tv::kVecBlock * sizeof(float), reinterpret_cast<void **>(&scales), &scales_bytes, cap == needed);
             if (e == hipSuccess) break;
             (void)device_free(ix->device, codes, codes_bytes);
         }
-        if (cap == std::max<size_t>(blocks, 64)) return fail_hip(e, "device_alloc(rows)");
+        if (cap == needed) return fail_hip(e, "device_alloc(rows)");
     }
     const size_t old_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
     const size_t clear = whole ? std::max(old_blocks, n_vectors / tv::kVecBlock) : old_blocks;
@@ -375,6 +407,7 @@ int ensure_capacity(tv_index *ix, size_t n_vectors, Outgrown &outgrown, bool who
     outgrown.codes_bytes = std::exchange(ix->codes_bytes, codes_bytes);
     outgrown.scales_bytes = std::exchange(ix->scales_bytes, scales_bytes);
     ix->cap_blocks = cap;
+    ahead.keep();
     return TV_OK;
 }
 int ensure_capacity(tv_index *ix, size_t n_vectors) {
@@ -1930,6 +1963,7 @@ int tv_index_destroy(tv_index *ix) {
         std::unique_lock<std::mutex> lock(pool.mu);
         (ix->newer ? ix->newer->older : pool.newest) = ix->older;
         if (ix->older) ix->older->newer = ix->newer;
+        pool.ahead -= ix->ahead;
         const bool last = --pool.indexes == 0;
         const auto blocks = last ? pool.empty() : decltype(pool.blocks){};
         uint8_t *pinned[DevicePool::kPinned];

@@ -292,6 +292,7 @@ struct tv_index {
     uint8_t *d_codes = nullptr;
     float *d_scales = nullptr;
     size_t codes_bytes = 0, scales_bytes = 0;   // allocated
+    size_t ahead = 0;              // ... of it beyond growing by half (guarded as the device's pool of blocks is)
     size_t cap_blocks = 0;
     size_t n = 0;
 
