@@ -16,7 +16,8 @@ typedef struct { uint32_t x, y, z; } dim3_t;
 
 /* ---- what a test sets and reads ---- */
 atomic_size_t fake_limit = (size_t)1 << 34, fake_used;
-atomic_int fake_stream_wait_us;       /* how long a stream's wait takes */
+atomic_int fake_stream_wait_us;       /* how long a stream's wait takes ... */
+atomic_int fake_stream_waits;         /* ... and how many there were */
 atomic_int fake_device_busy;          /* the device's wait does not end while this is set ... */
 atomic_int fake_device_waits;         /* ... and this many threads are in one */
 atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
@@ -88,7 +89,7 @@ int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) {
 int hipMemsetAsync(void *p, int v, size_t n, void *s) { (void)s; memset(p, v, n); return ok; }
 int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &last; return ok; }
 int hipStreamDestroy(void *s) { (void)s; return ok; }
-int hipStreamSynchronize(void *s) { (void)s; if (fake_stream_wait_us) usleep(fake_stream_wait_us); return ok; }
+int hipStreamSynchronize(void *s) { (void)s; ++fake_stream_waits; if (fake_stream_wait_us) usleep(fake_stream_wait_us); return ok; }
 int hipEventCreate(void **e) { *e = &last; return ok; }
 int hipEventDestroy(void *e) { (void)e; return ok; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }

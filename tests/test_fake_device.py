@@ -186,6 +186,20 @@ assert used.value == 0
 ''')
 
 
+def test_rows_that_have_room_wait_for_their_own_work_only(fake):
+    """Rows for which there is room: one wait for their codes, one for their scales, none for an index that did not grow."""
+    fake('''
+ix, waits = index(64), var("stream_waits")
+before = waits.value
+ix.append_rows(np.zeros((1, 32), np.uint8), np.zeros(1, np.float32))
+assert waits.value - before == 2, waits.value - before
+before = waits.value
+ix.add(np.ones((1, 64), np.float32))
+assert waits.value - before == 2, waits.value - before      # the row's way to the device, and the encoder
+ix.close()
+''')
+
+
 def test_room_to_grow_is_not_taken_from_others(fake):
     """Rows that fit as they are: the library gives nothing up, neither pooled blocks nor a filtered search's copy, for the room beyond them."""
     fake(FILTERED + '''

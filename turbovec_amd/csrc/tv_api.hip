@@ -412,8 +412,9 @@ int ensure_capacity(tv_index *ix, size_t n_vectors, Outgrown &outgrown, bool who
 }
 int ensure_capacity(tv_index *ix, size_t n_vectors) {
     Outgrown outgrown(ix);
+    const size_t before = ix->cap_blocks;
     const int rc = ensure_capacity(ix, n_vectors, outgrown, false);
-    if (rc != TV_OK || ix->d_codes == nullptr) return rc;
+    if (rc != TV_OK || ix->cap_blocks == before) return rc;
     TV_HIP(hipStreamSynchronize(ix->stream));
     TV_HIP(outgrown.release());
     return TV_OK;
