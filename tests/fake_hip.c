@@ -18,6 +18,7 @@ typedef struct { uint32_t x, y, z; } dim3_t;
 atomic_size_t fake_limit = (size_t)1 << 34, fake_used;
 atomic_int fake_stream_wait_us;       /* how long a stream's wait takes ... */
 atomic_int fake_stream_waits;         /* ... and how many there were */
+atomic_int fake_frees_refused;        /* so many of the next frees of device memory report an error */
 atomic_int fake_device_busy;          /* the device's wait does not end while this is set ... */
 atomic_int fake_device_waits;         /* ... and this many threads are in one */
 atomic_long fake_clock_reads;         /* std::chrono::steady_clock::now() */
@@ -57,7 +58,12 @@ int hipDeviceSynchronize(void) {
     return ok;
 }
 int hipMalloc(void **p, size_t n) { return take(p, n); }
-int hipFree(void *p) { if (p) hipDeviceSynchronize(); return give(p); }
+int hipFree(void *p) {
+    if (p) hipDeviceSynchronize();
+    give(p);
+    if (p && fake_frees_refused > 0) { --fake_frees_refused; return last = out_of_memory; }
+    return ok;
+}
 int hipHostMalloc(void **p, size_t n, unsigned flags) {
     (void)flags;
     const size_t counted = n >= 65536 ? n : 0;

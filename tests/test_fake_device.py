@@ -200,6 +200,25 @@ ix.close()
 ''')
 
 
+def test_an_add_that_fails_shows_none_of_its_rows(fake):
+    """The encoder has run and the outgrown memory cannot be given back: the call says so, and its rows are not the index's."""
+    fake('''
+ix = index(64)
+v = np.ones((10_000, 64), np.float32)
+var("frees_refused").value = 1
+try:
+    ix.add_dev(v.ctypes.data, len(v))
+    said = None
+except T.TurbovecHipError as e:
+    said = e.status
+assert said == T.ERR_HIP and len(ix) == 64, (said, len(ix))
+ix.add_dev(v.ctypes.data, len(v))
+assert len(ix) == 10_064
+ix.close()
+assert used.value == 0
+''')
+
+
 def test_room_to_grow_is_not_taken_from_others(fake):
     """Rows that fit as they are: the library gives nothing up, neither pooled blocks nor a filtered search's copy, for the room beyond them."""
     fake(FILTERED + '''

@@ -211,7 +211,9 @@ hipError_t device_free(int device, void *p, size_t bytes) {
         }
         lock.unlock();
     }
-    return hipFree(p);
+    const hipError_t e = hipFree(p);
+    if (e != hipSuccess) (void)hipGetLastError();     // reported by this call, not by a later launch
+    return e;
 }
 
 int ensure_workspace(tv_index *ix, size_t bytes) {
@@ -2154,11 +2156,11 @@ int tv_index_add_dev(tv_index *ix, const float *d_vectors, size_t n_new) {
     if (rc != TV_OK) return rc;
     rc = encode_rows(ix, d_vectors, n_new, ix->n);      // (waits for the stream)
     if (rc == TV_OK) {
-        ix->n += n_new;
-        TV_HIP(outgrown.release());
-    } else {
-        (void)clear_slots(ix, ix->n + n_new);
+        const hipError_t e = outgrown.release();
+        if (e != hipSuccess) rc = fail_hip(e, "device_free(outgrown rows)");
     }
+    if (rc == TV_OK) ix->n += n_new;      // (an add that fails adds nothing)
+    else (void)clear_slots(ix, ix->n + n_new);
     return rc;
 }
 
