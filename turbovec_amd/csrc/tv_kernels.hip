@@ -930,9 +930,10 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 // The work is a few thousand keys in a few hundred short segments, and all of
 // it is latency; a thousand queries share the chip.  So: a thread per segment,
 // its head requested together with its count -- four threads where queries are few, and
-// then the whole of it; the need-th largest of groups of threads' best keys is a threshold
-// few keys reach (select_top; more than 128 wanted are counted out into 1024
-// bins); those are collected in LDS and ranked by comparing each with all -- no sort, a handful of
+// then the whole of it; up to sixteen leading keys take the need-th largest of groups of threads' best keys
+// as a threshold few keys reach (select_top), and more are counted out into 1024 bins, since a few hundred keys in as many segments
+// give 256 groups too little to choose from (50K x 3072, 33 queries, k = 100 107 us a search and 92; 20K x 1024 3-bit, 4 queries,
+// k = 100 66 and 64); those are collected in LDS and ranked by comparing each with all -- no sort, a handful of
 // barriers, 30 KiB of LDS, and workgroups no larger than the segments need.
 // Per launch under the profiler, with waves sorting chunks in 64 KiB of LDS (1024 threads per query), with
 // every threshold counted out, and now: one query, k = 10, 12, 11, 10.5 us; k = 100, 60 and 33, 21 and 18, 12; 1000 queries,
@@ -1088,12 +1089,13 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     };
     // (256 keys are ranked as they are)
     uint32_t least = 1u;
-    if (total > 256u && need <= kSelectTopMost) {
+    const bool counted = total > 256u && need > kSelectTopFew;
+    if (total > 256u && !counted) {
         uint32_t most = 0u;
         each([&](uint64_t k) { most = max(most, uint32_t(k >> 32)); });
         least = select_top<T>(most, need, top);
     }
-    const uint32_t n = keep_best<T>(each, least, need, kept, n_kept, sh, need > kSelectTopMost && total > 256u);
+    const uint32_t n = keep_best<T>(each, least, need, kept, n_kept, sh, counted);
     const size_t row = row_map ? size_t(row_map[qn]) : size_t(qn);   // a repeated pass writes to the rows of the queries it repeats
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];

@@ -70,8 +70,9 @@ __device__ __forceinline__ uint64_t select_threshold(const Each &each, uint32_t 
 // A score word that at least `need` of the threads' words reach, or 1 where the threads hold fewer: the need-th largest of the
 // best words of groups of threads, 64 of them or, from 17 on, 256.  For words dealt out at random few more than `need` reach it
 // (k = 10 of 64 groups: 10.8; 100 of 256: 126): one pass over them and one barrier (two), where counting them into bins takes a range and two
-// passes of four barriers.  `most`: the largest of the calling thread's words, 0 for none.  Met by all T threads.
-constexpr uint32_t kSelectTopMost = 128;       // (of 256 groups)
+// passes of four barriers.  Words that lie with few threads (rows laid out by score) leave it far too low or give none: keep_best counts then.
+// `most`: the largest of the calling thread's words, 0 for none.  Met by all T threads.
+constexpr uint32_t kSelectTopFew = 16;         // (of 64 groups)
 struct TopShared {
     __attribute__((aligned(16))) uint32_t groups[256 + 16];      // (four words of padding after every 64: lanes that read 64 apart spread over the banks)
     uint32_t w_top[16];
@@ -89,7 +90,7 @@ __device__ __forceinline__ uint32_t select_top(uint32_t most, uint32_t need, Top
         }
         return n;
     };
-    const bool few = need <= 16u;
+    const bool few = need <= kSelectTopFew;
     // (groups of T / 64 lanes, or of T / 256)
     if (few || T >= 512) most = max(most, other(most, IntC<0xB1>{}));       // quad_perm [1,0,3,2]
     if (few || T >= 1024) most = max(most, other(most, IntC<0x4E>{}));      // quad_perm [2,3,0,1]
@@ -139,11 +140,11 @@ __device__ __forceinline__ uint32_t rank_in(const uint64_t *kept, uint32_t n, ui
 }
 
 // The keys whose score words reach `least`, which at least `need` of all keys do or which no key is below, into kept, two zeros behind
-// them: how many.  Where they are too many for it, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
-// behind a barrier that comes between; met by all T threads.  count: there are too many for it.
+// them: how many.  Where they are more than `most`, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
+// behind a barrier that comes between; met by all T threads.  count: there are too many.
 template <uint32_t T, typename Each>
 __device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, uint32_t need, uint64_t *kept, uint32_t &n_kept, SelectShared &sh,
-                                              bool count = false) {
+                                              bool count = false, uint32_t most = 256u) {
     const uint32_t t = threadIdx.x;
     uint32_t n = kSelectKept + 1u;
     if (!count) {
@@ -155,7 +156,7 @@ __device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, 
         __syncthreads();
         n = n_kept;
     }
-    if (n > kSelectKept) {
+    if (n > most) {
         for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
         uint32_t hi_max = 0u, hi_min_inv = 0u, mx, mn_inv;
         each([&](uint64_t k) {
