@@ -458,7 +458,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     };
     if (t == 0) n_kept = 0u;
     __syncthreads();
-    n = keep_best<T>(each_row, 1u, k_eff, kept, n_kept, sh, false, kSelectKept);       // (all of them, but for many ties)
+    n = keep_best<T>(each_row, 1u, k_eff, kept, n_kept, sh);       // (all of them, but for many ties)
     for (uint32_t i = t; i < n; i += T) {
         const uint64_t k = kept[i];
         const uint32_t rank = rank_in(kept, n, k);

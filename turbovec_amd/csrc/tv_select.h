@@ -70,7 +70,9 @@ __device__ __forceinline__ uint64_t select_threshold(const Each &each, uint32_t 
 // A score word that at least `need` of the threads' words reach, or 1 where the threads hold fewer: the need-th largest of the
 // best words of groups of threads, 64 of them or, from 17 on, 256.  For words dealt out at random few more than `need` reach it
 // (k = 10 of 64 groups: 10.8; 100 of 256: 126): one pass over them and one barrier (two), where counting them into bins takes a range and two
-// passes of four barriers.  Words that lie with few threads (rows laid out by score) leave it far too low or give none: keep_best counts then.
+// passes of four barriers.  Words that lie with few threads (rows laid out by score) give a low one
+// or none; up to kSelectKept keys are ranked all the same, which is still the faster way (100K x 128 by rising score, 64 queries, k = 100
+// 56 us a search, with more than 256 counted out 60; 2M x 128 by falling score, k = 10 83 and 94).
 // `most`: the largest of the calling thread's words, 0 for none.  Met by all T threads.
 constexpr uint32_t kSelectTopFew = 16;         // (of 64 groups)
 struct TopShared {
@@ -140,11 +142,11 @@ __device__ __forceinline__ uint32_t rank_in(const uint64_t *kept, uint32_t n, ui
 }
 
 // The keys whose score words reach `least`, which at least `need` of all keys do or which no key is below, into kept, two zeros behind
-// them: how many.  Where they are more than `most`, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
-// behind a barrier that comes between; met by all T threads.  count: there are too many.
+// them: how many.  Where they are too many for it, a threshold is counted out.  n_kept is 0, and its writing has been seen or is seen
+// behind a barrier that comes between; met by all T threads.  count: there are too many for it.
 template <uint32_t T, typename Each>
 __device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, uint32_t need, uint64_t *kept, uint32_t &n_kept, SelectShared &sh,
-                                              bool count = false, uint32_t most = 256u) {
+                                              bool count = false) {
     const uint32_t t = threadIdx.x;
     uint32_t n = kSelectKept + 1u;
     if (!count) {
@@ -156,7 +158,7 @@ __device__ __forceinline__ uint32_t keep_best(const Each &each, uint32_t least, 
         __syncthreads();
         n = n_kept;
     }
-    if (n > most) {
+    if (n > kSelectKept) {
         for (uint32_t i = t; i < kSelectBins; i += T) sh.bins[i] = 0u;
         uint32_t hi_max = 0u, hi_min_inv = 0u, mx, mn_inv;
         each([&](uint64_t k) {
