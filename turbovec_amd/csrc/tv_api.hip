@@ -1228,6 +1228,8 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 // pass needs no correction downstream.
                 const uint32_t off = repeat ? repeat_offset(steps[lv]) : 0u;
                 const size_t level_blocks = (n_blocks - off + steps[lv] - 1) / steps[lv];
+                // a floor is the k_floor-th best of the level before; without one every slot, or every block's best, is there
+                const double expected = lv > 0 ? double(k_floor) * steps[lv - 1] / steps[lv] : double(level_blocks) * (best_first ? 1 : int(tv::kVecBlock));
                 // level 1 appends every slot it reads: two blocks per workgroup fill a segment exactly
                 const int lgrid = int(std::min<size_t>(size_t(grid), std::max<size_t>(1, (level_blocks + 1) / 2)));
                 // A sampling level behind the first filters by the floor of the level before; when
@@ -1325,7 +1327,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                                             (lv > 0 || repeat) ? 1 : 0, (last && !repeat) ? d_raise + (q0 - g0) : nullptr,
                                             repeat ? d_rows + row0 : nullptr, lv_flag, attempt == 0 ? next_flag : nullptr,
                                             run_if, ix->rows().slots, !timed_pass ? nullptr : last ? ix->d_stamps + tv::kStampsBefore : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
-                                            ix->stream));
+                                            expected, ix->stream));
                 }
             }
             if (repeat) TV_HIP(hipMemcpyAsync(h_over, d_over, pq_n * sizeof(uint32_t), hipMemcpyDeviceToHost, ix->stream));
