@@ -254,6 +254,8 @@ __device__ __forceinline__ float lut_entry(const float *q, const float *cen, int
 // the stored slot's number (three of four bits, two of three), its highest the choice of positions, so
 // that entry 8 p + 2 g + s (4 p + 2 g + s) is the group g's fourth 2 p + s.
 // (In a launch of their own they took 5 us of 37 queries' 219 and the gap in front of it.)
+// (An instance of its own writes them: the code for both made the other searches' tables wait, 1024 dimensions 3-bit, 4 queries 11.7 us a
+// launch without it and 13.1 with, 1536 14.5 and 16.6.)
 __device__ __forceinline__ uint32_t zip_lo(uint32_t a, uint32_t b) { return (a & 0xffffu) | (b << 16); }
 __device__ __forceinline__ uint32_t zip_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 template <int BITS>
@@ -269,7 +271,7 @@ __device__ __forceinline__ void mx_put(uint8_t *mx, int nch, int qi, int g, uint
     }
 }
 
-template <int BITS>
+template <int BITS, bool MX>
 __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
     extern __shared__ __align__(16) float prep_lds[];
     __shared__ float red[4];
@@ -282,7 +284,7 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
     const int t = threadIdx.x, G = a.G;
     if (qi >= a.nq) {
         for (int i = t; i < a.nch * 64; i += kPrepThreads) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
-        if (a.mx != nullptr)
+        if constexpr (MX)
             for (int g = t; g < a.nch * 32; g += kPrepThreads) mx_put<BITS>(a.mx, a.nch, int(qi), g, make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0));
         if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
         return;
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         uint4 *o = reinterpret_cast<uint4 *>(dst + size_t(g) * 32);
         o[0] = hi;
         o[1] = lo;
-        if (a.mx != nullptr) mx_put<BITS>(a.mx, a.nch, int(qi), g, hi, lo);
+        if constexpr (MX) mx_put<BITS>(a.mx, a.nch, int(qi), g, hi, lo);
     }
     if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
     if (t == 0 && a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
@@ -366,7 +368,11 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
         return hipGetLastError();
     };
     if (r.permute_dot) return launch(k_prep_p, r.cs, r.split);
-    return g.bits == 2 ? launch(k_prep_lut<2>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3>, r.centroids) : launch(k_prep_lut<4>, r.centroids);
+    auto tables = [&](auto mx) -> hipError_t {
+        constexpr bool M = decltype(mx)::value != 0;
+        return g.bits == 2 ? launch(k_prep_lut<2, M>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3, M>, r.centroids) : launch(k_prep_lut<4, M>, r.centroids);
+    };
+    return r.tables_mx != nullptr ? tables(IntC<1>{}) : tables(IntC<0>{});
 }
 
 }  // namespace tv
