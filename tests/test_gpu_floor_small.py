@@ -43,6 +43,27 @@ def test_small_samples(T, dim, bits, nq, k):
     ix.close()
 
 
+# 256 words are ranked as they are, more are thinned out first; and of few rows that may be returned
+@pytest.mark.parametrize("bits,nq", [(4, 64), (2, 12)])
+@pytest.mark.parametrize("words", [255, 256, 257])
+def test_words_ranked_as_they_are(T, words, bits, nq):
+    dim, k, n = 1536, 100, words * 4 * 32
+    ix = T.NativeIndex(dim, bits)
+    ix.add(unit_gaussian(n, dim, seed=words))
+    q = unit_gaussian(nq, dim, seed=7)
+    assert list(ix.sampling_plan(nq, k)[0]) == [4, 1]
+    for m in (None, np.arange(n) % 128 < 3):      # (blocks of the sample alone)
+        mask = None if m is None else T.pack_mask(m)[0]
+        out = []
+        for path in (0, MASKED, EXACT):
+            ix.set_path(path)
+            out.append(ix.search(q, k, mask_words=mask))
+        for s, i in out[:2]:
+            assert np.array_equal(i, out[2][1]) and bits_equal(s, out[2][0])
+    assert ix.overflow_redos() == 0
+    ix.close()
+
+
 # 820 blocks and five tiles of queries are the fewest pairs the sparse table scan takes: a sample of 205 blocks
 @pytest.mark.parametrize("dim,bits,nq,k,n", [(1536, 2, 150, 61, 820 * 32), (1536, 2, 150, 64, 820 * 32 - 31), (1536, 3, 129, 62, 1500 * 32 + 1)])
 def test_small_samples_of_the_sparse_scan(T, dim, bits, nq, k, n):

@@ -252,7 +252,9 @@ __global__ __launch_bounds__(kFloorThreads) void k_floor_of_best(const uint32_t 
         for (uint32_t e = 0; e < kFloorHeld; ++e)
             if (v[e] != 0u) f((uint64_t(v[e]) << 32) | ~(e * T + t));
     };
-    const uint32_t n_of = keep_best<T>(each, select_top<T>(most, k_floor, top), k_floor, kept, n_kept, sh);
+    // (256 words are ranked as they are)
+    if (n <= 256u) __syncthreads();
+    const uint32_t n_of = keep_best<T>(each, n <= 256u ? 1u : select_top<T>(most, k_floor, top), k_floor, kept, n_kept, sh);
     int *out = tau_out + (qi / uint32_t(tau_stride_q)) * kQTile + qi % uint32_t(tau_stride_q);
     if (n_of < k_floor) {      // (a mask that leaves the sample too few rows)
         if (t == 0) *out = kTauInit;
