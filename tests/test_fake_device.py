@@ -154,14 +154,14 @@ for dim, bits, rows, nq, k, unsampled in ((64, 4, 60_000, 2, 10, True), (8, 4, 1
 
 
 def test_segments_are_read_by_four_threads_where_they_are_long(fake):
-    """One query's first level, where it fills its segments, and its other levels with eight candidates a segment expected: not
-    with fewer, nor for two queries."""
+    """One query's first level, where it fills its segments, and its other levels from eight candidates a segment on average on: not
+    with fewer, nor for two queries, nor for blocks' best rows, dealt out evenly, up to sixteen a segment."""
     fake('''
 parted = var("parted")
 # the levels' strides, and the launches of them: 64 dimensions, 18 and 1 from best rows of blocks, 625, 73, 8 and 1 with more segments than
 # 256 behind the first; 1536 dimensions 2-bit, 256 segments at the most: 31, 5 (2480 candidates, and its conditional repeat) and 1 (2000)
 for dim, bits, rows, nq, k, launches in ((64, 4, 300_000, 1, 64, 0), (64, 4, 2_000_000, 1, 400, 1), (64, 4, 2_000_000, 2, 400, 0),
-                                         (1536, 2, 100_000, 1, 10, 0), (1536, 2, 100_000, 1, 100, 1), (1536, 2, 100_000, 1, 400, 3)):
+                                         (1536, 2, 100_000, 1, 10, 0), (1536, 2, 1_200_000, 1, 128, 0), (1536, 2, 100_000, 1, 100, 1), (1536, 2, 100_000, 1, 400, 3)):
     ix = T.NativeIndex(dim, bits)
     ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
     ix.set_path(16)

@@ -1228,8 +1228,6 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 // pass needs no correction downstream.
                 const uint32_t off = repeat ? repeat_offset(steps[lv]) : 0u;
                 const size_t level_blocks = (n_blocks - off + steps[lv] - 1) / steps[lv];
-                // a floor is the k_floor-th best of the level before; without one every slot, or every block's best, is there
-                const double expected = lv > 0 ? double(k_floor) * steps[lv - 1] / steps[lv] : double(level_blocks) * (best_first ? 1 : int(tv::kVecBlock));
                 // level 1 appends every slot it reads: two blocks per workgroup fill a segment exactly
                 const int lgrid = int(std::min<size_t>(size_t(grid), std::max<size_t>(1, (level_blocks + 1) / 2)));
                 // A sampling level behind the first filters by the floor of the level before; when
@@ -1320,6 +1318,9 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                         stamped = steps.size() > 1;
                         n_timed = stamped ? launch_no : std::min<size_t>(launch_no, size_t(kMaxTimedTiles));
                     }
+                    // a floor is the k_floor-th best of the level before, and of 256 segments that hold eight candidates on average one holds
+                    // twice that; without a floor every slot, or every block's best, is there, dealt out evenly
+                    const double longest = (lv > 0 ? 2.0 * double(k_floor) * steps[lv - 1] / steps[lv] : double(level_blocks) * (best_first ? 1 : int(tv::kVecBlock))) / n_seg;
                     // the first final pass may hand raised floors to a repeated one; the repeated pass
                     // sends what still does not fit to the exact path
                     TV_HIP(tv::launch_final(d_cand, d_cnt, uint32_t(n_seg), uint32_t(seg_stride), int(k_eff), int(k_floor),
@@ -1327,7 +1328,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                                             (lv > 0 || repeat) ? 1 : 0, (last && !repeat) ? d_raise + (q0 - g0) : nullptr,
                                             repeat ? d_rows + row0 : nullptr, lv_flag, attempt == 0 ? next_flag : nullptr,
                                             run_if, ix->rows().slots, !timed_pass ? nullptr : last ? ix->d_stamps + tv::kStampsBefore : lv + 2 == steps.size() ? ix->d_stamps : nullptr,
-                                            expected, ix->stream));
+                                            longest, ix->stream));
                 }
             }
             if (repeat) TV_HIP(hipMemcpyAsync(h_over, d_over, pq_n * sizeof(uint32_t), hipMemcpyDeviceToHost, ix->stream));

@@ -205,11 +205,11 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 // level_over (sampling levels): set to 1 when some query's candidates of this level did not all fit
 // (its floor then comes from a subset and may be far too low); clear_flag: a word this launch resets
 // to 0 (the flag of the level after); run_if: when given and *run_if == 0 the launch does nothing; slots: when
-// given, the slot of each row, for out_idx; expected: about how many candidates a query has.
+// given, the slot of each row, for out_idx; longest: about how many candidates a query's longest segment holds.
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double expected, hipStream_t s);
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s);
 // Packs the queries rows[0..n_redo) of a chunk and their raised floors for one more full scan.
 hipError_t launch_gather_redo(const float *d_q, const uint32_t *d_rows, const int *d_raised, int dim, int tile_q,
                               size_t n_redo, float *d_q_out, int *d_tau_out, hipStream_t s);

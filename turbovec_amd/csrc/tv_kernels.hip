@@ -941,12 +941,12 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 // ===========================================================================
 constexpr uint32_t kFinalStage = 2048;     // candidates copied to LDS when some segment is long
 constexpr uint32_t kFinalLong = 128;       // ... of which this many segments can be
-// One query's segments are read by four threads each from where eight candidates a segment are expected: one of 256 segments then holds more
-// than sixteen as often as not, and one that does sends all of them through LDS, or, where they are too many for it, has each thread read its
-// segment twice.  (A first level of rows fills its few segments.)  us a search with one thread a segment and with four: k = 400 700K x
-// 1536 2-bit 230 and 186, 50K x 3072 190 and 156, 10M x 1536 4-bit 1602 and 1567; k = 256 2M x 128 166 and 139; k = 100 10M x 1536 2-bit (1900
-// candidates, 256 segments) 675 and 665, but with fewer candidates a segment 2M x 1536 2-bit, k = 64 179 and 185, 384 dimensions, k = 100 160 and 168.
-constexpr double kFinalPartsFrom = 8.0;
+// One query's segments are read by four threads each where one of them is expected to hold more than the sixteen candidates that a thread
+// keeps: it would send all of them through LDS, or, where they are too many for it, have each thread read its segment twice.  us a
+// search with one thread a segment and with four: k = 400 700K x 1536 2-bit 230 and 186, 50K x 3072 190 and 156, 10M x 1536 4-bit 1602 and 1567; k = 256
+// 2M x 128 166 and 139; k = 100 10M x 1536 2-bit 675 and 665; but with shorter ones 2M x 1536 2-bit, k = 100 182 and 187, 384
+// dimensions, k = 100 160 and 168.
+constexpr double kFinalLongest = 16.0;
 static_assert(kSelectKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
 
 template <uint32_t T, uint32_t PARTS>
@@ -1415,13 +1415,13 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double expected, hipStream_t s) {
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s) {
     if (nq == 0 || k_eff == 0) return hipSuccess;
     auto launch = [&](auto kernel, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
                            out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp);
     };
-    if (n_seg <= 256 && nq == 1 && expected >= kFinalPartsFrom * n_seg) launch(k_final<1024, 4>, 1024);
+    if (n_seg <= 256 && nq == 1 && longest > kFinalLongest) launch(k_final<1024, 4>, 1024);
     else if (n_seg <= 256) launch(k_final<256, 1>, 256);
     else if (n_seg <= 512) launch(k_final<512, 1>, 512);
     else launch(k_final<1024, 1>, 1024);
