@@ -30,7 +30,7 @@ def test_unsampled_search_matches_oracle(T, oracle, dim, n, nq):
     q = unit_gaussian(nq, dim, seed=78)
     ix = to_native(T, oidx)
     rng = np.random.default_rng(5)
-    redos = 0       # (k = 100 on long rows is sampled, and may repeat queries)
+    redos = 0       # (k = 100 on long rows and several tiles of queries is sampled, and may repeat queries)
     for m in (None, rng.random(n) < 0.5, rng.random(n) < 0.01, (np.arange(n) >= n // 3) & (np.arange(n) < n // 3 + 40)):
         if m is not None and not m.any():
             m[0] = True
@@ -112,9 +112,59 @@ def test_few_rows(T, oracle, n, dim, nq):
             m[0] = True
         words = None if m is None else T.pack_mask(m)[0]
         for k in (1, 16, 17, 100):
+            # (rows of which the search has room for a score are never sampled; a query that came up short would be repeated)
+            kept, redos = min(k, n if m is None else int(m.sum())), ix.overflow_redos()
+            if n <= 4096 and (nq <= 256 or n <= 75 * kept * dim // 64):
+                assert unsampled(ix, nq, k, m), k
             s, i = ix.search(q, k, mask_words=words)
             os_, oi = oidx.search(q, k, mask_words=words)
             assert np.array_equal(i, oi) and bits_equal(s, os_), k
+            assert not unsampled(ix, nq, k, m) or ix.overflow_redos() == redos
+    ix.close()
+
+
+# Long rows and few queries: the chosen blocks are dealt out to several workgroups (24 to 48 chunks times k; of tables three times that),
+# all of whose rows tie -- every one's share is full, and up to 3200 rows are left to rank -- or all but a few of which score -infinity.
+@pytest.mark.parametrize("dim,bits,n,nq", [(1536, 4, 30_000, 1), (1536, 4, 10_001, 33), (3072, 4, 5_001, 2), (1536, 2, 30_000, 1), (1024, 3, 9_999, 7)])
+def test_shared_blocks_that_tie(T, oracle, dim, bits, n, nq):
+    oidx = OracleIndex(oracle, dim, bits, np.tile(unit_gaussian(1, dim, seed=3), (n, 1)))
+    q = unit_gaussian(nq, dim, seed=4)
+    ix = to_native(T, oidx)
+    third = (np.arange(n) % 96 < 32) & (np.arange(n) % 3 == 0)      # (of every third block)
+    ran = 0
+    for m in (None, third):
+        words = None if m is None else T.pack_mask(m)[0]
+        first = np.arange(n) if m is None else np.flatnonzero(m)
+        for k in (9, 30, 63, 100):
+            ran += unsampled(ix, nq, k, m)
+            redos = ix.overflow_redos()
+            s, i = ix.search(q, k, mask_words=words)
+            os_, oi = oidx.search(q, k, mask_words=words)
+            assert np.array_equal(i, np.tile(first[:k], (nq, 1)))
+            assert np.array_equal(i, oi) and bits_equal(s, os_), k
+            assert not unsampled(ix, nq, k, m) or ix.overflow_redos() == redos, k
+    assert ran >= (8 if nq == 1 else 2)
+    ix.close()
+
+
+@pytest.mark.parametrize("k", [9, 20, 60])
+def test_shared_blocks_of_minus_infinity(T, oracle, k):
+    dim, n = 1536, 4_200
+    oidx = OracleIndex(oracle, dim, 4, unit_gaussian(n, dim, seed=1))
+    q = unit_gaussian(1, dim, seed=2) * np.float32(1e6)
+    ix = to_native(T, oidx)
+    raw = ix.debug_scan(q)[1][0]
+    ix.close()
+    oidx.scales = (np.float32(3e38) * -np.sign(raw)).astype(np.float32)
+    finite = [40, 41, 1050, 1060, 2000, 3000, 3500, 3600, 3700, 4000, 4100, 4199]
+    oidx.scales[finite] = 1.0
+    ix = to_native(T, oidx)
+    assert unsampled(ix, 1, k)
+    s, i = ix.search(q, k)
+    os_, oi = oidx.search(q, k)
+    assert np.isneginf(os_[0, len(finite):]).all() and np.isfinite(os_[0, :len(finite)]).all()
+    assert np.array_equal(i, oi) and bits_equal(s, os_)
+    assert ix.overflow_redos() == (1 if k > len(finite) else 0)      # (-infinity does not count: such a query goes to the exact path)
     ix.close()
 
 

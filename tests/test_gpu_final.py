@@ -16,21 +16,21 @@ def near(v, at, q, gen):
     v[torch.from_numpy(at).to("cuda:0")] = q[which] + 0.2 * torch.randn(len(at), q.shape[1], device="cuda:0", generator=gen)
 
 
-@pytest.mark.parametrize("dim,bits,nq", [(64, 4, 1), (128, 2, 1), (64, 4, 9), (64, 3, 20), (128, 4, 70), (64, 4, 150)])
+@pytest.mark.parametrize("dim,bits,nq", [(64, 4, 1), (128, 2, 1), (1536, 2, 1), (1024, 3, 1), (64, 4, 9), (64, 3, 20), (128, 4, 70), (64, 4, 150)])
 @pytest.mark.parametrize("together", [1, 15, 16, 17, 33, 48, 64, 65, 400])
 def test_candidates_in_few_segments(dim, bits, nq, together):
     from turbovec_amd import _lib as T
-    n = 300_001
+    n = 300_001 if dim <= 128 else 100_001      # (long rows: 256 segments at the most, which four threads each read for one query of many results)
     gen = torch.Generator(device="cuda:0").manual_seed(together + dim)
     v, q = torch.randn(n, dim, device="cuda:0", generator=gen), torch.randn(nq, dim, device="cuda:0", generator=gen)
     slots = np.arange(n)
-    for at in (slots[slots // 32 % 256 == 3], slots[100_000:]):
+    for at in (slots[slots // 32 % 256 == 3], slots[n // 3:]):
         near(v, at[:together * nq], q, gen)
     torch.cuda.synchronize()
     ix = T.NativeIndex(dim, bits)
     ix.add_dev(v.data_ptr(), n)
     queries = q.cpu().numpy()
-    for k in (1, 16, 17, 100, 129, 400):
+    for k in (1, 16, 17, 100, 129, 256, 400):
         ix.set_path(1)
         s1, i1 = ix.search(queries, k)
         ix.set_path(SAMPLED)

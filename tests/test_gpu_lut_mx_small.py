@@ -36,6 +36,8 @@ def test_few_blocks(dim, bits, n, nq):
             s1, i1 = ix.search(q, k, mask_words=words)
             for path in (0, SAMPLED, NO_LUT16):
                 ix.set_path(path)
+                redos = ix.overflow_redos()
                 s, i = ix.search(q, k, mask_words=words)
                 assert np.array_equal(i, i1) and bits_equal(s, s1), (k, path)
+                assert ix.overflow_redos() == redos, (k, path)      # (a candidate that got lost would show here, and not in the repeated answer)
     ix.close()

@@ -27,9 +27,11 @@ def test_rounds_that_end_between_hand_overs(dim, n, nq):
         words = None if m is None else T.pack_mask(m)[0]
         ix.set_path(1)
         s1, i1 = ix.search(q, 10, mask_words=words)
+        redos = ix.overflow_redos()
         for path in (0, SAMPLED):      # (SAMPLED also has masks read during the scan, not their rows gathered)
             ix.set_path(path)
             for _ in range(2):
                 s, i = ix.search(q, 10, mask_words=words)
                 assert np.array_equal(i, i1) and bits_equal(s, s1), path
+                assert ix.overflow_redos() == redos, path      # (a candidate that got lost would show here, and not in the repeated answer)
     ix.close()
