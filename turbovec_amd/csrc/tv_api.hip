@@ -113,8 +113,8 @@ constexpr uint32_t kTooLargeBits = 0x5a0e1bcau;      // 1e16f
 // kPoolBytes, handed on only to requests they exceed by a quarter at most, and given back when the last
 // index of the device goes or an allocation fails -- any of an index's, so all of them come through
 // device_alloc.  What filtered searches keep of their allowed rows (tv_spare) goes the same way when the pool was not
-// enough.  An index built by adds allocates up to 2.6 times its size on
-// the way; fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
+// enough.  An index built by four equal adds allocates 1.75 times its size on the way (by half each time, 2.6 times);
+// fresh memory costs 28 us per MB once the driver has to clear what was freed before (400K x
 // 1536 rows in four adds that grew by half: 4 ms a build while cleared memory lasts, 22.8 ms after).
 constexpr size_t kPoolBytes = size_t(2) << 30, kPoolMinBytes = size_t(1) << 20;
 // What the indexes of a device may hold beyond growing by half (ensure_capacity): nothing takes it back but their end, so it is
@@ -476,7 +476,8 @@ int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCOR
 // are the faster ones (20K x 1536 2-bit, 33 queries, 1250 pairs: 153 us against 155; 65K rows, 4096
 // pairs: 165 against 131).  From four passes on (us a search, the passes and the matrix-unit scan):
 //  - 1400 pairs: 12K x 1536 2-bit, 100 queries 75 and 62, 15K x 3072, 96 queries 106 and 91; 1000 pairs are level or worse (15K x 3072, 49 queries 83 and 90).
-//  - 3-bit codes, half the products per byte: 2000 x 3072, 65 queries 123 and 115, 700 x 1536, 65 queries, k = 100 183 and 79.
+//  - 3-bit codes, half the products per byte: 2000 x 3072, 65 queries 123 and 115, 700 x 1536, 65 queries, k = 100 183 and 79; 49 queries
+//    over 1000 x 3072 120 and 113, 10K x 1536 80 and 72.
 //  - up to six chunks: 1000 x 768 2-bit, 129 queries 44.5 and 43.1, x 128 37.5 and 32.1; twelve 57.5 and 59.2.
 //  - many passes, one after the other where the search is sampled: 6000 x 3072 2-bit, 1000 queries 197 either way, 3000 1430 and 166, without
 //    sampling 222 and 160; 4000, 400 queries 131 and 112, but 129 queries 86 and 92.

@@ -14,9 +14,9 @@
 //     rounding could depend on it.
 //
 // k_encode_rows takes rows of up to 4096 dimensions, a wave (or part of one) per
-// row and a group of four waves' rows through each step together, so that the
-// sequential chains of all of them run side by side in the lanes of one or two
-// waves.  k_encode takes one workgroup per row: longer rows, the rotated rows of
+// row and a group of four waves' rows (eight, up to 512 dimensions) through each step
+// together, so that the sequential chains of all of them run side by side in the lanes of
+// one or more waves.  k_encode takes one workgroup per row: longer rows, the rotated rows of
 // a TQ+ fit, and tables whose signs are not +-1.
 #include <hip/hip_runtime.h>
 
@@ -371,20 +371,20 @@ __device__ __forceinline__ float enc_in_order(const float (&v)[NG][8], const Rec
     return inner > 0.1 ? nrm / float(inner) : 0.0f;
 }
 
-// NG = groups of eight elements per lane.  The float work of a row is 1160 vector instructions of its wave at 1536 dimensions,
+// NG = groups of eight elements per lane.  The float work of a row is 1220 vector instructions of its wave at 1536 dimensions,
 // half of them butterflies, and its norm is a chain of 192 dependent f32 additions: a workgroup
 // per row spent most of its time waiting for chains.  Here the norm chains of a workgroup's rows run in one wave, while
 // other workgroups of the CU are in their parallel part; the f64 sum needs no chain (enc_slack).  A row is held in
 // registers and all stages of a round are done there (the same additions in the same pairs), between lanes through the
 // data-parallel path; it is in LDS for the norm and for the two gathers alone.  Its codes leave as
-// 16-byte stores that consecutive rows complete to whole lines.  The vector ALU bounds it, busy for 81 % of the clocks.  100K
+// 16-byte stores that consecutive rows complete to whole lines.  The vector ALU bounds it, busy for 80 % of the clocks.  100K
 // rows of 1536 dimensions: 2.02 ms with a workgroup per row, 0.39 with the stages through LDS three at a time, 1.75K instructions a
 // row, 0.28 now (2.5 TB/s, every byte once); an add of 100K x 1024: 320 us before, 217 now, 30K x 4096: 1020 and 370, 77K x 1000 with a pair 420 and 205.
 // CAL: there is a TQ+ pair.  FULL: rows of NG * 512 dimensions, in blocks as large as they can be: every lane has NG groups and
 // all the stages are there, known at compile time.
 // Waves per workgroup: four, so that the workgroups of a CU are in different steps and the registers of a SIMD are dealt out
 // evenly (us an add with four and eight: 100K x 1536 315 and 319, 200K x 768 387 and 432, 100K x 1024 217 and 238; with six: 40K x 3072
-// 351 and 462; with two: 60K x 2048 264 and 270); eight where a wave has several rows (400K x 128 120 and 121).
+// 351 and 462; with two: 60K x 2048 264 and 270); eight where a lane has one group of elements, rows of up to 512 dimensions (400K x 128 120 and 121).
 constexpr int enc_waves(int ng) { return ng == 1 ? 8 : 4; }
 constexpr int enc_waves_per_simd(int ng, bool full) { return ng == 1 ? 6 : ng == 2 ? 5 : ng <= 4 ? 4 : ng <= 6 && !full ? 3 : 2; }    // what their registers leave room for
 template <int NG, bool CAL, bool FULL>

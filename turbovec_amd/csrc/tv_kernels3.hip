@@ -160,7 +160,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     const int nq = a.nq_tile;
     const int nt = (nq + kQTile - 1) / kQTile;
     const int nq_pad = nt * kQTile;
-    const int n_slices = SPT * nt;                          // per pass over the tiles; the host guarantees >= kAhead
+    const int n_slices = SPT * nt;                          // per pass over the tiles; may be fewer than the ring holds (129 queries of 2 chunks: 5 of 17)
     WideQuery *sq = reinterpret_cast<WideQuery *>(smem + kWideRing * kSlot);
     WideQueryTail *sqt = reinterpret_cast<WideQueryTail *>(sq + nq_pad);
     float *s_vs = reinterpret_cast<float *>(sqt + nq_pad);  // [waves][BLK][32]: row scales, NaN where not allowed
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
 
     // The weights are one periodic stream of slices (slice s = part s % SPT of tile s / SPT, kSlice
     // contiguous bytes; after the last tile the first follows again for the next round of blocks).
-    // Stream position g lives in ring slot g % kWideRing.  Half way through the MFMAs of slice g
+    // Stream position g lives in ring slot g % kWideRing, so one slice may lie in several slots.  Half way through the MFMAs of slice g
     // every wave waits for its own pieces of slice g + 1, meets the others at a barrier -- after
     // which slice g + 1 is whole and slice g - 1 is read by nobody -- and requests slice g + 4 into
     // the slot of g - 1.  The hand-over thus sits inside a run of MFMAs, where the SIMD's other wave

@@ -21,8 +21,8 @@ namespace tv {
 // instructions, 240 cycles) and feeds NT tiles' MFMAs from it (64 NT cycles), so four tiles balance the
 // two units.  The tiles are split over workgroups because a small index has few blocks: 100K rows are
 // 3125 of them, which fill 65 of the 256 workgroups of a kernel that takes all queries through one.
-// 100K x 128, 1000 queries: 35 us, the vector ALU busy in 60 % of the clocks and the matrix unit in 15 %.  Rows that
-// short have two chunks, so of the 530 vector instructions per block and four tiles the decode is 120, the rest epilogue.
+// 100K x 128, 1000 queries: 31 us, the vector ALU busy in 55 % of the clocks and the matrix unit in 15 %.  Rows that
+// short have two chunks, so of the 456 vector instructions per block and four tiles the decode is 120, the rest epilogue.
 // Weights in plane order, or (kBestSplit) in the order of k_scan_p4, whose operands then take four byte permutes a chunk.  kBestRows: plane order,
 // and every row's score instead of the block's best (ScanArgs::best_rows; an instance of its own, as two of the others would spill).
 // a.b_step: every so many blocks only (the sample a floor is taken from), recorded by their place in the sample.
@@ -273,9 +273,9 @@ hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int 
 }
 
 // ===========================================================================
-// One workgroup per query: the k_eff best blocks (select_top, and counting where many tie), their rows scored as the
-// scans score them, ranked.  All latency (k = 10, a thousand queries: 17 us over 100K x 128; at 3072 dimensions, twenty-four
-// times the row, 80 over 2000 rows and 133 over 200K, where it takes workgroups of 1024).  With the threshold from groups' best words
+// A workgroup per query, or several that share its work: the k_eff best blocks (select_top, and counting where many tie), their rows scored as the
+// scans score them, ranked.  All latency (k = 10, a thousand queries: 16 us over 100K x 128; at 3072 dimensions, twenty-four
+// times the row, 133 over 200K, where it takes workgroups of 1024).  With the threshold from groups' best words
 // instead of counted out, us a search: 100K x 128, 1 query 30.2 -> 27.9, 64 queries, k = 100 41.8 -> 40.4; and of the floors' kernel 500K x
 // 768, 45 queries, k = 64 109 -> 92, 1M x 1536, 64 queries 198 -> 194.
 // ===========================================================================
@@ -429,6 +429,8 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         __syncthreads();
         const uint32_t cap = (k_eff + shares - 1u) / shares * 32u, own = n_list;
         uint64_t *area = a.lists + size_t(qi) * pick_shared_words(k_eff);
+        // What is handed over goes through put and get alone: the order below rests on every word of it passing the caches on both
+        // sides, which the language's memory model does not promise.  A plain store or load among them may come late or find old bytes.
         auto put = [](uint64_t *to, uint64_t v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
         auto get = [](uint64_t *from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
         for (uint32_t i = t; i < own; i += T) put(&area[kMaxShares + share * cap + i], list[i]);
