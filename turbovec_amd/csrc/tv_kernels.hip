@@ -936,7 +936,7 @@ __global__ __launch_bounds__(256) void k_merge(const float *__restrict__ part_sc
 // k = 100 66 and 64); those are collected in LDS and ranked by comparing each with all -- no sort, a handful of
 // barriers, 30 KiB of LDS, and workgroups no larger than the segments need.
 // Per launch under the profiler, with waves sorting chunks in 64 KiB of LDS (1024 threads per query), with
-// every threshold counted out, and now: one query, k = 10, 12, 11, 10.5 us; k = 100, 60 and 33, 21 and 18, 12; 1000 queries,
+// every threshold counted out, and now: one query, k = 10, 12, 11, 10.5 us; k = 100, 60 and 33, 21 and 18, 14 and 13; 1000 queries,
 // k = 10, 61 to 75, 13 to 19, 11 to 17.
 // ===========================================================================
 constexpr uint32_t kFinalStage = 2048;     // candidates copied to LDS when some segment is long
