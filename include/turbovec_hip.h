@@ -261,7 +261,10 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * LDS (at most 8 queries per pass) instead of the larger ones; bit 4 samples
  * small indexes (bits 1 and 2 do too), and those of up to 16384 blocks by the
  * levels of rows that tests lay data out against; bit 6 has filtered searches
- * gather the allowed rows first whatever their number; without it any other bit, bit 5
+ * gather the allowed rows first whatever their number; bit 7 has u8-LUT batches
+ * without a filter take the int8 scan in front of the tables (more than sixteen
+ * queries over a large index otherwise) wherever it has an instance for the row
+ * length; without bit 6 any other bit, bit 5
  * of no other meaning too, has them read the mask as they scan. */
 int tv_debug_set_path(tv_index *ix, int force_full_lists);
 /* The sampling ladder a search for the k best of nq queries (its first chunk of up to 1024) runs

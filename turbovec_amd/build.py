@@ -8,7 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libturbovec_hip.so")
 
-SOURCES = ["tv_kernels.hip", "tv_kernels2.hip", "tv_kernels3.hip", "tv_kernels4.hip", "tv_kernels5.hip", "tv_kernels6.hip", "tv_filter.hip", "tv_prep.hip", "tv_encode.hip", "tv_api.hip", "host_tables.cpp", "tv_snapshot.cpp"]
+SOURCES = ["tv_kernels.hip", "tv_kernels2.hip", "tv_kernels3.hip", "tv_kernels4.hip", "tv_kernels5.hip", "tv_kernels6.hip", "tv_kernels7.hip", "tv_filter.hip", "tv_prep.hip", "tv_encode.hip", "tv_api.hip", "host_tables.cpp", "tv_snapshot.cpp"]
 
 # -ffp-contract=off: the parity contract is bit-exact float arithmetic, fused
 # only where the code says fmaf.  The packed-FP32 feature is switched off for
@@ -37,8 +37,8 @@ SGPR_LANES = re.compile(r"k_scan_lut_mxI")
 # These address their byte -> levels table by the byte's value alone: the table must sit at LDS
 # address 0, i.e. the kernel may have no static LDS allocation in front of its dynamic one
 # (k_scan_p4, k_scan_p4_multi, and the instances of k_scan_p4_wide whose last template argument but
-# one, the split decode, is true).
-NO_STATIC_LDS = re.compile(r"k_scan_p4(_multi)?I|k_scan_p4_wideI.*Lb1ELb[01]EEEv")
+# two, the split decode, is true).
+NO_STATIC_LDS = re.compile(r"k_scan_p4(_multi)?I|k_scan_p4_wideI.*Lb1ELb[01]ELi0EEEv")
 
 
 def check_resources(src, remarks):

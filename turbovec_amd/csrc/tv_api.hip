@@ -144,7 +144,7 @@ void free_blocks(const std::vector<std::pair<size_t, void *>> &blocks) {
 // A block some index of the device keeps for its filtered searches and is not using, or null.  pool.mu held.
 void *take_spare(DevicePool &pool) {
     for (tv_index *ix = pool.newest; ix != nullptr; ix = ix->older)
-        for (tv_spare *s : {&ix->gathered, &ix->slots})
+        for (tv_spare *s : {&ix->gathered, &ix->slots, &ix->staged})
             if (!s->in_use && s->p != nullptr) { s->bytes = 0; return std::exchange(s->p, nullptr); }
     return nullptr;
 }
@@ -230,11 +230,11 @@ int ensure_workspace(tv_index *ix, size_t bytes) {
 }
 
 // An allocation of the index that grows on demand: what it held is gone then.
-int ensure_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
+int ensure_block(tv_index *ix, void *&p, size_t &have, size_t bytes, bool insist = true) {
     if (bytes <= have) return TV_OK;
     if (p) { TV_HIP(device_free(ix->device, p, have)); p = nullptr; have = 0; }
-    bytes = round_up(bytes + bytes / 4, size_t(1) << 16);
-    TV_HIP(device_alloc(ix->device, bytes, &p, &have));
+    bytes = round_up(bytes + (insist ? bytes / 4 : 0), size_t(1) << 16);
+    TV_HIP(device_alloc(ix->device, bytes, &p, &have, insist));
     return TV_OK;
 }
 int ensure_io(tv_index *ix, size_t bytes) { return ensure_block(ix, ix->io, ix->io_bytes, bytes); }
@@ -509,6 +509,8 @@ struct Prepared {
     uint8_t *d_tables16 = nullptr;   // mode L: the same tables entry-major for the sixteen-query scan (or null)
     uint8_t *d_tables_mx = nullptr;  // mode L: the same tables as matrix operands for the sparse scan (or null)
     float *d_qscale = nullptr, *d_qbias = nullptr;
+    uint8_t *d_near = nullptr;       // mode L: int8 weights of the scan in front of the tables (or null) ...
+    float *d_near_unit = nullptr, *d_near_err = nullptr;
     size_t table_bytes_per_tile = 0;
 };
 
@@ -518,8 +520,9 @@ struct Prepared {
 // `keep_rotated`: the rotated rows are wanted in device memory too (the debug read-back).
 // `for_append`: u8-LUT tables are wanted in the order of the batch's append scan too.
 // `cleared`: a word per query to set to zero.
+// `near`: what the two-step table scan reads as well (where the matrix-unit scan serves).
 int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepared &out, bool split = true,
-                    bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr, uint64_t *cleared = nullptr) {
+                    bool keep_rotated = false, bool for_append = false, uint64_t *stamp = nullptr, uint64_t *cleared = nullptr, bool near = false) {
     const tv::Geometry &g = ix->geo;
     const size_t nq_pad = round_up(nq, tv::kQTile);
     const int mode = effective_mode(ix);
@@ -545,6 +548,12 @@ int prepare_queries(tv_index *ix, Arena &ar, const float *d_q, size_t nq, Prepar
     if (mx) r.tables_mx = out.d_tables_mx = ar.take<uint8_t>(tv::mx_table_bytes(g.nch, g.bits, nq));
     r.stamp = stamp;
     r.cleared = cleared;
+    if (near) {
+        r.near = out.d_near = ar.take<uint8_t>(nq_pad * size_t(tv::near_nch(g.nch, g.bits)) * 32 * size_t(8 / g.bits));
+        r.near_unit = out.d_near_unit = ar.take<float>(nq_pad);
+        r.near_err = out.d_near_err = ar.take<float>(nq_pad);
+        std::memcpy(r.lv, ix->levels, sizeof r.lv);
+    }
     TV_HIP(tv::launch_prep(r, g, nq, nq_pad, ix->stream));
     if (!mode_p && !mx && for_append && lut16_serves(ix) && nq >= size_t(lut16_min_queries(ix))) {
         out.d_tables16 = ar.take<uint8_t>(tv::lut16_table_bytes(g.nch, nq));
@@ -558,7 +567,10 @@ size_t prepare_bytes(const tv_index *ix, size_t nq) {
     const size_t nq_pad = round_up(nq, tv::kQTile);
     size_t b = 2 * round_up(nq * g.dim * 4, 256) + 3 * round_up(nq_pad * 4, 256);
     b += round_up(nq_pad * size_t(g.nch) * 1024, 256) + 4096;
-    if (lut_mx_serves(ix, nq)) b += round_up(tv::mx_table_bytes(g.nch, g.bits, nq), 256);
+    if (lut_mx_serves(ix, nq)) {
+        b += round_up(tv::mx_table_bytes(g.nch, g.bits, nq), 256);
+        if (g.bits != 4) b += round_up(nq_pad * size_t(tv::near_nch(g.nch, g.bits)) * 32 * size_t(8 / g.bits), 256) + 2 * round_up(nq_pad * 4, 256);     // (the two-step scan's)
+    }
     else if (lut16_serves(ix)) b += round_up(tv::lut16_table_bytes(g.nch, nq), 256);
     return b;
 }
@@ -620,6 +632,7 @@ struct SampledPlan {
     bool wide;
     bool lut_mx;        // u8-LUT queries of this chunk take the sparse matrix-unit scan, all in one launch
     bool lut16;         // u8-LUT tiles of this chunk take the sixteen-query scan
+    int grid_near;      // workgroups of the int8 scan in front of the tables
     bool lut_single;    // one u8-LUT query, served by the byte-table scan
     int nt_batched;     // query tiles one launch of the tile-group kernels serves (0: one tile per launch)
     int grid;
@@ -640,6 +653,7 @@ SampledPlan sampled_plan(const tv_index *ix, size_t cq) {
     p.grid = p.wide ? tv::wide_grid_blocks(ix->device)
            : mode_p ? tv::scan_grid_blocks(ix->device, mode_p, g.nch, 0, int(p.tile_q))
                     : tv::lut_append_grid(ix->device, g.nch);
+    p.grid_near = tv::wide_grid_blocks(ix->device);
     p.lut_single = !mode_p && cq == 1 && effective_mode(ix) != TV_SCORE_L_SCALAR && tv::lut_single_uses_byte_tables(g.nch, p.grid);
     p.seg_stride = p.lut_mx ? size_t(tv::mx_segments()) : size_t(p.grid);
     // (a query keeps one candidate segment per workgroup of the launches that serve it: every launch
@@ -912,6 +926,94 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
            : plan.lut16 ? sampling_steps(n_blocks, k_floor, size_t(plan.grid) * tv::lut16_blocks_per_workgroup(effective_mode(ix) == TV_SCORE_L_CLASSIC))
                         : sampling_steps(n_blocks, k_floor);
 }
+// ---- u8-LUT batches over large indexes: an int8 scan in front of the tables (tv_kernels3.hip: NEAR, tv_kernels7.hip) ----
+// The index is passed over in stages, each spread over all of it: the int8 scan, the rows it leaves in from the tables, the
+// k_floor-th best so far as the next stage's floor.  A stage is about as large as everything before it, whole rounds of the
+// scan's grid, and its rows and masks fit kNearBytes.  The first floor comes from a sample of blocks on the matrix-unit scan.
+constexpr size_t kNearBytes = size_t(1) << 30;
+constexpr size_t kNearSample = 512;      // blocks
+constexpr int kNearMaxStages = 32;
+// Two tiles of queries are level at best, three ahead (us a search without and so: 2.3M x 384 2-bit, 47 queries 240 and 299; 6.2M x 768, 59
+// 975 and 901; 4.1M x 384, 64 397 and 378; 7.1M x 456, 84 1431 and 826; 2.8M x 1360, 75 1530 and 943; 2.4M x 512 3-bit, 76 587
+// and 480, 752 dimensions, 52 450 and 532; 1M x 1128, 86 557 and 485; 10M x 1536, 1024 45 900 and 15 900).
+constexpr size_t kNearMinQueries = 65;
+// Rows that have to be looked up for nothing cost the rest: the share of an index within the margin of the last result (long rows,
+// many results, few rows).  3072 dimensions 2-bit: 2.2M rows, 127 queries, k = 71, 1.1 % 2810 and 3623; 1.2M, 389 queries, k = 24, 0.8 % 4831
+// and 4070; 3.8M, 437 queries, k = 21, 0.5 % 14 583 and 6371; 3-bit: 2M x 976, 373 queries, k = 91, 1 % 2859 and 2480; 3M x 760, 225 queries,
+// k = 92, 0.5 % 2347 and 1271.
+constexpr double kNearShare2 = 0.01, kNearShare3 = 0.008;
+struct NearPlan {
+    size_t stages = 0;                    // 0: the search does not go this way
+    uint32_t groups[kNearMaxStages] = {};
+    int rank[kNearMaxStages + 1] = {};    // the floor of the sample, and of each stage: the so-manieth best
+    bool guessed = false;                 // ... of which k rows may fall short
+    uint32_t total = 0, mul = 1, step = 1, splits = 1, sub = 1;
+    size_t rows_bytes = 0, bytes = 0;     // of the largest stage
+};
+// A floor need not be one that k rows are sure to reach, if the end shows that k did: the r-th best of a share f of the rows is above the
+// k-th best of all only where r or more of the k best are among them -- a Poisson variable of mean f * k.  The least r that is
+// so with a chance of one in a million: 8 for k = 100 and a 150th of the rows, in place of 100.
+int guessed_rank(double share, size_t k) {
+    const double mean = share * double(k);
+    double term = std::exp(-mean), below = term;
+    int r = 1;
+    for (; r < int(k) && 1.0 - below > 1e-6; ++r) below += term *= mean / r;
+    return r;
+}
+NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_t k_eff, size_t n_blocks, bool masked) {
+    NearPlan p;
+    const size_t k_floor = std::max<size_t>(k_eff, 16);
+    const int nch = ix->geo.nch, bits = ix->geo.bits;
+    if (!plan.lut_mx || masked || ix->ws_fixed || ix->no_wide || ix->no_batched || ix->row_ladder_left != 0 || ix->allowed.in_place || k_floor > size_t(tv::kMaxPickK)) return p;
+    if (tv::near_chunks(nch, bits) == 0 || tv::near_rescore_queries(nch) == 0 || ix->rows().n >= (size_t(1) << 31)) return p;
+    const size_t round = size_t(plan.grid_near) * size_t(tv::near_blocks_per_workgroup(nch, bits)) / tv::kNearBlocks;      // groups
+    const size_t total = (n_blocks + tv::kNearBlocks - 1) / tv::kNearBlocks, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
+    if (ix->no_direct && n_blocks <= 16384) return p;
+    if (!ix->force_near && (total < 2 * round || cq < kNearMinQueries)) return p;
+    // how far above the int8 product a table sum may lie, in standard deviations of the score, about (measured at 128 to 3072 dimensions),
+    // and the share of rows that close to the last result's score, were scores normal
+    const double margin = (bits == 2 ? 0.028 : 0.045) * std::sqrt(double(ix->geo.dim));
+    const double tail = std::log(double(ix->rows().n) / double(2 * k_eff));
+    double z = std::sqrt(2.0 * std::max(tail, 1.0));
+    for (int i = 0; i < 2; ++i) z = std::sqrt(2.0 * std::max(tail - 0.919 - std::log(z), 0.5));
+    if (!ix->force_near && 0.5 * std::erfc((z - margin) * 0.70710678) > (bits == 2 ? kNearShare2 : kNearShare3)) return p;
+    const size_t group_rows = size_t(tv::kNearBlocks) * ix->geo.block_bytes(), group_masks = tiles * tv::kQTile * tv::kNearBlocks * 4;
+    const size_t most = std::max(round, kNearBytes / (group_rows + group_masks) / round * round);
+    const size_t per_group = size_t(tv::near_rescore_queries(nch)), query_groups = (cq + per_group - 1) / per_group;
+    p.splits = uint32_t(std::clamp<size_t>(std::max((6 * k_floor + tv::kSegCap - 1) / tv::kSegCap, (512 + query_groups - 1) / query_groups), 4, 16));
+    p.guessed = ix->near_sure_left == 0;
+    const size_t sample = std::min<size_t>({p.guessed ? std::max<size_t>(kNearSample, size_t(tv::mx_round_blocks(ix->device, cq))) : std::max({4 * kNearSample, 8 * k_floor, round * tv::kNearBlocks / 2}),
+                                            size_t(tv::kMaxFloorBlocks), n_blocks / 4});
+    p.step = uint32_t((n_blocks + sample - 1) / sample);
+    auto rank_of = [&](double share) { return p.guessed ? guessed_rank(share, k_eff) : int(k_floor); };
+    p.rank[0] = rank_of(1.0 / double(p.step));
+    if (sample < 2 * size_t(p.rank[0])) return p;
+    size_t seen = sample / tv::kNearBlocks, largest = 0;
+    const double grow = p.guessed ? (margin < 0.9 ? 6.0 : margin < 1.15 ? 4.0 : 2.0) : 2.0;
+    for (size_t done = 0; done < total;) {
+        const size_t left = total - done;
+        size_t g = std::min(most, std::max<size_t>(1, size_t(double(seen) * (grow - 1.0) / double(round) + 0.5)) * round);
+        if (left <= most && left <= g + g / 2) g = left;
+        else if (left < 2 * g) g = std::min(g, (left / 2 + round - 1) / round * round);
+        g = std::min(g, left);
+        if (p.stages == size_t(kNearMaxStages) || (p.stages + 1) * p.splits > plan.seg_stride) { p.stages = 0; return p; }
+        p.groups[p.stages++] = uint32_t(g);
+        largest = std::max(largest, g);
+        done += g;
+        seen += g;
+        p.rank[p.stages] = rank_of(double(done) / double(total));
+    }
+    while (p.sub < 8 && p.stages * p.splits * p.sub * 2 <= plan.seg_stride) p.sub *= 2;      // (room for neighbours that lie together)
+    p.total = uint32_t(total);
+    // (consecutive multiples of the golden section of the total, modulo it, lie evenly over it; coprime, so that each group comes up once)
+    auto gcd = [](size_t a, size_t b) { while (b) { const size_t t = a % b; a = b; b = t; } return a; };
+    size_t mul = std::max<size_t>(1, size_t(double(total) * 0.6180339887498949));
+    while (gcd(mul, total) != 1) ++mul;
+    p.mul = uint32_t(mul % total);
+    p.rows_bytes = round_up(largest * group_rows, 256);
+    p.bytes = p.rows_bytes + largest * group_masks;
+    return p;
+}
 // Block offset of a repeated pass's level of stride `step`: it samples other blocks than the pass
 // that misjudged the floor, half a stride in (an even number of blocks, so that mask words stay
 // aligned).
@@ -986,7 +1088,7 @@ bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blo
 }
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
     const int nch = ix->geo.nch;
-    if (ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct) return false;
+    if (ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct || ix->force_near) return false;
     if (k_eff > size_t(tv::kMaxPickK) || n_blocks > tv::kMaxPickBlocks) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks, k_eff) > ix->ws_bytes) return false;
@@ -1103,6 +1205,8 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
 }
 
 int leave_in_place(tv_index *ix, size_t nq, size_t k_eff);
+bool have_block(tv_index *ix, tv_spare &s, size_t bytes, bool insist = true);
+void use_staged(tv_index *ix, bool in_use);
 constexpr size_t kLiveUnknown = ~size_t(0);
 
 // The seam: search::search over device-resident inputs and outputs.
@@ -1147,11 +1251,29 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     if (ix->row_ladder_left > 0) --ix->row_ladder_left;
     if (ix->floorless_kept_left > 0) --ix->floorless_kept_left;
+    if (ix->near_sure_left > 0) --ix->near_sure_left;
     uint32_t *h_over = ix->h_flags;   // pinned, one flag per query of a group, then the groups' level flags
     const bool track_levels = ix->track_levels != 0;
     // sized once for the whole call, repeated passes included: nothing is reallocated while work is in flight
     rc = ensure_workspace(ix, sampled_need_worst(ix, nq));
     if (rc != TV_OK) return rc;
+
+    // The two-step table scan's stages: memory that nothing is given up for; without it the first passes take the matrix-unit scan alone.
+    struct Staged {
+        tv_index *ix;
+        bool there = false;
+        ~Staged() { if (there) use_staged(ix, false); }
+    } staged{ix};
+    {
+        size_t bytes = 0;
+        for (const size_t cq : {std::min(nq, kChunkQueries), nq % kChunkQueries})      // (a chunk, and the last one)
+            if (cq != 0 && mode != TV_SCORE_P) bytes = std::max(bytes, near_plan(ix, sampled_plan(ix, cq), cq, k_eff, n_blocks, mask != nullptr).bytes);
+        if (bytes > 0) {
+            use_staged(ix, true);
+            staged.there = true;
+            if (!have_block(ix, ix->staged, bytes, false)) { use_staged(ix, false); staged.there = false; }
+        }
+    }
 
     // (which rows a scan reads, and through which mask, changes between a group's first passes and its repeated ones)
     const tv_rows asked = ix->allowed;
@@ -1194,6 +1316,8 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const int grid = plan.grid;
             const SamplingSteps steps = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, repeat, mask != nullptr);
             const bool best_first = steps.best_first;
+            NearPlan near = repeat || !staged.there ? NearPlan{} : near_plan(ix, plan, pq_n, k_eff, n_blocks, mask != nullptr);
+            if (near.bytes > ix->staged.bytes) near = NearPlan{};      // (a group before this one changed the plan)
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
                 g_last_error = "internal: workspace smaller than the pass it was sized for";
@@ -1211,7 +1335,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             Prepared pq;
             const int nt_batched = plan.nt_batched;
             const bool split = wide ? tv::wide_weights_split(g.nch) : (nt_batched == 0 || tv::batched_weights_split(g.nch));
-            int prc = prepare_queries(ix, ar, repeat ? d_redo_q : d_q, pq_n, pq, split, false, true);
+            int prc = prepare_queries(ix, ar, repeat ? d_redo_q : d_q, pq_n, pq, split, false, true, nullptr, nullptr, near.stages > 0);
             if (prc != TV_OK) return prc;
             uint64_t *d_cand = ar.take<uint64_t>(cq_pad * seg_stride * tv::kSegCap);
             uint32_t *d_cnt = ar.take<uint32_t>(cq_pad * seg_stride);
@@ -1223,6 +1347,76 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const bool batched = nt_batched > 0 && !wide;
             const size_t tiles_per_launch = wide || plan.lut_mx ? n_tiles : batched ? size_t(nt_batched) : 1;
             if (!repeat && q0 == 0) ix->last_queries_per_launch = int(std::min(pq_n, tile_q * tiles_per_launch));   // the call's first chunk
+            // The floors of a sample's best words (in the candidates' place, which nothing has been written to yet: 512 bytes a segment
+            // against four a block).
+            auto floors_of_best = [&](uint32_t step, int rank) -> int {
+                const size_t level_blocks = (n_blocks + step - 1) / step;
+                tv::ScanArgs a;
+                fill_scan_args(ix, a);
+                a.mask = mask;
+                a.tables = pq.d_tables;
+                a.qscale = pq.d_qscale;
+                a.qbias = pq.d_qbias;
+                a.nq_tile = int(pq_n);
+                a.b_step = step;
+                a.best_out = reinterpret_cast<uint32_t *>(d_cand);
+                a.best_stride = uint32_t(round_up(level_blocks, 64));
+                if (a.best_stride > seg_stride * tv::kSegCap * 2) { g_last_error = "internal: a sample larger than the candidates' place"; return TV_ERR_BAD_ARGUMENT; }
+                if (mode_p) TV_HIP(tv::launch_scan_p4_best(a, split, ix->device, ix->stream));
+                else if (const int lrc = best_scan_lut(ix, a, pq, pq_n)) return lrc;
+                TV_HIP(tv::launch_floor(a.best_out, a.best_stride, uint32_t(level_blocks), rank, int(pq_n), d_tau, int(tile_q),
+                                        timed_pass ? ix->d_stamps : nullptr, ix->stream));
+                return TV_OK;
+            };
+            if (near.stages > 0) {
+                if (const int frc = floors_of_best(near.step, near.rank[0])) return frc;
+                tv::ScanArgs a;
+                fill_scan_args(ix, a);
+                a.tables = pq.d_near;
+                a.qscale = pq.d_qscale;
+                a.qbias = pq.d_qbias;
+                a.near_unit = pq.d_near_unit;
+                a.near_err = pq.d_near_err;
+                a.nq_tile = int(pq_n);
+                a.gtau = d_tau;
+                a.near = tv::NearStage{0, 0, near.total, near.mul, reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(ix->staged.p) + near.rows_bytes), static_cast<uint8_t *>(ix->staged.p)};
+                tv::NearRescore r{};
+                r.tables = pq.d_tables;
+                r.scales = a.scales;
+                r.qscale = pq.d_qscale;
+                r.qbias = pq.d_qbias;
+                r.gtau = d_tau;
+                r.cand = d_cand;
+                r.cand_cnt = d_cnt;
+                r.seg_stride = uint32_t(seg_stride);
+                r.splits = near.splits;
+                r.sub = near.sub;
+                r.n = a.n;
+                r.nq = int(pq_n);
+                r.nch = g.nch;
+                for (size_t st = 0; st < near.stages; ++st, a.near.first += a.near.groups) {
+                    const bool last = st + 1 == near.stages;
+                    a.near.groups = near.groups[st];
+                    TV_HIP(tv::launch_scan_near(a, g.bits, plan.grid_near, ix->stream));
+                    r.stage = a.near;
+                    r.seg0 = uint32_t(st) * near.splits * near.sub;
+                    TV_HIP(tv::launch_near_rescore(r, ix->stream));
+                    const uint32_t n_seg = r.seg0 + near.splits * near.sub;
+                    const int rank = near.rank[st + 1];
+                    if (!last)
+                        TV_HIP(tv::launch_final(d_cand, d_cnt, n_seg, uint32_t(seg_stride), rank, rank, int(pq_n), d_os, d_oi, d_over, d_tau, int(tile_q), 2, nullptr, nullptr,
+                                                nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, ix->stream));
+                    else
+                        TV_HIP(tv::launch_final(d_cand, d_cnt, n_seg, uint32_t(seg_stride), int(k_eff), int(k_floor), int(pq_n), d_os, d_oi, d_over, nullptr, int(tile_q), 1,
+                                                d_raise + (q0 - g0), nullptr, nullptr, nullptr, nullptr, ix->rows().slots, timed_pass ? ix->d_stamps + tv::kStampsBefore : nullptr, 0.0,
+                                                ix->stream, near.guessed ? d_tau : nullptr));
+                }
+                if (timed_pass) {
+                    stamped = true;
+                    n_timed = 2 * near.stages;
+                }
+                return TV_OK;
+            }
             for (size_t lv = 0; lv < steps.size(); ++lv) {
                 const bool last = lv + 1 == steps.size();
                 // Sampling levels only yield floors, never slots, so the shifted origin of a repeated
@@ -1239,22 +1433,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 uint32_t *lv_flag = (!last && (lv > 0 || repeat)) ? d_level_flags + lv : nullptr;
                 uint32_t *next_flag = (lv + 2 < steps.size()) ? d_level_flags + lv + 1 : nullptr;
                 if (lv == 0 && steps.best_words) {
-                    tv::ScanArgs a;
-                    fill_scan_args(ix, a);
-                    a.mask = mask;
-                    a.tables = pq.d_tables;
-                    a.qscale = pq.d_qscale;
-                    a.qbias = pq.d_qbias;
-                    a.nq_tile = int(pq_n);
-                    a.b_step = steps[0];
-                    // (in the candidates' place, which nothing has been written to yet: 512 bytes a segment against four a block)
-                    a.best_out = reinterpret_cast<uint32_t *>(d_cand);
-                    a.best_stride = uint32_t(round_up(level_blocks, 64));
-                    if (a.best_stride > seg_stride * tv::kSegCap * 2) { g_last_error = "internal: a sample larger than the candidates' place"; return TV_ERR_BAD_ARGUMENT; }
-                    if (mode_p) TV_HIP(tv::launch_scan_p4_best(a, split, ix->device, ix->stream));
-                    else if (const int lrc = best_scan_lut(ix, a, pq, pq_n)) return lrc;
-                    TV_HIP(tv::launch_floor(a.best_out, a.best_stride, uint32_t(level_blocks), int(k_floor), int(pq_n), d_tau, int(tile_q),
-                                            timed_pass ? ix->d_stamps : nullptr, ix->stream));
+                    if (const int frc = floors_of_best(steps[0], int(k_floor))) return frc;
                     continue;
                 }
                 for (int attempt = 0; attempt < (lv_flag ? 2 : 1); ++attempt) {
@@ -1348,6 +1527,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
                 const SampledPlan plan = sampled_plan(ix, chunk_at[c + 1] - chunk_at[c]);
+                if (staged.there && near_plan(ix, plan, chunk_at[c + 1] - chunk_at[c], k_eff, n_blocks, mask != nullptr).stages > 0) continue;
                 const size_t n_levels = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).size();
                 for (size_t lv = 1; lv + 1 < n_levels; ++lv)
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
@@ -1374,7 +1554,13 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         }
         ix->overflow_redos += redo_rows.size() + exact_rows.size();
         if ((redo_rows.size() + exact_rows.size()) * 8 >= gq) {
-            if (level_strides(ix, sampled_plan(ix, chunk_at[1] - chunk_at[0]), n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).best_first) {
+            const SampledPlan plan = sampled_plan(ix, chunk_at[1] - chunk_at[0]);
+            const NearPlan near = staged.there ? near_plan(ix, plan, chunk_at[1] - chunk_at[0], k_eff, n_blocks, mask != nullptr) : NearPlan{};
+            if (near.stages > 0 && near.guessed) {
+                // (neighbours that lie together: a share of the rows has all of a query's best or none)
+                ix->near_sure_left = kRowLadderSearches;
+            } else if (near.stages > 0 ||
+                level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).best_first) {
                 // from here on, the repeated passes below included -- unless the row-level ladder has just failed too
                 if (ix->floorless_kept_left == 0) ix->row_ladder_left = kRowLadderSearches;
             } else if (ix->row_ladder_left > 0) {
@@ -1479,14 +1665,18 @@ bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowe
     }
     return true;
 }
+void use_staged(tv_index *ix, bool in_use) {
+    std::lock_guard<std::mutex> lock(g_pool[ix->device].mu);
+    ix->staged.in_use = in_use;
+}
 // Spares in use, or free to be taken again.
 void use_spares(tv_index *ix, bool in_use) {
     std::lock_guard<std::mutex> lock(g_pool[ix->device].mu);
     ix->slots.in_use = ix->gathered.in_use = in_use;
 }
 // A block, in use already, where there is memory for it.  (The search reads the mask as it scans otherwise, as it would have.)
-bool have_block(tv_index *ix, tv_spare &s, size_t bytes) {
-    if (ensure_block(ix, s.p, s.bytes, bytes) == TV_OK) return true;
+bool have_block(tv_index *ix, tv_spare &s, size_t bytes, bool insist) {
+    if (ensure_block(ix, s.p, s.bytes, bytes, insist) == TV_OK) return true;
     g_last_error.clear();
     return false;
 }
@@ -1958,12 +2148,14 @@ int tv_index_destroy(tv_index *ix) {
     void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
                     ix->d_tau_open};
     use_spares(ix, true);      // (from here on they are freed below)
+    use_staged(ix, true);
     (void)device_free(ix->device, ix->d_codes, ix->codes_bytes);
     (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
     (void)device_free(ix->device, ix->ws, ix->ws_bytes);
     (void)device_free(ix->device, ix->io, ix->io_bytes);
     (void)device_free(ix->device, ix->slots.p, ix->slots.bytes);
     (void)device_free(ix->device, ix->gathered.p, ix->gathered.bytes);
+    (void)device_free(ix->device, ix->staged.p, ix->staged.bytes);
     for (void *p : ptrs) if (p) (void)hipFree(p);
     {
         DevicePool &pool = g_pool[ix->device];
@@ -2823,6 +3015,7 @@ int tv_debug_set_path(tv_index *ix, int force_full_lists) {
     ix->no_lut16 = (force_full_lists & 8) != 0;
     ix->no_direct = (force_full_lists & 16) != 0;
     ix->force_gather = (force_full_lists & 64) != 0;
+    ix->force_near = (force_full_lists & 128) != 0;
     ix->no_gather = !ix->force_gather && force_full_lists != 0;     // (a call that names its kernels means them with the mask)
     return TV_OK;
 }
@@ -2838,6 +3031,7 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (direct_serves(ix, nq, k_eff, n_blocks)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
+    if (near_plan(ix, plan, chunk_len(ix, nq), k_eff, n_blocks, false).stages > 0) return TV_OK;
     const SamplingSteps steps = level_strides(ix, plan, n_blocks, n_blocks, std::max<size_t>(k_eff, 16), false, false);
     *count = steps.size();
     for (size_t i = 0; i < steps.size() && i < cap; ++i) {
@@ -2860,7 +3054,7 @@ int tv_debug_workspace_bytes(const tv_index *cix, size_t *workspace, size_t *sta
     if (!ix) return TV_ERR_BAD_ARGUMENT;
     std::lock_guard<std::mutex> lock(ix->mu);
     std::lock_guard<std::mutex> kept(g_pool[ix->device].mu);
-    if (workspace) *workspace = ix->ws_bytes + ix->slots.bytes + ix->gathered.bytes;
+    if (workspace) *workspace = ix->ws_bytes + ix->slots.bytes + ix->gathered.bytes + ix->staged.bytes;
     if (staging) *staging = ix->io_bytes;
     return TV_OK;
 }

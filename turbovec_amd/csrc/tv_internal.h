@@ -42,6 +42,18 @@ struct Geometry {
     size_t block_bytes() const { return size_t(nch) * 1024; }
 };
 
+// A part of an index that k_scan_p4_wide (its instances for 2- and 3-bit codes) and k_near_rescore pass over together: `groups` groups of
+// eight blocks, from number `first` of a fixed order of all `total` groups, in which any run of consecutive ones lies spread over the whole index: number x
+// is group x * mul % total, and group g the blocks g, g + total, ... (the last of them may lie beyond the index): neighbouring rows, often neighbours
+// of one query, are of groups that lie apart in that order.
+constexpr int kNearBlocks = 8;
+struct NearStage {
+    uint32_t first, groups, total, mul;
+    uint16_t *masks;           // [tile][group][query of the tile][block][lane half]: bit 15 - r for row 8 (r / 4) + 4 half + r % 4
+    uint8_t *rows;             // the stage's rows one after the other, nch * 32 bytes each
+};
+__host__ __device__ constexpr uint32_t near_group(const NearStage &n, uint32_t x) { return uint32_t(uint64_t(x) * n.mul % n.total); }
+__host__ __device__ constexpr uint32_t near_block(const NearStage &n, uint32_t group, uint32_t w) { return group + w * n.total; }
 struct ScanArgs {
     const uint8_t *codes;
     const float *scales;       // padded to a multiple of 32 entries
@@ -74,6 +86,10 @@ struct ScanArgs {
     uint32_t best_stride;
     int best_rows;             // (of launch_scan_p4_best) ... every row's score as a float instead, NaN for rows that may not be returned: [nq_tile][best_stride], by row
     const uint32_t *rows;      // all-queries-per-pass kernel: when given, the slot of each of the n rows to scan, in order, 32 neighbours of them within 4 GiB
+    // Instances of the all-queries-per-pass kernel for 2- and 3-bit codes (NearStage): tables and lv are int8 weights and levels, and
+    // nothing is scored; per (tile, block of the stage, query) a bit for each row whose table sum may reach the floor.
+    const float *near_unit, *near_err;
+    NearStage near;
     const uint32_t *run_if;    // append mode: when given and *run_if == 0 the launch does nothing (a level's conditional repeat)
 };
 
@@ -118,6 +134,9 @@ struct PrepRequest {
     uint8_t *tables;
     uint8_t *tables_mx;             // or null: u8 tables also as the operands of k_scan_lut_mx
     float *qscale, *qbias;
+    uint8_t *near;                  // or null: u8 tables also as int8 weights (with tables_mx; cs and lv are read) ...
+    float *near_unit, *near_err;    // ... and per query what they leave out (tv_prep.hip: near_fit)
+    uint32_t lv[2];                 // the int8 levels of up to eight codes
     float *rot_out;                 // or null
     uint64_t *stamp;                // or null: kStampsBefore words
     uint64_t *cleared;              // or null: a word per query to set to zero
@@ -192,6 +211,25 @@ int wide_max_queries(int nch);
 bool wide_weights_split(int nch);
 bool wide_reads_rows(int nch, int nq);
 
+// The same over 2- and 3-bit codes, in front of their u8 tables (tv_kernels7.hip): an int8 scan that tells the rows whose table sum cannot reach
+// the floor, and the rest scored from the tables.
+int near_chunks(int nch, int bits);                    // chunks of 64 dimensions of the scan's instance; 0 = there is none
+int near_nch(int nch, int bits);                       // chunks of 32 byte-groups there: a row's, or more, with weights of zero
+int near_blocks_per_workgroup(int nch, int bits);
+hipError_t launch_scan_near(const ScanArgs &a, int bits, int grid, hipStream_t s);
+struct NearRescore {
+    NearStage stage;
+    const uint8_t *tables;     // launch_prep's u8 tables
+    const float *scales, *qscale, *qbias;
+    const int *gtau;
+    uint64_t *cand;            // as in ScanArgs; this stage's segments are numbers seg0 .. seg0 + splits * sub - 1, `sub` (a power of two) to a workgroup
+    uint32_t *cand_cnt;
+    uint32_t seg_stride, seg0, splits, sub, n;
+    int nq, nch;
+};
+int near_rescore_queries(int nch);                     // of one workgroup; 0: the tables do not fit
+hipError_t launch_near_rescore(const NearRescore &a, hipStream_t s);
+
 hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, const int *part_cnt, int total_threads,
                         int qmod, int k, int k_eff, int nq_tile, float *out_scores, int64_t *out_idx,
                         int *out_tau, hipStream_t s);
@@ -205,11 +243,13 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 // level_over (sampling levels): set to 1 when some query's candidates of this level did not all fit
 // (its floor then comes from a subset and may be far too low); clear_flag: a word this launch resets
 // to 0 (the flag of the level after); run_if: when given and *run_if == 0 the launch does nothing; slots: when
-// given, the slot of each row, for out_idx; longest: about how many candidates a query's longest segment holds.
+// given, the slot of each row, for out_idx; passed: (a final pass) floors laid out as tau_out that may be above the result's last row -- such a
+// query is flagged 1, and that row is its raised floor (open with fewer rows than k_eff); keep_floor == 2: no floor is lowered; longest: about how many candidates a query's longest segment holds.
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s);
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s,
+                        const int *passed = nullptr);
 // Packs the queries rows[0..n_redo) of a chunk and their raised floors for one more full scan.
 hipError_t launch_gather_redo(const float *d_q, const uint32_t *d_rows, const int *d_raised, int dim, int tile_q,
                               size_t n_redo, float *d_q_out, int *d_tau_out, hipStream_t s);
@@ -313,6 +353,7 @@ struct tv_index {
     size_t io_bytes = 0;
     size_t ws_bytes = 0;
     bool ws_fixed = false;         // ws is a lent buffer of fixed size (tv_search_dev_noalloc): never reallocated
+    tv_spare staged;               // the two-step table scan's stages (tv_api.hip: NearPlan)
     tv_spare slots, gathered;      // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
     tv_index *older = nullptr, *newer = nullptr;   // the device's indexes, linked (guarded as their pool of blocks is)
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
@@ -331,6 +372,7 @@ struct tv_index {
     bool no_lut_mx = false;        // for the length of a call: the scratch array holds only the sixteen-query passes' working set
     int no_wide = 0;               // test hook: large batches go through the tile-group kernels, not the wide one
     int no_direct = 0;             // test hook: small indexes are sampled, those of up to 16384 blocks by levels of rows where there are such
+    int force_near = 0;            // test hook: u8-LUT batches take the two-step scan wherever it has an instance for the row length
     int no_gather = 0;             // test hook: filtered searches read the mask as they scan ...
     int force_gather = 0;          // ... or gather their allowed rows whatever their number
     size_t gathered_searches = 0, in_place_searches = 0;   // searches that ran on the allowed rows alone, and those of them that read all of their queries' rows in place
@@ -343,6 +385,7 @@ struct tv_index {
     // back at once and stays for as many searches: its failure costs less.
     int row_ladder_left = 0;
     int floorless_kept_left = 0;
+    int near_sure_left = 0;        // the two-step table scan guessed floors too high for many queries: so many searches take floors that are sure
     int track_levels = 0;          // test hook: read the per-level flags back with the overflow flags and count them
     size_t level_repeats = 0;      // sampling levels that ran a second time because their candidates did not fit
 };

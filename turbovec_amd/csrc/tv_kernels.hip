@@ -957,7 +957,7 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                uint32_t *__restrict__ overflow, int *__restrict__ tau_out,
                                                int tau_stride_q, int keep_floor, int *__restrict__ raise_out,
                                                const uint32_t *__restrict__ row_map, uint32_t *level_over,
-                                               uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp) {
+                                               uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, const int *passed) {
     constexpr uint32_t W = T / 64;
     __shared__ __align__(16) uint64_t kept[kSelectKept + 2];
     __shared__ uint64_t stage[kFinalStage];
@@ -1031,7 +1031,10 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     if (!sampling) {
         const bool redo = too_many || any_full || total < uint32_t(k_eff);
         raising = redo && raise_out != nullptr && total >= uint32_t(k_eff);
-        if (t == 0) overflow[qn] = redo ? (raising ? 1u : 2u) : 0u;
+        // (floors that were guessed: a query that too few rows reached is repeated from an open one)
+        const bool missed = passed != nullptr && !too_many && !any_full && total < uint32_t(k_eff);
+        if (t == 0 && missed && raise_out != nullptr) raise_out[qn] = kTauInit;
+        if (t == 0 && (redo || passed == nullptr)) overflow[qn] = redo ? (raising || (missed && raise_out != nullptr) ? 1u : 2u) : 0u;
         if (redo && !raising) return;
     }
     // (the last query's workgroup is among the last to end)
@@ -1110,8 +1113,19 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
         sort_unkey(k, s, idx);
         if (sampling || raising) {
             // the floor: the k_floor-th best sampled score (k_floor >= k_eff steadies the estimate)
-            if (rank == need - 1u) *(sampling ? tau_slot : raise_out + qn) = order_key(s == 0.0f ? -0.0f : s);
+            if (rank == need - 1u) {
+                const int floor = order_key(s == 0.0f ? -0.0f : s);
+                *(sampling ? tau_slot : raise_out + qn) = sampling && keep_floor == 2 ? max(floor, *tau_slot) : floor;
+            }
         } else {
+            // Of floors that were guessed the highest is the last: what the scans left out lies below it, and the result is whole if its
+            // last row does not.  Otherwise that row is a floor k rows do reach.
+            if (passed != nullptr && rank == need - 1u) {
+                const int last = order_key(s == 0.0f ? -0.0f : s);
+                const bool missed = last < passed[(qn / tau_stride_q) * kQTile + qn % tau_stride_q];
+                overflow[qn] = missed ? (raise_out != nullptr ? 1u : 2u) : 0u;
+                if (missed && raise_out != nullptr) raise_out[qn] = last;
+            }
             out_scores[row * k_eff + rank] = s;
             out_idx[row * k_eff + rank] = int64_t(slots != nullptr ? slots[idx] : idx);
         }
@@ -1415,11 +1429,11 @@ hipError_t launch_merge(const float *part_scores, const uint32_t *part_idx, cons
 hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t n_seg, uint32_t seg_stride,
                         int k_eff, int k_floor, int nq, float *out_scores, int64_t *out_idx, uint32_t *overflow,
                         int *tau_out, int tau_stride_q, int keep_floor, int *raise_out, const uint32_t *row_map,
-                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s) {
+                        uint32_t *level_over, uint32_t *clear_flag, const uint32_t *run_if, const uint32_t *slots, uint64_t *stamp, double longest, hipStream_t s, const int *passed) {
     if (nq == 0 || k_eff == 0) return hipSuccess;
     auto launch = [&](auto kernel, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
-                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp);
+                           out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp, passed);
     };
     if (n_seg <= 256 && nq == 1 && longest > kFinalLongest) launch(k_final<1024, 4>, 1024);
     else if (n_seg <= 256) launch(k_final<256, 1>, 256);

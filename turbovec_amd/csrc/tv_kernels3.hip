@@ -127,8 +127,23 @@ constexpr int kWideTableBytes = 1024;    // the byte table of the split decode (
 // k_scan_p4 (code bytes 0-7 of a lane on the vector ALU, bytes 8-15 looked up whole); the weights
 // then come in that kernel's split order.  The decode is the block phase -- both waves of a SIMD
 // at it together, the matrix unit idle -- and the LDS has nothing else to do then.
-template <int NCH, int NB, int WAVES, int SPT, int BLK, int HO, int KS, bool SPLIT = false, bool ROWS = false>
+//
+// NEAR: 2- or 3-bit codes, whose score is a sum over u8 tables (tv_kernels5.hip); this scan goes before it.  A
+// row's table sum is at most unit * P + err with P the int8 product of the row's levels and the weights of k_prep_lut's near_fit,
+// so a row whose P stays below a bound of its query's floor and its own scale need not be looked up (10M x 1536 2-bit, 1024 queries, k =
+// 100: 45.9 ms a search on the one-hot products alone, 15.9 so, 12.9 of them here -- the matrix unit's rate for
+// the same products on 4-bit codes).  NCH counts chunks of 64
+// dimensions (a 2-bit row's 32 byte-groups are two of them).  Nothing is scored: a bit per row and query says whether it
+// is still in, and the rows are written out one after the other for k_near_rescore, which looks those up.  Each query
+// tile of a block costs the matrix unit a quarter of what k_scan_lut_mx's one-hot products do.
+// The bits of a tile: sums start at the bits of the float 1.5 * 2^23, so that they read as floats that much higher without a conversion (beyond
+// +-2^22 they read as higher than they are, which lets rows in, never out); a fused multiply-add by the row's
+// reciprocal scale gives the bound, and the sign of the difference is shifted into the lane's word.
+template <int NCH, int NB, int WAVES, int SPT, int BLK, int HO, int KS, bool SPLIT = false, bool ROWS = false, int NEAR = 0>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide(ScanArgs a) {
+    static_assert(NEAR == 0 || (!SPLIT && !ROWS && KS == 1 && (NEAR == 3 || (NEAR == 2 && NCH % 2 == 0))), "2- and 3-bit codes: whole rows, decoded on the vector ALU");
+    constexpr int kFields = NEAR == 2 ? 4 : 2;              // codes of a byte
+    constexpr int kRaw = NCH * 2 / kFields;                 // chunks of 32 byte-groups
     static_assert(NCH % SPT == 0, "a slice is a whole number of chunks");
     static_assert(!SPLIT || (WAVES == 8 && BLK == 1 && KS == 1), "the split decode is built for the one-block eight-wave forms");
     static_assert(KS == 1 || (KS == 2 && WAVES == 4 && BLK == 1 && HO == 1), "row halves go to the wave pairs of the four-wave form");
@@ -178,6 +193,18 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         const bool act = q < nq;
         const float qs = act ? a.qscale[q] : 0.0f, qb = act ? a.qbias[q] : 0.0f;
         const float tau = act ? order_unkey(a.gtau[q]) : __int_as_float(0x7fc00000);
+        if constexpr (NEAR != 0) {
+            // A row with scale v passes if (sum * qs + qb) * v >= tau, and then sum >= tau / (v * qs) - qb / qs; sum <= unit * P + err.
+            // Slack as below, in table units, and two of the product's.
+            const float unit = act ? a.near_unit[q] : 0.0f, err = act ? a.near_err[q] : 0.0f, rb = qb / qs;
+            const float low = fabsf(tau) < 1e-30f ? -1e-30f : tau, t = (low / qs) / unit;
+            const float tb = (((rb + err) + 1e-5f * fabsf(rb)) + 2.0f) / unit;
+            const bool usable = fabsf(low) <= 1e30f && qs >= 1e-30f && qs <= 1e30f && fabsf(qb) <= 1e30f && unit >= 1e-20f && unit <= 1e20f &&
+                                fabsf(t) <= 1e20f && fabsf(tb) <= 1e20f;
+            sq[q].ta = !act ? 0.0f : usable ? t - 1e-5f * fabsf(t) : 0.0f;
+            sq[q].tb = !act ? 3e38f : usable ? 12582912.0f - (tb + 1e-6f * fabsf(tb) + 2.0f) : -3e38f;     // added to ta / scale
+            continue;
+        }
         sqt[q].qs = qs;
         sqt[q].qb = qb;
         sqt[q].tau = tau;
@@ -206,7 +233,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
 
     const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
     const uint32_t step = a.b_step;
-    const uint32_t nj = (a.n_blocks + step - 1) / step;
+    const uint32_t nj = NEAR != 0 ? a.near.groups * uint32_t(kNearBlocks) : (a.n_blocks + step - 1) / step;
 
     // next live block of this workgroup (blocks m * gridDim.x + blockIdx.x), claimed wave by wave;
     // the two waves of a pair must arrive at the same block without talking: pair p takes the
@@ -222,6 +249,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                 if (lane == 0) m = atomicAdd(snext, 1u);
                 m = uint32_t(__builtin_amdgcn_readfirstlane(int(m)));
             }
+            if constexpr (NEAR != 0)      // (a group's blocks in one workgroup: its words of the masks are neighbours)
+                return (m / kNearBlocks * gridDim.x + blockIdx.x) * uint32_t(kNearBlocks) + m % kNearBlocks;
             const uint32_t j = m * gridDim.x + blockIdx.x;
             if (j >= nj || a.mask == nullptr) return j;
             const uint32_t b = j * step;
@@ -347,7 +376,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
 
     int inv_vmax[BLK];       // bits of 1 / (largest allowed row scale of the block); +inf when that is 0
     bool odd_block[BLK];
-    uint32_t blk[BLK];       // the wave's blocks of this round
+    uint32_t odd_rows[BLK];  // NEAR: rows that no bound holds for
+    uint32_t blk[BLK];       // the wave's blocks of this round (NEAR: their numbers in the stage)
     uint32_t round_no = 0;
     for (;;) {
         // ---- block phase: claim, load, decode into registers ----
@@ -363,12 +393,58 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         if constexpr (KS == 2) __syncthreads();
         // (read as LDS, not through a generic pointer: a flat load is counted by both memory
         // counters and the compiler would wait for every weight request in flight before it)
-        const bool futile = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_word(s_over_addr)))) >= uint32_t(nq);
+        const bool futile = NEAR == 0 && uint32_t(__builtin_amdgcn_readfirstlane(int(lds_word(s_over_addr)))) >= uint32_t(nq);
         static_for<BLK>([&](auto kk) {
             constexpr int k = decltype(kk)::value;
             const uint32_t j = futile ? nj : claim();
             const bool has_k = j < nj;
             has = has || has_k;
+            if constexpr (NEAR != 0) {
+                blk[k] = has_k ? j : nj;
+                float inv = __int_as_float(0x7fc00000);
+                bool odd = false;
+                if (has_k) {
+                    // (a block beyond the index: another one's codes, no row in)
+                    const uint32_t b = near_block(a.near, near_group(a.near, a.near.first + j / kNearBlocks), j % kNearBlocks);
+                    const uint8_t *p = a.codes + size_t(b < a.n_blocks ? b : 0u) * uint32_t(a.nch * 1024);
+                    uint8_t *out = a.near.rows + size_t(j) * uint32_t(a.nch * 1024);
+                    const uint32_t out_at = uint32_t(qn) * uint32_t(a.nch * 32) + uint32_t(h) * 16;
+                    const bool padded = a.nch < kRaw;
+                    u32x4 raw[kRaw];
+                    constexpr int kFirst = kHandMfma && NCH > kVecChunks ? kVecChunks * kRaw / NCH : 0;
+                    static_for<kRaw>([&](auto ii) {
+                        constexpr int c = (decltype(ii)::value + kFirst) % kRaw;
+                        // (the last chunk may lie beyond the row: another one, which meets weights of zero)
+                        load16_async_s(raw[c], p + (c + 1 == kRaw && kRaw > 1 && padded ? size_t(c - 1) : size_t(c)) * 1024, lane16);
+                    });
+                    static_for<kRaw>([&](auto ii) {
+                        constexpr int c = (decltype(ii)::value + kFirst) % kRaw;
+                        // (the rows written so far are younger requests too: the count holds for more than this one, never for less)
+                        wait_vm<kRaw - 1 - decltype(ii)::value>(raw[c]);
+                        if (c + 1 < kRaw || !padded) *reinterpret_cast<u32x4 *>(out + c * 32 + out_at) = raw[c];
+                        static_for<kFields>([&](auto ff) {
+                            constexpr int f = decltype(ff)::value, o = c * kFields + f, shift = 8 - 8 / kFields * (f + 1);
+                            v4i &to = (o & 1) == 0 ? alo[k][o / 2] : ahi[k][o / 2];
+#pragma unroll
+                            for (int d = 0; d < 4; ++d) {
+                                const uint32_t x = raw[c][d] >> shift;
+                                to[d] = NEAR == 2 ? int(__builtin_amdgcn_perm(0u, t0, x & 0x03030303u)) : int(__builtin_amdgcn_perm(t1, t0, x & 0x07070707u));
+                            }
+                            if constexpr (kHandMfma && o / 2 >= kVecChunks) asm volatile("" : "+a"(to));
+                        });
+                    });
+                    const uint32_t slot = b * 32u + uint32_t(qn);
+                    if (b < a.n_blocks && slot < a.n) {
+                        const float sc = a.scales[slot];
+                        // (a scale that is not a number gives no row a score)
+                        if (sc >= 1e-30f && sc <= 1e30f) inv = 1.0f / sc;
+                        else odd = sc == sc;
+                    }
+                }
+                if (lane < 32) s_vs[(wave * BLK + k) * 32 + lane] = inv;
+                odd_rows[k] = uint32_t(__ballot(odd));
+                return;
+            }
             const uint32_t b = has_k ? j * step : 0u;
             blk[k] = b;
             float sc = __int_as_float(0x7fc00000);
@@ -519,6 +595,29 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         // allowed row, the better of the two lanes that share a query, one candidate per block and
         // query -- a real score of a real row, so the k-th best of these is a floor k scanned rows
         // reach.  One launch over a round of blocks; the hot loop never comes here.
+        // NEAR: the rows of block k still in for the lane's query (half of them; the other lane has the others).
+        auto near_tile = [&](int t, float2 tq, auto kk) {
+            constexpr int k = decltype(kk)::value;
+            if (BLK > 1 && blk[k] >= nj) return;
+            const float4 *iv = reinterpret_cast<const float4 *>(s_vs + (wave * BLK + k) * 32 + 4 * h);
+            uint32_t in = 0u;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const float4 v = iv[2 * r4];
+                const float inv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int sum = kHandMfma ? acc[k][4 * r4 + e] + 0x4b400000 : acc[k][4 * r4 + e];
+                    in = __builtin_amdgcn_alignbit(in, __float_as_uint(fmaf(tq.x, inv[e], tq.y) - __int_as_float(sum)), 31);
+                }
+            }
+            if (odd_rows[k] != 0u) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) in |= ((odd_rows[k] >> (8 * (r >> 2) + 4 * h + (r & 3))) & 1u) << (15 - r);
+            }
+            uint16_t *out = a.near.masks + ((size_t(t) * a.near.groups + blk[k] / kNearBlocks) * 32 * kNearBlocks + blk[k] % kNearBlocks) * 2;
+            out[uint32_t(qn) * (kNearBlocks * 2) + uint32_t(h)] = uint16_t(in);
+        };
         auto best_tile = [&](int q, auto kk) {
             constexpr int k = decltype(kk)::value;
             const float2 qp = *reinterpret_cast<const float2 *>(&sqt[q].qs);
@@ -555,13 +654,15 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         for (int t = 0; t < nt; ++t) {
             const int q = t * kQTile + qn;
             if (has) {
-                if constexpr (!kHandMfma)
-                    static_for<BLK>([&](auto kk) { acc[decltype(kk)::value] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}; });
+                if constexpr (!kHandMfma) {
+                    constexpr int z = NEAR != 0 ? 0x4b400000 : 0;
+                    static_for<BLK>([&](auto kk) { acc[decltype(kk)::value] = v16i{z, z, z, z, z, z, z, z, z, z, z, z, z, z, z, z}; });
+                }
                 slice_mfmas(IntC<0>{});
                 // the tile's accumulator bounds, fetched and converted under the MFMAs
                 const float2 tq = *reinterpret_cast<const float2 *>(&sq[q].ta);
                 int bound[BLK];
-                static_for<BLK>([&](auto kk) {
+                if constexpr (NEAR == 0) static_for<BLK>([&](auto kk) {
                     constexpr int k = decltype(kk)::value;
                     const float bf = fmaf(tq.x, __int_as_float(inv_vmax[k]), -tq.y) - 1.0f;
                     asm("v_cvt_i32_f32 %0, %1" : "=v"(bound[k]) : "v"(bf));   // saturates; NaN gives 0
@@ -590,6 +691,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                 if (KS == 1 || part == 0) static_for<BLK>([&](auto kk) {
                     constexpr int k = decltype(kk)::value;
                     if constexpr (kHandMfma && KS == 1) mfma_settle(acc[k]);
+                    if constexpr (NEAR != 0) { near_tile(t, tq, kk); return; }
                     if constexpr (BLK == 1) {
                         if (best_mode) { best_tile(q, kk); return; }
                     }
@@ -616,6 +718,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
         if (has) close_stream();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // requests still in flight write this workgroup's LDS
+    if constexpr (NEAR != 0) return;
     if constexpr (BLK == 1) {
         if (a.best_out != nullptr) return;
     }
@@ -740,17 +843,62 @@ int wide_grid_blocks(int device) {
     return device_cus(device);      // one 8-wave workgroup per CU: its LDS holds the slice ring
 }
 
-template <int NCH, int NB, int WAVES = 8, int SPT = 2, int BLK = 1, int HO = 1, int KS = 1, bool SPLIT = false, bool ROWS = false>
+template <int NCH, int NB, int WAVES = 8, int SPT = 2, int BLK = 1, int HO = 1, int KS = 1, bool SPLIT = false, bool ROWS = false, int NEAR = 0>
 static hipError_t launch_wide_n(const ScanArgs &a, int grid, hipStream_t s) {
     const size_t lds = wide_lds_bytes(wide_ring(HO), KS * 2 * (NCH / SPT) * 1024, a.nq_tile, BLK, KS, SPLIT);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS, NEAR>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS>), dim3(grid), dim3(WAVES * 64), lds, s, a);
+    hipLaunchKernelGGL((k_scan_p4_wide<NCH, NB, WAVES, SPT, BLK, HO, KS, SPLIT, ROWS, NEAR>), dim3(grid), dim3(WAVES * 64), lds, s, a);
     return hipGetLastError();
+}
+
+// Instances for 2- and 3-bit codes: those for the same products a row without the byte table.
+template <int NEAR>
+static hipError_t launch_near_chunks(const ScanArgs &a, int chunks, int grid, hipStream_t s) {
+    switch (chunks) {
+        case 2: return launch_wide_n<2, 2, 8, 1, 6, 8, 1, false, false, NEAR>(a, grid, s);
+        case 4: return launch_wide_n<4, 2, 8, 1, 4, 6, 1, false, false, NEAR>(a, grid, s);
+        case 6: return launch_wide_n<6, 2, 8, 1, 3, 4, 1, false, false, NEAR>(a, grid, s);
+        case 8: return launch_wide_n<8, 4, 8, 1, 2, 3, 1, false, false, NEAR>(a, grid, s);
+        case 10: return launch_wide_n<10, 2, 8, 2, 2, 2, 1, false, false, NEAR>(a, grid, s);
+        case 12: return launch_wide_n<12, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 14: return launch_wide_n<14, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 16: return launch_wide_n<16, 4, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 18: return launch_wide_n<18, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 20: return launch_wide_n<20, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 22: return launch_wide_n<22, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        case 24: return launch_wide_n<24, 2, 8, 2, 1, 2, 1, false, false, NEAR>(a, grid, s);
+        default: break;
+    }
+    if constexpr (NEAR == 2) {
+        switch (chunks) {
+            case 28: return launch_wide_n<28, 2, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            case 32: return launch_wide_n<32, 4, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            case 36: return launch_wide_n<36, 2, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            case 40: return launch_wide_n<40, 4, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            case 44: return launch_wide_n<44, 2, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            case 48: return launch_wide_n<48, 4, 4, 4, 1, 1, 1, false, false, NEAR>(a, grid, s);
+            default: break;
+        }
+    }
+    return hipErrorInvalidValue;
+}
+// The least of them that holds the row (3-bit rows beyond 24 chunks leave too many rows in: 2.0 standard deviations at 2048 dimensions).
+int near_chunks(int nch, int bits) {
+    const int c = bits == 2 ? 2 * nch : bits == 3 ? nch : 0;
+    if (c == 0 || c > (bits == 2 ? 48 : 24)) return 0;
+    return c <= 24 ? c + (c & 1) : (c + 3) / 4 * 4;
+}
+int near_nch(int nch, int bits) { return bits == 2 ? near_chunks(nch, bits) / 2 : near_chunks(nch, bits); }
+int near_blocks_per_workgroup(int nch, int bits) { return wide_blocks_per_workgroup(near_chunks(nch, bits)); }
+hipError_t launch_scan_near(const ScanArgs &a, int bits, int grid, hipStream_t s) {
+    if (a.nq_tile <= 0 || a.mask != nullptr || a.rows != nullptr || a.near.groups == 0) return hipErrorInvalidValue;
+    const int chunks = near_chunks(a.nch, bits);
+    return bits == 2 ? launch_near_chunks<2>(a, chunks, grid, s) : launch_near_chunks<3>(a, chunks, grid, s);
 }
 
 // Row lengths whose instance decodes half of a chunk through the LDS byte table: their weights

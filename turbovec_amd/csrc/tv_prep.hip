@@ -21,6 +21,11 @@ struct PrepArgs {
     int dim, log_block, G, nch;
     uint8_t *tables, *mx;           // mx: or null
     float *qscale, *qbias;
+    int near_nch;                   // chunks of the row there, the last ones zero
+    uint8_t *near;                  // or null: int8 weights of the scan that goes before the tables, ...
+    float *near_unit, *near_err;    // ... per query what one unit of its sums is in table units, and how far a row's table sum may lie above
+    float cs;                       // the codebook over its int8 levels
+    uint32_t lv[2];                 // the levels
     float *rot_out;                 // when given: the rotated (and calibrated) rows
     size_t nq;
     uint64_t *stamp;
@@ -271,7 +276,40 @@ __device__ __forceinline__ void mx_put(uint8_t *mx, int nch, int qi, int g, uint
     }
 }
 
-template <int BITS, bool MX>
+// Field f of byte-group g of a query's int8 weights, as the B operands of k_scan_p4_wide's instances for such codes read them: per
+// chunk one 1 KiB fragment per field of a code byte (the highest bits first), in it 16 byte-groups to a lane.
+__device__ __forceinline__ size_t near_at(int qi, int nch, int fields, int g, int f) {
+    return (size_t(qi / kQTile) * nch + size_t(g >> 5)) * size_t(fields) * 1024 + size_t(f) * 1024 + size_t(((g & 31) >> 4) * 32 + qi % kQTile) * 16 + size_t(g & 15);
+}
+// The int8 weights of one nibble and what they leave out.  A row's table sum is, nibble by nibble, an entry
+// T[v] of a table of 16 (8); the scan in front of the tables takes unit * (weights . levels of the codes) in its place, and what
+// the entry exceeds that by is at most `over`, over all values of the nibble.  The weights are the query's dimensions in int8, or
+// their neighbours where those leave less: 9 (3) pairs, 1536 dimensions 2-bit 1.10 standard deviations of the score instead of 1.22.
+template <int BITS>
+__device__ __forceinline__ void near_fit(const uint32_t *w, const float *q, float inv_u, float unit, const PrepArgs &a, int8_t (&out)[2], float &over) {
+    constexpr int cpn = BITS == 2 ? 2 : 1, N = BITS == 2 ? 4 : 8;
+    float lev[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) lev[i] = unit * float(int8_t(a.lv[i / 4] >> (8 * (i & 3))));
+    int w0[2] = {0, 0};
+#pragma unroll
+    for (int c = 0; c < cpn; ++c) w0[c] = int(fminf(fmaxf(rintf(q[c] * inv_u), -127.0f), 127.0f));      // (NaN gives -127: any weights do)
+    over = __int_as_float(0x7f800000);
+    for (int d0 = -1; d0 <= 1; ++d0) {
+        for (int d1 = cpn == 2 ? -1 : 0; d1 <= (cpn == 2 ? 1 : 0); ++d1) {
+            const int a0 = min(max(w0[0] + d0, -127), 127), a1 = min(max(w0[1] + d1, -127), 127);
+            float most = -__int_as_float(0x7f800000);
+#pragma unroll
+            for (int v = 0; v < (BITS == 2 ? 16 : 8); ++v) {
+                const float t = float((w[v / 4] >> (8 * (v & 3))) & 0xffu);
+                most = fmaxf(most, BITS == 2 ? (t - float(a0) * lev[v >> 2]) - float(a1) * lev[v & 3] : t - float(a0) * lev[v & 7]);
+            }
+            if (most < over || (d0 == -1 && d1 <= 0 && over == __int_as_float(0x7f800000))) { over = most; out[0] = int8_t(a0); out[1] = int8_t(a1); }
+        }
+    }
+}
+
+template <int BITS, bool MX, bool NEAR>
 __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
     extern __shared__ __align__(16) float prep_lds[];
     __shared__ float red[4];
@@ -286,6 +324,11 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         for (int i = t; i < a.nch * 64; i += kPrepThreads) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
         if constexpr (MX)
             for (int g = t; g < a.nch * 32; g += kPrepThreads) mx_put<BITS>(a.mx, a.nch, int(qi), g, make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0));
+        if constexpr (NEAR)
+            for (int g = t; g < a.near_nch * 32; g += kPrepThreads) {
+#pragma unroll
+                for (int f = 0; f < cpb; ++f) a.near[near_at(int(qi), a.near_nch, cpb, g, f)] = 0;
+            }
         if (t == 0) { a.qscale[qi] = 0.0f; a.qbias[qi] = 0.0f; }
         return;
     }
@@ -325,8 +368,18 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         a.qscale[qi] = scale;
         a.qbias[qi] = bias + bias_corr;      // (+0 without a pair, search.rs:3176-3185)
     }
+    float near_inv = 0.0f, unit = 0.0f, over_sum = 0.0f;
+    if constexpr (NEAR) {
+        float m = 0.0f;
+        for (int d = t; d < a.dim; d += kPrepThreads) m = fmaxf(m, fabsf(A[d]));
+        float u = block_max_256(m, red) / 127.0f;
+        if (!(u >= FLT_MIN)) u = 1.0f;
+        near_inv = 1.0f / u;
+        unit = (inv_scale * u) * a.cs;
+    }
     for (int g = t; g < a.nch * 32; g += kPrepThreads) {
         uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        int8_t nw[4] = {0, 0, 0, 0};
         if (g < G) {
 #pragma unroll
             for (int sub = 0; sub < 2; ++sub) {
@@ -344,6 +397,34 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         o[0] = hi;
         o[1] = lo;
         if constexpr (MX) mx_put<BITS>(a.mx, a.nch, int(qi), g, hi, lo);
+        if constexpr (NEAR) {
+            if (g < G) {
+#pragma unroll
+                for (int sub = 0; sub < 2; ++sub) {
+                    int8_t to[2] = {0, 0};
+                    float over;
+                    near_fit<BITS>(w + 4 * sub, A + g * cpb + sub * (cpb / 2), near_inv, unit, a, to, over);
+                    over_sum += over;
+#pragma unroll
+                    for (int c = 0; c < cpb / 2; ++c) nw[sub * (cpb / 2) + c] = to[c];
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < cpb; ++f) a.near[near_at(int(qi), a.near_nch, cpb, g, f)] = uint8_t(nw[f]);
+        }
+    }
+    if constexpr (NEAR) {
+        for (int g = a.nch * 32 + t; g < a.near_nch * 32; g += kPrepThreads) {
+#pragma unroll
+            for (int f = 0; f < cpb; ++f) a.near[near_at(int(qi), a.near_nch, cpb, g, f)] = 0;
+        }
+        for (int d = 32; d >= 1; d >>= 1) over_sum += __shfl_xor(over_sum, d);
+        if ((t & 63) == 0) red[t >> 6] = over_sum;
+        __syncthreads();
+        if (t == 0) {
+            a.near_unit[qi] = unit;
+            a.near_err[qi] = (red[0] + red[1]) + (red[2] + red[3]);
+        }
     }
     if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
     if (t == 0 && a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
@@ -360,6 +441,7 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     a.dim = g.dim; a.log_block = __builtin_ctz(unsigned(r.block)); a.G = g.G; a.nch = g.nch;
     a.tables = r.tables; a.mx = r.tables_mx; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
     a.nq = nq; a.stamp = r.stamp; a.cleared = r.cleared;
+    a.near_nch = near_nch(g.nch, g.bits); a.near = r.near; a.near_unit = r.near_unit; a.near_err = r.near_err; a.cs = r.cs; a.lv[0] = r.lv[0]; a.lv[1] = r.lv[1];
     const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
     auto launch = [&](auto kernel, auto... rest) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
@@ -370,8 +452,12 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     if (r.permute_dot) return launch(k_prep_p, r.cs, r.split);
     auto tables = [&](auto mx) -> hipError_t {
         constexpr bool M = decltype(mx)::value != 0;
-        return g.bits == 2 ? launch(k_prep_lut<2, M>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3, M>, r.centroids) : launch(k_prep_lut<4, M>, r.centroids);
+        return g.bits == 2 ? launch(k_prep_lut<2, M, false>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3, M, false>, r.centroids) : launch(k_prep_lut<4, M, false>, r.centroids);
     };
+    if (r.near != nullptr) {
+        if (a.near_nch == 0 || r.tables_mx == nullptr) return hipErrorInvalidValue;
+        return g.bits == 2 ? launch(k_prep_lut<2, true, true>, r.centroids) : launch(k_prep_lut<3, true, true>, r.centroids);
+    }
     return r.tables_mx != nullptr ? tables(IntC<1>{}) : tables(IntC<0>{});
 }
 
