@@ -262,7 +262,7 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * small indexes (bits 1 and 2 do too), and those of up to 16384 blocks by the
  * levels of rows that tests lay data out against; bit 6 has filtered searches
  * gather the allowed rows first whatever their number; bit 7 has u8-LUT batches
- * without a filter take the int8 scan in front of the tables (more than sixteen
+ * take the int8 scan in front of the tables (more than sixteen
  * queries over a large index otherwise) wherever it has an instance for the row
  * length; without bit 6 any other bit, bit 5
  * of no other meaning too, has them read the mask as they scan. */

@@ -60,6 +60,36 @@ def test_matches_oracle(oracle, dim, bits, n, nq, calibrated):
     ix.close()
 
 
+@pytest.mark.parametrize("dim,bits,n,nq", [(128, 2, 700_017, 70), (1000, 3, 150_003, 33), (1536, 2, 150_031, 97)])
+def test_filters(dim, bits, n, nq):
+    """Masks read as the rows are, and searches of the allowed rows' copies."""
+    from turbovec_amd import _lib as T
+    gen = torch.Generator(device="cuda:0").manual_seed(dim)
+    ix = T.NativeIndex(dim, bits)
+    v = torch.randn(n, dim, device="cuda:0", generator=gen)
+    torch.cuda.synchronize()
+    ix.add_dev(v.data_ptr(), n)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    rng = np.random.default_rng(n)
+    for m in (rng.random(n) < 0.9, rng.random(n) < 0.3, np.arange(n) >= n // 2, np.arange(n) % 64 < 32):
+        words = T.pack_mask(m)[0]
+        for k in (1, 40):
+            ix.set_path(1)
+            s1, i1 = ix.search(q, k, mask_words=words)
+            for path in (TWO_STEP, TWO_STEP + 64):
+                ix.set_path(path)
+                s, i = ix.search(q, k, mask_words=words)
+                assert ix.last_scan_ms()[1] >= 2, path
+                assert np.array_equal(i, i1) and bits_equal(s, s1), path
+    few = T.pack_mask(rng.random(n) < 0.0005)[0]            # too few for a sample's floor: the other scans
+    ix.set_path(1)
+    s1, i1 = ix.search(q, 10, mask_words=few)
+    ix.set_path(TWO_STEP)
+    s, i = ix.search(q, 10, mask_words=few)
+    assert np.array_equal(i, i1) and bits_equal(s, s1)
+    ix.close()
+
+
 def test_row_scales_without_a_bound(oracle):
     """Scales that are zero, negative, subnormal, huge, infinite or no number, and rows that tie."""
     from turbovec_amd import _lib as T

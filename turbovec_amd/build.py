@@ -32,8 +32,9 @@ FLAGS = [
 # k_scan_p4_batched and the other LUT scans leave every wait to the compiler.)
 NO_SCRATCH = re.compile(r"k_scan_p4I|k_scan_p4_multiI|k_scan_p4_wideI|k_scan_lut16I|k_scan_lut_mxI|k_probe_mfma")
 # A scalar register kept in a lane of a vector register (no memory, and never a register a request
-# is on its way to) is harmless; this kernel's operand constants overflow the scalar file.
-SGPR_LANES = re.compile(r"k_scan_lut_mxI")
+# is on its way to) is harmless; these kernels' operand constants and arguments overflow the scalar file
+# (k_scan_p4_wide: its instances for 2- and 3-bit codes).
+SGPR_LANES = re.compile(r"k_scan_lut_mxI|k_scan_p4_wideI.*Li[23]EEEv")
 # These address their byte -> levels table by the byte's value alone: the table must sit at LDS
 # address 0, i.e. the kernel may have no static LDS allocation in front of its dynamic one
 # (k_scan_p4, k_scan_p4_multi, and the instances of k_scan_p4_wide whose last template argument but

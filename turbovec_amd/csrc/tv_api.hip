@@ -937,11 +937,17 @@ constexpr int kNearMaxStages = 32;
 // 975 and 901; 4.1M x 384, 64 397 and 378; 7.1M x 456, 84 1431 and 826; 2.8M x 1360, 75 1530 and 943; 2.4M x 512 3-bit, 76 587
 // and 480, 752 dimensions, 52 450 and 532; 1M x 1128, 86 557 and 485; 10M x 1536, 1024 45 900 and 15 900).
 constexpr size_t kNearMinQueries = 65;
+// ... and so many (block, query tile, chunk) triples of 2-bit codes (390K x 144, 636 queries, 480 000 triples, 459 and 220; 87K x 1536, 223,
+// k = 86, 230 000: 271 and 242), and of 3-bit ones, whose one-hot products are half as many (430K x 256, 349 queries, 590 000: 225 and 282; 890K x 280, 129,
+// 700 000: 272 and 284; 1.2M x 248, 319, 1.5e6: 705 and 329).
+constexpr size_t kNearMinWork2 = 200000, kNearMinWork3 = 1200000;
 // Rows that have to be looked up for nothing cost the rest: the share of an index within the margin of the last result (long rows,
 // many results, few rows).  3072 dimensions 2-bit: 2.2M rows, 127 queries, k = 71, 1.1 % 2810 and 3623; 1.2M, 389 queries, k = 24, 0.8 % 4831
 // and 4070; 3.8M, 437 queries, k = 21, 0.5 % 14 583 and 6371; 3-bit: 2M x 976, 373 queries, k = 91, 1 % 2859 and 2480; 3M x 760, 225 queries,
 // k = 92, 0.5 % 2347 and 1271.
-constexpr double kNearShare2 = 0.01, kNearShare3 = 0.008;
+// Less of them where queries are few and the one-hot products cheap: 3-bit, 954K x 1536, 94 queries, k = 3, 0.5 % 681 and 839; 838K x 768, 177, k =
+// 15, 0.3 % 477 and 537; 2.6M x 768, 175, k = 7, 0.1 % 1421 and 1060.
+constexpr double kNearShare2 = 0.01, kNearShare3 = 0.008, kNearShareTile2 = 0.0025, kNearShareTile3 = 0.0005;
 struct NearPlan {
     size_t stages = 0;                    // 0: the search does not go this way
     uint32_t groups[kNearMaxStages] = {};
@@ -960,23 +966,24 @@ int guessed_rank(double share, size_t k) {
     for (; r < int(k) && 1.0 - below > 1e-6; ++r) below += term *= mean / r;
     return r;
 }
-NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_t k_eff, size_t n_blocks, bool masked) {
+// rows: those the search may return, in at least `sure` of the blocks.
+NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_t k_eff, size_t n_blocks, size_t rows, size_t sure) {
     NearPlan p;
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     const int nch = ix->geo.nch, bits = ix->geo.bits;
-    if (!plan.lut_mx || masked || ix->ws_fixed || ix->no_wide || ix->no_batched || ix->row_ladder_left != 0 || ix->allowed.in_place || k_floor > size_t(tv::kMaxPickK)) return p;
+    if (!plan.lut_mx || ix->ws_fixed || ix->no_wide || ix->no_batched || ix->row_ladder_left != 0 || ix->allowed.in_place || k_floor > size_t(tv::kMaxPickK)) return p;
     if (tv::near_chunks(nch, bits) == 0 || tv::near_rescore_queries(nch) == 0 || ix->rows().n >= (size_t(1) << 31)) return p;
     const size_t round = size_t(plan.grid_near) * size_t(tv::near_blocks_per_workgroup(nch, bits)) / tv::kNearBlocks;      // groups
     const size_t total = (n_blocks + tv::kNearBlocks - 1) / tv::kNearBlocks, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
     if (ix->no_direct && n_blocks <= 16384) return p;
-    if (!ix->force_near && (total < 2 * round || cq < kNearMinQueries)) return p;
+    if (!ix->force_near && (cq < kNearMinQueries || n_blocks * tiles * size_t(nch) < (bits == 2 ? kNearMinWork2 : kNearMinWork3))) return p;
     // how far above the int8 product a table sum may lie, in standard deviations of the score, about (measured at 128 to 3072 dimensions),
     // and the share of rows that close to the last result's score, were scores normal
     const double margin = (bits == 2 ? 0.028 : 0.045) * std::sqrt(double(ix->geo.dim));
-    const double tail = std::log(double(ix->rows().n) / double(2 * k_eff));
+    const double tail = std::log(double(rows) / double(2 * k_eff));
     double z = std::sqrt(2.0 * std::max(tail, 1.0));
     for (int i = 0; i < 2; ++i) z = std::sqrt(2.0 * std::max(tail - 0.919 - std::log(z), 0.5));
-    if (!ix->force_near && 0.5 * std::erfc((z - margin) * 0.70710678) > (bits == 2 ? kNearShare2 : kNearShare3)) return p;
+    if (!ix->force_near && 0.5 * std::erfc((z - margin) * 0.70710678) > (bits == 2 ? std::min(kNearShare2, kNearShareTile2 * double(tiles)) : std::min(kNearShare3, kNearShareTile3 * double(tiles)))) return p;
     const size_t group_rows = size_t(tv::kNearBlocks) * ix->geo.block_bytes(), group_masks = tiles * tv::kQTile * tv::kNearBlocks * 4;
     const size_t most = std::max(round, kNearBytes / (group_rows + group_masks) / round * round);
     const size_t per_group = size_t(tv::near_rescore_queries(nch)), query_groups = (cq + per_group - 1) / per_group;
@@ -987,7 +994,7 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     p.step = uint32_t((n_blocks + sample - 1) / sample);
     auto rank_of = [&](double share) { return p.guessed ? guessed_rank(share, k_eff) : int(k_floor); };
     p.rank[0] = rank_of(1.0 / double(p.step));
-    if (sample < 2 * size_t(p.rank[0])) return p;
+    if (sure / p.step < 2 * size_t(p.rank[0])) return p;
     size_t seen = sample / tv::kNearBlocks, largest = 0;
     const double grow = p.guessed ? (margin < 0.9 ? 6.0 : margin < 1.15 ? 4.0 : 2.0) : 2.0;
     for (size_t done = 0; done < total;) {
@@ -1013,6 +1020,10 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     p.rows_bytes = round_up(largest * group_rows, 256);
     p.bytes = p.rows_bytes + largest * group_masks;
     return p;
+}
+bool near_takes(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+    const size_t cq = chunk_len(ix, nq);
+    return near_plan(ix, sampled_plan(ix, cq), cq, k_eff, n_blocks, n_blocks * tv::kVecBlock, n_blocks).stages > 0;
 }
 // Block offset of a repeated pass's level of stride `step`: it samples other blocks than the pass
 // that misjudged the floor, half a stride in (an even number of blocks, so that mask words stay
@@ -1078,21 +1089,24 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff)
 //  - The matrix-unit scan pays its epilogue on every (block, tile) pair: 400K x 1536, 500 queries (200K pairs) 983 and 1038, 1M x
 //    512 (500K pairs) 1060 and 955.
 constexpr size_t kSharedMost = 6000;      // (k times the chunks of a row, shared by eight: 100K x 3072, k = 100 is 4800)
-bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks, bool masked) {
     const size_t nch = size_t(ix->geo.nch), rescored = k_eff * nch, tiles = (std::min(nq, kChunkQueries) + tv::kQTile - 1) / tv::kQTile;
     if (effective_mode(ix) != TV_SCORE_L_U32 || ix->no_lut16 || tv::pick_lds_bytes(int(nch), k_eff, true) > tv::kPickLds) return false;
     const size_t shares = size_t(direct_shares(ix, nq, k_eff));
     if (nq == 1) return rescored <= (n_blocks > 64 ? (shares > 1 ? kSharedMost : 400u) : nch <= 16 ? 120u : 0u);
     if (nq <= size_t(tv::kLut16Queries)) return rescored <= (n_blocks >= 4096 ? 1200u : 720u);
+    // (the two-step scan, whose stages cost some 80 us at least, from so many triples: 560K x 1536, 287 queries, 1.9e6 875 and 546; 180K x 1024,
+    // 389, 6e5 299 and 239; 720K x 768, 188, 8e5 369 and 352; but 280K x 664, 155, 2.6e5 170 and 193; longer rows: 140K x 2048, 621, 1.4e6 610 and 642)
+    if (!masked && ix->geo.bits == 2 && nch <= 12 && tiles >= 3 && n_blocks * tiles * nch >= 600000 && near_takes(ix, nq, k_eff, n_blocks)) return false;
     return n_blocks * tiles <= 200000 && rescored <= std::max<size_t>(tiles <= 4 ? 1200u : 600u, 600u * shares);
 }
-bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks, bool masked) {
     const int nch = ix->geo.nch;
     if (ix->force_robust || ix->no_batched || ix->no_wide || ix->no_direct || ix->force_near) return false;
     if (k_eff > size_t(tv::kMaxPickK) || n_blocks > tv::kMaxPickBlocks) return false;
     const size_t cq = chunk_len(ix, nq), tiles = (cq + tv::kQTile - 1) / tv::kQTile, triples = n_blocks * tiles * nch;
     if (ix->ws_fixed && direct_need(ix, cq, n_blocks, k_eff) > ix->ws_bytes) return false;
-    if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks);
+    if (effective_mode(ix) != TV_SCORE_P) return direct_serves_lut(ix, nq, k_eff, n_blocks, masked);
     if (!tv::best_serves(nch)) return false;
     // (no block is scored again where rows' scores are kept)
     if (!direct_rows(ix, cq, n_blocks, k_eff) &&
@@ -1246,7 +1260,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         return search_robust(ix, d_queries, nq, k_eff, mask, d_out_scores, d_out_idx, timing);
 
     size_t n_blocks = (n + tv::kVecBlock - 1) / tv::kVecBlock;
-    if (direct_serves(ix, nq, k_eff, n_blocks)) return search_direct(ix, d_queries, nq, k_eff, mask, d_out_scores, d_out_idx, timing);
+    if (direct_serves(ix, nq, k_eff, n_blocks, mask != nullptr)) return search_direct(ix, d_queries, nq, k_eff, mask, d_out_scores, d_out_idx, timing);
     // sampling levels take the k_floor-th best as the floor: a deeper order statistic is steadier
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     if (ix->row_ladder_left > 0) --ix->row_ladder_left;
@@ -1258,6 +1272,9 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     rc = ensure_workspace(ix, sampled_need_worst(ix, nq));
     if (rc != TV_OK) return rc;
 
+    auto near_of = [&](const SampledPlan &plan, size_t cq) {
+        return near_plan(ix, plan, cq, k_eff, n_blocks, mask ? n_allowed : ix->rows().n, mask ? sure : n_blocks);
+    };
     // The two-step table scan's stages: memory that nothing is given up for; without it the first passes take the matrix-unit scan alone.
     struct Staged {
         tv_index *ix;
@@ -1267,7 +1284,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     {
         size_t bytes = 0;
         for (const size_t cq : {std::min(nq, kChunkQueries), nq % kChunkQueries})      // (a chunk, and the last one)
-            if (cq != 0 && mode != TV_SCORE_P) bytes = std::max(bytes, near_plan(ix, sampled_plan(ix, cq), cq, k_eff, n_blocks, mask != nullptr).bytes);
+            if (cq != 0 && mode != TV_SCORE_P) bytes = std::max(bytes, near_of(sampled_plan(ix, cq), cq).bytes);
         if (bytes > 0) {
             use_staged(ix, true);
             staged.there = true;
@@ -1316,7 +1333,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const int grid = plan.grid;
             const SamplingSteps steps = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, repeat, mask != nullptr);
             const bool best_first = steps.best_first;
-            NearPlan near = repeat || !staged.there ? NearPlan{} : near_plan(ix, plan, pq_n, k_eff, n_blocks, mask != nullptr);
+            NearPlan near = repeat || !staged.there ? NearPlan{} : near_of(plan, pq_n);
             if (near.bytes > ix->staged.bytes) near = NearPlan{};      // (a group before this one changed the plan)
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
@@ -1372,6 +1389,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 if (const int frc = floors_of_best(near.step, near.rank[0])) return frc;
                 tv::ScanArgs a;
                 fill_scan_args(ix, a);
+                a.mask = mask;
                 a.tables = pq.d_near;
                 a.qscale = pq.d_qscale;
                 a.qbias = pq.d_qbias;
@@ -1527,7 +1545,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
                 const SampledPlan plan = sampled_plan(ix, chunk_at[c + 1] - chunk_at[c]);
-                if (staged.there && near_plan(ix, plan, chunk_at[c + 1] - chunk_at[c], k_eff, n_blocks, mask != nullptr).stages > 0) continue;
+                if (staged.there && near_of(plan, chunk_at[c + 1] - chunk_at[c]).stages > 0) continue;
                 const size_t n_levels = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, false, mask != nullptr).size();
                 for (size_t lv = 1; lv + 1 < n_levels; ++lv)
                     ix->level_repeats += h_over[kGroupQueries + c * SamplingSteps::kMax + lv] != 0u;
@@ -1555,7 +1573,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         ix->overflow_redos += redo_rows.size() + exact_rows.size();
         if ((redo_rows.size() + exact_rows.size()) * 8 >= gq) {
             const SampledPlan plan = sampled_plan(ix, chunk_at[1] - chunk_at[0]);
-            const NearPlan near = staged.there ? near_plan(ix, plan, chunk_at[1] - chunk_at[0], k_eff, n_blocks, mask != nullptr) : NearPlan{};
+            const NearPlan near = staged.there ? near_of(plan, chunk_at[1] - chunk_at[0]) : NearPlan{};
             if (near.stages > 0 && near.guessed) {
                 // (neighbours that lie together: a share of the rows has all of a query's best or none)
                 ix->near_sure_left = kRowLadderSearches;
@@ -1641,10 +1659,17 @@ constexpr size_t kListedAtOnce = size_t(1) << 18;
 constexpr size_t kGatheredBytes = size_t(1) << 30;      // the largest such copy an index keeps room for
 bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed, bool in_place) {
     const double blocks = n_allowed / tv::kVecBlock + 1.0, each = scan_block_ns(ix, nq);
+    // (the two-step table scan, which skips no blocks, takes as much of that: 0.85 and 0.7 of the time for 3 and 4 tiles, 0.5 for 7, 0.38 for 32)
+    const double tiles = std::min(32.0, double((nq + tv::kQTile - 1) / tv::kQTile)), part = ix->geo.bits == 2 ? 0.33 + 1.5 / tiles : std::min(1.0, 0.4 + 2.5 / tiles);
+    auto near = [&](size_t count, bool masked) {
+        return effective_mode(ix) == TV_SCORE_L_U32 && !direct_serves(ix, nq, k, count, masked) && near_takes(ix, nq, k, count);
+    };
+    const double all = near(size_t(n_blocks), true) ? part * n_blocks * each : live_blocks * each;
+    const double few = near(size_t(blocks), false) ? part * each : each;
     const double passed = nq > size_t(tv::kQTile) ? kPassedBlockNs * double((nq + tv::kQTile - 1) / tv::kQTile) : 0.0;
     const double gather = kGatherNs * double(ix->geo.nch) * ((in_place ? -1.0 : 1.0) + std::min(8.0, live_blocks / blocks));
-    const bool shorter = direct_serves(ix, nq, k, size_t(blocks)) && !direct_serves(ix, nq, k, size_t(n_blocks));
-    return live_blocks * each + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > blocks * (each + passed + gather) + fixed;
+    const bool shorter = direct_serves(ix, nq, k, size_t(blocks), false) && !direct_serves(ix, nq, k, size_t(n_blocks), true);
+    return all + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > blocks * (few + passed + gather) + fixed;
 }
 size_t gathered_need(const tv_index *ix, size_t n_allowed) {
     const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
@@ -1654,7 +1679,7 @@ size_t gathered_need(const tv_index *ix, size_t n_allowed) {
 bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowed) {
     const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
     if (!wide_serves(ix) || !tv::wide_serves_best_of_block(ix->geo.nch)) return false;
-    if (k_eff > size_t(tv::kMaxSampledK) || ix->force_robust || direct_serves(ix, nq, k_eff, blocks)) return false;
+    if (k_eff > size_t(tv::kMaxSampledK) || ix->force_robust || direct_serves(ix, nq, k_eff, blocks, false)) return false;
     for (size_t g0 = 0; g0 < nq; g0 += kGroupQueries) {
         const size_t gq = std::min(kGroupQueries, nq - g0);
         for (size_t c0 = 0, cq; c0 < gq; c0 += cq) {
@@ -3029,9 +3054,9 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t k_eff = std::min(k, ix->n);
     if (k_eff == 0 || nq == 0 || k_eff > size_t(tv::kMaxSampledK) || ix->force_robust) return TV_OK;   // no ladder
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
-    if (direct_serves(ix, nq, k_eff, n_blocks)) return TV_OK;
+    if (direct_serves(ix, nq, k_eff, n_blocks, false)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
-    if (near_plan(ix, plan, chunk_len(ix, nq), k_eff, n_blocks, false).stages > 0) return TV_OK;
+    if (near_takes(ix, chunk_len(ix, nq), k_eff, n_blocks)) return TV_OK;
     const SamplingSteps steps = level_strides(ix, plan, n_blocks, n_blocks, std::max<size_t>(k_eff, 16), false, false);
     *count = steps.size();
     for (size_t i = 0; i < steps.size() && i < cap; ++i) {

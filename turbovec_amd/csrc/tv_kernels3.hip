@@ -434,7 +434,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
                         });
                     });
                     const uint32_t slot = b * 32u + uint32_t(qn);
-                    if (b < a.n_blocks && slot < a.n) {
+                    if (b < a.n_blocks && slot < a.n && (a.mask == nullptr || ((uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> qn) & 1u) != 0u)) {
                         const float sc = a.scales[slot];
                         // (a scale that is not a number gives no row a score)
                         if (sc >= 1e-30f && sc <= 1e30f) inv = 1.0f / sc;
@@ -896,7 +896,7 @@ int near_chunks(int nch, int bits) {
 int near_nch(int nch, int bits) { return bits == 2 ? near_chunks(nch, bits) / 2 : near_chunks(nch, bits); }
 int near_blocks_per_workgroup(int nch, int bits) { return wide_blocks_per_workgroup(near_chunks(nch, bits)); }
 hipError_t launch_scan_near(const ScanArgs &a, int bits, int grid, hipStream_t s) {
-    if (a.nq_tile <= 0 || a.mask != nullptr || a.rows != nullptr || a.near.groups == 0) return hipErrorInvalidValue;
+    if (a.nq_tile <= 0 || a.rows != nullptr || a.near.groups == 0) return hipErrorInvalidValue;
     const int chunks = near_chunks(a.nch, bits);
     return bits == 2 ? launch_near_chunks<2>(a, chunks, grid, s) : launch_near_chunks<3>(a, chunks, grid, s);
 }
