@@ -129,6 +129,8 @@ struct DevicePool {
     tv_index *newest = nullptr;      // of the device's indexes
     static constexpr int kPinned = 64;
     tv_pinned pinned[kPinned];       // host memory: pinned_take
+    static constexpr int kStaged = 4;
+    tv_spare staged[kStaged];        // staged_take
     bool takes(size_t bytes) const { return bytes >= kPoolMinBytes && held + bytes <= kPoolBytes && indexes != 0; }   // mu held
     std::vector<std::pair<size_t, void *>> empty() {      // mu held
         held = 0;
@@ -141,11 +143,13 @@ void free_blocks(const std::vector<std::pair<size_t, void *>> &blocks) {
     for (auto &b : blocks) (void)hipFree(b.second);
 }
 
-// A block some index of the device keeps for its filtered searches and is not using, or null.  pool.mu held.
+// A block some index of the device keeps for its filtered searches and is not using, or one of the table scans' stages, or null.  pool.mu held.
 void *take_spare(DevicePool &pool) {
     for (tv_index *ix = pool.newest; ix != nullptr; ix = ix->older)
-        for (tv_spare *s : {&ix->gathered, &ix->slots, &ix->staged})
+        for (tv_spare *s : {&ix->gathered, &ix->slots})
             if (!s->in_use && s->p != nullptr) { s->bytes = 0; return std::exchange(s->p, nullptr); }
+    for (tv_spare &s : pool.staged)
+        if (!s.in_use && s.p != nullptr) { s.bytes = 0; return std::exchange(s.p, nullptr); }
     return nullptr;
 }
 
@@ -216,6 +220,42 @@ hipError_t device_free(int device, void *p, size_t bytes) {
     return e;
 }
 
+// Room for the stages of one search's two-step table scan (NearPlan): lent to one search of the device at a time, whichever
+// index it is of, so that a device holds as many as it has such searches at once, kStagedBytes in all between them, and they do
+// not take the place of blocks that indexes give up and take again (in the pool a 1 GiB block did: building the next index of 10M x 1536 2-bit
+// rows 85 and 249 ms).  Null where there is no memory for one: nothing is given up for it.
+constexpr size_t kStagedBytes = size_t(2) << 30;
+tv_spare *staged_take(int device, size_t bytes) {
+    DevicePool &pool = g_pool[device];
+    tv_spare *s = nullptr;
+    void *old = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        size_t held = 0;
+        for (tv_spare &b : pool.staged) held += b.bytes;
+        for (tv_spare &b : pool.staged)      // the smallest that is large enough, otherwise the largest there is, or a free place
+            if (!b.in_use && (s == nullptr || (b.bytes >= bytes ? s->bytes < bytes || b.bytes < s->bytes : s->bytes < bytes && b.bytes > s->bytes))) s = &b;
+        if (s == nullptr || (s->bytes < bytes && held - s->bytes + bytes > kStagedBytes)) return nullptr;
+        s->in_use = true;
+        if (s->bytes >= bytes) return s;
+        old = std::exchange(s->p, nullptr);
+        s->bytes = 0;
+    }
+    if (old != nullptr) (void)hipFree(old);
+    void *p = nullptr;
+    size_t got = 0;
+    const hipError_t e = device_alloc(device, bytes, &p, &got, false);
+    std::lock_guard<std::mutex> lock(pool.mu);
+    s->p = p;
+    s->bytes = got;
+    s->in_use = e == hipSuccess;
+    return e == hipSuccess ? s : nullptr;
+}
+void staged_give(int device, tv_spare *s) {
+    std::lock_guard<std::mutex> lock(g_pool[device].mu);
+    s->in_use = false;
+}
+
 int ensure_workspace(tv_index *ix, size_t bytes) {
     if (bytes <= ix->ws_bytes) return TV_OK;
     if (ix->ws_fixed) {   // the caller lent a buffer of fixed size: never replaced
@@ -230,11 +270,11 @@ int ensure_workspace(tv_index *ix, size_t bytes) {
 }
 
 // An allocation of the index that grows on demand: what it held is gone then.
-int ensure_block(tv_index *ix, void *&p, size_t &have, size_t bytes, bool insist = true) {
+int ensure_block(tv_index *ix, void *&p, size_t &have, size_t bytes) {
     if (bytes <= have) return TV_OK;
     if (p) { TV_HIP(device_free(ix->device, p, have)); p = nullptr; have = 0; }
-    bytes = round_up(bytes + (insist ? bytes / 4 : 0), size_t(1) << 16);
-    TV_HIP(device_alloc(ix->device, bytes, &p, &have, insist));
+    bytes = round_up(bytes + bytes / 4, size_t(1) << 16);
+    TV_HIP(device_alloc(ix->device, bytes, &p, &have));
     return TV_OK;
 }
 int ensure_io(tv_index *ix, size_t bytes) { return ensure_block(ix, ix->io, ix->io_bytes, bytes); }
@@ -1219,8 +1259,6 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
 }
 
 int leave_in_place(tv_index *ix, size_t nq, size_t k_eff);
-bool have_block(tv_index *ix, tv_spare &s, size_t bytes, bool insist = true);
-void use_staged(tv_index *ix, bool in_use);
 constexpr size_t kLiveUnknown = ~size_t(0);
 
 // The seam: search::search over device-resident inputs and outputs.
@@ -1278,18 +1316,18 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
     // The two-step table scan's stages: memory that nothing is given up for; without it the first passes take the matrix-unit scan alone.
     struct Staged {
         tv_index *ix;
-        bool there = false;
-        ~Staged() { if (there) use_staged(ix, false); }
+        tv_spare *there = nullptr;
+        bool idle = true;      // (an error may leave launches that still use it)
+        ~Staged() {
+            if (there && !idle) (void)hipStreamSynchronize(ix->stream);
+            if (there) staged_give(ix->device, there);
+        }
     } staged{ix};
     {
         size_t bytes = 0;
         for (const size_t cq : {std::min(nq, kChunkQueries), nq % kChunkQueries})      // (a chunk, and the last one)
             if (cq != 0 && mode != TV_SCORE_P) bytes = std::max(bytes, near_of(sampled_plan(ix, cq), cq).bytes);
-        if (bytes > 0) {
-            use_staged(ix, true);
-            staged.there = true;
-            if (!have_block(ix, ix->staged, bytes, false)) { use_staged(ix, false); staged.there = false; }
-        }
+        if (bytes > 0) staged.there = staged_take(ix->device, bytes);
     }
 
     // (which rows a scan reads, and through which mask, changes between a group's first passes and its repeated ones)
@@ -1334,7 +1372,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
             const SamplingSteps steps = level_strides(ix, plan, n_blocks, mask ? sure : n_blocks, k_floor, repeat, mask != nullptr);
             const bool best_first = steps.best_first;
             NearPlan near = repeat || !staged.there ? NearPlan{} : near_of(plan, pq_n);
-            if (near.bytes > ix->staged.bytes) near = NearPlan{};      // (a group before this one changed the plan)
+            if (near.stages > 0 && near.bytes > staged.there->bytes) near = NearPlan{};      // (a group before this one changed the plan)
             uint32_t *d_level_flags = d_level_flags_all + chunk_no * SamplingSteps::kMax;
             if (head.used + plan.need > ix->ws_bytes) {
                 g_last_error = "internal: workspace smaller than the pass it was sized for";
@@ -1386,6 +1424,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 return TV_OK;
             };
             if (near.stages > 0) {
+                staged.idle = false;
                 if (const int frc = floors_of_best(near.step, near.rank[0])) return frc;
                 tv::ScanArgs a;
                 fill_scan_args(ix, a);
@@ -1397,7 +1436,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
                 a.near_err = pq.d_near_err;
                 a.nq_tile = int(pq_n);
                 a.gtau = d_tau;
-                a.near = tv::NearStage{0, 0, near.total, near.mul, reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(ix->staged.p) + near.rows_bytes), static_cast<uint8_t *>(ix->staged.p)};
+                a.near = tv::NearStage{0, 0, near.total, near.mul, reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(staged.there->p) + near.rows_bytes), static_cast<uint8_t *>(staged.there->p)};
                 tv::NearRescore r{};
                 r.tables = pq.d_tables;
                 r.scales = a.scales;
@@ -1541,6 +1580,7 @@ int search_rows(tv_index *ix, const float *d_queries, size_t nq, size_t k, const
         if (track_levels)
             TV_HIP(hipMemcpyAsync(h_over + kGroupQueries, d_level_flags_all, kLevelFlagWords * 4, hipMemcpyDeviceToHost, ix->stream));
         TV_HIP(hipStreamSynchronize(ix->stream));
+        staged.idle = true;
         if (track_levels) {
             // flags of levels the passes above did not use hold whatever the workspace held: count only the used ones
             for (size_t c = 0; c < n_chunks; ++c) {
@@ -1690,18 +1730,14 @@ bool scans_in_place(const tv_index *ix, size_t nq, size_t k_eff, size_t n_allowe
     }
     return true;
 }
-void use_staged(tv_index *ix, bool in_use) {
-    std::lock_guard<std::mutex> lock(g_pool[ix->device].mu);
-    ix->staged.in_use = in_use;
-}
 // Spares in use, or free to be taken again.
 void use_spares(tv_index *ix, bool in_use) {
     std::lock_guard<std::mutex> lock(g_pool[ix->device].mu);
     ix->slots.in_use = ix->gathered.in_use = in_use;
 }
 // A block, in use already, where there is memory for it.  (The search reads the mask as it scans otherwise, as it would have.)
-bool have_block(tv_index *ix, tv_spare &s, size_t bytes, bool insist) {
-    if (ensure_block(ix, s.p, s.bytes, bytes, insist) == TV_OK) return true;
+bool have_block(tv_index *ix, tv_spare &s, size_t bytes) {
+    if (ensure_block(ix, s.p, s.bytes, bytes) == TV_OK) return true;
     g_last_error.clear();
     return false;
 }
@@ -2173,14 +2209,12 @@ int tv_index_destroy(tv_index *ix) {
     void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
                     ix->d_tau_open};
     use_spares(ix, true);      // (from here on they are freed below)
-    use_staged(ix, true);
     (void)device_free(ix->device, ix->d_codes, ix->codes_bytes);
     (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
     (void)device_free(ix->device, ix->ws, ix->ws_bytes);
     (void)device_free(ix->device, ix->io, ix->io_bytes);
     (void)device_free(ix->device, ix->slots.p, ix->slots.bytes);
     (void)device_free(ix->device, ix->gathered.p, ix->gathered.bytes);
-    (void)device_free(ix->device, ix->staged.p, ix->staged.bytes);
     for (void *p : ptrs) if (p) (void)hipFree(p);
     {
         DevicePool &pool = g_pool[ix->device];
@@ -2190,12 +2224,16 @@ int tv_index_destroy(tv_index *ix) {
         pool.ahead -= ix->ahead;
         const bool last = --pool.indexes == 0;
         const auto blocks = last ? pool.empty() : decltype(pool.blocks){};
+        void *staged[DevicePool::kStaged] = {};
+        for (int i = 0; i < DevicePool::kStaged; ++i)
+            if (last && !pool.staged[i].in_use) { staged[i] = pool.staged[i].p; pool.staged[i] = tv_spare{}; }
         uint8_t *pinned[DevicePool::kPinned];
         int n_pinned = 0;
         for (tv_pinned &b : pool.pinned)
             if (last && !b.lent && b.host) { pinned[n_pinned++] = b.host; b = tv_pinned{}; }
         lock.unlock();
         free_blocks(blocks);
+        for (void *p : staged) if (p) (void)hipFree(p);
         for (int i = 0; i < n_pinned; ++i) (void)hipHostFree(pinned[i]);
     }
     if (ix->h_flags) (void)hipHostFree(ix->h_flags);
@@ -3079,7 +3117,7 @@ int tv_debug_workspace_bytes(const tv_index *cix, size_t *workspace, size_t *sta
     if (!ix) return TV_ERR_BAD_ARGUMENT;
     std::lock_guard<std::mutex> lock(ix->mu);
     std::lock_guard<std::mutex> kept(g_pool[ix->device].mu);
-    if (workspace) *workspace = ix->ws_bytes + ix->slots.bytes + ix->gathered.bytes + ix->staged.bytes;
+    if (workspace) *workspace = ix->ws_bytes + ix->slots.bytes + ix->gathered.bytes;
     if (staging) *staging = ix->io_bytes;
     return TV_OK;
 }

@@ -353,7 +353,6 @@ struct tv_index {
     size_t io_bytes = 0;
     size_t ws_bytes = 0;
     bool ws_fixed = false;         // ws is a lent buffer of fixed size (tv_search_dev_noalloc): never reallocated
-    tv_spare staged;               // the two-step table scan's stages (tv_api.hip: NearPlan)
     tv_spare slots, gathered;      // a filtered search's allowed rows: their slots, and their codes and scales (tv_api.hip: gather_allowed)
     tv_index *older = nullptr, *newer = nullptr;   // the device's indexes, linked (guarded as their pool of blocks is)
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
