@@ -129,7 +129,7 @@ struct PrepRequest {
     const float *shift, *scale;     // the TQ+ pair, or null
     bool permute_dot;               // int8 weights (cs, split: k_scan_p4's order) or u8 tables (centroids)
     bool split;
-    float cs;
+    float cs, near_cs;
     const float *centroids;
     uint8_t *tables;
     uint8_t *tables_mx;             // or null: u8 tables also as the operands of k_scan_lut_mx
@@ -317,6 +317,8 @@ struct tv_index {
     std::vector<float> tq_shift, tq_scale;
     int8_t levels[16] = {0};
     float cs = 1.0f;
+    int8_t near_levels[8] = {0};       // the same for 2- and 3-bit codes, as the scan in front of the tables takes them
+    float near_cs = 1.0f;
 
     hipStream_t stream = nullptr;
     hipEvent_t ev_start[tv::kTimedLaunches] = {}, ev_stop[tv::kTimedLaunches] = {};

@@ -284,7 +284,7 @@ __device__ __forceinline__ size_t near_at(int qi, int nch, int fields, int g, in
 // The int8 weights of one nibble and what they leave out.  A row's table sum is, nibble by nibble, an entry
 // T[v] of a table of 16 (8); the scan in front of the tables takes unit * (weights . levels of the codes) in its place, and what
 // the entry exceeds that by is at most `over`, over all values of the nibble.  The weights are the query's dimensions in int8, or
-// their neighbours where those leave less: 9 (3) pairs, 1536 dimensions 2-bit 1.10 standard deviations of the score instead of 1.22.
+// their neighbours where those leave less over the mean (levels may be lifted by a constant): 9 (3) pairs, 1536 dimensions 2-bit 1.10 standard deviations of the score instead of 1.22.
 template <int BITS>
 __device__ __forceinline__ void near_fit(const uint32_t *w, const float *q, float inv_u, float unit, const PrepArgs &a, int8_t (&out)[2], float &over) {
     constexpr int cpn = BITS == 2 ? 2 : 1, N = BITS == 2 ? 4 : 8;
@@ -294,17 +294,19 @@ __device__ __forceinline__ void near_fit(const uint32_t *w, const float *q, floa
     int w0[2] = {0, 0};
 #pragma unroll
     for (int c = 0; c < cpn; ++c) w0[c] = int(fminf(fmaxf(rintf(q[c] * inv_u), -127.0f), 127.0f));      // (NaN gives -127: any weights do)
-    over = __int_as_float(0x7f800000);
+    float best = __int_as_float(0x7f800000);
+    over = best;
     for (int d0 = -1; d0 <= 1; ++d0) {
         for (int d1 = cpn == 2 ? -1 : 0; d1 <= (cpn == 2 ? 1 : 0); ++d1) {
-            const int a0 = min(max(w0[0] + d0, -127), 127), a1 = min(max(w0[1] + d1, -127), 127);
+            const int a0 = min(max(w0[0] + d0, -127), 127), a1 = cpn == 2 ? min(max(w0[1] + d1, -127), 127) : 0;
             float most = -__int_as_float(0x7f800000);
 #pragma unroll
             for (int v = 0; v < (BITS == 2 ? 16 : 8); ++v) {
                 const float t = float((w[v / 4] >> (8 * (v & 3))) & 0xffu);
                 most = fmaxf(most, BITS == 2 ? (t - float(a0) * lev[v >> 2]) - float(a1) * lev[v & 3] : t - float(a0) * lev[v & 7]);
             }
-            if (most < over || (d0 == -1 && d1 <= 0 && over == __int_as_float(0x7f800000))) { over = most; out[0] = int8_t(a0); out[1] = int8_t(a1); }
+            const float cost = most + 0.5f * (lev[0] + lev[N - 1]) * float(a0 + a1);
+            if (cost < best || (d0 == -1 && d1 <= 0 && best == __int_as_float(0x7f800000))) { best = cost; over = most; out[0] = int8_t(a0); out[1] = int8_t(a1); }
         }
     }
 }
@@ -441,7 +443,7 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     a.dim = g.dim; a.log_block = __builtin_ctz(unsigned(r.block)); a.G = g.G; a.nch = g.nch;
     a.tables = r.tables; a.mx = r.tables_mx; a.qscale = r.qscale; a.qbias = r.qbias; a.rot_out = r.rot_out;
     a.nq = nq; a.stamp = r.stamp; a.cleared = r.cleared;
-    a.near_nch = near_nch(g.nch, g.bits); a.near = r.near; a.near_unit = r.near_unit; a.near_err = r.near_err; a.cs = r.cs; a.lv[0] = r.lv[0]; a.lv[1] = r.lv[1];
+    a.near_nch = near_nch(g.nch, g.bits); a.near = r.near; a.near_unit = r.near_unit; a.near_err = r.near_err; a.cs = r.near_cs; a.lv[0] = r.lv[0]; a.lv[1] = r.lv[1];
     const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
     auto launch = [&](auto kernel, auto... rest) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
