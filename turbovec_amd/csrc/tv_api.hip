@@ -497,22 +497,50 @@ void derive_levels(tv_index *ix) {
     }
 }
 
-int upload_tables(tv_index *ix) {
-    const size_t dim = size_t(ix->geo.dim);
-    TV_HIP(hipMemcpyAsync(ix->d_signs, ix->rot.signs.data(), 2 * dim * sizeof(float), hipMemcpyHostToDevice,
-                          ix->stream));
-    TV_HIP(hipMemcpyAsync(ix->d_perms, ix->rot.perms.data(), 2 * dim * sizeof(uint32_t), hipMemcpyHostToDevice,
-                          ix->stream));
-    std::vector<uint32_t> packed(2 * dim);
-    ix->packed_ok = tv::encode_pack_tables(ix->rot.signs.data(), ix->rot.perms.data(), int(dim), ix->rot.block, packed.data());
-    if (ix->packed_ok) TV_HIP(hipMemcpyAsync(ix->d_packed, packed.data(), 2 * dim * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
-    float cen[16] = {0};
-    for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
-    TV_HIP(hipMemcpyAsync(ix->d_centroids, cen, sizeof cen, hipMemcpyHostToDevice, ix->stream));
-    TV_HIP(hipStreamSynchronize(ix->stream));
-    return TV_OK;
+// The tables that only the dimension decides, with the encoder's form of them: as an index's device tables begin (signs, gathers,
+// packed words, two rounds each).  Drawing and packing them took 48 us of 1536 dimensions' 110 an index, 129 at 3072: the last kTableMemo are kept.
+struct TableImage {
+    tv::RotationTables rot;
+    std::vector<uint32_t> words;
+    bool packed_ok = false;
+};
+constexpr size_t kTableMemo = 8;
+void lay_out_tables(const tv::RotationTables &rot, TableImage &t) {
+    const size_t d2 = 2 * size_t(rot.dim);
+    t.words.assign(3 * d2, 0u);
+    std::memcpy(t.words.data(), rot.signs.data(), d2 * sizeof(float));
+    std::memcpy(t.words.data() + d2, rot.perms.data(), d2 * sizeof(uint32_t));
+    t.packed_ok = tv::encode_pack_tables(rot.signs.data(), rot.perms.data(), rot.dim, rot.block, t.words.data() + 2 * d2);
+}
+std::shared_ptr<const TableImage> default_tables(int dim) {
+    static std::mutex mu;
+    static std::vector<std::shared_ptr<const TableImage>> memo;      // the one used last first
+    std::lock_guard<std::mutex> lock(mu);
+    for (size_t i = 0; i < memo.size(); ++i)
+        if (memo[i]->rot.dim == dim) {
+            std::rotate(memo.begin(), memo.begin() + i, memo.begin() + i + 1);
+            return memo[0];
+        }
+    auto t = std::make_shared<TableImage>();
+    t->rot = tv::make_rotation_tables(dim);
+    lay_out_tables(t->rot, *t);
+    if (memo.size() == kTableMemo) memo.pop_back();
+    memo.insert(memo.begin(), t);
+    return t;
 }
 
+// On the index's stream, from pinned memory of its own: one copy (four from pageable memory, with a wait of their own, took 40 us of
+// an index's 90).  The caller has waited for the copy before.
+int upload_tables(tv_index *ix, const TableImage &t) {
+    const size_t words = t.words.size();
+    std::memcpy(ix->h_tables, t.words.data(), words * sizeof(uint32_t));
+    float *cen = reinterpret_cast<float *>(ix->h_tables + words);
+    std::fill_n(cen, 16, 0.0f);
+    for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
+    ix->packed_ok = t.packed_ok;
+    TV_HIP(hipMemcpyAsync(ix->d_signs, ix->h_tables, (words + 16) * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
+    return TV_OK;
+}
 int effective_mode(const tv_index *ix);
 // Queries one LUT-scan launch serves: the scalar definition's float chain runs one query at a time.
 int lut_tile_q(const tv_index *ix, int k) { return effective_mode(ix) == TV_SCORE_L_SCALAR ? 1 : tv::lut_tile_queries(ix->geo.nch, k); }
@@ -2166,27 +2194,33 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         else if (ix->geo.nch > 24 && ix->geo.nch <= 48) ix->geo.nch = (ix->geo.nch + 3) / 4 * 4;
         else if (ix->geo.nch <= 24) ix->geo.nch += ix->geo.nch & 1;
     }
-    ix->rot = tv::make_rotation_tables(dim);
+    const auto tables = default_tables(dim);
+    ix->rot = tables->rot;
     ix->cb = tv::make_codebook(bits, dim);
     derive_levels(ix);
     int rc = TV_OK;
     do {
         if (hipStreamCreateWithFlags(&ix->stream, hipStreamNonBlocking) != hipSuccess) { rc = TV_ERR_HIP; break; }
-        // (through device_alloc, which empties the pool before it refuses; too small for the pool themselves)
-        auto table = [&](auto *&p, size_t count) {
-            size_t got = 0;
-            return device_alloc(device, count * sizeof *p, reinterpret_cast<void **>(&p), &got) == hipSuccess;
-        };
-        if (!table(ix->d_signs, 2 * size_t(dim)) || !table(ix->d_perms, 2 * size_t(dim)) || !table(ix->d_packed, 2 * size_t(dim)) ||
-            !table(ix->d_centroids, 16) || !table(ix->d_tq_shift, size_t(dim)) || !table(ix->d_tq_scale, 2 * size_t(dim)) ||
-            !table(ix->d_tau_open, kTauOpenInts)) {
+        // One block (through device_alloc, which empties the pool before it refuses; too small for the pool itself): what upload_tables
+        // copies, the TQ+ pair, the open floors.
+        const size_t d = size_t(dim), words = 9 * d + 16 + kTauOpenInts;
+        size_t got = 0;
+        if (device_alloc(device, words * sizeof(uint32_t), reinterpret_cast<void **>(&ix->d_signs), &got) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
         }
-        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t) + (tv::kStampsBefore + 1) * sizeof(uint64_t), hipHostMallocMapped) != hipSuccess) {
+        ix->d_perms = reinterpret_cast<uint32_t *>(ix->d_signs) + 2 * d;
+        ix->d_packed = ix->d_perms + 2 * d;
+        ix->d_centroids = reinterpret_cast<float *>(ix->d_packed + 2 * d);
+        ix->d_tq_shift = ix->d_centroids + 16;
+        ix->d_tq_scale = ix->d_tq_shift + d;
+        ix->d_tau_open = reinterpret_cast<int *>(ix->d_tq_scale + 2 * d);
+        const size_t flag_bytes = (kGroupQueries + kLevelFlagWords) * sizeof(uint32_t) + (tv::kStampsBefore + 1) * sizeof(uint64_t);
+        if (hipHostMalloc(reinterpret_cast<void **>(&ix->h_flags), flag_bytes + (6 * d + 16) * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
         }
+        ix->h_tables = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(ix->h_flags) + flag_bytes);
         if (hipHostGetDevicePointer(reinterpret_cast<void **>(&ix->d_flags_host), ix->h_flags, 0) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
@@ -2198,12 +2232,11 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         rc = scratch_address(device, &ix->scratch);
         if (rc != TV_OK) break;
         // floors of a search's first sampling level: the order key of -inf for every query, written once
-        if (tv::launch_fill_i32(ix->d_tau_open, int(0x807fffffu), kTauOpenInts, ix->stream) != hipSuccess ||
-            hipStreamSynchronize(ix->stream) != hipSuccess) {
+        if (tv::launch_fill_i32(ix->d_tau_open, int(0x807fffffu), kTauOpenInts, ix->stream) != hipSuccess) {
             rc = TV_ERR_HIP;
             break;
         }
-        rc = upload_tables(ix);
+        rc = upload_tables(ix, *tables);      // (all use of them is on the index's stream, behind this)
     } while (0);
     if (rc != TV_OK) {
         if (g_last_error.empty()) g_last_error = "device allocation failed";
@@ -2218,8 +2251,6 @@ int tv_index_destroy(tv_index *ix) {
     if (!ix) return TV_OK;
     (void)hipSetDevice(ix->device);
     if (ix->stream) (void)hipStreamSynchronize(ix->stream);
-    void *ptrs[] = {ix->d_signs, ix->d_perms, ix->d_packed, ix->d_centroids, ix->d_tq_shift, ix->d_tq_scale,
-                    ix->d_tau_open};
     use_spares(ix, true);      // (from here on they are freed below)
     (void)device_free(ix->device, ix->d_codes, ix->codes_bytes);
     (void)device_free(ix->device, ix->d_scales, ix->scales_bytes);
@@ -2227,7 +2258,7 @@ int tv_index_destroy(tv_index *ix) {
     (void)device_free(ix->device, ix->io, ix->io_bytes);
     (void)device_free(ix->device, ix->slots.p, ix->slots.bytes);
     (void)device_free(ix->device, ix->gathered.p, ix->gathered.bytes);
-    for (void *p : ptrs) if (p) (void)hipFree(p);
+    if (ix->d_signs) (void)hipFree(ix->d_signs);      // (the other tables too)
     {
         DevicePool &pool = g_pool[ix->device];
         std::unique_lock<std::mutex> lock(pool.mu);
@@ -2275,7 +2306,12 @@ int tv_index_set_tables(tv_index *ix, const float *signs, const uint32_t *perms,
             ix->cb.boundaries[i] = (ix->cb.centroids[i] + ix->cb.centroids[i + 1]) * 0.5f;
         derive_levels(ix);
     }
-    return upload_tables(ix);
+    TableImage t;
+    lay_out_tables(ix->rot, t);
+    TV_HIP(hipStreamSynchronize(ix->stream));
+    const int rc = upload_tables(ix, t);
+    if (rc == TV_OK) TV_HIP(hipStreamSynchronize(ix->stream));
+    return rc;
 }
 
 int tv_index_set_calibration(tv_index *ix, const float *shift, const float *scale) {

@@ -360,6 +360,7 @@ struct tv_index {
     tv_rows allowed;               // for the length of such a search: what it reads in place of the index's rows (codes null otherwise)
     tv_rows rows() const { return allowed.codes ? allowed : tv_rows{d_codes, d_scales, n, nullptr, 0, false}; }
     void *scratch = nullptr;       // this device's copy of the library's static scratch array
+    uint32_t *h_tables = nullptr;  // in the allocation of h_flags: the tables on their way to the device
     uint32_t *h_flags = nullptr;   // pinned host memory: the overflow flags of one group of chunks, then the rows to repeat (before a search: a mask's totals)
     uint32_t *d_flags_host = nullptr;   // the device's address of h_flags
     uint64_t *h_stamps = nullptr, *d_stamps = nullptr;   // in the same allocation: the device clock before and after a full scan
