@@ -170,6 +170,19 @@ __device__ __forceinline__ uint32_t byte_x2(uint32_t x) {
     return r;
 }
 
+// A byte of LDS by its address.
+typedef const __attribute__((address_space(3))) uint8_t LdsByte;
+// at + byte B of x, in one instruction.
+template <int B>
+__device__ __forceinline__ uint32_t plus_byte(uint32_t at, uint32_t x) {
+    uint32_t r;
+    if (B == 0) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "v"(at), "v"(x));
+    if (B == 1) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "v"(at), "v"(x));
+    if (B == 2) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "v"(at), "v"(x));
+    if (B == 3) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "v"(at), "v"(x));
+    return r;
+}
+
 // A conditional launch: true when the flag it depends on says there is nothing to do.  The flag is
 // uniform over the grid and written by an earlier launch of the same stream.
 __device__ __forceinline__ bool launch_switched_off(const uint32_t *run_if) {

@@ -176,7 +176,7 @@ hipError_t launch_scan_p4(const ScanArgs &a, int grid, int mode, hipStream_t s);
 // Small indexes without sampling (tv_kernels6.hip): the best row of every block, then the best blocks' rows.
 constexpr int kMaxPickK = 128;             // most results k_pick ranks
 constexpr size_t kMaxPickBlocks = 32768;   // most blocks it chooses from
-constexpr size_t kPickLds = 128 * 1024;    // rows' keys and the query's tables, beside its 13 KiB of fixed buffers
+constexpr size_t kPickLds = 144 * 1024;    // rows' keys and sums and the query's tables, beside its 15 KiB of fixed buffers
 bool best_serves(int nch);
 hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStream_t s);
 // The k_floor-th best of n score words per query as its floor, to tau_out like launch_final.

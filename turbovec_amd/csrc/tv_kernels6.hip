@@ -296,7 +296,7 @@ struct PickArgs {
     int64_t *out_idx;
     const uint32_t *slots;      // when given: the slot of each row, for out_idx
     uint32_t *overflow;
-    uint32_t nq, shares;
+    uint32_t nq, shares, parts;
     uint64_t *counts, *lists;   // shares > 1: per query the number of workgroups that are through with it, and what they found (pick_shared_words)
     uint64_t *stamp;
 };
@@ -321,6 +321,7 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     __shared__ uint32_t n_kept, n_list, s_floor, s_last;
     uint64_t *list = reinterpret_cast<uint64_t *>(dyn);                     // rows of the chosen blocks that can still matter
     uint8_t *wts = dyn + size_t(a.k_eff) * 32 * 8;                          // this query's weights
+    int *s_acc = reinterpret_cast<int *>(wts + size_t(a.nch) * (LUT ? 1024 : 64));     // parts > 1: sums of rows scored in parts
     const uint32_t qi = SHARED ? blockIdx.x % a.nq : blockIdx.x, share = SHARED ? blockIdx.x / a.nq : 0u, shares = SHARED ? a.shares : 1u;
     const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
     const uint32_t k_eff = uint32_t(a.k_eff);
@@ -364,27 +365,46 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     const uint32_t floor_word = s_floor, h = lane >> 5;
     const float qs = a.qscale[qi], qb = a.qbias[qi];
     const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
-    for (uint32_t i = wv * shares + share; i < need; i += W * shares) {
-        const uint32_t b = blocks[i], slot = b * 32u + (lane & 31u);
+    // blocks of this workgroup's share: numbers share, share + shares, ...; parts (a power of two) of a block's chunks to as many waves
+    const uint32_t mine = need > share ? (need - share + shares - 1u) / shares : 0u, log_parts = uint32_t(__builtin_ctz(a.parts));
+    const uint32_t lds_w = uint32_t(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) uint8_t *)wts));
+    auto take = [&](uint32_t b, uint32_t row, int acc) {
+        const uint32_t slot = b * 32u + row;
         const float vs = a.scales[slot];
+        const float s = LUT ? ((float(acc) * qs) + qb) * vs : fmaf(float(acc), qs, qb) * vs;      // search.rs:1174-1177, 1519-1524
+        // (A score of -infinity does not count here either, as it does not in a block's best word: rows that tie there
+        // with rows of blocks that were not chosen are for the exact path to order.)
+        bool ok = slot < a.n && s > -__int_as_float(0x7f800000);
+        if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> row) & 1u;
+        const uint64_t key = sort_key(s, slot);
+        if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
+    };
+    if (a.parts > 1u) {
+        for (uint32_t i = t; i < mine * 32u; i += T) s_acc[i] = 0;
+        __syncthreads();
+    }
+    for (uint32_t it = wv; it < mine << log_parts; it += W) {
+        const uint32_t at = it >> log_parts, part = it & (a.parts - 1u), b = blocks[at * shares + share];
+        const int first = int(uint32_t(a.nch) * part >> log_parts), end = int(uint32_t(a.nch) * (part + 1u) >> log_parts);
         const uint4 *src = reinterpret_cast<const uint4 *>(a.codes) + size_t(b) * a.nch * 64 + lane;
         int acc = 0;
         constexpr int kBurst = 8;
-        for (int c0 = 0; c0 < a.nch; c0 += kBurst) {
+        for (int c0 = first; c0 < end; c0 += kBurst) {
             uint4 x[kBurst];
 #pragma unroll
-            for (int u = 0; u < kBurst; ++u) x[u] = c0 + u < a.nch ? src[(c0 + u) * 64] : make_uint4(0, 0, 0, 0);
+            for (int u = 0; u < kBurst; ++u) x[u] = c0 + u < end ? src[(c0 + u) * 64] : make_uint4(0, 0, 0, 0);
 #pragma unroll
             for (int u = 0; u < kBurst; ++u) {
-                if (c0 + u >= a.nch) break;
+                if (c0 + u >= end) break;
                 const uint32_t d[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
                 if constexpr (LUT) {
-                    const uint8_t *row = wts + ((c0 + u) * 32 + int(h) * 16) * 32;
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const uint32_t byte = (d[e >> 2] >> (8 * (e & 3))) & 0xffu;
-                        acc += int(row[e * 32 + int(byte >> 4)]) + int(row[e * 32 + 16 + int(byte & 15u)]);
-                    }
+                    const uint32_t row = lds_w + uint32_t(((c0 + u) * 32 + int(h) * 16) * 32);
+                    static_for<16>([&](auto ee) {
+                        constexpr int e = decltype(ee)::value;
+                        const uint32_t high = (d[e >> 2] >> 4) & 0x0f0f0f0fu, low = d[e >> 2] & 0x0f0f0f0fu;
+                        acc += int(reinterpret_cast<LdsByte *>(uintptr_t(plus_byte<(e & 3)>(row, high)))[e * 32]) +
+                               int(reinterpret_cast<LdsByte *>(uintptr_t(plus_byte<(e & 3)>(row, low)))[e * 32 + 16]);
+                    });
                     continue;
                 }
                 const uint4 *wq = reinterpret_cast<const uint4 *>(wts) + ((c0 + u) * 2 + h) * 2;
@@ -417,13 +437,14 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
             }
         }
         acc += __shfl_xor(acc, 32);
-        const float s = LUT ? ((float(acc) * qs) + qb) * vs : fmaf(float(acc), qs, qb) * vs;      // search.rs:1174-1177, 1519-1524
-        // (A score of -infinity does not count here either, as it does not in a block's best word: rows that tie there
-        // with rows of blocks that were not chosen are for the exact path to order.)
-        bool ok = lane < 32u && slot < a.n && s > -__int_as_float(0x7f800000);
-        if (ok && a.mask != nullptr) ok = (uint32_t(a.mask[b >> 1] >> ((b & 1) * 32)) >> (lane & 31u)) & 1u;
-        const uint64_t key = sort_key(s, slot);
-        if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
+        if (lane < 32u) {
+            if (a.parts > 1u) atomicAdd(&s_acc[at * 32u + lane], acc);
+            else take(b, lane, acc);
+        }
+    }
+    if (a.parts > 1u) {
+        __syncthreads();
+        for (uint32_t i = t; i < mine * 32u; i += T) take(blocks[(i >> 5) * shares + share], i & 31u, s_acc[i]);
     }
     if constexpr (SHARED) {
         __syncthreads();
@@ -525,7 +546,7 @@ hipError_t launch_pick_rows(const float *scores, uint32_t stride, uint32_t n, in
     return hipGetLastError();
 }
 
-size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64); }
+size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64) + k_eff * 32 * 4; }
 int pick_shares(int device, int nch, size_t k_eff, size_t nq, bool lut) {
     // (a SIMD's worth of blocks at least for each workgroup)
     if (nq == 0 || k_eff * size_t(nch) * (lut ? 3 : 1) < kSharedWork) return 1;
@@ -556,6 +577,17 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     };
     // few queries leave the chip empty: as many waves as there are blocks to score again
     const bool small = a.nq_tile > 256 && a.n_blocks <= 256 * 16;
+    // A block to a wave leaves most of sixteen waves without one where results are few, and the others with a row's chunks one after the
+    // other: parts of a block's chunks go to as many waves, as make the busiest wave's share least, where the chip is empty enough for it to
+    // show.  us a search with whole blocks and so: 60K x 3072, one query, k = 1 60.1 and 51.2; 40K x 3032 3-bit, k = 4 88.8 and 82.4; 24K x 2760 2-bit, k = 2
+    // 62.4 and 58.1; 16K x 1424 3-bit, 4 queries, k = 12 61.0 and 58.6; 50K x 768, 8 queries, k = 1 33.1 and 31.7; short rows level.
+    const size_t waves = small ? 4 : 16, share_blocks = (size_t(k_eff) + size_t(shares) - 1) / size_t(shares);
+    p.parts = 1;
+    if (size_t(a.nq_tile) * size_t(shares) <= size_t(2) * 256) {
+        auto busiest = [&](size_t parts) { return double((share_blocks * parts + waves - 1) / waves) / double(parts); };
+        for (uint32_t parts = 2; parts <= 16 && int(parts) <= a.nch; parts *= 2)
+            if (busiest(parts) < 0.85 * busiest(p.parts)) p.parts = parts;
+    }
     auto form = [&](auto lut_, auto shared_) -> hipError_t {
         constexpr bool L = decltype(lut_)::value != 0, S = decltype(shared_)::value != 0;
         if (a.n_blocks > 1024 * 16) return launch(k_pick<1024, 32, L, S>, 1024);

@@ -30,18 +30,6 @@ constexpr size_t near_lds_bytes(int nch, int qw) {
     return size_t(qw) * near_table_stride(nch) + size_t(kNearWaves) * kNearQueue * 8 + size_t(qw) * (12 + 4 * kNearSubs) + 64;
 }
 
-typedef const __attribute__((address_space(3))) uint8_t LdsByte;
-// at + byte B of x, in one instruction.
-template <int B>
-__device__ __forceinline__ uint32_t plus_byte(uint32_t at, uint32_t x) {
-    uint32_t r;
-    if (B == 0) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "v"(at), "v"(x));
-    if (B == 1) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "v"(at), "v"(x));
-    if (B == 2) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "v"(at), "v"(x));
-    if (B == 3) asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "v"(at), "v"(x));
-    return r;
-}
-
 template <int QW>
 __global__ __launch_bounds__(kNearThreads, QW <= 4 ? 8 : 4) void k_near_rescore(NearRescore a) {
     static_assert(QW >= 1 && QW <= 8 && 8 % QW == 0, "a wave's 64 words are whole groups of eight blocks");
