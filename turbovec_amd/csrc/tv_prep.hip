@@ -10,7 +10,6 @@
 
 namespace tv {
 
-constexpr int kPrepThreads = 256;
 constexpr int kPrepPiece = 1024;     // products of the bias chain in LDS at a time
 
 struct PrepArgs {
@@ -41,10 +40,10 @@ __host__ __device__ constexpr int prep_floats(int dim) { return prep_at(dim - 1)
 typedef float RowPiece __attribute__((ext_vector_type(4), aligned(4)));
 
 // R butterfly stages from stride 2^S on over the whole row.
-template <int R>
+template <int T, int R>
 __device__ __forceinline__ void prep_pass(float *buf, int dim, int S) {
     constexpr int N = 1 << R;
-    for (int g = threadIdx.x; g < dim / N; g += kPrepThreads) {
+    for (int g = threadIdx.x; g < dim / N; g += T) {
         const int base = ((g >> S) << (S + R)) + (g & ((1 << S) - 1));
         float v[N];
 #pragma unroll
@@ -60,10 +59,11 @@ __device__ __forceinline__ void prep_pass(float *buf, int dim, int S) {
 // to be multiplied by inv_sqrt_block, at B's padded places.  Three stages at a time through registers: a
 // barrier per pass instead of one per stage (1536 dimensions: 8 instead of 20, which was most of the time
 // one query's preparation took).
+template <int T>
 __device__ __forceinline__ void rotate_row(const float *src, const float *signs, const uint32_t *perms, int dim, int log_block,
                                            float inv_sqrt_block, float *A, float *B) {
     // the row itself first, 16 bytes at a time: it may lie in host memory, where a gather would fetch it piece by piece
-    for (int i = threadIdx.x; i < dim / 4; i += kPrepThreads) {
+    for (int i = threadIdx.x; i < dim / 4; i += T) {
         const RowPiece p = reinterpret_cast<const RowPiece *>(src)[i];
         *reinterpret_cast<float4 *>(B + 4 * i) = float4{p.x, p.y, p.z, p.w};
     }
@@ -71,7 +71,7 @@ __device__ __forceinline__ void rotate_row(const float *src, const float *signs,
 #pragma unroll
     for (int round = 0; round < 2; ++round) {
         float *buf = round == 0 ? A : B;
-        for (int g = threadIdx.x; g < dim / 8; g += kPrepThreads) {
+        for (int g = threadIdx.x; g < dim / 8; g += T) {
             const uint4 *p4 = reinterpret_cast<const uint4 *>(perms + size_t(round) * dim + 8 * g);
             const float4 *s4 = reinterpret_cast<const float4 *>(signs + size_t(round) * dim + 8 * g);
             const uint4 pa = p4[0], pb = p4[1];
@@ -89,9 +89,9 @@ __device__ __forceinline__ void rotate_row(const float *src, const float *signs,
         }
         __syncthreads();
         for (int S = 3; S < log_block; S += 3) {
-            if (log_block - S >= 3) prep_pass<3>(buf, dim, S);
-            else if (log_block - S == 2) prep_pass<2>(buf, dim, S);
-            else prep_pass<1>(buf, dim, S);
+            if (log_block - S >= 3) prep_pass<T, 3>(buf, dim, S);
+            else if (log_block - S == 2) prep_pass<T, 2>(buf, dim, S);
+            else prep_pass<T, 1>(buf, dim, S);
         }
     }
 }
@@ -102,13 +102,14 @@ __device__ __forceinline__ void rotate_row(const float *src, const float *signs,
 // way of a term there, dim / 256 + 9 here, and those of the magnitude's sum -- rounds to the same float, that is it.
 // Otherwise (one query in 10^5) one thread adds in order.  With the chain always: 3032 dimensions 47 us for one query, now 25.
 // late: becomes true there.
+template <int T>
 __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs &a, float *A, float *B, double *prod, bool &late) {
     const int t = threadIdx.x, dim = a.dim;
-    rotate_row(src, a.signs, a.perms, dim, a.log_block, a.inv_sqrt_block, A, B);
+    rotate_row<T>(src, a.signs, a.perms, dim, a.log_block, a.inv_sqrt_block, A, B);
     float bias = 0.0f;
     if (a.scale != nullptr) {
         double sum = 0.0, mass = 0.0;
-        for (int i = t; i < dim; i += kPrepThreads) {
+        for (int i = t; i < dim; i += T) {
             const double p = double(B[prep_at(i)] * a.inv_sqrt_block) * double(a.shift[i]);
             sum -= p;
             mass += fabs(p);
@@ -117,10 +118,15 @@ __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs
             sum += __shfl_xor(sum, d);
             mass += __shfl_xor(mass, d);
         }
-        if ((t & 63) == 0) { prod[t >> 6] = sum; prod[4 + (t >> 6)] = mass; }
+        if ((t & 63) == 0) { prod[t >> 6] = sum; prod[T / 64 + (t >> 6)] = mass; }
         __syncthreads();
-        sum = (prod[0] + prod[1]) + (prod[2] + prod[3]);
-        mass = (prod[4] + prod[5]) + (prod[6] + prod[7]);
+        sum = 0.0;
+        mass = 0.0;
+#pragma unroll
+        for (int i = 0; i < T / 64; i += 4) {
+            sum += (prod[i] + prod[i + 1]) + (prod[i + 2] + prod[i + 3]);
+            mass += (prod[T / 64 + i] + prod[T / 64 + i + 1]) + (prod[T / 64 + i + 2] + prod[T / 64 + i + 3]);
+        }
         __syncthreads();
         const double slack = double(2 * dim + 256) * 0x1p-53 * mass;
         bias = float(sum - slack);
@@ -129,7 +135,7 @@ __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs
             double bc = 0.0;
             for (int d0 = 0; d0 < dim; d0 += kPrepPiece) {
                 const int m = min(kPrepPiece, dim - d0);      // (a multiple of eight, as dim is)
-                for (int i = t; i < m; i += kPrepThreads) prod[i] = double(B[prep_at(d0 + i)] * a.inv_sqrt_block) * double(a.shift[d0 + i]);
+                for (int i = t; i < m; i += T) prod[i] = double(B[prep_at(d0 + i)] * a.inv_sqrt_block) * double(a.shift[d0 + i]);
                 __syncthreads();
                 if (t == 0) {
                     for (int i = 0; i < m; i += 8) {
@@ -145,7 +151,7 @@ __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs
             bias = float(bc);                                 // (for thread 0, which uses it)
         }
     }
-    for (int i = t; i < dim; i += kPrepThreads) {
+    for (int i = t; i < dim; i += T) {
         float x = B[prep_at(i)] * a.inv_sqrt_block;
         if (a.scale != nullptr) x = x / a.scale[i];
         A[i] = x;
@@ -155,12 +161,15 @@ __device__ __forceinline__ float calibrated_row(const float *src, const PrepArgs
     return bias;
 }
 
-__device__ __forceinline__ float block_max_256(float v, float *red) {
+template <int T>
+__device__ __forceinline__ float block_max(float v, float *red) {
     // exact: max is order-free
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < T / 64; ++i) v = fmaxf(v, red[i]);
     __syncthreads();
     return v;
 }
@@ -192,16 +201,17 @@ __device__ __forceinline__ size_t wfrag_offset(int g, int n, int plane, bool spl
     return size_t(g >> 5) * 2048 + size_t(plane) * 1024 + lane16 + size_t(g & 15);
 }
 
-__global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split) {
+template <int T>
+__global__ __launch_bounds__(T) void k_prep_p(PrepArgs a, float cs, bool split) {
     extern __shared__ __align__(16) float prep_lds[];
-    __shared__ float red[4];
+    __shared__ float red[T / 64];
     __shared__ __align__(16) double prod[kPrepPiece];
     float *A = prep_lds, *B = prep_lds + prep_floats(a.dim);
     const size_t qi = blockIdx.x;
     const int n = int(qi % kQTile), t = threadIdx.x;
     uint8_t *base = a.tables + qi / kQTile * size_t(a.nch) * 2048;
     if (qi >= a.nq) {  // padding query of the last tile: zero weights
-        for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+        for (int g = t; g < a.nch * 32; g += T) {
             base[wfrag_offset(g, n, 0, split)] = 0;
             base[wfrag_offset(g, n, 1, split)] = 0;
         }
@@ -209,13 +219,13 @@ __global__ __launch_bounds__(256) void k_prep_p(PrepArgs a, float cs, bool split
         return;
     }
     bool late = false;
-    const float bias = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod, late);
+    const float bias = calibrated_row<T>(a.q + qi * size_t(a.dim), a, A, B, prod, late);
     float m = 0.0f;
-    for (int d = t; d < a.dim; d += kPrepThreads) m = fmaxf(m, fabsf(A[d]));
-    const float qmax = block_max_256(m, red);
+    for (int d = t; d < a.dim; d += T) m = fmaxf(m, fabsf(A[d]));
+    const float qmax = block_max<T>(m, red);
     float qs = qmax / 127.0f, inv_qs;
     if (qs >= FLT_MIN) inv_qs = 1.0f / qs; else { qs = 1.0f; inv_qs = 1.0f; }
-    for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+    for (int g = t; g < a.nch * 32; g += T) {
         int8_t lo = 0, hi = 0;
         if (g < a.G) {
             lo = int8_t(clamp_round_i8(A[2 * g + 1] * inv_qs));
@@ -311,23 +321,25 @@ __device__ __forceinline__ void near_fit(const uint32_t *w, const float *q, floa
     }
 }
 
-template <int BITS, bool MX, bool NEAR>
-__global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
+template <int T, int BITS, bool MX, bool NEAR>
+__global__ __launch_bounds__(T) void k_prep_lut(PrepArgs a, const float *__restrict__ centroids) {
     extern __shared__ __align__(16) float prep_lds[];
-    __shared__ float red[4];
+    __shared__ float red[T / 64];
     __shared__ __align__(16) double prod[kPrepPiece];
     __shared__ float cen[16];
+    __shared__ uint32_t next;
     constexpr int cpb = 8 / BITS;
+    constexpr int kEntries = BITS == 3 ? 8 : 16;        // of a nibble that differ
     float *A = prep_lds, *B = prep_lds + prep_floats(a.dim);
     const size_t qi = blockIdx.x;
     uint8_t *dst = a.tables + qi * size_t(a.nch) * 1024;
     const int t = threadIdx.x, G = a.G;
     if (qi >= a.nq) {
-        for (int i = t; i < a.nch * 64; i += kPrepThreads) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
+        for (int i = t; i < a.nch * 64; i += T) reinterpret_cast<uint4 *>(dst)[i] = make_uint4(0, 0, 0, 0);
         if constexpr (MX)
-            for (int g = t; g < a.nch * 32; g += kPrepThreads) mx_put<BITS>(a.mx, a.nch, int(qi), g, make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0));
+            for (int g = t; g < a.nch * 32; g += T) mx_put<BITS>(a.mx, a.nch, int(qi), g, make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0));
         if constexpr (NEAR)
-            for (int g = t; g < a.near_nch * 32; g += kPrepThreads) {
+            for (int g = t; g < a.near_nch * 32; g += T) {
 #pragma unroll
                 for (int f = 0; f < cpb; ++f) a.near[near_at(int(qi), a.near_nch, cpb, g, f)] = 0;
             }
@@ -335,16 +347,19 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         return;
     }
     if (t < (1 << BITS)) cen[t] = centroids[t];
+    if (t == 0) next = 0u;
     bool late = false;
-    const float bias_corr = calibrated_row(a.q + qi * size_t(a.dim), a, A, B, prod, late);
+    const float bias_corr = calibrated_row<T>(a.q + qi * size_t(a.dim), a, A, B, prod, late);
     float *mins = B;                                   // two per group: at most a row's length
+    float *pairs = reinterpret_cast<float *>(prod);    // their sums, where they fit
+    const bool paired = G <= 2 * kPrepPiece;
     float span = 0.0f;
-    for (int g = t; g < G; g += kPrepThreads) {
+    for (int g = t; g < G; g += T) {
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             float mn = FLT_MAX, mx = -FLT_MAX;
 #pragma unroll
-            for (int nv = 0; nv < 16; ++nv) {
+            for (int nv = 0; nv < kEntries; ++nv) {
                 const float s = lut_entry<BITS>(A, cen, g * cpb, sub, nv);
                 if (s < mn) mn = s;
                 if (s > mx) mx = s;
@@ -352,13 +367,47 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
             mins[2 * g + sub] = mn;
             span = fmaxf(span, mx - mn);
         }
+        if (paired) pairs[g] = mins[2 * g] + mins[2 * g + 1];
     }
-    const float max_span = block_max_256(span, red);   // also orders the writes of mins
+    const float max_span = block_max<T>(span, red);   // also orders the writes of mins
     float scale = max_span > 0.0f ? max_span / 127.0f : 1.0f, inv_scale;
     if (scale >= FLT_MIN) inv_scale = 1.0f / scale; else { scale = 1.0f; inv_scale = 1.0f; }
     if (t == 0) {
-        float bias = 0.0f;  // sequential f32 sum over groups, inner add first (search.rs:2910)
+        // Sequential f32 sum over groups, inner add first (search.rs:2910): one lane's chain of additions, 16 clocks a group with both of them
+        // in it, so the inner ones are done before and the other waves work on the tables below meanwhile (3072 dimensions 3-bit, one query 26.4 us a launch and
+        // 18.8; 1536 2-bit 12.0 and 10.7; 768 3-bit, 300 queries 13.6 and 10.7).
+        float bias = 0.0f;
         int g = 0;
+        if (paired) {
+            // (the groups after next are on their way from LDS)
+            constexpr int kAtOnce = 32;
+            float4 m[2][kAtOnce / 4];
+            auto fetch = [&](auto set, int from) {
+#pragma unroll
+                for (int e = 0; e < kAtOnce / 4; ++e) m[decltype(set)::value][e] = reinterpret_cast<const float4 *>(pairs + from)[e];
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto add = [&](auto set) {
+#pragma unroll
+                for (int e = 0; e < kAtOnce / 4; ++e) {
+                    const float4 v = m[decltype(set)::value][e];
+                    bias += v.x;
+                    bias += v.y;
+                    bias += v.z;
+                    bias += v.w;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            const int whole = G / (2 * kAtOnce) * (2 * kAtOnce);
+            if (whole != 0) fetch(IntC<0>{}, 0);
+            for (; g < whole; g += 2 * kAtOnce) {
+                fetch(IntC<1>{}, g + kAtOnce);
+                add(IntC<0>{});
+                fetch(IntC<0>{}, min(g + 2 * kAtOnce, whole - kAtOnce));
+                add(IntC<1>{});
+            }
+            for (; g < G; ++g) bias += pairs[g];
+        }
         for (; g + 8 <= G; g += 8) {
             float4 m[4];
 #pragma unroll
@@ -373,13 +422,24 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
     float near_inv = 0.0f, unit = 0.0f, over_sum = 0.0f;
     if constexpr (NEAR) {
         float m = 0.0f;
-        for (int d = t; d < a.dim; d += kPrepThreads) m = fmaxf(m, fabsf(A[d]));
-        float u = block_max_256(m, red) / 127.0f;
+        for (int d = t; d < a.dim; d += T) m = fmaxf(m, fabsf(A[d]));
+        float u = block_max<T>(m, red) / 127.0f;
         if (!(u >= FLT_MIN)) u = 1.0f;
         near_inv = 1.0f / u;
         unit = (inv_scale * u) * a.cs;
     }
-    for (int g = t; g < a.nch * 32; g += kPrepThreads) {
+    // 64 byte-groups at a time, to whichever wave is free: the one with the chain comes late (dealt out beforehand where other
+    // workgroups fill the time: 1024 queries of 1536 dimensions 20.3 and, claimed, 21.1 us)
+    const bool dealt = gridDim.x > 512u;
+    for (uint32_t turn = 0;; ++turn) {
+        uint32_t claimed = turn * uint32_t(T) + uint32_t(t & ~63);
+        if (!dealt) {
+            if ((t & 63) == 0) claimed = atomicAdd(&next, 64u);
+            claimed = uint32_t(__builtin_amdgcn_readfirstlane(int(claimed)));
+        }
+        const int g = int(claimed) + (t & 63);
+        if (int(claimed) >= a.nch * 32) break;
+        if (g >= a.nch * 32) continue;
         uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         int8_t nw[4] = {0, 0, 0, 0};
         if (g < G) {
@@ -387,11 +447,12 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
             for (int sub = 0; sub < 2; ++sub) {
                 const float mn = mins[2 * g + sub];
 #pragma unroll
-                for (int nv = 0; nv < 16; ++nv) {
+                for (int nv = 0; nv < kEntries; ++nv) {
                     float v = roundf((lut_entry<BITS>(A, cen, g * cpb, sub, nv) - mn) * inv_scale);
                     v = v < 0.0f ? 0.0f : (v > 127.0f ? 127.0f : v);
                     w[sub * 4 + nv / 4] |= uint32_t(uint8_t(v)) << (8 * (nv & 3));
                 }
+                if constexpr (BITS == 3) { w[sub * 4 + 2] = w[sub * 4]; w[sub * 4 + 3] = w[sub * 4 + 1]; }
             }
         }
         const uint4 hi = make_uint4(w[0], w[1], w[2], w[3]), lo = make_uint4(w[4], w[5], w[6], w[7]);
@@ -416,7 +477,7 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         }
     }
     if constexpr (NEAR) {
-        for (int g = a.nch * 32 + t; g < a.near_nch * 32; g += kPrepThreads) {
+        for (int g = a.nch * 32 + t; g < a.near_nch * 32; g += T) {
 #pragma unroll
             for (int f = 0; f < cpb; ++f) a.near[near_at(int(qi), a.near_nch, cpb, g, f)] = 0;
         }
@@ -425,14 +486,16 @@ __global__ __launch_bounds__(256) void k_prep_lut(PrepArgs a, const float *__res
         __syncthreads();
         if (t == 0) {
             a.near_unit[qi] = unit;
-            a.near_err[qi] = (red[0] + red[1]) + (red[2] + red[3]);
+            float all = 0.0f;
+            for (int i = 0; i < T / 64; ++i) all += red[i];
+            a.near_err[qi] = all;
         }
     }
     if (t == 0 && a.cleared != nullptr) a.cleared[qi] = 0;
     if (t == 0 && a.stamp != nullptr && (late || qi + kStampsBefore >= a.nq)) a.stamp[qi % kStampsBefore] = wall_clock64();      // (among the last to end)
 }
 
-static_assert(size_t(2) * prep_floats(16384) * sizeof(float) + kPrepPiece * sizeof(double) + 128 <= 160 * 1024,
+static_assert(size_t(2) * prep_floats(16384) * sizeof(float) + kPrepPiece * sizeof(double) + 256 <= 160 * 1024,
               "the longest row the index accepts must fit a workgroup's LDS");
 
 hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_t nq_padded, hipStream_t s) {
@@ -445,22 +508,29 @@ hipError_t launch_prep(const PrepRequest &r, const Geometry &g, size_t nq, size_
     a.nq = nq; a.stamp = r.stamp; a.cleared = r.cleared;
     a.near_nch = near_nch(g.nch, g.bits); a.near = r.near; a.near_unit = r.near_unit; a.near_err = r.near_err; a.cs = r.near_cs; a.lv[0] = r.lv[0]; a.lv[1] = r.lv[1];
     const size_t lds = size_t(2) * prep_floats(g.dim) * sizeof(float);
-    auto launch = [&](auto kernel, auto... rest) -> hipError_t {
+    auto launch = [&](auto kernel, int threads, auto... rest) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kernel, dim3(unsigned(nq_padded)), dim3(kPrepThreads), lds, s, a, rest...);
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nq_padded)), dim3(unsigned(threads)), lds, s, a, rest...);
         return hipGetLastError();
     };
-    if (r.permute_dot) return launch(k_prep_p, r.cs, r.split);
-    auto tables = [&](auto mx) -> hipError_t {
-        constexpr bool M = decltype(mx)::value != 0;
-        return g.bits == 2 ? launch(k_prep_lut<2, M, false>, r.centroids) : g.bits == 3 ? launch(k_prep_lut<3, M, false>, r.centroids) : launch(k_prep_lut<4, M, false>, r.centroids);
+    auto all = [&](auto threads) -> hipError_t {
+        constexpr int T = decltype(threads)::value;
+        if (r.permute_dot) return launch(k_prep_p<T>, T, r.cs, r.split);
+        auto tables = [&](auto mx) -> hipError_t {
+            constexpr bool M = decltype(mx)::value != 0;
+            return g.bits == 2 ? launch(k_prep_lut<T, 2, M, false>, T, r.centroids) : g.bits == 3 ? launch(k_prep_lut<T, 3, M, false>, T, r.centroids) : launch(k_prep_lut<T, 4, M, false>, T, r.centroids);
+        };
+        return r.tables_mx != nullptr ? tables(IntC<1>{}) : tables(IntC<0>{});
     };
     if (r.near != nullptr) {
         if (a.near_nch == 0 || r.tables_mx == nullptr) return hipErrorInvalidValue;
-        return g.bits == 2 ? launch(k_prep_lut<2, true, true>, r.centroids) : launch(k_prep_lut<3, true, true>, r.centroids);
+        return g.bits == 2 ? launch(k_prep_lut<256, 2, true, true>, 256, r.centroids) : launch(k_prep_lut<256, 3, true, true>, 256, r.centroids);
     }
-    return r.tables_mx != nullptr ? tables(IntC<1>{}) : tables(IntC<0>{});
+    // A workgroup's time is latency, pass after pass with a barrier each: where queries leave the chip empty, twice the threads halve a long row's
+    // passes.  20K rows, us a search with 256 threads and 512: x 3072 3-bit, one query 73.9 and 69.1, 4-bit 55.4 and 52.1, 64 queries 57.2 and 53.9; x 1536
+    // 2-bit 43.3 and 41.3, 4-bit, 200 queries 62.9 and 62.0; x 768 38.1 and 37.9, x 512 level; 1024 threads gain nothing more.
+    return nq > 256 || g.dim < 768 ? all(IntC<256>{}) : all(IntC<512>{});
 }
 
 }  // namespace tv
