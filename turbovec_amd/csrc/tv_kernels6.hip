@@ -303,6 +303,8 @@ struct PickArgs {
 // Chunks of a query to score again (of tables: thirds), from where sharing them pays (less: 100K x 768, 64 queries, k = 10 43.3 us and, shared,
 // 44.2; 100K x 512 2-bit, one query 35.1 and 36.4; 20K x 384, one query, k = 20 31.9 and 31.1).
 constexpr size_t kSharedWork = 200;
+// Chunks (of tables: thirds) that parts have to save the busiest wave, against two barriers and the sums' way through LDS.
+constexpr double kPartsChunks = 10.0;
 // H: blocks a thread keeps in registers -- all of them, T * H at most.
 // LUT: score mode L with the u32 epilogue.
 // Scoring a block again is 70 (LUT: 200) vector instructions a chunk, on one CU for all of a query's blocks.  Where queries are too few for
@@ -310,7 +312,8 @@ constexpr size_t kSharedWork = 200;
 // the one that finds itself last ranks it.  Nobody waits for another.  us a search with one workgroup each and so: 100K x 768, one query, k = 50
 // 60.6 -> 43.5; 100K x 1536, 8 queries, k = 25 66.5 -> 54.5, one query, k = 10 55.4 -> 52.6; 778K x 1000 3-bit, 37 queries, k = 33 218 -> 216 (this
 // kernel 37 -> 25).
-template <uint32_t T, uint32_t H, bool LUT, bool SHARED>
+// PARTS: a block's chunks in parts to several waves (launch_pick; an instance of its own, as the others lost 2 to 5 % to it).
+template <uint32_t T, uint32_t H, bool LUT, bool SHARED, bool PARTS>
 __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     constexpr uint32_t W = T / 64;
     extern __shared__ __align__(16) uint8_t dyn[];
@@ -366,11 +369,10 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
     const float qs = a.qscale[qi], qb = a.qbias[qi];
     const uint32_t t0 = a.lv[0], t1 = a.lv[1], t2 = a.lv[2], t3 = a.lv[3];
     // blocks of this workgroup's share: numbers share, share + shares, ...; parts (a power of two) of a block's chunks to as many waves
-    const uint32_t mine = need > share ? (need - share + shares - 1u) / shares : 0u, log_parts = uint32_t(__builtin_ctz(a.parts));
+    const uint32_t mine = need > share ? (need - share + shares - 1u) / shares : 0u, log_parts = PARTS ? uint32_t(__builtin_ctz(a.parts)) : 0u;
     const uint32_t lds_w = uint32_t(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) uint8_t *)wts));
-    auto take = [&](uint32_t b, uint32_t row, int acc) {
+    auto take = [&](uint32_t b, uint32_t row, int acc, float vs) {
         const uint32_t slot = b * 32u + row;
-        const float vs = a.scales[slot];
         const float s = LUT ? ((float(acc) * qs) + qb) * vs : fmaf(float(acc), qs, qb) * vs;      // search.rs:1174-1177, 1519-1524
         // (A score of -infinity does not count here either, as it does not in a block's best word: rows that tie there
         // with rows of blocks that were not chosen are for the exact path to order.)
@@ -379,13 +381,14 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         const uint64_t key = sort_key(s, slot);
         if (ok && uint32_t(key >> 32) >= floor_word) list[atomicAdd(&n_list, 1u)] = key;
     };
-    if (a.parts > 1u) {
+    if constexpr (PARTS) {
         for (uint32_t i = t; i < mine * 32u; i += T) s_acc[i] = 0;
         __syncthreads();
     }
     for (uint32_t it = wv; it < mine << log_parts; it += W) {
-        const uint32_t at = it >> log_parts, part = it & (a.parts - 1u), b = blocks[at * shares + share];
-        const int first = int(uint32_t(a.nch) * part >> log_parts), end = int(uint32_t(a.nch) * (part + 1u) >> log_parts);
+        const uint32_t at = it >> log_parts, part = PARTS ? it & (a.parts - 1u) : 0u, b = blocks[at * shares + share];
+        const int first = PARTS ? int(uint32_t(a.nch) * part >> log_parts) : 0, end = PARTS ? int(uint32_t(a.nch) * (part + 1u) >> log_parts) : a.nch;
+        const float vs = a.scales[b * 32u + (lane & 31u)];      // (requested ahead of the codes)
         const uint4 *src = reinterpret_cast<const uint4 *>(a.codes) + size_t(b) * a.nch * 64 + lane;
         int acc = 0;
         constexpr int kBurst = 8;
@@ -438,13 +441,16 @@ __global__ __launch_bounds__(T) void k_pick(PickArgs a) {
         }
         acc += __shfl_xor(acc, 32);
         if (lane < 32u) {
-            if (a.parts > 1u) atomicAdd(&s_acc[at * 32u + lane], acc);
-            else take(b, lane, acc);
+            if constexpr (PARTS) atomicAdd(&s_acc[at * 32u + lane], acc);
+            else take(b, lane, acc, vs);
         }
     }
-    if (a.parts > 1u) {
+    if constexpr (PARTS) {
         __syncthreads();
-        for (uint32_t i = t; i < mine * 32u; i += T) take(blocks[(i >> 5) * shares + share], i & 31u, s_acc[i]);
+        for (uint32_t i = t; i < mine * 32u; i += T) {
+            const uint32_t b = blocks[(i >> 5) * shares + share];
+            take(b, i & 31u, s_acc[i], a.scales[b * 32u + (i & 31u)]);
+        }
     }
     if constexpr (SHARED) {
         __syncthreads();
@@ -581,20 +587,20 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     // other: parts of a block's chunks go to as many waves, as make the busiest wave's share least, where the chip is empty enough for it to
     // show.  us a search with whole blocks and so: 60K x 3072, one query, k = 1 60.1 and 51.2; 40K x 3032 3-bit, k = 4 88.8 and 82.4; 24K x 2760 2-bit, k = 2
     // 62.4 and 58.1; 16K x 1424 3-bit, 4 queries, k = 12 61.0 and 58.6; 50K x 768, 8 queries, k = 1 33.1 and 31.7; short rows level.
-    const size_t waves = small ? 4 : 16, share_blocks = (size_t(k_eff) + size_t(shares) - 1) / size_t(shares);
+    const size_t waves = 16, share_blocks = (size_t(k_eff) + size_t(shares) - 1) / size_t(shares);
     p.parts = 1;
     if (size_t(a.nq_tile) * size_t(shares) <= size_t(2) * 256) {
         auto busiest = [&](size_t parts) { return double((share_blocks * parts + waves - 1) / waves) / double(parts); };
         for (uint32_t parts = 2; parts <= 16 && int(parts) <= a.nch; parts *= 2)
-            if (busiest(parts) < 0.85 * busiest(p.parts)) p.parts = parts;
+            if (busiest(parts) < 0.85 * busiest(p.parts) && (busiest(1) - busiest(parts)) * double(a.nch) * (lut ? 3.0 : 1.0) > kPartsChunks) p.parts = parts;
     }
     auto form = [&](auto lut_, auto shared_) -> hipError_t {
         constexpr bool L = decltype(lut_)::value != 0, S = decltype(shared_)::value != 0;
-        if (a.n_blocks > 1024 * 16) return launch(k_pick<1024, 32, L, S>, 1024);
         if constexpr (!S) {
-            if (small) return launch(k_pick<256, 16, L, S>, 256);
+            if (small) return launch(k_pick<256, 16, L, S, false>, 256);
         }
-        return launch(k_pick<1024, 16, L, S>, 1024);
+        if (p.parts > 1) return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, L, S, true>, 1024) : launch(k_pick<1024, 16, L, S, true>, 1024);
+        return a.n_blocks > 1024 * 16 ? launch(k_pick<1024, 32, L, S, false>, 1024) : launch(k_pick<1024, 16, L, S, false>, 1024);
     };
     if (shares > 1) return lut ? form(IntC<1>{}, IntC<1>{}) : form(IntC<0>{}, IntC<1>{});
     return lut ? form(IntC<1>{}, IntC<0>{}) : form(IntC<0>{}, IntC<0>{});

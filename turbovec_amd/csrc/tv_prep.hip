@@ -352,7 +352,10 @@ __global__ __launch_bounds__(T) void k_prep_lut(PrepArgs a, const float *__restr
     const float bias_corr = calibrated_row<T>(a.q + qi * size_t(a.dim), a, A, B, prod, late);
     float *mins = B;                                   // two per group: at most a row's length
     float *pairs = reinterpret_cast<float *>(prod);    // their sums, where they fit
-    const bool paired = G <= 2 * kPrepPiece;
+    constexpr int kAtOnce = 16;                        // of them in registers, twice
+    const int padded = (G + 2 * kAtOnce - 1) / (2 * kAtOnce) * (2 * kAtOnce);      // (zeros behind the last, which change nothing)
+    const bool paired = padded <= 2 * kPrepPiece;
+    if (paired && t < padded - G) pairs[G + t] = 0.0f;
     float span = 0.0f;
     for (int g = t; g < G; g += T) {
 #pragma unroll
@@ -380,7 +383,6 @@ __global__ __launch_bounds__(T) void k_prep_lut(PrepArgs a, const float *__restr
         int g = 0;
         if (paired) {
             // (the groups after next are on their way from LDS)
-            constexpr int kAtOnce = 32;
             float4 m[2][kAtOnce / 4];
             auto fetch = [&](auto set, int from) {
 #pragma unroll
@@ -398,15 +400,13 @@ __global__ __launch_bounds__(T) void k_prep_lut(PrepArgs a, const float *__restr
                 }
                 __builtin_amdgcn_sched_barrier(0);
             };
-            const int whole = G / (2 * kAtOnce) * (2 * kAtOnce);
-            if (whole != 0) fetch(IntC<0>{}, 0);
-            for (; g < whole; g += 2 * kAtOnce) {
+            fetch(IntC<0>{}, 0);
+            for (; g < padded; g += 2 * kAtOnce) {
                 fetch(IntC<1>{}, g + kAtOnce);
                 add(IntC<0>{});
-                fetch(IntC<0>{}, min(g + 2 * kAtOnce, whole - kAtOnce));
+                fetch(IntC<0>{}, min(g + 2 * kAtOnce, padded - kAtOnce));
                 add(IntC<1>{});
             }
-            for (; g < G; ++g) bias += pairs[g];
         }
         for (; g + 8 <= G; g += 8) {
             float4 m[4];
