@@ -162,7 +162,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     constexpr int kM = 2 * kSC;                             // MFMAs per wave and slice: (low, high) of each chunk
     constexpr int kSlice = kM * 1024;                       // bytes: one 1 KiB B operand per MFMA
     constexpr int kSlot = KS * kSlice;                      // a ring slot: the slice of every row part
-    constexpr int kLoaders = kWideWaves / KS;               // waves that share the loading of one row part's slice
+    // Half of eight waves request the weights, twice as many pieces each, and the others wait for none of them at a hand-over (us a search with
+    // all eight and so: 10M x 1536, 1024 queries 13 370 and 13 265, 2-bit 16 110 and 15 790; 2.5M x 1152 2-bit, 150 queries 926 and 894; 4M x 768, 150
+    // queries level; a quarter of them 15 880; half of four waves 2 to 6 % more: 2M x 3072, 1024 queries 6300 and 6440.  Having the others touch the next round's
+    // blocks meanwhile, to find them in the caches: 4M x 768, 300 queries, half allowed 745 and 805).
+    constexpr bool kFewLoad = WAVES == 8 && KS == 1;
+    constexpr int kLoaders = kFewLoad ? 4 : kWideWaves / KS;  // waves that share the loading of one row part's slice
     constexpr int kPieces = kM / kLoaders;                  // direct-to-LDS loads per wave and slice ...
     constexpr int kExtra = kM % kLoaders;                   // ... plus one more in the first kExtra waves
     static_assert(KS == 1 || kExtra == 0, "the pair form deals a slice's pieces evenly");
@@ -189,6 +194,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     const uint32_t lane16 = uint32_t(lane) * 16;
     const int part = KS == 2 ? (wave & 1) : 0;              // which half of the row this wave holds
     const int loader = KS == 2 ? (wave >> 1) : wave;        // its rank among the waves loading that part's slices
+    const bool loads = !kFewLoad || wave < kLoaders;
     for (int q = tid; q < nq_pad; q += kWideThreads) {
         const bool act = q < nq;
         const float qs = act ? a.qscale[q] : 0.0f, qb = act ? a.qbias[q] : 0.0f;
@@ -269,6 +275,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     // (waves below kExtra request one piece more).
     int req_slice = 0, req_slot = 0;                        // next stream position to request
     auto request_next = [&]() {
+        if (!loads) return;
         // KS = 1: the stream is contiguous in memory.  KS = 2: a tile holds the first half of the
         // row's chunks, then the second; slice s is part s % SPT of each half of tile s / SPT.
         const uint8_t *src = KS == 1 ? a.tables + size_t(req_slice) * kSlice + size_t(loader) * 1024
@@ -285,7 +292,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     };
     auto hand_over = [&](auto younger_slices) {
         constexpr int ys = decltype(younger_slices)::value;
-        if (kExtra != 0 && wave < kExtra)
+        if (!loads) {
+        } else if (kExtra != 0 && wave < kExtra)
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ys * (kPieces + 1)) : "memory");
         else
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ys * kPieces) : "memory");
@@ -299,7 +307,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     // behind g are free: the next HO slices are requested into their slots.
     // HO > SPT: in the last slice of every HO / SPT-th tile of the stream, wherever a round of tiles ends.
     auto hand_over_group = [&]() {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (loads) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < HO; ++i) request_next();
@@ -311,7 +319,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     } else {
         // slices 0 .. 2 HO - 1 requested, the first HO whole: the state the first group hand-over expects
         for (int i = 0; i < 2 * HO; ++i) request_next();
-        if (kExtra != 0 && wave < kExtra) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HO * (kPieces + 1)) : "memory");
+        if (!loads) {
+        } else if (kExtra != 0 && wave < kExtra) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HO * (kPieces + 1)) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HO * kPieces) : "memory");
         __syncthreads();
     }
