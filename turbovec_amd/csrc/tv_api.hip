@@ -1197,7 +1197,7 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks,
 }
 // The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
 // whole tables in LDS for a few, tables streamed for up to sixteen (tiles side by side beyond) or the
-// sparse matrix instruction.
+// sparse matrix instruction; up to eight queries over few blocks with each block's chunks on several waves (tv_kernels8.hip).
 int best_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
     const int nch = a.nch;
     const size_t blocks = (a.n_blocks + a.b_step - 1) / a.b_step;
@@ -1212,6 +1212,8 @@ int best_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
         const int tiles = int((cq + tv::kLut16Queries - 1) / tv::kLut16Queries);
         const int grid = int(std::min<size_t>(size_t(tv::device_cus(ix->device)), (blocks + 7) / 8));
         TV_HIP(tv::launch_scan_lut16(a, grid, tiles, ix->stream));
+    } else if (const int parts = a.classic == 0 ? tv::lut_parts(nch, int(cq), blocks, tv::device_cus(ix->device)) : 1; parts > 1) {
+        TV_HIP(tv::launch_scan_lut_parts(a, parts, ix->device, ix->stream));
     } else {
         const int grid = int(std::min<size_t>(size_t(tv::lut_append_grid(ix->device, nch)), (blocks + 1) / 2));
         TV_HIP(tv::launch_scan_lut(a, grid, tv::kModeAppend, ix->stream));

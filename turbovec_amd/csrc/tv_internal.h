@@ -179,6 +179,11 @@ constexpr size_t kMaxPickBlocks = 32768;   // most blocks it chooses from
 constexpr size_t kPickLds = 144 * 1024;    // rows' keys and sums and the query's tables, beside its 15 KiB of fixed buffers
 bool best_serves(int nch);
 hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStream_t s);
+// The same where blocks are few: a block's chunks over `parts` waves (tv_kernels8.hip); 1 where that does not pay.
+int p4_parts(int nch, size_t n_blocks, int tiles, int cus);
+hipError_t launch_scan_p4_parts(const ScanArgs &a, bool split, int parts, int device, hipStream_t s);
+int lut_parts(int nch, int nq, size_t n_blocks, int cus);      // u8 tables, u32 epilogue, up to eight queries
+hipError_t launch_scan_lut_parts(const ScanArgs &a, int parts, int device, hipStream_t s);
 // The k_floor-th best of n score words per query as its floor, to tau_out like launch_final.
 constexpr uint32_t kMaxFloorBlocks = 8192;
 hipError_t launch_floor(const uint32_t *words, uint32_t stride, uint32_t n, int k_floor, int nq, int *tau_out, int tau_stride_q, uint64_t *stamp,

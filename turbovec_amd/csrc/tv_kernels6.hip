@@ -219,6 +219,8 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
     const uint32_t nj = a.b_step ? (a.n_blocks + a.b_step - 1) / a.b_step : 0u;
     if (a.nq_tile <= 0 || nj == 0 || !best_serves(a.nch) || a.best_out == nullptr || a.best_stride / (a.best_rows ? 32u : 1u) < nj || (a.best_rows && (a.b_step != 1 || split))) return hipErrorInvalidValue;
     const int nt = best_tiles(a.nch, nj, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device));
+    if (nt == 1)
+        if (const int parts = p4_parts(a.nch, nj, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device)); parts > 1) return launch_scan_p4_parts(a, split, parts, device, s);
     auto form = [&](auto f) -> hipError_t {
         constexpr int F = decltype(f)::value;
         return nt == 1 ? launch_best_u<1, F>(a, nj, device, s) : nt == 2 ? launch_best_u<2, F>(a, nj, device, s) : launch_best_u<4, F>(a, nj, device, s);
