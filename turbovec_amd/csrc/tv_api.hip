@@ -1197,7 +1197,7 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks,
 }
 // The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
 // whole tables in LDS for a few, tables streamed for up to sixteen (tiles side by side beyond) or the
-// sparse matrix instruction; up to eight queries over few blocks with each block's chunks on several waves (tv_kernels8.hip).
+// sparse matrix instruction; a few queries over few blocks with each block's chunks on several waves (tv_kernels8.hip).
 int best_scan_lut(tv_index *ix, tv::ScanArgs a, const Prepared &pq, size_t cq) {
     const int nch = a.nch;
     const size_t blocks = (a.n_blocks + a.b_step - 1) / a.b_step;
@@ -1250,7 +1250,8 @@ int search_direct(tv_index *ix, const float *d_queries, size_t nq, size_t k_eff,
             Prepared pq;
             const int shares = direct_rows(ix, cq, n_blocks, k_eff) ? 1 : direct_shares(ix, cq, k_eff);
             uint64_t *shared = shares > 1 ? ar.take<uint64_t>(tv::pick_shared_bytes(k_eff, cq) / sizeof(uint64_t)) : nullptr;
-            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, true, timed ? ix->d_stamps : nullptr, shared);
+            const bool parts = effective_mode(ix) == TV_SCORE_L_U32 && !lut_mx_serves(ix, cq) && tv::lut_parts(g.nch, int(cq), n_blocks, tv::device_cus(ix->device)) > 1;
+            rc = prepare_queries(ix, ar, d_queries + q0 * g.dim, cq, pq, split, false, !parts, timed ? ix->d_stamps : nullptr, shared);
             if (rc != TV_OK) return rc;
             tv::ScanArgs a;
             fill_scan_args(ix, a);

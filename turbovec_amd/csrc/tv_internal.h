@@ -182,7 +182,7 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
 // The same where blocks are few: a block's chunks over `parts` waves (tv_kernels8.hip); 1 where that does not pay.
 int p4_parts(int nch, size_t n_blocks, int tiles, int cus);
 hipError_t launch_scan_p4_parts(const ScanArgs &a, bool split, int parts, int device, hipStream_t s);
-int lut_parts(int nch, int nq, size_t n_blocks, int cus);      // u8 tables, u32 epilogue, up to eight queries
+int lut_parts(int nch, int nq, size_t n_blocks, int cus);      // u8 tables, u32 epilogue
 hipError_t launch_scan_lut_parts(const ScanArgs &a, int parts, int device, hipStream_t s);
 // The k_floor-th best of n score words per query as its floor, to tau_out like launch_final.
 constexpr uint32_t kMaxFloorBlocks = 8192;

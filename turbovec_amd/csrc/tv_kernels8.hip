@@ -171,6 +171,7 @@ hipError_t launch_scan_p4_parts(const ScanArgs &a, bool split, int parts, int de
 // waves, one block a workgroup where the CUs are as many.  Nibble tables also for one query: byte tables (k_scan_lut_bt) halve the reads,
 // but setting out 32 times as many entries as a block has look-ups takes longer than the reads they save.
 // ===========================================================================
+constexpr int kMaxLutGroups = 8;
 constexpr int kLutPartsThreads = 1024, kLutPartsWaves = kLutPartsThreads / 64;
 
 // Four words, each four entries of one query, as four words, each an entry of the four.
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(kLutPartsThreads) void k_scan_lut_parts(ScanArgs a,
     typedef typename PartsWord<QL>::type word_t;
     typedef const __attribute__((address_space(3))) word_t lds_word_t;
     extern __shared__ __align__(16) uint8_t smem[];
-    const int nch = a.nch, tid = threadIdx.x, lane = tid & 63, vi = lane & 31, h = lane >> 5;
+    const int nch = a.nch, tid = threadIdx.x, lane = tid & 63, vi = lane & 31, h = lane >> 5, q0 = int(blockIdx.y) * QL, nq = min(QL, a.nq_tile - q0);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave & (parts - 1), block = wave / parts;
     uint32_t *s_sum = reinterpret_cast<uint32_t *>(smem + size_t(nch) * 1024 * QL);      // [block][query][row]
     const uint32_t step = a.b_step, nj = (a.n_blocks + step - 1) / step, j = blockIdx.x * per + uint32_t(block);
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(kLutPartsThreads) void k_scan_lut_parts(ScanArgs a,
         uint32_t v[QL < 4 ? 4 : QL] = {};
 #pragma unroll
         for (int qq = 0; qq < QL; ++qq)
-            if (qq < a.nq_tile) v[qq] = reinterpret_cast<const uint32_t *>(a.tables + size_t(qq) * nch * 1024)[w];
+            v[qq] = reinterpret_cast<const uint32_t *>(a.tables + size_t(q0 + min(qq, nq - 1)) * nch * 1024)[w];      // (sums of queries past the last are not read)
         if constexpr (QL == 1) reinterpret_cast<uint32_t *>(smem)[w] = v[0];
         if constexpr (QL == 2) {
             reinterpret_cast<uint2 *>(smem)[w] = make_uint2(__builtin_amdgcn_perm(v[1], v[0], 0x05010400u), __builtin_amdgcn_perm(v[1], v[0], 0x07030602u));
@@ -282,43 +283,52 @@ __global__ __launch_bounds__(kLutPartsThreads) void k_scan_lut_parts(ScanArgs a,
     __syncthreads();
     if (!there) return;
     if (slot0 + 32u > a.n) mw &= (1u << (a.n - slot0)) - 1u;
-    for (int qq = part; qq < QL && qq < a.nq_tile; qq += parts) {
+    for (int qq = part; qq < nq; qq += parts) {
         // ((f32(sum) * scale) + bias) * vec_scale (turbovec/src/search.rs:1174-1177); NaN never wins
-        const float score = ((float(int(s_sum[(block * QL + qq) * 32 + vi])) * a.qscale[qq]) + a.qbias[qq]) * vs;
+        const float score = ((float(int(s_sum[(block * QL + qq) * 32 + vi])) * a.qscale[q0 + qq]) + a.qbias[q0 + qq]) * vs;
         float m = -__int_as_float(0x7f800000);
         if ((mw >> vi) & 1u) m = fmaxf(m, score);
 #pragma unroll
         for (int d = 1; d < 32; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-        if (lane == 0) a.best_out[size_t(qq) * a.best_stride + j] = live ? best_word(m) : 0u;
+        if (lane == 0) a.best_out[size_t(q0 + qq) * a.best_stride + j] = live ? best_word(m) : 0u;
     }
 }
 
-static int lut_parts_queries(int nq) { return nq <= 1 ? 1 : nq <= 2 ? 2 : nq <= 4 ? 4 : 8; }
 static size_t lut_parts_lds(int nch, int ql) { return size_t(nch) * 1024 * size_t(ql) + size_t(kLutPartsWaves / 2) * size_t(ql) * 32 * 4; }
+// Queries of a workgroup: all of up to eight, as far as their tables fit.
+static int lut_parts_queries(int nch, int nq) {
+    int ql = nq <= 1 ? 1 : nq <= 2 ? 2 : nq <= 4 ? 4 : 8;
+    while (ql > 1 && lut_parts_lds(nch, ql) > 160 * 1024) ql /= 2;
+    return ql;
+}
 
 // As many waves as are resident -- up to two queries, whose look-ups the LDS bounds: more queries add up on the vector ALU what k_scan_lut adds on the
 // matrix unit, and pay only where the chip is rather empty (us one wave a block and parts on four times as many waves: 8 queries 99K x 960 2-bit 42 and
-// 51, 56K x 728 3-bit 49 and 52; 4 queries 67K x 1024 3-bit, filtered, 44 and 52).
+// 51, 56K x 728 3-bit 49 and 52; 4 queries 67K x 1024 3-bit, filtered, 44 and 52).  Queries beyond a workgroup's go to more of them, side by
+// side, where there is room by the same count; k_scan_lut16 takes sixteen at a time, but wants its tables in another order, 5 to 7 us a launch
+// more (us so and with parts: 500 x 2880 2-bit, 16 queries 49 and 36; 5K x 1024 2-bit, 16 43 and 34; 1.5K x 448 3-bit, 47 38 and 31; 5K x 3072 2-bit, 5 68 and 51;
+// 25K x 3072 3-bit, 3 80 and 64; on twice the waves 22K x 1024 3-bit, 22 57 and 74, but 24K x 384 2-bit, 15 44 and 39: rows up to three chunks have twice).
 int lut_parts(int nch, int nq, size_t n_blocks, int cus) {
-    const size_t lds = lut_parts_lds(nch, lut_parts_queries(nq));
-    if (nq > 8 || lds > 160 * 1024) return 1;
-    const size_t waves = nq > 4 ? kLutPartsWaves / 2 : nq > 2 || lds > 80 * 1024 ? kLutPartsWaves : 2 * kLutPartsWaves;
-    return parts_of(n_blocks, nch, size_t(cus) * waves, 1, kLutPartsWaves);
+    const int ql = lut_parts_queries(nch, nq), groups = (nq + ql - 1) / ql;
+    const size_t lds = lut_parts_lds(nch, ql);
+    if (groups > kMaxLutGroups || lds > 160 * 1024) return 1;
+    const size_t waves = ql > 4 ? kLutPartsWaves / (nch <= 3 ? 1 : 2) : ql > 2 || lds > 80 * 1024 ? kLutPartsWaves : 2 * kLutPartsWaves;
+    return parts_of(n_blocks * size_t(groups), nch, size_t(cus) * waves, 1, kLutPartsWaves);
 }
 
 hipError_t launch_scan_lut_parts(const ScanArgs &a, int parts, int device, hipStream_t s) {
     const uint32_t nj = a.b_step ? (a.n_blocks + a.b_step - 1) / a.b_step : 0u;
-    const int ql = lut_parts_queries(a.nq_tile);
+    const int ql = lut_parts_queries(a.nch, a.nq_tile), groups = (a.nq_tile + ql - 1) / ql;
     const size_t lds = lut_parts_lds(a.nch, ql);
-    if (a.nq_tile <= 0 || a.nq_tile > 8 || nj == 0 || a.best_out == nullptr || a.best_stride < nj || a.classic != 0 || lds > 160 * 1024 ||
+    if (a.nq_tile <= 0 || groups > kMaxLutGroups || nj == 0 || a.best_out == nullptr || a.best_stride < nj || a.classic != 0 || lds > 160 * 1024 ||
         (parts != 2 && parts != 4 && parts != 8 && parts != 16))
         return hipErrorInvalidValue;
-    const uint32_t per = blocks_of(nj, device_cus(device), kLutPartsWaves, parts);
+    const uint32_t per = blocks_of(size_t(nj) * groups, device_cus(device), kLutPartsWaves, parts);
     auto launch = [&](auto q) -> hipError_t {
         constexpr int Q = decltype(q)::value;
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_lut_parts<Q>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_scan_lut_parts<Q>), dim3((nj + per - 1) / per), dim3(kLutPartsThreads), lds, s, a, parts, per);
+        hipLaunchKernelGGL((k_scan_lut_parts<Q>), dim3((nj + per - 1) / per, groups), dim3(kLutPartsThreads), lds, s, a, parts, per);
         return hipGetLastError();
     };
     return ql == 1 ? launch(IntC<1>{}) : ql == 2 ? launch(IntC<2>{}) : ql == 4 ? launch(IntC<4>{}) : launch(IntC<8>{});
