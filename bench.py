@@ -157,10 +157,19 @@ def sparse_roofline(launch_s, queries, n, dim, bits):
             "stored_ops_per_launch": ops}
 
 
+def two_step_roofline(scan_s, queries, n, dim):
+    """Roofline of the two-step table scan, all stages of it: an int8 product of every query and row (k_scan_p4_wide over 2- or
+    3-bit levels) says which rows may reach the floor, and k_near_rescore sums the tables of those.  The products alone
+    are counted, against the dense int8 peak."""
+    ops = 2.0 * queries * n * dim
+    return {"bound": "mfma", "achieved": ops / scan_s / 1e12, "peak": 5000.0, "unit": "TFLOP/s", "frac": ops / scan_s / 1e12 / 5000.0,
+            "kernel": "k_scan_p4_wide, k_near_rescore", "traffic": None}
+
+
 def config3_extra(T, torch, build_index, run, args):
     """Configuration 3 beside the headline: 10M x 1536 2-bit, k=100 (u8 LUT, u32 epilogue), batches 1
     and 1024, each with the roofline of its scan launch: HBM for the single query (algorithmic bytes = codes +
-    row scales), the sparse matrix instruction for the batch."""
+    row scales), the int8 matrix unit for the batch."""
     n, dim, bits, k = 10_000_000, 1536, 2, 100
     ix = build_index(dim, bits, n)
     alg = ((n + 31) // 32) * (dim // 4) * 32 + 4 * n
@@ -169,12 +178,18 @@ def config3_extra(T, torch, build_index, run, args):
     for nq, steps in ((1024, max(3, args.steps // 2)), (1, max(args.steps, 15))):
         dt, scan_ms, launches, q_full = run(nq, steps, 1, ix=ix, k=k, dim=dim)
         launch_s = scan_ms * 1e-3 / max(launches, 1)
-        # byte tables serve single queries; a batch is one launch of the sparse matrix-unit scan
+        # byte tables serve single queries; a batch is one launch of the sparse matrix-unit scan, or stages of
+        # two launches (then the scan is all of them)
+        two_step = q_full > 16 and launches > steps
+        if two_step:
+            launch_s = scan_ms * 1e-3 / steps
         kern = "k_scan_lut_bt" if q_full == 1 else "k_scan_lut_mx" if q_full > 16 else "k_scan_lut16" if q_full > 8 else "k_scan_lut"
         roofline = {"bound": "hbm", "achieved": alg / launch_s / 1e9, "peak": 8000.0,
                     "unit": "GB/s", "frac": alg / launch_s / 1e9 / 8000.0,
                     "traffic": MEASURED_TRAFFIC.get((kern, n, dim, bits)), "kernel": kern}
-        if kern == "k_scan_lut_mx":
+        if two_step:
+            roofline = two_step_roofline(launch_s, min(nq, q_full), n, dim)
+        elif kern == "k_scan_lut_mx":
             roofline = sparse_roofline(launch_s, min(nq, q_full), n, dim, bits)
         res[f"batch{nq}"] = {"queries_per_s": nq * steps / dt, "ms_per_step": dt / steps * 1e3,
                              "queries_per_launch": q_full, "scan_launch_ms": launch_s * 1e3, "roofline": roofline}
