@@ -193,10 +193,12 @@ static hipError_t launch_best_one(const ScanArgs &a, uint32_t nj, int device, hi
     const size_t lds = size_t(NT) * a.nch * 2048;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_scan_p4_best<NT, U, FORM, ONE>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
-    // a workgroup keeps its weights for all its blocks: about as many workgroups as are resident
+    // A workgroup keeps its weights for all its blocks: as many workgroups as are resident, and none more, which would
+    // start when the others end (us a search with 258 or 260 for 256 places and so: 194K x 560, 696 queries 241 and 173, 350K x 512, 300
+    // 184 and 134, 1M x 256, 600 464 and 314; 513 for 512: 333K x 2424, 67 280 and 249, 50K x 3072, 96 106 and 91).
     const unsigned per_cu = unsigned(std::min<size_t>(NT <= 2 ? 2 : 1, 160 * 1024 / lds));
     const unsigned resident = unsigned(device_cus(device)) * std::max(1u, per_cu);
-    const unsigned x = std::max(1u, std::min((nj + kBestWaves - 1) / kBestWaves, (resident + groups_y - 1) / groups_y));
+    const unsigned x = std::max(1u, std::min((nj + kBestWaves - 1) / kBestWaves, resident / unsigned(groups_y)));
     hipLaunchKernelGGL((k_scan_p4_best<NT, U, FORM, ONE>), dim3(x, groups_y), dim3(kBestThreads), lds, s, a);
     return hipGetLastError();
 }
