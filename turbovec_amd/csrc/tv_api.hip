@@ -1149,11 +1149,16 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff)
 //  - One tile of queries: a full scan of so many bytes that two more launches no longer show.  1.04M rows x 128
 //    51 and 63, x 512 80 and 92, x 640 99 and 101, x 768 113 and 115, x 1024 140 and 140; 600K x 1024 95 and 105, x 1536 132 and 131.
 //  - More tiles on k_scan_p4_best, which decodes a block once per tile group: won up to a number of (block,
-//    tile, chunk) triples that depends on the kernel it replaces -- rows of less than 12 chunks (600K x 640, 1000 queries,
-//    6e6 triples: 563 and 677; 1.04M x 512, 8.3e6: 929 and 829; 1.04M x 128, 2.1e6: 400 and 781), rows whose tiles
+//    tile, chunk) triples that depends on the kernel it replaces -- rows whose tiles
 //    stay in LDS and that this kernel too keeps two tiles of (1.04M x 1024, 64 queries, 1.04e6: 172 and 193) or only one (100K x 1536,
 //    100 queries, 3e5: 100 and 99; 600K x 1536, 64 queries, 9e5: 211 and 185), rows whose tiles are streamed (260K x 3072, 100 queries, 1.6e6:
 //    308 and 528; 500K, 3e6: 489 and 437).
+//  - Rows of 3 to 11 chunks, more than four tiles: the sample's floors cost some 60 us and the all-queries kernel then decodes a block once, not once a
+//    tile group: won up to a number of blocks that falls with the groups and with the tiles the last one lacks (a missing one is level), fitted to 150 queries 450K x 384 90 and 93,
+//    700K x 384 123 and 114; 244 queries 446K x 640 127 and 152, 716K x 640 177 and 206, 1.04M x 448 198 and 177; 300 queries 300K x 256 84 and 103, 450K x 384 132
+//    and 133, 700K x 384 191 and 162; 512 queries 600K x 576 277 and 279, 800K x 576 379 and 343; 600 queries 700K x 512 347 and 308; 1000 queries 200K x 512 196
+//    and 201, 450K x 512 354 and 322, 700K x 384 432 and 363.  Of one or two chunks: 1M x 128, 300 queries 128 and 135, 1000 296 and 283.  Up to four tiles the other
+//    kernel is k_scan_p4_multi: 100 queries 1M x 256 86 and 98, x 640 143 and 137.
 //  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about 700K
 //    rows (1000 queries: 600K x 768 570 and 621, x 1536 972 and 999; 1.04M x 768 935 and 895, x 1536 1611 and 1523),
 //    earlier where many rows are scored again (500K x 768, k = 45: 556 and 540).
@@ -1192,7 +1197,11 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks,
         (k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds)) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
-    if (nch < 12) return triples <= 6000000;
+    if (nch <= 2 || (nch < 12 && tiles <= 4)) return true;
+    if (nch < 12) {
+        const double groups = double((tiles + 3) / 4), full = std::min(1.0, double(tiles + 1) / (4.0 * groups));
+        return double(n_blocks) <= (4000.0 + 50000.0 / groups) * full * std::sqrt(full) * (nch == 3 ? 1.5 : 1.0);
+    }
     return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 16 ? 1050000 : 250000) || n_blocks <= 512;
 }
 // The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
