@@ -1066,7 +1066,9 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     const size_t group_rows = size_t(tv::kNearBlocks) * ix->geo.block_bytes(), group_masks = tiles * tv::kQTile * tv::kNearBlocks * 4;
     const size_t most = std::max(round, kNearBytes / (group_rows + group_masks) / round * round);
     const size_t per_group = size_t(tv::near_rescore_queries(nch)), query_groups = (cq + per_group - 1) / per_group;
-    p.splits = uint32_t(std::clamp<size_t>(std::max((6 * k_floor + tv::kSegCap - 1) / tv::kSegCap, (512 + query_groups - 1) / query_groups), 4, 16));
+    // workgroups of the rescore: up to two a CU at once, and none that wait for a place among those (us a search rounded up and so, all 2-bit: 4M x 256, 800
+    // queries 1338 and 1254, 3M x 384, 500 944 and 871, 2M x 768, 300 842 and 794, 2M x 1536, 500 1926 and 1906; the one the other way 1.5M x 1536, 200, k = 50, 975 and 990)
+    p.splits = uint32_t(std::clamp<size_t>(std::max((6 * k_floor + tv::kSegCap - 1) / tv::kSegCap, 512 / query_groups), 4, 16));
     p.guessed = ix->near_sure_left == 0;
     const size_t sample = std::min<size_t>({p.guessed ? std::max<size_t>(kNearSample, size_t(tv::mx_round_blocks(ix->device, cq))) : std::max({4 * kNearSample, 8 * k_floor, round * tv::kNearBlocks / 2}),
                                             size_t(tv::kMaxFloorBlocks), n_blocks / 4});
