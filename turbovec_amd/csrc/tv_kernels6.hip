@@ -177,12 +177,13 @@ __global__ __launch_bounds__(kBestThreads, NT <= 2 ? 4 : 2) void k_scan_p4_best(
 }
 
 // Query tiles per workgroup: as many as the LDS holds beside another workgroup's -- four at most -- but no
-// more than leave the chip with a workgroup per CU.
+// more than leave the chip with a workgroup per CU.  Three where that makes no more groups (us a search with four and three: 3 tiles
+// 310K x 384 53.5 and 51.3; 5 tiles 537K x 352 110 and 94, 35K x 640 43.2 and 41.4; 9 tiles 269K x 640 133 and 116, 152K x 384 68 and 63).
 static int best_tiles(int nch, size_t n_blocks, int tiles, int cus) {
-    int nt = tiles >= 4 ? 4 : tiles == 3 ? 4 : tiles;
-    while (nt > 1 && size_t(nt) * nch * 2048 > 80 * 1024) nt /= 2;
+    int nt = tiles == 3 || tiles == 5 || tiles == 6 || tiles == 9 ? 3 : std::min(tiles, 4);
+    while (nt > 1 && size_t(nt) * nch * 2048 > 80 * 1024) nt = nt == 3 ? 2 : nt / 2;
     const size_t groups = (n_blocks + kBestWaves - 1) / kBestWaves;
-    while (nt > 1 && groups * size_t((tiles + nt - 1) / nt) < size_t(cus)) nt /= 2;
+    while (nt > 1 && groups * size_t((tiles + nt - 1) / nt) < size_t(cus)) nt = nt == 3 ? 2 : nt / 2;
     return nt;
 }
 bool best_serves(int nch) { return size_t(nch) * 2048 <= 160 * 1024; }
@@ -225,7 +226,7 @@ hipError_t launch_scan_p4_best(const ScanArgs &a, bool split, int device, hipStr
         if (const int parts = p4_parts(a.nch, nj, (a.nq_tile + kQTile - 1) / kQTile, device_cus(device)); parts > 1) return launch_scan_p4_parts(a, split, parts, device, s);
     auto form = [&](auto f) -> hipError_t {
         constexpr int F = decltype(f)::value;
-        return nt == 1 ? launch_best_u<1, F>(a, nj, device, s) : nt == 2 ? launch_best_u<2, F>(a, nj, device, s) : launch_best_u<4, F>(a, nj, device, s);
+        return nt == 1 ? launch_best_u<1, F>(a, nj, device, s) : nt == 2 ? launch_best_u<2, F>(a, nj, device, s) : nt == 3 ? launch_best_u<3, F>(a, nj, device, s) : launch_best_u<4, F>(a, nj, device, s);
     };
     return a.best_rows ? form(IntC<kBestRows>{}) : split ? form(IntC<kBestSplit>{}) : form(IntC<kBestPlane>{});
 }
