@@ -308,7 +308,7 @@ struct PickArgs {
 // Chunks of a query to score again (of tables: thirds), from where sharing them pays (less: 100K x 768, 64 queries, k = 10 43.3 us and, shared,
 // 44.2; 100K x 512 2-bit, one query 35.1 and 36.4; 20K x 384, one query, k = 20 31.9 and 31.1).
 constexpr size_t kSharedWork = 200;
-// Chunks (of tables: thirds) that parts have to save the busiest wave, against two barriers and the sums' way through LDS.
+// Chunks (of tables: halves) that parts have to save the busiest wave, against two barriers and the sums' way through LDS.
 constexpr double kPartsChunks = 10.0;
 // H: blocks a thread keeps in registers -- all of them, T * H at most.
 // LUT: score mode L with the u32 epilogue.
@@ -591,13 +591,14 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     // A block to a wave leaves most of sixteen waves without one where results are few, and the others with a row's chunks one after the
     // other: parts of a block's chunks go to as many waves, as make the busiest wave's share least, where the chip is empty enough for it to
     // show.  us a search with whole blocks and so: 60K x 3072, one query, k = 1 60.1 and 51.2; 40K x 3032 3-bit, k = 4 88.8 and 82.4; 24K x 2760 2-bit, k = 2
-    // 62.4 and 58.1; 16K x 1424 3-bit, 4 queries, k = 12 61.0 and 58.6; 50K x 768, 8 queries, k = 1 33.1 and 31.7; short rows level.
+    // 62.4 and 58.1; 16K x 1424 3-bit, 4 queries, k = 12 61.0 and 58.6; 50K x 768, 8 queries, k = 1 33.1 and 31.7; short rows level (or worse: 95K
+    // x 272 3-bit, 100 queries, k = 33, in two workgroups each, 59.9 and 61.1).
     const size_t waves = 16, share_blocks = (size_t(k_eff) + size_t(shares) - 1) / size_t(shares);
     p.parts = 1;
     if (size_t(a.nq_tile) * size_t(shares) <= size_t(2) * 256) {
         auto busiest = [&](size_t parts) { return double((share_blocks * parts + waves - 1) / waves) / double(parts); };
         for (uint32_t parts = 2; parts <= 16 && int(parts) <= a.nch; parts *= 2)
-            if (busiest(parts) < 0.85 * busiest(p.parts) && (busiest(1) - busiest(parts)) * double(a.nch) * (lut ? 3.0 : 1.0) > kPartsChunks) p.parts = parts;
+            if (busiest(parts) < 0.85 * busiest(p.parts) && (busiest(1) - busiest(parts)) * double(a.nch) * (lut ? 2.0 : 1.0) > kPartsChunks) p.parts = parts;
     }
     auto form = [&](auto lut_, auto shared_) -> hipError_t {
         constexpr bool L = decltype(lut_)::value != 0, S = decltype(shared_)::value != 0;
