@@ -1182,8 +1182,10 @@ bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blo
     if (nq == 1) return rescored <= (n_blocks > 64 ? (shares > 1 ? kSharedMost : 400u) : nch <= 16 ? 120u : 0u);
     if (nq <= size_t(tv::kLut16Queries)) return rescored <= (n_blocks >= 4096 ? 1200u : 720u);
     // (the two-step scan, whose stages cost some 80 us at least, from so many triples: 560K x 1536, 287 queries, 1.9e6 875 and 546; 180K x 1024,
-    // 389, 6e5 299 and 239; 720K x 768, 188, 8e5 369 and 352; but 280K x 664, 155, 2.6e5 170 and 193; longer rows: 140K x 2048, 621, 1.4e6 610 and 642)
-    if (!masked && ix->geo.bits == 2 && nch <= 12 && tiles >= 3 && n_blocks * tiles * nch >= 600000 && near_takes(ix, nq, k_eff, n_blocks)) return false;
+    // 389, 6e5 299 and 239; 720K x 768, 188, 8e5 369 and 352; 530K x 384, 273, 4.5e5 296 and
+    // 262, 130K x 512, 870, 4.5e5 258 and 207, 120K x 1024, 481, 4.8e5 270 and 241, 460K x 1536, 87, 5.2e5 308 and 288, 98K x 1536, 472, 5.5e5 284 and 294, 99K x 768, 890, 5.2e5 264 and 292; but 116K x 1536, 298, 4.4e5 241 and 264, 650K x 384, 168,
+    // 3.7e5 222 and 249, 280K x 664, 155, 2.6e5 170 and 193; longer rows: 140K x 2048, 621, 1.4e6 610 and 642)
+    if (!masked && ix->geo.bits == 2 && nch <= 12 && tiles >= 3 && n_blocks * tiles * nch >= (nch <= 8 && n_blocks >= 3500 ? 450000u : 600000u) && near_takes(ix, nq, k_eff, n_blocks)) return false;
     return n_blocks * tiles <= 200000 && rescored <= std::max<size_t>(tiles <= 4 ? 1200u : 600u, 600u * shares);
 }
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks, bool masked) {
