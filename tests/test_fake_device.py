@@ -428,3 +428,25 @@ for rows, gathers in ((np.arange(n) // 2 % 10 == 0, True), ((np.arange(n) > 30_0
     assert ix.gathered_searches()[0] == before + 2 * gathers and counts.value == 1
     counts.value = 0
 ''')
+
+
+# (a 2-bit batch takes the matrix-unit scan over so few blocks from 385 queries on, a 3-bit one from 49)
+@pytest.mark.parametrize("bits,nq", [(2, 400), (3, 65)])
+def test_the_two_step_scan_of_a_few_rows(fake, bits, nq):
+    """Asked for by the test hook over fewer blocks than a sample takes one of: the other scans."""
+    fake(f'''
+for rows in (1, 31, 96, 97, 128, 129):
+    ix = T.NativeIndex(64, {bits})
+    ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
+    ix.set_path(128)
+    ix.sampling_plan({nq}, 3)
+    ix.search(np.ones(({nq}, 64), np.float32), 3)
+    assert ix.last_scan_ms()[1] == 1
+    ix.close()
+ix = T.NativeIndex(64, {bits})           # a filter's few rows, gathered
+ix.append_rows(np.zeros((40_000, ix.n_byte_groups), np.uint8), np.zeros(40_000, np.float32))
+ix.set_path(128 + 64)
+ix.search(np.ones(({nq}, 64), np.float32), 3, mask_words=T.pack_mask(np.arange(40_000) % 1000 == 7)[0])
+assert ix.gathered_searches()[0] == 1
+ix.close()
+''')

@@ -203,3 +203,19 @@ def test_queries_that_are_not_finite():
     good = [r for r in range(70) if r not in (5, 17, 40, 41)]
     assert np.array_equal(i[good], i1[good]) and bits_equal(s[good], s1[good])
     ix.close()
+
+
+@pytest.mark.parametrize("bits,nq", [(2, 400), (3, 65)])
+def test_fewer_blocks_than_a_sample(bits, nq):
+    """The hook asks for two steps where there is no sample to take a floor from: the other scans."""
+    from turbovec_amd import _lib as T
+    dim = 64
+    gen = torch.Generator(device="cuda:0").manual_seed(bits)
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    for n in (1, 31, 96, 97, 129):
+        ix = T.NativeIndex(dim, bits)
+        v = torch.randn(n, dim, device="cuda:0", generator=gen)
+        torch.cuda.synchronize()
+        ix.add_dev(v.data_ptr(), n)
+        check(ix, q, (1, 10), always=False)
+        ix.close()

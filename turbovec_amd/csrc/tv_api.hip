@@ -1055,6 +1055,7 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     const size_t round = size_t(plan.grid_near) * size_t(tv::near_blocks_per_workgroup(nch, bits)) / tv::kNearBlocks;      // groups
     const size_t total = (n_blocks + tv::kNearBlocks - 1) / tv::kNearBlocks, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
     if (ix->no_direct && n_blocks <= 16384) return p;
+    if (n_blocks < 4) return p;      // (a sample is a quarter of the blocks at most, and one at least)
     if (!ix->force_near && (cq < kNearMinQueries || n_blocks * tiles * size_t(nch) < (bits == 2 ? kNearMinWork2 : kNearMinWork3))) return p;
     // how far above the int8 product a table sum may lie, in standard deviations of the score, about (measured at 128 to 3072 dimensions),
     // and the share of rows that close to the last result's score, were scores normal
