@@ -450,3 +450,25 @@ ix.search(np.ones(({nq}, 64), np.float32), 3, mask_words=T.pack_mask(np.arange(4
 assert ix.gathered_searches()[0] == 1
 ix.close()
 ''')
+
+
+@pytest.mark.parametrize("dim,bits,nq", [(1536, 2, 372), (1024, 2, 416), (640, 2, 424)])
+def test_fixed_scratch_is_not_charged_for_the_two_step_scan(fake, dim, bits, nq):
+    """Batches on lent scratch, which never go in two steps: the largest that fit on the matrix-unit scan are all served in one launch."""
+    fake(f'''
+ix = T.NativeIndex({dim}, {bits})
+ix.append_rows(np.zeros((20_000, ix.n_byte_groups), np.uint8), np.zeros(20_000, np.float32))
+def served(nq):
+    q, s, i = np.ones((nq, {dim}), np.float32), np.zeros((nq, 10), np.float32), np.zeros((nq, 10), np.int64)
+    ix.search_dev_noalloc(q.ctypes.data, nq, 10, s.ctypes.data, i.ctypes.data)
+    return ix.queries_per_launch()
+assert served({nq}) == {nq}
+try:
+    served({nq + 1})
+    raise SystemExit("one more was searched")
+except T.TurbovecHipError as e:
+    assert e.status == T.ERR_BAD_ARGUMENT
+ix.set_path(128)                         # the hook does not change what fits
+assert served({nq}) == {nq}
+ix.close()
+''')

@@ -646,10 +646,7 @@ size_t prepare_bytes(const tv_index *ix, size_t nq) {
     const size_t nq_pad = round_up(nq, tv::kQTile);
     size_t b = 2 * round_up(nq * g.dim * 4, 256) + 3 * round_up(nq_pad * 4, 256);
     b += round_up(nq_pad * size_t(g.nch) * 1024, 256) + 4096;
-    if (lut_mx_serves(ix, nq)) {
-        b += round_up(tv::mx_table_bytes(g.nch, g.bits, nq), 256);
-        if (g.bits != 4) b += round_up(nq_pad * size_t(tv::near_nch(g.nch, g.bits)) * 32 * size_t(8 / g.bits), 256) + 2 * round_up(nq_pad * 4, 256);     // (the two-step scan's)
-    }
+    if (lut_mx_serves(ix, nq)) b += round_up(tv::mx_table_bytes(g.nch, g.bits, nq), 256);
     else if (lut16_serves(ix)) b += round_up(tv::lut16_table_bytes(g.nch, nq), 256);
     return b;
 }
@@ -686,6 +683,19 @@ int ensure_events(tv_index *ix) {
     }
     ix->events_ready = true;
     return TV_OK;
+}
+
+// The two-step table scan: two tiles of queries are level at best, three ahead (us a search without and so: 2.3M x 384 2-bit, 47 queries 240 and 299; 6.2M x 768, 59
+// 975 and 901; 4.1M x 384, 64 397 and 378; 7.1M x 456, 84 1431 and 826; 2.8M x 1360, 75 1530 and 943; 2.4M x 512 3-bit, 76 587
+// and 480, 752 dimensions, 52 450 and 532; 1M x 1128, 86 557 and 485; 10M x 1536, 1024 45 900 and 15 900).
+constexpr size_t kNearMinQueries = 65;
+// Bytes of the operands it takes beside the tables; 0 where a chunk of so many queries cannot go that way, as on scratch of a fixed
+// size, whose limits they would lower.
+size_t near_bytes(const tv_index *ix, size_t cq) {
+    const tv::Geometry &g = ix->geo;
+    if (ix->ws_fixed || (!ix->force_near && cq < kNearMinQueries) || !lut_mx_serves(ix, cq) || tv::near_chunks(g.nch, g.bits) == 0) return 0;
+    const size_t nq_pad = round_up(cq, tv::kQTile);
+    return round_up(nq_pad * size_t(tv::near_nch(g.nch, g.bits)) * 32 * size_t(8 / g.bits), 256) + 2 * round_up(nq_pad * 4, 256);
 }
 
 // Workspace bytes one chunk of cq queries needs on the exact path (search_robust) ...
@@ -738,7 +748,7 @@ SampledPlan sampled_plan(const tv_index *ix, size_t cq) {
     // (a query keeps one candidate segment per workgroup of the launches that serve it: every launch
     // of a chunk the tile-group kernels serve is one of theirs, and their grid is not the single-tile scan's)
     if (p.nt_batched > 0 && !p.wide) p.seg_stride = size_t(tv::batched_grid_blocks(ix->device, g.nch));
-    p.need = prepare_bytes(ix, cq) + round_up(p.n_tiles * tv::kQTile * 4, 256) +
+    p.need = prepare_bytes(ix, cq) + near_bytes(ix, cq) + round_up(p.n_tiles * tv::kQTile * 4, 256) +
              round_up(p.cq_pad * p.seg_stride * tv::kSegCap * 8, 256) + round_up(p.cq_pad * p.seg_stride * 4, 256) +
              round_up(p.cq_pad * 4, 256) + 65536;
     return p;
@@ -1012,10 +1022,6 @@ SamplingSteps level_strides(const tv_index *ix, const SampledPlan &plan, size_t 
 constexpr size_t kNearBytes = size_t(1) << 30;
 constexpr size_t kNearSample = 512;      // blocks
 constexpr int kNearMaxStages = 32;
-// Two tiles of queries are level at best, three ahead (us a search without and so: 2.3M x 384 2-bit, 47 queries 240 and 299; 6.2M x 768, 59
-// 975 and 901; 4.1M x 384, 64 397 and 378; 7.1M x 456, 84 1431 and 826; 2.8M x 1360, 75 1530 and 943; 2.4M x 512 3-bit, 76 587
-// and 480, 752 dimensions, 52 450 and 532; 1M x 1128, 86 557 and 485; 10M x 1536, 1024 45 900 and 15 900).
-constexpr size_t kNearMinQueries = 65;
 // ... and so many (block, query tile, chunk) triples of 2-bit codes (390K x 144, 636 queries, 480 000 triples, 459 and 220; 87K x 1536, 223,
 // k = 86, 230 000: 271 and 242), and of 3-bit ones, whose one-hot products are half as many (430K x 256, 349 queries, 590 000: 225 and 282; 890K x 280, 129,
 // 700 000: 272 and 284; 1.2M x 248, 319, 1.5e6: 705 and 329).
@@ -1050,13 +1056,13 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     NearPlan p;
     const size_t k_floor = std::max<size_t>(k_eff, 16);
     const int nch = ix->geo.nch, bits = ix->geo.bits;
-    if (!plan.lut_mx || ix->ws_fixed || ix->no_wide || ix->no_batched || ix->row_ladder_left != 0 || ix->allowed.in_place || k_floor > size_t(tv::kMaxPickK)) return p;
-    if (tv::near_chunks(nch, bits) == 0 || tv::near_rescore_queries(nch) == 0 || ix->rows().n >= (size_t(1) << 31)) return p;
+    if (near_bytes(ix, cq) == 0 || ix->no_wide || ix->no_batched || ix->row_ladder_left != 0 || ix->allowed.in_place || k_floor > size_t(tv::kMaxPickK)) return p;
+    if (tv::near_rescore_queries(nch) == 0 || ix->rows().n >= (size_t(1) << 31)) return p;
     const size_t round = size_t(plan.grid_near) * size_t(tv::near_blocks_per_workgroup(nch, bits)) / tv::kNearBlocks;      // groups
     const size_t total = (n_blocks + tv::kNearBlocks - 1) / tv::kNearBlocks, tiles = (cq + tv::kQTile - 1) / tv::kQTile;
     if (ix->no_direct && n_blocks <= 16384) return p;
     if (n_blocks < 4) return p;      // (a sample is a quarter of the blocks at most, and one at least)
-    if (!ix->force_near && (cq < kNearMinQueries || n_blocks * tiles * size_t(nch) < (bits == 2 ? kNearMinWork2 : kNearMinWork3))) return p;
+    if (!ix->force_near && n_blocks * tiles * size_t(nch) < (bits == 2 ? kNearMinWork2 : kNearMinWork3)) return p;
     // how far above the int8 product a table sum may lie, in standard deviations of the score, about (measured at 128 to 3072 dimensions),
     // and the share of rows that close to the last result's score, were scores normal
     const double margin = (bits == 2 ? 0.028 : 0.045) * std::sqrt(double(ix->geo.dim));
@@ -2778,6 +2784,7 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
         const size_t exact = robust_need(ix, cq, k_eff);
         return k_eff <= size_t(tv::kMaxSampledK) && !ix->force_robust ? std::max(exact, sampled_need_worst(ix, nq)) : exact;
     };
+    ix->ws_fixed = true;      // (what is carved depends on it)
     size_t need = carve();
     if (need > kScratchBytes) {
         ix->no_lut_mx = true;
@@ -2785,6 +2792,7 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     }
     if (need > kScratchBytes) {
         ix->no_lut_mx = false;
+        ix->ws_fixed = false;
         g_last_error = "tv_search_dev_noalloc: " + std::to_string(nq) + " queries, k=" + std::to_string(k) + " over " +
                        std::to_string(ix->n) + " rows may need " + std::to_string(need) +
                        " bytes of scratch; the fixed buffer holds " + std::to_string(kScratchBytes) +
@@ -2796,7 +2804,6 @@ int tv_search_dev_noalloc(tv_index *ix, const float *d_queries, size_t nq, size_
     const size_t own_bytes = ix->ws_bytes;
     ix->ws = ix->scratch;
     ix->ws_bytes = kScratchBytes;
-    ix->ws_fixed = true;
     const int rc = search_device(ix, d_queries, nq, k, d_mask_words, n_allowed, kLiveUnknown, d_out_scores, d_out_indices, out_k_eff);
     ix->ws = own_ws;
     ix->ws_bytes = own_bytes;
