@@ -472,3 +472,40 @@ ix.set_path(128)                         # the hook does not change what fits
 assert served({nq}) == {nq}
 ix.close()
 ''')
+
+
+STAGES = '''
+def batch_index(rows):
+    """An index whose batches of 1024 queries go in two steps, with a stage of about 20 KB for every 256 rows."""
+    ix = T.NativeIndex(8, 2)
+    ix.append_rows(np.zeros((rows, 2), np.uint8), np.zeros(rows, np.float32))
+    return ix
+queries = np.ones((1024, 8), np.float32)
+def together(indexes):
+    """All at once; whether each went in two steps."""
+    var("stream_wait_us").value = 500_000
+    calls = [threading.Thread(target=ix.search, args=(queries, 10)) for ix in indexes]
+    for t in calls: t.start()
+    for t in calls: t.join()
+    var("stream_wait_us").value = 0
+    return [ix.last_scan_ms()[1] > 1 for ix in indexes]
+def rooms(indexes):
+    """What the searches' stages hold, of an amount of memory that was read before any search."""
+    return used.value - start - sum(ix.workspace_bytes()[0] for ix in indexes)
+'''
+
+
+def test_room_for_stages_that_nobody_uses_makes_way(fake):
+    """Three searches at once, which leave almost all that stages may hold; a later one that wants more than any of the three had."""
+    fake(STAGES + '''
+small, large = [batch_index(6_600_000) for _ in range(3)], batch_index(20_000_000)
+start = used.value
+assert together(small) == [True] * 3
+held = rooms(small)
+assert 1.8 * 2**30 < held < 2**31, held
+assert together([large]) == [True]
+assert held / 3 * 1.5 < rooms(small + [large]) <= 2**31, rooms(small + [large])
+assert together(small[:1]) == [True]
+for ix in small + [large]: ix.close()
+assert used.value == 0
+''')

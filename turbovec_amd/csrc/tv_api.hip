@@ -223,25 +223,31 @@ hipError_t device_free(int device, void *p, size_t bytes) {
 // Room for the stages of one search's two-step table scan (NearPlan): lent to one search of the device at a time, whichever
 // index it is of, so that a device holds as many as it has such searches at once, kStagedBytes in all between them, and they do
 // not take the place of blocks that indexes give up and take again (in the pool a 1 GiB block did: building the next index of 10M x 1536 2-bit
-// rows 85 and 249 ms).  Null where there is no memory for one: nothing is given up for it.
+// rows 85 and 249 ms).  What idle places hold makes way where it stands between a search and that limit.  Null where there is no
+// memory for one, or the searches that run hold too much: nothing else is given up for it.
 constexpr size_t kStagedBytes = size_t(2) << 30;
 tv_spare *staged_take(int device, size_t bytes) {
     DevicePool &pool = g_pool[device];
     tv_spare *s = nullptr;
-    void *old = nullptr;
+    void *old[DevicePool::kStaged] = {};
     {
         std::lock_guard<std::mutex> lock(pool.mu);
-        size_t held = 0;
-        for (tv_spare &b : pool.staged) held += b.bytes;
+        size_t held = 0, lent = 0;
+        for (tv_spare &b : pool.staged) held += b.bytes, lent += b.in_use ? b.bytes : 0;
         for (tv_spare &b : pool.staged)      // the smallest that is large enough, otherwise the largest there is, or a free place
             if (!b.in_use && (s == nullptr || (b.bytes >= bytes ? s->bytes < bytes || b.bytes < s->bytes : s->bytes < bytes && b.bytes > s->bytes))) s = &b;
-        if (s == nullptr || (s->bytes < bytes && held - s->bytes + bytes > kStagedBytes)) return nullptr;
+        if (s == nullptr || (s->bytes < bytes && lent + bytes > kStagedBytes)) return nullptr;
         s->in_use = true;
         if (s->bytes >= bytes) return s;
-        old = std::exchange(s->p, nullptr);
-        s->bytes = 0;
+        for (int i = 0; i < DevicePool::kStaged; ++i) {
+            tv_spare &b = pool.staged[i];
+            if (&b != s && (b.in_use || held - s->bytes + bytes <= kStagedBytes)) continue;
+            held -= b.bytes;
+            old[i] = std::exchange(b.p, nullptr);
+            b.bytes = 0;
+        }
     }
-    if (old != nullptr) (void)hipFree(old);
+    for (void *p : old) if (p != nullptr) (void)hipFree(p);
     void *p = nullptr;
     size_t got = 0;
     const hipError_t e = device_alloc(device, bytes, &p, &got, false);
