@@ -16,6 +16,7 @@ typedef struct { uint32_t x, y, z; } dim3_t;
 
 /* ---- what a test sets and reads ---- */
 atomic_size_t fake_limit = (size_t)1 << 34, fake_used;
+atomic_int fake_large_alloc_us;       /* how long an allocation of 256 MiB and more takes */
 atomic_int fake_stream_wait_us;       /* how long a stream's wait takes ... */
 atomic_int fake_stream_waits;         /* ... and how many there were */
 atomic_int fake_frees_refused;        /* so many of the next frees of device memory report an error */
@@ -57,7 +58,10 @@ int hipDeviceSynchronize(void) {
     --fake_device_waits;
     return ok;
 }
-int hipMalloc(void **p, size_t n) { return take(p, n); }
+int hipMalloc(void **p, size_t n) {
+    if (n >= (size_t)256 << 20 && fake_large_alloc_us) usleep(fake_large_alloc_us);
+    return take(p, n);
+}
 int hipFree(void *p) {
     if (p) hipDeviceSynchronize();
     give(p);

@@ -509,3 +509,26 @@ assert together(small[:1]) == [True]
 for ix in small + [large]: ix.close()
 assert used.value == 0
 ''')
+
+
+def test_room_for_stages_has_a_limit(fake):
+    """Searches that start together count what the others are still allocating: 2 GiB for all, and the rest go without.  A block
+    that the library holds already, larger than asked for, counts whole."""
+    fake(STAGES + '''
+made = [batch_index(20_000_000) for _ in range(4)]
+start = used.value
+var("large_alloc_us").value = 200_000
+took = together(made)
+var("large_alloc_us").value = 0
+assert sum(took) == 2 and rooms(made) <= 2**31, (took, rooms(made))
+for ix in made: ix.close()
+assert used.value == 0
+made = [batch_index(20_000_000) for _ in range(2)]
+start = used.value
+gone = batch_index(37_000_000)           # 1.10 GiB of codes, which go to the pool when their index does
+gone.close()
+took = together(made)
+assert sum(took) == 1 and rooms(made) < 1.5 * 2**30, (took, rooms(made))      # (with what else is in the pool)
+for ix in made: ix.close()
+assert used.value == 0
+''')

@@ -153,6 +153,23 @@ void *take_spare(DevicePool &pool) {
     return nullptr;
 }
 
+// The smallest block of the pool that holds so much, a quarter more or `most` at most, or null.  pool.mu held.
+void *take_pooled(DevicePool &pool, size_t bytes, size_t *got, size_t most = ~size_t(0)) {
+    most = std::min(most, bytes + bytes / 4);
+    size_t best = pool.blocks.size();
+    for (size_t i = 0; i < pool.blocks.size(); ++i) {
+        const size_t have = pool.blocks[i].first;
+        if (have >= bytes && have <= most && (best == pool.blocks.size() || have < pool.blocks[best].first)) best = i;
+    }
+    if (best == pool.blocks.size()) return nullptr;
+    void *p = pool.blocks[best].second;
+    *got = pool.blocks[best].first;
+    pool.held -= *got;
+    pool.blocks[best] = pool.blocks.back();
+    pool.blocks.pop_back();
+    return p;
+}
+
 thread_local bool g_refused;      // an allocation of this thread's call was refused for good
 // `device` is current.  *got: what the block holds, 0 on failure.  insist: nothing is refused for what the library only keeps;
 // without, nothing is given up for a block that the caller can do without.
@@ -160,19 +177,7 @@ hipError_t device_alloc(int device, size_t bytes, void **out, size_t *got, bool 
     DevicePool &pool = g_pool[device];
     {
         std::lock_guard<std::mutex> lock(pool.mu);
-        size_t best = pool.blocks.size();
-        for (size_t i = 0; i < pool.blocks.size(); ++i) {
-            const size_t have = pool.blocks[i].first;
-            if (have >= bytes && have <= bytes + bytes / 4 && (best == pool.blocks.size() || have < pool.blocks[best].first)) best = i;
-        }
-        if (best < pool.blocks.size()) {
-            *out = pool.blocks[best].second;
-            *got = pool.blocks[best].first;
-            pool.held -= *got;
-            pool.blocks[best] = pool.blocks.back();
-            pool.blocks.pop_back();
-            return hipSuccess;
-        }
+        if (void *p = take_pooled(pool, bytes, got)) { *out = p; return hipSuccess; }
     }
     hipError_t e = hipMalloc(out, bytes);
     if (e != hipSuccess && insist) {
@@ -239,21 +244,26 @@ tv_spare *staged_take(int device, size_t bytes) {
         if (s == nullptr || (s->bytes < bytes && lent + bytes > kStagedBytes)) return nullptr;
         s->in_use = true;
         if (s->bytes >= bytes) return s;
-        for (int i = 0; i < DevicePool::kStaged; ++i) {
+        held -= s->bytes;
+        old[0] = std::exchange(s->p, nullptr);
+        s->bytes = bytes;      // (counted while it is being allocated)
+        s->p = take_pooled(pool, bytes, &s->bytes, kStagedBytes - lent);
+        for (int i = 0, n = 1; i < DevicePool::kStaged; ++i) {
             tv_spare &b = pool.staged[i];
-            if (&b != s && (b.in_use || held - s->bytes + bytes <= kStagedBytes)) continue;
+            if (b.in_use || held + s->bytes <= kStagedBytes) continue;
             held -= b.bytes;
-            old[i] = std::exchange(b.p, nullptr);
+            old[n++] = std::exchange(b.p, nullptr);
             b.bytes = 0;
         }
     }
     for (void *p : old) if (p != nullptr) (void)hipFree(p);
+    if (s->p != nullptr) return s;      // (lent: nobody else changes it)
     void *p = nullptr;
-    size_t got = 0;
-    const hipError_t e = device_alloc(device, bytes, &p, &got, false);
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
     std::lock_guard<std::mutex> lock(pool.mu);
-    s->p = p;
-    s->bytes = got;
+    s->p = e == hipSuccess ? p : nullptr;
+    if (e != hipSuccess) s->bytes = 0;
     s->in_use = e == hipSuccess;
     return e == hipSuccess ? s : nullptr;
 }
