@@ -19,6 +19,7 @@ atomic_size_t fake_limit = (size_t)1 << 34, fake_used;
 atomic_int fake_large_alloc_us;       /* how long an allocation of 256 MiB and more takes */
 atomic_int fake_stream_wait_us;       /* how long a stream's wait takes ... */
 atomic_int fake_stream_waits;         /* ... and how many there were */
+atomic_int fake_stream_waits_refused; /* so many of the next ones report an error */
 atomic_int fake_frees_refused;        /* so many of the next frees of device memory report an error */
 atomic_int fake_device_busy;          /* the device's wait does not end while this is set ... */
 atomic_int fake_device_waits;         /* ... and this many threads are in one */
@@ -99,7 +100,13 @@ int hipMemcpyAsync(void *to, const void *from, size_t n, int kind, void *s) {
 int hipMemsetAsync(void *p, int v, size_t n, void *s) { (void)s; memset(p, v, n); return ok; }
 int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &last; return ok; }
 int hipStreamDestroy(void *s) { (void)s; return ok; }
-int hipStreamSynchronize(void *s) { (void)s; ++fake_stream_waits; if (fake_stream_wait_us) usleep(fake_stream_wait_us); return ok; }
+int hipStreamSynchronize(void *s) {
+    (void)s;
+    ++fake_stream_waits;
+    if (fake_stream_wait_us) usleep(fake_stream_wait_us);
+    if (fake_stream_waits_refused > 0) { --fake_stream_waits_refused; return last = out_of_memory; }
+    return ok;
+}
 int hipEventCreate(void **e) { *e = &last; return ok; }
 int hipEventDestroy(void *e) { (void)e; return ok; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return ok; }

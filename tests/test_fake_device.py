@@ -532,3 +532,22 @@ assert sum(took) == 1 and rooms(made) < 1.5 * 2**30, (took, rooms(made))      # 
 for ix in made: ix.close()
 assert used.value == 0
 ''')
+
+
+def test_an_index_is_made_when_its_tables_are_there(fake):
+    """The call that makes an index waits for its tables, and an error on their way is that call's."""
+    fake('''
+waits, refused = var("stream_waits"), var("stream_waits_refused")
+before = waits.value
+a = index(0)
+assert waits.value > before
+refused.value = 1
+try:
+    index(0)
+    said = None
+except T.TurbovecHipError as e:
+    said = e.status
+assert said == T.ERR_HIP, said
+a.close()
+assert used.value == 0
+''')

@@ -545,8 +545,8 @@ std::shared_ptr<const TableImage> default_tables(int dim) {
     return t;
 }
 
-// On the index's stream, from pinned memory of its own: one copy (four from pageable memory, with a wait of their own, took 40 us of
-// an index's 90).  The caller has waited for the copy before.
+// On the index's stream, from pinned memory of its own: one copy (four from pageable memory took 40 us of an index's 90).  Waits, so
+// that the tables are there and an error is the call's own.
 int upload_tables(tv_index *ix, const TableImage &t) {
     const size_t words = t.words.size();
     std::memcpy(ix->h_tables, t.words.data(), words * sizeof(uint32_t));
@@ -555,6 +555,7 @@ int upload_tables(tv_index *ix, const TableImage &t) {
     for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
     ix->packed_ok = t.packed_ok;
     TV_HIP(hipMemcpyAsync(ix->d_signs, ix->h_tables, (words + 16) * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
+    TV_HIP(hipStreamSynchronize(ix->stream));
     return TV_OK;
 }
 int effective_mode(const tv_index *ix);
@@ -2275,7 +2276,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
             rc = TV_ERR_HIP;
             break;
         }
-        rc = upload_tables(ix, *tables);      // (all use of them is on the index's stream, behind this)
+        rc = upload_tables(ix, *tables);
     } while (0);
     if (rc != TV_OK) {
         if (g_last_error.empty()) g_last_error = "device allocation failed";
@@ -2347,10 +2348,7 @@ int tv_index_set_tables(tv_index *ix, const float *signs, const uint32_t *perms,
     }
     TableImage t;
     lay_out_tables(ix->rot, t);
-    TV_HIP(hipStreamSynchronize(ix->stream));
-    const int rc = upload_tables(ix, t);
-    if (rc == TV_OK) TV_HIP(hipStreamSynchronize(ix->stream));
-    return rc;
+    return upload_tables(ix, t);
 }
 
 int tv_index_set_calibration(tv_index *ix, const float *shift, const float *scale) {
