@@ -551,3 +551,17 @@ assert said == T.ERR_HIP, said
 a.close()
 assert used.value == 0
 ''')
+
+
+def test_the_line_between_unsampled_and_sampled_of_short_rows(fake):
+    """Short 4-bit rows and many queries: unsampled as far as decoding a block once more for every further four tiles costs less
+    than a sample's floors."""
+    fake('''
+for dim, rows, nq, unsampled in ((256, 350_000, 1024, True), (256, 650_000, 160, True), (256, 850_000, 192, True), (200, 575_273, 512, True), (192, 453_543, 907, True),
+                                 (256, 466_200, 1000, True), (256, 466_400, 1000, False), (384, 700_000, 1000, False), (640, 850_000, 300, False), (512, 850_000, 512, False),
+                                 (192, 900_000, 1024, False), (128, 1_000_000, 1024, True), (640, 1_000_000, 128, True)):
+    ix = index(0, dim)
+    ix.append_rows(np.zeros((rows, dim // 2), np.uint8), np.zeros(rows, np.float32))
+    assert (len(ix.sampling_plan(nq, 10)[0]) == 0) == unsampled, (dim, rows, nq)
+    ix.close()
+''')

@@ -1179,11 +1179,13 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff)
 //    stay in LDS and that this kernel too keeps two tiles of (1.04M x 1024, 64 queries, 1.04e6: 172 and 193) or only one (100K x 1536,
 //    100 queries, 3e5: 100 and 99; 600K x 1536, 64 queries, 9e5: 211 and 185), rows whose tiles are streamed (260K x 3072, 100 queries, 1.6e6:
 //    308 and 528; 500K, 3e6: 489 and 437).
-//  - Rows of 3 to 11 chunks, more than four tiles: the sample's floors cost some 60 us and the all-queries kernel then decodes a block once, not once a
-//    tile group: won up to a number of blocks that falls with the groups and with the tiles the last one lacks (a missing one is level), fitted to 150 queries 450K x 384 90 and 93,
-//    700K x 384 123 and 114; 244 queries 446K x 640 127 and 152, 716K x 640 177 and 206, 1.04M x 448 198 and 177; 300 queries 300K x 256 84 and 103, 450K x 384 132
-//    and 133, 700K x 384 191 and 162; 512 queries 600K x 576 277 and 279, 800K x 576 379 and 343; 600 queries 700K x 512 347 and 308; 1000 queries 200K x 512 196
-//    and 201, 450K x 512 354 and 322, 700K x 384 432 and 363.  Of one or two chunks: 1M x 128, 300 queries 128 and 135, 1000 296 and 283.  Up to four tiles the other
+//  - Rows of 3 to 11 chunks: this kernel decodes a block once for every four tiles, the all-queries kernel once for all of them, but needs a
+//    sample's floors first.  Fitted to 2100 shapes (3 to 10 chunks, 129 to 1024 queries, 150K to 1.04M rows), the (block, chunk) pairs that are
+//    decoded once more cost 0.107 ns each and the floors 22 us, which is 210 000 pairs; the line lies higher, at 280 000 and 4000 a tile, for
+//    the rounds of the other kernel, whose last may be nearly empty (150K x 640, 1024 queries 189 and 221; 350K x 256, 1024 195 and 248): 3 of those shapes
+//    then lose more than 4 % to the search without sampling, and 1.2 % are left lying on the mean.  160 queries 650K x 256 85 and 103; 320, 650K x 384 181 and 175; 512,
+//    550K x 256 156 and 183, 850K x 512 329 and 307; 800, 350K x 512 262 and 241, 850K x 256 374 and 327; 1024, 550K x 192 275 and 287, 550K x 384 360 and 322.
+//    Of one or two chunks: 1M x 128, 300 queries 128 and 135, 1000 296 and 283, 750K x 64, 1000 237 and 402.  Up to four tiles the other
 //    kernel is k_scan_p4_multi: 100 queries 1M x 256 86 and 98, x 640 143 and 137.
 //  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about 700K
 //    rows (1000 queries: 600K x 768 570 and 621, x 1536 972 and 999; 1.04M x 768 935 and 895, x 1536 1611 and 1523),
@@ -1225,11 +1227,7 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks,
         (k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds)) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
-    if (nch <= 2 || (nch < 12 && tiles <= 4)) return true;
-    if (nch < 12) {
-        const double groups = double((tiles + 3) / 4), full = std::min(1.0, double(tiles + 1) / (4.0 * groups));
-        return double(n_blocks) <= (4000.0 + 50000.0 / groups) * full * std::sqrt(full) * (nch == 3 ? 1.5 : 1.0);
-    }
+    if (nch < 12) return nch <= 2 || n_blocks * size_t(nch) * ((tiles + 3) / 4 - 1) <= 280000 + 4000 * tiles;
     return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 16 ? 1050000 : 250000) || n_blocks <= 512;
 }
 // The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
