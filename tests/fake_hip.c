@@ -118,14 +118,35 @@ static const void *mask_count;
 /* tv_kernels.hip's selection by four threads a segment */
 atomic_int fake_parted;               /* launches of it */
 static const void *parted;
+/* every kernel by its mangled name */
+enum { most_kernels = 2048 };
+static struct { const void *host; const char *name; atomic_int launches; size_t lds; } kernels[most_kernels];
+static int n_kernels;
+/* launches of those whose name has `part` in it, and the dynamic LDS of their last ones, at most */
+int fake_launched(const char *part) {
+    int n = 0;
+    for (int i = 0; i < n_kernels; ++i) if (strstr(kernels[i].name, part)) n += kernels[i].launches;
+    return n;
+}
+size_t fake_lds(const char *part) {
+    size_t most = 0;
+    for (int i = 0; i < n_kernels; ++i) if (strstr(kernels[i].name, part) && kernels[i].lds > most) most = kernels[i].lds;
+    return most;
+}
 void __hipRegisterFunction(void **modules, const void *host, char *device, const char *name, unsigned limit, void *a, void *b, void *c, void *d, int *e) {
     (void)modules; (void)device; (void)limit; (void)a; (void)b; (void)c; (void)d; (void)e;
+    if (n_kernels < most_kernels) {
+        kernels[n_kernels].host = host;
+        kernels[n_kernels++].name = strdup(name);
+    }
     if (strstr(name, "k_mask_count")) mask_count = host;
     if (strstr(name, "k_finalILj1024ELj4E")) parted = host;
 }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *s) {
-    (void)g; (void)b; (void)lds; (void)s;
+    (void)g; (void)b; (void)s;
     ++fake_launches;
+    for (int i = 0; i < n_kernels; ++i)
+        if (kernels[i].host == f) { ++kernels[i].launches; kernels[i].lds = lds; }
     fake_parted += f == parted;
     if (f == mask_count && *(uint64_t **)args[5] != NULL) {
         ++fake_counts;
@@ -143,15 +164,17 @@ int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, 
     }
     return ok;
 }
+static _Thread_local size_t pushed_lds;
 int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *s) {
-    (void)b; (void)lds; (void)s;
+    (void)b; (void)s;
+    pushed_lds = lds;
     const int n = (int)(g.x * g.y * g.z);
     if (n > fake_largest_grid) fake_largest_grid = n;
     return ok;
 }
 int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *lds, void **s) {
     *g = *b = (dim3_t){1, 1, 1};
-    *lds = 0;
+    *lds = pushed_lds;
     *s = NULL;
     return ok;
 }

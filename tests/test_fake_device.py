@@ -18,6 +18,9 @@ from turbovec_amd import _lib as T
 def var(name, kind=C.c_int):
     return kind.in_dll(fake, "fake_" + name)
 limit, used = var("limit", C.c_size_t), var("used", C.c_size_t)
+fake.fake_lds.restype = C.c_size_t
+def launched(part):
+    return fake.fake_launched(part.encode())
 def index(rows, dim=64):
     ix = T.NativeIndex(dim, 4)
     if rows:
@@ -563,5 +566,17 @@ for dim, rows, nq, unsampled in ((256, 350_000, 1024, True), (256, 650_000, 160,
     ix = index(0, dim)
     ix.append_rows(np.zeros((rows, dim // 2), np.uint8), np.zeros(rows, np.float32))
     assert (len(ix.sampling_plan(nq, 10)[0]) == 0) == unsampled, (dim, rows, nq)
+    ix.close()
+''')
+
+
+def test_rows_scored_again_whole_have_no_room_for_parts(fake):
+    """The second scoring of a search without sampling: only where a block's chunks go to several waves is there LDS for their sums."""
+    fake('''
+for dim, bits, rows, nq, k, chunks, table in ((1536, 2, 3_000, 800, 14, 12, 1024), (64, 4, 10_000, 900, 82, 1, 64), (320, 3, 5_000, 700, 96, 5, 1024)):
+    ix = T.NativeIndex(dim, bits)
+    ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
+    ix.search(np.ones((nq, dim), np.float32), k)
+    assert fake.fake_lds(b"k_pickI") == k * 256 + chunks * table, (dim, fake.fake_lds(b"k_pickI"))
     ix.close()
 ''')

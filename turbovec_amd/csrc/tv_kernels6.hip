@@ -557,7 +557,8 @@ hipError_t launch_pick_rows(const float *scores, uint32_t stride, uint32_t n, in
     return hipGetLastError();
 }
 
-size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64) + k_eff * 32 * 4; }
+static size_t pick_sum_bytes(size_t k_eff) { return k_eff * 32 * 4; }      // (where a block's chunks go to several waves)
+size_t pick_lds_bytes(int nch, size_t k_eff, bool lut) { return k_eff * 32 * 8 + size_t(nch) * (lut ? 1024 : 64) + pick_sum_bytes(k_eff); }
 int pick_shares(int device, int nch, size_t k_eff, size_t nq, bool lut) {
     // (a SIMD's worth of blocks at least for each workgroup)
     if (nq == 0 || k_eff * size_t(nch) * (lut ? 3 : 1) < kSharedWork) return 1;
@@ -570,8 +571,8 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
                        int shares, uint64_t *shared, uint64_t *stamp, hipStream_t s) {
     if (a.nq_tile <= 0) return hipSuccess;
     if (shares < 1 || (shares > 1 && shared == nullptr)) return hipErrorInvalidValue;
-    const size_t lds = pick_lds_bytes(a.nch, size_t(k_eff), lut);
-    if (k_eff <= 0 || k_eff > kMaxPickK || lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
+    const size_t most_lds = pick_lds_bytes(a.nch, size_t(k_eff), lut);
+    if (k_eff <= 0 || k_eff > kMaxPickK || most_lds > kPickLds || a.b_step != 1 || a.n_blocks > kMaxPickBlocks) return hipErrorInvalidValue;
     PickArgs p;
     p.best = a.best_out; p.best_stride = a.best_stride; p.n_blocks = a.n_blocks; p.n = a.n;
     p.codes = a.codes; p.scales = a.scales; p.mask = a.mask; p.tables = a.tables;
@@ -580,12 +581,6 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     p.nch = a.nch; p.k_eff = k_eff; p.split = split ? 1 : 0;
     p.out_scores = out_scores; p.out_idx = out_idx; p.slots = slots; p.overflow = overflow; p.stamp = stamp;
     p.nq = uint32_t(a.nq_tile); p.shares = uint32_t(shares); p.counts = shared; p.lists = shared + a.nq_tile;
-    auto launch = [&](auto kernel, unsigned threads) -> hipError_t {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kernel, dim3(unsigned(a.nq_tile) * unsigned(shares)), dim3(threads), lds, s, p);
-        return hipGetLastError();
-    };
     // few queries leave the chip empty: as many waves as there are blocks to score again
     const bool small = a.nq_tile > 256 && a.n_blocks <= 256 * 16;
     // A block to a wave leaves most of sixteen waves without one where results are few, and the others with a row's chunks one after the
@@ -600,6 +595,15 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
         for (uint32_t parts = 2; parts <= 16 && int(parts) <= a.nch; parts *= 2)
             if (busiest(parts) < 0.85 * busiest(p.parts) && (busiest(1) - busiest(parts)) * double(a.nch) * (lut ? 2.0 : 1.0) > kPartsChunks) p.parts = parts;
     }
+    // (LDS decides how many queries' workgroups a CU runs at once: with room for sums that are not used 5K x 320 3-bit, 750 queries, k = 92
+    // 128.7 us a search and 106, 10.9K x 64 4-bit, 910, k = 82 68.4 and 57.0, 27K x 768 2-bit, 610, k = 98 217 and 177)
+    const size_t lds = most_lds - (p.parts > 1 ? 0 : pick_sum_bytes(size_t(k_eff)));
+    auto launch = [&](auto kernel, unsigned threads) -> hipError_t {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(a.nq_tile) * unsigned(shares)), dim3(threads), lds, s, p);
+        return hipGetLastError();
+    };
     auto form = [&](auto lut_, auto shared_) -> hipError_t {
         constexpr bool L = decltype(lut_)::value != 0, S = decltype(shared_)::value != 0;
         if constexpr (!S) {
