@@ -580,3 +580,23 @@ for dim, bits, rows, nq, k, chunks, table in ((1536, 2, 3_000, 800, 14, 12, 1024
     assert fake.fake_lds(b"k_pickI") == k * 256 + chunks * table, (dim, fake.fake_lds(b"k_pickI"))
     ix.close()
 ''')
+
+
+def test_parts_of_blocks_are_as_many_as_save_time(fake):
+    """The second scoring in parts: where few results leave waves idle, not in so many turns of short parts that they cost more, and not where
+    several queries share a CU."""
+    fake('''
+def scored(dim, bits, rows, nq, k):
+    ix = T.NativeIndex(dim, bits)
+    ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
+    # (blocks a thread keeps: 16; tables; several workgroups a query; parts)
+    before = [launched(f"k_pickILj1024ELj16ELb{lut}ELb{shared}ELb1EE") for lut in (0, 1) for shared in (0, 1)]
+    ix.search(np.ones((nq, dim), np.float32), k)
+    after = [launched(f"k_pickILj1024ELj16ELb{lut}ELb{shared}ELb1EE") for lut in (0, 1) for shared in (0, 1)]
+    ix.close()
+    return sum(after) - sum(before)
+for shape in ((3072, 4, 40_001, 1, 1), (3072, 4, 40_001, 1, 12), (1000, 3, 20_015, 3, 4), (1416, 2, 20_001, 1, 3), (776, 4, 9_001, 100, 2)):
+    assert scored(*shape) == 1, shape
+for shape in ((1152, 4, 9_638, 168, 23), (720, 4, 153_761, 200, 34), (1536, 3, 4_000, 300, 1), (768, 4, 6_722, 257, 1), (64, 2, 30_031, 1, 1), (768, 4, 50_000, 8, 16)):
+    assert scored(*shape) == 0, shape
+''')

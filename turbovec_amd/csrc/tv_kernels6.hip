@@ -308,8 +308,8 @@ struct PickArgs {
 // Chunks of a query to score again (of tables: thirds), from where sharing them pays (less: 100K x 768, 64 queries, k = 10 43.3 us and, shared,
 // 44.2; 100K x 512 2-bit, one query 35.1 and 36.4; 20K x 384, one query, k = 20 31.9 and 31.1).
 constexpr size_t kSharedWork = 200;
-// Chunks (of tables: halves) that parts have to save the busiest wave, against two barriers and the sums' way through LDS.
-constexpr double kPartsChunks = 10.0;
+// What a part of a block costs beside its chunks, and parts at all -- two barriers, the sums' way through LDS -- in chunks' time.
+constexpr size_t kPartCost = 1, kPartsCost = 3;
 // H: blocks a thread keeps in registers -- all of them, T * H at most.
 // LUT: score mode L with the u32 epilogue.
 // Scoring a block again is 70 (LUT: 200) vector instructions a chunk, on one CU for all of a query's blocks.  Where queries are too few for
@@ -584,16 +584,20 @@ hipError_t launch_pick(const ScanArgs &a, bool lut, bool split, int k_eff, float
     // few queries leave the chip empty: as many waves as there are blocks to score again
     const bool small = a.nq_tile > 256 && a.n_blocks <= 256 * 16;
     // A block to a wave leaves most of sixteen waves without one where results are few, and the others with a row's chunks one after the
-    // other: parts of a block's chunks go to as many waves, as make the busiest wave's share least, where the chip is empty enough for it to
-    // show.  us a search with whole blocks and so: 60K x 3072, one query, k = 1 60.1 and 51.2; 40K x 3032 3-bit, k = 4 88.8 and 82.4; 24K x 2760 2-bit, k = 2
-    // 62.4 and 58.1; 16K x 1424 3-bit, 4 queries, k = 12 61.0 and 58.6; 50K x 768, 8 queries, k = 1 33.1 and 31.7; short rows level (or worse: 95K
-    // x 272 3-bit, 100 queries, k = 33, in two workgroups each, 59.9 and 61.1).
+    // other: so many parts of a block's chunks go to as many waves as make the longest wave's time least, by turns of a wave, chunks of a part and what comes on
+    // top, where a workgroup has a CU to itself and there are no more blocks than waves (more of them fill the waves whole: 23 blocks of 20 chunks in 1, 2, 4, 8 and 16
+    // parts 49.1, 52.0, 52.4, 57.6 and 64.1 us a search).  11 500 shapes, every number of parts: 2.5 % less time than with whole blocks on the mean, 0.6 % more than with
+    // the best number each, and 1 in 2000 shapes more than 3 % slower than with whole blocks.  us a search with whole blocks and so: 60K x 3072, one query, k = 1 60.1 and 51.2; 40K x 3032 3-bit, k = 4 88.8 and 82.4; 24K
+    // x 2760 2-bit, k = 2 62.4 and 58.1; 50K x 768, 8 queries, k = 1 33.1 and 31.7.  Seven blocks of 20 chunks in 1, 2, 4, 8 and 16 parts 33.2, 33.1, 31.7, 33.7 and 37.4; two
+    // workgroups a CU, 352 queries, k = 1, 7 chunks 3-bit, 41.5, 47.8, 47.1, 47.0 and 47.1.
     const size_t waves = 16, share_blocks = (size_t(k_eff) + size_t(shares) - 1) / size_t(shares);
     p.parts = 1;
-    if (size_t(a.nq_tile) * size_t(shares) <= size_t(2) * 256) {
-        auto busiest = [&](size_t parts) { return double((share_blocks * parts + waves - 1) / waves) / double(parts); };
+    if (size_t(a.nq_tile) * size_t(shares) <= 256 && share_blocks <= waves) {
+        auto longest = [&](size_t parts) {
+            return (share_blocks * parts + waves - 1) / waves * (kPartCost + (size_t(a.nch) + parts - 1) / parts) + (parts > 1 ? kPartsCost : 0);
+        };
         for (uint32_t parts = 2; parts <= 16 && int(parts) <= a.nch; parts *= 2)
-            if (busiest(parts) < 0.85 * busiest(p.parts) && (busiest(1) - busiest(parts)) * double(a.nch) * (lut ? 2.0 : 1.0) > kPartsChunks) p.parts = parts;
+            if (longest(parts) < longest(p.parts)) p.parts = parts;
     }
     // (LDS decides how many queries' workgroups a CU runs at once: with room for sums that are not used 5K x 320 3-bit, 750 queries, k = 92
     // 128.7 us a search and 106, 10.9K x 64 4-bit, 910, k = 82 68.4 and 57.0, 27K x 768 2-bit, 610, k = 98 217 and 177)
