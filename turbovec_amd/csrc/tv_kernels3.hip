@@ -165,8 +165,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void k_scan_p4_wide
     // Half of eight waves request the weights, twice as many pieces each, and the others wait for none of them at a hand-over (us a search with
     // all eight and so: 10M x 1536, 1024 queries 13 370 and 13 265, 2-bit 16 110 and 15 790; 2.5M x 1152 2-bit, 150 queries 926 and 894; 4M x 768, 150
     // queries level; a quarter of them 15 880; half of four waves 2 to 6 % more: 2M x 3072, 1024 queries 6300 and 6440.  Having the others touch the next round's
-    // blocks meanwhile, to find them in the caches: 4M x 768, 300 queries, half allowed 745 and 805).
-    constexpr bool kFewLoad = WAVES == 8 && KS == 1;
+    // blocks meanwhile, to find them in the caches: 4M x 768, 300 queries, half allowed 745 and 805).  Not at 12 chunks, the shortest tile of a block a
+    // wave, which the four are late for where the scan is a round or two: 84K x 768, 684 queries 94 with all eight and 99, 154K x 720, 355, k = 34 127 and 131; 1M x 768
+    // 3-bit, 300 715 and 726; 2M x 768 level (1.2M x 512, 300 queries 293 and 287, 2M x 192, 600 385 and 380).
+    constexpr bool kFewLoad = WAVES == 8 && KS == 1 && NCH != 12;
     constexpr int kLoaders = kFewLoad ? 4 : kWideWaves / KS;  // waves that share the loading of one row part's slice
     constexpr int kPieces = kM / kLoaders;                  // direct-to-LDS loads per wave and slice ...
     constexpr int kExtra = kM % kLoaders;                   // ... plus one more in the first kExtra waves
