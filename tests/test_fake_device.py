@@ -600,3 +600,17 @@ for shape in ((3072, 4, 40_001, 1, 1), (3072, 4, 40_001, 1, 12), (1000, 3, 20_01
 for shape in ((1152, 4, 9_638, 168, 23), (720, 4, 153_761, 200, 34), (1536, 3, 4_000, 300, 1), (768, 4, 6_722, 257, 1), (64, 2, 30_031, 1, 1), (768, 4, 50_000, 8, 16)):
     assert scored(*shape) == 0, shape
 ''')
+
+
+def test_filtered_batches_of_tables_gather_where_that_is_less(fake):
+    """Half of the rows at random: whether the two-step scan could take the index with its mask goes by the rows allowed, and what it
+    takes counts its stages' launches."""
+    fake('''
+for dim, bits, rows, nq, k in ((384, 3, 225_592, 929, 40), (2048, 2, 398_963, 780, 26), (512, 3, 352_922, 810, 54), (256, 3, 400_795, 916, 80), (320, 2, 322_259, 705, 2)):
+    ix = T.NativeIndex(dim, bits)
+    ix.append_rows(np.zeros((rows, ix.n_byte_groups), np.uint8), np.zeros(rows, np.float32))
+    words = T.pack_mask(np.random.default_rng(7).random(rows) < 0.5)[0]
+    ix.search(np.ones((nq, dim), np.float32), k, mask_words=words)
+    assert ix.gathered_searches()[0] == 1, (dim, bits)
+    ix.close()
+''')

@@ -1126,9 +1126,10 @@ NearPlan near_plan(const tv_index *ix, const SampledPlan &plan, size_t cq, size_
     p.bytes = p.rows_bytes + largest * group_masks;
     return p;
 }
-bool near_takes(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks) {
+// rows: those of the n_blocks blocks that the search may return.
+bool near_takes(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks, size_t rows) {
     const size_t cq = chunk_len(ix, nq);
-    return near_plan(ix, sampled_plan(ix, cq), cq, k_eff, n_blocks, n_blocks * tv::kVecBlock, n_blocks).stages > 0;
+    return near_plan(ix, sampled_plan(ix, cq), cq, k_eff, n_blocks, rows, rows / tv::kVecBlock).stages > 0;
 }
 // Block offset of a repeated pass's level of stride `step`: it samples other blocks than the pass
 // that misjudged the floor, half a stride in (an even number of blocks, so that mask words stay
@@ -1211,7 +1212,7 @@ bool direct_serves_lut(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blo
     // 389, 6e5 299 and 239; 720K x 768, 188, 8e5 369 and 352; 530K x 384, 273, 4.5e5 296 and
     // 262, 130K x 512, 870, 4.5e5 258 and 207, 120K x 1024, 481, 4.8e5 270 and 241, 460K x 1536, 87, 5.2e5 308 and 288, 98K x 1536, 472, 5.5e5 284 and 294, 99K x 768, 890, 5.2e5 264 and 292; but 116K x 1536, 298, 4.4e5 241 and 264, 650K x 384, 168,
     // 3.7e5 222 and 249, 280K x 664, 155, 2.6e5 170 and 193; longer rows: 140K x 2048, 621, 1.4e6 610 and 642)
-    if (!masked && ix->geo.bits == 2 && nch <= 12 && tiles >= 3 && n_blocks * tiles * nch >= (nch <= 8 && n_blocks >= 3500 ? 450000u : 600000u) && near_takes(ix, nq, k_eff, n_blocks)) return false;
+    if (!masked && ix->geo.bits == 2 && nch <= 12 && tiles >= 3 && n_blocks * tiles * nch >= (nch <= 8 && n_blocks >= 3500 ? 450000u : 600000u) && near_takes(ix, nq, k_eff, n_blocks, n_blocks * tv::kVecBlock)) return false;
     return n_blocks * tiles <= 200000 && rescored <= std::max<size_t>(tiles <= 4 ? 1200u : 600u, 600u * shares);
 }
 bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks, bool masked) {
@@ -1770,24 +1771,23 @@ constexpr double kPassedBlockNs = 0.08;
 // launches and the wait for the count, or what is left of them once the blocks are counted, or where the host knew.  (22 us: half the rows of
 // 100K x 128 at random, 1024 queries, are 20 by this count, and gathering them gains 4 of 78; 10 us from the host: a range of 1 % of
 // 100K x 1536, 1024 queries, is 7.7, and 370 us with the mask and 374 gathered.)  The launches that a search without sampling saves.
-constexpr double kGatherNs = 0.2, kGatherFixedNs = 22000.0, kCountedNs = 5000.0, kKnownNs = 10000.0, kUnsampledNs = 25000.0;
+constexpr double kGatherNs = 0.2, kGatherFixedNs = 22000.0, kCountedNs = 5000.0, kKnownNs = 10000.0, kUnsampledNs = 25000.0, kNearFixedNs = 80000.0;
 // Rows listed while the host waits for the count, and for nothing where it then reads the mask (2M rows of 4M x 256, 40 queries: 181 us
 // with the mask and 201 listed first).
 constexpr size_t kListedAtOnce = size_t(1) << 18;
 constexpr size_t kGatheredBytes = size_t(1) << 30;      // the largest such copy an index keeps room for
 bool gather_pays(const tv_index *ix, size_t nq, size_t k, double n_blocks, double live_blocks, double n_allowed, double fixed, bool in_place) {
     const double blocks = n_allowed / tv::kVecBlock + 1.0, each = scan_block_ns(ix, nq);
-    // (the two-step table scan, which skips no blocks, takes as much of that: 0.85 and 0.7 of the time for 3 and 4 tiles, 0.5 for 7, 0.38 for 32)
+    // (the two-step table scan, which skips no blocks, takes as much of that beside its stages' launches: 0.85 and 0.7 of the time for 3 and 4 tiles, 0.5 for 7, 0.38 for 32)
     const double tiles = std::min(32.0, double((nq + tv::kQTile - 1) / tv::kQTile)), part = ix->geo.bits == 2 ? 0.33 + 1.5 / tiles : std::min(1.0, 0.4 + 2.5 / tiles);
-    auto near = [&](size_t count, bool masked) {
-        return effective_mode(ix) == TV_SCORE_L_U32 && !direct_serves(ix, nq, k, count, masked) && near_takes(ix, nq, k, count);
+    auto scan = [&](double count, double read, bool masked) {
+        const bool near = effective_mode(ix) == TV_SCORE_L_U32 && !direct_serves(ix, nq, k, size_t(count), masked) && near_takes(ix, nq, k, size_t(count), size_t(n_allowed));
+        return near ? kNearFixedNs + part * count * each : read * each;
     };
-    const double all = near(size_t(n_blocks), true) ? part * n_blocks * each : live_blocks * each;
-    const double few = near(size_t(blocks), false) ? part * each : each;
     const double passed = nq > size_t(tv::kQTile) ? kPassedBlockNs * double((nq + tv::kQTile - 1) / tv::kQTile) : 0.0;
     const double gather = kGatherNs * double(ix->geo.nch) * ((in_place ? -1.0 : 1.0) + std::min(8.0, live_blocks / blocks));
     const bool shorter = direct_serves(ix, nq, k, size_t(blocks), false) && !direct_serves(ix, nq, k, size_t(n_blocks), true);
-    return all + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > blocks * (few + passed + gather) + fixed;
+    return scan(n_blocks, live_blocks, true) + n_blocks * passed + (shorter ? kUnsampledNs : 0.0) > scan(blocks, blocks, false) + blocks * (passed + gather) + fixed;
 }
 size_t gathered_need(const tv_index *ix, size_t n_allowed) {
     const size_t blocks = (n_allowed + tv::kVecBlock - 1) / tv::kVecBlock;
@@ -3178,7 +3178,7 @@ int tv_debug_sampling_plan(const tv_index *cix, size_t nq, size_t k, uint32_t *s
     const size_t n_blocks = (ix->n + tv::kVecBlock - 1) / tv::kVecBlock;
     if (direct_serves(ix, nq, k_eff, n_blocks, false)) return TV_OK;
     const SampledPlan plan = sampled_plan(ix, chunk_len(ix, nq));
-    if (near_takes(ix, chunk_len(ix, nq), k_eff, n_blocks)) return TV_OK;
+    if (near_takes(ix, chunk_len(ix, nq), k_eff, n_blocks, ix->n)) return TV_OK;
     const SamplingSteps steps = level_strides(ix, plan, n_blocks, n_blocks, std::max<size_t>(k_eff, 16), false, false);
     *count = steps.size();
     for (size_t i = 0; i < steps.size() && i < cap; ++i) {
