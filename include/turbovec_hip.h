@@ -82,8 +82,13 @@ const char *tv_last_error(void);
  * given back to the device when an allocation of this library fails and when
  * the device's last index is destroyed.  When that is not enough, a failing
  * allocation also takes what the device's indexes keep of filtered searches'
- * allowed rows (tv_debug_workspace_bytes).  Other allocators of the process do
- * not see them.  Calls on host arrays pass through pinned host memory that the
+ * allowed rows (tv_debug_workspace_bytes), and room that no search is using of
+ * the next kind.  Batches of 65 queries and more over large indexes of 2- or
+ * 3-bit codes need room for the rows that they look at twice: up to 1 GiB a
+ * search, 2 GiB in all, lent to one search of the device at a time and kept for
+ * the next until the device's last index is destroyed; a search that finds none
+ * runs without, up to three times as long.  Other allocators of the process do
+ * not see any of this.  Calls on host arrays pass through pinned host memory that the
  * device's indexes share too: allocated on first use, up to 256 MiB, freed with
  * the last index. */
 int tv_index_create(int dim, int bits, int device, tv_index **out);
@@ -262,9 +267,9 @@ int tv_debug_queries_per_launch(const tv_index *ix, int *queries);
  * small indexes (bits 1 and 2 do too), and those of up to 16384 blocks by the
  * levels of rows that tests lay data out against; bit 6 has filtered searches
  * gather the allowed rows first whatever their number; bit 7 has u8-LUT batches
- * take the int8 scan in front of the tables (more than sixteen
- * queries over a large index otherwise) wherever it has an instance for the row
- * length; without bit 6 any other bit, bit 5
+ * take the int8 scan in front of the tables (65 queries and more over a large
+ * index of 2- or 3-bit codes otherwise) wherever it has an instance for the row
+ * length and there are four blocks of rows to sample; without bit 6 any other bit, bit 5
  * of no other meaning too, has them read the mask as they scan. */
 int tv_debug_set_path(tv_index *ix, int force_full_lists);
 /* The sampling ladder a search for the k best of nq queries (its first chunk of up to 1024) runs
@@ -285,7 +290,8 @@ int tv_debug_level_repeats(tv_index *ix, int track, size_t *count);
 /* Bytes of the index's cached search workspace -- with what its filtered searches keep of their
  * allowed rows, up to 1.25 GiB and four bytes a row, which is given back when an allocation of this
  * library fails on that device -- and of its host-call staging allocation (either pointer may be
- * NULL).  They grow otherwise, and tv_search_dev_noalloc touches neither. */
+ * NULL).  They grow otherwise, and tv_search_dev_noalloc touches neither.  What the device's indexes
+ * share (tv_index_create) is not in them. */
 int tv_debug_workspace_bytes(const tv_index *ix, size_t *workspace, size_t *staging);
 /* How many filtered searches so far ran on their allowed rows alone, and how many of
  * those read them in place, without a copy. */

@@ -134,7 +134,7 @@ struct PrepRequest {
     uint8_t *tables;
     uint8_t *tables_mx;             // or null: u8 tables also as the operands of k_scan_lut_mx
     float *qscale, *qbias;
-    uint8_t *near;                  // or null: u8 tables also as int8 weights (with tables_mx; cs and lv are read) ...
+    uint8_t *near;                  // or null: u8 tables also as int8 weights (with tables_mx; near_cs and lv are read) ...
     float *near_unit, *near_err;    // ... and per query what they leave out (tv_prep.hip: near_fit)
     uint32_t lv[2];                 // the int8 levels of up to eight codes
     float *rot_out;                 // or null
