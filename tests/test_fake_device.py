@@ -614,3 +614,47 @@ for dim, bits, rows, nq, k in ((384, 3, 225_592, 929, 40), (2048, 2, 398_963, 78
     assert ix.gathered_searches()[0] == 1, (dim, bits)
     ix.close()
 ''')
+
+
+CHOSEN = '''
+def launches(part, dim, bits, n, nq, k=10, allowed=1.0):
+    """Launches of kernels with `part` in their name in one search."""
+    ix = T.NativeIndex(dim, bits)
+    ix.append_rows(np.zeros((n, ix.n_byte_groups), np.uint8), np.zeros(n, np.float32))
+    before = launched(part)
+    ix.search(np.ones((nq, dim), np.float32), k, mask_words=T.pack_mask(np.random.default_rng(n).random(n) < allowed)[0] if allowed < 1 else None)
+    ix.close()
+    return launched(part) - before
+'''
+
+
+def test_where_the_two_step_scan_starts(fake):
+    """Batches of tables, on both sides of the least blocks and queries; under a filter too."""
+    fake(CHOSEN + '''
+for dim, bits, n, nq, k, takes in ((768, 2, 342_848, 200, 10, False), (768, 2, 342_849, 200, 10, True), (64, 2, 3_400_001, 64, 3, False), (64, 2, 3_400_001, 65, 3, True),
+                                   (256, 3, 738_432, 400, 10, False), (256, 3, 738_433, 400, 10, True)):
+    assert (launches("k_near_rescore", dim, bits, n, nq, k) > 0) == takes, (dim, bits, n, nq)
+for dim, bits, n, nq, k in ((64, 2, 3_400_001, 65, 3), (768, 2, 1_000_001, 200, 10), (256, 3, 800_001, 400, 10)):
+    assert launches("k_near_rescore", dim, bits, n, nq, k, 0.95) > 0, (dim, bits, n, nq)
+''')
+
+
+def test_blocks_in_parts_are_scanned_so(fake):
+    """Few blocks: the scans whose waves take parts of one -- and not where blocks are many or rows of one chunk."""
+    fake(CHOSEN + '''
+for dim, n, nq, parts in ((512, 1, 1, 1), (512, 33, 33, 1), (584, 8_200, 64, 1), (1536, 4_097, 40, 1), (1536, 20_000, 40, 0), (1536, 65_537, 1, 0), (2056, 9_001, 1, 1),
+                          (2056, 9_001, 100, 0), (3072, 30_000, 8, 1), (128, 3_000, 1, 0)):
+    assert launches("k_scan_p4_partsI", dim, 4, n, nq) == parts, (dim, n, nq)
+for dim, bits, n, nq, parts in ((200, 3, 64, 5, 1), (384, 2, 60_001, 8, 1), (1000, 3, 12_345, 8, 1), (1400, 2, 50_001, 2, 1), (1400, 2, 50_001, 6, 0), (3072, 3, 16_411, 3, 1),
+                                (3072, 2, 24_033, 4, 1), (384, 3, 16_001, 16, 1), (384, 3, 16_001, 47, 0), (1536, 2, 5_001, 18, 1), (2432, 3, 4_700, 16, 1), (128, 2, 3_333, 2, 0)):
+    assert launches("k_scan_lut_partsI", dim, bits, n, nq) == parts, (dim, bits, n, nq)
+''')
+
+
+def test_three_tiles_to_a_workgroup(fake):
+    """As many tiles of queries as make no more workgroups so than with four each."""
+    fake(CHOSEN + '''
+for dim, n, nq, three in ((64, 66_001, 65, 1), (128, 40_011, 161, 1), (192, 25_000, 288, 1), (256, 70_003, 150, 1), (448, 66_017, 192, 1), (768, 66_001, 96, 1),
+                          (256, 70_003, 64, 0), (256, 70_003, 128, 0), (256, 70_003, 256, 0), (1536, 70_003, 96, 0), (256, 2_000, 96, 0)):
+    assert launches("k_scan_p4_bestILi3E", dim, 4, n, nq) == three, (dim, n, nq)
+''')
