@@ -219,3 +219,56 @@ def test_fewer_blocks_than_a_sample(bits, nq):
         ix.add_dev(v.data_ptr(), n)
         check(ix, q, (1, 10), always=False)
         ix.close()
+
+
+@pytest.mark.parametrize("dim,bits,n", [(128, 2, 700_000), (128, 3, 700_001), (1536, 2, 105_239), (3072, 2, 55_017)])
+def test_queries_of_zero_and_of_extreme_size(dim, bits, n):
+    """Valid queries that no bound can be had for (zero, and so small or large that a unit of their tables is out of range), among others."""
+    from turbovec_amd import _lib as T
+    gen = torch.Generator(device="cuda:0").manual_seed(dim + bits)
+    ix = T.NativeIndex(dim, bits)
+    v = torch.randn(n, dim, device="cuda:0", generator=gen)
+    torch.cuda.synchronize()
+    ix.add_dev(v.data_ptr(), n)
+    q = torch.randn(70, dim, device="cuda:0", generator=gen).cpu().numpy()
+    q[40] = 0.0
+    for row, size in ((41, 1e-30), (3, 1e-19), (12, 1e-25), (32, 1e-36), (50, 1e-44), (63, 1e15), (64, 1e25), (69, 1e33)):
+        q[row] *= np.float32(size)
+    q[20] = 0.0
+    q[20, 1] = 1.0
+    assert np.isfinite(q).all()
+    ix.set_path(1)
+    s1, i1 = ix.search(q, 10)
+    ix.set_path(TWO_STEP)
+    s, i = ix.search(q, 10)
+    assert ix.last_scan_ms()[1] >= 2
+    assert np.array_equal(i, i1) and bits_equal(s, s1)
+    check(ix, q, always=False)      # (so many queries repeated, with those that share their workgroups, have the searches after it go other ways)
+    ix.close()
+
+
+@pytest.mark.parametrize("dim,bits,n,nq,two_step", [
+    (768, 2, 342_848, 200, False), (768, 2, 342_849, 200, True), (64, 2, 3_400_001, 64, False), (64, 2, 3_400_001, 65, True),
+    (256, 3, 738_432, 400, False), (256, 3, 738_433, 400, True)])
+def test_where_it_starts(dim, bits, n, nq, two_step):
+    """What users get, with and without a filter, on both sides of the least blocks and queries."""
+    from turbovec_amd import _lib as T
+    gen = torch.Generator(device="cuda:0").manual_seed(n)
+    ix = T.NativeIndex(dim, bits)
+    for at in range(0, n, 400_000):
+        v = torch.randn(min(400_000, n - at), dim, device="cuda:0", generator=gen)
+        torch.cuda.synchronize()
+        ix.add_dev(v.data_ptr(), len(v))
+    q = torch.randn(nq, dim, device="cuda:0", generator=gen).cpu().numpy()
+    words = T.pack_mask(np.random.default_rng(n).random(n) < 0.95)[0]
+    some = np.unique(np.linspace(0, nq - 1, 40).astype(int))
+    for m in (None, words):
+        ix.set_path(1)
+        s1, i1 = ix.search(q[some], 3, mask_words=m)
+        ix.set_path(0)
+        for _ in range(2):
+            s, i = ix.search(q, 3, mask_words=m)
+            if m is None:       # (launches: both steps')
+                assert (ix.last_scan_ms()[1] >= 2) == two_step
+            assert np.array_equal(i[some], i1) and bits_equal(s[some], s1)
+    ix.close()
