@@ -658,3 +658,29 @@ for dim, n, nq, three in ((64, 66_001, 65, 1), (128, 40_011, 161, 1), (192, 25_0
                           (256, 70_003, 64, 0), (256, 70_003, 128, 0), (256, 70_003, 256, 0), (1536, 70_003, 96, 0), (256, 2_000, 96, 0)):
     assert launches("k_scan_p4_bestILi3E", dim, 4, n, nq) == three, (dim, n, nq)
 ''')
+
+
+def test_values_are_refused_wherever_they_are(fake):
+    """Searches of host arrays look at every value of what they copy: first and last, next to the ends of the runs that are looked
+    at together; the largest that is accepted is."""
+    fake('''
+ix = index(1000, 8)
+largest = np.nextafter(np.float32(1e16), np.float32(0))
+for nq in (1, 3, 512, 513, 2049):
+    q = np.full((nq, 8), 0.5, np.float32)
+    q[::2] *= -1
+    places = sorted({p for p in (0, 1, 7, 4095, 4096, 4097, nq * 8 // 2, nq * 8 - 9, nq * 8 - 1) if 0 <= p < nq * 8})
+    for p in places:
+        for value in (np.nan, -np.nan, np.inf, -np.inf, 1e16, -1e16, np.float32(3e38), largest, -largest, np.float32(1e-45), -0.0):
+            held = q.flat[p]
+            q.flat[p] = value
+            try:
+                ix.search(q, 3, checked=True)
+                refused = False
+            except T.TurbovecHipError as e:
+                assert e.status == T.ERR_INVALID_QUERY_VALUE
+                refused = True
+            assert refused == (not abs(np.float32(value)) < np.float32(1e16)), (nq, p, value)
+            q.flat[p] = held
+ix.close()
+''')
