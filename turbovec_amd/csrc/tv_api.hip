@@ -552,8 +552,12 @@ std::shared_ptr<const TableImage> default_tables(int dim) {
     return t;
 }
 
-// On the index's stream, from pinned memory of its own: one copy (four from pageable memory took 40 us of an index's 90).  Waits, so
-// that the tables are there and an error is the call's own.
+constexpr size_t kChunkQueries = 1024;
+// a chunk's floors are laid out tile by tile, kQTile slots per tile, and a tile may hold one query
+constexpr size_t kTauOpenInts = kChunkQueries * tv::kQTile;
+
+// On the index's stream, from pinned memory of its own, which the device reads where it lies (four copies from pageable memory took 40 us
+// of an index's 90).  The caller waits before its call ends, so that the tables are there and an error is that call's own.
 int upload_tables(tv_index *ix, const TableImage &t) {
     const size_t words = t.words.size();
     std::memcpy(ix->h_tables, t.words.data(), words * sizeof(uint32_t));
@@ -561,8 +565,8 @@ int upload_tables(tv_index *ix, const TableImage &t) {
     std::fill_n(cen, 16, 0.0f);
     for (size_t i = 0; i < ix->cb.centroids.size(); ++i) cen[i] = ix->cb.centroids[i];
     ix->packed_ok = t.packed_ok;
-    TV_HIP(hipMemcpyAsync(ix->d_signs, ix->h_tables, (words + 16) * sizeof(uint32_t), hipMemcpyHostToDevice, ix->stream));
-    TV_HIP(hipStreamSynchronize(ix->stream));
+    // (and the floors of a search's first sampling level: the order key of -inf for every query)
+    TV_HIP(tv::launch_lay_tables(ix->d_flags_host + (ix->h_tables - ix->h_flags), reinterpret_cast<uint32_t *>(ix->d_signs), words + 16, ix->d_tau_open, int(0x807fffffu), kTauOpenInts, ix->stream));
     return TV_OK;
 }
 int effective_mode(const tv_index *ix);
@@ -690,9 +694,6 @@ void fill_scan_args(const tv_index *ix, tv::ScanArgs &a) {
     a.b_step = 1;
 }
 
-constexpr size_t kChunkQueries = 1024;
-// a chunk's floors are laid out tile by tile, kQTile slots per tile, and a tile may hold one query
-constexpr size_t kTauOpenInts = kChunkQueries * tv::kQTile;
 constexpr int kMaxTimedTiles = int(kChunkQueries / tv::kQTile);
 
 static_assert(kMaxTimedTiles == tv::kTimedLaunches, "the index holds one event pair per timed launch");
@@ -2240,9 +2241,7 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         else if (ix->geo.nch <= 24) ix->geo.nch += ix->geo.nch & 1;
     }
     const auto tables = default_tables(dim);
-    ix->rot = tables->rot;
     ix->cb = tv::make_codebook(bits, dim);
-    derive_levels(ix);
     int rc = TV_OK;
     do {
         if (hipStreamCreateWithFlags(&ix->stream, hipStreamNonBlocking) != hipSuccess) { rc = TV_ERR_HIP; break; }
@@ -2274,14 +2273,13 @@ int tv_index_create(int dim, int bits, int device, tv_index **out) {
         ix->h_stamps = reinterpret_cast<uint64_t *>(ix->h_flags + kGroupQueries + kLevelFlagWords);
         ix->d_stamps = reinterpret_cast<uint64_t *>(ix->d_flags_host + kGroupQueries + kLevelFlagWords);
         std::fill_n(ix->h_stamps, tv::kStampsBefore + 1, uint64_t(0));
+        rc = upload_tables(ix, *tables);
+        if (rc != TV_OK) break;
         rc = scratch_address(device, &ix->scratch);
         if (rc != TV_OK) break;
-        // floors of a search's first sampling level: the order key of -inf for every query, written once
-        if (tv::launch_fill_i32(ix->d_tau_open, int(0x807fffffu), kTauOpenInts, ix->stream) != hipSuccess) {
-            rc = TV_ERR_HIP;
-            break;
-        }
-        rc = upload_tables(ix, *tables);
+        ix->rot = tables->rot;      // (while the device reads)
+        derive_levels(ix);
+        if (hipStreamSynchronize(ix->stream) != hipSuccess) rc = TV_ERR_HIP;
     } while (0);
     if (rc != TV_OK) {
         if (g_last_error.empty()) g_last_error = "device allocation failed";
@@ -2353,7 +2351,9 @@ int tv_index_set_tables(tv_index *ix, const float *signs, const uint32_t *perms,
     }
     TableImage t;
     lay_out_tables(ix->rot, t);
-    return upload_tables(ix, t);
+    const int rc = upload_tables(ix, t);
+    if (rc == TV_OK) TV_HIP(hipStreamSynchronize(ix->stream));
+    return rc;
 }
 
 int tv_index_set_calibration(tv_index *ix, const float *shift, const float *scale) {

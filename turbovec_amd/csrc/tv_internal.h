@@ -259,6 +259,7 @@ hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t
 hipError_t launch_gather_redo(const float *d_q, const uint32_t *d_rows, const int *d_raised, int dim, int tile_q,
                               size_t n_redo, float *d_q_out, int *d_tau_out, hipStream_t s);
 hipError_t launch_fill_i32(int *p, int v, size_t n, hipStream_t s);
+hipError_t launch_lay_tables(const uint32_t *from, uint32_t *to, size_t n, int *floors, int v, size_t n_floors, hipStream_t s);
 hipError_t launch_probe(const void *src, void *dst, size_t bytes, int copy, uint32_t *sink, hipStream_t s);
 hipError_t launch_probe_mfma(int device, int iters, uint32_t *sink, double *ops, hipStream_t s);
 // Exact top-k of a dense score row per query (NaN = excluded slot).
