@@ -557,15 +557,17 @@ assert used.value == 0
 
 
 def test_the_line_between_unsampled_and_sampled_of_short_rows(fake):
-    """Short 4-bit rows and many queries: unsampled as far as decoding a block once more for every further four tiles costs less
-    than a sample's floors."""
+    """Short 4-bit rows and many queries: unsampled as far as decoding a block once more for every further four tiles, and scoring the
+    results' blocks again, cost less than a sample's floors and the empty places of the other kernel's last round."""
     fake('''
-for dim, rows, nq, unsampled in ((256, 350_000, 1024, True), (256, 650_000, 160, True), (256, 850_000, 192, True), (200, 575_273, 512, True), (192, 453_543, 907, True),
-                                 (256, 466_200, 1000, True), (256, 466_400, 1000, False), (384, 700_000, 1000, False), (640, 850_000, 300, False), (512, 850_000, 512, False),
-                                 (192, 900_000, 1024, False), (128, 1_000_000, 1024, True), (640, 1_000_000, 128, True)):
+for dim, rows, nq, k, unsampled in ((256, 350_000, 1024, 10, True), (256, 650_000, 160, 10, True), (256, 418_176, 1000, 10, True), (256, 418_177, 1000, 10, False),
+                                    (192, 469_376, 1024, 10, True), (192, 469_377, 1024, 10, False), (192, 524_289, 1024, 10, True), (640, 667_872, 150, 10, True),
+                                    (640, 667_873, 150, 10, False), (384, 700_000, 1000, 10, False), (640, 850_000, 300, 10, False), (512, 850_000, 512, 10, False),
+                                    (136, 729_140, 397, 59, False), (368, 388_650, 928, 75, False), (168, 318_674, 387, 100, True), (256, 350_000, 1024, 100, False),
+                                    (640, 4_096, 1024, 100, True), (640, 4_200, 1024, 60, True), (128, 1_000_000, 1024, 100, True), (640, 1_000_000, 128, 60, True)):
     ix = index(0, dim)
     ix.append_rows(np.zeros((rows, dim // 2), np.uint8), np.zeros(rows, np.float32))
-    assert (len(ix.sampling_plan(nq, 10)[0]) == 0) == unsampled, (dim, rows, nq)
+    assert (len(ix.sampling_plan(nq, k)[0]) == 0) == unsampled, (dim, rows, nq, k)
     ix.close()
 ''')
 

@@ -34,6 +34,6 @@ def test_both_sides(dim, n, nq):
     ix.close()
 
 
-@pytest.mark.parametrize("dim,n,nq", [(256, 466_200, 1000), (256, 466_400, 1000), (192, 621_600, 1024), (192, 621_900, 1024), (640, 959_900, 150), (640, 960_100, 150)])
+@pytest.mark.parametrize("dim,n,nq", [(256, 418_176, 1000), (256, 418_177, 1000), (192, 469_376, 1024), (192, 469_377, 1024), (640, 667_872, 150), (640, 667_873, 150)])
 def test_both_sides_of_decoding_blocks_again(dim, n, nq):
     test_both_sides(dim, n, nq)

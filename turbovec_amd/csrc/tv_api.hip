@@ -1188,12 +1188,13 @@ size_t direct_need(const tv_index *ix, size_t cq, size_t n_blocks, size_t k_eff)
 //    stay in LDS and that this kernel too keeps two tiles of (1.04M x 1024, 64 queries, 1.04e6: 172 and 193) or only one (100K x 1536,
 //    100 queries, 3e5: 100 and 99; 600K x 1536, 64 queries, 9e5: 211 and 185), rows whose tiles are streamed (260K x 3072, 100 queries, 1.6e6:
 //    308 and 528; 500K, 3e6: 489 and 437).
-//  - Rows of 3 to 11 chunks: this kernel decodes a block once for every four tiles, the all-queries kernel once for all of them, but needs a
-//    sample's floors first.  Fitted to 2100 shapes (3 to 10 chunks, 129 to 1024 queries, 150K to 1.04M rows), the (block, chunk) pairs that are
-//    decoded once more cost 0.107 ns each and the floors 22 us, which is 210 000 pairs; the line lies higher, at 280 000 and 4000 a tile, for
-//    the rounds of the other kernel, whose last may be nearly empty (150K x 640, 1024 queries 189 and 221; 350K x 256, 1024 195 and 248): 3 of those shapes
-//    then lose more than 4 % to the search without sampling, and 1.2 % are left lying on the mean.  160 queries 650K x 256 85 and 103; 320, 650K x 384 181 and 175; 512,
-//    550K x 256 156 and 183, 850K x 512 329 and 307; 800, 350K x 512 262 and 241, 850K x 256 374 and 327; 1024, 550K x 192 275 and 287, 550K x 384 360 and 322.
+//  - Rows of 3 to 11 chunks: this kernel decodes a block once for every four tiles and scores k blocks a query again, the all-queries kernel decodes it
+//    once for all tiles, but needs a sample's floors first and takes whole rounds of blocks.  By 22 000 searches both ways (3 to 10 chunks, 129 to 1024 queries, 4200 to
+//    1.04M rows, k = 1 to 120, Gaussian and clustered), in the time of one (block, chunk) pair decoded once more, about 0.1 ns: a block scored again 176 a
+//    chunk for every 256 queries, which is one a CU; the floors 160 000 and 4000 a tile; a place of the last round that no block takes, a quarter a chunk and tile.  0.6 % off the
+//    faster way on the mean, 4.8 % of the searches by more than 4 %; without the second and the last of these 1.2 % and 8.4 %.  k = 10:
+//    491K x 176, 182 queries 70 and 83; 164K x 616, 562 137 and 147; 130K x 264, 964 99 and 133; 864K x 608, 329 302 and 273; 638K x 488, 505 246 and 221.  More
+//    results: 729K x 136, 397, k = 59 193 and 174; 389K x 368, 928, k = 75 319 and 255; 319K x 168, 387, k = 100 116 and 131, k = 33 98 and 114.
 //    Of one or two chunks: 1M x 128, 300 queries 128 and 135, 1000 296 and 283, 750K x 64, 1000 237 and 402.  Up to four tiles the other
 //    kernel is k_scan_p4_multi: 100 queries 1M x 256 86 and 98, x 640 143 and 137.
 //  - On the all-queries kernel its epilogue over every pair costs as much as sampling saves at about 700K
@@ -1236,7 +1237,12 @@ bool direct_serves(const tv_index *ix, size_t nq, size_t k_eff, size_t n_blocks,
         (k_eff * nch > (tiles == 1 && direct_shares(ix, nq, k_eff) > 1 ? kSharedMost : 600u) || tv::pick_lds_bytes(nch, k_eff, false) > tv::kPickLds)) return false;
     if (direct_wide(ix, cq, n_blocks)) return n_blocks <= (k_eff * nch <= 300 ? kDirectWideBlocks : kDirectWideBlocks / 2);
     if (tiles == 1) return n_blocks <= (nch <= 24 ? 16384u : 8192u) || triples <= 327680;
-    if (nch < 12) return nch <= 2 || n_blocks * size_t(nch) * ((tiles + 3) / 4 - 1) <= 280000 + 4000 * tiles;
+    if (nch <= 2) return true;
+    if (nch < 12) {
+        const size_t round = size_t(tv::wide_grid_blocks(ix->device)) * size_t(tv::wide_blocks_per_workgroup(nch)), empty = (n_blocks + round - 1) / round * round - n_blocks;
+        const size_t again = direct_rows(ix, cq, n_blocks, k_eff) ? 0 : 176 * k_eff * ((cq + 255) / 256);
+        return (n_blocks * ((tiles + 3) / 4 - 1) + again) * size_t(nch) <= 160000 + 4000 * tiles + empty * tiles * size_t(nch) / 4;
+    }
     return triples <= (!tv::batched_weights_split(nch) ? 1600000 : nch <= 16 ? 1050000 : 250000) || n_blocks <= 512;
 }
 // The best score of every scanned block for u8-LUT queries, on the kernel that serves so many in a full scan: byte tables for one,
