@@ -686,3 +686,15 @@ for nq in (1, 3, 512, 513, 2049):
             q.flat[p] = held
 ix.close()
 ''')
+
+
+def test_selections_that_check_guessed_floors(fake):
+    """Only the two-step table scan's selections are the instances that know of guessed floors."""
+    fake(CHOSEN + '''
+def guessed(*shape):
+    # (threads, threads a segment, guessed floors)
+    return sum(launches(f"k_finalILj{t}ELj1ELb1EE", *shape) for t in (256, 512, 1024)) > 0
+assert guessed(64, 2, 3_400_001, 65, 3)
+for shape in ((64, 2, 3_400_001, 64, 3), (128, 4, 1_472_940, 7, 66), (64, 4, 1_200_000, 1024, 10), (768, 4, 200_000, 2, 200)):
+    assert launches("k_finalI", *shape) > 0 and not guessed(*shape), shape
+''')

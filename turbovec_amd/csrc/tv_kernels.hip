@@ -957,7 +957,9 @@ constexpr uint32_t kFinalLong = 128;       // ... of which this many segments ca
 constexpr double kFinalLongest = 16.0;
 static_assert(kSelectKept > uint32_t(kMaxSampledK) && kFinalStage / 17 < kFinalLong, "k_final's buffers");
 
-template <uint32_t T, uint32_t PARTS>
+// GUESSED: the two-step table scan's selections, with `passed` or keep_floor == 2 (an instance of its own: the others lost 0.4 us a launch to
+// it, 1.47M x 128, 7 queries, k = 66 95.5 us a search and, without, 93.9).
+template <uint32_t T, uint32_t PARTS, bool GUESSED>
 __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
                                                const uint32_t *__restrict__ cand_cnt, uint32_t n_seg,
                                                uint32_t seg_stride, int k_eff, int k_floor,
@@ -1039,10 +1041,14 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
     if (!sampling) {
         const bool redo = too_many || any_full || total < uint32_t(k_eff);
         raising = redo && raise_out != nullptr && total >= uint32_t(k_eff);
-        // (floors that were guessed: a query that too few rows reached is repeated from an open one)
-        const bool missed = passed != nullptr && !too_many && !any_full && total < uint32_t(k_eff);
-        if (t == 0 && missed && raise_out != nullptr) raise_out[qn] = kTauInit;
-        if (t == 0 && (redo || passed == nullptr)) overflow[qn] = redo ? (raising || (missed && raise_out != nullptr) ? 1u : 2u) : 0u;
+        if constexpr (GUESSED) {
+            // (floors that were guessed: a query that too few rows reached is repeated from an open one)
+            const bool missed = passed != nullptr && !too_many && !any_full && total < uint32_t(k_eff);
+            if (t == 0 && missed && raise_out != nullptr) raise_out[qn] = kTauInit;
+            if (t == 0 && (redo || passed == nullptr)) overflow[qn] = redo ? (raising || (missed && raise_out != nullptr) ? 1u : 2u) : 0u;
+        } else if (t == 0) {
+            overflow[qn] = redo ? (raising ? 1u : 2u) : 0u;
+        }
         if (redo && !raising) return;
     }
     // (the last query's workgroup is among the last to end)
@@ -1123,12 +1129,12 @@ __global__ __launch_bounds__(T) void k_final(const uint64_t *__restrict__ cand,
             // the floor: the k_floor-th best sampled score (k_floor >= k_eff steadies the estimate)
             if (rank == need - 1u) {
                 const int floor = order_key(s == 0.0f ? -0.0f : s);
-                *(sampling ? tau_slot : raise_out + qn) = sampling && keep_floor == 2 ? max(floor, *tau_slot) : floor;
+                *(sampling ? tau_slot : raise_out + qn) = GUESSED && sampling && keep_floor == 2 ? max(floor, *tau_slot) : floor;
             }
         } else {
             // Of floors that were guessed the highest is the last: what the scans left out lies below it, and the result is whole if its
             // last row does not.  Otherwise that row is a floor k rows do reach.
-            if (passed != nullptr && rank == need - 1u) {
+            if (GUESSED && passed != nullptr && rank == need - 1u) {
                 const int last = order_key(s == 0.0f ? -0.0f : s);
                 const bool missed = last < passed[(qn / tau_stride_q) * kQTile + qn % tau_stride_q];
                 overflow[qn] = missed ? (raise_out != nullptr ? 1u : 2u) : 0u;
@@ -1450,10 +1456,14 @@ hipError_t launch_final(const uint64_t *cand, const uint32_t *cand_cnt, uint32_t
         hipLaunchKernelGGL(kernel, dim3(nq), dim3(threads), 0, s, cand, cand_cnt, n_seg, seg_stride, k_eff, k_floor, out_scores,
                            out_idx, overflow, tau_out, tau_stride_q, keep_floor, raise_out, row_map, level_over, clear_flag, run_if, slots, stamp, passed);
     };
-    if (n_seg <= 256 && nq == 1 && longest > kFinalLongest) launch(k_final<1024, 4>, 1024);
-    else if (n_seg <= 256) launch(k_final<256, 1>, 256);
-    else if (n_seg <= 512) launch(k_final<512, 1>, 512);
-    else launch(k_final<1024, 1>, 1024);
+    if (passed != nullptr || keep_floor == 2) {
+        if (n_seg <= 256) launch(k_final<256, 1, true>, 256);
+        else if (n_seg <= 512) launch(k_final<512, 1, true>, 512);
+        else launch(k_final<1024, 1, true>, 1024);
+    } else if (n_seg <= 256 && nq == 1 && longest > kFinalLongest) launch(k_final<1024, 4, false>, 1024);
+    else if (n_seg <= 256) launch(k_final<256, 1, false>, 256);
+    else if (n_seg <= 512) launch(k_final<512, 1, false>, 512);
+    else launch(k_final<1024, 1, false>, 1024);
     return hipGetLastError();
 }
 
