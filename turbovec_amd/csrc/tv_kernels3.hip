@@ -131,7 +131,7 @@ constexpr int kWideTableBytes = 1024;    // the byte table of the split decode (
 // NEAR: 2- or 3-bit codes, whose score is a sum over u8 tables (tv_kernels5.hip); this scan goes before it.  A
 // row's table sum is at most unit * P + err with P the int8 product of the row's levels and the weights of k_prep_lut's near_fit,
 // so a row whose P stays below a bound of its query's floor and its own scale need not be looked up (10M x 1536 2-bit, 1024 queries, k =
-// 100: 45.9 ms a search on the one-hot products alone, 15.2 to 16.0 so, 11.9 to 12.3 of them here -- the matrix unit's rate for
+// 100: 45.9 ms a search on the one-hot products alone, 15.2 to 16.4 so, 11.9 to 12.3 of them here -- the matrix unit's rate for
 // the same products on 4-bit codes).  NCH counts chunks of 64
 // dimensions (a 2-bit row's 32 byte-groups are two of them).  Nothing is scored: a bit per row and query says whether it
 // is still in, and the rows are written out one after the other for k_near_rescore, which looks those up.  Each query

@@ -10,7 +10,7 @@
 //
 // What bounds it: one LDS instruction per look-up, six clocks each with 32 waves per CU (no bank conflicts by the counters; one or
 // two vector instructions beside it), and the latency of a row's first line.  10M rows x 1536 2-bit, 1024 queries, k = 100: 14 000 rows
-// a query, 2.9 ms of the search's 15.2 to 16.0.  With eight queries and sixteen waves per CU, where the tables of four would let 32
+// a query, 2.9 ms of the search's 15.2 to 16.4.  With eight queries and sixteen waves per CU, where the tables of four would let 32
 // run, 20 to 40 % longer over short stages (890K x 920, 640 queries: 66 us a launch and 45), level over long ones.
 #include "tv_device.h"
 #include "tv_internal.h"
